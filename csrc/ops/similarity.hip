@@ -18,10 +18,10 @@
 // 16 rows x 64 B — half the load-path work per streamed byte), the (<= 64) queries sit in LDS as B operands, so a 205 GB
 // 100M x 1024 index is read exactly once per batch of agent queries. Scores
 // above a query's running threshold (and passing the filters) are appended to
-// that query's candidate buffer (global workspace, per workgroup); a full buffer
-// is sorted (bitonic, in LDS) and the threshold raised to its k-th best. Each
+// that query's candidate buffer (global workspace, per workgroup); one wave cuts a
+// full buffer to its k best (topk_select.h) and raises the threshold to the k-th. Each
 // slice writes its top-k. Stage 2 (one WG per query) merges the slices' lists.
-#include "common.h"
+#include "topk_select.h"
 
 namespace pa {
 
@@ -31,7 +31,10 @@ constexpr int SIM_QT = 16;        // queries per MFMA tile (N = 16)
 constexpr int SIM_MAXQ = 64;      // queries per pass (4 tiles resident in LDS)
 constexpr int SIM_MAXD = 1024;    // LDS query capacity per query (bf16)
 constexpr int SIM_THREADS = 1024; // 16 waves: 128 KB of row loads in flight per CU
-constexpr int SIM_MIN_ROWS_PER_WG = 2048;
+// one round of 16 waves x 16 rows a slice at least: 20,000 rows give 79 slices (10 with the 2,048 rows that the sorting
+// compactions needed: 126 us for 3 queries)
+constexpr int SIM_MIN_ROWS_PER_WG = 256;
+constexpr int SIM_LIM = 2 * SIM_MAXK;  // entries of a buffer between rounds; a round may admit 256 more
 constexpr int SIM_KB = 8;         // k-steps per row-load batch (two batches in flight)
 constexpr int SIM_MAX_WG = 256;    // one resident workgroup per CU: the threshold warm-up is paid once per CU
 
@@ -42,59 +45,46 @@ __host__ __device__ inline int sim_num_wg(int N) {
   return nwg;
 }
 
-// Sort cand_s/cand_r[0..SIM_CAND) descending by score (whole workgroup, >= SIM_CAND threads).
-__device__ void bitonic_desc(float* cs, int* cr) {
-  for (int k = 2; k <= SIM_CAND; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      __syncthreads();
-      const int i = threadIdx.x;
-      const int p = i ^ j;
-      if (i < SIM_CAND && p > i) {
-        const bool desc = (i & k) == 0;
-        const float a = cs[i], b = cs[p];
-        const bool swap = desc ? (a < b) : (a > b);
-        if (swap) {
-          cs[i] = b; cs[p] = a;
-          const int t = cr[i]; cr[i] = cr[p]; cr[p] = t;
-        }
-      }
+// Cut query buffer `gs/gr` to its best K and raise the threshold: one wave, no barrier, about a microsecond (a bitonic sort
+// by the workgroup took ten, one query after the other). os / orow: where the slice's list goes, or null to keep it.
+__device__ __forceinline__ void compact_global(float* gs, int* gr, int* cnt, float* theta, int K, float* os = nullptr,
+                                               int* orow = nullptr) {
+  constexpr int PER = SIM_CAND / 64;
+  const int lane = threadIdx.x & 63, n = min(*cnt, SIM_CAND);
+  uint32_t key[PER];
+  int row[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = i * 64 + lane;
+    key[i] = e < n ? ord_key(gs[e]) : 0;
+    row[i] = e < n ? gr[e] : -1;
+  }
+  uint32_t cut = 1;  // entries above it stay, and of those at it as many as there is room for
+  int room = K, at = 0;
+  if (n >= K) {
+    cut = wave_select(key, K);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) room -= __popcll(__ballot(key[i] > cut));
+  }
+  if (os) { gs = os; gr = orow; }
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const unsigned long long ties = __ballot(key[i] == cut);
+    const bool keep = key[i] > cut || (key[i] == cut && rank_in(ties) < room);
+    room -= __popcll(ties);
+    const unsigned long long kept = __ballot(keep);
+    if (keep) {
+      const int p = at + rank_in(kept);
+      gs[p] = key_value(key[i]);
+      gr[p] = row[i];
     }
+    at += __popcll(kept);
   }
-  __syncthreads();
-}
-
-// Compact query c's buffer to its best K entries and update its threshold.
-__device__ void compact_query(float* cs, int* cr, int* cnt, float* theta, int K) {
-  const int n = min(*cnt, SIM_CAND);
-  if (threadIdx.x < SIM_CAND && threadIdx.x >= n) { cs[threadIdx.x] = -INFINITY; cr[threadIdx.x] = -1; }
-  bitonic_desc(cs, cr);
-  if (threadIdx.x == 0) {
-    const int keep = min(n, K);
-    *cnt = keep;
-    if (keep == K) *theta = cs[K - 1];
+  if (os && lane >= at && lane < K) { gs[lane] = -INFINITY; gr[lane] = -1; }
+  if (lane == 0) {
+    *cnt = at;
+    if (at == K) *theta = key_value(cut);
   }
-  __syncthreads();
-}
-
-// Sort the global candidate buffer `gs/gr` of one query through the LDS scratch,
-// keep the best K, raise the threshold.
-__device__ void compact_global(float* gs, int* gr, float* cs, int* cr, int* cnt, float* theta, int K) {
-  const int n = min(*cnt, SIM_CAND);
-  if (threadIdx.x < SIM_CAND) {
-    cs[threadIdx.x] = threadIdx.x < n ? gs[threadIdx.x] : -INFINITY;
-    cr[threadIdx.x] = threadIdx.x < n ? gr[threadIdx.x] : -1;
-  }
-  bitonic_desc(cs, cr);  // begins and ends with a barrier
-  if (threadIdx.x < K) {
-    gs[threadIdx.x] = cs[threadIdx.x];
-    gr[threadIdx.x] = cr[threadIdx.x];
-  }
-  if (threadIdx.x == 0) {
-    const int keep = min(n, K);
-    *cnt = keep;
-    if (keep == K) *theta = cs[K - 1];
-  }
-  __syncthreads();
 }
 
 __global__ __launch_bounds__(SIM_THREADS) void cosine_stage1_kernel(
@@ -107,12 +97,12 @@ __global__ __launch_bounds__(SIM_THREADS) void cosine_stage1_kernel(
   const int NQT = (Q + SIM_QT - 1) / SIM_QT;
   const int QLD = D + 8;  // padded LDS row: the 16 query rows of a B fragment hit distinct bank slots
   bf16* qt = reinterpret_cast<bf16*>(smem);                                     // [NQT*16][QLD]
-  float* cs = reinterpret_cast<float*>(smem + (size_t)NQT * SIM_QT * QLD * 2);  // sort scratch [CAND]
-  int* cr = reinterpret_cast<int*>(cs + SIM_CAND);                            // [CAND]
-  int* cnt = cr + SIM_CAND;                                                   // [MAXQ]
+  int* cnt = reinterpret_cast<int*>(smem + (size_t)NQT * SIM_QT * QLD * 2);      // [MAXQ]
   float* theta = reinterpret_cast<float*>(cnt + SIM_MAXQ);                    // [MAXQ]
   int* minp = reinterpret_cast<int*>(theta + SIM_MAXQ);                       // [MAXQ]
   uint64_t* qtag = reinterpret_cast<uint64_t*>(minp + SIM_MAXQ);              // [MAXQ]
+  int* need = reinterpret_cast<int*>(qtag + SIM_MAXQ);  // [2] some buffer is full, by rounds in turn: a wave that is a
+                                                        // round ahead must not be taken for this one's
 
   const int nwg = gridDim.x, wg = blockIdx.x;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -134,6 +124,7 @@ __global__ __launch_bounds__(SIM_THREADS) void cosine_stage1_kernel(
     minp[q] = q < Q ? q_minp[q] : 0x7fffffff;
     qtag[q] = q < Q ? q_tags[q] : 0ull;
   }
+  if (threadIdx.x < 2) need[threadIdx.x] = 0;
   __syncthreads();
 
   float* my_s = cand_s + (size_t)wg * SIM_MAXQ * SIM_CAND;
@@ -210,59 +201,53 @@ __global__ __launch_bounds__(SIM_THREADS) void cosine_stage1_kernel(
             my_s[q * SIM_CAND + pos] = sc;
             my_r[q * SIM_CAND + pos] = row;
           }
+          if (pos == SIM_LIM) need[round & 1] = 1;
         }
       }
     }
     __syncthreads();
-    // a buffer must absorb the next round (NW waves x 16 rows)
-    for (int q = 0; q < Q; ++q)
-      if (cnt[q] > SIM_CAND - NW * 16)
-        compact_global(my_s + q * SIM_CAND, my_r + q * SIM_CAND, cs, cr, &cnt[q], &theta[q], K);
+    static_assert(SIM_LIM + NW * 16 <= SIM_CAND, "a buffer must absorb a round");
+    if (need[round & 1]) {
+      __syncthreads();
+      if (threadIdx.x == 0) need[round & 1] = 0;
+      for (int q = wid; q < Q; q += NW)  // (those that would be due soon with them)
+        if (cnt[q] > SIM_MAXK) compact_global(my_s + q * SIM_CAND, my_r + q * SIM_CAND, &cnt[q], &theta[q], K);
+      __syncthreads();
+    }
   }
   __syncthreads();
-  for (int q = 0; q < Q; ++q) {
-    compact_global(my_s + q * SIM_CAND, my_r + q * SIM_CAND, cs, cr, &cnt[q], &theta[q], K);
-    const int n = cnt[q];
-    if (threadIdx.x < K) {
-      const size_t o = ((size_t)q * nwg + wg) * K + threadIdx.x;
-      ws_s[o] = threadIdx.x < n ? cs[threadIdx.x] : -INFINITY;
-      ws_r[o] = threadIdx.x < n ? cr[threadIdx.x] : -1;
-    }
-    __syncthreads();
+  for (int q = wid; q < Q; q += NW) {
+    const size_t o = ((size_t)q * nwg + wg) * K;
+    compact_global(my_s + q * SIM_CAND, my_r + q * SIM_CAND, &cnt[q], &theta[q], K, ws_s + o, ws_r + o);
   }
 }
 
-__global__ __launch_bounds__(SIM_CAND) void cosine_stage2_kernel(float* __restrict__ out_s,
-                                                            int* __restrict__ out_r,
-                                                            const float* __restrict__ ws_s,
-                                                            const int* __restrict__ ws_r,
-                                                            int nwg, int K) {
-  __shared__ float cs[SIM_CAND];
-  __shared__ int cr[SIM_CAND];
-  __shared__ int cnt;
-  __shared__ float theta;
-  const int q = blockIdx.x;
-  if (threadIdx.x == 0) { cnt = 0; theta = -INFINITY; }
-  __syncthreads();
-  const int total = nwg * K;
+// Stage 2: one workgroup per query picks the best K of the slices' lists, PER entries a thread.
+template <int PER>
+__global__ __launch_bounds__(1024) void cosine_stage2_kernel(float* __restrict__ out_s, int* __restrict__ out_r,
+                                                             const float* __restrict__ ws_s, const int* __restrict__ ws_r,
+                                                             int nwg, int K) {
+  __shared__ Selection sel;
+  __shared__ int red[2 * 16];
+  const int q = blockIdx.x, total = nwg * K;
   const float* s = ws_s + (size_t)q * total;
   const int* r = ws_r + (size_t)q * total;
-  for (int base = 0; base < total; base += 64) {
-    if (threadIdx.x < 64) {
-      const int i = base + threadIdx.x;
-      if (i < total && r[i] >= 0 && s[i] > theta) {
-        const int pos = atomicAdd(&cnt, 1);
-        if (pos < SIM_CAND) { cs[pos] = s[i]; cr[pos] = r[i]; }
-      }
-    }
-    __syncthreads();
-    if (cnt > SIM_CAND - 64) compact_query(cs, cr, &cnt, &theta, K);
+  uint32_t key[PER];
+  int row[PER], have = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = i * 1024 + threadIdx.x;
+    row[i] = e < total ? r[e] : -1;
+    key[i] = row[i] >= 0 ? ord_key(s[e]) : 0;
+    have += __popcll(__ballot(row[i] >= 0));
   }
-  compact_query(cs, cr, &cnt, &theta, K);
-  if (threadIdx.x < K) {
-    out_s[(size_t)q * K + threadIdx.x] = threadIdx.x < cnt ? cs[threadIdx.x] : -INFINITY;
-    out_r[(size_t)q * K + threadIdx.x] = threadIdx.x < cnt ? cr[threadIdx.x] : -1;
-  }
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = have;
+  __syncthreads();
+  have = 0;
+#pragma unroll
+  for (int w = 0; w < 16; ++w) have += red[w];
+  const uint32_t kth = have > K ? block_select<PER, 16>(key, K, red) : 1;
+  write_best(key, row, kth, K, sel, out_s + (size_t)q * K, out_r + (size_t)q * K);
 }
 
 }  // namespace pa
@@ -294,7 +279,7 @@ extern "C" int pa_cosine_topk(float* out_scores, int* out_rows, void* workspace,
   float* cand_s = reinterpret_cast<float*>(ws_r + (size_t)Q * nwg * K);
   int* cand_r = reinterpret_cast<int*>(cand_s + (size_t)nwg * pa::SIM_MAXQ * pa::SIM_CAND);
   const int nqt = (Q + pa::SIM_QT - 1) / pa::SIM_QT;
-  const size_t lds = (size_t)nqt * pa::SIM_QT * (D + 8) * 2 + pa::SIM_CAND * 8 + pa::SIM_MAXQ * (4 + 4 + 4 + 8);
+  const size_t lds = (size_t)nqt * pa::SIM_QT * (D + 8) * 2 + pa::SIM_MAXQ * (4 + 4 + 4 + 8) + 16;
   static bool attr_set = false;
   if (!attr_set) {
     (void)hipFuncSetAttribute((const void*)pa::cosine_stage1_kernel,
@@ -304,7 +289,9 @@ extern "C" int pa_cosine_topk(float* out_scores, int* out_rows, void* workspace,
   hipLaunchKernelGGL(pa::cosine_stage1_kernel, dim3(nwg), dim3(pa::SIM_THREADS), lds, st, ws_s, ws_r,
                      cand_s, cand_r, (const pa::bf16*)queries, (const pa::bf16*)index, Q, N, D, K,
                      row_priority, row_tags, row_expiry, q_min_priority, q_tags, now);
-  hipLaunchKernelGGL(pa::cosine_stage2_kernel, dim3(Q), dim3(pa::SIM_CAND), 0, st, out_scores, out_rows,
-                     ws_s, ws_r, nwg, K);
+  static_assert(pa::SIM_MAX_WG * pa::SIM_MAXK <= 16 * 1024, "stage 2 holds all lists");
+  auto* merge = nwg * K <= 1024 ? pa::cosine_stage2_kernel<1>
+                                : nwg * K <= 4096 ? pa::cosine_stage2_kernel<4> : pa::cosine_stage2_kernel<16>;
+  hipLaunchKernelGGL(merge, dim3(Q), dim3(1024), 0, st, out_scores, out_rows, ws_s, ws_r, nwg, K);
   return (int)hipGetLastError();
 }

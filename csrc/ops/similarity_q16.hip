@@ -32,9 +32,7 @@
 // exact scan (EXACT = true: both planes, exact scores in stage 1), so the result is always
 // exact. On random unit vectors at 100M rows the band [tau - 2E, tau] holds a few hundred rows
 // (E ~ 0.008 against a score spread of 1/sqrt(D) = 0.031), far below the lists' 16K entries.
-#include <cstdlib>
-
-#include "common.h"
+#include "topk_select.h"
 
 namespace pa {
 namespace q16 {
@@ -50,7 +48,9 @@ constexpr int MAXQ = 64;
 constexpr int MAXD = 1024;
 constexpr int THREADS = 1024; // 16 waves
 constexpr int NW = THREADS / 64;
-constexpr int MIN_ROWS_PER_WG = 2048;
+// One round of the bound scan (8 waves x 32 rows) a slice at least: 20,000 rows give 79 slices. With 2,048 rows a slice,
+// which the sorting compactions needed, they gave 10 and the pass took 0.5 ms.
+constexpr int MIN_ROWS_PER_WG = 256;
 constexpr int MAX_WG = 256;   // one resident workgroup per CU
 
 __host__ __device__ inline int num_wg(int N) {
@@ -66,28 +66,6 @@ __device__ __forceinline__ float exact_score(int hh, int hl, int lh, int ll, flo
   return (float)((double)I * ((double)sr * (double)sq));
 }
 
-// Bitonic sort of NC entries descending by key, carrying two payloads (whole block, >= NC threads).
-template <int NC = CAND>
-__device__ void bitonic3(float* key, float* p1, int* p2) {
-  for (int k = 2; k <= NC; k <<= 1) {
-    for (int j = k >> 1; j > 0; j >>= 1) {
-      __syncthreads();
-      const int i = threadIdx.x;
-      const int p = i ^ j;
-      if (i < NC && p > i) {
-        const bool desc = (i & k) == 0;
-        const float a = key[i], b = key[p];
-        if (desc ? (a < b) : (a > b)) {
-          key[i] = b; key[p] = a;
-          const float t1 = p1[i]; p1[i] = p1[p]; p1[p] = t1;
-          const int t2 = p2[i]; p2[i] = p2[p]; p2[p] = t2;
-        }
-      }
-    }
-  }
-  __syncthreads();
-}
-
 struct QState {  // per-query admission state of one slice (LDS)
   int cnt[MAXQ];
   float theta[MAXQ];    // admission threshold = max(cap, tauL)
@@ -100,64 +78,78 @@ struct QState {  // per-query admission state of one slice (LDS)
   float cq[MAXQ];
 };
 
-// Compact query q's global buffer (NC entries) to its best C upper bounds; refresh cap / tauL /
-// theta.
-template <int NC = CAND>
-__device__ void compact(float* gu, float* gl, int* gr, float* su, float* sl, int* sr, QState& st, int q, int K) {
-  const int n = min(st.cnt[q], NC);
-  if (threadIdx.x < NC) {
-    const bool ok = threadIdx.x < n;
-    su[threadIdx.x] = ok ? gu[threadIdx.x] : -INFINITY;
-    sl[threadIdx.x] = ok ? gl[threadIdx.x] : -INFINITY;
-    sr[threadIdx.x] = ok ? gr[threadIdx.x] : -1;
+// Compact query q's global buffer to its best C upper bounds and refresh cap / tauL / theta: one wave a query, so a
+// workgroup's waves compact as many queries at once, with no barrier. Selecting by bits takes about a microsecond a
+// query; a bitonic sort by the whole workgroup took 15, one query after the other (3 of the 4 ms of a pass over 4M rows).
+// ou / ol / orow: where the slice's list goes, or null to keep it in the buffer.
+__device__ __forceinline__ void compact(float* gu, float* gl, int* gr, QState& st, int q, int K, float* ou = nullptr,
+                                        float* ol = nullptr, int* orow = nullptr) {
+  constexpr int PER = CAND / 64;
+  const int lane = threadIdx.x & 63, n = min(st.cnt[q], CAND);
+  uint32_t ku[PER], kl[PER];
+  int rows[PER];
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = i * 64 + lane;
+    const bool ok = e < n;
+    ku[i] = ok ? ord_key(gu[e]) : 0;
+    kl[i] = ok ? ord_key(gl[e]) : 0;
+    rows[i] = ok ? gr[e] : -1;
   }
-  bitonic3<NC>(su, sl, sr);  // begins and ends with a barrier
-  const int keep = min(n, C);
-  if (threadIdx.x < keep) {
-    gu[threadIdx.x] = su[threadIdx.x];
-    gl[threadIdx.x] = sl[threadIdx.x];
-    gr[threadIdx.x] = sr[threadIdx.x];
-    if (keep >= K) {  // rank of this entry's L among the kept ones (ties by position)
-      const float me = sl[threadIdx.x];
-      int rank = 0;
-      for (int j = 0; j < keep; ++j) {
-        const float o = sl[j];
-        rank += (o > me) || (o == me && j < (int)threadIdx.x);
-      }
-      if (rank == K - 1) st.tauL[q] = fmaxf(st.tauL[q], me);  // any subset's K-th best is a valid bound
+  uint32_t cut = 1;  // entries above it stay, and of those at it as many as there is room for
+  int room = C;
+  if (n >= C) {
+    cut = wave_select(ku, C);
+#pragma unroll
+    for (int i = 0; i < PER; ++i) room -= __popcll(__ballot(ku[i] > cut));
+  }
+  if (ou) { gu = ou; gl = ol; gr = orow; }
+  int at = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const unsigned long long ties = __ballot(ku[i] == cut);
+    const bool keep = ku[i] > cut || (ku[i] == cut && rank_in(ties) < room);
+    room -= __popcll(ties);
+    const unsigned long long kept = __ballot(keep);
+    if (keep) {
+      const int p = at + rank_in(kept);
+      gu[p] = key_value(ku[i]);
+      gl[p] = key_value(kl[i]);
+      gr[p] = rows[i];
+    } else {
+      kl[i] = 0;
     }
+    at += __popcll(kept);
   }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    st.cnt[q] = keep;
+  if (ou && lane >= at) { gu[lane] = -INFINITY; gl[lane] = -INFINITY; gr[lane] = -1; }
+  uint32_t kth = 0;
+  if (at >= K) kth = wave_select(kl, K);  // any subset's K-th best L is a valid bound
+  if (lane == 0) {
+    st.cnt[q] = at;
     if (n > C) st.dropped[q] = 1;
-    if (keep == C) st.cap[q] = su[C - 1];
+    if (at == C) st.cap[q] = key_value(cut);
+    if (at >= K) st.tauL[q] = fmaxf(st.tauL[q], key_value(kth));
     st.theta[q] = fmaxf(st.cap[q], st.tauL[q]);
   }
-  __syncthreads();
 }
 
-// Stage 1. EXACT: both planes, U = L = the exact score (the fallback / reference scan).
-template <bool EXACT>
-__global__ __launch_bounds__(EXACT ? 512 : 1024) void stage1_kernel(
+// Stage 1 over both planes, U = L = the exact score (the fallback scan): 8 waves, four accumulators per query tile.
+__global__ __launch_bounds__(512) void stage1_exact_kernel(
     float* __restrict__ out_u, float* __restrict__ out_l, int* __restrict__ out_r, float* __restrict__ out_drop,
     float* __restrict__ cand_u, float* __restrict__ cand_l, int* __restrict__ cand_r,
     const signed char* __restrict__ qv, const float* __restrict__ qmeta, const signed char* __restrict__ hi,
     const signed char* __restrict__ lo, const float* __restrict__ rmeta, int Q, int N, int D, int K,
     const int* __restrict__ row_prio, const uint64_t* __restrict__ row_tags, const float* __restrict__ row_exp,
     const int* __restrict__ q_minp, const uint64_t* __restrict__ q_tags, float now) {
-  // the exact scan holds four accumulators per query tile: 8 waves, 256 registers each
-  constexpr int TH = EXACT ? 512 : 1024, NWV = TH / 64;
-  constexpr int KB = EXACT ? 2 : 4;  // k-steps per load batch (16 B per lane per plane and step)
+  constexpr int TH = 512, NWV = TH / 64;
+  constexpr int KB = 2;  // k-steps per load batch (16 B per lane per plane and step)
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int NQT = (Q + QT - 1) / QT;
   const int QLD = D + 16;  // padded LDS row (bytes): the 16 query rows of a fragment spread over the banks
   signed char* qh = reinterpret_cast<signed char*>(smem);           // [NQT*16][QLD]
   signed char* ql = qh + (size_t)NQT * QT * QLD;                    // [NQT*16][QLD]
-  float* su = reinterpret_cast<float*>(ql + (size_t)NQT * QT * QLD);
-  float* sl = su + CAND;
-  int* sr = reinterpret_cast<int*>(sl + CAND);
-  QState& st = *reinterpret_cast<QState*>(sr + CAND);
+  QState& st = *reinterpret_cast<QState*>(ql + (size_t)NQT * QT * QLD);
+  int* need = reinterpret_cast<int*>(&st + 1);  // as in the bound scan
 
   const int nwg = gridDim.x, wg = blockIdx.x;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -183,6 +175,7 @@ __global__ __launch_bounds__(EXACT ? 512 : 1024) void stage1_kernel(
     st.sq[q] = q < Q ? qmeta[2 * q] : 0.f;
     st.cq[q] = q < Q ? qmeta[2 * q + 1] : 0.f;
   }
+  if (threadIdx.x < 2) need[threadIdx.x] = 0;
   __syncthreads();
 
   float* my_u = cand_u + (size_t)wg * MAXQ * CAND;
@@ -206,7 +199,7 @@ __global__ __launch_bounds__(EXACT ? 512 : 1024) void stage1_kernel(
   i32x4 hA[KB], hB[KB], lA[KB], lB[KB];
   if (wid < ngroups) {
     load(hi, wid, 0, hA);
-    if (EXACT) load(lo, wid, 0, lA);
+    load(lo, wid, 0, lA);
   }
 
   for (int round = 0; round < nrounds; ++round) {
@@ -239,10 +232,8 @@ __global__ __launch_bounds__(EXACT ? 512 : 1024) void stage1_kernel(
               const i32x4 bl = *reinterpret_cast<const i32x4*>(ql + qo);
               acc_hh[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ah[u], bh, acc_hh[t], 0, 0, 0);
               acc_lh[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(ah[u], bl, acc_lh[t], 0, 0, 0);
-              if (EXACT) {
-                acc_hl[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[u], bh, acc_hl[t], 0, 0, 0);
-                acc_ll[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[u], bl, acc_ll[t], 0, 0, 0);
-              }
+              acc_hl[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[u], bh, acc_hl[t], 0, 0, 0);
+              acc_ll[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(al[u], bl, acc_ll[t], 0, 0, 0);
             }
           }
         }
@@ -250,15 +241,15 @@ __global__ __launch_bounds__(EXACT ? 512 : 1024) void stage1_kernel(
       for (int m = 0; m < DS; m += 2 * KB) {
         if (m + KB < DS) {
           load(hi, grp, m + KB, hB);
-          if (EXACT) load(lo, grp, m + KB, lB);
+          load(lo, grp, m + KB, lB);
         }
         compute(hA, lA, m);
         if (m + 2 * KB < DS) {
           load(hi, grp, m + 2 * KB, hA);
-          if (EXACT) load(lo, grp, m + 2 * KB, lA);
+          load(lo, grp, m + 2 * KB, lA);
         } else if (grp + NWV < ngroups) {  // the next group's first batch stays in flight
           load(hi, grp + NWV, 0, hA);
-          if (EXACT) load(lo, grp + NWV, 0, lA);
+          load(lo, grp + NWV, 0, lA);
         }
         if (m + KB < DS) compute(hB, lB, m + KB);
       }
@@ -272,15 +263,7 @@ __global__ __launch_bounds__(EXACT ? 512 : 1024) void stage1_kernel(
         for (int t = 0; t < MAXQ / QT; ++t) {
           const int q = t * QT + col;
           if (t >= NQT || q >= Q) continue;
-          float U, L;
-          if (EXACT) {
-            U = L = exact_score(acc_hh[t][r], acc_hl[t][r], acc_lh[t][r], acc_ll[t][r], rm.x, st.sq[q]);
-          } else {
-            const float s = ((float)acc_hh[t][r] * 65536.f + (float)acc_lh[t][r] * 256.f) * (rm.x * st.sq[q]);
-            const float e = rm.y * st.cq[q] * 1.0001f + 1e-6f;  // margin: fp32 rounding of s and e
-            U = s + e;
-            L = s - e;
-          }
+          const float U = exact_score(acc_hh[t][r], acc_hl[t][r], acc_lh[t][r], acc_ll[t][r], rm.x, st.sq[q]);
           if (!(U > st.theta[q])) {
             if (U > st.tauL[q]) st.dropped[q] = 1;  // refused for capacity, not by the k-th bound
             continue;
@@ -292,35 +275,30 @@ __global__ __launch_bounds__(EXACT ? 512 : 1024) void stage1_kernel(
           const int pos = atomicAdd(&st.cnt[q], 1);
           if (pos < CAND) {
             my_u[q * CAND + pos] = U;
-            my_l[q * CAND + pos] = L;
+            my_l[q * CAND + pos] = U;
             my_r[q * CAND + pos] = row;
           }
+          if (pos == CAND - NWV * 16) need[round & 1] = 1;  // a buffer must absorb a round
         }
       }
     }
     __syncthreads();
-    for (int q = 0; q < Q; ++q)  // a buffer must absorb the next round (NWV waves x 16 rows)
-      if (st.cnt[q] > CAND - NWV * 16)
-        compact(my_u + q * CAND, my_l + q * CAND, my_r + q * CAND, su, sl, sr, st, q, K);
-  }
-  __syncthreads();
-  for (int q = 0; q < Q; ++q) {
-    compact(my_u + q * CAND, my_l + q * CAND, my_r + q * CAND, su, sl, sr, st, q, K);
-    const int n = st.cnt[q];
-    if (threadIdx.x < C) {
-      const size_t o = ((size_t)q * nwg + wg) * C + threadIdx.x;
-      const bool ok = (int)threadIdx.x < n;
-      out_u[o] = ok ? su[threadIdx.x] : -INFINITY;
-      out_l[o] = ok ? sl[threadIdx.x] : -INFINITY;
-      out_r[o] = ok ? sr[threadIdx.x] : -1;
+    if (need[round & 1]) {
+      __syncthreads();
+      if (threadIdx.x == 0) need[round & 1] = 0;
+      for (int q = wid; q < Q; q += NWV)
+        if (st.cnt[q] > C) compact(my_u + q * CAND, my_l + q * CAND, my_r + q * CAND, st, q, K);
     }
-    if (threadIdx.x == 0) out_drop[(size_t)q * nwg + wg] = st.dropped[q] ? st.cap[q] : -INFINITY;
     __syncthreads();
+  }
+  for (int q = wid; q < Q; q += NWV) {
+    const size_t o = ((size_t)q * nwg + wg) * C;
+    compact(my_u + q * CAND, my_l + q * CAND, my_r + q * CAND, st, q, K, out_u + o, out_l + o, out_r + o);
+    if (lane == 0) out_drop[(size_t)q * nwg + wg] = st.dropped[q] ? st.cap[q] : -INFINITY;
   }
 }
 
-// Stage 1, the bound scan as run (stage1_kernel<false> is the first form, kept as variant 0 for
-// A/B; profiles/r6_q16_stage1.md). 8 waves, two per SIMD (the 32x32 accumulators of 64 queries
+// Stage 1, the bound scan (profiles/r6_q16_stage1.md). 8 waves, two per SIMD (the 32x32 accumulators of 64 queries
 // and two 4-k-step batches need ~170 registers); a wave owns 32-row groups and runs
 // v_mfma_i32_32x32x32_i8 (rows x 32 queries): per byte of index it reads half the LDS query
 // fragments of the 16x16x64 form (4 KiB per KiB of rows instead of 8) at the same MFMA cycles.
@@ -334,8 +312,10 @@ __global__ __launch_bounds__(EXACT ? 512 : 1024) void stage1_kernel(
 // for LDS only -- a branchy load block, a fenced __syncthreads or loads left to the scheduler
 // each made the wait-count pass drain the row loads in flight (the first form: 3.2 TB/s).
 // Candidate stores are made visible by a full barrier only before a compaction.
-constexpr int CAND_B = CAND;  // per-(slice, query) candidate buffer: a round admits up to 8 x 32 rows
-template <int DSC, int ABL = 0>  // ABL (timing ablations, tools/q16_ablate): 1 = no epilogue, 2 = loads only
+// A buffer holds LIM entries between rounds and 8 x 32 more that a round may admit. Compacting early (two lists' worth)
+// keeps the thresholds tight, and so the admissions few, now that a compaction costs a microsecond.
+constexpr int LIM = 2 * C;
+template <int DSC>
 __global__ __launch_bounds__(512) void stage1_bound_kernel(
     float* __restrict__ out_u, float* __restrict__ out_l, int* __restrict__ out_r, float* __restrict__ out_drop,
     float* __restrict__ cand_u, float* __restrict__ cand_l, int* __restrict__ cand_r,
@@ -350,11 +330,10 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
   extern __shared__ __attribute__((aligned(16))) char smem[];
   signed char* qh = reinterpret_cast<signed char*>(smem);  // [64][QLD]
   signed char* ql = qh + (size_t)MAXQ * QLD;                // [64][QLD]
-  float* su = reinterpret_cast<float*>(ql + (size_t)MAXQ * QLD);
-  float* sl = su + CAND_B;
-  int* sr = reinterpret_cast<int*>(sl + CAND_B);
-  QState& st = *reinterpret_cast<QState*>(sr + CAND_B);
-  int* need = reinterpret_cast<int*>(&st + 1);  // some query's buffer must be compacted
+  QState& st = *reinterpret_cast<QState*>(ql + (size_t)MAXQ * QLD);
+  // [2] some query's buffer must be compacted, by rounds in turn: a wave that is a round ahead must not be taken for this
+  // one's (the others would miss its barrier)
+  int* need = reinterpret_cast<int*>(&st + 1);
   // [NWV][32] per group row: (s_r, b_r), then the filter words (priority, expiry, tags)
   float2* rm_lds = reinterpret_cast<float2*>(need + 4);
   int* pr_lds = reinterpret_cast<int*>(rm_lds + NWV * 32);
@@ -384,19 +363,19 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
     st.sq[q] = q < Q ? qmeta[2 * q] : 0.f;
     st.cq[q] = q < Q ? qmeta[2 * q + 1] : 0.f;
   }
-  if (threadIdx.x == 0) *need = 0;
+  if (threadIdx.x < 2) need[threadIdx.x] = 0;
   __syncthreads();
 
-  float* my_u = cand_u + (size_t)wg * MAXQ * CAND_B;
-  float* my_l = cand_l + (size_t)wg * MAXQ * CAND_B;
-  int* my_r = cand_r + (size_t)wg * MAXQ * CAND_B;
+  float* my_u = cand_u + (size_t)wg * MAXQ * CAND;
+  float* my_l = cand_l + (size_t)wg * MAXQ * CAND;
+  int* my_r = cand_r + (size_t)wg * MAXQ * CAND;
   const int per = ((N + nwg - 1) / nwg + 31) / 32 * 32;
   const int r0 = wg * per, r1 = min(N, r0 + per);
   const int ngroups = (max(0, r1 - r0) + 31) / 32;
   if (ngroups > 0) {  // workgroup-uniform
     const int nrounds = (ngroups + NWV - 1) / NWV;
     const int last_tile = (r1 - 1) >> 4;
-    const int CUT = CAND_B - NWV * 32;  // a buffer must absorb the next round
+    static_assert(LIM + NWV * 32 <= CAND, "a buffer must absorb a round");
     // this lane's two 16-B A pieces (k-halves) of k-step m + u, group grp_
     auto load = [&](int grp_, int m, i32x4 (&dst)[KB][2]) {
       const int tile = min((r0 >> 4) + 2 * min(grp_, ngroups - 1) + (lr >> 4), last_tile);
@@ -439,12 +418,8 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
               const int qo = (32 * t + lr) * QLD + 64 * (m + u) + 32 * kh + 16 * lh;
               const i32x4 bh = *reinterpret_cast<const i32x4*>(qh + qo);
               const i32x4 bl = *reinterpret_cast<const i32x4*>(ql + qo);
-              if constexpr (ABL == 2) {
-                acc_hh[t][0] ^= ah[u][kh][0] ^ ah[u][kh][1] ^ ah[u][kh][2] ^ ah[u][kh][3];
-              } else {
-                acc_hh[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[u][kh], bh, acc_hh[t], 0, 0, 0);
-                acc_lh[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[u][kh], bl, acc_lh[t], 0, 0, 0);
-              }
+              acc_hh[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[u][kh], bh, acc_hh[t], 0, 0, 0);
+              acc_lh[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[u][kh], bl, acc_lh[t], 0, 0, 0);
             }
       };
       // sched_barrier pins each batch's loads where they are issued: left to the scheduler they
@@ -467,14 +442,7 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
         __builtin_amdgcn_sched_barrier(0);
         compute(Y, m + KB);
       }
-      if constexpr (ABL != 0) {
-        int x = 0;
-#pragma unroll
-        for (int t = 0; t < NTQ; ++t)
-#pragma unroll
-          for (int j = 0; j < 16; ++j) x ^= acc_hh[t][j] ^ acc_lh[t][j];
-        if (x == 0x7fffffff && rmine.x == 12345.f) my_u[0] = 1.f;  // keeps the work alive
-      } else if (grp < ngroups) {
+      if (grp < ngroups) {
         // lane holds queries 32 t + lr, rows gbase + (j & 3) + 8 (j >> 2) + 4 lh (j = 0..15).
         // Fast path, branch-free: every (row, query) bound against its query's admission threshold
         // theta (-> adm) and k-th lower bound tauL (tauL < U <= theta: refused for capacity ->
@@ -531,12 +499,12 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
               const float ex = ex_lds[wid * 32 + ri];
               if (ex != 0.f && !(ex > now)) continue;
               const int pos = atomicAdd(&st.cnt[q], 1);
-              if (pos < CAND_B) {
-                my_u[q * CAND_B + pos] = sc + e;
-                my_l[q * CAND_B + pos] = sc - e;
-                my_r[q * CAND_B + pos] = gbase + ri;
+              if (pos < CAND) {
+                my_u[q * CAND + pos] = sc + e;
+                my_l[q * CAND + pos] = sc - e;
+                my_r[q * CAND + pos] = gbase + ri;
               }
-              if (pos == CUT) *need = 1;
+              if (pos == LIM) need[round & 1] = 1;
             }
           }
         }
@@ -545,12 +513,11 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      if (*need) {  // workgroup-uniform; rare after the first rounds
+      if (need[round & 1]) {  // workgroup-uniform; rare after the first rounds
         __syncthreads();  // candidate stores complete and visible
-        for (int q = 0; q < Q; ++q)
-          if (st.cnt[q] > CUT)
-            compact<CAND_B>(my_u + q * CAND_B, my_l + q * CAND_B, my_r + q * CAND_B, su, sl, sr, st, q, K);
-        if (threadIdx.x == 0) *need = 0;
+        if (threadIdx.x == 0) need[round & 1] = 0;
+        for (int q = wid; q < Q; q += NWV)  // (those that would be due soon with them)
+          if (st.cnt[q] > C + C / 2) compact(my_u + q * CAND, my_l + q * CAND, my_r + q * CAND, st, q, K);
         __syncthreads();
       }
     };
@@ -559,44 +526,15 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
     for (int round = 0; round < nrounds; ++round) body(round, bA, bB);
   }
   __syncthreads();
-  for (int q = 0; q < Q; ++q) {
-    compact<CAND_B>(my_u + q * CAND_B, my_l + q * CAND_B, my_r + q * CAND_B, su, sl, sr, st, q, K);
-    const int n = st.cnt[q];
-    if (threadIdx.x < C) {
-      const size_t o = ((size_t)q * nwg + wg) * C + threadIdx.x;
-      const bool ok = (int)threadIdx.x < n;
-      out_u[o] = ok ? su[threadIdx.x] : -INFINITY;
-      out_l[o] = ok ? sl[threadIdx.x] : -INFINITY;
-      out_r[o] = ok ? sr[threadIdx.x] : -1;
-    }
-    if (threadIdx.x == 0) out_drop[(size_t)q * nwg + wg] = st.dropped[q] ? st.cap[q] : -INFINITY;
-    __syncthreads();
+  for (int q = wid; q < Q; q += NWV) {
+    const size_t o = ((size_t)q * nwg + wg) * C;
+    compact(my_u + q * CAND, my_l + q * CAND, my_r + q * CAND, st, q, K, out_u + o, out_l + o, out_r + o);
+    if (lane == 0) out_drop[(size_t)q * nwg + wg] = st.dropped[q] ? st.cap[q] : -INFINITY;
   }
 }
 
-// Insert (key, row) into the block's top-k buffer under its threshold (one thread per call).
-__device__ __forceinline__ void offer(float* bs, int* br, int* cnt, const float* theta, float key, int row) {
-  if (key > *theta) {
-    const int pos = atomicAdd(cnt, 1);
-    if (pos < CAND) { bs[pos] = key; br[pos] = row; }
-  }
-}
-
-// Sort the block buffer, keep the best K, raise the threshold (whole block).
-__device__ void keep_best(float* bs, int* br, float* dummy, int* cnt, float* theta, int K) {
-  const int n = min(*cnt, CAND);
-  if (threadIdx.x < CAND && (int)threadIdx.x >= n) { bs[threadIdx.x] = -INFINITY; br[threadIdx.x] = -1; }
-  if (threadIdx.x < CAND) dummy[threadIdx.x] = 0.f;
-  bitonic3(bs, dummy, br);
-  if (threadIdx.x == 0) {
-    const int keep = min(n, K);
-    *cnt = keep;
-    if (keep == K) *theta = bs[K - 1];
-  }
-  __syncthreads();
-}
-
-// Stage 2: one workgroup per query (see the header). EXACT: the lists hold exact scores.
+// Stage 2: one workgroup per query (see the header), 16 list entries a thread in registers. EXACT: the lists hold exact
+// scores. Both selections go by bits (topk_select.h); with sorted buffers the launch took 130 us for 16,384 entries.
 template <bool EXACT>
 __global__ __launch_bounds__(THREADS) void stage2_kernel(
     float* __restrict__ out_s, int* __restrict__ out_rows, int* __restrict__ unsafe,
@@ -604,90 +542,113 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
     const float* __restrict__ ldrop, int nwg, const signed char* __restrict__ qv,
     const float* __restrict__ qmeta, const signed char* __restrict__ hi, const signed char* __restrict__ lo,
     const float* __restrict__ rmeta, int D, int K) {
-  __shared__ float bs[CAND];
-  __shared__ int br[CAND];
-  __shared__ float dummy[CAND];
-  __shared__ int cnt;
-  __shared__ float theta;
-  __shared__ float red[NW];
-  __shared__ __attribute__((aligned(16))) signed char q_lds[2 * MAXD];
-  constexpr int CL = 4096;  // list entries scanned per chunk (all of them may qualify)
+  constexpr int PER = MAX_WG * C / THREADS;  // entries a thread
+  constexpr int CL = 8 * THREADS;            // re-ranked entries at a time
+  constexpr int RR = CL / THREADS + 1;
+  __shared__ int red[2 * NW];
+  __shared__ Selection sel;
+  __shared__ int crow[EXACT ? 1 : CL + MAXK];
+  __shared__ uint32_t ckey[EXACT ? 1 : CL + MAXK];
+  __shared__ float best_s[MAXK];
+  __shared__ int best_r[MAXK];
   __shared__ int ncand;
-  __shared__ int clist[CL];
   const int q = blockIdx.x;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int total = nwg * C;
   const float* u = lu + (size_t)q * total;
   const float* l = ll + (size_t)q * total;
   const int* r = lr + (size_t)q * total;
-  if (threadIdx.x == 0) { cnt = 0; theta = -INFINITY; }
-  for (int i = threadIdx.x; i < 2 * D / 16; i += THREADS)
-    *reinterpret_cast<i32x4*>(q_lds + 16 * i) = *reinterpret_cast<const i32x4*>(qv + (size_t)q * 2 * D + 16 * i);
-  __syncthreads();
-  // ---- A: tau = the K-th best lower bound over every slice's list (256 offers per round:
-  // the buffer keeps room for a round on top of the K it holds after a compaction)
-  constexpr int OFR = 256;
-  for (int base = 0; base < total; base += OFR) {
-    const int i = base + threadIdx.x;
-    if (threadIdx.x < OFR && i < total && r[i] >= 0) offer(bs, br, &cnt, &theta, l[i], r[i]);
-    __syncthreads();
-    if (cnt > CAND - OFR) keep_best(bs, br, dummy, &cnt, &theta, K);
+  float* os = out_s + (size_t)q * K;
+  int* orow = out_rows + (size_t)q * K;
+  // ---- A: tau = the K-th best lower bound over every slice's list (no bound with fewer than K entries)
+  uint32_t key[PER];
+  int row[PER], have = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = i * THREADS + threadIdx.x;
+    row[i] = e < total ? r[e] : -1;
+    key[i] = row[i] >= 0 ? ord_key(l[e]) : 0;
+    have += __popcll(__ballot(row[i] >= 0));
   }
-  keep_best(bs, br, dummy, &cnt, &theta, K);
-  const float tau = cnt == K ? theta : -INFINITY;
+  if (lane == 0) red[wid] = have;
+  __syncthreads();
+  have = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) have += red[w];
+  const uint32_t tau = have >= K ? block_select<PER, NW>(key, K, red) : 1;
   // ---- B: a slice that refused a row for capacity at a level >= tau may have lost a top-k row
-  float dmax = -INFINITY;
-  for (int i = threadIdx.x; i < nwg; i += THREADS) dmax = fmaxf(dmax, ldrop[(size_t)q * nwg + i]);
-  dmax = wave_max(dmax);
-  if (lane == 0) red[wid] = dmax;
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    float m = -INFINITY;
-    for (int w = 0; w < NW; ++w) m = fmaxf(m, red[w]);
-    unsafe[q] = (!EXACT && m > -INFINITY && m >= tau) ? 1 : 0;
-  }
-  if (EXACT) {  // the lists hold exact scores: A's buffer is the answer
-    if (threadIdx.x < K) {
-      out_s[(size_t)q * K + threadIdx.x] = (int)threadIdx.x < cnt ? bs[threadIdx.x] : -INFINITY;
-      out_rows[(size_t)q * K + threadIdx.x] = (int)threadIdx.x < cnt ? br[threadIdx.x] : -1;
-    }
+  if (EXACT) {  // the lists hold exact scores
+    if (threadIdx.x == 0) unsafe[q] = 0;
+    write_best(key, row, tau, K, sel, os, orow);
     return;
   }
+  uint32_t none = ord_key(-INFINITY), drop = none;
+  for (int i = threadIdx.x; i < nwg; i += THREADS) drop = max(drop, ord_key(ldrop[(size_t)q * nwg + i]));
+  const bool lost = __syncthreads_or(drop > none && drop >= tau);
+  if (threadIdx.x == 0) unsafe[q] = lost;
   // ---- C: re-rank every listed row whose upper bound reaches tau, exactly
+  int cand = 0;
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int e = i * THREADS + threadIdx.x;
+    if (row[i] >= 0 && ord_key(u[e]) < tau) row[i] = -1;
+    cand += __popcll(__ballot(row[i] >= 0));
+  }
+  if (lane == 0) red[wid] = cand;
+  if (threadIdx.x == 0) ncand = 0;
   __syncthreads();
-  if (threadIdx.x == 0) { cnt = 0; theta = -INFINITY; ncand = 0; }
-  __syncthreads();
+  cand = 0;
+#pragma unroll
+  for (int w = 0; w < NW; ++w) cand += red[w];
   const float sq = qmeta[2 * q];
   const int DS = D / 64;
-  for (int base = 0; base < total; base += CL) {
-    // the chunk's listed rows whose upper bound reaches tau -> LDS
-    for (int i = base + threadIdx.x; i < min(total, base + CL); i += THREADS)
-      if (r[i] >= 0 && u[i] >= tau) {
-        const int pos = atomicAdd(&ncand, 1);
-        clist[pos] = r[i];
-      }
-    __syncthreads();
-    const int nc = ncand;
-    for (int j0 = 0; j0 < nc; j0 += NW) {  // one row per wave and round
-      const int j = j0 + wid;
-      if (j < nc) {
-        const int row = clist[j];
-        const int t = row >> 4, c = row & 15;
-        int hh = 0, hl = 0, lh = 0, lls = 0;
-        for (int p = lane; p < DS * 4; p += 64) {  // (k-step, lane group) pieces of 16 dims
-          const int s = p >> 2, gg = p & 3;
-          const size_t off = (((size_t)t * DS + s) * 64 + 16 * gg + c) * 16;
-          const i8x16 a = *reinterpret_cast<const i8x16*>(hi + off);
-          const i8x16 b = *reinterpret_cast<const i8x16*>(lo + off);
-          const i8x16 qa = *reinterpret_cast<const i8x16*>(q_lds + 64 * s + 16 * gg);
-          const i8x16 qb = *reinterpret_cast<const i8x16*>(q_lds + D + 64 * s + 16 * gg);
+  // a lane holds 16 dimensions of a row: k-step lane / 4, lane group lane % 4 of it (D <= 1024)
+  const bool on = lane < DS * 4;
+  i32x4 qa = i32x4{0, 0, 0, 0}, qb = qa;
+  if (on) {
+    const signed char* qp = qv + (size_t)q * 2 * D + 16 * lane;
+    qa = *reinterpret_cast<const i32x4*>(qp);
+    qb = *reinterpret_cast<const i32x4*>(qp + D);
+  }
+  int kept = 0;  // best entries so far, ahead of the next ones in crow / ckey
+  const int step = cand <= CL ? PER : CL / THREADS;
+#pragma unroll 1
+  for (int part = 0; part < PER; part += step) {
 #pragma unroll
-          for (int e = 0; e < 16; ++e) {
-            hh += (int)qa[e] * (int)a[e];
-            hl += (int)qa[e] * (int)b[e];
-            lh += (int)qb[e] * (int)a[e];
-            lls += (int)qb[e] * (int)b[e];
-          }
+    for (int i = 0; i < PER; ++i) {
+      if (i < part || i >= part + step) continue;
+      const unsigned long long m = __ballot(row[i] >= 0);
+      int at = 0;
+      if (lane == 0 && m) at = atomicAdd(&ncand, (int)__popcll(m));
+      at = __shfl(at, 0, 64) + kept + rank_in(m);
+      if (row[i] >= 0) crow[at] = row[i];
+    }
+    __syncthreads();
+    const int n = kept + ncand;
+    constexpr int RB = 4;  // rows a wave reads at once: the launch is a chain of such reads
+    for (int j0 = kept + wid * RB; j0 < n; j0 += NW * RB) {
+      i32x4 a[RB], b[RB];
+      int rw[RB];
+#pragma unroll
+      for (int k = 0; k < RB; ++k) {
+        rw[k] = crow[min(j0 + k, n - 1)];
+        if (on) {
+          const size_t off = (((size_t)(rw[k] >> 4) * DS + (lane >> 2)) * 64 + 16 * (lane & 3) + (rw[k] & 15)) * 16;
+          a[k] = *reinterpret_cast<const i32x4*>(hi + off);
+          b[k] = *reinterpret_cast<const i32x4*>(lo + off);
+        } else {
+          a[k] = b[k] = i32x4{0, 0, 0, 0};
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < RB; ++k) {
+        int hh = 0, hl = 0, lh = 0, lls = 0;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          hh = __builtin_amdgcn_sdot4(qa[e], a[k][e], hh, false);
+          hl = __builtin_amdgcn_sdot4(qa[e], b[k][e], hl, false);
+          lh = __builtin_amdgcn_sdot4(qb[e], a[k][e], lh, false);
+          lls = __builtin_amdgcn_sdot4(qb[e], b[k][e], lls, false);
         }
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) {
@@ -696,19 +657,31 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
           lh += __shfl_xor(lh, o, 64);
           lls += __shfl_xor(lls, o, 64);
         }
-        if (lane == 0) offer(bs, br, &cnt, &theta, exact_score(hh, hl, lh, lls, rmeta[2 * (size_t)row], sq), row);
+        if (lane == 0 && j0 + k < n) ckey[j0 + k] = ord_key(exact_score(hh, hl, lh, lls, rmeta[2 * (size_t)rw[k]], sq));
       }
-      __syncthreads();
-      if (cnt > CAND - NW) keep_best(bs, br, dummy, &cnt, &theta, K);
     }
     __syncthreads();
-    if (threadIdx.x == 0) ncand = 0;
-    __syncthreads();
-  }
-  keep_best(bs, br, dummy, &cnt, &theta, K);
-  if (threadIdx.x < K) {
-    out_s[(size_t)q * K + threadIdx.x] = (int)threadIdx.x < cnt ? bs[threadIdx.x] : -INFINITY;
-    out_rows[(size_t)q * K + threadIdx.x] = (int)threadIdx.x < cnt ? br[threadIdx.x] : -1;
+    uint32_t ck[RR];
+    int cr[RR];
+#pragma unroll
+    for (int i = 0; i < RR; ++i) {
+      const int e = i * THREADS + threadIdx.x;
+      ck[i] = e < n ? ckey[e] : 0;
+      cr[i] = e < n ? crow[e] : -1;
+    }
+    const uint32_t kth = n > K ? block_select<RR, NW>(ck, K, red) : 1;
+    const bool last = part + step >= PER;
+    write_best(ck, cr, kth, K, sel, last ? os : best_s, last ? orow : best_r);
+    if (!last) {
+      __syncthreads();
+      kept = min(n, K);
+      if (threadIdx.x < kept) {
+        ckey[threadIdx.x] = ord_key(best_s[threadIdx.x]);
+        crow[threadIdx.x] = best_r[threadIdx.x];
+      }
+      if (threadIdx.x == 0) ncand = 0;
+      __syncthreads();
+    }
   }
 }
 
@@ -719,7 +692,7 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
 // candidate buffers [3][nwg][64][CAND]
 extern "C" long long pa_q16_topk_workspace_bytes(int Q, int N) {
   const long long w = pa::q16::num_wg(N);
-  return 3LL * Q * w * pa::q16::C * 4 + (long long)Q * w * 4 + 3LL * w * pa::q16::MAXQ * pa::q16::CAND_B * 4;
+  return 3LL * Q * w * pa::q16::C * 4 + (long long)Q * w * 4 + 3LL * w * pa::q16::MAXQ * pa::q16::CAND * 4;
 }
 
 // queries_q: [Q][2][D] int8 (qh, ql); qmeta [Q][2] (s_q, c_q); hi / lo: [N/16][D/64][64][16]
@@ -744,52 +717,32 @@ extern "C" int pa_q16_topk(float* out_scores, int* out_rows, int* unsafe, void* 
   int* lr = reinterpret_cast<int*>(ll + (size_t)Q * nwg * C);
   float* ldrop = reinterpret_cast<float*>(lr + (size_t)Q * nwg * C);
   float* cu = ldrop + (size_t)Q * nwg;
-  // candidate buffers laid out for the bound kernel's CAND_B (the first form / the exact scan
-  // use the first CAND entries of each)
-  float* cl = cu + (size_t)nwg * MAXQ * CAND_B;
-  int* cr = reinterpret_cast<int*>(cl + (size_t)nwg * MAXQ * CAND_B);
+  float* cl = cu + (size_t)nwg * MAXQ * CAND;
+  int* cr = reinterpret_cast<int*>(cl + (size_t)nwg * MAXQ * CAND);
   const int nqt = (Q + QT - 1) / QT;
-  const size_t lds = (size_t)nqt * QT * (D + 16) * 2 + CAND * 12 + sizeof(QState);
+  const size_t lds = (size_t)nqt * QT * (D + 16) * 2 + sizeof(QState) + 16;
   static bool attr_set = false;
   if (!attr_set) {
     (void)hipFuncSetAttribute((const void*)stage1_bound_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     (void)hipFuncSetAttribute((const void*)stage1_bound_kernel<8>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     (void)hipFuncSetAttribute((const void*)stage1_bound_kernel<16>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    (void)hipFuncSetAttribute((const void*)stage1_bound_kernel<16, 1>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    (void)hipFuncSetAttribute((const void*)stage1_bound_kernel<16, 2>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    (void)hipFuncSetAttribute((const void*)stage1_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    (void)hipFuncSetAttribute((const void*)stage1_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    (void)hipFuncSetAttribute((const void*)stage1_exact_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     attr_set = true;
   }
   const signed char* qv = (const signed char*)queries_q;
   const signed char* h = (const signed char*)hi;
   const signed char* l = (const signed char*)lo;
   if (exact) {
-    hipLaunchKernelGGL(stage1_kernel<true>, dim3(nwg), dim3(512), lds, st, lu, ll, lr, ldrop, cu, cl, cr, qv, qmeta,
+    hipLaunchKernelGGL(stage1_exact_kernel, dim3(nwg), dim3(512), lds, st, lu, ll, lr, ldrop, cu, cl, cr, qv, qmeta,
                        h, l, rmeta, Q, N, D, K, row_priority, row_tags, row_expiry, q_min_priority, q_tags, now);
     hipLaunchKernelGGL(stage2_kernel<true>, dim3(Q), dim3(THREADS), 0, st, out_scores, out_rows, unsafe, lu, ll, lr,
                        ldrop, nwg, qv, qmeta, h, l, rmeta, D, K);
   } else {
-    static const int variant = [] { const char* e = getenv("PILOTTAI_Q16_STAGE1"); return e ? atoi(e) : 1; }();
-    if (variant == 0) {
-      hipLaunchKernelGGL(stage1_kernel<false>, dim3(nwg), dim3(THREADS), lds, st, lu, ll, lr, ldrop, cu, cl, cr, qv,
-                         qmeta, h, l, rmeta, Q, N, D, K, row_priority, row_tags, row_expiry, q_min_priority, q_tags,
-                         now);
-    } else {
-      const int dsc = D <= 256 ? 4 : (D <= 512 ? 8 : 16);
-      const size_t ldsb = (size_t)MAXQ * (dsc * 64 + 16) * 2 + CAND_B * 12 + sizeof(QState) + 16 + 8 * 32 * 24;
-#define COMMA ,
-#define Q16_BOUND(KERN_)                                                                                     \
-      hipLaunchKernelGGL(KERN_, dim3(nwg), dim3(512), ldsb, st, lu, ll, lr, ldrop, cu, cl, cr, \
-                         qv, qmeta, h, rmeta, Q, N, D, K, row_priority, row_tags, row_expiry, q_min_priority,       \
-                         q_tags, now)
-      if (dsc == 4) Q16_BOUND((stage1_bound_kernel<4>));
-      else if (dsc == 8) Q16_BOUND((stage1_bound_kernel<8>));
-      else if (variant == 2) Q16_BOUND((stage1_bound_kernel<16, 1>));
-      else if (variant == 3) Q16_BOUND((stage1_bound_kernel<16, 2>));
-      else Q16_BOUND((stage1_bound_kernel<16>));
-#undef Q16_BOUND
-    }
+    const int dsc = D <= 256 ? 4 : (D <= 512 ? 8 : 16);
+    const size_t ldsb = (size_t)MAXQ * (dsc * 64 + 16) * 2 + sizeof(QState) + 16 + 8 * 32 * 24;
+    auto* bound = dsc == 4 ? stage1_bound_kernel<4> : dsc == 8 ? stage1_bound_kernel<8> : stage1_bound_kernel<16>;
+    hipLaunchKernelGGL(bound, dim3(nwg), dim3(512), ldsb, st, lu, ll, lr, ldrop, cu, cl, cr, qv, qmeta, h, rmeta, Q, N, D,
+                       K, row_priority, row_tags, row_expiry, q_min_priority, q_tags, now);
     hipLaunchKernelGGL(stage2_kernel<false>, dim3(Q), dim3(THREADS), 0, st, out_scores, out_rows, unsafe, lu, ll, lr,
                        ldrop, nwg, qv, qmeta, h, l, rmeta, D, K);
   }

@@ -1,0 +1,120 @@
+// Selection of the k best of a few hundred keys by a wave, and of a few thousand by a workgroup, without sorting: the
+// k-th best key is found bit by bit from the counts of keys that reach a trial value (a ballot per key and bit).
+#pragma once
+#include "common.h"
+
+namespace pa {
+
+// Floats as unsigned integers in the same order; 0 lies below all of them and stands for "no entry".
+__device__ __forceinline__ uint32_t ord_key(float x) {
+  const uint32_t u = __float_as_uint(x);
+  return (u >> 31) ? ~u : u | 0x80000000u;
+}
+__device__ __forceinline__ float key_value(uint32_t k) {
+  return __uint_as_float((k >> 31) ? k & 0x7fffffffu : ~k);
+}
+
+__device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, o, 64));
+  return v;
+}
+
+// entries of the lanes before this one that `p` holds for
+__device__ __forceinline__ int rank_in(unsigned long long ballot) {
+  return __builtin_amdgcn_mbcnt_hi((uint32_t)(ballot >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ballot, 0));
+}
+
+// The `want`-th largest of a wave's keys (N a lane; at least `want` of them are not 0).
+template <int N>
+__device__ __forceinline__ uint32_t wave_select(const uint32_t (&key)[N], int want) {
+  uint32_t v = 0;
+  for (int b = 31; b >= 0; --b) {
+    const uint32_t t = v | (1u << b);
+    int c = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) c += __popcll(__ballot(key[i] >= t));
+    if (c >= want) {
+      v = t;
+      if (c == want) break;
+    }
+  }
+  uint32_t m = 0xffffffffu;
+#pragma unroll
+  for (int i = 0; i < N; ++i) m = key[i] >= v ? min(m, key[i]) : m;
+  return wave_umin(m);
+}
+
+// The same over a workgroup of NW waves; every thread calls it. `red` holds 2 * NW integers in LDS.
+template <int N, int NW>
+__device__ __forceinline__ uint32_t block_select(const uint32_t (&key)[N], int want, int* red) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  __syncthreads();  // (earlier readers of red)
+  uint32_t v = 0;
+  int flip = 0;
+  for (int b = 31; b >= 0; --b) {
+    const uint32_t t = v | (1u << b);
+    int c = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) c += __popcll(__ballot(key[i] >= t));
+    if (lane == 0) red[flip * NW + wid] = c;
+    __syncthreads();
+    c = 0;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) c += red[flip * NW + w];
+    flip ^= 1;
+    if (c >= want) {
+      v = t;
+      if (c == want) break;
+    }
+  }
+  uint32_t m = 0xffffffffu;
+#pragma unroll
+  for (int i = 0; i < N; ++i) m = key[i] >= v ? min(m, key[i]) : m;
+  m = wave_umin(m);
+  __syncthreads();
+  if (lane == 0) red[wid] = (int)m;
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < NW; ++w) m = min(m, (uint32_t)red[w]);
+  return m;
+}
+
+// The `K` best of (key, row) entries that gather() names, in order (key down, row up), to out_s / out_r, padded with
+// (-inf, -1). Every thread of a workgroup of at least SEL threads calls it with its N entries; `kth`: the K-th best key
+// (block_select), or 1 where there are at most K entries. More than SEL entries that tie with kth: any of them.
+constexpr int SEL = 512;
+struct Selection {
+  uint32_t key[SEL];
+  int row[SEL], n;
+};
+template <int N>
+__device__ __forceinline__ void write_best(const uint32_t (&key)[N], const int (&row)[N], uint32_t kth, int K, Selection& s,
+                                           float* out_s, int* out_r) {
+  __syncthreads();
+  if (threadIdx.x == 0) s.n = 0;
+  __syncthreads();
+  auto take = [&](bool yes, uint32_t k, int r) {
+    if (yes) {
+      const int p = atomicAdd(&s.n, 1);
+      if (p < SEL) { s.key[p] = k; s.row[p] = r; }
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < N; ++i) take(key[i] > kth, key[i], row[i]);  // fewer than K
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; ++i) take(key[i] == kth, key[i], row[i]);
+  __syncthreads();
+  const int n = min(s.n, SEL), t = threadIdx.x;
+  if (t < n) {
+    const uint32_t k = s.key[t];
+    const int r = s.row[t];
+    int rank = 0;
+    for (int j = 0; j < n; ++j) rank += s.key[j] > k || (s.key[j] == k && s.row[j] < r);
+    if (rank < K) { out_s[rank] = key_value(k); out_r[rank] = r; }
+  }
+  if (t < K && t >= n) { out_s[t] = -INFINITY; out_r[t] = -1; }
+}
+
+}  // namespace pa
