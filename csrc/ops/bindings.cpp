@@ -67,6 +67,7 @@ int pa_cosine_topk(float* out_scores, int* out_rows, void* workspace, const void
                    const uint64_t* row_tags, const float* row_expiry, const int* q_min_priority,
                    const uint64_t* q_tags, float now, int n_valid, hipStream_t st);
 long long pa_q16_topk_workspace_bytes(int Q, int N);
+int pa_prepare_queries(const float* x, int Q, int D, int normalize, void* out, void* qv, float* qmeta, hipStream_t st);
 int pa_q16_topk(float* out_scores, int* out_rows, int* unsafe, void* workspace, const void* queries_q,
                 const float* qmeta, const void* hi, const void* lo, const float* rmeta, int Q, int N, int D, int K,
                 const int* row_priority, const uint64_t* row_tags, const float* row_expiry,
@@ -574,6 +575,31 @@ void cosine_topk(at::Tensor out_scores, at::Tensor out_rows, at::Tensor workspac
            "cosine_topk");
 }
 
+// Queries as the index's kernels read them: bf16 rows (out), or 16-bit fixed point (qv, qmeta).
+void prepare_queries(at::Tensor x, bool normalize, c10::optional<at::Tensor> out, c10::optional<at::Tensor> qv,
+                     c10::optional<at::Tensor> qmeta) {
+  check_gpu(x, "queries");
+  check_dtype(x, at::kFloat, "queries");
+  TORCH_CHECK(x.dim() == 2 && x.is_contiguous(), "queries [Q, D] contiguous");
+  const int64_t n = x.numel();
+  if (out) {
+    check_gpu(*out, "out");
+    check_dtype(*out, at::kBFloat16, "out");
+    TORCH_CHECK(out->is_contiguous() && out->numel() == n, "out [Q, D]");
+  } else {
+    TORCH_CHECK(qv && qmeta, "either out or qv and qmeta");
+    check_gpu(*qv, "qv");
+    check_gpu(*qmeta, "qmeta");
+    check_dtype(*qv, at::kChar, "qv");
+    check_dtype(*qmeta, at::kFloat, "qmeta");
+    TORCH_CHECK(qv->is_contiguous() && qv->numel() == 2 * n, "qv [Q, 2, D]");
+    TORCH_CHECK(qmeta->is_contiguous() && qmeta->numel() == 2 * x.size(0), "qmeta [Q, 2]");
+  }
+  check_rc(pa_prepare_queries(x.data_ptr<float>(), (int)x.size(0), (int)x.size(1), normalize, out ? out->data_ptr() : nullptr,
+                              out ? nullptr : qv->data_ptr(), out ? nullptr : qmeta->data_ptr<float>(), cur_stream()),
+           "prepare_queries");
+}
+
 int64_t q16_topk_workspace_bytes(int64_t Q, int64_t N) { return pa_q16_topk_workspace_bytes(Q, N); }
 
 // Two-stage exact top-k over the 16-bit fixed-point index (csrc/ops/similarity_q16.hip).
@@ -857,6 +883,8 @@ PYBIND11_MODULE(_C, m) {
   m.def("tp_topkp_phase", &tp_topkp_phase);
   m.def("cosine_topk_workspace_bytes", &cosine_topk_workspace_bytes);
   m.def("cosine_topk", &cosine_topk);
+  m.def("prepare_queries", &prepare_queries, py::arg("x"), py::arg("normalize"), py::arg("out") = py::none(),
+        py::arg("qv") = py::none(), py::arg("qmeta") = py::none());
   m.def("q16_topk_workspace_bytes", &q16_topk_workspace_bytes);
   m.def("q16_topk", &q16_topk);
   m.def("car_alloc", &car_alloc);

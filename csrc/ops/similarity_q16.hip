@@ -765,6 +765,64 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
   }
 }
 
+// ---- queries ------------------------------------------------------------------------------------------
+// x / y rounded as IEEE does, whatever the compiler may do with a float division (fast-math): the double quotient
+// rounds to the same float, and the empty asm keeps the two steps apart.
+__device__ __forceinline__ float div_rn(float x, float y) {
+  double d = (double)x / (double)y;
+  asm volatile("" : "+v"(d));
+  return (float)d;
+}
+
+// One workgroup a query: normalised (if asked), then rounded to bf16, or to 16-bit fixed point as q16_quantize does:
+// s_q = max|x| / 32512, v = round(x / s_q) = 256 qh + ql, c_q = s_q ||v||_2 (a hair above). One launch in place of the 28
+// elementwise ones that took as long as the search of a small index.
+__global__ __launch_bounds__(256) void prepare_kernel(const float* __restrict__ x, int D, int normalize, bf16* __restrict__ out,
+                                                      signed char* __restrict__ qv, float* __restrict__ qmeta) {
+  __shared__ double red[4];
+  __shared__ float redm[4];
+  const int q = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  x += (size_t)q * D;
+  auto sum = [&](double v) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
+    __syncthreads();
+    if (lane == 0) red[wid] = v;
+    __syncthreads();
+    return red[0] + red[1] + red[2] + red[3];
+  };
+  float by = 1.f;
+  if (normalize) {
+    double ss = 0.;
+    for (int i = threadIdx.x; i < D; i += 256) ss += (double)x[i] * (double)x[i];
+    by = fmaxf((float)sqrt(sum(ss)), 1e-12f);
+  }
+  if (out) {
+    for (int i = threadIdx.x; i < D; i += 256) out[(size_t)q * D + i] = (bf16)(normalize ? div_rn(x[i], by) : x[i]);
+    return;
+  }
+  float m = 0.f;
+  for (int i = threadIdx.x; i < D; i += 256) m = fmaxf(m, fabsf(normalize ? div_rn(x[i], by) : x[i]));
+  m = wave_max(m);
+  if (lane == 0) redm[wid] = m;
+  __syncthreads();
+  m = fmaxf(fmaxf(redm[0], redm[1]), fmaxf(redm[2], redm[3]));
+  const float sc = m > 0.f ? div_rn(m, 32512.f) : 1.f;
+  double vv = 0.;
+  for (int i = threadIdx.x; i < D; i += 256) {
+    const float f = rintf(div_rn(normalize ? div_rn(x[i], by) : x[i], sc));
+    const int v = (int)fminf(fmaxf(f, -32512.f), 32512.f), h = (v + 128) >> 8;
+    qv[(size_t)q * 2 * D + i] = (signed char)h;
+    qv[(size_t)q * 2 * D + D + i] = (signed char)(v - 256 * h);
+    vv += (double)v * (double)v;  // whole numbers below 2^53: exact in any order
+  }
+  vv = sum(vv);
+  if (threadIdx.x == 0) {
+    qmeta[2 * q] = sc;
+    qmeta[2 * q + 1] = (float)((double)sc * sqrt(vv)) * (1.f + 1e-6f);
+  }
+}
+
 }  // namespace q16
 }  // namespace pa
 
@@ -829,5 +887,14 @@ extern "C" int pa_q16_topk(float* out_scores, int* out_rows, int* unsafe, void* 
     hipLaunchKernelGGL(stage2_kernel<false>, dim3(Q), dim3(THREADS), 0, st, out_scores, out_rows, unsafe, lu, ll, lr,
                        ldrop, nwg, qv, qmeta, h, l, rmeta, D, K);
   }
+  return (int)hipGetLastError();
+}
+
+// x fp32 [Q][D] -> bf16 [Q][D] (out), or, with out null, int8 [Q][2][D] (qv) and fp32 [Q][2] (qmeta).
+extern "C" int pa_prepare_queries(const float* x, int Q, int D, int normalize, void* out, void* qv, float* qmeta,
+                                  hipStream_t st) {
+  if (Q <= 0) return 0;
+  hipLaunchKernelGGL(pa::q16::prepare_kernel, dim3(Q), dim3(256), 0, st, x, D, normalize, (pa::bf16*)out, (signed char*)qv,
+                     qmeta);
   return (int)hipGetLastError();
 }

@@ -306,26 +306,73 @@ class SemanticIndex:
         with self._lock, self._stream_ctx():
             if caller is not None:  # `q` was produced on the caller's stream
                 torch.cuda.current_stream(self.device).wait_stream(caller)
-            qd = torch.nn.functional.normalize(q.to(self.device, torch.float32), dim=1)
-            if self.storage != "q16":  # q16 quantises the fp32 query itself (16-bit fixed point)
-                qd = qd.to(torch.bfloat16)
+            qd = q.to(self.device, torch.float32).contiguous()
             minp = torch.as_tensor(min_priority, dtype=torch.int32).to(self.device)
             qt = torch.as_tensor(qmasks, dtype=torch.int64).to(self.device)
-            ev = None
-            if self.pass_events is not None and self.device.type == "cuda":
-                ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
-                ev[0].record()
+            ev = self._pass_event()
             t_now = self.now() if now is None else now - self.epoch
-            if self.storage == "q16":
-                s, r = ops.q16_topk(qd, self.hi, self.lo, self.rmeta, self.count, k, self.priority,
-                                    self.tagbits, self.expiry, minp, qt, t_now, workspace=self._ws, stats=self.stats)
+            if self.storage == "q16":  # (the fp32 query is quantised itself, to 16-bit fixed point)
+                s, r = ops.q16_topk(qd, self.hi, self.lo, self.rmeta, self.count, k, self.priority, self.tagbits,
+                                    self.expiry, minp, qt, t_now, workspace=self._ws, stats=self.stats, normalize=True)
             else:
-                s, r = ops.cosine_topk(qd, self.packed, self.count, k, self.priority, self.tagbits, self.expiry, minp,
-                                       qt, t_now, workspace=self._ws)
+                s, r = ops.cosine_topk(ops.unit_queries(qd), self.packed, self.count, k, self.priority, self.tagbits,
+                                       self.expiry, minp, qt, t_now, workspace=self._ws)
             if ev is not None:
                 ev[1].record()
                 self.pass_events.append(ev)
         return s, r
+
+    def _pass_event(self):
+        """(start, end) events around a pass, the first recorded, where passes are timed."""
+        if self.pass_events is None or self.device.type != "cuda":
+            return None
+        ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
+        ev[0].record()
+        return ev
+
+    def _search_host(self, q: torch.Tensor, k: int, min_priority, qmasks, now: Optional[float]):
+        """search_tensors for a caller that waits for the answer: (scores, rows) as arrays, [Q, k]. What the pass reads
+        goes to the device in one pinned copy and comes back in one (queries and filters, scores, rows and flags were
+        four copies out and up to three back, each with its own wait)."""
+        Q, D = q.shape
+        caller = torch.cuda.current_stream(self.device) if q.is_cuda else None
+        with self._lock, self._stream_ctx():
+            here = torch.cuda.current_stream(self.device)
+            if caller is not None:
+                here.wait_stream(caller)
+            host = torch.empty(16 * Q + (0 if q.is_cuda else 4 * Q * D), dtype=torch.uint8, pin_memory=True)
+            h = host.numpy()
+            h[:8 * Q].view(np.int64)[:] = qmasks
+            h[8 * Q:12 * Q].view(np.int32)[:] = min_priority
+            if not q.is_cuda:
+                h[16 * Q:].view(np.float32).reshape(Q, D)[:] = q.detach().float().numpy()
+            dev = host.to(self.device, non_blocking=True)
+            qt, minp = dev[:8 * Q].view(torch.int64), dev[8 * Q:12 * Q].view(torch.int32)
+            qd = q.to(self.device, torch.float32).contiguous() if q.is_cuda else dev[16 * Q:].view(torch.float32).view(Q, D)
+            ev = self._pass_event()
+            t_now = self.now() if now is None else now - self.epoch
+            buf, s, r, unsafe = ops.topk_result(Q, k, self.device)
+            filters = (self.priority, self.tagbits, self.expiry, minp, qt, t_now)
+            if self.storage == "q16":
+                qv, qm = ops.q16_queries(qd, normalize=True)
+                args = (qv, qm, self.hi, self.lo, self.rmeta, self.count, k, *filters, (s, r, unsafe))
+                ops.q16_pass(*args, False, self._ws)
+            else:
+                ops.cosine_topk(ops.unit_queries(qd), self.packed, self.count, k, *filters, workspace=self._ws, out=(s, r))
+            if ev is not None:
+                ev[1].record()
+                self.pass_events.append(ev)
+            back = torch.empty(buf.shape, dtype=torch.int32, pin_memory=True)
+            back.copy_(buf, non_blocking=True)
+        a = back.numpy()
+        here.synchronize()
+        if self.storage == "q16" and a[2 * Q * k:].any():  # a slice refused a row that might be in the top-k
+            with self._lock, self._stream_ctx():
+                self.stats["q16_fallbacks"] += 1
+                ops.q16_pass(*args, True, self._ws)
+                back.copy_(buf, non_blocking=True)
+            here.synchronize()
+        return a[:Q * k].view(np.float32).reshape(Q, k), a[Q * k:2 * Q * k].reshape(Q, k)
 
     def search(self, queries, k: int, min_priority: Sequence[int], tags: Sequence[Iterable[str]],
                now: Optional[float] = None) -> List[List[Tuple[int, float]]]:
@@ -340,9 +387,10 @@ class SemanticIndex:
         if self.count == 0:
             return [[] for _ in range(Q)]
         kk = k if all(exact) else min(64, 4 * k)
-        s, r = self.search_tensors(q, kk, list(min_priority), qmasks, now)
-        with self._stream_ctx():
-            s, r = s.cpu().numpy(), r.cpu().numpy()
+        if self.device.type == "cuda":
+            s, r = self._search_host(q, kk, list(min_priority), qmasks, now)
+        else:
+            s, r = (t.numpy() for t in self.search_tensors(q, kk, list(min_priority), qmasks, now))
         out = []
         for i in range(Q):
             res = []

@@ -258,13 +258,28 @@ def sample(logits, temperature, mask_class, class_masks, seeds, offsets, forced=
 COSINE_MAX_Q = 64  # queries per index pass (LDS-resident query tiles)
 
 
+def unit_queries(q: torch.Tensor) -> torch.Tensor:
+    """bf16 rows of unit length from fp32 ones."""
+    if not _on_gpu(q):
+        return torch.nn.functional.normalize(q, dim=1).to(torch.bfloat16)
+    out = torch.empty_like(q, dtype=torch.bfloat16)
+    require_native().prepare_queries(q, True, out=out)
+    return out
+
+
+def topk_result(Q: int, K: int, device):
+    """(buffer, scores [Q, K], rows [Q, K], flags [Q]) of a lookup: one buffer, so that one copy brings it to the host."""
+    buf = torch.empty(Q * (2 * K + 1), dtype=torch.int32, device=device)
+    return buf, buf[:Q * K].view(torch.float32).view(Q, K), buf[Q * K:2 * Q * K].view(Q, K), buf[2 * Q * K:]
+
+
 def cosine_topk(queries, index, n_valid: int, K: int, row_priority, row_tags, row_expiry,
-                q_min_priority, q_tags, now: float, workspace: Optional[torch.Tensor] = None):
+                q_min_priority, q_tags, now: float, workspace: Optional[torch.Tensor] = None, out=None):
+    """`out`: (scores, rows) to write to."""
     if _on_gpu(index):
         C = require_native()
         Q = queries.shape[0]
-        out_s = torch.empty(Q, K, dtype=torch.float32, device=index.device)
-        out_r = torch.empty(Q, K, dtype=torch.int32, device=index.device)
+        out_s, out_r = out if out is not None else topk_result(Q, K, index.device)[1:3]
         qc = min(Q, COSINE_MAX_Q)
         need = C.cosine_topk_workspace_bytes(qc, max(1, int(n_valid)), K)
         if workspace is None or workspace.numel() * workspace.element_size() < need:
@@ -312,46 +327,59 @@ def q16_unpack(tiles: torch.Tensor) -> torch.Tensor:
     return tiles.view(T, DS, 4, 16, 16).permute(0, 3, 1, 2, 4).reshape(T * 16, DS * 64)
 
 
-def q16_queries(q: torch.Tensor):
-    """Queries -> (qv int8 [Q, 2, D] = (qh, ql), qmeta fp32 [Q, 2] = (scale, scale * ||v||_2))."""
+def q16_queries(q: torch.Tensor, normalize: bool = False):
+    """Queries -> (qv int8 [Q, 2, D] = (qh, ql), qmeta fp32 [Q, 2] = (scale, scale * ||v||_2)); the same bits from the
+    kernel and on the CPU."""
+    if _on_gpu(q):
+        q = q.float().contiguous()
+        Q, D = q.shape
+        qv = torch.empty(Q, 2, D, dtype=torch.int8, device=q.device)
+        qm = torch.empty(Q, 2, dtype=torch.float32, device=q.device)
+        require_native().prepare_queries(q, normalize, qv=qv, qmeta=qm)
+        return qv, qm
+    if normalize:
+        q = torch.nn.functional.normalize(q.float(), dim=1)
     hi, lo, sc, _ = q16_quantize(q)
     v = 256 * hi.double() + lo.double()
     cq = (sc.double() * v.norm(dim=1)).float() * (1 + 1e-6)
     return torch.stack([hi, lo], 1).contiguous(), torch.stack([sc, cq], 1).contiguous()
 
 
+def q16_pass(qv, qm, hi, lo, rmeta, n_valid: int, K: int, row_priority, row_tags, row_expiry, q_min_priority, q_tags,
+             now: float, out, exact: bool, workspace: Optional[torch.Tensor] = None) -> None:
+    """One pass of quantised queries over a GPU's index into `out` (scores, rows, flags): flags[q] != 0 asks for the batch
+    again with exact = True."""
+    C = require_native()
+    Q = qv.shape[0]
+    out_s, out_r, unsafe = out
+    qc = min(Q, COSINE_MAX_Q)
+    need = C.q16_topk_workspace_bytes(qc, max(1, int(n_valid)))
+    if workspace is None or workspace.numel() * workspace.element_size() < need:
+        workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=hi.device)
+    for q0 in range(0, Q, COSINE_MAX_Q):
+        q1 = min(Q, q0 + COSINE_MAX_Q)
+        C.q16_topk(out_s[q0:q1], out_r[q0:q1], unsafe[q0:q1], workspace, qv[q0:q1], qm[q0:q1], hi, lo, rmeta,
+                   int(n_valid), int(K), row_priority, row_tags, row_expiry,
+                   q_min_priority[q0:q1].contiguous(), q_tags[q0:q1].contiguous(), float(now), int(exact))
+
+
 def q16_topk(queries, hi, lo, rmeta, n_valid: int, K: int, row_priority, row_tags, row_expiry,
              q_min_priority, q_tags, now: float, workspace: Optional[torch.Tensor] = None, exact: bool = False,
-             stats: Optional[dict] = None):
+             stats: Optional[dict] = None, normalize: bool = False):
     """Exact filtered top-k over a q16 index (scores of the 16-bit fixed-point vectors, the
     same on the GPU and in ops.reference.q16_topk). GPU: the two-stage kernel, hi plane only in
     the streaming pass; a batch whose drop check fails is re-run with the exact scan (counted
-    in stats["q16_fallbacks"]). queries: fp32 / bf16 [Q, D] (quantised here)."""
-    qv, qm = q16_queries(queries)
+    in stats["q16_fallbacks"]). queries: fp32 / bf16 [Q, D] (quantised here; `normalize`: brought to unit length first)."""
+    qv, qm = q16_queries(queries, normalize)
     if _on_gpu(hi):
-        C = require_native()
-        Q = qv.shape[0]
-        out_s = torch.empty(Q, K, dtype=torch.float32, device=hi.device)
-        out_r = torch.empty(Q, K, dtype=torch.int32, device=hi.device)
-        unsafe = torch.zeros(Q, dtype=torch.int32, device=hi.device)
-        qc = min(Q, COSINE_MAX_Q)
-        need = C.q16_topk_workspace_bytes(qc, max(1, int(n_valid)))
-        if workspace is None or workspace.numel() * workspace.element_size() < need:
-            workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=hi.device)
-        for q0 in range(0, Q, COSINE_MAX_Q):
-            q1 = min(Q, q0 + COSINE_MAX_Q)
-            C.q16_topk(out_s[q0:q1], out_r[q0:q1], unsafe[q0:q1], workspace, qv[q0:q1], qm[q0:q1], hi, lo, rmeta,
-                       int(n_valid), int(K), row_priority, row_tags, row_expiry,
-                       q_min_priority[q0:q1].contiguous(), q_tags[q0:q1].contiguous(), float(now), int(exact))
+        _, s, r, unsafe = topk_result(qv.shape[0], K, hi.device)
+        args = (qv, qm, hi, lo, rmeta, n_valid, K, row_priority, row_tags, row_expiry, q_min_priority, q_tags, now)
+        q16_pass(*args, (s, r, unsafe), exact, workspace)
         if not exact and bool(unsafe.any()):  # a slice refused a row that might be in the top-k
             if stats is not None:
                 stats["q16_fallbacks"] = stats.get("q16_fallbacks", 0) + 1
-            for q0 in range(0, Q, COSINE_MAX_Q):
-                q1 = min(Q, q0 + COSINE_MAX_Q)
-                C.q16_topk(out_s[q0:q1], out_r[q0:q1], unsafe[q0:q1], workspace, qv[q0:q1], qm[q0:q1], hi, lo,
-                           rmeta, int(n_valid), int(K), row_priority, row_tags, row_expiry,
-                           q_min_priority[q0:q1].contiguous(), q_tags[q0:q1].contiguous(), float(now), 1)
-        return out_s, out_r
+            q16_pass(*args, (s, r, unsafe), True, workspace)
+        return s, r
     return ref.q16_topk(qv, qm, hi, lo, rmeta, n_valid, K, row_priority, row_tags, row_expiry,
                         q_min_priority, q_tags, now)
 

@@ -68,6 +68,48 @@ def test_q16_exact_scan_matches_reference(gpu, N, Q, K):
     _check(gpu, N, 1024, Q, K, True, exact=True, seed=5)
 
 
+@pytest.mark.parametrize("N,D,Q,K,filters", [
+    (255, 64, 3, 64, False), (257, 192, 2, 7, True),  # one slice, two slices
+    (65_536 + 31, 256, 64, 33, True), (2 * 65_536, 256, 64, 64, False),  # the last size before slices share bounds
+    (2 * 65_536 + 1, 256, 64, 1, True), (600_011, 256, 5, 64, True)])  # and with them
+def test_q16_slices_and_shared_bounds(gpu, N, D, Q, K, filters):
+    _check(gpu, N, D, Q, K, filters, seed=11)
+
+
+def test_q16_fewer_hits_than_k(gpu):
+    """Rows that pass the filters are fewer than K, and lie in few slices."""
+    N, D, Q, K = 200_000, 256, 3, 9
+    hi, lo, rmeta = _index(N, D, gpu, 4)
+    prio = torch.zeros(N, dtype=torch.int32, device=gpu)
+    prio[[5, 70_000, 199_999]] = 7
+    tags, exp = torch.zeros(N, dtype=torch.int64, device=gpu), torch.zeros(N, device=gpu)
+    minp = torch.full((Q,), 7, dtype=torch.int32, device=gpu)
+    q = torch.randn(Q, D, device=gpu)
+    s, r = ops.q16_topk(q, hi, lo, rmeta, N, K, prio, tags, exp, minp, torch.zeros_like(minp, dtype=torch.int64), 0.0)
+    assert (r[:, 3:] == -1).all() and bool((s[:, 3:] == -float("inf")).all())
+    assert all(sorted(x[:3]) == [5, 70_000, 199_999] for x in r.tolist())
+
+
+@pytest.mark.parametrize("Q,D", [(1, 64), (64, 1024), (5, 320)])
+def test_query_preparation_matches_torch(gpu, Q, D):
+    """The kernel's fixed-point queries have the bits of the CPU's; normalised ones differ by the rounding of the norm
+    (a sum in float64 against one in float32): at most 2 ulp of a coordinate, 1 unit of its 16-bit form."""
+    q = torch.randn(Q, D, device=gpu) * 3.0
+    q[0, 1:] = 0.0
+    if Q > 2:
+        q[2] = 0.0
+    qv, qm = ops.q16_queries(q)
+    rv, rm = ops.q16_queries(q.cpu())
+    assert torch.equal(qv.cpu(), rv) and torch.equal(qm.cpu(), rm)
+    qv, qm = ops.q16_queries(q, normalize=True)
+    rv, rm = ops.q16_queries(q.cpu(), normalize=True)
+    whole = lambda v: 256 * v[:, 0].int() + v[:, 1].int()  # noqa: E731
+    assert int((whole(qv.cpu()) - whole(rv)).abs().max()) <= 1
+    assert torch.allclose(qm.cpu(), rm, rtol=4 * 2.0 ** -24, atol=0)
+    u = torch.nn.functional.normalize(q.cpu(), dim=1)
+    assert (ops.unit_queries(q).cpu().float() - u).abs().max() <= 2.0 ** -8 * u.abs().max()
+
+
 def test_q16_planted_neighbours_found(gpu):
     _check(gpu, 400_000, 1024, 32, 5, False, seed=7, planted=True)
 
