@@ -13,6 +13,7 @@ extern "C" {
 int pa_decode_gemm(void* y, const void* x, const void* wp, const void* resid, int M, int N, int K,
                    int ldx, int ldy, int ldr, int epi, int norm, float eps, int nt, int waves, int splits,
                    float* ws, long long ws_floats, int* counters, int n_counters, hipStream_t st);
+int pa_rows_gemm(void* y, const void* x, const void* wp, int M, int N, int K, int ldx, int ldy, hipStream_t st);
 int pa_prefill_gemm(void* y, const void* x, const void* wp, const void* resid, float* ws, long long ws_floats,
                     int* counters, int n_counters, int M, int N, int K, int ldx, int ldy, int ldr, int epi,
                     const float* ss_in, float* ss_out, float* ss_zero, float eps, int full, int splits, int bn,
@@ -86,6 +87,22 @@ bool decode_gemm(at::Tensor y, at::Tensor x, at::Tensor wp, c10::optional<at::Te
                                 ldr, (int)epi, norm ? 1 : 0, (float)eps, (int)nt, (int)waves, (int)splits, wsp, wsn,
                                 cp, cn, cur_stream());
   TORCH_CHECK(rc >= 0, "decode_gemm launch failed");
+  return rc == 0;
+}
+
+// y = x W^T on packed weights, as decode_gemm's plain form, for more rows (gemm_decode.hip dispatch_rows). Returns false if
+// the sizes are not handled.
+bool rows_gemm(at::Tensor y, at::Tensor x, at::Tensor wp) {
+  check_gpu(wp, "wp");
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1, "x must be a 2-D GPU tensor, unit inner stride");
+  TORCH_CHECK(y.is_cuda() && y.dim() == 2 && y.stride(1) == 1, "y must be a 2-D GPU tensor, unit inner stride");
+  check_dtype(x, at::kBFloat16, "x"); check_dtype(wp, at::kBFloat16, "wp"); check_dtype(y, at::kBFloat16, "y");
+  TORCH_CHECK(wp.dim() == 4 && wp.size(2) == 64 && wp.size(3) == 8, "wp must be packed [N/16, K/32, 64, 8]");
+  const int M = x.size(0), K = x.size(1), N = wp.size(0) * 16;
+  TORCH_CHECK(wp.size(1) * 32 == K, "packed weight K ", wp.size(1) * 32, " != x K ", K);
+  TORCH_CHECK(y.size(0) == M && y.size(1) == N, "y shape [", y.size(0), ", ", y.size(1), "] != [", M, ", ", N, "]");
+  const int rc = pa_rows_gemm(y.data_ptr(), x.data_ptr(), wp.data_ptr(), M, N, K, x.stride(0), y.stride(0), cur_stream());
+  TORCH_CHECK(rc >= 0, "rows_gemm launch failed");
   return rc == 0;
 }
 

@@ -286,5 +286,6 @@ PYBIND11_MODULE(_hybrid, m) {
   m.def("expert_gemm", &expert_gemm);
   m.def("empty_uncached", &empty_uncached);
   m.def("decode_gemm", &decode_gemm);
+  m.def("rows_gemm", &rows_gemm);
   m.def("prefill_gemm", &prefill_gemm);
 }

@@ -45,5 +45,6 @@ PYBIND11_MODULE(_latent, m) {
   m.def("expert_gemm", &expert_gemm);
   m.def("empty_uncached", &empty_uncached);
   m.def("decode_gemm", &decode_gemm);
+  m.def("rows_gemm", &rows_gemm);
   m.def("prefill_gemm", &prefill_gemm);
 }

@@ -356,6 +356,151 @@ static int pick_nw(int nt, int waves, const DgArgs& a, hipStream_t st) {
   return 1;
 }
 
+// ---- more than 16 rows, plain epilogue: x through LDS --------------------------------------------------
+// decode_gemm_kernel's fragment loads of x (16 rows x 64 B an instruction) take about 88 cycles of a CU each, however many
+// are in flight: at 64 rows and K = 8192, x alone cost 37 us beside 34 MB of weights (7 us). Here a workgroup loads whole
+// runs of rows, 64 WK k a stage, and its waves read the fragments from LDS. WK waves split the k-steps of a stage, the
+// others lie side by side over NT tiles each; rows beyond 16 MT go to workgroups of their own on the same XCD, whose
+// second pass over the weights is its L2's. Weights and x are one in-order ring of loads, D stages deep, so that neither
+// drains the other, and the stage barrier waits for LDS alone. What bounds it then is the L2s' rate on x, which every
+// column group reads whole: hence the largest tile that still gives every CU one (dispatch_rows).
+// us at 64 rows, before -> after (x from L2, cold weights): N x K 2048 x 8192 37 -> 20, 2048 x 4096 20 -> 11.4, 2048 x 2048
+// 11.7 -> 7.3, 10368 x 2048 17.8 -> 15.8, 128256 x 2048 144 -> 105.
+template <int MT, int NT, int WK, int D>
+__global__ __launch_bounds__(512) void decode_rows_kernel(const DgArgs A) {
+  constexpr int WN = 8 / WK;                // waves side by side, NT tiles each
+  constexpr int TM = MT * 16, TN = NT * WN * 16, NTH = 512;
+  constexpr int KW = 2, KC = 64 * WK;       // k-steps a wave and k of a stage
+  constexpr int XLD = KC * 2 + 16;          // LDS row, padded: the 16 rows of a fragment lie in different banks
+  constexpr int LR = KC / 8, RL = NTH / LR, XL = TM / RL;  // threads a row, rows a load, x loads a thread and stage
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // [2][TM][XLD], then the waves' partial tiles
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int g = lane >> 4, c = lane & 15, wk = wid % WK, wn = wid / WK;
+  const int xrow = threadIdx.x / LR, xu = threadIdx.x % LR;
+  const int nwg = gridDim.x, bid = blockIdx.x, q = nwg / 8, rr = nwg % 8, xcd = bid % 8;
+  const int work = (xcd < rr ? xcd * (q + 1) : rr * (q + 1) + (xcd - rr) * q) + bid / 8;
+  const int RG = (A.M + TM - 1) / TM;
+  const int row0 = (work % RG) * TM, tile0 = (work / RG) * NT * WN, tiles = A.N / 16;
+  const int K = A.K, KS = K / 32, nst = (K + KC - 1) / KC;
+  const bf16x8* wt[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    wt[j] = reinterpret_cast<const bf16x8*>(A.wp + (size_t)min(tile0 + wn * NT + j, tiles - 1) * KS * 512) + lane;
+  const bf16* xr[XL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) xr[i] = A.x + (size_t)min(row0 + xrow + RL * i, A.M - 1) * A.ldx;
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 wb[D][KW][NT], xb[D][XL];
+  // (past the end: the last ones again, unconditional, so that the waits stay counted)
+  auto load = [&](int st, int d) {
+    __builtin_amdgcn_sched_barrier(0);
+    const int k = min(st * KC + 8 * xu, K - 8);
+#pragma unroll
+    for (int i = 0; i < XL; ++i) xb[d][i] = *reinterpret_cast<const bf16x8*>(xr[i] + k);
+#pragma unroll
+    for (int u = 0; u < KW; ++u) {
+      const int ks = min(st * (KC / 32) + wk * KW + u, KS - 1);
+#pragma unroll
+      for (int j = 0; j < NT; ++j)
+        wb[d][u][j] = __builtin_nontemporal_load(wt[j] + (size_t)ks * 64);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, d);
+  for (int st0 = 0; st0 < nst; st0 += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int st = st0 + d;
+      if (st < nst) {  // uniform
+        char* slot = smem + (st & 1) * TM * XLD;
+#pragma unroll
+        for (int i = 0; i < XL; ++i) *reinterpret_cast<bf16x8*>(slot + (xrow + RL * i) * XLD + 16 * xu) = xb[d][i];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int u = 0; u < KW; ++u) {
+          if (st * (KC / 32) + wk * KW + u < KS) {
+            bf16x8 a[MT];
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+              a[i] = *reinterpret_cast<const bf16x8*>(slot + (16 * i + c) * XLD + (wk * KW + u) * 64 + 16 * g);
+#pragma unroll
+            for (int i = 0; i < MT; ++i)
+#pragma unroll
+              for (int j = 0; j < NT; ++j)
+                acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], wb[d][u][j], acc[i][j], 0, 0, 0);
+          }
+        }
+        load(st + D, d);
+      }
+    }
+  }
+  __syncthreads();
+  float* red = reinterpret_cast<float*>(smem);  // [WK][TM][TN]
+#pragma unroll
+  for (int i = 0; i < MT; ++i)
+#pragma unroll
+    for (int j = 0; j < NT; ++j)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        red[(wk * TM + 16 * i + 4 * g + r) * TN + (wn * NT + j) * 16 + c] = acc[i][j][r];
+  __syncthreads();
+  for (int e = threadIdx.x * 4; e < TM * TN; e += NTH * 4) {
+    f32x4 t = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int wv = 0; wv < WK; ++wv) t += *reinterpret_cast<const f32x4*>(red + wv * TM * TN + e);
+    const int m = row0 + e / TN, n = tile0 * 16 + e % TN;
+    if (m < A.M && n < A.N) {
+      bf16x4 o;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) o[r] = (bf16)t[r];
+      *reinterpret_cast<bf16x4*>(A.y + (size_t)m * A.ldy + n) = o;
+    }
+  }
+}
+
+template <int MT, int NT, int WK>
+static int launch_rows(const DgArgs& a, hipStream_t st) {
+  constexpr int D = 2;  // (4 stages deep: no faster)
+  constexpr int TM = MT * 16, TN = NT * (8 / WK) * 16;
+  constexpr size_t lds = std::max((size_t)2 * TM * (128 * WK + 16), (size_t)WK * TM * TN * sizeof(float));
+  static_assert(lds <= 160 * 1024, "LDS of a CU");
+  auto kern = decode_rows_kernel<MT, NT, WK, D>;
+  static bool attr = false;
+  if (!attr) {
+    hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+    attr = true;
+  }
+  hipLaunchKernelGGL(kern, dim3((a.N + TN - 1) / TN * ((a.M + TM - 1) / TM)), dim3(512), lds, st, a);
+  return (int)hipGetLastError() == 0 ? 0 : -2;
+}
+
+// The smallest tile that leaves at most one workgroup a CU (a second round of workgroups, or half the CUs idle, both
+// measured slower for every shape of 16 to 512 rows and 1,408 to 10,368 outputs): 64 rows x 2048 outputs 32x16 (20 us at K
+// = 8192; 32x32 23), 3072 32x32 (8.2 us at K = 2048; 32x16 10.1), 10368 64x64; 512 rows x 2048 64x64 (13.3 us, the
+// 256-row prefill tiles 19.8), 3072 64x128 (18.3 / 22.0). Where not even 64x128 does (1): up to 64 rows tiles of 64 columns
+// with the waves' loads side by side, which stream the weights at 5 TB/s (64 rows x 128256 x 2048: 105 us); above, the
+// prefill kernels (512 rows x 10368: 30 us against 52).
+static int dispatch_rows(const DgArgs& a, hipStream_t st) {
+  if (a.M <= 0) return 0;
+  if (a.K % 32 || a.N % 16 || a.ldx % 8 || a.ldy % 4 || ((uintptr_t)a.x & 15) || ((uintptr_t)a.wp & 15) || ((uintptr_t)a.y & 7)) return 1;
+  auto fits = [&](int tm, int tn) { return (long long)((a.M + tm - 1) / tm) * ((a.N + tn - 1) / tn) <= 256; };
+  if (fits(32, 16)) return launch_rows<2, 1, 8>(a, st);
+  if (fits(32, 32)) return launch_rows<2, 2, 8>(a, st);
+  if (fits(32, 64)) return launch_rows<2, 4, 8>(a, st);
+  if (fits(64, 64)) return launch_rows<4, 4, 8>(a, st);
+  if (fits(64, 128)) return launch_rows<4, 4, 4>(a, st);
+  if (a.M <= 32) return launch_rows<2, 2, 4>(a, st);
+  if (a.M <= 64) return launch_rows<4, 2, 4>(a, st);
+  return 1;
+}
+
 // Default (tile width, waves, K slices) per shape, from tools/decode_gemm_bench.py on
 // MI355X (profiles/r1_decode_gemm.md, r1_decode_gemm_splitk.jsonl): 2 column tiles per
 // workgroup once there are >= 384 tiles (x fragments re-used across both), 4 for wide
@@ -380,6 +525,10 @@ static int dispatch(DgArgs a, int epi, int norm, int nt, int waves, int splits, 
   if (M > 64 || a.K % 32 != 0 || N % 16 != 0 || epi < 0 || epi > 3) return 1;
   if ((epi == EPI_SILU || epi == EPI_ROPE) && (N / 16) % 2) return 1;
   if (epi == EPI_RESID && !a.resid) return 1;
+  if (M > 16 && epi == EPI_PLAIN && !norm && nt <= 0 && waves <= 0 && splits <= 0) {
+    const int rc = dispatch_rows(a, st);
+    if (rc <= 0) return rc;
+  }
   const int MT = M <= 16 ? 1 : (M <= 32 ? 2 : 4);
   int dn, dw, dS;
   default_cfg(MT, M, N, a.K, epi, dn, dw, dS);
@@ -454,4 +603,11 @@ extern "C" int pa_decode_qkv_rope(const void* x, const void* wp, int M, int N, i
            RopeArgs{(bf16*)q_out, (bf16*)k_cache, (bf16*)v_cache, positions, slots, cos_sin, H, KV},
            1, ws, counters};
   return dispatch(a, EPI_ROPE, 1, nt, waves, splits, ws_floats, n_counters, st);
+}
+
+// y = x W^T for any number of rows whose tiles leave one workgroup a CU (and up to 64 always); 1 if not.
+extern "C" int pa_rows_gemm(void* y, const void* x, const void* wp, int M, int N, int K, int ldx, int ldy, hipStream_t st) {
+  using namespace pa;
+  DgArgs a{(bf16*)y, (const bf16*)x, (const bf16*)wp, nullptr, M, N, K, ldx, ldy, 0, 0.f, RopeArgs{}, 1, nullptr, nullptr};
+  return dispatch_rows(a, st);
 }

@@ -482,6 +482,18 @@ def decode_gemm(x: torch.Tensor, wp: torch.Tensor, epi: str = "plain", norm: boo
     return out
 
 
+def rows_gemm(x: torch.Tensor, wp: torch.Tensor, out: Optional[torch.Tensor] = None) -> Optional[torch.Tensor]:
+    """y = x W^T with W packed by pack_decode_weight, for as many rows as leave the kernel's tiles one workgroup a CU
+    (csrc/ops/gemm_decode.hip dispatch_rows); None beyond."""
+    M, N = x.shape[0], wp.shape[0] * 16
+    if M > 64 and -(-M // 64) * -(-N // 128) > 256:
+        return None
+    if not _on_gpu(x):
+        return decode_gemm(x, wp, out=out)
+    y = out if out is not None else torch.empty(M, N, dtype=x.dtype, device=x.device)
+    return y if _packed_module().rows_gemm(y, x, wp) else None
+
+
 # per-head tile order of the rope-fused QKV weights: tiles (i, i + 4) adjacent
 _ROPE_TILE_ORDER = (0, 4, 1, 5, 2, 6, 3, 7)
 

@@ -371,6 +371,25 @@ def test_decode_gemm(gpu, M, N, K, epi, norm):
         torch.testing.assert_close(r2, y, atol=0, rtol=0)
 
 
+@pytest.mark.parametrize("M,N,K", [
+    (17, 16, 32), (32, 4096, 96), (33, 2048, 544), (64, 2048, 8192), (64, 128256, 64), (31, 40_960, 160),  # up to 64 rows
+    (65, 2064, 512), (96, 10368, 2048), (129, 4112, 1056), (512, 2048, 768), (1000, 1040, 64)])             # and more
+def test_rows_gemm(gpu, M, N, K):
+    """Every tile of dispatch_rows, at its edges: rows and columns past the tiles, k past the last stage. A bf16 result
+    rounds by 2^-8 of itself at most, and a sum of K products in fp32 errs by K 2^-24 of their magnitudes at most."""
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, device=gpu, generator=g).bfloat16()[:, :K]
+    w = torch.randn(N, K, device=gpu, generator=g).bfloat16()
+    buf = torch.full((M, N + 4), 7.0, device=gpu, dtype=torch.bfloat16)
+    y = ops.rows_gemm(x, ops.pack_decode_weight(w), out=buf[:, :N])
+    assert y is not None
+    ref, size = x.float() @ w.float().T, x.float().abs() @ w.float().abs().T
+    assert bool(((y.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + K * 2.0 ** -24 * size).all())
+    assert bool((buf[:, N:] == 7.0).all())
+    assert ops.rows_gemm(torch.empty(513, 64, device=gpu, dtype=torch.bfloat16),
+                         ops.pack_decode_weight(torch.zeros(4096, 64, device=gpu, dtype=torch.bfloat16))) is None
+
+
 @pytest.mark.parametrize("nt,waves,splits", [(1, 8, 1), (1, 16, 1), (2, 8, 1), (2, 16, 1), (4, 8, 1), (4, 16, 1),
                                              (2, 8, 4), (4, 8, 2), (1, 16, 3), (2, 4, 8)])
 def test_decode_gemm_configs(gpu, nt, waves, splits):
