@@ -8,9 +8,8 @@
 // Weights are packed per group like the other projections ([N/16, K/32, 64, 8], one 16-B lane
 // vector per MFMA operand). The MFMA's A operand is W and its B operand x, so a lane's four
 // accumulators are four consecutive outputs of one row: 8-byte stores, and the gated pair
-// (tiles 2i: gate, 2i + 1: up) is lane-local. Tiles of 16 rows stream the weights (decode steps); 64
-// rows share them; prompts with 256 rows and more per group run the ping-pong kernels instead
-// (gemm_prefill.hip pa_expert_tiles).
+// (tiles 2i: gate, 2i + 1: up) is lane-local. Sorted rows go in tiles of 16 to 128, as many as a group
+// has on average; prompts with more run the ping-pong kernels instead (gemm_prefill.hip pa_expert_tiles).
 //
 // Epilogues: plain, the gated unit of packed_epi.h (limit, alpha, cubic, bias), or the square of relu; of dense rows
 // also the product times sigmoid(gate), and the gated unit whose second factor is the row's embedding in a table.
@@ -117,22 +116,12 @@ __device__ __forceinline__ float times(float a, float f, const Args& A) {
   return glu(a, f, A);
 }
 
+// Dense rows: tiles of 16 MT rows and 16 NT outputs a wave (PLAIN, GATED).
 template <int MT, int NT, int KU, int EPI>
 __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int c = lane & 15, g = lane >> 4;
-  int grp, start, n;
-  if (A.tiles) {
-    if ((int)blockIdx.y >= A.n_tiles[0]) return;
-    const int4 tl = A.tiles[blockIdx.y];
-    grp = tl.x;
-    start = tl.y;
-    n = tl.z;
-  } else {
-    grp = blockIdx.z;
-    start = blockIdx.y * (16 * MT);
-    n = min(16 * MT, A.rows - start);
-  }
+  const int grp = blockIdx.z, start = blockIdx.y * (16 * MT), n = min(16 * MT, A.rows - start);
   if (A.rp && blockIdx.x == 0) {
     rotate_rows<bf16>(A, grp, start, n);
     return;
@@ -149,9 +138,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
   for (int m = 0; m < MT; ++m) {
     const int i = min(16 * m + c, n - 1);
     pos[m] = start + i;
-    int row = pos[m];
-    if (A.tiles && A.x_div) row = A.order[pos[m]] / A.x_div;
-    xr[m] = (const bf16*)A.x + (size_t)row * A.ldx + (A.tiles ? 0 : (size_t)grp * A.xg) + 8 * g;
+    xr[m] = (const bf16*)A.x + (size_t)pos[m] * A.ldx + (size_t)grp * A.xg + 8 * g;
   }
   f32x4 acc[MT][NT];
 #pragma unroll
@@ -190,19 +177,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
     if (16 * m + c >= n) continue;
-    const int orow = (A.tiles && A.out_order) ? A.order[pos[m]] : pos[m];
-    bf16* o = (bf16*)A.out + (size_t)orow * A.ldo + (A.tiles ? 0 : (size_t)grp * A.og) + 4 * g;
-    if constexpr (EPI == GLU) {
-      const float rw = A.row_w ? A.row_w[A.order[pos[m]]] : 1.f;
-#pragma unroll
-      for (int i = 0; i + 1 < NT; i += 2) {
-        if (nt0 + i >= A.N16) break;
-        bf16x4 v;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = (bf16)glu(acc[m][i][j] * rw, acc[m][i + 1][j] * rw, A);
-        *reinterpret_cast<bf16x4*>(o + (nt0 + i) * 8) = v;
-      }
-    } else if constexpr (EPI == GATED) {
+    bf16* o = (bf16*)A.out + (size_t)pos[m] * A.ldo + (size_t)grp * A.og + 4 * g;
+    if constexpr (EPI == GATED) {
       const bf16* f = factor_row<bf16, EPI>(A, pos[m], grp) + 4 * g;
 #pragma unroll
       for (int i = 0; i < NT; ++i) {
@@ -219,7 +195,7 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
 #pragma unroll
       for (int i = 0; i + 1 < NT; i += 2) {
         if (nt0 + i >= A.N16) break;
-        pk::store_pair_wide<EPI == RELU2 ? pk::EP_RELU2 : pk::EP_PLAIN>(row, 0, nt0 + i, g, acc[m][i], acc[m][i + 1]);
+        pk::store_pair_wide<pk::EP_PLAIN>(row, 0, nt0 + i, g, acc[m][i], acc[m][i + 1]);
       }
     } else {
 #pragma unroll
@@ -227,11 +203,197 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
         if (nt0 + i >= A.N16) break;
         bf16x4 v;
 #pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = (bf16)(EPI == RELU2 ? pk::relu2(acc[m][i][j]) : acc[m][i][j]);
+        for (int j = 0; j < 4; ++j) v[j] = (bf16)acc[m][i][j];
         *reinterpret_cast<bf16x4*>(o + (nt0 + i) * 16) = v;
       }
     }
   }
+}
+
+// Sorted rows in tiles of 16 MT = 16 to 128: the rows of a group go through its weights together, so that these leave
+// memory once. A workgroup loads its rows (wherever they lie) in whole lines, 64 WK k a stage, and its waves read the
+// fragments from LDS: a wave's own fragment loads, 16 rows x 64 B an instruction, cost more than the weights. 8 waves lie
+// side by side over a pair of 16-output tiles each; with WK > 1, WK of them share one pair and split the k-steps of a
+// stage, which leaves more workgroups. Weights and rows are one in-order ring of loads, D stages deep; the stage barrier
+// waits for LDS alone. NTW: weights that no other tile reads are loaded non-temporal.
+// Bound by the weights' bytes up to 128 rows a group: 64 experts of 2 x 1408 x 2048 and 2048 x 1408 and a shared one,
+// both products, us before -> after: 64 tokens 215 -> 182 (5.4 TB/s), 400 275 -> 228, 750 414 -> 284, 1000 456 -> 295; a
+// dense 2 x 8192 x 2048 gate and up of 64 rows 30 -> 17, of 256 rows 45 -> 33.
+template <int MT, int WK, int EPI, bool NTW>
+__global__ __launch_bounds__(512, MT == 8 ? 4 : 2) void rows_kernel(const Args A) {
+  constexpr int WN = 8 / WK, NT = 2, KW = 2, D = 2;
+  constexpr int TM = 16 * MT, KC = 64 * WK, XLD = KC * 2 + 16;
+  constexpr int LR = KC / 8, RL = 512 / LR, XL = (TM + RL - 1) / RL;  // threads a row, rows a load, loads a stage
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // [2][TM][XLD], then the partial sums
+  // A group's tiles read the same weights: the same block of outputs of each goes to one XCD, in turn, and finds them in
+  // its L2 (the first block's XCD moves with the group, so that all have as many). Not with the 11 blocks or so of WK =
+  // 1, which do not divide over 8 XCDs, and where most groups have one tile.
+  const int blocks = (A.N16 + WN * NT - 1) / (WN * NT);
+  int tile, block;
+  if constexpr (WK == 1) {
+    tile = blockIdx.x / blocks;
+    block = blockIdx.x % blocks;
+  } else {
+    const int b8 = (blocks + 7) >> 3, seq = blockIdx.x >> 3;
+    tile = seq / b8;
+    block = seq % b8 * 8;
+  }
+  if (tile >= A.n_tiles[0]) return;
+  const int4 tl = A.tiles[tile];
+  const int grp = tl.x, start = tl.y, n = tl.z;
+  if (WK > 1) block += (blockIdx.x + grp) & 7;
+  if (block >= blocks) return;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, c = lane & 15, g = lane >> 4;
+  const int wk = wid % WK, wn = wid / WK, xrow = threadIdx.x / LR, xu = threadIdx.x % LR;
+  const int nt0 = (block * WN + wn) * NT, KS = A.K32, nst = (KS * 32 + KC - 1) / KC;
+  const bf16x8* wt[NT];
+#pragma unroll
+  for (int j = 0; j < NT; ++j)
+    wt[j] = reinterpret_cast<const bf16x8*>((const bf16*)A.w + (size_t)grp * A.wstride +
+                                            (size_t)min(nt0 + j, A.N16 - 1) * KS * 512) + lane;
+  const bf16* xr[XL];
+#pragma unroll
+  for (int i = 0; i < XL; ++i) {
+    const int pos = start + min(xrow + RL * i, n - 1);
+    xr[i] = (const bf16*)A.x + (size_t)(A.x_div ? A.order[pos] / A.x_div : pos) * A.ldx;
+  }
+  f32x4 acc[MT][NT];
+#pragma unroll
+  for (int m = 0; m < MT; ++m)
+#pragma unroll
+    for (int j = 0; j < NT; ++j) acc[m][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  bf16x8 wb[D][KW][NT], xb[D][XL];
+  // (past the end: the last ones again, unconditional, so that the waits stay counted)
+  auto load = [&](int st, int d) {
+    __builtin_amdgcn_sched_barrier(0);
+    const int k = min(st * KC + 8 * xu, KS * 32 - 8);
+#pragma unroll
+    for (int i = 0; i < XL; ++i) xb[d][i] = *reinterpret_cast<const bf16x8*>(xr[i] + k);
+#pragma unroll
+    for (int u = 0; u < KW; ++u) {
+      const int ks = min(st * (KC / 32) + wk * KW + u, KS - 1);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        if constexpr (NTW) wb[d][u][j] = __builtin_nontemporal_load(wt[j] + (size_t)ks * 64);
+        else wb[d][u][j] = wt[j][(size_t)ks * 64];
+      }
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+#pragma unroll
+  for (int d = 0; d < D; ++d) load(d, d);
+  for (int st0 = 0; st0 < nst; st0 += D) {
+#pragma unroll
+    for (int d = 0; d < D; ++d) {
+      const int st = st0 + d;
+      if (st < nst) {  // uniform
+        char* slot = smem + (st & 1) * TM * XLD;
+#pragma unroll
+        for (int i = 0; i < XL; ++i)
+          if (TM % RL == 0 || xrow + RL * i < TM)
+            *reinterpret_cast<bf16x8*>(slot + (xrow + RL * i) * XLD + 16 * xu) = xb[d][i];
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+#pragma unroll
+        for (int u = 0; u < KW; ++u) {
+          if (st * (KC / 32) + wk * KW + u < KS) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+              const bf16x8 b = *reinterpret_cast<const bf16x8*>(slot + (16 * m + c) * XLD + (wk * KW + u) * 64 + 16 * g);
+#pragma unroll
+              for (int j = 0; j < NT; ++j)
+                acc[m][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wb[d][u][j], b, acc[m][j], 0, 0, 0);
+            }
+          }
+        }
+        load(st + D, d);
+      }
+    }
+  }
+  // the pair of tiles nt of the rows 16 m + c
+  auto store = [&](int m, int nt, f32x4 v0, f32x4 v1) {
+    if (16 * m + c >= n || nt >= A.N16) return;
+    const int p = start + 16 * m + c;
+    bf16* o = (bf16*)A.out + (size_t)(A.out_order ? A.order[p] : p) * A.ldo + 4 * g;
+    if constexpr (EPI == GLU) {
+      const float rw = A.row_w ? A.row_w[A.order[p]] : 1.f;
+      bf16x4 v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = (bf16)glu(v0[j] * rw, v1[j] * rw, A);
+      *reinterpret_cast<bf16x4*>(o + nt * 8) = v;
+    } else if (A.N16 % 2 == 0 && A.wide) {
+      const struct { bf16* y; int ldy; } row{o - 4 * g, 0};
+      pk::store_pair_wide<EPI == RELU2 ? pk::EP_RELU2 : pk::EP_PLAIN>(row, 0, nt, g, v0, v1);
+    } else {
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        if (nt + i >= A.N16) break;
+        bf16x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const float a = i ? v1[j] : v0[j];
+          v[j] = (bf16)(EPI == RELU2 ? pk::relu2(a) : a);
+        }
+        *reinterpret_cast<bf16x4*>(o + (nt + i) * 16) = v;
+      }
+    }
+  };
+  if constexpr (WK == 1) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) store(m, nt0, acc[m][0], acc[m][1]);
+  } else {
+    __syncthreads();
+    f32x4* red = reinterpret_cast<f32x4*>(smem);  // [WK][WN][MT][NT][64]
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+      for (int j = 0; j < NT; ++j) red[(((wk * WN + wn) * MT + m) * NT + j) * 64 + lane] = acc[m][j];
+    __syncthreads();
+    for (int t = wid; t < WN * MT; t += 8) {
+      f32x4 v[NT];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        v[j] = red[(t * NT + j) * 64 + lane];
+#pragma unroll
+        for (int w = 1; w < WK; ++w) v[j] += red[((w * WN * MT + t) * NT + j) * 64 + lane];
+      }
+      store(t % MT, (block * WN + t / MT) * NT, v[0], v[1]);
+    }
+  }
+}
+
+template <int MT, int WK, bool NTW>
+static int launch_rows(const Args& A, int epi, int max_tiles, hipStream_t st) {
+  constexpr int TN = (8 / WK) * 32;
+  constexpr int x = 2 * 16 * MT * (128 * WK + 16), sums = WK > 1 ? 8 * MT * 2 * 1024 : 0, lds = x > sums ? x : sums;
+  static_assert(lds <= 160 * 1024, "LDS of a CU");
+  static bool attr = false;
+  if (!attr) {
+    for (auto* k : {rows_kernel<MT, WK, PLAIN, NTW>, rows_kernel<MT, WK, GLU, NTW>, rows_kernel<MT, WK, RELU2, NTW>})
+      (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    attr = true;
+  }
+  const int blocks = (A.N16 * 16 + TN - 1) / TN;
+  hipLaunchKernelGGL((epi == 1 ? rows_kernel<MT, WK, GLU, NTW> : epi == 2 ? rows_kernel<MT, WK, RELU2, NTW> : rows_kernel<MT, WK, PLAIN, NTW>),
+                     dim3((WK > 1 ? (blocks + 7) / 8 * 8 : blocks) * max_tiles), dim3(512), lds, st, A);
+  return (int)hipGetLastError();
+}
+
+// Waves over k (WK): 4 for few rows; with 64-row tiles of many groups 2 (T = 400: 228 us both products, 4: 246, 1: 254),
+// with those of one group as many as leave at most two workgroups a CU (2 x 8192 x 2048 outputs of 128 rows: 4 26 us, of 256: 2
+// 33 us, 4 45; of 512: 1 46 us, 2 57); 1 with 128 rows, whose accumulators fill a wave. Non-temporal weights where
+// no more than every third tile is a group's second (64 tokens 192 -> 182 us; 400 tokens 240 -> 250).
+static int sorted_rows(const Args& A, int epi, int tm, int groups, int max_tiles, hipStream_t st) {
+  const bool once = (max_tiles - groups) * 2 <= groups;
+  auto fits = [&](int wk) { return (A.N16 * 16 + 256 / wk - 1) / (256 / wk) * max_tiles <= 512; };
+  if (tm == 16) return once ? launch_rows<1, 4, true>(A, epi, max_tiles, st) : launch_rows<1, 4, false>(A, epi, max_tiles, st);
+  if (tm == 32) return once ? launch_rows<2, 4, true>(A, epi, max_tiles, st) : launch_rows<2, 4, false>(A, epi, max_tiles, st);
+  if (tm == 128) return launch_rows<8, 1, false>(A, epi, max_tiles, st);
+  if (tm != 64) return -2;
+  if (groups == 1 && fits(4)) return once ? launch_rows<4, 4, true>(A, epi, max_tiles, st) : launch_rows<4, 4, false>(A, epi, max_tiles, st);
+  if (groups == 1 && !fits(2)) return launch_rows<4, 1, false>(A, epi, max_tiles, st);
+  return launch_rows<4, 2, false>(A, epi, max_tiles, st);
 }
 
 // Dense rows through one group of few outputs (TABLE): 8 waves share a tile of 16 MT rows and 16 NT outputs, each every
@@ -429,7 +591,7 @@ extern "C" int pa_table_route(const int* tables, const int* desc, int layers, co
   return (int)hipGetLastError();
 }
 
-// tm: rows per sorted tile (16, 64 or 256; dense: the kernel's choice by row count)
+// tm: rows per sorted tile (16, 32, 64, 128 or 256; dense: the kernel's choice by row count)
 extern "C" int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out, long long wstride, int groups,
                                int ldx, int xg, int ldo, int og, int rows, int N16, int K32, const int* tiles,
                                int max_tiles, const int* n_tiles, const int* order, int x_div, int out_order, int tm,
@@ -477,14 +639,12 @@ extern "C" int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out
 #undef PA_SK
     return (int)hipGetLastError();
   }
+  if (tiles) return pa::gg::sorted_rows(A, epi, tm, groups, max_tiles, st);
   // dense: 64-row tiles once they fill the chip
-  if (!tiles) tm = (N16 + 15) / 16 * ((rows + 63) / 64) * groups < 256 ? 16 : 64;
-  if (tm != 16 && tm != 64) return -2;
+  tm = (N16 + 15) / 16 * ((rows + 63) / 64) * groups < 256 ? 16 : 64;
 #define PA_GG(MT, NT, KU, G)                                                                                   \
   hipLaunchKernelGGL((pa::gg::gemm_kernel<MT, NT, KU, G>),                                                     \
-                     dim3((N16 + 4 * NT - 1) / (4 * NT) + rot, tiles ? max_tiles : (rows + 16 * MT - 1) / (16 * MT), \
-                          tiles ? 1 : groups),                                                                 \
-                     dim3(256), 0, st, A)
+                     dim3((N16 + 4 * NT - 1) / (4 * NT) + rot, (rows + 16 * MT - 1) / (16 * MT), groups), dim3(256), 0, st, A)
 #define PA_GGK(MT, NT, G)                      \
   do {                                         \
     if (K32 % 4 == 0) PA_GG(MT, NT, 4, G);     \
@@ -492,14 +652,10 @@ extern "C" int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out
     else PA_GG(MT, NT, 1, G);                  \
   } while (0)
   if (tm == 16) {
-    if (epi == 1) PA_GGK(1, 2, pa::gg::GLU);
-    else if (epi == 2) PA_GGK(1, 1, pa::gg::RELU2);
-    else if (epi == 3) PA_GGK(1, 1, pa::gg::GATED);
+    if (epi == 3) PA_GGK(1, 1, pa::gg::GATED);
     else PA_GGK(1, 1, pa::gg::PLAIN);
   } else {
-    if (epi == 1) PA_GG(4, 4, 1, pa::gg::GLU);
-    else if (epi == 2) PA_GG(4, 4, 1, pa::gg::RELU2);
-    else if (epi == 3) PA_GG(4, 4, 1, pa::gg::GATED);
+    if (epi == 3) PA_GG(4, 4, 1, pa::gg::GATED);
     else PA_GG(4, 4, 1, pa::gg::PLAIN);
   }
 #undef PA_GGK

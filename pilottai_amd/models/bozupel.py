@@ -182,9 +182,6 @@ class BozupelModel:
     PREFILL_MAX_T = 1 << 30
     ATT_DECODE_WAVES = 4
     PF_MIDRANGE = frozenset()
-    # average rows per expert above which an expert's rows go in tiles of 64 / 256
-    EXPERT_ROWS_64 = 32
-    EXPERT_ROWS_256 = 96
     decode_packed = True
     KERNELS = "latent"  # the module of its kernels (_build.py)
 
@@ -305,7 +302,7 @@ class BozupelModel:
             per = T * max(p.top / p.experts for p in mlps)  # rows an expert gets on average
             rows, tab, o, t = [], 0, 0, 0
             min_k = min([L["mlp"].fp for L in self.layers if L["mlp"]] + [pad_to(self.cfg.hidden_size, 64)])
-            tm = expert_tile_rows(per, self.dtype, min_k, self.EXPERT_ROWS_64, self.EXPERT_ROWS_256)
+            tm = expert_tile_rows(per, self.dtype, min_k)
             for p in mlps:
                 n = T * p.top
                 cap = n // tm + min(p.experts, n)

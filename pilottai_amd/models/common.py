@@ -83,9 +83,18 @@ def layer_runs(layers: int, loop: Optional[Tuple[int, int, int]]) -> List[Tuple[
     return out + [(i, False) for i in range(stop, layers)]
 
 
-def expert_tile_rows(rows: float, dtype, min_k: int, above_64: int, above_256: int) -> int:
-    """Rows per sorted tile of the grouped projections: 16 streams the weights, 64 shares them, 256 runs the
-    ping-pong kernels (bf16, every K of at least 128), by the rows an expert gets on average."""
-    if dtype != torch.bfloat16 or rows <= above_64:
+# (most rows a group has on average, rows per sorted tile) of the grouped projections: the fewest that hold a group's rows,
+# with room for uneven groups, so that its weights are read once; above, 256 (the ping-pong kernels). 64 experts of 3 x 1408
+# x 2048 and a shared one, us for both products: 6 rows an expert 16: 182, 32: 191; 19 rows 32: 209, 16: 231, 64: 222; 56 rows 64: 238,
+# 128: 295; 94 rows 128: 295, 64: 320, 256: 329; 150 rows 256: 373, 128: 462.
+GROUP_TILES = ((10, 16), (24, 32), (72, 64), (128, 128))
+# of one group: 64 rows share the weights through the caches of an XCD up to 448 rows (2 x 8192 x 2048: 42 us at 384 rows, 256-row
+# tiles 45), with weights above 128 MB up to 128 (2 x 14336 x 4096: 67 us, 82; 256 rows 89, 83)
+ONE_GROUP_TILES, ONE_LARGE_GROUP_TILES = ((16, 16), (32, 32), (448, 64)), ((16, 16), (32, 32), (128, 64))
+
+
+def expert_tile_rows(rows: float, dtype, min_k: int, steps=GROUP_TILES) -> int:
+    """Rows per sorted tile by the rows a group gets on average (fp32: 16; the 256-row kernels take every K of 128 on)."""
+    if dtype != torch.bfloat16:
         return 16
-    return 256 if min_k >= 128 and rows > above_256 else 64
+    return next((tm for most, tm in steps if rows <= most), 256 if min_k >= 128 else steps[-1][1])

@@ -21,7 +21,8 @@ import torch
 
 from pilottai_amd import ops
 from pilottai_amd.models.cache import HybridCache, StepMeta
-from pilottai_amd.models.common import PackedLinear, checkpoint_reader, expert_tile_rows
+from pilottai_amd.models.common import (ONE_GROUP_TILES, ONE_LARGE_GROUP_TILES, PackedLinear, checkpoint_reader,
+                                         expert_tile_rows)
 from pilottai_amd.ops.latent import pad_to
 from pilottai_amd.parallel.comm import TPGroup
 
@@ -502,8 +503,7 @@ def _pack_gate_up(gate, up, fp: int, dk: int, dtype, device):
 class GatedMLP:
     """down(act(gate h) * up h): the gate and up rows interleaved in one grouped projection of one group."""
 
-    # 16-row tiles (each streams the weights) up to this many rows, by weights that passes find in the caches again
-    ROWS_16, ROWS_16_LARGE, LARGE = 80, 40, 1 << 26
+    LARGE = 1 << 26  # elements of weights that the next tile does not find in the caches again
 
     def __init__(self, spec: DenseSpec, t: Dict[str, torch.Tensor], width: int, dtype, device, alone: bool = True):
         self.spec, self.dtype, self.device = spec, dtype, device
@@ -519,8 +519,8 @@ class GatedMLP:
     def activate(self, h, act):
         T = h.shape[0]
         if T not in self._tiles:  # (before graph capture: the capture's warm-up runs come first)
-            few = self.ROWS_16 if self.w13.numel() <= self.LARGE else self.ROWS_16_LARGE
-            tm = expert_tile_rows(T, self.dtype, self.dk, few, few)
+            tm = expert_tile_rows(T, self.dtype, self.dk,
+                                  ONE_GROUP_TILES if self.w13.numel() <= self.LARGE else ONE_LARGE_GROUP_TILES)
             tiles = torch.tensor([[0, i, min(tm, T - i), 0] for i in range(0, T, tm)], dtype=torch.int32)
             self._tiles[T] = (tiles.to(self.device), torch.tensor([len(tiles)], dtype=torch.int32, device=self.device),
                               torch.arange(T, dtype=torch.int32, device=self.device), tm)
@@ -552,8 +552,6 @@ class PolyMLP:
 class ScoredExperts:
     """Experts chosen by the scores of a router, and a shared expert whose pieces are further experts that
     every token uses; one partial output per (token, expert) with its weight."""
-
-    ROWS_64, ROWS_256 = 32, 96  # average rows per expert above which they go in tiles of 64 / 256
 
     def __init__(self, spec: ScoredExpertsSpec, t: Dict[str, torch.Tensor], width: int, dtype, device):
         s = self.spec = spec
@@ -590,7 +588,7 @@ class ScoredExperts:
     def __call__(self, h, meta: StepMeta):
         s, T, dev = self.spec, h.shape[0], self.device
         E, K = s.experts + s.always, s.top + s.always
-        tm = expert_tile_rows(T * s.top / s.experts, self.dtype, min(self.fp, self.dk), self.ROWS_64, self.ROWS_256)
+        tm = expert_tile_rows(T * s.top / s.experts, self.dtype, min(self.fp, self.dk))
         rows = T * K
         ints = lambda *n: torch.empty(*n, dtype=torch.int32, device=dev)  # noqa: E731
         weights = torch.empty(T, K, dtype=torch.float32, device=dev)

@@ -108,6 +108,57 @@ def test_table_experts(gpu, dt, tm, T, E, top, ff, D):
             torch.testing.assert_close(y[t, k], (a * torch.sigmoid(1.702 * a) * (u + 1)) @ w2[e].float().T, **tol(dt))
 
 
+@pytest.mark.parametrize("tm", [16, 32, 64, 128])
+@pytest.mark.parametrize("counts,N,K", [
+    ([1, 0, 16, 17, 40, 130, 3], 96, 96),       # empty and single-row groups, remainders of every tile, k past no stage's end
+    ([5, 33], 80, 2048), ([200] * 3, 2816, 32),  # an odd number of 16-row blocks; more blocks than XCDs
+    ([7], 16384, 64), ([100], 16384, 320), ([300], 4096, 160), ([300], 16384, 96)])  # one group: 4, 2 and 1 waves over k
+def test_sorted_rows(gpu, tm, counts, N, K):
+    """The grouped projections of sorted rows at every tile size: plain, the square of relu and gated with weights of rows,
+    gathered and scattered. Sums of K products in fp32 err by K 2^-24 of their magnitudes at most, a bf16 result rounds by
+    2^-8; silu(g) u moves by at most 1.1 |u| dg + |g| du."""
+    from pilottai_amd import ops
+
+    g = torch.Generator(device=gpu).manual_seed(N + K + len(counts))
+    rnd = lambda *s: torch.randn(*s, device=gpu, generator=g)  # noqa: E731
+    G, rows, top = len(counts), sum(counts), 2
+    T = (rows + top - 1) // top
+    x, w = rnd(T, K + 8).bfloat16()[:, :K], (rnd(G, N, K) / math.sqrt(K)).bfloat16()
+    order = torch.randperm(T * top, device=gpu, generator=g)[:rows].int()
+    tl, p = [], 0
+    for e, n in enumerate(counts):
+        tl += [[e, p + i, min(tm, n - i), 0] for i in range(0, n, tm)]
+        p += n
+    nt = torch.tensor([len(tl)], dtype=torch.int32, device=gpu)
+    cap = rows // tm + min(G, rows)
+    assert len(tl) <= cap
+    tiles = torch.tensor(tl + [[0, 0, 0, 0]] * (cap - len(tl)), dtype=torch.int32, device=gpu)
+    of = torch.repeat_interleave(torch.arange(G, device=gpu), torch.tensor(counts, device=gpu))
+    xs = x.float()[order.long() // top]
+    z, size = torch.empty(rows, N, device=gpu), torch.empty(rows, N, device=gpu)
+    for e in range(G):
+        z[of == e], size[of == e] = xs[of == e] @ w[e].float().T, xs[of == e].abs() @ w[e].float().abs().T
+    slack = K * 2.0 ** -24 * size
+    pw, args = ops.pack_groups(w, torch.bfloat16), (tiles, nt, order, rows)
+    out = torch.full((T * top, N + 8), 9.0, dtype=torch.bfloat16, device=gpu)
+    for relu2 in (False, True):
+        want = z.clamp(min=0) ** 2 if relu2 else z
+        err = 2.0 ** -8 * want.abs() + slack * ((2 * z.abs() + slack) if relu2 else 1)
+        ops.expert_gemm(x, pw, out[:, :N], *args, x_div=top, out_order=True, tm=tm, relu2=relu2)
+        assert bool(((out[order.long(), :N].float() - want).abs() <= err).all()) and bool((out[:, N:] == 9.0).all())
+    if N % 32:
+        return
+    rw = torch.rand(T * top, device=gpu, generator=g) + 0.5
+    zg = z.view(rows, N // 32, 2, 16) * rw[order.long(), None, None, None]
+    sl = slack.view(rows, N // 32, 2, 16) * rw[order.long(), None, None, None] + 2.0 ** -22 * zg.abs()
+    a, u = zg[:, :, 0], zg[:, :, 1]
+    want = torch.nn.functional.silu(a) * u
+    err = 2.0 ** -8 * want.abs() + 1.1 * u.abs() * sl[:, :, 0] + a.abs() * sl[:, :, 1] + 2.0 ** -20 * want.abs() + 1e-30
+    out = torch.empty(rows, N // 2, dtype=torch.bfloat16, device=gpu)
+    ops.expert_gemm(x, pw, out, *args, x_div=top, out_order=False, tm=tm, glu=(3e38, 1.0, 0.0), row_w=rw)
+    assert bool(((out.float() - want.reshape(rows, -1)).abs() <= err.reshape(rows, -1)).all())
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("NQ,R,r,rd,H", [(72, 104, 48, 48, 3), (50, 70, 24, 12, 5), (256, 512, 64, 64, 2)])
 def test_latent_cache_and_query_rotation(gpu, dt, NQ, R, r, rd, H):
