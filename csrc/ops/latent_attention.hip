@@ -346,11 +346,8 @@ __device__ __forceinline__ void tile_item(const Args& A, const int4 it, char* sm
   const size_t row0 = (size_t)(A.q_start[s] + qb) * A.H;
   const int* bt = A.block_table + (size_t)s * A.max_blocks;
   int ci[CT], cpos[CT], klo[CT];
-  // the widest rows keep their rotated part's queries in LDS (lane-private, above the key tiles)
-  constexpr int NQ = NK > 17 ? RT : NK;
   const int loff = (g * 16 + c) * 16;
-  char* qs = smem + 2 * TILE + wid * (CT * (NK - NQ) * 1024) + loff;
-  bf16x8 qf[CT][NQ];
+  bf16x8 qf[CT][NK];
 #pragma unroll
   for (int t = 0; t < CT; ++t) {
     ci[t] = cw + (wid * CT + t) * 16 + c;
@@ -358,11 +355,8 @@ __device__ __forceinline__ void tile_item(const Args& A, const int4 it, char* sm
     cpos[t] = pos0 + cc / A.H;
     klo[t] = A.window > 0 ? max(0, cpos[t] - A.window + 1) : 0;
 #pragma unroll
-    for (int m = 0; m < NK; ++m) {
-      const bf16x8 v = *reinterpret_cast<const bf16x8*>((const bf16*)A.q + (row0 + cc) * D + 32 * m + 8 * g);
-      if (m < NQ) qf[t][m] = v;
-      else *reinterpret_cast<bf16x8*>(qs + (t * (NK - NQ) + m - NQ) * 1024) = v;
-    }
+    for (int m = 0; m < NK; ++m)
+      qf[t][m] = *reinterpret_cast<const bf16x8*>((const bf16*)A.q + (row0 + cc) * D + 32 * m + 8 * g);
   }
   // positions of the workgroup's columns -> its key tiles
   const int f = pos0 + cw / A.H, e = pos0 + min(cw + 16 * NW * CT - 1, cols - 1) / A.H;
@@ -420,11 +414,7 @@ __device__ __forceinline__ void tile_item(const Args& A, const int4 it, char* sm
       for (int k = 0; k < 2; ++k) {
         const bf16x8 kf = *reinterpret_cast<const bf16x8*>(cur + k * (D * 32) + m * 1024 + loff);
 #pragma unroll
-        for (int x = 0; x < CT; ++x) {
-          const bf16x8 q = m < NQ ? qf[x][m < NQ ? m : 0]
-                                  : *reinterpret_cast<const bf16x8*>(qs + (x * (NK - NQ) + m - NQ) * 1024);
-          sc[x][k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, q, sc[x][k], 0, 0, 0);
-        }
+        for (int x = 0; x < CT; ++x) sc[x][k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf, qf[x][m], sc[x][k], 0, 0, 0);
       }
     const bool mask = 32 * t < full_lo || 32 * t + 31 > full_hi;  // wave-uniform
     bf16x8 pf[CT];
@@ -504,9 +494,256 @@ __device__ __forceinline__ void tile_item(const Args& A, const int4 it, char* sm
   }
 }
 
+// The same for the widest latents, whose tile loop is bound by LDS reads: there every wave reads the whole tile for its own
+// 16 columns, 68 KB for 68 MFMAs. Here two waves share 32 columns. Each takes half the dimensions of the scores (its
+// half of the queries fits the registers) and half the dimensions of the outputs, of both column blocks, so a fragment
+// read serves two MFMAs: 40 KB a wave. Between the halves, a wave sends the partner its part of the
+// partner's scores and gets its own completed, does the softmax of its 16 columns, and the two trade weights. The
+// next tile's scores run ahead of this tile's outputs (three tile buffers), so softmax and outputs overlap.
+// 4,096 tokens, 16 heads, 512 + 64: 493 -> 380 us; the MFMAs alone, at 2,176 cycles a tile and CU, 116 us.
+// What is left is the wait at each tile's barriers, with one workgroup a CU.
+template <int RT, int PT>
+constexpr int pair_lds_bytes() { return 3 * 32 * 32 * (RT + PT) * 2 + NW * (2048 + 2 * (1024 + 64) + (RT >= 16 ? 2048 : 0)); }
+
+template <int RT, int PT>
+__device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* smem) {
+  constexpr int NK = RT + PT, NH = (NK + 1) / 2, D = 32 * NK, RP = 32 * RT, TILE = 32 * D * 2;
+  const int s = it.x, qb = it.y, nq = it.z & 0xff, part = (it.z >> 8) & 0xfff, nparts = it.z >> 20;
+  const int cols = nq * A.H, cw = blockIdx.x * (16 * NW);
+  if (cw >= cols) return;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, g = lane >> 4, c = lane & 15;
+  const int half = __builtin_amdgcn_readfirstlane(wid & 1);
+  const int ctx = A.ctx_len[s], ql = A.q_len[s];
+  const int pos0 = ctx - ql + qb;
+  const size_t row0 = (size_t)(A.q_start[s] + qb) * A.H;
+  const int* bt = A.block_table + (size_t)s * A.max_blocks;
+  // column block 0: this wave's own, 1: the partner's
+  auto col = [&](int x) { return cw + (x ? wid ^ 1 : wid) * 16 + c; };
+  const int cpos = pos0 + min(col(0), cols - 1) / A.H;
+  const int klo = A.window > 0 ? max(0, cpos - A.window + 1) : 0;
+  const int loff = (g * 16 + c) * 16;
+  // (the widest keep the queries of a wave's last step in LDS: with them in registers the tile loop spills)
+  constexpr int NQ = RT >= 16 ? NH - 1 : NH;
+  char* qs = smem + 3 * TILE + NW * (2048 + 2 * (1024 + 64)) + wid * 2048 + loff;
+  bf16x8 qf[2][NQ];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int m = 0; m < NH; ++m) {
+      const int mm = half * NH + m;
+      const bf16* src = (const bf16*)A.q + (row0 + min(col(x), cols - 1)) * D + 32 * min(mm, NK - 1) + 8 * g;
+      bf16x8 v = *reinterpret_cast<const bf16x8*>(src);
+      if (2 * NH != NK && mm >= NK) v = bf16x8{};  // (an odd number of steps: none is left for the second half)
+      if (m < NQ) qf[x][m < NQ ? m : 0] = v;
+      else *reinterpret_cast<bf16x8*>(qs + x * 1024) = v;
+    }
+  const int f = pos0 + cw / A.H, e = pos0 + min(cw + 16 * NW - 1, cols - 1) / A.H;
+  int t_lo = (A.window > 0 ? max(0, f - A.window + 1) : 0) >> 5, t_hi = (e + 32) >> 5;
+  if (nparts > 1) {  // this partition's tiles (possibly none)
+    const int per = (t_hi - t_lo + nparts - 1) / nparts;
+    t_lo += part * per;
+    t_hi = min(t_hi, t_lo + per);
+  }
+  const int nblk = (ctx + 15) >> 4, n_t = t_hi - t_lo;
+  // (t needs no mask when every column of the wave sees all its 32 keys)
+  const int wf = pos0 + min(cw + wid * 16, cols - 1) / A.H, we = pos0 + min(cw + wid * 16 + 15, cols - 1) / A.H;
+  const int full_lo = A.window > 0 ? we - A.window + 1 : 0, full_hi = wf;
+
+  f32x4 o[2][RT];
+#pragma unroll
+  for (int x = 0; x < 2; ++x)
+#pragma unroll
+    for (int n = 0; n < RT; ++n) o[x][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float m_run = NEG_BIG, l_run = 0.f;
+  char* xs = smem + 3 * TILE;                                    // [NW][2][1 KB] scores for the partner
+  char* xp = xs + NW * 2048;                                     // [2][NW][1 KB] weights, of tiles in turn
+  float* xa = reinterpret_cast<float*>(xp + 2 * NW * 1024);      // [2][NW][16] factors of the outputs so far
+  // page ids, 64 at a time, a lane each: read where they are used, their latency was a stall of every tile
+  const int swid = __builtin_amdgcn_readfirstlane(wid);
+  int ids = 0, ids_at = -64;
+  auto issue = [&](int t, char* dst) {
+    if (2 * t >= ids_at + 64) {  // uniform
+      ids_at = 2 * t;
+      ids = bt[min(2 * t + lane, nblk - 1)];
+    }
+    const int i0 = __builtin_amdgcn_readlane(ids, 2 * t - ids_at), i1 = __builtin_amdgcn_readlane(ids, 2 * t + 1 - ids_at);
+    const char* src0 = (const char*)A.pages + (size_t)i0 * (D * 32);
+    const char* src1 = (const char*)A.pages + (size_t)i1 * (D * 32) - NK * 1024;
+#pragma unroll
+    for (int i = 0; i < (2 * NK + NW - 1) / NW; ++i) {
+      const int ch = i * NW + swid;
+      if (2 * NK % NW == 0 || ch < 2 * NK)
+        __builtin_amdgcn_global_load_lds((glb_void*)((ch < NK ? src0 : src1) + ch * 1024 + lane * 16),
+                                         (lds_void*)(dst + ch * 1024), 16, 0, 0);
+    }
+  };
+  const int toff = half * (RT * 512) + ((c & 3) >> 1) * 256 + (4 * g + (c >> 2)) * 16 + (c & 1) * 8;
+  f32x4 sc[2];
+  // both column blocks' scores over this half of the dimensions; the partner's go to LDS. Fragments are read AHEAD steps
+  // before their use: left to itself the compiler, short of registers, reads each right before its MFMAs.
+  constexpr int AHEAD = 2;
+  auto scores = [&](const char* tile) {
+    bf16x8 kb[AHEAD + 1];
+    auto frag = [&](int i) {
+      const int k = i / NH, m = i % NH, mm = 2 * NH == NK ? half * NH + m : min(half * NH + m, NK - 1);
+      bf16x8 v = *reinterpret_cast<const bf16x8*>(tile + k * (D * 32) + mm * 1024 + loff);
+      if (2 * NH != NK && m == NH - 1 && half) v = bf16x8{};
+      return v;
+    };
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) kb[i] = frag(i);
+    f32x4 other = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int i = 0; i < 2 * NH; ++i) {
+      const int k = i / NH, m = i % NH;
+      if (m == 0) other = sc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (i + AHEAD < 2 * NH) kb[(i + AHEAD) % (AHEAD + 1)] = frag(i + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
+      const bf16x8 q0 = m < NQ ? qf[0][m < NQ ? m : 0] : *reinterpret_cast<const bf16x8*>(qs);
+      const bf16x8 q1 = m < NQ ? qf[1][m < NQ ? m : 0] : *reinterpret_cast<const bf16x8*>(qs + 1024);
+      other = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb[i % (AHEAD + 1)], q1, other, 0, 0, 0);
+      sc[k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb[i % (AHEAD + 1)], q0, sc[k], 0, 0, 0);
+      if (m == NH - 1) *reinterpret_cast<f32x4*>(xs + (wid * 2 + k) * 1024 + lane * 16) = other;
+    }
+  };
+  // softmax of the own columns' completed scores of tile t; weights and factors to LDS
+  auto softmax = [&](int t) {
+    bf16x8 pf;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) sc[k] += *reinterpret_cast<const f32x4*>(xs + ((wid ^ 1) * 2 + k) * 1024 + lane * 16);
+    if (32 * t < full_lo || 32 * t + 31 > full_hi) {  // wave-uniform
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int key = 32 * t + 16 * k + 4 * g + r;
+          if (key > cpos || key < klo) sc[k][r] = NEG_BIG;
+        }
+    }
+    float tmax = NEG_BIG;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, sc[k][r]);
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    const float m_new = fmaxf(m_run, fmaxf(tmax * A.scale_log2, NEG_BIG));
+    const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+    m_run = m_new;
+    l_run *= alpha;
+    // a column that has seen no key yet (its window starts in a later tile): every weight is 0
+    const float nm = m_run < 0.01f * NEG_BIG ? 0.f : -m_run;
+#pragma unroll
+    for (int k = 0; k < 2; ++k)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const float p = __builtin_amdgcn_exp2f(fmaf(sc[k][r], A.scale_log2, nm));
+        l_run += p;
+        pf[4 * k + r] = (bf16)p;
+      }
+    const int at = ((t - t_lo) & 1) * NW + wid;
+    *reinterpret_cast<bf16x8*>(xp + at * 1024 + lane * 16) = pf;
+    if (g == 0) xa[at * 16 + c] = alpha;
+  };
+  auto outputs = [&](const char* tile, const bf16x8 (&p)[2]) {
+    bf16x4 v0[AHEAD + 1], v1[AHEAD + 1];
+    auto read = [&](int n) {
+      v0[n % (AHEAD + 1)] = tr_read(tile + n * 512 + toff);
+      v1[n % (AHEAD + 1)] = tr_read(tile + D * 32 + n * 512 + toff);
+    };
+#pragma unroll
+    for (int n = 0; n < AHEAD; ++n) read(n);
+#pragma unroll
+    for (int n = 0; n < RT; ++n) {
+      if (n + AHEAD < RT) read(n + AHEAD);
+      __builtin_amdgcn_sched_barrier(0);
+      bf16x8 v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[j] = v0[n % (AHEAD + 1)][j];
+        v[4 + j] = v1[n % (AHEAD + 1)][j];
+      }
+#pragma unroll
+      for (int x = 0; x < 2; ++x) o[x][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, p[x], o[x][n], 0, 0, 0);
+    }
+  };
+  auto lds_barrier = [] {  // tile loads stay in flight across it
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  auto landed = [] {  // and this one waits for them
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+  };
+  if (n_t > 0) {
+    issue(t_lo, smem);
+    landed();
+    if (n_t > 1) issue(t_lo + 1, smem + TILE);
+    scores(smem);
+    lds_barrier();
+    softmax(t_lo);
+    landed();
+  }
+  int cur = 0, nxt = 1;  // buffers of tiles i and i + 1
+  for (int i = 0; i < n_t; ++i) {
+    const int far = 3 - cur - nxt;
+    // tile i + 2 goes where i - 1 was, whose outputs everybody has done
+    if (i + 2 < n_t) issue(t_lo + i + 2, smem + far * TILE);
+    if (i + 1 < n_t) scores(smem + nxt * TILE);
+    lds_barrier();
+    const int own = (i & 1) * NW + wid, other = (i & 1) * NW + (wid ^ 1);
+    const bf16x8 p[2] = {*reinterpret_cast<const bf16x8*>(xp + own * 1024 + lane * 16),
+                         *reinterpret_cast<const bf16x8*>(xp + other * 1024 + lane * 16)};
+    const float a0 = xa[own * 16 + c], a1 = xa[other * 16 + c];
+    if (__any(a0 != 1.f || a1 != 1.f)) {
+#pragma unroll
+      for (int n = 0; n < RT; ++n) {
+        o[0][n] *= a0;
+        o[1][n] *= a1;
+      }
+    }
+    outputs(smem + cur * TILE, p);
+    if (i + 1 < n_t) softmax(t_lo + i + 1);
+    landed();
+    cur = nxt;
+    nxt = far;
+  }
+  float l = l_run;
+  l += __shfl_xor(l, 16, 64);
+  l += __shfl_xor(l, 32, 64);
+  if (g == 0) xa[wid * 16 + c] = l;
+  lds_barrier();
+  const float lx[2] = {l, xa[(wid ^ 1) * 16 + c]};
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    if (col(x) >= cols) continue;
+    if (nparts > 1) {  // 8 slots hold the item's columns in a row
+      const size_t pc = (size_t)it.w * A.NB * 16 + col(x);
+      float* po = A.part_o + pc * RP + half * (16 * RT) + 4 * g;
+#pragma unroll
+      for (int n = 0; n < RT; ++n) *reinterpret_cast<f32x4*>(po + 16 * n) = o[x][n];
+      if (x == 0 && g == 0) reinterpret_cast<float2*>(A.part_ml)[pc] = float2{m_run, l};
+      continue;
+    }
+    const float inv = 1.f / lx[x];
+    bf16* orow = (bf16*)A.out + (row0 + col(x)) * RP + half * (16 * RT) + 4 * g;
+#pragma unroll
+    for (int n = 0; n < RT; ++n) {
+      bf16x4 v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] = (bf16)(o[x][n][r] * inv);
+      *reinterpret_cast<bf16x4*>(orow + 16 * n) = v;
+    }
+  }
+}
+
+constexpr int PAIRS = 8;  // latents of 32 * PAIRS and more: pair_item
+
 template <int RT, int PT>
 constexpr int lds_bytes() {
-  return std::max({2 * 32 * 32 * (RT + PT) * 2 + (RT + PT > 17 ? NW * PT * 1024 : 0), NW * 32 * 32 * RT + 1024 * (RT + PT),
+  return std::max({RT >= PAIRS ? pair_lds_bytes<RT, PT>() : 2 * 32 * 32 * (RT + PT) * 2, NW * 32 * 32 * RT + 1024 * (RT + PT),
                    NW * 16 * MERGE_LD * 4 + 2 * NW * 16 * 4});
 }
 
@@ -514,11 +751,17 @@ template <int RT, int PT, int CT>
 __global__ __launch_bounds__(64 * NW, 2) void mfma_kernel(const Args A) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int n = A.n_items[0];
-  // two passes over the workgroup's items, so that neither path's registers carry the other's
-  for (int item = blockIdx.y; item < n; item += gridDim.y) {
+  // Two passes over the workgroup's items, so that neither path's registers carry the other's. Tiles are dealt in rounds
+  // over the workgroups, every second one from its end: a prompt's later items have more keys, and with one workgroup a CU
+  // each gets as many keys in all (dealt in one direction, CUs were busy two thirds of the time:
+  // 500 us at 4,096 tokens instead of 380).
+  for (int r = 0, b = blockIdx.y; r * (int)gridDim.y < n; ++r, b = gridDim.y - 1 - b) {
+    const int item = r * gridDim.y + b;
+    if (item >= n) continue;
     const int4 it = A.items[item];
     if ((it.z & 0xff) <= A.dec_tokens) continue;
-    tile_item<RT, PT, CT>(A, it, smem);
+    if constexpr (RT >= PAIRS) pair_item<RT, PT>(A, it, smem);
+    else tile_item<RT, PT, CT>(A, it, smem);
     __syncthreads();
   }
   for (int item = blockIdx.y; item < n; item += gridDim.y) {
@@ -567,7 +810,7 @@ extern "C" int pa_latent_attention(int fp32, void* out, float* part_o, float* pa
     }                                                                                                         \
     const int cw = 16 * pa::la::NW * CT, gt = (tile_tokens * H + cw - 1) / cw, gx = NB > gt ? NB : gt;                       \
     /* items are strided over the grid: at least one workgroup per CU */                                      \
-    const int gy = max_items < 256 ? 256 : (max_items < 4096 ? max_items : 4096);                             \
+    const int gy = R >= pa::la::PAIRS || max_items < 256 ? 256 : (max_items < 4096 ? max_items : 4096);       \
     hipLaunchKernelGGL((pa::la::mfma_kernel<R, P, CT>), dim3(gx, gy), dim3(64 * pa::la::NW), lds, st, A);     \
     hipLaunchKernelGGL((pa::la::merge_kernel<R>), dim3(16, std::min(gy, 256)), dim3(256), 0, st, A);           \
     return (int)hipGetLastError();                                                                            \
@@ -587,3 +830,4 @@ extern "C" int pa_latent_attention(int fp32, void* out, float* part_o, float* pa
   else hipLaunchKernelGGL((pa::la::simple_kernel<pa::bf16>), grid, dim3(256), lds, st, A);
   return (int)hipGetLastError();
 }
+

@@ -294,6 +294,12 @@ def test_latent_attention_split_tiles(gpu, H, R, r, window):
     run_attention(gpu, torch.bfloat16, H, R, r, [(1500, tile + 1), (900, 2 * tile + 16 // min(H, 16))], window, tiles=64, part=256)
 
 
+@pytest.mark.parametrize("R,r", [(256, 32), (512, 64)])
+def test_latent_attention_item_rounds(gpu, R, r):
+    """More items than workgroups, a round that is not full, decode rows among them."""
+    run_attention(gpu, torch.bfloat16, 16, R, r, [(0, 2100), (33, 100), (500, 1), (200, 60)], 900)
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("window", [0, 45])
 @pytest.mark.parametrize("step", ["decode", "mixed"])
