@@ -124,7 +124,8 @@ __global__ __launch_bounds__(256) void simple_kernel(const Args A) {
 // ---------------------------------------------------------------------------
 // c^T operand: lanes 16g + i of the result hold dim i of keys 4g .. 4g + 3; each lane names the
 // 8 bytes (key 4g + i/4, dims 4 (i%4) .. + 3) of the 4 x 16 block its group transposes
-__device__ __forceinline__ bf16x4 tr_read(const char* p) {
+// (restrict: an intrinsic without alias information waits for every direct load to LDS in flight)
+__device__ __forceinline__ bf16x4 tr_read(const char* __restrict__ p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)p);
 }
 
@@ -500,8 +501,9 @@ __device__ __forceinline__ void tile_item(const Args& A, const int4 it, char* sm
 // read serves two MFMAs: 40 KB a wave. Between the halves, a wave sends the partner its part of the
 // partner's scores and gets its own completed, does the softmax of its 16 columns, and the two trade weights. The
 // next tile's scores run ahead of this tile's outputs (three tile buffers), so softmax and outputs overlap.
-// 4,096 tokens, 16 heads, 512 + 64: 493 -> 380 us; the MFMAs alone, at 2,176 cycles a tile and CU, 116 us.
-// What is left is the wait at each tile's barriers, with one workgroup a CU.
+// 4,096 tokens, 16 heads, 512 + 64: 493 -> 330 us; the MFMAs alone, at 2,176 cycles a tile and CU, 116 us.
+// Left out in turn, scores, outputs, softmax and loads each give 70 to 90 us back: with two waves a SIMD and two barriers
+// a tile they overlap little. Reads 2, 3, 4 steps ahead: 365, 344, 330 us; the registers end there.
 template <int RT, int PT>
 constexpr int pair_lds_bytes() { return 3 * 32 * 32 * (RT + PT) * 2 + NW * (2048 + 2 * (1024 + 64) + (RT >= 16 ? 2048 : 0)); }
 
@@ -559,7 +561,7 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
   char* xp = xs + NW * 2048;                                     // [2][NW][1 KB] weights, of tiles in turn
   float* xa = reinterpret_cast<float*>(xp + 2 * NW * 1024);      // [2][NW][16] factors of the outputs so far
   // page ids, 64 at a time, a lane each: read where they are used, their latency was a stall of every tile
-  const int swid = __builtin_amdgcn_readfirstlane(wid);
+  const int swid = __builtin_amdgcn_readfirstlane(wid), grp = swid >> 2;
   int ids = 0, ids_at = -64;
   auto issue = [&](int t, char* dst) {
     if (2 * t >= ids_at + 64) {  // uniform
@@ -581,7 +583,7 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
   f32x4 sc[2];
   // both column blocks' scores over this half of the dimensions; the partner's go to LDS. Fragments are read AHEAD steps
   // before their use: left to itself the compiler, short of registers, reads each right before its MFMAs.
-  constexpr int AHEAD = 2;
+  constexpr int AHEAD = 4;
   auto scores = [&](const char* tile) {
     bf16x8 kb[AHEAD + 1];
     auto frag = [&](int i) {
@@ -595,6 +597,7 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
     f32x4 other = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int i = 0; i < 2 * NH; ++i) {
+      __builtin_amdgcn_sched_barrier(0);
       const int k = i / NH, m = i % NH;
       if (m == 0) other = sc[k] = f32x4{0.f, 0.f, 0.f, 0.f};
       if (i + AHEAD < 2 * NH) kb[(i + AHEAD) % (AHEAD + 1)] = frag(i + AHEAD);
@@ -606,6 +609,9 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
       if (m == NH - 1) *reinterpret_cast<f32x4*>(xs + (wid * 2 + k) * 1024 + lane * 16) = other;
     }
   };
+  // (the subtracted maximum follows the true one only when it falls LAG behind: weights stay below 2^LAG, exact in the same
+  // bits, and the outputs are seldom rescaled)
+  constexpr float LAG = 8.f;
   // softmax of the own columns' completed scores of tile t; weights and factors to LDS
   auto softmax = [&](int t) {
     bf16x8 pf;
@@ -627,7 +633,8 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
       for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, sc[k][r]);
     tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float m_new = fmaxf(m_run, fmaxf(tmax * A.scale_log2, NEG_BIG));
+    const float m_top = fmaxf(m_run, fmaxf(tmax * A.scale_log2, NEG_BIG));
+    const float m_new = m_top > m_run + LAG ? m_top : m_run;
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     m_run = m_new;
     l_run *= alpha;
@@ -667,13 +674,17 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
       for (int x = 0; x < 2; ++x) o[x][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, p[x], o[x][n], 0, 0, 0);
     }
   };
+  // (Waits by the builtin: of a wait in asm the compiler knows nothing, and at the loop's first use of the queries it then
+  // waited for every load, the tile's just issued among them.)
   auto lds_barrier = [] {  // tile loads stay in flight across it
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
   auto landed = [] {  // and this one waits for them
-    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+    asm volatile("" ::: "memory");
+    __builtin_amdgcn_s_waitcnt(0x0070);  // vmcnt(0) lgkmcnt(0)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
   };
@@ -686,6 +697,7 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
     softmax(t_lo);
     landed();
   }
+  __builtin_amdgcn_s_waitcnt(0x0070);  // (also for the path past the branch)
   int cur = 0, nxt = 1;  // buffers of tiles i and i + 1
   for (int i = 0; i < n_t; ++i) {
     const int far = 3 - cur - nxt;
@@ -693,6 +705,7 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
     if (i + 2 < n_t) issue(t_lo + i + 2, smem + far * TILE);
     if (i + 1 < n_t) scores(smem + nxt * TILE);
     lds_barrier();
+    if (grp && i + 1 < n_t) softmax(t_lo + i + 1);
     const int own = (i & 1) * NW + wid, other = (i & 1) * NW + (wid ^ 1);
     const bf16x8 p[2] = {*reinterpret_cast<const bf16x8*>(xp + own * 1024 + lane * 16),
                          *reinterpret_cast<const bf16x8*>(xp + other * 1024 + lane * 16)};
@@ -705,7 +718,7 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
       }
     }
     outputs(smem + cur * TILE, p);
-    if (i + 1 < n_t) softmax(t_lo + i + 1);
+    if (!grp && i + 1 < n_t) softmax(t_lo + i + 1);
     landed();
     cur = nxt;
     nxt = far;
@@ -754,7 +767,7 @@ __global__ __launch_bounds__(64 * NW, 2) void mfma_kernel(const Args A) {
   // Two passes over the workgroup's items, so that neither path's registers carry the other's. Tiles are dealt in rounds
   // over the workgroups, every second one from its end: a prompt's later items have more keys, and with one workgroup a CU
   // each gets as many keys in all (dealt in one direction, CUs were busy two thirds of the time:
-  // 500 us at 4,096 tokens instead of 380).
+  // 500 us at 4,096 tokens instead of 380 with the loop of then).
   for (int r = 0, b = blockIdx.y; r * (int)gridDim.y < n; ++r, b = gridDim.y - 1 - b) {
     const int item = r * gridDim.y + b;
     if (item >= n) continue;

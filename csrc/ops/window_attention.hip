@@ -199,7 +199,8 @@ __global__ __launch_bounds__(256) void simple_kernel(const Args A) {
 // ---------------------------------------------------------------------------
 // V^T operand: lanes 16g + i of the result hold dim i of keys 4g .. 4g + 3; each lane names the
 // 8 bytes (key 4g + i/4, dims 4 (i%4) .. + 3) of the 4 x 16 block its group transposes
-__device__ __forceinline__ bf16x4 tr_read(const char* p) {
+// (restrict: an intrinsic without alias information waits for every direct load to LDS in flight)
+__device__ __forceinline__ bf16x4 tr_read(const char* __restrict__ p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)p);
 }
 
