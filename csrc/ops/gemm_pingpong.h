@@ -105,15 +105,18 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
   // W part r: chunk q = 2 wid + h (h = 0, 1) is n-frag (wid & 3) of group (wid >> 2),
   // k-half h of the 64-k tile: n16 tile nt * 16 + (wid >> 2) * 8 + r * 4 + (wid & 3).
   const int KS = A.K >> 5;
-  // x part c: LDS row lr = (2 wid + h) * 8 + (lane >> 3) holds token (lr >> 5) * 64 + 32 c +
-  // (lr & 31); its 16-B unit (lane & 7) is the row's logical unit (lane & 7) ^ ((lr >> 1) & 7).
+  // token (of the tile) of wave column w's fragment j, row r: a wave has 64 in a row; of a group's tile, which may
+  // hold few rows, its fragments lie 64 apart, so that fragments past the last row are the same of all waves
+  auto token = [](int w, int j, int r) { return GR ? 64 * j + 16 * w + r : 64 * w + 16 * j + r; };
+  // x part c: LDS row lr = (2 wid + h) * 8 + (lane >> 3) holds row lr & 15 of wave column lr >> 5's
+  // fragment 2 c + (lr >> 4 & 1); its 16-B unit (lane & 7) is the row's logical unit (lane & 7) ^ ((lr >> 1) & 7).
   int xrow[2][2], xunit[2][2];
 #pragma unroll
   for (int cc = 0; cc < 2; ++cc)
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int lr = (2 * wid + h) * 8 + (lane >> 3);
-      xrow[cc][h] = min(row0 + (lr >> 5) * 64 + cc * 32 + (lr & 31), A.M - 1);
+      xrow[cc][h] = min(row0 + token(lr >> 5, 2 * cc + ((lr >> 4) & 1), lr & 15), A.M - 1);
       xunit[cc][h] = (lane & 7) ^ ((lr >> 1) & 7);
       if constexpr (GR)
         if (A.xmap) xrow[cc][h] = A.xmap[xrow[cc][h]] / A.xdiv;
@@ -200,30 +203,30 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
     for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
 
   // 16 MFMAs of quadrant (W part r, x part cc)
-  auto mma = [&](auto rr, auto ccc, const bf16x8(&af)[4][2], const bf16x8(&bfr)[2][2]) {
-    constexpr int r = decltype(rr)::value, cc = decltype(ccc)::value;
+  auto mma = [&](auto rr, auto ccc, auto jn, const bf16x8(&af)[4][2], const bf16x8(&bfr)[2][2]) {
+    constexpr int r = decltype(rr)::value, cc = decltype(ccc)::value, JN = decltype(jn)::value;
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 2; ++j)
+        for (int j = 0; j < 2 && 2 * cc + j < JN; ++j)
           acc[r * 4 + i][cc * 2 + j] =
               __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i][h], bfr[j][h], acc[r * 4 + i][cc * 2 + j], 0, 0, 0);
     __builtin_amdgcn_s_setprio(0);
   };
   auto lgkm0 = [] { __builtin_amdgcn_s_waitcnt(0xC07F); };
-  // 32 MFMAs: W part r (4 n-frags) x all 4 token frags x K = 64
-  auto mma32 = [&](auto rr, const bf16x8(&af)[4][2], const bf16x8(&b0)[2][2], const bf16x8(&b1)[2][2]) {
-    constexpr int r = decltype(rr)::value;
+  // 32 MFMAs: W part r (4 n-frags) x all 4 token frags (or the first JN) x K = 64
+  auto mma32 = [&](auto rr, auto jn, const bf16x8(&af)[4][2], const bf16x8(&b0)[2][2], const bf16x8(&b1)[2][2]) {
+    constexpr int r = decltype(rr)::value, JN = decltype(jn)::value;
     __builtin_amdgcn_s_setprio(1);
 #pragma unroll
     for (int h = 0; h < 2; ++h)
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
+        for (int j = 0; j < JN; ++j)
           acc[r * 4 + i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(af[i][h], j < 2 ? b0[j][h] : b1[j - 2][h],
                                                                       acc[r * 4 + i][j], 0, 0, 0);
     __builtin_amdgcn_s_setprio(0);
@@ -253,33 +256,34 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
   //     1      B1 (4)           A x B1      B1 of tile t + 2           8
   // (a part is restaged two phases after its last read; the wait before a phase's first
   // barrier retires exactly what the next phase reads)
-  auto body4 = [&](int t, auto st) {
+  auto body4 = [&](int t, auto st, auto jn) {
     constexpr int S = decltype(st)::value;  // 0 steady, 1 tile nk - 2, 2 the last tile
+    constexpr bool B1 = decltype(jn)::value > 2;
     read_w(0, t, af);
     read_x(0, t, bx0);
     if constexpr (S == 0) {
       issue_w(0, t + 2);
       issue_x(0, t + 2);
-      wait_vm<10>();
+      wait_vm<B1 ? 10 : 8>();
     } else if constexpr (S == 1) {
-      wait_vm<6>();
+      wait_vm<B1 ? 6 : 4>();
     } else {
       wait_vm<0>();
     }
     raw_barrier();
     lgkm0();
-    mma(ic<0>{}, ic<0>{}, af, bx0);
+    mma(ic<0>{}, ic<0>{}, jn, af, bx0);
     raw_barrier();
-    read_x(1, t, bx1);
+    if constexpr (B1) read_x(1, t, bx1);
     if constexpr (S == 0) {
-      issue_x(1, t + 2);
-      wait_vm<8>();
+      if constexpr (B1) issue_x(1, t + 2);
+      wait_vm<B1 ? 8 : 4>();
     } else if constexpr (S == 1) {
-      wait_vm<2>();
+      wait_vm<B1 ? 2 : 0>();
     }
     raw_barrier();
     lgkm0();
-    mma(ic<0>{}, ic<1>{}, af, bx1);
+    if constexpr (B1) mma(ic<0>{}, ic<1>{}, jn, af, bx1);
     raw_barrier();
   };
 
@@ -289,21 +293,22 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
   //     1      A1 (8)                  A1 x (B0, B1)     A0, B0 of tile t + 2      6
   // lgkmcnt(0) before each load segment's barrier, so a part is restaged one phase after its
   // last read (the partner group's reads of that phase are retired behind the same barrier).
-  auto body2 = [&](int t, auto st) {
+  auto body2 = [&](int t, auto st, auto jn) {
     constexpr int S = decltype(st)::value;  // 0 steady, 1 tile nk - 2, 2 the last tile
+    constexpr bool B1 = decltype(jn)::value > 2;
     read_w(0, t, af);
     read_x(0, t, bx0);
-    read_x(1, t, bx1);
+    if constexpr (B1) read_x(1, t, bx1);
     if constexpr (S < 2) {
-      issue_x(1, t + 1);
+      if constexpr (B1) issue_x(1, t + 1);
       issue_w(1, t + 1);
-      wait_vm<8>();
+      wait_vm<B1 ? 8 : 6>();
     } else {
       wait_vm<0>();
     }
     lgkm0();
     raw_barrier();
-    mma32(ic<0>{}, af, bx0, bx1);
+    mma32(ic<0>{}, jn, af, bx0, bx1);
     raw_barrier();
     read_w(1, t, af);
     if constexpr (S == 0) {
@@ -315,7 +320,7 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
     }
     lgkm0();
     raw_barrier();
-    mma32(ic<1>{}, af, bx0, bx1);
+    mma32(ic<1>{}, jn, af, bx0, bx1);
     raw_barrier();
   };
 
@@ -366,34 +371,43 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
     for (; t + 2 < nk; ++t) body6(t, ic<0>{});
     body6(t, ic<1>{});
     body6(t + 1, ic<2>{});
-  } else if constexpr (F == 8) {
-    issue_w(0, 0);
-    issue_x(0, 0);
-    issue_x(1, 0);
-    issue_w(1, 0);
-    issue_w(0, 1);
-    issue_x(0, 1);
-    wait_vm<6>();  // A0, B0 and B1 of tile 0 landed
-    raw_barrier();
-    if (G == 1) raw_barrier();
-    if constexpr (STAMP) st1 = __builtin_amdgcn_s_memtime();
-    for (; t + 2 < nk; ++t) body2(t, ic<0>{});
-    body2(t, ic<1>{});
-    body2(t + 1, ic<2>{});
   } else {
-    issue_w(0, 0);
-    issue_x(0, 0);
-    issue_x(1, 0);
-    issue_w(0, 1);
-    issue_x(0, 1);
-    issue_x(1, 1);
-    wait_vm<8>();  // A and B0 of tile 0 landed
-    raw_barrier();
-    if (G == 1) raw_barrier();
-    if constexpr (STAMP) st1 = __builtin_amdgcn_s_memtime();
-    for (; t + 2 < nk; ++t) body4(t, ic<0>{});
-    body4(t, ic<1>{});
-    body4(t + 1, ic<2>{});
+    // with JN token frags of 4 (below 3, B1 is neither staged nor read)
+    auto run = [&](auto jn) {
+      constexpr bool B1 = decltype(jn)::value > 2;
+      issue_w(0, 0);
+      issue_x(0, 0);
+      if constexpr (B1) issue_x(1, 0);
+      if constexpr (F == 8) issue_w(1, 0);
+      issue_w(0, 1);
+      issue_x(0, 1);
+      if constexpr (F == 8) {
+        wait_vm<6>();  // A0, B0 and B1 of tile 0 landed
+      } else {
+        if constexpr (B1) issue_x(1, 1);
+        wait_vm<B1 ? 8 : 4>();  // A and B0 of tile 0 landed
+      }
+      raw_barrier();
+      if (G == 1) raw_barrier();
+      if constexpr (STAMP) st1 = __builtin_amdgcn_s_memtime();
+      auto body = [&](int tt, auto st) {
+        if constexpr (F == 8) body2(tt, st, jn);
+        else body4(tt, st, jn);
+      };
+      for (; t + 2 < nk; ++t) body(t, ic<0>{});
+      body(t, ic<1>{});
+      body(t + 1, ic<2>{});
+    };
+    // a group's last tile may hold few rows: each 64 fewer leave out a quarter of the MFMAs (4,096 tokens, 6 of 64
+    // experts of 2,048 x 2 x 1,408 and back, 384 rows each on average: 322 + 167 -> 284 + 156 us)
+    if constexpr (GR) {
+      if (A.M > 192) run(ic<4>{});
+      else if (A.M > 128) run(ic<3>{});
+      else if (A.M > 64) run(ic<2>{});
+      else run(ic<1>{});
+    } else {
+      run(ic<4>{});
+    }
   }
   if (G == 0) raw_barrier();  // balance the stagger
   if constexpr (STAMP) st2 = __builtin_amdgcn_s_memtime();
@@ -434,12 +448,12 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
     }
   }
 
-  // ---- register epilogue: acc[i][j] holds token row0 + 64 wc + 16 j + c, columns
+  // ---- register epilogue: acc[i][j] holds token row0 + token(wc, j, c), columns
   // 4 g .. 4 g + 3 of 16-column tile nt * 2F + F G + i
   const float inv_k = 1.f / (float)A.K;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    int m = row0 + wc * 64 + 16 * j + c;
+    int m = row0 + token(wc, j, c);
     const bool ok = m < A.M;
     float rs = 1.f;
     if constexpr (GR) {

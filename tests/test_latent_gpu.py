@@ -108,13 +108,8 @@ def test_table_experts(gpu, dt, tm, T, E, top, ff, D):
             torch.testing.assert_close(y[t, k], (a * torch.sigmoid(1.702 * a) * (u + 1)) @ w2[e].float().T, **tol(dt))
 
 
-@pytest.mark.parametrize("tm", [16, 32, 64, 128])
-@pytest.mark.parametrize("counts,N,K", [
-    ([1, 0, 16, 17, 40, 130, 3], 96, 96),       # empty and single-row groups, remainders of every tile, k past no stage's end
-    ([5, 33], 80, 2048), ([200] * 3, 2816, 32),  # an odd number of 16-row blocks; more blocks than XCDs
-    ([7], 16384, 64), ([100], 16384, 320), ([300], 4096, 160), ([300], 16384, 96)])  # one group: 4, 2 and 1 waves over k
-def test_sorted_rows(gpu, tm, counts, N, K):
-    """The grouped projections of sorted rows at every tile size: plain, the square of relu and gated with weights of rows,
+def sorted_rows(gpu, tm, counts, N, K):
+    """The grouped projections of sorted rows of one tile size: plain, the square of relu and gated with weights of rows,
     gathered and scattered. Sums of K products in fp32 err by K 2^-24 of their magnitudes at most, a bf16 result rounds by
     2^-8; silu(g) u moves by at most 1.1 |u| dg + |g| du."""
     from pilottai_amd import ops
@@ -157,6 +152,22 @@ def test_sorted_rows(gpu, tm, counts, N, K):
     out = torch.empty(rows, N // 2, dtype=torch.bfloat16, device=gpu)
     ops.expert_gemm(x, pw, out, *args, x_div=top, out_order=False, tm=tm, glu=(3e38, 1.0, 0.0), row_w=rw)
     assert bool(((out.float() - want.reshape(rows, -1)).abs() <= err.reshape(rows, -1)).all())
+
+
+@pytest.mark.parametrize("tm", [16, 32, 64, 128])
+@pytest.mark.parametrize("counts,N,K", [
+    ([1, 0, 16, 17, 40, 130, 3], 96, 96),       # empty and single-row groups, remainders of every tile, k past no stage's end
+    ([5, 33], 80, 2048), ([200] * 3, 2816, 32),  # an odd number of 16-row blocks; more blocks than XCDs
+    ([7], 16384, 64), ([100], 16384, 320), ([300], 4096, 160), ([300], 16384, 96)])  # one group: 4, 2 and 1 waves over k
+def test_sorted_rows(gpu, tm, counts, N, K):
+    sorted_rows(gpu, tm, counts, N, K)
+
+
+@pytest.mark.parametrize("counts", [[1, 64, 65, 0, 128, 129], [192, 193, 256], [257, 320, 321, 2], [384, 385, 449]])
+@pytest.mark.parametrize("N,K", [(256, 128), (384, 192), (512, 320)])  # 256 and 128 columns a tile; 2, 3 and 5 steps over k
+def test_sorted_rows_of_whole_tiles(gpu, counts, N, K):
+    """Tiles of 256 rows that hold every number of their 64-row parts."""
+    sorted_rows(gpu, 256, counts, N, K)
 
 
 @pytest.mark.parametrize("dt", DTYPES)
