@@ -471,9 +471,32 @@ int32_t Scheduler::emit(int32_t* buf) {
           const int64_t np = (tgt + ndec * kv - 1) / (ndec * kv);
           cand = std::max<int64_t>(cfg_.att_min_part, std::min(((maxc + np - 1) / np + 31) / 32 * 32, share));
         }
-        int64_t parts = 0;
-        for (const Planned& p : last_plan_)
-          if (p.n <= tpw) parts += std::max<int64_t>(1, (att_keys(p) + cand - 1) / cand);
+        auto parts_of = [&](int64_t size) {
+          int64_t n = 0;
+          for (const Planned& p : last_plan_)
+            if (p.n <= tpw) n += std::max<int64_t>(1, (att_keys(p) + size - 1) / size);
+          return n;
+        };
+        int64_t parts = parts_of(cand);
+        if (cfg_.decode_part_fit && parts * kv > tgt) {
+          // A few parts more than workgroups run at once are a second round for all (64 rows of about 2,048 latents in
+          // 269 parts on 256 CUs: 51 us, in 241 larger ones 41): of the larger sizes, the one whose longest part, or
+          // whose rounds and half a part more, end first. A part costs about 256 keys beside its own.
+          auto cost = [&](int64_t size, int64_t n) {
+            const int64_t longest = std::min(size, maxc) + 256;
+            return n * kv <= tgt ? longest : (sumc + 256 * n) * kv / tgt + longest / 2;
+          };
+          int64_t best = cost(cand, parts);
+          const int64_t by = std::max<int64_t>(32, (maxc - cand) / 32 / 32 * 32);
+          for (int64_t size = cand + by; size < maxc + by; size += by) {
+            const int64_t n = parts_of(size), x = cost(size, n);
+            if (x < best) {
+              best = x;
+              cand = size;
+              parts = n;
+            }
+          }
+        }
         if (nprefill + parts <= L.max_items) psz = (int32_t)cand;
       }
     }

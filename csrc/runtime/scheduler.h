@@ -77,6 +77,7 @@ struct SchedulerConfig {
   // equal partitions of the longest context (multiples of 32 keys, >= 128); 0 = the 512 / 256-key
   // rule
   int32_t decode_part_target = 0;
+  bool decode_part_fit = false;  // and, were they more than that many, for as many as end first
   // the same rule for the decode-sized steps that run 8-wave attention (small_step_part > 0,
   // t_step <= small_step_tokens; one 8-wave workgroup per CU): 0 = small_step_part
   int32_t small_step_target = 0;

@@ -682,7 +682,7 @@ class HybridModel:
         keys = [m.max_keys for m in self.attention]
         pools = [m.pool for m in self.attention if m.pool]
         out = {"gqa_group": self._group, "kv_heads": self._kv_heads, "att_qcols": 128, "att_narrow_qcols": 128,
-               "prefill_split_keys": 0, "decode_part_target": 256, "att_min_part": 256,
+               "prefill_split_keys": 0, "decode_part_target": 256, "decode_part_fit": True, "att_min_part": 256,
                "att_tile_target": max(16, 256 // self._kv_heads), "att_max_keys": max(keys) if keys and all(keys) else 0,
                "att_pool": min(pools, default=0)}
         if self.state_bytes_per_slot():  # a page's worth of state is not kept, so a prefix cannot be taken from the cache

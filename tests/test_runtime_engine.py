@@ -907,3 +907,29 @@ def test_engine_split_ticket_room_only_with_split_keys():
     # per (sequence, KV head) tickets only, vs + per (partial slot, KV head) ones
     assert off._att_counters.numel() < on._att_counters.numel()
     assert off._att_counters.numel() % kv == 0 and on._att_counters.numel() % kv == 0
+
+
+@pytest.mark.parametrize("kv,contexts,most,longest", [
+    (1, [1600 + 13 * i for i in range(64)], 256, 640),  # a little more than 256 parts of the balanced share
+    (1, [2000] * 8, 256, 256),                          # already fewer
+    (4, [1900 + 5 * i for i in range(64)], 256, 2300),  # as many as fit only with a part each
+    (4, [300] * 63 + [4000], None, 640),                # one long row among short ones stays split
+])
+def test_scheduler_decode_parts_fit_one_round(kv, contexts, most, longest):
+    """decode_part_fit: partitions cover every row's keys, are no more than run at once where that ends sooner, and no
+    longer than `longest` keys."""
+    s = _runtime.Scheduler({"num_blocks": 12000, "block_size": 16, "max_num_seqs": 64, "max_num_batched_tokens": 4096,
+                            "max_model_len": 8192, "gqa_group": 16 // kv, "kv_heads": kv, "att_qcols": 128, "att_min_part": 256,
+                            "att_narrow_qcols": 128, "prefix_caching": False, "decode_part_target": 256, "decode_part_fit": True})
+    L = s.layout()
+    buf = np.zeros(L["total"], dtype=np.int32)
+    for i, n in enumerate(contexts):
+        s.schedule_fed(buf.ctypes.data, [(i + 1, [1] * (n - 1))])
+        s.commit(0, 0)
+    assert s.schedule_fed(buf.ctypes.data, [(i + 1, [1]) for i in range(len(contexts))]) == len(contexts)
+    items = buf[L["items"]:L["items"] + 4 * int(buf[L["n_items"]])].reshape(-1, 4)
+    part, seqs = int(buf[L["part_size"]]), items[:, 0]
+    assert part <= longest and (most is None or len(items) * kv <= most)
+    for i, n in enumerate(contexts):
+        of = items[seqs == i]
+        assert len(of) == max(1, -(-n // part)) and sorted((of[:, 2] >> 8) & 0xfff) == list(range(len(of)))
