@@ -126,9 +126,7 @@ def state_scan(proj, y, state, ring, conv_w, conv_b, dt_bias, a, d, q_start, q_l
     items = 0 if T <= scan_min else min(scan_items.shape[0], T // SCAN_CHUNK + min(seqs, T // (scan_min + 1)) + 1)
     new = lambda dt, *s: torch.empty(*s, dtype=dt, device=proj.device)  # noqa: E731
     u = new(proj.dtype, T if items else 0, ring.shape[2])
-    chunked = items if proj.dtype == torch.bfloat16 else 0
-    work, total = new(torch.float32, chunked, H, V, N), new(torch.float32, chunked, H)
-    require_hybrid().state_scan(proj, u, y, state, ring, work, total, conv_w, conv_b, dt_bias, a, d, q_start, q_len, ctx_len,
+    require_hybrid().state_scan(proj, u, y, state, ring, conv_w, conv_b, dt_bias, a, d, q_start, q_len, ctx_len,
                                 state_slot, scan_first, scan_items, n_scan, int(items), int(seqs), int(groups),
                                 int(scan_min))
     return y

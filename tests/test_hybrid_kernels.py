@@ -347,6 +347,58 @@ def test_state_scan(device, dt, H, V, N, G, taps):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("V,N,lens", [
+    (48, 128, [9 + 7 * (i % 9) for i in range(41)]),           # more portions than the grid has rows for
+    (16, 64, [64, 128, 65, 127, 1, 8, 9]), (64, 160, [63, 200]),  # whole chunks and one past; columns past N
+    (32, 288, [130, 20])])                                     # a state that is stepped through instead
+def test_state_scan_portions(gpu, V, N, lens):
+    """Portions of one step, every second one from a state, against a pass in fp64 over the same convolved rows."""
+    from pilottai_amd import ops
+
+    H, G, taps = 4, 2, 4
+    g = gen(V + N)
+    inner, bc, S, T = H * V, G * N, len(lens), sum(lens)
+    C = inner + 2 * bc
+    proj = torch.randn(T, (inner + C + H + 7) // 8 * 8, generator=g).to(BF16)
+    conv, cb = torch.randn(taps, C, generator=g) * 0.5, torch.randn(C, generator=g) * 0.2
+    dt_bias, a, d = torch.randn(H, generator=g) - 2, torch.linspace(0.02, 2.0, H), torch.randn(H, generator=g)
+    state = torch.randn(S, H, V, N, generator=g)
+    ring = torch.randn(S, taps - 1 + ops.SCAN_MIN, C, generator=g).to(BF16)
+    starts, past = np.cumsum([0] + lens), [0 if i % 2 else 100 + i for i in range(S)]
+    want, after = torch.empty(T, inner, dtype=torch.float64), torch.empty(S, H, V, N, dtype=torch.float64)
+    most = torch.zeros(())  # the largest dt |x| |B|
+    for i, n in enumerate(lens):
+        rows = proj[starts[i]:starts[i + 1]].double()
+        before = [ring[i, (past[i] + t) % ring.shape[1]].double() if past[i] + t >= 0 else torch.zeros(C).double() for t in range(1 - taps, 0)]
+        x = torch.cat([torch.stack(before), rows[:, inner:inner + C]])
+        u = oracle.silu(sum(conv[k].double() * x[k:k + n] for k in range(taps)) + cb.double()).to(BF16).double()
+        step = torch.nn.functional.softplus(rows[:, inner + C:inner + C + H] + dt_bias.double())
+        s = state[i].double() if past[i] else torch.zeros(H, V, N, dtype=torch.float64)
+        xs, B, Cm = u[:, :inner].view(n, H, V), *(u[:, inner + k * bc:inner + (k + 1) * bc].view(n, G, N).repeat_interleave(H // G, 1) for k in (0, 1))
+        most = torch.maximum(most, (step * xs.abs().amax(2) * B.abs().amax(2)).max())
+        for t in range(n):
+            s = s * torch.exp(-a.double() * step[t])[:, None, None] + (step[t, :, None] * xs[t])[:, :, None] * B[t][:, None]
+            want[starts[i] + t] = ((s * Cm[t][:, None]).sum(-1) + d.double()[:, None] * xs[t]).reshape(-1)
+        after[i] = s
+    items = [[i, b, min(ops.SCAN_CHUNK, n - b), 0] for i, n in enumerate(lens) if n > ops.SCAN_MIN for b in range(0, n, ops.SCAN_CHUNK)]
+    iv = lambda v: torch.tensor([int(x) if not isinstance(x, list) else x for x in v], dtype=torch.int32, device=gpu)  # noqa: E731
+    f = lambda t: t.float().to(gpu)  # noqa: E731
+    y, st = torch.full((T, inner), 5.0, dtype=BF16, device=gpu), state.to(gpu)
+    first, k = [], 0
+    for n in lens:
+        first.append(k if n > ops.SCAN_MIN else -1)
+        k += -(-n // ops.SCAN_CHUNK) if n > ops.SCAN_MIN else 0
+    ops.state_scan(proj.to(gpu), y, st, ring.to(gpu), f(conv), f(cb), f(dt_bias), f(a), f(d), iv(starts[:-1]), iv(lens),
+                   iv([p + n for p, n in zip(past, lens)]), iv(range(S)), iv(first), iv(items + [[0, 0, 0, 0]] * 3), iv([len(items)]), G)
+    torch.testing.assert_close(y.double().cpu(), want, **tol(BF16, float(want.abs().mean()) + 0.1))
+    # The state: products of bf16 values with weights of 16 bits of mantissa, summed in fp32: 2e-4 all in all. A convolved
+    # value within fp32's error of the middle of two bf16 values may round to the other one, here and there: by 2^-8 of it,
+    # so a state value moves by 2^-8 dt |x| |B| at most, or twice that where two meet.
+    err = (st.double().cpu() - after).abs()
+    assert float((err / (after.abs() + after.abs().mean())).square().mean().sqrt()) < 2e-4
+    assert float((err - 2e-4 * after.abs()).max()) < 2e-4 * float(after.abs().mean()) + 2 * 2.0 ** -8 * float(most)
+
+
 def test_state_scan_keeps_the_state_in_fp32(gpu):
     """The state a chunked portion leaves equals the one that single tokens leave to fp32's order, not bf16's."""
     from pilottai_amd import ops
