@@ -116,6 +116,47 @@ __device__ __forceinline__ float times(float a, float f, const Args& A) {
   return glu(a, f, A);
 }
 
+// A wave's outputs: 16 NT of a group's columns from nt0 on, of the rows m * 16 + c < n from `start`.
+template <int MT, int NT, int EPI>
+__device__ __forceinline__ void store_rows(const Args& A, int grp, int start, int n, int nt0, const f32x4 (&acc)[MT][NT]) {
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+#pragma unroll
+  for (int m = 0; m < MT; ++m) {
+    if (16 * m + c >= n) continue;
+    const int at = start + 16 * m + c;
+    bf16* o = (bf16*)A.out + (size_t)at * A.ldo + (size_t)grp * A.og + 4 * g;
+    if constexpr (EPI == GATED) {
+      const bf16* f = factor_row<bf16, EPI>(A, at, grp) + 4 * g;
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        if (nt0 + i >= A.N16) break;
+        const bf16x4 fv = *reinterpret_cast<const bf16x4*>(f + (nt0 + i) * 16);
+        bf16x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = (bf16)times<EPI>(acc[m][i][j], (float)fv[j], A);
+        *reinterpret_cast<bf16x4*>(o + (nt0 + i) * 16) = v;
+      }
+    } else if (NT % 2 == 0 && A.N16 % 2 == 0 && A.wide) {
+      // 16-byte stores: lanes of neighbouring lane groups trade halves
+      const struct { bf16* y; int ldy; } row{o - 4 * g, 0};
+#pragma unroll
+      for (int i = 0; i + 1 < NT; i += 2) {
+        if (nt0 + i >= A.N16) break;
+        pk::store_pair_wide<pk::EP_PLAIN>(row, 0, nt0 + i, g, acc[m][i], acc[m][i + 1]);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < NT; ++i) {
+        if (nt0 + i >= A.N16) break;
+        bf16x4 v;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) v[j] = (bf16)acc[m][i][j];
+        *reinterpret_cast<bf16x4*>(o + (nt0 + i) * 16) = v;
+      }
+    }
+  }
+}
+
 // Dense rows: tiles of 16 MT rows and 16 NT outputs a wave (PLAIN, GATED).
 template <int MT, int NT, int KU, int EPI>
 __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
@@ -133,12 +174,9 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
 #pragma unroll
   for (int i = 0; i < NT; ++i) wt[i] = wp + (size_t)min(nt0 + i, A.N16 - 1) * A.K32 * 512;
   const bf16* xr[MT];
-  int pos[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
-    const int i = min(16 * m + c, n - 1);
-    pos[m] = start + i;
-    xr[m] = (const bf16*)A.x + (size_t)pos[m] * A.ldx + (size_t)grp * A.xg + 8 * g;
+    xr[m] = (const bf16*)A.x + (size_t)(start + min(16 * m + c, n - 1)) * A.ldx + (size_t)grp * A.xg + 8 * g;
   }
   f32x4 acc[MT][NT];
 #pragma unroll
@@ -174,39 +212,82 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
       for (int m = 0; m < MT; ++m) b[k][m] = bn[k][m];
     }
   }
+  store_rows<MT, NT, EPI>(A, grp, start, n, nt0, acc);
+}
+
+// Many dense rows of groups with few inputs (the heads of a latent attention): 64 rows of a group's inputs whole in LDS,
+// every one of its outputs from there. In gemm_kernel each wave fetches them by itself, in pieces of 64 bytes, for every
+// 64 outputs. Units of 8 inputs, [K / 8][64 rows][8] and a row of padding, so that rows are written and fragments read
+// without conflicts. 4,096 rows, 16 heads: 128 -> 512 beside 64 rotated 43 -> 34 us (88 MB:
+// 18 us at the rate of a copy). 512 -> 128 stays there: 29 us, here 31, as the rows arrive before the first product; and so
+// do fewer than two workgroups a CU (512 rows of 16 heads: 10 us, here 11).
+constexpr int HEAD_UNIT = 65 * 16, HEAD_K32 = 8;
+
+template <int EPI>
+__global__ __launch_bounds__(256, 2) void head_rows_kernel(const Args A) {
+  constexpr int NT = 4;
+  extern __shared__ __attribute__((aligned(16))) char xs[];
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
+  const int grp = blockIdx.y, start = blockIdx.x * 64, n = min(64, A.rows - start), U = 4 * A.K32;
+  const bf16* x = (const bf16*)A.x + (size_t)start * A.ldx + (size_t)grp * A.xg;
+  const unsigned inv = ((1u << 20) + U - 1) / U;  // e / U of e < 4096
+  bf16x8 v[HEAD_K32];
+  auto unit = [&](int k, int& j) {
+    const unsigned e = k * 256 + threadIdx.x;
+    j = e * inv >> 20;
+    return (int)e - j * U;
+  };
 #pragma unroll
-  for (int m = 0; m < MT; ++m) {
-    if (16 * m + c >= n) continue;
-    bf16* o = (bf16*)A.out + (size_t)pos[m] * A.ldo + (size_t)grp * A.og + 4 * g;
-    if constexpr (EPI == GATED) {
-      const bf16* f = factor_row<bf16, EPI>(A, pos[m], grp) + 4 * g;
-#pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        if (nt0 + i >= A.N16) break;
-        const bf16x4 fv = *reinterpret_cast<const bf16x4*>(f + (nt0 + i) * 16);
-        bf16x4 v;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = (bf16)times<EPI>(acc[m][i][j], (float)fv[j], A);
-        *reinterpret_cast<bf16x4*>(o + (nt0 + i) * 16) = v;
-      }
-    } else if (NT % 2 == 0 && A.N16 % 2 == 0 && A.wide) {
-      // 16-byte stores: lanes of neighbouring lane groups trade halves
-      const struct { bf16* y; int ldy; } row{o - 4 * g, 0};
-#pragma unroll
-      for (int i = 0; i + 1 < NT; i += 2) {
-        if (nt0 + i >= A.N16) break;
-        pk::store_pair_wide<pk::EP_PLAIN>(row, 0, nt0 + i, g, acc[m][i], acc[m][i + 1]);
-      }
-    } else {
-#pragma unroll
-      for (int i = 0; i < NT; ++i) {
-        if (nt0 + i >= A.N16) break;
-        bf16x4 v;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) v[j] = (bf16)acc[m][i][j];
-        *reinterpret_cast<bf16x4*>(o + (nt0 + i) * 16) = v;
-      }
+  for (int k = 0; k < HEAD_K32; ++k)
+    if (k < A.K32) {
+      int j;
+      const int u = unit(k, j);
+      v[k] = *reinterpret_cast<const bf16x8*>(x + (size_t)min(j, n - 1) * A.ldx + 8 * u);
     }
+#pragma unroll
+  for (int k = 0; k < HEAD_K32; ++k)
+    if (k < A.K32) {
+      int j;
+      const int u = unit(k, j);
+      *reinterpret_cast<bf16x8*>(xs + u * HEAD_UNIT + j * 16) = v[k];
+    }
+  if (A.rp) rotate_rows<bf16>(A, grp, start, n);
+  __syncthreads();
+  const bf16* wp = (const bf16*)A.w + (size_t)grp * A.wstride + lane * 8;
+  const char* xf = xs + g * HEAD_UNIT + c * 16;
+  for (int nt0 = wid * NT; nt0 < A.N16; nt0 += 4 * NT) {
+    const bf16* wt[NT];
+#pragma unroll
+    for (int i = 0; i < NT; ++i) wt[i] = wp + (size_t)min(nt0 + i, A.N16 - 1) * A.K32 * 512;
+    f32x4 acc[4][NT];
+#pragma unroll
+    for (int m = 0; m < 4; ++m)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) acc[m][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto load = [&](int s, bf16x8 (&a)[NT]) {  // (past the end: the last step's again)
+#pragma unroll
+      for (int i = 0; i < NT; ++i) a[i] = *reinterpret_cast<const bf16x8*>(wt[i] + (size_t)min(s, A.K32 - 1) * 512);
+    };
+    auto step = [&](int s, const bf16x8 (&a)[NT]) {
+#pragma unroll
+      for (int m = 0; m < 4; ++m) {
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(xf + s * (4 * HEAD_UNIT) + m * 256);
+#pragma unroll
+        for (int i = 0; i < NT; ++i) acc[m][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], b, acc[m][i], 0, 0, 0);
+      }
+    };
+    bf16x8 a0[NT], a1[NT];
+    load(0, a0);
+    load(1, a1);
+    int s = 0;
+    for (; s + 1 < A.K32; s += 2) {
+      step(s, a0);
+      load(s + 2, a0);
+      step(s + 1, a1);
+      load(s + 3, a1);
+    }
+    if (s < A.K32) step(s, a0);
+    store_rows<4, NT, EPI>(A, grp, start, n, nt0, acc);
   }
 }
 
@@ -654,6 +735,11 @@ extern "C" int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out
   if (tm == 16) {
     if (epi == 3) PA_GGK(1, 1, pa::gg::GATED);
     else PA_GGK(1, 1, pa::gg::PLAIN);
+  } else if (K32 <= pa::gg::HEAD_K32 && N16 >= 16 && (rows + 63) / 64 * groups >= 512) {
+    const dim3 grid((rows + 63) / 64, groups);
+    const int lds = 4 * K32 * pa::gg::HEAD_UNIT;
+    if (epi == 3) hipLaunchKernelGGL((pa::gg::head_rows_kernel<pa::gg::GATED>), grid, dim3(256), lds, st, A);
+    else hipLaunchKernelGGL((pa::gg::head_rows_kernel<pa::gg::PLAIN>), grid, dim3(256), lds, st, A);
   } else {
     if (epi == 3) PA_GG(4, 4, 1, pa::gg::GATED);
     else PA_GG(4, 4, 1, pa::gg::PLAIN);

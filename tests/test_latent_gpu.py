@@ -64,6 +64,37 @@ def test_head_gemm(gpu, dt, T, G, N, K):
     assert (o[:, :, N:] == 5.0).all()
 
 
+@pytest.mark.parametrize("gated", [False, True])
+@pytest.mark.parametrize("T,G,N,K", [(32705, 1, 256, 32), (2049, 16, 272, 160), (1100, 33, 512, 256), (4095, 8, 512, 128)])
+def test_head_gemm_of_many_rows(gpu, T, G, N, K, gated):
+    """Two workgroups of 64 rows a CU and more: sizes that are no multiple of a tile, the widest inputs, beside rotated
+    columns. Sums of K products in fp32 err by K 2^-24 of their magnitudes at most, a bf16 result rounds by 2^-8."""
+    from pilottai_amd import ops
+
+    g = torch.Generator(device=gpu).manual_seed(T)
+    rnd = lambda *s: torch.randn(*s, device=gpu, generator=g)  # noqa: E731
+    hs, r = K + 24, 16
+    x, w = rnd(T, G * hs).bfloat16(), (rnd(G, N, K) / math.sqrt(K)).bfloat16()
+    pos = torch.randint(0, 50, (T,), device=gpu, generator=g, dtype=torch.int32)
+    ang = rnd(50, r // 2)
+    cs = torch.cat([ang.cos(), ang.sin()], 1).contiguous()
+    out = torch.full((T, G * (N + 32 + 8)), 5.0, dtype=torch.bfloat16, device=gpu)
+    gate = rnd(T, G * (N + 40)).bfloat16() if gated else None
+    ops.head_gemm(x, hs, ops.pack_groups(w, torch.bfloat16), out, N + 40, None if gated else (pos, cs, K, r, 32), gate)
+    for h in range(G):
+        xs, o = x[:, h * hs:(h + 1) * hs].float(), out[:, h * (N + 40):(h + 1) * (N + 40)].float()
+        want, slack = xs[:, :K] @ w[h].float().T, K * 2.0 ** -24 * (xs[:, :K].abs() @ w[h].float().abs().T)
+        if gated:
+            s = torch.sigmoid(gate[:, h * (N + 40):h * (N + 40) + N].float())
+            want, slack = want * s, slack * s + 2.0 ** -20 * want.abs()
+        assert bool(((o[:, :N] - want).abs() <= 2.0 ** -8 * want.abs() + slack + 1e-30).all()) and bool((o[:, N + 32:] == 5.0).all())
+        if not gated:
+            u, v, c, sn = xs[:, K:K + r // 2], xs[:, K + r // 2:K + r], cs[pos.long(), :r // 2], cs[pos.long(), r // 2:]
+            turned = torch.cat([u * c - v * sn, v * c + u * sn], 1)
+            torch.testing.assert_close(o[:, N:N + r], turned, **tol(torch.bfloat16))
+            assert not o[:, N + r:N + 32].any()
+
+
 @pytest.mark.parametrize("dt,tm", [(torch.bfloat16, 16), (torch.bfloat16, 64), (torch.bfloat16, 256), (torch.float32, 16)])
 @pytest.mark.parametrize("T,E,top,ff,D", [(1, 5, 2, 40, 96), (900, 4, 2, 72, 200), (600, 2, 2, 128, 256), (77, 7, 3, 96, 160), (300, 12, 1, 64, 64), (130, 70, 5, 32, 128)])
 def test_table_experts(gpu, dt, tm, T, E, top, ff, D):
