@@ -59,10 +59,9 @@ log = logging.getLogger("pilottai_amd.engine")
 # hipGraph token buckets: a step of T tokens replays the smallest bucket >= T, so
 # the spacing bounds the padded (wasted) work: 16-token steps up to 512 (graph padding 1.9 ->
 # 1.1 % of step tokens at 64 workers; profiles/r2_buckets16_ab.jsonl), 64 up to 2048
-# (prefill-heavy agent steps sit at 400-1000 tokens), then 256, a row tile of the projections, up to 4096 and
-# 512 up to 8192 (3658 tokens of three prompts on mudepel-base: 5.88 ms as 4096 rows, 5.44 as 3840).
+# (prefill-heavy agent steps sit at 400-1000 tokens).
 DEFAULT_BUCKETS = ([8, 16, 32, 48, 64, 80] + list(range(96, 513, 16)) + list(range(576, 2049, 64))
-                   + list(range(2304, 4097, 256)) + list(range(4608, 8193, 512)))
+                   + [3072, 4096, 6144, 8192])
 
 
 @dataclass
