@@ -34,10 +34,11 @@ struct Args {
   float eps;
 };
 
-template <typename T, int VEC, int S>
-__global__ __launch_bounds__(256) void hyper_norm_kernel(const Args A) {
+template <typename T, int VEC, int S, int NW>
+__global__ __launch_bounds__(64 * NW) void hyper_norm_kernel(const Args A) {
+  constexpr int NT = 64 * NW;
   extern __shared__ __attribute__((aligned(16))) float row[];
-  __shared__ float red[4];
+  __shared__ float red[NW];
   const int t = A.rows ? A.rows[blockIdx.x] : blockIdx.x, D = A.D;
   float* xr = A.x + (size_t)t * S * D;
   float mix[S][S], post[S], pre[S];
@@ -52,7 +53,7 @@ __global__ __launch_bounds__(256) void hyper_norm_kernel(const Args A) {
   const float* yw = A.y_w ? A.y_w + (size_t)t * A.K : nullptr;
   const T* er = A.emb ? (const T*)A.emb + (size_t)min(max(A.ids[t], 0), A.vocab - 1) * D : nullptr;
   float ss = 0.f;
-  for (int i = threadIdx.x * VEC; i < D; i += 256 * VEC) {
+  for (int i = threadIdx.x * VEC; i < D; i += NT * VEC) {
     float x[S][VEC], u[VEC];
     T a[VEC];
 #pragma unroll
@@ -113,15 +114,15 @@ __global__ __launch_bounds__(256) void hyper_norm_kernel(const Args A) {
     }
   }
   if (!A.w_next) return;
-  const float inv = 1.f / sqrtf(block_sum<4>(ss, red) / (float)D + A.eps);
+  const float inv = 1.f / sqrtf(block_sum<NW>(ss, red) / (float)D + A.eps);
   T* o = (T*)A.out + (size_t)blockIdx.x * A.ldo;
-  for (int i = threadIdx.x * VEC; i < D; i += 256 * VEC) {
+  for (int i = threadIdx.x * VEC; i < D; i += NT * VEC) {
     T a[VEC];
 #pragma unroll
     for (int j = 0; j < VEC; ++j) a[j] = (T)(row[i + j] * inv * A.w_next[i + j]);
     __builtin_memcpy(__builtin_assume_aligned(o + i, sizeof(T) * VEC), a, sizeof(T) * VEC);
   }
-  for (int i = D + threadIdx.x; i < A.ldo; i += 256) o[i] = (T)0.f;
+  for (int i = D + threadIdx.x; i < A.ldo; i += NT) o[i] = (T)0.f;
 }
 
 template <typename T, int VEC>
@@ -148,21 +149,26 @@ extern "C" int pa_hyper_norm(int fp32, float* x, int S, const void* y, int K, in
   if (n <= 0) return 0;
   if (D <= 0 || D * 4 > 96 * 1024 || S < 1 || S > MAX_S) return -1;
   const Args A{x, y, y_w, y2, bias, mix, post, pre, emb, ids, w_next, out, rows, K, ldy, ldy2, vocab, ldo, D, eps};
+  // fewer rows than CUs: twice the waves to a row, all of it in one pass up to 2,048 columns (64 rows, 4 streams of 2,048:
+  // 6.8 -> 5.7 us)
+  const bool few = n <= 256 && D > 1024;
   const bool vec = D % 4 == 0 && (!y || ldy % 4 == 0) && (!y2 || ldy2 % 4 == 0) && (!out || ldo % 4 == 0);
-#define PA_HN(T, V, N)                                                                                          \
+#define PA_HN(T, V, N, W)                                                                                       \
   do {                                                                                                          \
     static bool attr = false;                                                                                   \
     if (!attr) {                                                                                                \
-      (void)hipFuncSetAttribute((const void*)hyper_norm_kernel<T, V, N>,                                        \
+      (void)hipFuncSetAttribute((const void*)hyper_norm_kernel<T, V, N, W>,                                     \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);                         \
       attr = true;                                                                                              \
     }                                                                                                           \
-    hipLaunchKernelGGL((hyper_norm_kernel<T, V, N>), dim3(n), dim3(256), (size_t)D * 4, st, A);                 \
+    hipLaunchKernelGGL((hyper_norm_kernel<T, V, N, W>), dim3(n), dim3(64 * W), (size_t)D * 4, st, A);           \
   } while (0)
 #define PA_HN_S(N)                                                             \
   case N:                                                                      \
-    if (fp32) { if (vec) PA_HN(float, 4, N); else PA_HN(float, 1, N); }        \
-    else { if (vec) PA_HN(pa::bf16, 4, N); else PA_HN(pa::bf16, 1, N); }       \
+    if (fp32) { if (vec) PA_HN(float, 4, N, 4); else PA_HN(float, 1, N, 4); }  \
+    else if (!vec) PA_HN(pa::bf16, 1, N, 4);                                   \
+    else if (few) PA_HN(pa::bf16, 4, N, 8);                                    \
+    else PA_HN(pa::bf16, 4, N, 4);                                             \
     break
   switch (S) {
     PA_HN_S(1); PA_HN_S(2); PA_HN_S(3); PA_HN_S(4); PA_HN_S(5); PA_HN_S(6); PA_HN_S(7); PA_HN_S(8);

@@ -60,6 +60,12 @@ def test_hyper_norm(device, dt, S, D, K, weighted):
     assert not o[:, D:].any()
 
 
+@pytest.mark.parametrize("S,D", [(2, 1028), (3, 2052), (1, 4100)])
+def test_hyper_norm_of_few_wide_rows(gpu, S, D):
+    """Widths around one and two passes of the wider workgroup."""
+    test_hyper_norm(gpu, BF16, S, D, 2, False)
+
+
 @kinds
 def test_softcap(device, dt):
     from pilottai_amd import ops
