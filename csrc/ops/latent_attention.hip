@@ -501,9 +501,12 @@ __device__ __forceinline__ void tile_item(const Args& A, const int4 it, char* sm
 // read serves two MFMAs: 40 KB a wave. Between the halves, a wave sends the partner its part of the
 // partner's scores and gets its own completed, does the softmax of its 16 columns, and the two trade weights. The
 // next tile's scores run ahead of this tile's outputs (three tile buffers), so softmax and outputs overlap.
-// 4,096 tokens, 16 heads, 512 + 64: 493 -> 330 us; the MFMAs alone, at 2,176 cycles a tile and CU, 116 us.
-// Left out in turn, scores, outputs, softmax and loads each give 70 to 90 us back: with two waves a SIMD and two barriers
-// a tile they overlap little. Reads 2, 3, 4 steps ahead: 365, 344, 330 us; the registers end there.
+// 4,096 tokens, 16 heads, 512 + 64: 425 -> 318 us; the MFMAs alone, at 2,176 cycles a tile and CU, 116 us: with two
+// waves a SIMD and two barriers a tile, scores, outputs, softmax and loads overlap little. Reads 2, 3, 4 steps ahead: 324,
+// 318, 321 us, and 4 prompts of 1,024 115, 114, 118: at 4 the registers end. The subtracted maximum is the true one of the
+// keys so far: the largest weight is then exactly 1 and, in 16 bits, has no rounding of its own (letting it fall behind
+// saves 10 us of rescaling, and peaked rows err up to twice as much). Of a pair's two blocks only the one whose maximum
+// moved is rescaled (both together: 337 us).
 template <int RT, int PT>
 constexpr int pair_lds_bytes() { return 3 * 32 * 32 * (RT + PT) * 2 + NW * (2048 + 2 * (1024 + 64) + (RT >= 16 ? 2048 : 0)); }
 
@@ -583,7 +586,7 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
   f32x4 sc[2];
   // both column blocks' scores over this half of the dimensions; the partner's go to LDS. Fragments are read AHEAD steps
   // before their use: left to itself the compiler, short of registers, reads each right before its MFMAs.
-  constexpr int AHEAD = 4;
+  constexpr int AHEAD = 3;
   auto scores = [&](const char* tile) {
     bf16x8 kb[AHEAD + 1];
     auto frag = [&](int i) {
@@ -609,9 +612,6 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
       if (m == NH - 1) *reinterpret_cast<f32x4*>(xs + (wid * 2 + k) * 1024 + lane * 16) = other;
     }
   };
-  // (the subtracted maximum follows the true one only when it falls LAG behind: weights stay below 2^LAG, exact in the same
-  // bits, and the outputs are seldom rescaled)
-  constexpr float LAG = 8.f;
   // softmax of the own columns' completed scores of tile t; weights and factors to LDS
   auto softmax = [&](int t) {
     bf16x8 pf;
@@ -633,8 +633,7 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
       for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, sc[k][r]);
     tmax = fmaxf(tmax, __shfl_xor(tmax, 16, 64));
     tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-    const float m_top = fmaxf(m_run, fmaxf(tmax * A.scale_log2, NEG_BIG));
-    const float m_new = m_top > m_run + LAG ? m_top : m_run;
+    const float m_new = fmaxf(m_run, fmaxf(tmax * A.scale_log2, NEG_BIG));
     const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
     m_run = m_new;
     l_run *= alpha;
@@ -710,12 +709,13 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
     const bf16x8 p[2] = {*reinterpret_cast<const bf16x8*>(xp + own * 1024 + lane * 16),
                          *reinterpret_cast<const bf16x8*>(xp + other * 1024 + lane * 16)};
     const float a0 = xa[own * 16 + c], a1 = xa[other * 16 + c];
-    if (__any(a0 != 1.f || a1 != 1.f)) {
+    if (__any(a0 != 1.f)) {
 #pragma unroll
-      for (int n = 0; n < RT; ++n) {
-        o[0][n] *= a0;
-        o[1][n] *= a1;
-      }
+      for (int n = 0; n < RT; ++n) o[0][n] *= a0;
+    }
+    if (__any(a1 != 1.f)) {
+#pragma unroll
+      for (int n = 0; n < RT; ++n) o[1][n] *= a1;
     }
     outputs(smem + cur * TILE, p);
     if (!grp && i + 1 < n_t) softmax(t_lo + i + 1);

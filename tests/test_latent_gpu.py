@@ -342,6 +342,47 @@ def test_latent_attention_item_rounds(gpu, R, r):
     run_attention(gpu, torch.bfloat16, 16, R, r, [(0, 2100), (33, 100), (500, 1), (200, 60)], 900)
 
 
+@pytest.mark.parametrize("tiles,part", [(0, 128), (64, 256)])  # whole prompts, and cut over their keys
+@pytest.mark.parametrize("H,R,r", [(16, 512, 64), (20, 256, 32), (8, 384, 0), (40, 192, 64)])
+def test_latent_attention_of_peaked_scores(gpu, H, R, r, tiles, part):
+    """Queries that point at one key, 2 to 6 nats above the others. The largest weight is exactly 1 where the running maximum
+    is the true one, so of the weights only the others' roundings (2^-9 each) move the output; its own rounding averages out
+    along the output's direction (6 sigma of steps of 2^-7 at most), and sums of 600 products in fp32 and the exponent of two
+    err by 2^-14."""
+    from pilottai_amd import ops
+    from pilottai_amd.ops.latent import latent_pad, pad_to
+
+    g, reqs, bf = torch.Generator().manual_seed(H + R), [(0, 300), (1000, 60)], torch.bfloat16
+    Rp, rp = latent_pad(R), pad_to(r, 32)
+    D, scale = Rp + rp, 1 / math.sqrt(R + r)
+    T, m, dec, tile = fed_meta(gpu, H, reqs, tiles=tiles, part=part)
+    pages = torch.randn(600, D // 8, 16, 8, generator=g).to(bf)
+    q, rows = torch.zeros(T, H, D, dtype=bf), []
+    for i, (c, n) in enumerate(reqs):
+        rows.append(pages[m["block_table"][i, :(c + n + 15) // 16].long()].permute(0, 2, 1, 3).reshape(-1, D)[:c + n])
+        at = (torch.rand(n, H, generator=g) * torch.arange(c + 1, c + n + 1)[:, None]).long()
+        nats = torch.rand(n, H, 1, generator=g) * 4 + 2
+        q[int(m["q_start"][i]):][:n] = (rows[i].float()[at] * nats / (scale * D)).to(bf)
+    NB, mi = (dec * H + 15) // 16, m["items"].shape[0]
+    out = torch.empty(T, H, Rp, dtype=bf, device=gpu)
+    po, pm = torch.empty(mi * NB * 16 * Rp, device=gpu), torch.empty(mi * NB * 32, device=gpu)
+    mg = {k: v.to(gpu) for k, v in m.items()}
+    ops.latent_attention(out, po, pm, q.to(gpu), pages.to(gpu), mg["items"], mg["n_items"], mg["q_start"], mg["q_len"],
+                         mg["ctx_len"], mg["block_table"], scale, 0, dec, tile)
+    for i, (c, n) in enumerate(reqs):
+        q0, k = int(m["q_start"][i]), rows[i].double()
+        sc = torch.matmul(q[q0:q0 + n].double().transpose(0, 1).contiguous(), k.T.contiguous()) * scale  # [H, n, keys]
+        sc.masked_fill_(torch.arange(c + n)[None, :] > torch.arange(c, c + n)[:, None], -math.inf)
+        w = torch.softmax(sc, -1)
+        want = torch.matmul(w, k[:, :Rp].contiguous())
+        size = want.square().sum(-1)
+        along = ((out[q0:q0 + n].double().cpu().transpose(0, 1) - want) * want).sum(-1) / size
+        others = w.scatter(-1, w.argmax(-1, keepdim=True), 0.0)
+        each = (others * torch.matmul(want, k[:, :Rp].T.contiguous()).abs()).sum(-1) / size
+        rounding = 6 * 2.0 ** -7 / math.sqrt(12) * want.pow(4).sum(-1).sqrt() / size
+        assert bool((along.abs() <= 2.0 ** -9 * each + rounding + 2.0 ** -14).all()), (reqs[i], float(along.abs().max()))
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("window", [0, 45])
 @pytest.mark.parametrize("step", ["decode", "mixed"])
