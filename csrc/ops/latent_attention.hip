@@ -124,8 +124,12 @@ __global__ __launch_bounds__(256) void simple_kernel(const Args A) {
 // ---------------------------------------------------------------------------
 // c^T operand: lanes 16g + i of the result hold dim i of keys 4g .. 4g + 3; each lane names the
 // 8 bytes (key 4g + i/4, dims 4 (i%4) .. + 3) of the 4 x 16 block its group transposes
-// (restrict: an intrinsic without alias information waits for every direct load to LDS in flight)
-__device__ __forceinline__ bf16x4 tr_read(const char* __restrict__ p) {
+__device__ __forceinline__ bf16x4 tr_read(const char* p) {
+  return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)p);
+}
+// The same for pair_item: without alias information the compiler waits there for the direct loads to LDS in flight. (In
+// split_item and tile_item it only orders the loop differently: 192 + 64, 4,096 tokens 171 us, without it 167.)
+__device__ __forceinline__ bf16x4 tr_read_ahead(const char* __restrict__ p) {
   return __builtin_amdgcn_ds_read_tr16_b64_v4bf16((lds_bf16x4*)p);
 }
 
@@ -508,7 +512,7 @@ __device__ __forceinline__ void tile_item(const Args& A, const int4 it, char* sm
 // saves 10 us of rescaling, and peaked rows err up to twice as much). Of a pair's two blocks only the one whose maximum
 // moved is rescaled (both together: 337 us).
 template <int RT, int PT>
-constexpr int pair_lds_bytes() { return 3 * 32 * 32 * (RT + PT) * 2 + NW * (2048 + 2 * (1024 + 64) + (RT >= 16 ? 2048 : 0)); }
+constexpr int pair_lds_bytes() { return 3 * 32 * 32 * (RT + PT) * 2 + NW * (2048 + 2 * (1024 + 64) + 2048); }
 
 template <int RT, int PT>
 __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* smem) {
@@ -527,8 +531,8 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
   const int cpos = pos0 + min(col(0), cols - 1) / A.H;
   const int klo = A.window > 0 ? max(0, cpos - A.window + 1) : 0;
   const int loff = (g * 16 + c) * 16;
-  // (the widest keep the queries of a wave's last step in LDS: with them in registers the tile loop spills)
-  constexpr int NQ = RT >= 16 ? NH - 1 : NH;
+  // (the queries of a wave's last step stay in LDS: with them in registers the tile loop spills)
+  constexpr int NQ = NH - 1;
   char* qs = smem + 3 * TILE + NW * (2048 + 2 * (1024 + 64)) + wid * 2048 + loff;
   bf16x8 qf[2][NQ];
 #pragma unroll
@@ -654,8 +658,8 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
   auto outputs = [&](const char* tile, const bf16x8 (&p)[2]) {
     bf16x4 v0[AHEAD + 1], v1[AHEAD + 1];
     auto read = [&](int n) {
-      v0[n % (AHEAD + 1)] = tr_read(tile + n * 512 + toff);
-      v1[n % (AHEAD + 1)] = tr_read(tile + D * 32 + n * 512 + toff);
+      v0[n % (AHEAD + 1)] = tr_read_ahead(tile + n * 512 + toff);
+      v1[n % (AHEAD + 1)] = tr_read_ahead(tile + D * 32 + n * 512 + toff);
     };
 #pragma unroll
     for (int n = 0; n < AHEAD; ++n) read(n);
@@ -752,7 +756,10 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
   }
 }
 
-constexpr int PAIRS = 8;  // latents of 32 * PAIRS and more: pair_item
+// Latents of 32 PAIRS and more: pair_item, on 256 workgroups. us of 16 heads, tile_item and as many workgroups as items
+// against pair_item: 512 + 64, 4 x 1,024 tokens 137, 114, 512 after 3,584 129, 108, 40 decode rows and 9 x 210 after 320
+// 77, 74; 384 + 64: 90, 91; 87, 89; 55, 61; 256 + 32: 77, 73; 76, 74; 47, 50.
+constexpr int PAIRS = 16;
 
 template <int RT, int PT>
 constexpr int lds_bytes() {
@@ -764,18 +771,26 @@ template <int RT, int PT, int CT>
 __global__ __launch_bounds__(64 * NW, 2) void mfma_kernel(const Args A) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int n = A.n_items[0];
-  // Two passes over the workgroup's items, so that neither path's registers carry the other's. Tiles are dealt in rounds
-  // over the workgroups, every second one from its end: a prompt's later items have more keys, and with one workgroup a CU
-  // each gets as many keys in all (dealt in one direction, CUs were busy two thirds of the time:
-  // 500 us at 4,096 tokens instead of 380 with the loop of then).
-  for (int r = 0, b = blockIdx.y; r * (int)gridDim.y < n; ++r, b = gridDim.y - 1 - b) {
-    const int item = r * gridDim.y + b;
-    if (item >= n) continue;
-    const int4 it = A.items[item];
-    if ((it.z & 0xff) <= A.dec_tokens) continue;
-    if constexpr (RT >= PAIRS) pair_item<RT, PT>(A, it, smem);
-    else tile_item<RT, PT, CT>(A, it, smem);
-    __syncthreads();
+  // Two passes over the workgroup's items, so that neither path's registers carry the other's.
+  if constexpr (RT >= PAIRS) {
+    // Tiles are dealt in rounds over the workgroups, every second one from its end: a prompt's later items have more keys,
+    // and with one workgroup a CU each gets as many keys in all (4,096 tokens, dealt in one direction: 341 us, CUs busy two
+    // thirds of the time; here 318).
+    for (int r = 0, b = blockIdx.y; r * (int)gridDim.y < n; ++r, b = gridDim.y - 1 - b) {
+      const int item = r * gridDim.y + b;
+      if (item >= n) continue;
+      const int4 it = A.items[item];
+      if ((it.z & 0xff) <= A.dec_tokens) continue;
+      pair_item<RT, PT>(A, it, smem);
+      __syncthreads();
+    }
+  } else {
+    for (int item = blockIdx.y; item < n; item += gridDim.y) {
+      const int4 it = A.items[item];
+      if ((it.z & 0xff) <= A.dec_tokens) continue;
+      tile_item<RT, PT, CT>(A, it, smem);
+      __syncthreads();
+    }
   }
   for (int item = blockIdx.y; item < n; item += gridDim.y) {
     const int4 it = A.items[item];
