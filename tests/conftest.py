@@ -16,6 +16,13 @@ def pytest_configure(config):
 
 
 @pytest.hookimpl(tryfirst=True)
+def pytest_collection_modifyitems(items):
+    for item in items:  # (before -m selects)
+        if "gpu" in getattr(item, "fixturenames", ()):
+            item.add_marker(pytest.mark.gpu)
+
+
+@pytest.hookimpl(tryfirst=True)
 def pytest_pyfunc_call(pyfuncitem):
     """Run `async def` tests on a fresh event loop (pytest-asyncio is not installed)."""
     fn = pyfuncitem.obj

@@ -60,6 +60,7 @@ def test_hyper_norm(device, dt, S, D, K, weighted):
     assert not o[:, D:].any()
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("S,D", [(2, 1028), (3, 2052), (1, 4100)])
 def test_hyper_norm_of_few_wide_rows(gpu, S, D):
     """Widths around one and two passes of the wider workgroup."""
@@ -405,6 +406,7 @@ def test_state_scan_portions(gpu, V, N, lens):
     assert float((err - 2e-4 * after.abs()).max()) < 2e-4 * float(after.abs().mean()) + 2 * 2.0 ** -8 * float(most)
 
 
+@pytest.mark.gpu
 def test_state_scan_keeps_the_state_in_fp32(gpu):
     """The state a chunked portion leaves equals the one that single tokens leave to fp32's order, not bf16's."""
     from pilottai_amd import ops
