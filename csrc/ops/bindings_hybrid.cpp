@@ -29,10 +29,10 @@ int pa_matrix_memory(int fp32, const void* x, int ldx, void* y, int ldy, float* 
                      const int* ctx_len, const int* state_slot, const int* items, const int* n_items, int max_items, int seqs,
                      int H, int V, int N, int cq, int ck, int cv, int ci, int vin, int vdim, float cap, float q_scale,
                      int scan_min, hipStream_t st);
-int pa_state_scan(int fp32, const void* proj, int ldp, void* u, void* y, int ldy, float* state, void* ring,
-                  const float* conv_w, const float* conv_b, const float* dt_bias, const float* a,
-                  const float* d, const int* q_start, const int* q_len, const int* ctx_len, const int* state_slot,
-                  const int* scan_first, const int* items, const int* n_items, int max_items, int seqs, int H, int G,
+int pa_state_scan(int fp32, const void* proj, int ldp, void* u, void* y, int ldy, float* state, void* ring, float* work,
+                  float* total, float chain, float fixed, const float* conv_w, const float* conv_b, const float* dt_bias,
+                  const float* a, const float* d, const int* q_start, const int* q_len, const int* ctx_len,
+                  const int* state_slot, const int* items, const int* n_items, int max_items, int seqs, int H, int G,
                   int V, int N, int taps, int ring_rows, int scan_min, hipStream_t st);
 }
 
@@ -198,9 +198,9 @@ void head_difference(at::Tensor a, at::Tensor out, at::Tensor gate, int64_t grou
            "head_difference");
 }
 
-void state_scan(at::Tensor proj, at::Tensor u, at::Tensor y, at::Tensor state, at::Tensor ring,
-                at::Tensor conv_w, at::Tensor conv_b, at::Tensor dt_bias, at::Tensor a, at::Tensor d,
-                at::Tensor q_start, at::Tensor q_len, at::Tensor ctx_len, at::Tensor state_slot, at::Tensor scan_first,
+void state_scan(at::Tensor proj, at::Tensor u, at::Tensor y, at::Tensor state, at::Tensor ring, Opt work, Opt total,
+                double chain, double fixed, at::Tensor conv_w, at::Tensor conv_b, at::Tensor dt_bias, at::Tensor a,
+                at::Tensor d, at::Tensor q_start, at::Tensor q_len, at::Tensor ctx_len, at::Tensor state_slot,
                 at::Tensor items, at::Tensor n_items, int64_t max_items, int64_t seqs, int64_t G, int64_t scan_min) {
   const int f = is_f32(proj, "proj");
   check_rows(proj, proj.scalar_type(), "proj");
@@ -220,12 +220,14 @@ void state_scan(at::Tensor proj, at::Tensor u, at::Tensor y, at::Tensor state, a
     check_gpu(u, "u");
     check_dtype(u, proj.scalar_type(), "u");
     TORCH_CHECK(u.numel() >= T * Cc, "u must be [T, channels]");
+    TORCH_CHECK(work.has_value() == total.has_value(), "state_scan: work and total go together");
   }
   check_rc(pa_state_scan(f, proj.data_ptr(), proj.stride(0), u.data_ptr(), y.data_ptr(), y.stride(0),
-                         state.data_ptr<float>(), ring.data_ptr(), opt_f32(conv_w, 0, "conv_w"), opt_f32(conv_b, Cc, "conv_b"),
+                         state.data_ptr<float>(), ring.data_ptr(), (float*)opt_f32(work, max_items * H * V * N, "work"),
+                         (float*)opt_f32(total, max_items * H + 1, "total"), (float)chain, (float)fixed, opt_f32(conv_w, 0, "conv_w"), opt_f32(conv_b, Cc, "conv_b"),
                          opt_f32(dt_bias, H, "dt_bias"), opt_f32(a, H, "a"), opt_f32(d, H, "d"),
                          ints(q_start, seqs, "q_start"), ints(q_len, seqs, "q_len"), ints(ctx_len, seqs, "ctx_len"),
-                         ints(state_slot, seqs, "state_slot"), ints(scan_first, seqs, "scan_first"),
+                         ints(state_slot, seqs, "state_slot"),
                          ints(items, 0, "items"), ints(n_items, 1, "n_items"), max_items, seqs, H, G, V, N,
                          conv_w.size(0), ring.size(1), scan_min, cur_stream()),
            "state_scan");

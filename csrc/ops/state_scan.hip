@@ -17,10 +17,11 @@
 //   conv_kernel   u for all their rows
 //   scan_kernel   y_i = exp(l_i) C_i . S + sum_{j <= i} exp(l_i - l_j) dt_j (C_i . B_j) x_j + D x_i,
 //                 S <- exp(L) S + sum_j exp(L - l_j) dt_j B_j x_j^T, chunk after chunk
+//   or the same in three launches, each over all chunks: chunk_state_kernel, state_pass_kernel, chunk_out_kernel
 // The MFMA operands are bf16. B, C and x are bf16 values; everything that carries a decay, a step size or
 // the state goes in as a pair of bf16 (value and remainder), 16 bits of mantissa: the recurrence keeps
 // the accuracy of fp32 to that order, and chunked and stepped portions agree.
-// fp32 models, and N above 256: conv_kernel and step_kernel for long portions too.
+// fp32 models: conv_kernel and step_kernel for long portions too.
 #include "common.h"
 
 #include <algorithm>
@@ -40,10 +41,14 @@ struct Args {
   void* ring;              // [slots, RING, Cc]
   const void* conv_w;      // [taps, Cc] fp32, oldest first
   const float *conv_b, *dt_bias, *a, *d;
-  const int *q_start, *q_len, *ctx_len, *state_slot, *scan_first;
+  const int *q_start, *q_len, *ctx_len, *state_slot;
   const int4* items;
   const int* n_items;
-  int ldp, ldy, H, G, V, N, Cc, taps, RING, scan_min, max_seqs, long_too, vsplit;
+  int ldp, ldy, H, G, V, N, Cc, taps, RING, scan_min, long_too, vsplit;
+  float* work;   // [items, H, V, N]: every chunk's state
+  float* total;  // [items, H]: a chunk's summed log2 decay
+  int* form;     // null, or 1 where the step's long portions go through the three launches, else 0 (pick_form)
+  float chain, fixed;
 };
 
 template <typename T>
@@ -58,8 +63,25 @@ __device__ __forceinline__ void split(float x, bf16& hi, bf16& lo) {
 }
 
 // ---- convolution of long portions: 8 channels x 16 tokens a thread ---------------------------------
+// Which form the step's long portions take (one wave): the chain of the longest one's chunks, or all chunks' work.
+__device__ __forceinline__ void pick_form(const Args& A) {
+  const int n_items = A.n_items[0], lane = threadIdx.x;
+  int most = 0;
+  for (int i = lane; i < n_items; i += 64) {
+    const int4 it = A.items[i];
+    if (it.y == 0) most = max(most, (A.q_len[it.x] + LC - 1) / LC);
+  }
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) most = max(most, __shfl_xor(most, o, 64));
+  if (lane == 0) A.form[0] = A.chain * most > A.fixed + n_items;
+}
+
 template <typename T, int TAPS>
 __global__ __launch_bounds__(256) void conv_kernel(const Args A) {
+  if (A.form && blockIdx.x == gridDim.x - 1) {  // (a column of workgroups past the channels)
+    if (blockIdx.y == 0 && threadIdx.x < 64) pick_form(A);
+    return;
+  }
   const int c8 = (blockIdx.x * 64 + (threadIdx.x & 63)) * 8, sub = threadIdx.x >> 6;
   if (c8 >= A.Cc) return;
   const int inner = A.H * A.V;
@@ -307,6 +329,7 @@ __global__ __launch_bounds__(256, 2) void scan_kernel(const Args A) {
   using L = ScanLds<NK>;
   extern __shared__ __attribute__((aligned(16))) char smem[];
   static_assert(NK * VT % 2 == 0, "every wave keeps as many blocks");
+  if (A.form && A.form[0]) return;
   constexpr int PAIRS = NK * VT / 2;  // 16 x 16 blocks of the state a wave keeps
   // heads of a group, which share B and C, on one XCD
   const int parts = gridDim.x / A.H, per = gridDim.x >> 3;
@@ -512,25 +535,328 @@ __global__ __launch_bounds__(256, 2) void scan_kernel(const Args A) {
   }
 }
 
+// ---- the same in three launches: every chunk on its own -----------------------------------------------
+// For states wider than scan_kernel is built for, and for few heads, whose portions leave it few workgroups that each walk
+// all chunks in turn. Two of the three launches run all chunks at once, and every chunk's state goes through memory.
+// A token's step size before softplus (wave 0), rows past the end whatever the last one has
+__device__ __forceinline__ float load_step(const Args& A, int h, int row0, int n) {
+  if (threadIdx.x >= 64) return 0.f;
+  return (float)((const bf16*)A.proj)[(size_t)(row0 + min((int)threadIdx.x, n - 1)) * A.ldp + A.H * A.V + A.Cc + h] + A.dt_bias[h];
+}
+// 8 columns of one of a chunk's rows (unit e of D / 8 columns x 64 rows); rows past the end repeat the
+// last one, and meet weights of 0
+__device__ __forceinline__ bf16x8 load_cols(const bf16* u, int ld, int e, int D, int n) {
+  return *reinterpret_cast<const bf16x8*>(u + (size_t)min(e & (LC - 1), n - 1) * ld + min((e >> 6) * 8, D - 8));
+}
+constexpr int XB = 2, BB = 4, SB = 8;  // units of x, B and the state that a thread loads ahead
+
+// U_c = sum_j exp(L - l_j) dt_j B_j x_j^T of every chunk
+__global__ __launch_bounds__(256) void chunk_state_kernel(const Args A) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  if (A.form && !A.form[0]) return;
+  const int h = blockIdx.x, n_items = A.n_items[0];
+  const int V = A.V, N = A.N, g = h / (A.H / A.G), inner = A.H * V;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, lg = lane >> 4, c = lane & 15;
+  float *dt = (float*)smem, *l = dt + LC;
+  bf16* bt = (bf16*)(smem + 2 * LC * 4);  // [N][LD]: B transposed
+  bf16 *xh = bt + N * LD, *xl = xh + V * LD;  // [V][LD]: weighted x transposed, value and remainder
+  for (int item = blockIdx.y; item < n_items; item += gridDim.y) {
+    const int4 it = A.items[item];
+    const int n = it.z, row0 = A.q_start[it.x] + it.y;
+    const bf16 *ux = (const bf16*)A.u + (size_t)row0 * A.Cc + h * V, *ub = (const bf16*)A.u + (size_t)row0 * A.Cc + inner + g * N;
+    const float raw = load_step(A, h, row0, n);
+    bf16x8 xv[XB], bv[BB];
+#pragma unroll
+    for (int i = 0; i < BB; ++i) bv[i] = load_cols(ub, A.Cc, threadIdx.x + 256 * i, N, n);
+#pragma unroll
+    for (int i = 0; i < XB; ++i) xv[i] = load_cols(ux, A.Cc, threadIdx.x + 256 * i, V, n);
+    __syncthreads();
+    chunk_steps(raw, A.a[h], n, dt, l);
+    auto put_b = [&](int e, const bf16x8& b) {
+      const int j = e & (LC - 1), i = (e >> 6) * 8;
+      if (i >= N) return;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) bt[(i + k) * LD + j] = b[k];
+    };
+#pragma unroll
+    for (int i = 0; i < BB; ++i) put_b(threadIdx.x + 256 * i, bv[i]);
+    for (int e = threadIdx.x + 256 * BB; e < (N >> 3) * LC; e += 256) put_b(e, load_cols(ub, A.Cc, e, N, n));
+    __syncthreads();
+    const float end = l[LC - 1];
+    auto put_x = [&](int e, const bf16x8& x) {
+      const int j = e & (LC - 1), i = (e >> 6) * 8;
+      if (i >= V) return;
+      const float w = j < n ? dt[j] * __builtin_amdgcn_exp2f(end - l[j]) : 0.f;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) {
+        bf16 hi, lo;
+        split(w * (float)x[k], hi, lo);
+        xh[(i + k) * LD + j] = hi;
+        xl[(i + k) * LD + j] = lo;
+      }
+    };
+#pragma unroll
+    for (int i = 0; i < XB; ++i) put_x(threadIdx.x + 256 * i, xv[i]);
+    for (int e = threadIdx.x + 256 * XB; e < (V >> 3) * LC; e += 256) put_x(e, load_cols(ux, A.Cc, e, V, n));
+    __syncthreads();
+    float* out = A.work + ((size_t)item * A.H + h) * V * N;
+    const int tn = N >> 4, tv = V >> 4;
+    for (int t = wid; t < tn * tv; t += 4) {
+      const int n0 = (t % tn) * 16, v0 = (t / tn) * 16;
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const bf16x8 b = *reinterpret_cast<const bf16x8*>(bt + (n0 + c) * LD + 32 * k + 8 * lg);
+        const bf16x8 x0 = *reinterpret_cast<const bf16x8*>(xh + (v0 + c) * LD + 32 * k + 8 * lg);
+        const bf16x8 x1 = *reinterpret_cast<const bf16x8*>(xl + (v0 + c) * LD + 32 * k + 8 * lg);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, x0, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, x1, acc, 0, 0, 0);
+      }
+      *reinterpret_cast<f32x4*>(out + (size_t)(v0 + c) * N + n0 + 4 * lg) = acc;
+    }
+    if (threadIdx.x == 0) A.total[(size_t)item * A.H + h] = end;
+  }
+}
+
+// The state before every chunk, in place of U_c, and the last one to the slot: 4 values a thread, chunk after chunk; the next 8 chunks are on their way while 8 are written
+__global__ __launch_bounds__(256) void state_pass_kernel(const Args A) {
+  const int h = blockIdx.z, VN = A.V * A.N, e = (blockIdx.x * 256 + threadIdx.x) * 4, n_items = A.n_items[0];
+  if (e >= VN || (A.form && !A.form[0])) return;
+  const size_t step = (size_t)A.H * VN;
+  for (int item = blockIdx.y; item < n_items; item += gridDim.y) {
+    const int4 it = A.items[item];
+    if (it.y != 0) continue;  // a portion's first item takes all of them
+    const int s = it.x, n = A.q_len[s], chunks = (n + LC - 1) / LC;
+    float* S = A.state + ((size_t)A.state_slot[s] * A.H + h) * VN + e;
+    f32x4 st = {0.f, 0.f, 0.f, 0.f};
+    if (A.ctx_len[s] > n) st = *reinterpret_cast<const f32x4*>(S);
+    float* w = A.work + ((size_t)item * A.H + h) * VN + e;
+    const float* tot = A.total + (size_t)item * A.H + h;
+    f32x4 u[8], un[8];
+    float d[8], dn[8];
+    auto load = [&](int c0, f32x4 (&uu)[8], float (&ddd)[8]) {
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        const int k = min(c0 + i, chunks - 1);
+        uu[i] = *reinterpret_cast<const f32x4*>(w + k * step);
+        ddd[i] = tot[(size_t)k * A.H];
+      }
+    };
+    load(0, u, d);
+    for (int c0 = 0; c0 < chunks; c0 += 8) {
+      if (c0 + 8 < chunks) load(c0 + 8, un, dn);
+#pragma unroll
+      for (int i = 0; i < 8; ++i)
+        if (c0 + i < chunks) {
+          *reinterpret_cast<f32x4*>(w + (c0 + i) * step) = st;
+          const float f = __builtin_amdgcn_exp2f(d[i]);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) st[j] = st[j] * f + u[i][j];
+        }
+#pragma unroll
+      for (int i = 0; i < 8; ++i) {
+        u[i] = un[i];
+        d[i] = dn[i];
+      }
+    }
+    *reinterpret_cast<f32x4*>(S) = st;
+  }
+}
+
+// Outputs of every chunk. STAGED: the incoming state is split into LDS once; otherwise every wave reads it from memory.
+// NK: N / 32 as a constant, for which C stays in registers and B's loads go out together; 0: any N.
+template <bool STAGED, int NK>
+__global__ __launch_bounds__(256) void chunk_out_kernel(const Args A) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  if (A.form && !A.form[0]) return;
+  const int h = blockIdx.x, n_items = A.n_items[0];
+  const int V = A.V, N = NK ? 32 * NK : A.N, g = h / (A.H / A.G), inner = A.H * V, NL = N + 8;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, lg = lane >> 4, c = lane & 15;
+  float *dt = (float*)smem, *l = dt + LC;
+  bf16 *mh = (bf16*)(smem + 2 * LC * 4), *ml = mh + LC * LD;  // [i][LD], value and remainder
+  bf16* xt = ml + LC * LD;                                    // [V][LD]
+  bf16 *sh = xt + V * LD, *sl = sh + V * NL;                  // [V][NL], value and remainder
+  for (int item = blockIdx.y; item < n_items; item += gridDim.y) {
+    const int4 it = A.items[item];
+    const int n = it.z, row0 = A.q_start[it.x] + it.y;
+    const bf16* u = (const bf16*)A.u + (size_t)row0 * A.Cc;
+    const float* S = A.work + ((size_t)item * A.H + h) * V * N;
+    // (rows past the end repeat the last one; their results are dropped)
+    const int i = 16 * wid + c, ri = min(i, n - 1);
+    const bf16* cr = u + (size_t)ri * A.Cc + inner + A.G * N + g * N + 8 * lg;
+    const bf16* ux = u + h * V;
+    const float raw = load_step(A, h, row0, n);
+    bf16x8 cf[NK ? NK : 1], xv[XB];
+    f32x4 cb[4];  // C_i . B_j
+    f32x4 sv[STAGED ? SB : 1];
+#pragma unroll
+    for (int k = 0; k < XB; ++k) xv[k] = load_cols(ux, A.Cc, threadIdx.x + 256 * k, V, n);
+    auto load_state = [&](int e) { return *reinterpret_cast<const f32x4*>(S + min(e, V * N - 4)); };
+    if constexpr (STAGED) {
+#pragma unroll
+      for (int k = 0; k < SB; ++k) sv[k] = load_state(1024 * k + threadIdx.x * 4);
+    }
+    if constexpr (NK > 0) {
+#pragma unroll
+      for (int k = 0; k < NK; ++k) cf[k] = *reinterpret_cast<const bf16x8*>(cr + 32 * k);
+#pragma unroll
+      for (int jt = 0; jt < 4; ++jt) {
+        cb[jt] = f32x4{0.f, 0.f, 0.f, 0.f};
+        if (jt <= wid) {
+          const bf16* br = u + (size_t)min(16 * jt + c, n - 1) * A.Cc + inner + g * N + 8 * lg;
+          bf16x8 bf[NK ? NK : 1];
+#pragma unroll
+          for (int k = 0; k < NK; ++k) bf[k] = *reinterpret_cast<const bf16x8*>(br + 32 * k);
+#pragma unroll
+          for (int k = 0; k < NK; ++k) cb[jt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[k], cf[k], cb[jt], 0, 0, 0);
+        }
+      }
+    }
+    __syncthreads();
+    chunk_steps(raw, A.a[h], n, dt, l);
+    auto put_x = [&](int e, const bf16x8& x) {
+      const int j = e & (LC - 1), i = (e >> 6) * 8;
+      if (i >= V) return;
+#pragma unroll
+      for (int k = 0; k < 8; ++k) xt[(i + k) * LD + j] = x[k];
+    };
+#pragma unroll
+    for (int k = 0; k < XB; ++k) put_x(threadIdx.x + 256 * k, xv[k]);
+    for (int e = threadIdx.x + 256 * XB; e < (V >> 3) * LC; e += 256) put_x(e, load_cols(ux, A.Cc, e, V, n));
+    if constexpr (STAGED) {
+      auto put_state = [&](int e, const f32x4& v) {
+        if (e >= V * N) return;
+        const int r = e / N, k0 = e - r * N;
+        bf16x4 hi, lo;
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          bf16 a, b;
+          split(v[k], a, b);
+          hi[k] = a;
+          lo[k] = b;
+        }
+        *reinterpret_cast<bf16x4*>(sh + r * NL + k0) = hi;
+        *reinterpret_cast<bf16x4*>(sl + r * NL + k0) = lo;
+      };
+#pragma unroll
+      for (int k = 0; k < SB; ++k) put_state(1024 * k + threadIdx.x * 4, sv[k]);
+      for (int e = 1024 * SB + threadIdx.x * 4; e < V * N; e += 1024) put_state(e, load_state(e));
+    }
+    __syncthreads();
+    // M[i][j] = exp(l_i - l_j) dt_j (C_i . B_j), a lane's row i, its columns j = 16 jt + 4 lg ..
+    const float li = l[i];
+#pragma unroll
+    for (int jt = 0; jt < 4; ++jt) {
+      bf16x4 hi = {(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f}, lo = hi;
+      if (jt <= wid) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+        if constexpr (NK > 0) {
+          acc = cb[jt];
+        } else {
+          const bf16* br = u + (size_t)min(16 * jt + c, n - 1) * A.Cc + inner + g * N + 8 * lg;
+          for (int k = 0; k < N; k += 32)
+            acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(br + k),
+                                                          *reinterpret_cast<const bf16x8*>(cr + k), acc, 0, 0, 0);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int j = 16 * jt + 4 * lg + r;
+          bf16 a, b;
+          split(j <= i ? acc[r] * (__builtin_amdgcn_exp2f(li - l[j]) * dt[j]) : 0.f, a, b);
+          hi[r] = a;
+          lo[r] = b;
+        }
+      }
+      *reinterpret_cast<bf16x4*>(mh + i * LD + 16 * jt + 4 * lg) = hi;
+      *reinterpret_cast<bf16x4*>(ml + i * LD + 16 * jt + 4 * lg) = lo;
+    }
+    __syncthreads();
+    bf16x8 m0[2], m1[2];
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      m0[k] = *reinterpret_cast<const bf16x8*>(mh + i * LD + 32 * k + 8 * lg);
+      m1[k] = *reinterpret_cast<const bf16x8*>(ml + i * LD + 32 * k + 8 * lg);
+    }
+    const float ei = __builtin_amdgcn_exp2f(li), dd = A.d[h];
+    for (int v0 = 0; v0 < V; v0 += 16) {
+      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+      auto from_state = [&](int k) {
+        bf16x8 s0, s1;
+        if (STAGED) {
+          s0 = *reinterpret_cast<const bf16x8*>(sh + (v0 + c) * NL + k + 8 * lg);
+          s1 = *reinterpret_cast<const bf16x8*>(sl + (v0 + c) * NL + k + 8 * lg);
+        } else {
+          const float* p = S + (size_t)(v0 + c) * N + k + 8 * lg;
+#pragma unroll
+          for (int q = 0; q < 8; ++q) {
+            bf16 a, b;
+            split(p[q], a, b);
+            s0[q] = a;
+            s1[q] = b;
+          }
+        }
+        const bf16x8 cv = NK ? cf[NK ? k / 32 : 0] : *reinterpret_cast<const bf16x8*>(cr + k);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s0, cv, acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(s1, cv, acc, 0, 0, 0);
+      };
+      if constexpr (NK > 0) {
+#pragma unroll
+        for (int k = 0; k < NK; ++k) from_state(32 * k);
+      } else {
+        for (int k = 0; k < N; k += 32) from_state(k);
+      }
+      acc *= ei;
+#pragma unroll
+      for (int k = 0; k < 2; ++k) {
+        const bf16x8 x = *reinterpret_cast<const bf16x8*>(xt + (v0 + c) * LD + 32 * k + 8 * lg);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, m0[k], acc, 0, 0, 0);
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(x, m1[k], acc, 0, 0, 0);
+      }
+      if (i < n) {
+        bf16x4 o;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = (bf16)(acc[r] + dd * (float)xt[(v0 + 4 * lg + r) * LD + i]);
+        *reinterpret_cast<bf16x4*>((bf16*)A.y + (size_t)(row0 + i) * A.ldy + h * V + v0 + 4 * lg) = o;
+      }
+    }
+    if (it.y == 0) {  // the portion's first chunk: this head's share of the channels
+      const int per = (A.Cc + A.H - 1) / A.H;
+      store_ring<bf16>(A, it.x, min(A.Cc, h * per), min(A.Cc, (h + 1) * per));
+    }
+  }
+}
+
 }  // namespace ss
 }  // namespace pa
 
-// max_items: room of the scan items; 0 when no portion of this launch can be longer than scan_min
+// max_items: room of the scan items; 0 when no portion of this launch can be longer than scan_min. work [max_items, H, V, N]
+// and total [max_items * H + 1]: null where chunks need not go through memory; they must be there for bf16 and N above 256.
+// With N up to 256 the step's portions then choose: three launches if chain * (the longest one's chunks) > fixed + all chunks.
 extern "C" int pa_state_scan(int fp32, const void* proj, int ldp, void* u, void* y, int ldy, float* state, void* ring,
-                             const float* conv_w, const float* conv_b, const float* dt_bias,
-                             const float* a, const float* d, const int* q_start, const int* q_len, const int* ctx_len,
-                             const int* state_slot, const int* scan_first, const int* items, const int* n_items,
+                             float* work, float* total, float chain, float fixed, const float* conv_w, const float* conv_b,
+                             const float* dt_bias, const float* a, const float* d, const int* q_start, const int* q_len,
+                             const int* ctx_len, const int* state_slot, const int* items, const int* n_items,
                              int max_items, int seqs, int H, int G, int V, int N, int taps, int ring_rows,
                              int scan_min, hipStream_t st) {
   using namespace pa::ss;
   if (seqs <= 0) return 0;
   if (V % 16 || N % 32 || H % G || scan_min > MAX_SHORT || ring_rows < taps - 1 + scan_min || (taps != 4 && taps != 8)) return -1;  // (shorter ones are padded)
   Args A{proj, u, y, state, ring, conv_w, conv_b, dt_bias, a, d, q_start, q_len, ctx_len, state_slot,
-         scan_first, (const int4*)items, n_items, ldp, ldy, H, G, V, N, H * V + 2 * G * N, taps, ring_rows, scan_min,
-         seqs, fp32 || N > 256, 1};
+         (const int4*)items, n_items, ldp, ldy, H, G, V, N, H * V + 2 * G * N, taps, ring_rows, scan_min, fp32, 1,
+         work, total, nullptr, chain, fixed};
   if (A.Cc % 8 || ldp % 8) return -1;
+  // the three launches: (bf16) states that scan_kernel is not built for, or a choice
+  const int lds_s = 2 * LC * 4 + (N + 2 * V) * LD * 2;
+  const int lds_o = 2 * LC * 4 + (2 * LC + V) * LD * 2, staged = lds_o + 2 * V * (N + 8) * 2;
+  constexpr int MAX_LDS = 160 * 1024;
+  const bool fits = lds_s <= MAX_LDS && lds_o <= MAX_LDS, wide = N > 256, three = !fp32 && max_items > 0 && work && fits;
+  if (!fp32 && wide && !three) {
+    if (max_items > 0 && fits) return -1;  // (no workspace)
+    A.long_too = 1;
+  }
+  if (three && !wide) A.form = (int*)(total + (size_t)max_items * H);
   if (max_items > 0) {
-    const dim3 grid((A.Cc / 8 + 63) / 64, std::min(max_items, 4096));
+    const dim3 grid((A.Cc / 8 + 63) / 64 + (A.form ? 1 : 0), std::min(max_items, 4096));
 #define PA_CONV(T)                                                                                        \
   do {                                                                                                    \
     if (taps == 4) hipLaunchKernelGGL((conv_kernel<T, 4>), grid, dim3(256), 0, st, A);                    \
@@ -562,6 +888,34 @@ extern "C" int pa_state_scan(int fp32, const void* proj, int ldp, void* u, void*
 #undef PA_STEP
 #undef PA_STEP_N
   if (A.long_too || max_items <= 0) return (int)hipGetLastError();
+  if (three) {
+    static bool attr = false;
+    if (!attr) {
+      (void)hipFuncSetAttribute((const void*)chunk_state_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS);
+      attr = true;
+    }
+    const dim3 grid(H, std::min(max_items, 4096));
+    hipLaunchKernelGGL(chunk_state_kernel, grid, dim3(256), lds_s, st, A);
+    hipLaunchKernelGGL(state_pass_kernel, dim3((V * N / 4 + 255) / 256, std::min(max_items, 16), H), dim3(256), 0, st, A);
+    const bool in_lds = staged <= 80 * 1024;
+    const int lds = in_lds ? staged : lds_o;
+#define PA_OUT(S, K)                                                                                                       \
+  do {                                                                                                                     \
+    static bool set = false;                                                                                               \
+    if (!set) {                                                                                                            \
+      (void)hipFuncSetAttribute((const void*)chunk_out_kernel<S, K>, hipFuncAttributeMaxDynamicSharedMemorySize, MAX_LDS); \
+      set = true;                                                                                                          \
+    }                                                                                                                      \
+    hipLaunchKernelGGL((chunk_out_kernel<S, K>), grid, dim3(256), lds, st, A);                                             \
+  } while (0)
+    if (!in_lds) PA_OUT(false, 0);
+    else if (N == 32) PA_OUT(true, 1);
+    else if (N == 64) PA_OUT(true, 2);
+    else if (N == 128) PA_OUT(true, 4);
+    else PA_OUT(true, 0);
+#undef PA_OUT
+    if (wide) return (int)hipGetLastError();
+  }
   // portions loop over the grid's rows
 #define PA_SCAN(K)                                                                                                        \
   do {                                                                                                                    \

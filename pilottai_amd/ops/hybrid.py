@@ -7,7 +7,7 @@ ops/reference.py. Every function takes its constants as arguments and works in b
 """
 from __future__ import annotations
 
-from typing import Optional
+from typing import Optional, Tuple
 
 import torch
 
@@ -115,7 +115,8 @@ def head_difference(a, out, gate, groups: int, lam: float, gain: float, vdim: in
 def state_scan(proj, y, state, ring, conv_w, conv_b, dt_bias, a, d, q_start, q_len, ctx_len, state_slot, scan_first,
                scan_items, n_scan, groups: int, scan_min: int = SCAN_MIN, num_seqs: Optional[int] = None):
     """Convolution, silu and the recurrence S <- exp(-a dt) S + dt B x^T, y = S^T C + d x over the step's
-    portions, from and to the sequences' state slots (csrc/ops/state_scan.hip). proj rows [z | x | B | C | dt]."""
+    portions, from and to the sequences' state slots (csrc/ops/state_scan.hip). proj rows [z | x | B | C | dt];
+    scan_first, every portion's first item, is not read (items name their portions)."""
     H, V, N = state.shape[1:]
     if not _on_gpu(proj):
         ref.state_scan(proj, y, state, ring, conv_w, conv_b, dt_bias, a, d, q_start, q_len, ctx_len, state_slot, groups,
@@ -126,10 +127,28 @@ def state_scan(proj, y, state, ring, conv_w, conv_b, dt_bias, a, d, q_start, q_l
     items = 0 if T <= scan_min else min(scan_items.shape[0], T // SCAN_CHUNK + min(seqs, T // (scan_min + 1)) + 1)
     new = lambda dt, *s: torch.empty(*s, dtype=dt, device=proj.device)  # noqa: E731
     u = new(proj.dtype, T if items else 0, ring.shape[2])
-    require_hybrid().state_scan(proj, u, y, state, ring, conv_w, conv_b, dt_bias, a, d, q_start, q_len, ctx_len,
-                                state_slot, scan_first, scan_items, n_scan, int(items), int(seqs), int(groups),
-                                int(scan_min))
+    chain, chunk, fixed = scan_times(H, V, N)
+    chunks = bool(items) and proj.dtype == torch.bfloat16 and \
+        (N > SCAN_MAX_N or (chain - chunk) * (T // SCAN_CHUNK) > fixed + SCAN_IDLE[0])
+    work, total = (new(torch.float32, items * H * V * N), new(torch.float32, items * H + 1)) if chunks else (None, None)
+    require_hybrid().state_scan(proj, u, y, state, ring, work, total, chain / chunk, (fixed - SCAN_IDLE[1]) / chunk, conv_w,
+                                conv_b, dt_bias, a, d, q_start, q_len, ctx_len, state_slot, scan_items, n_scan, int(items),
+                                int(seqs), int(groups), int(scan_min))
     return y
+
+
+SCAN_MAX_N = 256  # the widest state that one launch holds from chunk to chunk
+# us of the launches that find that the other form was chosen: the three, and what they take more than the one
+SCAN_IDLE = (8, 5)
+
+
+def scan_times(H: int, V: int, N: int) -> Tuple[float, float, float]:
+    """us of a chunk where one launch takes a portion's chunks in turn, of a chunk of any portion where three launches take
+    all chunks at once, and of the latter beside their chunks. Where a step's rows might be one portion for which the three
+    are faster, the portions on the device decide (state_scan.hip pick_form). us of one launch, three, and the choice between
+    them: 8 heads of 64 x 128, a prompt of 4,096 tokens 193, 72, 73, 8 of 450 46, 64, 52; 32 heads 196, 140, 140 and 64, 135,
+    74; 64 heads 202, 238 and 106, 250 (never offered)."""
+    return 1 + N / 64, max(0.2, H * V * (3.7e-4 + 3.3e-6 * N)), 8 + N / 20
 
 
 def matrix_memory(x, y, div, state, top, i_bias, f_bias, q_start, q_len, ctx_len, state_slot, scan_items, n_scan, cols,

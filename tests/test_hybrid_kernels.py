@@ -357,7 +357,9 @@ def test_state_scan(device, dt, H, V, N, G, taps):
 @pytest.mark.parametrize("V,N,lens", [
     (48, 128, [9 + 7 * (i % 9) for i in range(41)]),           # more portions than the grid has rows for
     (16, 64, [64, 128, 65, 127, 1, 8, 9]), (64, 160, [63, 200]),  # whole chunks and one past; columns past N
-    (32, 288, [130, 20])])                                     # a state that is stepped through instead
+    (32, 288, [130, 20, 64, 1]),                               # a state too wide for one launch
+    (64, 128, [1, 1700, 9]), (32, 32, [1025, 64]),             # one long portion of few heads: three launches
+    (64, 128, [200, 190, 1] * 3), (64, 64, [150] * 8)])        # several shorter ones: one launch, where three were possible
 def test_state_scan_portions(gpu, V, N, lens):
     """Portions of one step, every second one from a state, against a pass in fp64 over the same convolved rows."""
     from pilottai_amd import ops
