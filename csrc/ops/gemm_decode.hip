@@ -501,6 +501,17 @@ static int dispatch_rows(const DgArgs& a, hipStream_t st) {
   return 1;
 }
 
+// Of up to 64 rows, where x through LDS pays for its stages (us, decode_gemm_kernel against decode_rows_kernel): not up to
+// 24 rows, of which the other kernel reads only those there are (17 x 2048 x 8192 15.9, 19.8; 24 18.7, 19.9) unless the
+// outputs fill the chip several times (24 x 10368 x 2048 14.7, 12.3; x 8192 48.8, 40.0), and not for few k (64 x 2048 x 256
+// 4.1, 4.0; 48 x 8192 x 256 4.9, 5.6, x 512 5.9, 6.3, x 768 7.6, 7.5; 64 x 2048 x 512 5.3, 4.3, 32 4.1, 4.4). Wide outputs that not even
+// 64 columns a tile leave one workgroup a CU stream either way (64 x 28672 x 128 10.0, 7.7; x 4096 69, 51).
+static bool rows_pay(const DgArgs& a) {
+  if (a.M <= 16) return false;
+  if (a.M <= 24) return a.N > 8192 && a.K >= 2048;
+  return a.N > 16384 || a.K >= 768 || (a.M > 32 && a.K >= 512 && a.N <= 4096);
+}
+
 // Default (tile width, waves, K slices) per shape, from tools/decode_gemm_bench.py on
 // MI355X (profiles/r1_decode_gemm.md, r1_decode_gemm_splitk.jsonl): 2 column tiles per
 // workgroup once there are >= 384 tiles (x fragments re-used across both), 4 for wide
@@ -525,7 +536,7 @@ static int dispatch(DgArgs a, int epi, int norm, int nt, int waves, int splits, 
   if (M > 64 || a.K % 32 != 0 || N % 16 != 0 || epi < 0 || epi > 3) return 1;
   if ((epi == EPI_SILU || epi == EPI_ROPE) && (N / 16) % 2) return 1;
   if (epi == EPI_RESID && !a.resid) return 1;
-  if (M > 16 && epi == EPI_PLAIN && !norm && nt <= 0 && waves <= 0 && splits <= 0) {
+  if (rows_pay(a) && epi == EPI_PLAIN && !norm && nt <= 0 && waves <= 0 && splits <= 0) {
     const int rc = dispatch_rows(a, st);
     if (rc <= 0) return rc;
   }

@@ -13,7 +13,7 @@ from pilottai_amd.ops.latent import pad_to
 
 class PackedLinear:
     """y = x W^T with W [N, K] padded to [128 n, 64 k] by zeros: the packed projections in bf16
-    (decode kernels up to 64 rows and where a step has few tiles, prefill kernel above), the library's fp32 GEMM in fp32."""
+    (decode kernels up to 64 rows and where rows_gemm_pays, prefill kernel above), the library's fp32 GEMM in fp32."""
 
     def __init__(self, w: torch.Tensor, dtype, device):
         N, K = w.shape
@@ -27,7 +27,7 @@ class PackedLinear:
             return F.linear(x, self.w)
         if x.shape[0] <= 64:
             return ops.decode_gemm(x, self.w)
-        y = ops.rows_gemm(x, self.w)
+        y = ops.rows_gemm(x, self.w) if ops.rows_gemm_pays(x.shape[0], self.w.shape[0] * 16, x.shape[1]) else None
         return ops.prefill_gemm(x, self.w) if y is None else y
 
 

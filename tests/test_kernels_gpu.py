@@ -390,6 +390,30 @@ def test_rows_gemm(gpu, M, N, K):
                          ops.pack_decode_weight(torch.zeros(4096, 64, device=gpu, dtype=torch.bfloat16))) is None
 
 
+@pytest.mark.parametrize("M,N,K", [(24, 8192, 2048), (24, 8208, 2048), (24, 8208, 2016), (25, 2048, 736), (25, 2048, 768), (32, 64, 512),
+                                   (33, 64, 512), (33, 4112, 512), (64, 80, 480), (40, 16384, 64), (40, 16400, 64), (17, 16, 14336)])
+def test_decode_gemm_of_17_to_64_rows(gpu, M, N, K):
+    """Both sides of the lines between its two kernels (rows_pay), with test_rows_gemm's bound."""
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    x, w = torch.randn(M, K, device=gpu, generator=g).bfloat16(), torch.randn(N, K, device=gpu, generator=g).bfloat16()
+    y = ops.decode_gemm(x, ops.pack_decode_weight(w))
+    ref, size = x.float() @ w.float().T, x.float().abs() @ w.float().abs().T
+    assert bool(((y.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + K * 2.0 ** -24 * size).all())
+
+
+@pytest.mark.parametrize("M,N,K", [(300, 512, 128), (300, 512, 8192), (300, 1408, 192), (300, 1408, 256), (128, 3072, 8192),
+                                   (256, 2048, 4096), (256, 2048, 4160), (1600, 512, 3072), (1600, 512, 3136), (512, 3072, 3136)])
+def test_packed_linear_of_many_rows(gpu, M, N, K):
+    """Both sides of the lines between rows_gemm and prefill_gemm (rows_gemm_pays), with test_rows_gemm's bound."""
+    from pilottai_amd.models.common import PackedLinear
+
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    x, w = torch.randn(M, K, device=gpu, generator=g).bfloat16(), torch.randn(N, K, device=gpu, generator=g).bfloat16()
+    y = PackedLinear(w, torch.bfloat16, gpu)(x)
+    ref, size = x.float() @ w.float().T, x.float().abs() @ w.float().abs().T
+    assert bool(((y.float() - ref).abs() <= 2.0 ** -8 * ref.abs() + K * 2.0 ** -24 * size).all())
+
+
 @pytest.mark.parametrize("nt,waves,splits", [(1, 8, 1), (1, 16, 1), (2, 8, 1), (2, 16, 1), (4, 8, 1), (4, 16, 1),
                                              (2, 8, 4), (4, 8, 2), (1, 16, 3), (2, 4, 8)])
 def test_decode_gemm_configs(gpu, nt, waves, splits):
