@@ -157,12 +157,52 @@ __device__ __forceinline__ void store_rows(const Args& A, int grp, int start, in
   }
 }
 
-// Dense rows: tiles of 16 MT rows and 16 NT outputs a wave (PLAIN, GATED).
-template <int MT, int NT, int KU, int EPI>
+// Sorted rows: the NT tiles from nt on of the row 16 m + c (GLU: a gate and an up tile).
+template <int EPI, int NT>
+__device__ __forceinline__ void store_sorted(const Args& A, int start, int n, int m, int nt, const f32x4 (&a)[NT]) {
+  const int lane = threadIdx.x & 63, c = lane & 15, g = lane >> 4;
+  if (16 * m + c >= n || nt >= A.N16) return;
+  const int p = start + 16 * m + c;
+  bf16* o = (bf16*)A.out + (size_t)(A.out_order ? A.order[p] : p) * A.ldo + 4 * g;
+  if constexpr (EPI == GLU) {
+    const float rw = A.row_w ? A.row_w[A.order[p]] : 1.f;
+    bf16x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = (bf16)glu(a[0][j] * rw, a[1][j] * rw, A);
+    *reinterpret_cast<bf16x4*>(o + nt * 8) = v;
+    return;
+  }
+  if constexpr (NT == 2) {
+    if (A.N16 % 2 == 0 && A.wide) {
+      const struct { bf16* y; int ldy; } row{o - 4 * g, 0};
+      pk::store_pair_wide<EPI == RELU2 ? pk::EP_RELU2 : pk::EP_PLAIN>(row, 0, nt, g, a[0], a[1]);
+      return;
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < NT; ++i) {
+    if (nt + i >= A.N16) break;
+    bf16x4 v;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) v[j] = (bf16)(EPI == RELU2 ? pk::relu2(a[i][j]) : a[i][j]);
+    *reinterpret_cast<bf16x4*>(o + (nt + i) * 16) = v;
+  }
+}
+
+// Tiles of 16 MT rows and 16 NT outputs a wave, straight from memory: dense rows (PLAIN, GATED), and sorted ones (PLAIN, GLU,
+// RELU2) of few inputs (sorted_rows).
+template <int MT, int NT, int KU, int EPI, bool SORTED = false>
 __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int c = lane & 15, g = lane >> 4;
-  const int grp = blockIdx.z, start = blockIdx.y * (16 * MT), n = min(16 * MT, A.rows - start);
+  int grp = blockIdx.z, start = blockIdx.y * (16 * MT), n = min(16 * MT, A.rows - start);
+  if constexpr (SORTED) {
+    if ((int)blockIdx.y >= A.n_tiles[0]) return;
+    const int4 tl = A.tiles[blockIdx.y];
+    grp = tl.x;
+    start = tl.y;
+    n = tl.z;
+  }
   if (A.rp && blockIdx.x == 0) {
     rotate_rows<bf16>(A, grp, start, n);
     return;
@@ -176,7 +216,9 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
   const bf16* xr[MT];
 #pragma unroll
   for (int m = 0; m < MT; ++m) {
-    xr[m] = (const bf16*)A.x + (size_t)(start + min(16 * m + c, n - 1)) * A.ldx + (size_t)grp * A.xg + 8 * g;
+    int row = start + min(16 * m + c, n - 1);
+    if (SORTED && A.x_div) row = A.order[row] / A.x_div;
+    xr[m] = (const bf16*)A.x + (size_t)row * A.ldx + (SORTED ? 0 : (size_t)grp * A.xg) + 8 * g;
   }
   f32x4 acc[MT][NT];
 #pragma unroll
@@ -212,7 +254,12 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
       for (int m = 0; m < MT; ++m) b[k][m] = bn[k][m];
     }
   }
-  store_rows<MT, NT, EPI>(A, grp, start, n, nt0, acc);
+  if constexpr (SORTED) {
+#pragma unroll
+    for (int m = 0; m < MT; ++m) store_sorted<EPI, NT>(A, start, n, m, nt0, acc[m]);
+  } else {
+    store_rows<MT, NT, EPI>(A, grp, start, n, nt0, acc);
+  }
 }
 
 // Many dense rows of groups with few inputs (the heads of a latent attention): 64 rows of a group's inputs whole in LDS,
@@ -392,37 +439,9 @@ __global__ __launch_bounds__(512, MT == 8 ? 4 : 2) void rows_kernel(const Args A
       }
     }
   }
-  // the pair of tiles nt of the rows 16 m + c
-  auto store = [&](int m, int nt, f32x4 v0, f32x4 v1) {
-    if (16 * m + c >= n || nt >= A.N16) return;
-    const int p = start + 16 * m + c;
-    bf16* o = (bf16*)A.out + (size_t)(A.out_order ? A.order[p] : p) * A.ldo + 4 * g;
-    if constexpr (EPI == GLU) {
-      const float rw = A.row_w ? A.row_w[A.order[p]] : 1.f;
-      bf16x4 v;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) v[j] = (bf16)glu(v0[j] * rw, v1[j] * rw, A);
-      *reinterpret_cast<bf16x4*>(o + nt * 8) = v;
-    } else if (A.N16 % 2 == 0 && A.wide) {
-      const struct { bf16* y; int ldy; } row{o - 4 * g, 0};
-      pk::store_pair_wide<EPI == RELU2 ? pk::EP_RELU2 : pk::EP_PLAIN>(row, 0, nt, g, v0, v1);
-    } else {
-#pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        if (nt + i >= A.N16) break;
-        bf16x4 v;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          const float a = i ? v1[j] : v0[j];
-          v[j] = (bf16)(EPI == RELU2 ? pk::relu2(a) : a);
-        }
-        *reinterpret_cast<bf16x4*>(o + (nt + i) * 16) = v;
-      }
-    }
-  };
   if constexpr (WK == 1) {
 #pragma unroll
-    for (int m = 0; m < MT; ++m) store(m, nt0, acc[m][0], acc[m][1]);
+    for (int m = 0; m < MT; ++m) store_sorted<EPI, NT>(A, start, n, m, nt0, acc[m]);
   } else {
     __syncthreads();
     f32x4* red = reinterpret_cast<f32x4*>(smem);  // [WK][WN][MT][NT][64]
@@ -439,7 +458,7 @@ __global__ __launch_bounds__(512, MT == 8 ? 4 : 2) void rows_kernel(const Args A
 #pragma unroll
         for (int w = 1; w < WK; ++w) v[j] += red[((w * WN * MT + t) * NT + j) * 64 + lane];
       }
-      store(t % MT, (block * WN + t / MT) * NT, v[0], v[1]);
+      store_sorted<EPI, NT>(A, start, n, t % MT, (block * WN + t / MT) * NT, v);
     }
   }
 }
@@ -461,11 +480,43 @@ static int launch_rows(const Args& A, int epi, int max_tiles, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
+// Tiles of 16 and 32 rows whose stages of LDS do not pay: a wave's fragments straight from memory (gemm_kernel). us at 16 rows a tile,
+// rows_kernel against gemm_kernel: 64 experts of 2 x 256 x K and 96 rows, K = 256 6.9, 5.6, 512 9.3, 8.5, 1024 13.7, 14.2; of 2048 x K 16.3,
+// 13.1, 25.4, 23.8, 38.9, 45.0; few tiles end with their slowest (16 of 1024 x 512, 64 rows 6.6, 6.5; 24 of 2048 x 512 12.7, 13.3), and
+// few outputs leave rows_kernel few workgroups a group (64 of 128 x 2048, 600 rows 22, 16).
+static bool few_inputs(const Args& A, bool glu, int max_tiles) {
+  if (max_tiles > 65535) return false;  // (a dimension of its grid)
+  const bool narrow = A.N16 <= 16 && max_tiles >= (A.K32 <= 16 ? 64 : 96);
+  return A.K32 <= (glu ? 4 : 8) || narrow || (A.K32 <= 16 && max_tiles * A.N16 >= 1536);
+}
+
 // Waves over k (WK): 4 for few rows; with 64-row tiles of many groups 2 (T = 400: 228 us both products, 4: 246, 1: 254),
 // with those of one group as many as leave at most two workgroups a CU (2 x 8192 x 2048 outputs of 128 rows: 4 26 us, of 256: 2
 // 33 us, 4 45; of 512: 1 46 us, 2 57); 1 with 128 rows, whose accumulators fill a wave. Non-temporal weights where
 // no more than every third tile is a group's second (64 tokens 192 -> 182 us; 400 tokens 240 -> 250).
 static int sorted_rows(const Args& A, int epi, int tm, int groups, int max_tiles, hipStream_t st) {
+  if (tm <= 32 && few_inputs(A, epi == 1, max_tiles)) {
+#define PA_S(MT, NT, KU, G)                                                                                               \
+  hipLaunchKernelGGL((gemm_kernel<MT, NT, KU, G, true>), dim3((A.N16 + 4 * NT - 1) / (4 * NT), max_tiles), dim3(256), 0, st, A)
+#define PA_SK(MT, NT, G)                     \
+  do {                                       \
+    if (A.K32 % 4 == 0) PA_S(MT, NT, 4, G);  \
+    else if (A.K32 % 2 == 0) PA_S(MT, NT, 2, G); \
+    else PA_S(MT, NT, 1, G);                 \
+  } while (0)
+    if (tm == 16) {
+      if (epi == 1) PA_SK(1, 2, GLU);
+      else if (epi == 2) PA_SK(1, 1, RELU2);
+      else PA_SK(1, 1, PLAIN);
+    } else {
+      if (epi == 1) PA_SK(2, 2, GLU);
+      else if (epi == 2) PA_SK(2, 1, RELU2);
+      else PA_SK(2, 1, PLAIN);
+    }
+#undef PA_SK
+#undef PA_S
+    return (int)hipGetLastError();
+  }
   const bool once = (max_tiles - groups) * 2 <= groups;
   auto fits = [&](int wk) { return (A.N16 * 16 + 256 / wk - 1) / (256 / wk) * max_tiles <= 512; };
   if (tm == 16) return once ? launch_rows<1, 4, true>(A, epi, max_tiles, st) : launch_rows<1, 4, false>(A, epi, max_tiles, st);

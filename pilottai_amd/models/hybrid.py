@@ -21,8 +21,8 @@ import torch
 
 from pilottai_amd import ops
 from pilottai_amd.models.cache import HybridCache, StepMeta
-from pilottai_amd.models.common import (ONE_GROUP_TILES, ONE_LARGE_GROUP_TILES, PackedLinear, checkpoint_reader,
-                                         expert_tile_rows)
+from pilottai_amd.models.common import (ONE_GROUP_TILES, ONE_LARGE_GROUP_TILES, ONE_SMALL_GROUP_TILES, PackedLinear,
+                                         checkpoint_reader, expert_tile_rows)
 from pilottai_amd.ops.latent import pad_to
 from pilottai_amd.parallel.comm import TPGroup
 
@@ -503,7 +503,7 @@ def _pack_gate_up(gate, up, fp: int, dk: int, dtype, device):
 class GatedMLP:
     """down(act(gate h) * up h): the gate and up rows interleaved in one grouped projection of one group."""
 
-    LARGE = 1 << 26  # elements of weights that the next tile does not find in the caches again
+    SMALL, LARGE = 1 << 24, 1 << 26  # elements of weights: few workgroups; not found in the caches by the next tile again
 
     def __init__(self, spec: DenseSpec, t: Dict[str, torch.Tensor], width: int, dtype, device, alone: bool = True):
         self.spec, self.dtype, self.device = spec, dtype, device
@@ -519,8 +519,9 @@ class GatedMLP:
     def activate(self, h, act):
         T = h.shape[0]
         if T not in self._tiles:  # (before graph capture: the capture's warm-up runs come first)
-            tm = expert_tile_rows(T, self.dtype, self.dk,
-                                  ONE_GROUP_TILES if self.w13.numel() <= self.LARGE else ONE_LARGE_GROUP_TILES)
+            n = self.w13.numel()
+            tm = expert_tile_rows(T, self.dtype, self.dk, ONE_SMALL_GROUP_TILES if n <= self.SMALL else
+                                  ONE_GROUP_TILES if n <= self.LARGE else ONE_LARGE_GROUP_TILES)
             tiles = torch.tensor([[0, i, min(tm, T - i), 0] for i in range(0, T, tm)], dtype=torch.int32)
             self._tiles[T] = (tiles.to(self.device), torch.tensor([len(tiles)], dtype=torch.int32, device=self.device),
                               torch.arange(T, dtype=torch.int32, device=self.device), tm)

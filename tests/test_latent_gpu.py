@@ -189,7 +189,8 @@ def sorted_rows(gpu, tm, counts, N, K):
 @pytest.mark.parametrize("counts,N,K", [
     ([1, 0, 16, 17, 40, 130, 3], 96, 96),       # empty and single-row groups, remainders of every tile, k past no stage's end
     ([5, 33], 80, 2048), ([200] * 3, 2816, 32),  # an odd number of 16-row blocks; more blocks than XCDs
-    ([7], 16384, 64), ([100], 16384, 320), ([300], 4096, 160), ([300], 16384, 96)])  # one group: 4, 2 and 1 waves over k
+    ([7], 16384, 64), ([100], 16384, 320), ([300], 4096, 160), ([300], 16384, 96),   # one group: 4, 2 and 1 waves over k
+    ([30, 1] * 20, 1040, 512), ([40] * 20, 1024, 512), ([7] * 100, 80, 1088), ([20, 2, 33], 288, 256)])  # few inputs, few outputs
 def test_sorted_rows(gpu, tm, counts, N, K):
     sorted_rows(gpu, tm, counts, N, K)
 
