@@ -732,7 +732,7 @@ extern "C" int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out
                                int ldg, const void* table, const int* ids, int ldt, int tcol, int vocab, hipStream_t st) {
   if (N16 <= 0 || K32 <= 0 || (epi == 1 && N16 % 2)) return -1;
   if (row_w && (!tiles || epi != 1 || !x_div)) return -1;
-  if (tiles ? epi > 2 : (epi == 3 && !gate) || (epi == 4 && (!table || !ids))) return -1;
+  if (tiles ? epi > 2 : epi == 1 || epi == 2 || (epi == 3 && !gate) || (epi == 4 && (!table || !ids))) return -1;
   if (tiles ? max_tiles <= 0 : rows <= 0) return 0;
   const pa::gg::Args A{x, w, out, wstride, ldx, xg, ldo, og, rows, N16, K32, (const int4*)tiles, n_tiles,
                        order, x_div, out_order, limit, alpha, cubic, bias, positions, cos_sin, rskip, r, rp, rd,
