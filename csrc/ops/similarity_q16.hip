@@ -767,20 +767,23 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
 
 // ---- queries ------------------------------------------------------------------------------------------
 // x / y rounded as IEEE does, whatever the compiler may do with a float division (fast-math): the double quotient
-// rounds to the same float, and the empty asm keeps the two steps apart.
+// rounds to the same float, and the empty asm keeps the two steps apart, and a rounding to 16 bits behind them.
 __device__ __forceinline__ float div_rn(float x, float y) {
   double d = (double)x / (double)y;
   asm volatile("" : "+v"(d));
-  return (float)d;
+  float f = (float)d;
+  asm volatile("" : "+v"(f));
+  return f;
 }
 
 // One workgroup a query: normalised (if asked), then rounded to bf16, or to 16-bit fixed point as q16_quantize does:
-// s_q = max|x| / 32512, v = round(x / s_q) = 256 qh + ql, c_q = s_q ||v||_2 (a hair above). One launch in place of the 28
+// s_q = max|x| / 32512, v = round(x / s_q) = 256 qh + ql, c_q = s_q ||v||_2 (a hair above). NaN goes where torch's
+// operations take it: a norm or a maximum of a query that holds one is one (s_q is then 1), and in v it is 0. One launch in place of the 28
 // elementwise ones that took as long as the search of a small index.
 __global__ __launch_bounds__(256) void prepare_kernel(const float* __restrict__ x, int D, int normalize, bf16* __restrict__ out,
                                                       signed char* __restrict__ qv, float* __restrict__ qmeta) {
   __shared__ double red[4];
-  __shared__ float redm[4];
+  __shared__ uint32_t redm[4];
   const int q = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   x += (size_t)q * D;
   auto sum = [&](double v) {
@@ -791,27 +794,50 @@ __global__ __launch_bounds__(256) void prepare_kernel(const float* __restrict__ 
     __syncthreads();
     return red[0] + red[1] + red[2] + red[3];
   };
+  // (what is not finite is told by its bits: the compiler is told that there is none)
+  auto size = [](float v) { return __float_as_uint(v) & 0x7fffffffu; };
+  constexpr uint32_t INF = 0x7f800000u;
   float by = 1.f;
   if (normalize) {
     double ss = 0.;
     for (int i = threadIdx.x; i < D; i += 256) ss += (double)x[i] * (double)x[i];
-    by = fmaxf((float)sqrt(sum(ss)), 1e-12f);
+    ss = sum(ss);
+    const long long over = __double_as_longlong(ss) - 0x7ff0000000000000ll;  // the norm is infinite (0) or NaN (above)
+    by = fmaxf((float)sqrt(ss), 1e-12f);
+    if (over >= 0 || size(by) == INF) {  // finite values become 0 or NaN, the others NaN
+      for (int i = threadIdx.x; i < D; i += 256) {
+        if (out) {
+          reinterpret_cast<uint16_t*>(out)[(size_t)q * D + i] =
+              over > 0 || size(x[i]) >= INF ? 0x7fc0 : __float_as_uint(x[i]) >> 16 & 0x8000;
+        } else {
+          qv[(size_t)q * 2 * D + i] = 0;
+          qv[(size_t)q * 2 * D + D + i] = 0;
+        }
+      }
+      if (!out && threadIdx.x == 0) {
+        qmeta[2 * q] = 1.f;
+        qmeta[2 * q + 1] = 0.f;
+      }
+      return;
+    }
   }
+  auto at = [&](int i) { return normalize ? div_rn(x[i], by) : x[i]; };
   if (out) {
-    for (int i = threadIdx.x; i < D; i += 256) out[(size_t)q * D + i] = (bf16)(normalize ? div_rn(x[i], by) : x[i]);
+    for (int i = threadIdx.x; i < D; i += 256) out[(size_t)q * D + i] = (bf16)at(i);
     return;
   }
-  float m = 0.f;
-  for (int i = threadIdx.x; i < D; i += 256) m = fmaxf(m, fabsf(normalize ? div_rn(x[i], by) : x[i]));
-  m = wave_max(m);
-  if (lane == 0) redm[wid] = m;
+  uint32_t mb = 0;  // magnitudes in their bits' order, NaN above all
+  for (int i = threadIdx.x; i < D; i += 256) mb = max(mb, size(at(i)));
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o, 64));
+  if (lane == 0) redm[wid] = mb;
   __syncthreads();
-  m = fmaxf(fmaxf(redm[0], redm[1]), fmaxf(redm[2], redm[3]));
-  const float sc = m > 0.f ? div_rn(m, 32512.f) : 1.f;
+  mb = max(max(redm[0], redm[1]), max(redm[2], redm[3]));
+  const float sc = mb > 0 && mb <= INF ? div_rn(__uint_as_float(mb), 32512.f) : 1.f;
   double vv = 0.;
   for (int i = threadIdx.x; i < D; i += 256) {
-    const float f = rintf(div_rn(normalize ? div_rn(x[i], by) : x[i], sc));
-    const int v = (int)fminf(fmaxf(f, -32512.f), 32512.f), h = (v + 128) >> 8;
+    const float f = rintf(div_rn(at(i), sc));
+    const int v = size(f) > INF ? 0 : (int)fminf(fmaxf(f, -32512.f), 32512.f), h = (v + 128) >> 8;
     qv[(size_t)q * 2 * D + i] = (signed char)h;
     qv[(size_t)q * 2 * D + D + i] = (signed char)(v - 256 * h);
     vv += (double)v * (double)v;  // whole numbers below 2^53: exact in any order

@@ -258,10 +258,16 @@ def sample(logits, temperature, mask_class, class_masks, seeds, offsets, forced=
 COSINE_MAX_Q = 64  # queries per index pass (LDS-resident query tiles)
 
 
+def _unit_rows(q: torch.Tensor) -> torch.Tensor:
+    """fp32 rows of unit length as the kernel makes them: the norm summed in float64, all else in fp32."""
+    q = q.float()
+    return q / q.double().square().sum(1, keepdim=True).sqrt().float().clamp_min(1e-12)
+
+
 def unit_queries(q: torch.Tensor) -> torch.Tensor:
-    """bf16 rows of unit length from fp32 ones."""
+    """bf16 rows of unit length from fp32 ones; the same bits from the kernel and on the CPU."""
     if not _on_gpu(q):
-        return torch.nn.functional.normalize(q, dim=1).to(torch.bfloat16)
+        return _unit_rows(q).to(torch.bfloat16)
     out = torch.empty_like(q, dtype=torch.bfloat16)
     require_native().prepare_queries(q, True, out=out)
     return out
@@ -338,7 +344,7 @@ def q16_queries(q: torch.Tensor, normalize: bool = False):
         require_native().prepare_queries(q, normalize, qv=qv, qmeta=qm)
         return qv, qm
     if normalize:
-        q = torch.nn.functional.normalize(q.float(), dim=1)
+        q = _unit_rows(q)
     hi, lo, sc, _ = q16_quantize(q)
     v = 256 * hi.double() + lo.double()
     cq = (sc.double() * v.norm(dim=1)).float() * (1 + 1e-6)

@@ -110,6 +110,20 @@ def test_query_preparation_matches_torch(gpu, Q, D):
     assert (ops.unit_queries(q).cpu().float() - u).abs().max() <= 2.0 ** -8 * u.abs().max()
 
 
+@pytest.mark.parametrize("normalize", [False, True])
+def test_query_preparation_has_the_bits_of_the_cpu(gpu, normalize):
+    """Both forms of a query, bit for bit; zeros, tiny and huge values, NaN and infinities among them."""
+    q = torch.randn(40, 512, generator=torch.Generator().manual_seed(2)) * torch.logspace(-18, 17, 40)[:, None]
+    q[3], q[5, 7], q[6, 100], q[8, 5:9], q[9] = 0.0, float("nan"), float("inf"), -float("inf"), float("nan")
+    bits = lambda t: t.contiguous().cpu().view(torch.int32)  # noqa: E731
+    nan = lambda t: torch.where(torch.isnan(t), torch.full_like(t, 7.0), t)  # noqa: E731  (whichever NaN)
+    qv, qm = ops.q16_queries(q.to(gpu), normalize=normalize)
+    rv, rm = ops.q16_queries(q, normalize=normalize)
+    assert torch.equal(qv.cpu(), rv) and torch.equal(bits(nan(qm)), bits(nan(rm)))
+    if normalize:
+        assert torch.equal(bits(nan(ops.unit_queries(q.to(gpu)).cpu().float())), bits(nan(ops.unit_queries(q).float())))
+
+
 def test_q16_planted_neighbours_found(gpu):
     _check(gpu, 400_000, 1024, 32, 5, False, seed=7, planted=True)
 
