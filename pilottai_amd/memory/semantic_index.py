@@ -342,8 +342,11 @@ class SemanticIndex:
                 here.wait_stream(caller)
             host = torch.empty(16 * Q + (0 if q.is_cuda else 4 * Q * D), dtype=torch.uint8, pin_memory=True)
             h = host.numpy()
-            h[:8 * Q].view(np.int64)[:] = qmasks
-            h[8 * Q:12 * Q].view(np.int32)[:] = min_priority
+            for name, v, to in (("qmasks", torch.as_tensor(qmasks, dtype=torch.int64), h[:8 * Q].view(np.int64)),
+                                ("min_priority", torch.as_tensor(min_priority, dtype=torch.int32), h[8 * Q:12 * Q].view(np.int32))):
+                if v.numel() < Q:
+                    raise ValueError(f"{v.numel()} {name} for {Q} queries")
+                to[:] = v.reshape(-1)[:Q].cpu().numpy()
             if not q.is_cuda:
                 h[16 * Q:].view(np.float32).reshape(Q, D)[:] = q.detach().float().numpy()
             dev = host.to(self.device, non_blocking=True)

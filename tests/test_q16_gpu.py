@@ -168,3 +168,30 @@ def test_q16_semantic_index_on_gpu(gpu):
     for a, b in zip(res[0], res[1]):
         for (_, sa), (_, sb) in zip(a, b):
             assert abs(sa - sb) <= 1e-6 * max(1.0, abs(sb))
+
+
+def _small_index(gpu, storage="q16", n=3000, same=False):
+    import numpy as np
+
+    from pilottai_amd.memory.semantic_index import SemanticIndex
+
+    v = np.random.default_rng(5).standard_normal((1 if same else n, 256)).astype(np.float32)
+    idx = SemanticIndex(dim=256, capacity=n, device=gpu, storage=storage)
+    idx.add(np.repeat(v, n, 0) if same else v, [i % 3 for i in range(n)], [()] * n, [None] * n)
+    return idx, v
+
+
+@pytest.mark.parametrize("storage", ["bf16", "q16"])
+def test_search_takes_any_sequence_of_filters(gpu, storage):
+    """Filters as numbers, as tensors on either device, and more of them than queries; fewer are refused, not repeated."""
+    idx, v = _small_index(gpu, storage)
+    q, none = v[:3], [()] * 3
+    want = idx.search(q, 4, [0, 1, 2], none)
+    for p in ((0, 1, 2), torch.tensor([0, 1, 2]), torch.tensor([0, 1, 2], device=gpu), [0, 1, 2, 0, 1], [0.5, 1.5, 2.0]):
+        assert idx.search(q, 4, p, none) == want
+    assert idx.search(q, 4, [0, 1, 2], [()] * 5) == want
+    for p, t in (([1], none), ([0, 1, 2], [()])):
+        with pytest.raises(ValueError):
+            idx.search(q, 4, p, t)
+    with pytest.raises((RuntimeError, OverflowError)):
+        idx.search(q, 4, [0, 1, 1 << 40], none)
