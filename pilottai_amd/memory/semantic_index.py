@@ -364,7 +364,6 @@ class SemanticIndex:
                 ops.cosine_topk(ops.unit_queries(qd), self.packed, self.count, k, *filters, workspace=self._ws, out=(s, r))
             if ev is not None:
                 ev[1].record()
-                self.pass_events.append(ev)
             back = torch.empty(buf.shape, dtype=torch.int32, pin_memory=True)
             back.copy_(buf, non_blocking=True)
         a = back.numpy()
@@ -373,8 +372,12 @@ class SemanticIndex:
             with self._lock, self._stream_ctx():
                 self.stats["q16_fallbacks"] += 1
                 ops.q16_pass(*args, True, self._ws)
+                if ev is not None:  # (both passes, as search_tensors has it)
+                    ev[1].record()
                 back.copy_(buf, non_blocking=True)
             here.synchronize()
+        if ev is not None:
+            self.pass_events.append(ev)
         return a[:Q * k].view(np.float32).reshape(Q, k), a[Q * k:2 * Q * k].reshape(Q, k)
 
     def search(self, queries, k: int, min_priority: Sequence[int], tags: Sequence[Iterable[str]],

@@ -195,3 +195,19 @@ def test_search_takes_any_sequence_of_filters(gpu, storage):
             idx.search(q, 4, p, t)
     with pytest.raises((RuntimeError, OverflowError)):
         idx.search(q, 4, [0, 1, 1 << 40], none)
+
+
+def test_search_times_its_second_pass_too(gpu, monkeypatch):
+    """The events around a search that falls back to the exact scan lie around both passes."""
+    idx, v = _small_index(gpu, n=40_000, same=True)
+    idx.pass_events, ends, run = [], [], ops.q16_pass
+
+    def noted(*args):
+        run(*args)
+        ends.append(torch.cuda.Event(enable_timing=True))
+        ends[-1].record()
+    monkeypatch.setattr(ops, "q16_pass", noted)
+    idx.search(v, 5, [0], [()])
+    assert idx.stats["q16_fallbacks"] == 1 and len(ends) == 2 and len(idx.pass_events) == 1
+    (start, end), = idx.pass_events
+    assert 0 < start.elapsed_time(ends[0]) < start.elapsed_time(ends[1]) <= start.elapsed_time(end)
