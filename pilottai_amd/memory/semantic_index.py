@@ -331,9 +331,9 @@ class SemanticIndex:
         return ev
 
     def _search_host(self, q: torch.Tensor, k: int, min_priority, qmasks, now: Optional[float]):
-        """search_tensors for a caller that waits for the answer: (scores, rows) as arrays, [Q, k]. What the pass reads
-        goes to the device in one pinned copy and comes back in one (queries and filters, scores, rows and flags were
-        four copies out and up to three back, each with its own wait)."""
+        """search_tensors for a caller that waits for the answer, with filters as lists: (scores, rows) as arrays, [Q, k].
+        What the pass reads goes to the device in one pinned copy and comes back in one (queries and filters, scores, rows
+        and flags were four copies out and up to three back, each with its own wait)."""
         Q, D = q.shape
         caller = torch.cuda.current_stream(self.device) if q.is_cuda else None
         with self._lock, self._stream_ctx():
@@ -342,11 +342,13 @@ class SemanticIndex:
                 here.wait_stream(caller)
             host = torch.empty(16 * Q + (0 if q.is_cuda else 4 * Q * D), dtype=torch.uint8, pin_memory=True)
             h = host.numpy()
-            for name, v, to in (("qmasks", torch.as_tensor(qmasks, dtype=torch.int64), h[:8 * Q].view(np.int64)),
-                                ("min_priority", torch.as_tensor(min_priority, dtype=torch.int32), h[8 * Q:12 * Q].view(np.int32))):
-                if v.numel() < Q:
-                    raise ValueError(f"{v.numel()} {name} for {Q} queries")
-                to[:] = v.reshape(-1)[:Q].cpu().numpy()
+            for values, to in ((qmasks, h[:8 * Q].view(np.int64)), (min_priority, h[8 * Q:12 * Q].view(np.int32))):
+                if len(values) < Q:
+                    raise ValueError(f"{len(values)} filters for {Q} queries")
+                try:
+                    to[:] = values[:Q]
+                except TypeError:  # (numbers on the GPU)
+                    to[:] = torch.as_tensor(values[:Q]).cpu().numpy()
             if not q.is_cuda:
                 h[16 * Q:].view(np.float32).reshape(Q, D)[:] = q.detach().float().numpy()
             dev = host.to(self.device, non_blocking=True)
