@@ -267,7 +267,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
 // 64 outputs. Units of 8 inputs, [K / 8][64 rows][8] and a row of padding, so that rows are written and fragments read
 // without conflicts. 4,096 rows, 16 heads: 128 -> 512 beside 64 rotated 43 -> 34 us (88 MB:
 // 18 us at the rate of a copy). 512 -> 128 stays there: 29 us, here 31, as the rows arrive before the first product; and so
-// do fewer than two workgroups a CU (512 rows of 16 heads: 10 us, here 11).
+// do fewer than two workgroups a CU (512 rows of 16 heads: 10 us, here 11), and gated outputs of many workgroups and fewer
+// inputs (4,096 rows, 16 heads of 1,024, times a gate: of 64 inputs 117 us, here 145, of 128 136, 149; of 8 heads 46, 38 and 51, 42).
 constexpr int HEAD_UNIT = 65 * 16, HEAD_K32 = 8;
 
 template <int EPI>
@@ -773,6 +774,7 @@ extern "C" int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out
   }
   if (tiles) return pa::gg::sorted_rows(A, epi, tm, groups, max_tiles, st);
   // dense: 64-row tiles once they fill the chip
+  const int head_wgs = (rows + 63) / 64 * groups;
   tm = (N16 + 15) / 16 * ((rows + 63) / 64) * groups < 256 ? 16 : 64;
 #define PA_GG(MT, NT, KU, G)                                                                                   \
   hipLaunchKernelGGL((pa::gg::gemm_kernel<MT, NT, KU, G>),                                                     \
@@ -786,7 +788,8 @@ extern "C" int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out
   if (tm == 16) {
     if (epi == 3) PA_GGK(1, 1, pa::gg::GATED);
     else PA_GGK(1, 1, pa::gg::PLAIN);
-  } else if (K32 <= pa::gg::HEAD_K32 && N16 >= 16 && (rows + 63) / 64 * groups >= 512) {
+  } else if (K32 <= pa::gg::HEAD_K32 && N16 >= 16 && head_wgs >= 512 &&
+             (epi != 3 || head_wgs <= 768 || (K32 == 8 && N16 <= 32))) {
     const dim3 grid((rows + 63) / 64, groups);
     const int lds = 4 * K32 * pa::gg::HEAD_UNIT;
     if (epi == 3) hipLaunchKernelGGL((pa::gg::head_rows_kernel<pa::gg::GATED>), grid, dim3(256), lds, st, A);

@@ -65,7 +65,7 @@ def test_head_gemm(gpu, dt, T, G, N, K):
 
 
 @pytest.mark.parametrize("gated", [False, True])
-@pytest.mark.parametrize("T,G,N,K", [(32705, 1, 256, 32), (2049, 16, 272, 160), (1100, 33, 512, 256), (4095, 8, 512, 128)])
+@pytest.mark.parametrize("T,G,N,K", [(32705, 1, 256, 32), (2049, 16, 272, 160), (1100, 33, 512, 256), (4095, 8, 512, 128), (4097, 16, 544, 256), (3100, 17, 256, 96)])
 def test_head_gemm_of_many_rows(gpu, T, G, N, K, gated):
     """Two workgroups of 64 rows a CU and more: sizes that are no multiple of a tile, the widest inputs, beside rotated
     columns. Sums of K products in fp32 err by K 2^-24 of their magnitudes at most, a bf16 result rounds by 2^-8."""
