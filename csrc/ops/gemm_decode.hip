@@ -1,4 +1,4 @@
-// Decode-step projections on pre-packed weights (fused):
+// Decode-step projections on pre-packed weights, fused:
 //
 //     y[M, N] = epi( r[m] * x[M, K] · W[N, K]^T )        bf16 in/out, fp32 accumulate, M <= 64
 //
@@ -313,7 +313,7 @@ static int g_dg_variant = 1;
 //     so the cause is not a stale L2 copy of the slab; mode 2 stays
 //     (profiles/r4_handoff_uncached.md).
 //   attention partition merge: 1 = last-arriver agent acquire on uncached partials: 0 bad runs
-//     in 10,000 poisoned repetitions for each of ten 256/512-key, 4/8-wave cases (round 4); the
+//     in 10,000 poisoned repetitions for each of ten 256/512-key, 4/8-wave cases; the
 //     release costs +77 us at 64 rows x 1,000 keys there (it writes back every dirty L2 line of
 //     the XCD, and this launch leaves many).
 int g_handoff_acquire = 2;

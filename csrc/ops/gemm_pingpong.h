@@ -1,4 +1,4 @@
-// Ping-pong 256 x 256 MFMA GEMM for the large-M projections (SURVEY §2.5 N6; included by
+// Ping-pong 256 x 256 MFMA GEMM for the large-M projections (included by
 // gemm_prefill.hip, which owns the argument struct, the planner and the launcher).
 //
 //     y[M, N] = epi( rownorm(x)[M, K] · W[N, K]^T )      bf16 in/out, fp32 accumulate

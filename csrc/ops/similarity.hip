@@ -1,5 +1,5 @@
 // HBM-resident semantic index: fused filter + cosine similarity + top-k
-// (SURVEY §2.5 N9/N10; backs EnhancedMemory.semantic_search,
+// (backs EnhancedMemory.semantic_search,
 // reference pilott/memory/enhanced_memory.py:93-131).
 //
 // index   [N, D] bf16, rows L2-normalised on insert (so cosine == dot)
@@ -268,8 +268,7 @@ extern "C" int pa_cosine_topk(float* out_scores, int* out_rows, void* workspace,
   if (Q <= 0) return 0;
   if (D % 32 != 0 || D > pa::SIM_MAXD || K < 1 || K > pa::SIM_MAXK || Q > pa::SIM_MAXQ) return -1;
   if (N <= 0) {
-    // empty index: every query gets an empty result (the reference raised here;
-    // SURVEY App. A #26)
+    // empty index: every query gets an empty result (the reference raised here)
     (void)hipMemsetAsync(out_rows, 0xff, (size_t)Q * K * sizeof(int), st);
     return (int)hipGetLastError();
   }

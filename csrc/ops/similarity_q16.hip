@@ -1,5 +1,5 @@
-// Two-stage EXACT filtered top-k over a 16-bit fixed-point semantic index (
-// "halve the bytes per config-4 pass"; reference semantics pilott/memory/enhanced_memory.py:
+// Two-stage EXACT filtered top-k over a 16-bit fixed-point semantic index: half the bytes
+// a pass of the bf16 one (reference semantics pilott/memory/enhanced_memory.py:
 // 93-116 semantic_search, filters as csrc/ops/similarity.hip).
 //
 // Storage (memory/semantic_index.py storage="q16"): every L2-normalised row x is kept as

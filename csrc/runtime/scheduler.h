@@ -1,5 +1,5 @@
 // Continuous-batching scheduler for the on-node inference engine
-// (SURVEY §2.5 N7/N16; replaces the reference's bounded asyncio.Queue +
+// (replaces the reference's bounded asyncio.Queue +
 // LLMHandler Semaphore(5) — pilott/pilott.py:105,272-303, engine/llm.py:36).
 //
 // Every engine step runs ONE forward over a ragged token batch that mixes

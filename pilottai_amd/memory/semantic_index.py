@@ -1,4 +1,4 @@
-"""HBM-resident embedding index with fused filter + cosine top-k (SURVEY §2.5 N9/N10/N13).
+"""HBM-resident embedding index with fused filter + cosine top-k.
 
 Rows are L2-normalised bf16 vectors in one preallocated device matrix
 [capacity, D] (100M x 1024 bf16 = 204.8 GB fits one 288 GB MI355X next to an 8B
@@ -435,7 +435,7 @@ class SemanticIndex:
         rows = sum(p.numel() * p.element_size() for _, p in self._planes())
         return rows + self.capacity * (4 + 8 + 4 + (8 if self.storage == "q16" else 0))
 
-    # -- checkpoint / resume (SURVEY §5: the embedding matrix as per-GPU binary shards
+    # -- checkpoint / resume (the embedding matrix as per-GPU binary shards
     # next to the JSON metadata; reference item form pilott/memory/enhanced_memory.py:9-21) --
     CKPT_VERSION = 1
 

@@ -117,8 +117,8 @@ def empty_handoff(numel: int, dtype=torch.float32, device=None) -> torch.Tensor:
     attention partition partials). On the GPU it lives in uncached device memory
     (hipDeviceMallocUncached): no CU or XCD can hold a stale copy of its lines, so the
     in-launch hand-off is correct for any workgroup placement with a relaxed ticket and the
-    last arriver's acquire, and needs no producer-side L2 write-back (
-    profiles/r4_handoff_uncached.md). Zero-filled. Allocate outside graph capture."""
+    last arriver's acquire, and needs no producer-side L2 write-back
+    (profiles/r4_handoff_uncached.md). Zero-filled. Allocate outside graph capture."""
     device = torch.device(device) if device is not None else torch.device("cpu")
     if device.type == "cuda":
         idx = device.index if device.index is not None else torch.cuda.current_device()
