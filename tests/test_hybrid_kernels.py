@@ -409,6 +409,49 @@ def test_state_scan_portions(gpu, V, N, lens):
 
 
 @pytest.mark.gpu
+def test_state_scan_form_in_a_graph(gpu):
+    """One captured step whose portions take three launches, one, and three again: each replay as the eager step."""
+    from pilottai_amd import ops
+
+    H, V, N, G, T, S = 4, 64, 128, 1, 2048, 16
+    g, C = gen(9), H * V + 2 * G * N
+    proj = torch.randn(T, (H * V + C + H + 7) // 8 * 8, generator=g).to(BF16).to(gpu)
+    w, cb = (torch.randn(4, C, generator=g) * 0.5).to(gpu), torch.zeros(C, device=gpu)
+    bias, a, d = torch.full((H,), -2.0, device=gpu), torch.linspace(0.05, 1.0, H, device=gpu), torch.ones(H, device=gpu)
+    ints = lambda *n: torch.zeros(*n, dtype=torch.int32, device=gpu)  # noqa: E731
+    q_start, q_len, ctx, slot, first, items, n = ints(S), ints(S), ints(S), ints(S), ints(S), ints(60, 4), ints(1)
+    state, ring = torch.zeros(S, H, V, N, device=gpu), torch.zeros(S, 3 + ops.SCAN_MIN, C, dtype=BF16, device=gpu)
+    y = torch.zeros(T, H * V, dtype=BF16, device=gpu)
+
+    def fill(lens):
+        it = [[i, b, min(64, k - b), 0] for i, k in enumerate(lens) for b in range(0, k, 64)]
+        put = lambda t, v: t.copy_(torch.tensor(v, dtype=torch.int32))  # noqa: E731
+        put(q_start, [sum(lens[:i]) for i in range(S)]), put(q_len, list(lens) + [0] * (S - len(lens)))
+        put(ctx, q_len.tolist()), put(slot, [i if i < len(lens) else -1 for i in range(S)]), put(n, [len(it)])
+        items.zero_(), put(items[:len(it)], it), y.zero_(), state.zero_()
+
+    def step():
+        ops.state_scan(proj, y, state, ring, w, cb, bias, a, d, q_start, q_len, ctx, slot, first, items, n, G)
+    plans, graph = ([2048], [128] * 16, [2000, 30]), torch.cuda.CUDAGraph()
+    fill(plans[0])
+    side = torch.cuda.Stream()
+    side.wait_stream(torch.cuda.current_stream())
+    with torch.cuda.stream(side):
+        step()
+    torch.cuda.current_stream().wait_stream(side)
+    with torch.cuda.graph(graph):
+        step()
+    for lens in plans * 2:
+        fill(lens)
+        step()
+        want = y.clone(), state.clone()
+        fill(lens)
+        graph.replay()
+        assert torch.equal(y, want[0]) and torch.equal(state, want[1]), lens
+        assert bool(y[:sum(lens)].any(1).all()) and not y[sum(lens):].any()
+
+
+@pytest.mark.gpu
 def test_state_scan_keeps_the_state_in_fp32(gpu):
     """The state a chunked portion leaves equals the one that single tokens leave to fp32's order, not bf16's."""
     from pilottai_amd import ops
