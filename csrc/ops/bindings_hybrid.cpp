@@ -224,8 +224,8 @@ void state_scan(at::Tensor proj, at::Tensor u, at::Tensor y, at::Tensor state, a
   }
   check_rc(pa_state_scan(f, proj.data_ptr(), proj.stride(0), u.data_ptr(), y.data_ptr(), y.stride(0),
                          state.data_ptr<float>(), ring.data_ptr(), (float*)opt_f32(work, max_items * H * V * N, "work"),
-                         (float*)opt_f32(total, max_items * H + 1, "total"), (float)chain, (float)fixed, opt_f32(conv_w, 0, "conv_w"), opt_f32(conv_b, Cc, "conv_b"),
-                         opt_f32(dt_bias, H, "dt_bias"), opt_f32(a, H, "a"), opt_f32(d, H, "d"),
+                         (float*)opt_f32(total, max_items * H + 1, "total"), (float)chain, (float)fixed,
+                         opt_f32(conv_w, 0, "conv_w"), opt_f32(conv_b, Cc, "conv_b"), opt_f32(dt_bias, H, "dt_bias"), opt_f32(a, H, "a"), opt_f32(d, H, "d"),
                          ints(q_start, seqs, "q_start"), ints(q_len, seqs, "q_len"), ints(ctx_len, seqs, "ctx_len"),
                          ints(state_slot, seqs, "state_slot"),
                          ints(items, 0, "items"), ints(n_items, 1, "n_items"), max_items, seqs, H, G, V, N,

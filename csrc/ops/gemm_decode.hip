@@ -501,11 +501,12 @@ static int dispatch_rows(const DgArgs& a, hipStream_t st) {
   return 1;
 }
 
-// Of up to 64 rows, where x through LDS pays for its stages (us, decode_gemm_kernel against decode_rows_kernel): not up to
-// 24 rows, of which the other kernel reads only those there are (17 x 2048 x 8192 15.9, 19.8; 24 18.7, 19.9) unless the
-// outputs fill the chip several times (24 x 10368 x 2048 14.7, 12.3; x 8192 48.8, 40.0), and not for few k (64 x 2048 x 256
-// 4.1, 4.0; 48 x 8192 x 256 4.9, 5.6, x 512 5.9, 6.3, x 768 7.6, 7.5; 64 x 2048 x 512 5.3, 4.3, 32 4.1, 4.4). Wide outputs that not even
-// 64 columns a tile leave one workgroup a CU stream either way (64 x 28672 x 128 10.0, 7.7; x 4096 69, 51).
+// Of up to 64 rows, where x through LDS pays for its stages (rows x N x K us, decode_gemm_kernel against
+// decode_rows_kernel): not up to 24 rows, of which the other kernel reads only those there are (17 x 2048 x 8192 15.9, 19.8;
+// 24 18.7, 19.9) unless the outputs fill the chip several times (24 x 10368 x 2048 14.7, 12.3; x 8192 48.8, 40.0), and not for
+// few k (64 x 2048 x 256 4.1, 4.0, x 512 5.3, 4.3; 32 x 2048 x 512 4.1, 4.4; 48 x 8192 x 256 4.9, 5.6, x 512 5.9, 6.3, x 768
+// 7.6, 7.5). Wide outputs that not even 64 columns a tile leave one workgroup a CU stream either way (64 x 28672 x 128 10.0,
+// 7.7; x 4096 69, 51).
 static bool rows_pay(const DgArgs& a) {
   if (a.M <= 16) return false;
   if (a.M <= 24) return a.N > 8192 && a.K >= 2048;

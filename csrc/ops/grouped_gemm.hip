@@ -268,7 +268,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
 // without conflicts. 4,096 rows, 16 heads: 128 -> 512 beside 64 rotated 43 -> 34 us (88 MB:
 // 18 us at the rate of a copy). 512 -> 128 stays there: 29 us, here 31, as the rows arrive before the first product; and so
 // do fewer than two workgroups a CU (512 rows of 16 heads: 10 us, here 11), and gated outputs of many workgroups and fewer
-// inputs (4,096 rows, 16 heads of 1,024, times a gate: of 64 inputs 117 us, here 145, of 128 136, 149; of 8 heads 46, 38 and 51, 42).
+// inputs (4,096 rows, 16 heads of 1,024, times a gate: of 64 inputs 117 us, here 145, of 128 136, 149; 8 heads 46, 38 and 51,
+// 42).
 constexpr int HEAD_UNIT = 65 * 16, HEAD_K32 = 8;
 
 template <int EPI>
@@ -481,10 +482,10 @@ static int launch_rows(const Args& A, int epi, int max_tiles, hipStream_t st) {
   return (int)hipGetLastError();
 }
 
-// Tiles of 16 and 32 rows whose stages of LDS do not pay: a wave's fragments straight from memory (gemm_kernel). us at 16 rows a tile,
-// rows_kernel against gemm_kernel: 64 experts of 2 x 256 x K and 96 rows, K = 256 6.9, 5.6, 512 9.3, 8.5, 1024 13.7, 14.2; of 2048 x K 16.3,
-// 13.1, 25.4, 23.8, 38.9, 45.0; few tiles end with their slowest (16 of 1024 x 512, 64 rows 6.6, 6.5; 24 of 2048 x 512 12.7, 13.3), and
-// few outputs leave rows_kernel few workgroups a group (64 of 128 x 2048, 600 rows 22, 16).
+// Tiles of 16 and 32 rows whose stages of LDS do not pay: a wave's fragments straight from memory (gemm_kernel). us at 16
+// rows a tile, rows_kernel against gemm_kernel: 64 experts of 2 x 256 x K and 96 rows, K = 256 6.9, 5.6, 512 9.3, 8.5, 1024
+// 13.7, 14.2; of 2048 x K 16.3, 13.1, 25.4, 23.8, 38.9, 45.0. Few tiles end with their slowest (16 of 1024 x 512, 64 rows 6.6,
+// 6.5; 24 of 2048 x 512 12.7, 13.3); few outputs leave rows_kernel few workgroups a group (64 of 128 x 2048, 600 rows 22, 16).
 static bool few_inputs(const Args& A, bool glu, int max_tiles) {
   if (max_tiles > 65535) return false;  // (a dimension of its grid)
   const bool narrow = A.N16 <= 16 && max_tiles >= (A.K32 <= 16 ? 64 : 96);

@@ -774,8 +774,8 @@ __global__ __launch_bounds__(64 * NW, 2) void mfma_kernel(const Args A) {
   // Two passes over the workgroup's items, so that neither path's registers carry the other's.
   if constexpr (RT >= PAIRS) {
     // Tiles are dealt in rounds over the workgroups, every second one from its end: a prompt's later items have more keys,
-    // and with one workgroup a CU each gets as many keys in all (4,096 tokens, dealt in one direction: 341 us, CUs busy two
-    // thirds of the time; here 318).
+    // and with one workgroup a CU each gets as many keys in all (4,096 tokens, as many workgroups as items: 341 us, here
+    // 318).
     for (int r = 0, b = blockIdx.y; r * (int)gridDim.y < n; ++r, b = gridDim.y - 1 - b) {
       const int item = r * gridDim.y + b;
       if (item >= n) continue;

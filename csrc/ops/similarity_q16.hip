@@ -778,8 +778,8 @@ __device__ __forceinline__ float div_rn(float x, float y) {
 
 // One workgroup a query: normalised (if asked), then rounded to bf16, or to 16-bit fixed point as q16_quantize does:
 // s_q = max|x| / 32512, v = round(x / s_q) = 256 qh + ql, c_q = s_q ||v||_2 (a hair above). NaN goes where torch's
-// operations take it: a norm or a maximum of a query that holds one is one (s_q is then 1), and in v it is 0. One launch in place of the 28
-// elementwise ones that took as long as the search of a small index.
+// operations take it: a norm or a maximum of a query that holds one is one (s_q is then 1), and in v it is 0. One launch in
+// place of the 28 elementwise ones that took as long as the search of a small index.
 __global__ __launch_bounds__(256) void prepare_kernel(const float* __restrict__ x, int D, int normalize, bf16* __restrict__ out,
                                                       signed char* __restrict__ qv, float* __restrict__ qmeta) {
   __shared__ double red[4];

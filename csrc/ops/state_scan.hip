@@ -618,7 +618,8 @@ __global__ __launch_bounds__(256) void chunk_state_kernel(const Args A) {
   }
 }
 
-// The state before every chunk, in place of U_c, and the last one to the slot: 4 values a thread, chunk after chunk; the next 8 chunks are on their way while 8 are written
+// The state before every chunk, in place of U_c, and the last one to the slot: 4 values a thread, chunk after chunk; the
+// next 8 chunks are on their way while 8 are written
 __global__ __launch_bounds__(256) void state_pass_kernel(const Args A) {
   const int h = blockIdx.z, VN = A.V * A.N, e = (blockIdx.x * 256 + threadIdx.x) * 4, n_items = A.n_items[0];
   if (e >= VN || (A.form && !A.form[0])) return;

@@ -85,15 +85,15 @@ def layer_runs(layers: int, loop: Optional[Tuple[int, int, int]]) -> List[Tuple[
 
 # (most rows a group has on average, rows per sorted tile) of the grouped projections: the fewest that hold a group's rows,
 # with room for uneven groups, so that its weights are read once; above, 256 (the ping-pong kernels, whose MFMAs end with a
-# tile's last 64 rows). us of both products, weights cold: 64 experts of 3 x 1408 x 2048, 6 rows an expert 16: 180, 32: 189; 14 rows 16:
-# 203, 32: 194, 256: 201; 28 rows 32: 223, 64: 211, 256: 203; 94 rows 64: 289, 128: 253, 256: 225; 8 of 3 x 14336 x 4096, 16 rows 16: 579,
-# 32: 460, 256: 513; 37 rows 32: 744, 64: 519, 256: 529; 75 rows 64: 713, 128: 727, 256: 556. Of few inputs 16 rows go further (64 of
-# 3 x 192 x 512, 14 rows 16: 16.1, 32: 17.8, 256: 18.6; 28 rows 32: 19.6, 64: 22.9, 256: 19.0).
+# tile's last 64 rows). us of both products, weights cold: 64 experts of 3 x 1408 x 2048, 6 rows an expert 16: 180, 32: 189;
+# 14 rows 16: 203, 32: 194, 256: 201; 28 rows 32: 223, 64: 211, 256: 203; 94 rows 64: 289, 128: 253, 256: 225; 8 of 3 x 14336
+# x 4096, 16 rows 16: 579, 32: 460, 256: 513; 37 rows 32: 744, 64: 519, 256: 529; 75 rows 64: 713, 128: 727, 256: 556. Of few
+# inputs 16 rows go further (64 of 3 x 192 x 512, 14 rows 16: 16.1, 32: 17.8, 256: 18.6; 28 rows 32: 19.6, 64: 22.9, 256: 19.0).
 GROUP_TILES, SHORT_GROUP_TILES = ((10, 16), (24, 32)), ((16, 16), (24, 32))
-# of one group (gate and up of a dense unit): 64 rows share the weights through the caches of an XCD up to 448 rows (2 x 8192 x 2048:
-# 44 us at 400 rows, 256-row tiles 47), with weights above 128 MB up to 128 (2 x 14336 x 4096: 66 us at 100 rows, 81; 256 rows 89, 88);
-# weights below 32 MB, whose 64-row tiles are few workgroups, take 32 up to 64 rows (2 x 4096 x 1024: 8.9 us at 64 rows, 64-row
-# tiles 10.9; 2 x 8192 x 2048 23, 21)
+# of one group (gate and up of a dense unit): 64 rows share the weights through the caches of an XCD up to 448 rows (2 x 8192
+# x 2048: 44 us at 400 rows, 256-row tiles 47), with weights above 128 MB up to 128 (2 x 14336 x 4096: 66 us at 100 rows, 81;
+# 256 rows 89, 88); weights below 32 MB, whose 64-row tiles are few workgroups, take 32 up to 64 rows (2 x 4096 x 1024: 8.9 us
+# at 64 rows, 64-row tiles 10.9; 2 x 8192 x 2048 23, 21)
 ONE_SMALL_GROUP_TILES, ONE_GROUP_TILES = ((16, 16), (64, 32), (448, 64)), ((16, 16), (32, 32), (448, 64))
 ONE_LARGE_GROUP_TILES = ((16, 16), (32, 32), (128, 64))
 

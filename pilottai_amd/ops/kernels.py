@@ -490,10 +490,10 @@ def decode_gemm(x: torch.Tensor, wp: torch.Tensor, epi: str = "plain", norm: boo
 
 def rows_gemm_pays(M: int, N: int, K: int) -> bool:
     """Whether rows_gemm is the faster one for more than 64 rows: its workgroups walk the whole of K, prefill_gemm's split it.
-    us, prefill_gemm against rows_gemm: tiles of 32 x 32 and smaller (512 x 512) K 128 6.2, 5.0, 14336 51, 38; of 32 x 64 (1408
-    outputs of 300 rows) K 128 6.3, 6.1, 8192 33, 30, 14336 48, 50, (512 of 768) K 128 6.2, 6.6; of 64 x 64 (3072 of 128) K 8192 35, 29,
-    (2048 of 300) K 128 6.3, 6.6, 4096 25, 21, 8192 34, 38, (512 of 2048) K 2048 20, 17, 4096 26, 27; of 64 x 128 (10368 of 128) K 4096
-    41, 38, 8192 61, 70, (4096 of 512) K 2048 25, 18, 4096 31, 34."""
+    us, prefill_gemm against rows_gemm: tiles of 32 x 32 and smaller (512 x 512) K 128 6.2, 5.0, 14336 51, 38; of 32 x 64
+    (1408 outputs of 300 rows) K 128 6.3, 6.1, 8192 33, 30, 14336 48, 50, (512 of 768) K 128 6.2, 6.6; of 64 x 64 (3072 of 128)
+    K 8192 35, 29, (2048 of 300) K 128 6.3, 6.6, 4096 25, 21, 8192 34, 38, (512 of 2048) K 2048 20, 17, 4096 26, 27; of 64 x 128
+    (10368 of 128) K 4096 41, 38, 8192 61, 70, (4096 of 512) K 2048 25, 18, 4096 31, 34."""
     fits = lambda m, n: -(-M // m) * -(-N // n) <= 256  # noqa: E731  (dispatch_rows' choice of a tile)
     if fits(32, 32):
         return True

@@ -92,8 +92,7 @@ def test_q16_fewer_hits_than_k(gpu):
 
 @pytest.mark.parametrize("Q,D", [(1, 64), (64, 1024), (5, 320)])
 def test_query_preparation_matches_torch(gpu, Q, D):
-    """The kernel's fixed-point queries have the bits of the CPU's; normalised ones differ by the rounding of the norm
-    (a sum in float64 against one in float32): at most 2 ulp of a coordinate, 1 unit of its 16-bit form."""
+    """The kernel's queries against the CPU's at several shapes, and against torch's normalised rows: bf16's rounding."""
     q = torch.randn(Q, D, device=gpu) * 3.0
     q[0, 1:] = 0.0
     if Q > 2:
