@@ -105,9 +105,8 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
   // W part r: chunk q = 2 wid + h (h = 0, 1) is n-frag (wid & 3) of group (wid >> 2),
   // k-half h of the 64-k tile: n16 tile nt * 16 + (wid >> 2) * 8 + r * 4 + (wid & 3).
   const int KS = A.K >> 5;
-  // token (of the tile) of wave column w's fragment j, row r: a wave has 64 in a row; of a group's tile, which may
-  // hold few rows, its fragments lie 64 apart, so that fragments past the last row are the same of all waves
-  auto token = [](int w, int j, int r) { return GR ? 64 * j + 16 * w + r : 64 * w + 16 * j + r; };
+  // Wave column w's fragment j, row r is token 64 w + 16 j + r of the tile; of a group's tile, which may hold few rows,
+  // 64 j + 16 w + r, so that fragments past the last row are the same of all waves.
   // x part c: LDS row lr = (2 wid + h) * 8 + (lane >> 3) holds row lr & 15 of wave column lr >> 5's
   // fragment 2 c + (lr >> 4 & 1); its 16-B unit (lane & 7) is the row's logical unit (lane & 7) ^ ((lr >> 1) & 7).
   int xrow[2][2], xunit[2][2];
@@ -116,7 +115,8 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int lr = (2 * wid + h) * 8 + (lane >> 3);
-      xrow[cc][h] = min(row0 + token(lr >> 5, 2 * cc + ((lr >> 4) & 1), lr & 15), A.M - 1);
+      const int m = GR ? row0 + 64 * (2 * cc + (lr >> 4 & 1)) + 16 * (lr >> 5) + (lr & 15) : row0 + (lr >> 5) * 64 + cc * 32 + (lr & 31);
+      xrow[cc][h] = min(m, A.M - 1);
       xunit[cc][h] = (lane & 7) ^ ((lr >> 1) & 7);
       if constexpr (GR)
         if (A.xmap) xrow[cc][h] = A.xmap[xrow[cc][h]] / A.xdiv;
@@ -372,41 +372,53 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
     body6(t, ic<1>{});
     body6(t + 1, ic<2>{});
   } else {
-    // with JN token frags of 4 (below 3, B1 is neither staged nor read)
-    auto run = [&](auto jn) {
-      constexpr bool B1 = decltype(jn)::value > 2;
+    auto body = [&](int tt, auto st, auto jn) {
+      if constexpr (F == 8) body2(tt, st, jn);
+      else body4(tt, st, jn);
+    };
+    if constexpr (GR) {
+      // with JN token frags of 4 (below 3, B1 is neither staged nor read)
+      auto run = [&](auto jn) {
+        constexpr bool B1 = decltype(jn)::value > 2;
+        issue_w(0, 0);
+        issue_x(0, 0);
+        if constexpr (B1) issue_x(1, 0);
+        if constexpr (F == 8) issue_w(1, 0);
+        issue_w(0, 1);
+        issue_x(0, 1);
+        if constexpr (B1 && F == 4) issue_x(1, 1);
+        wait_vm<F == 8 ? 6 : B1 ? 8 : 4>();  // as below
+        raw_barrier();
+        if (G == 1) raw_barrier();
+        for (; t + 2 < nk; ++t) body(t, ic<0>{}, jn);
+        body(t, ic<1>{}, jn);
+        body(t + 1, ic<2>{}, jn);
+      };
+      // a group's last tile may hold few rows: each 64 fewer leave out a quarter of the MFMAs (4,096 tokens, 6 of 64
+      // experts of 2,048 x 2 x 1,408 and back, 384 rows each on average: 322 + 167 -> 284 + 156 us)
+      if (A.M > 192) run(ic<4>{});
+      else if (A.M > 128) run(ic<3>{});
+      else if (A.M > 64) run(ic<2>{});
+      else run(ic<1>{});
+    } else {  // (written out: as run(ic<4>{}) the dense kernels get other code, 0.4 to 0.7 % of a step of 2,048 rows slower)
       issue_w(0, 0);
       issue_x(0, 0);
-      if constexpr (B1) issue_x(1, 0);
+      issue_x(1, 0);
       if constexpr (F == 8) issue_w(1, 0);
       issue_w(0, 1);
       issue_x(0, 1);
       if constexpr (F == 8) {
         wait_vm<6>();  // A0, B0 and B1 of tile 0 landed
       } else {
-        if constexpr (B1) issue_x(1, 1);
-        wait_vm<B1 ? 8 : 4>();  // A and B0 of tile 0 landed
+        issue_x(1, 1);
+        wait_vm<8>();  // A and B0 of tile 0 landed
       }
       raw_barrier();
       if (G == 1) raw_barrier();
       if constexpr (STAMP) st1 = __builtin_amdgcn_s_memtime();
-      auto body = [&](int tt, auto st) {
-        if constexpr (F == 8) body2(tt, st, jn);
-        else body4(tt, st, jn);
-      };
-      for (; t + 2 < nk; ++t) body(t, ic<0>{});
-      body(t, ic<1>{});
-      body(t + 1, ic<2>{});
-    };
-    // a group's last tile may hold few rows: each 64 fewer leave out a quarter of the MFMAs (4,096 tokens, 6 of 64
-    // experts of 2,048 x 2 x 1,408 and back, 384 rows each on average: 322 + 167 -> 284 + 156 us)
-    if constexpr (GR) {
-      if (A.M > 192) run(ic<4>{});
-      else if (A.M > 128) run(ic<3>{});
-      else if (A.M > 64) run(ic<2>{});
-      else run(ic<1>{});
-    } else {
-      run(ic<4>{});
+      for (; t + 2 < nk; ++t) body(t, ic<0>{}, ic<4>{});
+      body(t, ic<1>{}, ic<4>{});
+      body(t + 1, ic<2>{}, ic<4>{});
     }
   }
   if (G == 0) raw_barrier();  // balance the stagger
@@ -448,12 +460,12 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
     }
   }
 
-  // ---- register epilogue: acc[i][j] holds token row0 + token(wc, j, c), columns
+  // ---- register epilogue: acc[i][j] holds token row0 + 64 wc + 16 j + c (a group's: row0 + 64 j + 16 wc + c), columns
   // 4 g .. 4 g + 3 of 16-column tile nt * 2F + F G + i
   const float inv_k = 1.f / (float)A.K;
 #pragma unroll
   for (int j = 0; j < 4; ++j) {
-    int m = row0 + token(wc, j, c);
+    int m = GR ? row0 + 64 * j + 16 * wc + c : row0 + wc * 64 + 16 * j + c;
     const bool ok = m < A.M;
     float rs = 1.f;
     if constexpr (GR) {
