@@ -115,7 +115,8 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
       const int lr = (2 * wid + h) * 8 + (lane >> 3);
-      const int m = GR ? row0 + 64 * (2 * cc + (lr >> 4 & 1)) + 16 * (lr >> 5) + (lr & 15) : row0 + (lr >> 5) * 64 + cc * 32 + (lr & 31);
+      const int m = GR ? row0 + 64 * (2 * cc + (lr >> 4 & 1)) + 16 * (lr >> 5) + (lr & 15)
+                       : row0 + (lr >> 5) * 64 + cc * 32 + (lr & 31);
       xrow[cc][h] = min(m, A.M - 1);
       xunit[cc][h] = (lane & 7) ^ ((lr >> 1) & 7);
       if constexpr (GR)
@@ -400,7 +401,8 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
       else if (A.M > 128) run(ic<3>{});
       else if (A.M > 64) run(ic<2>{});
       else run(ic<1>{});
-    } else {  // (written out: as run(ic<4>{}) the dense kernels get other code, 0.4 to 0.7 % of a step of 2,048 rows slower)
+    } else {
+      // (Written out: through run, the dense kernels get other code, and a step of 2,048 rows takes 0.4 to 0.7 % longer.)
       issue_w(0, 0);
       issue_x(0, 0);
       issue_x(1, 0);
