@@ -8,8 +8,8 @@
 // Weights are packed per group like the other projections ([N/16, K/32, 64, 8], one 16-B lane
 // vector per MFMA operand). The MFMA's A operand is W and its B operand x, so a lane's four
 // accumulators are four consecutive outputs of one row: 8-byte stores, and the gated pair
-// (tiles 2i: gate, 2i + 1: up) is lane-local. Sorted rows go in tiles of 16 to 128, as many as a group
-// has on average; prompts with more run the ping-pong kernels instead (gemm_prefill.hip pa_expert_tiles).
+// (tiles 2i: gate, 2i + 1: up) is lane-local. Sorted rows go in tiles of 16 to 128, as the caller asks (experts: 16
+// and 32 up to 24 rows on average, one group: up to 64); more run the ping-pong kernels (gemm_prefill.hip pa_expert_tiles).
 //
 // Epilogues: plain, the gated unit of packed_epi.h (limit, alpha, cubic, bias), or the square of relu; of dense rows
 // also the product times sigmoid(gate), and the gated unit whose second factor is the row's embedding in a table.
@@ -346,9 +346,10 @@ __global__ __launch_bounds__(256, 2) void head_rows_kernel(const Args A) {
 // side by side over a pair of 16-output tiles each; with WK > 1, WK of them share one pair and split the k-steps of a
 // stage, which leaves more workgroups. Weights and rows are one in-order ring of loads, D stages deep; the stage barrier
 // waits for LDS alone. NTW: weights that no other tile reads are loaded non-temporal.
-// Bound by the weights' bytes up to 128 rows a group: 64 experts of 2 x 1408 x 2048 and 2048 x 1408 and a shared one,
-// both products, us before -> after: 64 tokens 215 -> 182 (5.4 TB/s), 400 275 -> 228, 750 414 -> 284, 1000 456 -> 295; a
-// dense 2 x 8192 x 2048 gate and up of 64 rows 30 -> 17, of 256 rows 45 -> 33.
+// Bound by the weights' bytes: 64 experts of 2 x 1408 x 2048 and 2048 x 1408 and a shared one, both products, us before ->
+// after: 64 tokens 215 -> 182 (5.4 TB/s), 400 275 -> 228, 1000 456 -> 295 (the ping-pong kernels are the
+// faster ones from 25 rows a group on: GROUP_TILES in models/common.py); a dense 2 x 8192 x 2048 gate and up of 64 rows
+// 30 -> 17, of 256 rows 45 -> 33.
 template <int MT, int WK, int EPI, bool NTW>
 __global__ __launch_bounds__(512, MT == 8 ? 4 : 2) void rows_kernel(const Args A) {
   constexpr int WN = 8 / WK, NT = 2, KW = 2, D = 2;
