@@ -8,7 +8,8 @@ int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out, long long
                     int ldo, int og, int rows, int N16, int K32, const int* tiles, int max_tiles, const int* n_tiles,
                     const int* order, int x_div, int out_order, int tm, int epi, float limit, float alpha, float cubic, float bias,
                     const int* positions, const float* cos_sin, int rskip, int r, int rp, int rd, const float* row_w,
-                    const void* gate, int ldg, const void* table, const int* ids, int ldt, int tcol, int vocab, hipStream_t st);
+                    const void* gate, int ldg, const void* table, const int* ids, int ldt, int tcol, int vocab, const int* skip,
+                    hipStream_t st);
 }
 
 namespace {
@@ -55,9 +56,9 @@ void dims(const at::Tensor& w, int f, int64_t* G, int64_t* N, int64_t* K) {
 
 // every row of x through every group: x columns g * xg .. + K -> out columns g * og .. + N; with
 // positions / cos_sin also the rotated part: x columns g * xg + rskip .. + r -> out columns g * og + N .. + rp; with gate
-// times sigmoid(gate), whose columns are out's
+// times sigmoid(gate), whose columns are out's; rows whose entry of skip is not 0 stay as they are
 void head_gemm(at::Tensor x, int64_t xg, at::Tensor w, at::Tensor out, int64_t og, Opt positions, Opt cos_sin,
-               int64_t rskip, int64_t r, int64_t rp, Opt gate) {
+               int64_t rskip, int64_t r, int64_t rp, Opt gate, Opt skip) {
   const int f = is_f32(x, "x");
   check_rows(x, x.scalar_type(), "x");
   check_rows(out, x.scalar_type(), "out");
@@ -89,7 +90,8 @@ void head_gemm(at::Tensor x, int64_t xg, at::Tensor w, at::Tensor out, int64_t o
   check_rc(pa_grouped_gemm(f, x.data_ptr(), w.data_ptr(), out.data_ptr(), N * K, G, x.stride(0), xg, out.stride(0), og,
                            x.size(0), N / 16, K / 32, nullptr, 0, nullptr, nullptr, 0, 0, 0, gate.has_value() ? 3 : 0, 0.f, 0.f,
                            0.f, 0.f, pos, cs, rskip, r, rp, rd, nullptr, gate.has_value() ? gate->data_ptr() : nullptr,
-                           gate.has_value() ? gate->stride(0) : 0, nullptr, nullptr, 0, 0, 0, cur_stream()),
+                           gate.has_value() ? gate->stride(0) : 0, nullptr, nullptr, 0, 0, 0,
+                           skip.has_value() ? ints(*skip, x.size(0), "skip") : nullptr, cur_stream()),
            "head_gemm");
 }
 
@@ -109,7 +111,7 @@ void table_gemm(at::Tensor x, at::Tensor w, at::Tensor out, at::Tensor table, at
   check_rc(pa_grouped_gemm(f, x.data_ptr(), w.data_ptr(), out.data_ptr(), N * K, 1, x.stride(0), 0, out.stride(0), 0,
                            x.size(0), N / 16, K / 32, nullptr, 0, nullptr, nullptr, 0, 0, 0, 4, (float)limit, (float)alpha,
                            (float)cubic, (float)bias, nullptr, nullptr, 0, 0, 0, 0, nullptr, nullptr, 0, table.data_ptr(),
-                           ints(ids, x.size(0), "ids"), table.stride(0), (int)tcol, table.size(0), cur_stream()),
+                           ints(ids, x.size(0), "ids"), table.stride(0), (int)tcol, table.size(0), nullptr, cur_stream()),
            "table_gemm");
 }
 
@@ -136,7 +138,7 @@ void expert_gemm(at::Tensor x, at::Tensor w, at::Tensor out, at::Tensor tiles, a
                            N / 16, K / 32, ints(tiles, 4, "tiles"), tiles.size(0), ints(n_tiles, 1, "n_tiles"),
                            ints(order, rows, "order"), x_div, out_order ? 1 : 0, tm, (int)epi, (float)limit,
                            (float)alpha, (float)cubic, (float)bias, nullptr, nullptr, 0, 0, 0, 0, opt_f32(row_w, rows, "row_w"),
-                           nullptr, 0, nullptr, nullptr, 0, 0, 0, cur_stream()),
+                           nullptr, 0, nullptr, nullptr, 0, 0, 0, nullptr, cur_stream()),
            "expert_gemm");
 }
 

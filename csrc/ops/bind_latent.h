@@ -2,6 +2,7 @@
 // and the attention over it.
 #pragma once
 #include "bind_grouped.h"
+#include "latent_expand.h"
 
 extern "C" {
 int pa_residual_norm(int fp32, float* resid, const void* y, int K, int ldy, float y_scale, const float* w_post,
@@ -16,7 +17,11 @@ int pa_latent_attention(int fp32, void* out, float* part_o, float* part_ml, cons
                         const int* items, const int* n_items, int max_items, const int* q_start,
                         const int* q_len, const int* ctx_len, const int* block_table, int max_blocks, int H, int Rp,
                         int rp, int dec_tokens, int tile_tokens, int window, float scale_log2, int simple,
-                        hipStream_t st);
+                        const pa::la::Expand* expand, hipStream_t st);
+int pa_latent_plan(const pa::la::Expand* X, const int* q_start, const int* q_len, const int* ctx_len, int S, int T, int H, int window,
+                   int room, int max_att, int max_tiles, int slots, hipStream_t st);
+int pa_latent_expand(const pa::la::Expand* X, const void* pages, const void* wk, const void* wv, const int* block_table, int max_blocks, int H, int D,
+                     int max_tiles, hipStream_t st);
 }
 
 namespace {
@@ -95,10 +100,71 @@ void latent_cache(at::Tensor x, int64_t NQ, int64_t R, int64_t r, Opt w_q, at::T
            "latent_cache");
 }
 
+// What a step's plan of expanded requests holds: [counts, base, form, attention items, expansion tiles] (latent_expand.h)
+using Tensors = std::vector<at::Tensor>;
+pa::la::Expand expand_plan(const Tensors& p, int64_t S, int64_t T) {
+  TORCH_CHECK(p.size() == 5 && p[3].dim() == 2 && p[3].size(1) == 4 && p[4].dim() == 2 && p[4].size(1) == 4,
+              "a plan is [counts, base, form, items [n, 4], tiles [n, 4]]");
+  pa::la::Expand X{};
+  X.counts = (int*)ints(p[0], 2, "counts");
+  X.base = (int*)ints(p[1], S, "base");
+  X.form = (int*)ints(p[2], T, "form");
+  X.att = (int4*)ints(p[3], 4, "items");
+  X.tiles = (int4*)ints(p[4], 4, "tiles");
+  return X;
+}
+
+// The workspace: kx [blocks, H, 32, 16, 8] and kr [blocks, 8, 16, 8]
+void expand_room(pa::la::Expand& X, const at::Tensor& kx, const at::Tensor& kr, int64_t H) {
+  for (auto* t : {&kx, &kr}) {
+    check_gpu(*t, "workspace");
+    check_dtype(*t, at::kBFloat16, "workspace");
+  }
+  TORCH_CHECK(kx.dim() == 5 && kx.size(1) == H && kx.size(2) * 8 == 2 * pa::la::X_DIM && kx.size(3) == 16 && kx.size(4) == 8 &&
+                  kr.dim() == 4 && kr.size(0) == kx.size(0) && kr.size(1) * 8 == pa::la::X_ROT && kr.size(2) == 16 && kr.size(3) == 8,
+              "workspace must be [blocks, H, 32, 16, 8] and [blocks, 8, 16, 8]");
+  X.kx = kx.data_ptr();
+  X.kr = kr.data_ptr();
+}
+
+// Decides which requests of the step have their keys expanded and writes the plan; `slots` partial results and `room` blocks
+// are what the launches with this plan have.
+void latent_plan(const Tensors& plan, at::Tensor q_start, at::Tensor q_len, at::Tensor ctx_len, int64_t T, int64_t H, int64_t window,
+                 int64_t room, int64_t slots) {
+  const int64_t S = q_len.numel();
+  const pa::la::Expand X = expand_plan(plan, S, T);
+  TORCH_CHECK(T >= 1 && H >= 1 && room >= 1 && slots >= 0 &&
+                  plan[3].size(0) >= T / pa::la::X_COLS + pa::la::X_REQS + slots, "latent_plan sizes");
+  check_rc(pa_latent_plan(&X, ints(q_start, S, "q_start"), ints(q_len, S, "q_len"), ints(ctx_len, S, "ctx_len"), S, T, H, window, room,
+                          plan[3].size(0), plan[4].size(0), slots, cur_stream()),
+           "latent_plan");
+}
+
+// keys and values of the planned requests from their pages: wk, wv [H, 8, 16, 64, 8], the heads' rows of W_uk and of W_uv
+void latent_expand(const Tensors& plan, at::Tensor kx, at::Tensor kr, at::Tensor pages, at::Tensor wk, at::Tensor wv,
+                   at::Tensor block_table) {
+  pa::la::Expand X = expand_plan(plan, block_table.size(0), 0);
+  const int64_t H = wk.size(0);
+  for (auto* t : {&pages, &wk, &wv}) {
+    check_gpu(*t, "latent_expand arg");
+    check_dtype(*t, at::kBFloat16, "latent_expand arg");
+  }
+  for (auto* w : {&wk, &wv})
+    TORCH_CHECK(w->dim() == 5 && w->size(0) == H && w->size(1) * 16 == pa::la::X_DIM && w->size(2) * 32 == pa::la::X_RANK &&
+                    w->size(3) == 64 && w->size(4) == 8, "weights must be packed [H, 8, 16, 64, 8]");
+  TORCH_CHECK(pages.dim() == 4 && pages.size(1) * 8 == pa::la::X_RANK + pa::la::X_ROT && pages.size(2) == 16 && pages.size(3) == 8,
+              "pages must be [blocks, 72, 16, 8]");
+  TORCH_CHECK(block_table.dim() == 2, "block_table [seqs, blocks]");
+  expand_room(X, kx, kr, H);
+  check_rc(pa_latent_expand(&X, pages.data_ptr(), wk.data_ptr(), wv.data_ptr(), ints(block_table, 0, "block_table"), block_table.size(1),
+                            H, pages.size(1) * 8, plan[4].size(0), cur_stream()),
+           "latent_expand");
+}
+
 void latent_attention(at::Tensor out, at::Tensor part_o, at::Tensor part_ml, at::Tensor q,
                       at::Tensor pages, at::Tensor items, at::Tensor n_items, at::Tensor q_start, at::Tensor q_len,
                       at::Tensor ctx_len, at::Tensor block_table, int64_t dec_tokens, int64_t tile_tokens,
-                      int64_t window, double scale, bool simple) {
+                      int64_t window, double scale, bool simple, const Tensors& plan, const Tensors& expand) {
   const int f = is_f32(q, "q");
   for (auto* t : {&out, &q, &pages}) {
     check_gpu(*t, "latent_attention arg");
@@ -113,12 +179,35 @@ void latent_attention(at::Tensor out, at::Tensor part_o, at::Tensor part_ml, at:
   const int64_t NB = (dec_tokens * H + 15) / 16;
   TORCH_CHECK(Rp > 0 && rp >= 0 && dec_tokens >= 1 && tile_tokens >= 1, "latent_attention sizes");
   TORCH_CHECK(part_o.numel() >= mi * NB * 16 * Rp && part_ml.numel() >= mi * NB * 32, "partition workspace too small");
+  // expanded requests: expand = [kx, kr, q not yet absorbed or rotated, cos_sin, their outputs, partial outputs and (max, sum)]
+  pa::la::Expand X{};
+  if (!expand.empty()) {
+    const int64_t T = q.size(0), slot = H * pa::la::X_COLS, slots = expand.size() == 7 ? expand[6].numel() / (2 * slot) : 0;
+    TORCH_CHECK(!f && expand.size() == 7 && Rp == pa::la::X_RANK && rp == pa::la::X_ROT, "latent_attention: expanded sizes");
+    X = expand_plan(plan, S, T);
+    expand_room(X, expand[0], expand[1], H);
+    const at::Tensor &xq = expand[2], &xo = expand[4];
+    check_rows(xq, at::kBFloat16, "q");
+    check_rows(xo, at::kBFloat16, "expanded out");
+    TORCH_CHECK(xq.size(0) == T && xq.size(1) >= H * (pa::la::X_DIM + pa::la::X_ROT) && xq.stride(0) % 8 == 0 &&
+                    ((uintptr_t)xq.data_ptr() & 15) == 0 && xo.size(0) == T && xo.size(1) >= H * pa::la::X_DIM &&
+                    xo.stride(0) % 4 == 0 && ((uintptr_t)xo.data_ptr() & 7) == 0, "latent_attention: rows of expanded requests");
+    TORCH_CHECK(expand[3].dim() == 2 && expand[3].size(1) == pa::la::X_ROT, "cos_sin must be [positions, 64]");
+    X.q = xq.data_ptr();
+    X.ldq = xq.stride(0);
+    X.cos_sin = opt_f32(expand[3], 0, "cos_sin");
+    X.out = xo.data_ptr();
+    X.ldo = xo.stride(0);
+    X.part_o = (float*)opt_f32(expand[5], slots * slot * pa::la::X_DIM, "partial outputs");
+    X.part_ml = (float*)opt_f32(expand[6], 0, "partial sums");
+  }
   check_rc(pa_latent_attention(f, out.data_ptr(), (float*)opt_f32(part_o, 0, "part_o"),
                                (float*)opt_f32(part_ml, 0, "part_ml"), q.data_ptr(),
                                pages.data_ptr(), ints(items, 0, "items"), ints(n_items, 1, "n_items"), mi,
                                ints(q_start, S, "q_start"), ints(q_len, S, "q_len"), ints(ctx_len, S, "ctx_len"),
                                ints(block_table, 0, "block_table"), block_table.size(1), H, Rp, rp, dec_tokens,
-                               tile_tokens, window, (float)(scale * 1.4426950408889634), simple ? 1 : 0, cur_stream()),
+                               tile_tokens, window, (float)(scale * 1.4426950408889634), simple ? 1 : 0,
+                               expand.empty() ? nullptr : &X, cur_stream()),
            "latent_attention");
 }
 

@@ -39,6 +39,8 @@ PYBIND11_MODULE(_latent, m) {
   m.def("latent_cache", &latent_cache);
   m.def("latent_pad", [](int R) { return pa_latent_pad(R); });
   m.def("latent_attention", &latent_attention);
+  m.def("latent_plan", &latent_plan);
+  m.def("latent_expand", &latent_expand);
   m.def("table_route", &table_route);
   m.def("head_gemm", &head_gemm);
   m.def("table_gemm", &table_gemm);

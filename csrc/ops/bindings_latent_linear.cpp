@@ -69,6 +69,8 @@ PYBIND11_MODULE(_latent_linear, m) {
   m.def("latent_cache", &latent_cache);
   m.def("latent_pad", [](int R) { return pa_latent_pad(R); });
   m.def("latent_attention", &latent_attention);
+  m.def("latent_plan", &latent_plan);
+  m.def("latent_expand", &latent_expand);
   m.def("linear_attention", &linear_attention);
   m.def("gated_norm", &gated_norm);
   m.def("poly_norm", &poly_norm);

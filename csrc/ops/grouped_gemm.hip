@@ -48,7 +48,15 @@ struct Args {
   const void *gate, *table;
   const int* ids;
   int ldg, ldt, tcol, vocab;
+  const int* skip;  // dense, optional: rows that are not 0 here stay as they are
 };
+
+// all of a tile's rows (64 at most) are left out
+__device__ __forceinline__ bool skipped(const Args& A, int start, int n) {
+  if (!A.skip) return false;
+  const int lane = threadIdx.x & 63;
+  return __all(lane >= n || A.skip[start + min(lane, n - 1)] != 0);
+}
 
 // The rotated columns of `n` rows from `start` of group grp (one workgroup).
 template <typename T>
@@ -124,6 +132,7 @@ __device__ __forceinline__ void store_rows(const Args& A, int grp, int start, in
   for (int m = 0; m < MT; ++m) {
     if (16 * m + c >= n) continue;
     const int at = start + 16 * m + c;
+    if (A.skip && A.skip[at]) continue;
     bf16* o = (bf16*)A.out + (size_t)at * A.ldo + (size_t)grp * A.og + 4 * g;
     if constexpr (EPI == GATED) {
       const bf16* f = factor_row<bf16, EPI>(A, at, grp) + 4 * g;
@@ -202,6 +211,8 @@ __global__ __launch_bounds__(256) void gemm_kernel(const Args A) {
     grp = tl.x;
     start = tl.y;
     n = tl.z;
+  } else {
+    if (skipped(A, start, n)) return;
   }
   if (A.rp && blockIdx.x == 0) {
     rotate_rows<bf16>(A, grp, start, n);
@@ -278,6 +289,7 @@ __global__ __launch_bounds__(256, 2) void head_rows_kernel(const Args A) {
   extern __shared__ __attribute__((aligned(16))) char xs[];
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), c = lane & 15, g = lane >> 4;
   const int grp = blockIdx.y, start = blockIdx.x * 64, n = min(64, A.rows - start), U = 4 * A.K32;
+  if (skipped(A, start, n)) return;
   const bf16* x = (const bf16*)A.x + (size_t)start * A.ldx + (size_t)grp * A.xg;
   const unsigned inv = ((1u << 20) + U - 1) / U;  // e / U of e < 4096
   bf16x8 v[HEAD_K32];
@@ -732,14 +744,15 @@ extern "C" int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out
                                int max_tiles, const int* n_tiles, const int* order, int x_div, int out_order, int tm,
                                int epi, float limit, float alpha, float cubic, float bias, const int* positions,
                                const float* cos_sin, int rskip, int r, int rp, int rd, const float* row_w, const void* gate,
-                               int ldg, const void* table, const int* ids, int ldt, int tcol, int vocab, hipStream_t st) {
+                               int ldg, const void* table, const int* ids, int ldt, int tcol, int vocab, const int* skip, hipStream_t st) {
+  if (skip && (fp32 || tiles || epi == 4)) return -1;
   if (N16 <= 0 || K32 <= 0 || (epi == 1 && N16 % 2)) return -1;
   if (row_w && (!tiles || epi != 1 || !x_div)) return -1;
   if (tiles ? epi > 2 : epi == 1 || epi == 2 || (epi == 3 && !gate) || (epi == 4 && (!table || !ids))) return -1;
   if (tiles ? max_tiles <= 0 : rows <= 0) return 0;
   const pa::gg::Args A{x, w, out, wstride, ldx, xg, ldo, og, rows, N16, K32, (const int4*)tiles, n_tiles,
                        order, x_div, out_order, limit, alpha, cubic, bias, positions, cos_sin, rskip, r, rp, rd,
-                       ldo % 8 == 0 && og % 8 == 0 && ((uintptr_t)out & 15) == 0, row_w, gate, table, ids, ldg, ldt, tcol, vocab};
+                       ldo % 8 == 0 && og % 8 == 0 && ((uintptr_t)out & 15) == 0, row_w, gate, table, ids, ldg, ldt, tcol, vocab, skip};
   const int rot = rp > 0 ? 1 : 0;  // one more column of workgroups
   if (fp32) {
     if (tiles && tm != 16) return -2;

@@ -27,7 +27,10 @@
 //   otherwise:        128 columns per workgroup, 16 per wave; all waves share double-buffered 32-key
 //                     tiles that arrive by direct global -> LDS loads. A step with few such items
 //                     has them cut into partitions of their keys too (8 slots each).
+//
+// Prompt portions of the widest latents have a second form (latent_expand.h), whose units the same launches run.
 #include "common.h"
+#include "latent_expand.h"
 
 #include <algorithm>
 
@@ -51,7 +54,12 @@ struct Args {
   const int *q_start, *q_len, *ctx_len, *block_table;
   int max_blocks, H, NB, Rp, D, dec_tokens, window;
   float scale_log2;
+  Expand X;
 };
+
+// requests whose keys are expanded take no part in the absorbed form
+template <bool XP>
+__device__ __forceinline__ bool expanded(const Args& A, int s) { return XP && A.X.base[s] != X_NONE; }
 
 // ---------------------------------------------------------------------------
 // Any sizes, bf16 or fp32: one workgroup per (token of an item, head). The exact path.
@@ -275,16 +283,44 @@ __device__ __forceinline__ void split_item(const Args& A, const int4 it, char* s
     reinterpret_cast<float2*>(A.part_ml)[((size_t)pidx * A.NB + cb) * 16 + ccol] = float2{mt, L};
 }
 
+// The partitions of the expanded units: a wave per (item, head, token), 2 dims per lane.
+__device__ __forceinline__ void merge_expanded(const Args& A) {
+  const int lane = threadIdx.x & 63, n = A.X.counts[0] * A.H * X_COLS;
+  const int waves = gridDim.x * gridDim.y * 4, w0 = (blockIdx.y * gridDim.x + blockIdx.x) * 4 + (threadIdx.x >> 6);
+  for (int w = w0; w < n; w += waves) {
+    const int4 it = A.X.att[w / (A.H * X_COLS)];
+    const int rest = w % (A.H * X_COLS), h = rest / X_COLS, tok = it.y * X_COLS + rest % X_COLS, parts = it.z >> 16;
+    if (parts <= 1 || (it.z & 0xffff) || tok >= A.q_len[it.x]) continue;
+    auto slot = [&](int p) { return (size_t)(it.w + p) * A.H * X_COLS + rest; };
+    float m = NEG_BIG, L = 0.f;
+    float2 v = {0.f, 0.f};
+    for (int p = 0; p < parts; ++p) m = fmaxf(m, reinterpret_cast<const float2*>(A.X.part_ml)[slot(p)].x);
+    for (int p = 0; p < parts; ++p) {
+      const float2 ml = reinterpret_cast<const float2*>(A.X.part_ml)[slot(p)];
+      const float2 o = reinterpret_cast<const float2*>(A.X.part_o)[slot(p) * (X_DIM / 2) + lane];
+      const float f = exp2f(ml.x - m);
+      L += f * ml.y;
+      v.x += f * o.x;
+      v.y += f * o.y;
+    }
+    const float inv = 1.f / L;
+    bf16* o = (bf16*)A.X.out + (size_t)(A.q_start[it.x] + tok) * A.X.ldo + h * X_DIM + 2 * lane;
+    o[0] = (bf16)(v.x * inv);
+    o[1] = (bf16)(v.y * inv);
+  }
+}
+
 // The partitions of an item, merged: a wave per (item, column), 8 dims per lane and step.
-template <int RT>
+template <int RT, bool XP = false>
 __global__ __launch_bounds__(256) void merge_kernel(const Args A) {
   constexpr int RP = 32 * RT;
   const int lane = threadIdx.x & 63;
   const int n = A.n_items[0];
+  if constexpr (XP) merge_expanded(A);
   for (int item = blockIdx.y; item < n; item += gridDim.y) {
     const int4 it = A.items[item];
     const int nq = it.z & 0xff, nparts = it.z >> 20;
-    if (nparts <= 1 || ((it.z >> 8) & 0xfff) != 0) continue;
+    if (nparts <= 1 || ((it.z >> 8) & 0xfff) != 0 || expanded<XP>(A, it.x)) continue;
     const int step = nq <= A.dec_tokens ? 1 : 8;  // slots of a partition
     for (int col = blockIdx.x * 4 + (threadIdx.x >> 6); col < nq * A.H; col += gridDim.x * 4) {
       auto slot = [&](int p) { return (size_t)(it.w + p * step) * A.NB * 16 + col; };
@@ -756,45 +792,463 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
   }
 }
 
+// A unit of the expanded form: X_COLS tokens of a request, one head, a part of their keys. Four column groups of 32 tokens
+// and two waves each, which take the 32-key tiles of a 64-key stage: a fragment read from LDS then serves two MFMAs, as many
+// bytes as the MFMAs take time for, and the two waves of a SIMD run the same columns, and the second adds its
+// outputs a stage late, so that one's softmax lies under the other's products. Stages arrive by direct loads two ahead (four
+// buffers), one barrier each; the two waves' outputs meet in LDS. 4,096 tokens, 16 heads: 125 us back to back with the merge
+// launch (MFMAs 38, without the softmax 102, without the loads 104: LDS reads, 1,280 cycles a stage as the MFMAs, and the
+// softmax's 1,600 of a SIMD's VALU overlap in part); pair_item takes 318 and two head projections of 32 each, here the
+// expansion's 25. 499 tokens after 3,584: 49 and 25 us, 110 and 22 in the absorbed form.
+constexpr int X_BLOCK = (2 * X_DIM + X_ROT) * 32, X_STAGE = 4 * X_BLOCK;  // bytes of 16 keys, of a stage
+
+// stages [lo, hi) of 64 keys that the tokens of a tile see
+__device__ __forceinline__ void unit_stages(int pos0, int n, int window, int& lo, int& hi) {
+  lo = (window > 0 ? max(0, pos0 - window + 1) : 0) >> 6;
+  hi = (pos0 + n + 63) >> 6;
+}
+
+__device__ __forceinline__ void expanded_unit(const Args& A, const int4 it, int h, char* smem) {
+  constexpr int NQ = (X_DIM + X_ROT) / 32, NV = X_DIM / 16;
+  const int s = it.x, part = it.z & 0xffff, nparts = it.z >> 16;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
+  const int cg = wid & 3, kp = wid >> 2;
+  const int ctx = A.ctx_len[s], ql = A.q_len[s], nq = min(X_COLS, ql - it.y * X_COLS);
+  const int pos0 = ctx - ql + it.y * X_COLS;
+  const size_t row0 = (size_t)A.q_start[s] + it.y * X_COLS;
+  int s_lo, s_hi;
+  unit_stages(pos0, nq, A.window, s_lo, s_hi);
+  if (nparts > 1) {  // this part's stages (possibly none)
+    const int per = (s_hi - s_lo + nparts - 1) / nparts;
+    s_lo += part * per;
+    s_hi = min(s_hi, s_lo + per);
+  }
+  const int n_st = s_hi - s_lo, last_blk = ((ctx + 15) >> 4) - 1, base = A.X.base[s];
+  // this wave's columns see some / all of the keys in [some_lo, some_hi] / [all_lo, all_hi]
+  const int wf = pos0 + min(cg * 32, nq - 1), we = pos0 + min(cg * 32 + 31, nq - 1);
+  const int some_lo = A.window > 0 ? wf - A.window + 1 : 0, all_lo = A.window > 0 ? we - A.window + 1 : 0;
+
+  f32x4 o[2][NV];
+  float m_run[2], l_run[2];
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+#pragma unroll
+    for (int n = 0; n < NV; ++n) o[x][n] = f32x4{0.f, 0.f, 0.f, 0.f};
+    m_run[x] = NEG_BIG;
+    l_run[x] = 0.f;
+  }
+  static_assert(2 * X_DIM * 32 == NW * 1024 && X_ROT * 32 * 4 == NW * 1024, "a stage is five loads a wave, which the waits below count");
+  const char* kx = (const char*)A.X.kx + (size_t)h * (X_DIM * 64) + wid * 1024 + lane * 16;
+  const char* kr = (const char*)A.X.kr + (wid & 1) * 1024 + lane * 16;
+  auto issue = [&](int st, char* dst) {
+    auto blk = [&](int b) { return (size_t)(base + min(4 * st + b, last_blk)); };
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+      __builtin_amdgcn_global_load_lds((glb_void*)(kx + blk(b) * A.H * (X_DIM * 64)), (lds_void*)(dst + b * X_BLOCK + wid * 1024), 16, 0, 0);
+    __builtin_amdgcn_global_load_lds((glb_void*)(kr + blk(wid >> 1) * (X_ROT * 32)),
+                                     (lds_void*)(dst + (wid >> 1) * X_BLOCK + 2 * X_DIM * 32 + (wid & 1) * 1024), 16, 0, 0);
+  };
+  auto buffer = [&](int i) { return smem + (i & 3) * X_STAGE; };
+  // (the first stages are under way while the queries arrive and turn)
+  if (n_st > 0) issue(s_lo, buffer(0));
+  if (n_st > 1) issue(s_lo + 1, buffer(1));
+  int cpos[2], klo[2];
+  bf16x8 qf[2][NQ];
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    const int col = min(cg * 32 + x * 16 + c, nq - 1);
+    cpos[x] = pos0 + col;
+    klo[x] = A.window > 0 ? max(0, cpos[x] - A.window + 1) : 0;
+    const bf16* src = (const bf16*)A.X.q + (row0 + col) * A.X.ldq + h * (X_DIM + X_ROT) + 8 * g;
+#pragma unroll
+    for (int m = 0; m < NQ; ++m) qf[x][m] = *reinterpret_cast<const bf16x8*>(src + 32 * m);
+    // the rotated part: the two halves turn together
+    const float* cs = A.X.cos_sin + (size_t)cpos[x] * X_ROT + 8 * g;
+    float co[8], si[8];
+    __builtin_memcpy(co, cs, 32);
+    __builtin_memcpy(si, cs + X_ROT / 2, 32);
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const float u = (float)qf[x][NQ - 2][k], v = (float)qf[x][NQ - 1][k];
+      qf[x][NQ - 2][k] = (bf16)(u * co[k] - v * si[k]);
+      qf[x][NQ - 1][k] = (bf16)(v * co[k] + u * si[k]);
+    }
+  }
+  const int loff = (g * 16 + c) * 16;
+  const int toff = ((c & 3) >> 1) * 256 + (4 * g + (c >> 2)) * 16 + (c & 1) * 8;
+  // Fragments are read AHEAD steps before their use: left to itself the compiler waits for each.
+  constexpr int AHEAD = 4;
+  f32x4 sc[2][2];
+  bf16x8 pf[2];
+  auto scores = [&](const char* tile) {
+    bf16x8 kb[AHEAD];
+    auto frag = [&](int i) {
+      const int k = i & 1, m = i >> 1;
+      return *reinterpret_cast<const bf16x8*>(tile + k * X_BLOCK + (m < X_DIM / 32 ? m * 1024 : 2 * X_DIM * 32 + (m - X_DIM / 32) * 1024) + loff);
+    };
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) kb[i] = frag(i);
+#pragma unroll
+    for (int i = 0; i < 2 * NQ; ++i) {
+      const int k = i & 1, m = i >> 1;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        if (m == 0) sc[x][k] = f32x4{0.f, 0.f, 0.f, 0.f};
+        sc[x][k] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kb[i % AHEAD], qf[x][m], sc[x][k], 0, 0, 0);
+      }
+      if (i + AHEAD < 2 * NQ) kb[i % AHEAD] = frag(i + AHEAD);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  // the largest of a column's values, which its four lanes hold: rows of 16 lanes, then halves, change places
+  auto column_max = [](float v) {
+    auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+    r = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(r[0]), __uint_as_float(r[1]));
+  };
+  auto softmax = [&](int key0) {
+    if (key0 < all_lo || key0 + 31 > wf) {  // wave-uniform
+#pragma unroll
+      for (int x = 0; x < 2; ++x)
+#pragma unroll
+        for (int k = 0; k < 2; ++k)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int key = key0 + 16 * k + 4 * g + r;
+            if (key > cpos[x] || key < klo[x]) sc[x][k][r] = NEG_BIG;
+          }
+    }
+    float m_new[2];
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      float tmax = NEG_BIG;
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) tmax = fmaxf(tmax, sc[x][k][r]);
+      m_new[x] = fmaxf(m_run[x], fmaxf(column_max(tmax) * A.scale_log2, NEG_BIG));
+    }
+    if (__any(m_new[0] > m_run[0] || m_new[1] > m_run[1])) {
+#pragma unroll
+      for (int x = 0; x < 2; ++x) {
+        const float alpha = __builtin_amdgcn_exp2f(m_run[x] - m_new[x]);
+        l_run[x] *= alpha;
+#pragma unroll
+        for (int n = 0; n < NV; ++n) o[x][n] *= alpha;
+        m_run[x] = m_new[x];
+      }
+    }
+#pragma unroll
+    for (int x = 0; x < 2; ++x) {
+      // a column that has seen no key yet: every weight is 0
+      const float nm = m_run[x] < 0.01f * NEG_BIG ? 0.f : -m_run[x];
+#pragma unroll
+      for (int k = 0; k < 2; ++k)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const float p = __builtin_amdgcn_exp2f(fmaf(sc[x][k][r], A.scale_log2, nm));
+          l_run[x] += p;
+          pf[x][4 * k + r] = (bf16)p;
+        }
+    }
+  };
+  auto outputs = [&](const char* tile) {
+    bf16x4 v0[AHEAD], v1[AHEAD];
+    auto read = [&](int n) {
+      v0[n % AHEAD] = tr_read_ahead(tile + X_DIM * 32 + n * 512 + toff);
+      v1[n % AHEAD] = tr_read_ahead(tile + X_BLOCK + X_DIM * 32 + n * 512 + toff);
+    };
+#pragma unroll
+    for (int n = 0; n < AHEAD; ++n) read(n);
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {
+      __builtin_amdgcn_sched_barrier(0);
+      bf16x8 v;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        v[j] = v0[n % AHEAD][j];
+        v[4 + j] = v1[n % AHEAD][j];
+      }
+#pragma unroll
+      for (int x = 0; x < 2; ++x) o[x][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pf[x], o[x][n], 0, 0, 0);
+      if (n + AHEAD < NV) read(n + AHEAD);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+  };
+  int late = -1;  // the stage whose outputs the second waves have yet to add
+  for (int i = 0; i < n_st; ++i) {
+    asm volatile("" ::: "memory");
+    if (i + 1 < n_st) __builtin_amdgcn_s_waitcnt(0x0075);  // vmcnt(5) lgkmcnt(0): the next stage's loads stay in flight
+    else __builtin_amdgcn_s_waitcnt(0x0070);
+    __builtin_amdgcn_s_barrier();  // stage i is whole, and nobody reads stage i - 2 any more
+    asm volatile("" ::: "memory");
+    if (i + 2 < n_st) issue(s_lo + i + 2, buffer(i + 2));
+    if (late >= 0) outputs(buffer(late) + 2 * X_BLOCK);
+    late = -1;
+    const char* tile = buffer(i) + kp * (2 * X_BLOCK);
+    const int key0 = 64 * (s_lo + i) + 32 * kp;
+    if (key0 > we || key0 + 31 < some_lo) continue;  // wave-uniform: no column sees the tile
+    scores(tile);
+    softmax(key0);
+    if (kp) late = i;
+    else outputs(tile);
+  }
+  if (late >= 0) outputs(buffer(late) + 2 * X_BLOCK);
+  // each of a column group's two waves sends the partner 16 columns and completes the other 16
+#pragma unroll
+  for (int x = 0; x < 2; ++x) {
+    l_run[x] += __shfl_xor(l_run[x], 16, 64);
+    l_run[x] += __shfl_xor(l_run[x], 32, 64);
+  }
+  f32x4* send = reinterpret_cast<f32x4*>(smem) + wid * (NV * 64);
+  float2* send_ml = reinterpret_cast<float2*>(smem + NW * NV * 1024) + wid * 16;
+  __syncthreads();  // (also the waits for every load to LDS)
+#pragma unroll
+  for (int n = 0; n < NV; ++n) send[n * 64 + lane] = kp ? o[0][n] : o[1][n];
+  if (g == 0) send_ml[c] = kp ? float2{m_run[0], l_run[0]} : float2{m_run[1], l_run[1]};
+  __syncthreads();
+  const f32x4* got = reinterpret_cast<const f32x4*>(smem) + (wid ^ 4) * (NV * 64);
+  const float2 ml = (reinterpret_cast<const float2*>(smem + NW * NV * 1024) + (wid ^ 4) * 16)[c];
+  const float m_own = kp ? m_run[1] : m_run[0], l_own = kp ? l_run[1] : l_run[0];
+  const float m = fmaxf(m_own, ml.x), f0 = exp2f(m_own - m), f1 = exp2f(ml.x - m), L = f0 * l_own + f1 * ml.y;
+  const int col = cg * 32 + kp * 16 + c;
+  if (col >= nq) return;
+  const size_t pc = ((size_t)(it.w + part) * A.H + h) * X_COLS + col;
+  if (nparts > 1 && g == 0) reinterpret_cast<float2*>(A.X.part_ml)[pc] = float2{m, L};
+  const float inv = 1.f / L;
+  bf16* out = (bf16*)A.X.out + (row0 + col) * A.X.ldo + h * X_DIM + 4 * g;
+#pragma unroll
+  for (int n = 0; n < NV; ++n) {
+    const f32x4 mine = kp ? o[1][n] : o[0][n];
+    const f32x4 v = mine * f0 + got[n * 64 + lane] * f1;
+    if (nparts > 1) {
+      *reinterpret_cast<f32x4*>(A.X.part_o + pc * X_DIM + 16 * n + 4 * g) = v;
+      continue;
+    }
+    bf16x4 b;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) b[r] = (bf16)(v[r] * inv);
+    *reinterpret_cast<bf16x4*>(out + 16 * n) = b;
+  }
+}
+
+// Which requests of a step are expanded, where their keys go, and the launches' work lists (one workgroup): those of at least
+// X_MIN new tokens, however many are cached. A step of 8 layers, us, absorbed and expanded: 1 prompt of 20 new tokens after
+// 500 2,098, 1,898; of 28 after 3,000 2,172, 2,177, of 70 2,313, 2,295; 4 of 20 after 500 2,336, 2,249; of 500 after 300 4,355, 4,221; 8
+// of 400 5,832, 5,628; one of 2,500 6,037, 5,228. Fewer tokens fill too little of a unit's 128 columns. Requests beyond X_REQS
+// or the workspace's `room` blocks keep the absorbed form. Tiles whose keys are more than a workgroup's average are split.
+constexpr int X_MIN = 12;
+__global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const int* __restrict__ q_start,
+                                                           const int* __restrict__ q_len, const int* __restrict__ ctx_len, int S,
+                                                           int T, int H, int window, int room, int max_att, int max_tiles, int slots) {
+  __shared__ int ws[16], req[X_REQS], qs[X_REQS], ql[X_REQS], cl[X_REQS], to[X_REQS], tiles[X_REQS], n_req, n_tiles;
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  for (int t = threadIdx.x; t < T; t += 1024) X.form[t] = 0;
+  int found = 0;
+  for (int s0 = 0; s0 < S; s0 += 1024) {
+    const int s = s0 + threadIdx.x, n = s < S ? q_len[s] : 0;
+    const bool yes = n >= X_MIN && s < S && q_start[s] + n <= T;
+    if (s < S) X.base[s] = X_NONE;
+    const unsigned long long b = __ballot(yes);
+    if (lane == 0) ws[wid] = __popcll(b);
+    __syncthreads();
+    int at = found + (int)__popcll(b & ((1ull << lane) - 1));
+    for (int w = 0; w < 16; ++w) {
+      if (w < wid) at += ws[w];
+      found += ws[w];
+    }
+    if (yes && at < X_REQS) {
+      req[at] = s;
+      qs[at] = q_start[s];
+      ql[at] = n;
+      cl[at] = ctx_len[s];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) {
+    const int n = min(found, X_REQS);
+    int used = 0, nt = 0, total = 0;
+    for (int i = 0; i < n; ++i) {
+      const int p0 = cl[i] - ql[i];
+      int lo, hi;
+      unit_stages(p0, ql[i], window, lo, hi);
+      const int blocks = ((cl[i] + 15) >> 4) - 4 * lo, t = (blocks + 3) >> 2;
+      to[i] = X_NONE;
+      if (used + blocks > room || nt + t > max_tiles) continue;
+      to[i] = used - 4 * lo;
+      tiles[i] = nt;
+      used += blocks;
+      nt += t;
+      for (int q = 0; q < ql[i]; q += X_COLS) {
+        unit_stages(p0 + q, min(X_COLS, ql[i] - q), window, lo, hi);
+        total += hi - lo;
+      }
+    }
+    const int fair = max(8, (total * H + 255) / 256);
+    int na = 0, slot = 0;
+    for (int i = 0; i < n; ++i) {
+      if (to[i] == X_NONE) continue;
+      for (int q = 0; q < ql[i]; q += X_COLS) {
+        int lo, hi;
+        unit_stages(cl[i] - ql[i] + q, min(X_COLS, ql[i] - q), window, lo, hi);
+        int parts = min(8, (hi - lo + fair - 1) / fair);
+        if (slot + parts > slots) parts = 1;
+        for (int p = 0; p < parts && na < max_att; ++p) X.att[na++] = int4{req[i], q / X_COLS, p | parts << 16, slot};
+        if (parts > 1) slot += parts;
+      }
+    }
+    X.counts[0] = na;
+    X.counts[1] = nt;
+    n_req = n;
+  }
+  __syncthreads();
+  for (int i = 0; i < n_req; ++i) {
+    if (to[i] == X_NONE) continue;
+    int lo, hi;
+    unit_stages(cl[i] - ql[i], ql[i], window, lo, hi);
+    const int nb = (cl[i] + 15) >> 4;
+    if (threadIdx.x == 0) X.base[req[i]] = to[i];
+    for (int j = threadIdx.x; 4 * (lo + j) < nb; j += 1024)
+      X.tiles[tiles[i] + j] = int4{req[i], 4 * (lo + j), min(4, nb - 4 * (lo + j)), to[i] + 4 * (lo + j)};
+    for (int t = threadIdx.x; t < ql[i]; t += 1024) X.form[qs[i] + t] = 1;
+  }
+}
+
+// Keys and values of the heads: 64 keys' latents in LDS, as the pages hold them, times W_uk,h and W_uv,h, the 256 outputs of a
+// head a round; a wave 64 of them. The outputs' lanes hold 4 dims of a key: 512 bytes of the workspace a store. A
+// head pair's weights (512 KB) stay on one XCD. Bound by the weights' way from L2, a step of 64 x 64 outputs 4 KB a wave: 4,096
+// keys of 16 heads 25 us (17 GFLOP, 34 MB written), with the next step's weights alone in flight and keys held over heads 90.
+__global__ __launch_bounds__(256, 2) void expand_kernel(const Expand X, const bf16* __restrict__ pages, const bf16* __restrict__ wk,
+                                                        const bf16* __restrict__ wv, const int* __restrict__ block_table, int max_blocks, int H, int D, int per) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // [4][X_RANK / 32][1 KB]
+  constexpr int KS = X_RANK / 32, NT = 4, RING = 4;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
+  const int groups = H / per, n = X.counts[1] * groups;
+  for (int u = blockIdx.x; u < n; u += gridDim.x) {
+    const int4 tl = X.tiles[u / groups];
+    const int h0 = u % groups * per;
+    const int* bt = block_table + (size_t)tl.x * max_blocks + tl.y;
+    __syncthreads();  // (the last unit's reads)
+    int ids[4];
+#pragma unroll
+    for (int b = 0; b < 4; ++b) ids[b] = bt[min(b, tl.z - 1)];
+#pragma unroll
+    for (int b = 0; b < 4; ++b)
+#pragma unroll
+      for (int i = 0; i < KS / 4; ++i) {
+        const int m = i * 4 + wid;
+        __builtin_amdgcn_global_load_lds((glb_void*)(pages + (size_t)ids[b] * (D * 16) + m * 512 + lane * 8),
+                                         (lds_void*)(smem + (b * KS + m) * 1024), 16, 0, 0);
+      }
+    if (h0 == 0 && wid < tl.z) {  // the rotated part, a block a wave
+      const bf16x8* src = reinterpret_cast<const bf16x8*>(pages + (size_t)bt[wid] * (D * 16) + X_RANK * 16) + lane;
+      bf16x8* dst = reinterpret_cast<bf16x8*>((bf16*)X.kr + (size_t)(tl.w + wid) * (X_ROT * 16)) + lane;
+      dst[0] = src[0];
+      dst[64] = src[64];
+    }
+    // the weights of all `per` heads are one stream, loaded RING steps ahead
+    const bf16* wp = (wid < 2 ? wk : wv) + ((size_t)h0 * 8 + (wid & 1) * NT) * (KS * 512) + lane * 8;
+    bf16x8 a[RING][NT];
+    auto load = [&](int q, bf16x8 (&a)[NT]) {  // (past the end: the last step's again)
+      q = min(q, per * KS - 1);
+      const bf16* from = wp + ((size_t)(q / KS) * 8 * KS + q % KS) * 512;
+#pragma unroll
+      for (int i = 0; i < NT; ++i) a[i] = *reinterpret_cast<const bf16x8*>(from + i * (KS * 512));
+    };
+#pragma unroll
+    for (int d = 0; d < RING; ++d) load(d, a[d]);
+    __syncthreads();  // (waits for the loads to LDS)
+    for (int j = 0; j < per; ++j) {
+      f32x4 acc[4][NT];
+#pragma unroll
+      for (int b = 0; b < 4; ++b)
+#pragma unroll
+        for (int i = 0; i < NT; ++i) acc[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll 1
+      for (int s = 0; s < KS; s += RING)
+#pragma unroll
+        for (int d = 0; d < RING; ++d) {
+          bf16x8 k[4];
+#pragma unroll
+          for (int b = 0; b < 4; ++b) k[b] = *reinterpret_cast<const bf16x8*>(smem + (b * KS + s + d) * 1024 + lane * 16);
+#pragma unroll
+          for (int b = 0; b < 4; ++b)
+#pragma unroll
+            for (int i = 0; i < NT; ++i) acc[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][i], k[b], acc[b][i], 0, 0, 0);
+          __builtin_amdgcn_sched_barrier(0);
+          load(j * KS + s + d + RING, a[d]);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+      for (int b = 0; b < 4; ++b) {
+        if (b >= tl.z) break;
+        bf16* dst = (bf16*)X.kx + ((size_t)(tl.w + b) * H + h0 + j) * (X_DIM * 32) + (2 * NT * wid + (g >> 1)) * 128 + c * 8 + (g & 1) * 4;
+#pragma unroll
+        for (int i = 0; i < NT; ++i) {
+          bf16x4 v;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) v[r] = (bf16)acc[b][i][r];
+          *reinterpret_cast<bf16x4*>(dst + i * 256) = v;
+        }
+      }
+    }
+  }
+}
+
 // Latents of 32 PAIRS and more: pair_item, on 256 workgroups. us of 16 heads, tile_item and as many workgroups as items
 // against pair_item: 512 + 64, 4 x 1,024 tokens 137, 114, 512 after 3,584 129, 108, 40 decode rows and 9 x 210 after 320
 // 77, 74; 384 + 64: 90, 91; 87, 89; 55, 61; 256 + 32: 77, 73; 76, 74; 47, 50.
 constexpr int PAIRS = 16;
 
-template <int RT, int PT>
+template <int RT, int PT, bool XP = false>
 constexpr int lds_bytes() {
-  return std::max({RT >= PAIRS ? pair_lds_bytes<RT, PT>() : 2 * 32 * 32 * (RT + PT) * 2, NW * 32 * 32 * RT + 1024 * (RT + PT),
+  return std::max({XP ? 4 * X_STAGE : 0, RT >= PAIRS ? pair_lds_bytes<RT, PT>() : 2 * 32 * 32 * (RT + PT) * 2, NW * 32 * 32 * RT + 1024 * (RT + PT),
                    NW * 16 * MERGE_LD * 4 + 2 * NW * 16 * 4});
 }
 
-template <int RT, int PT, int CT>
+template <int RT, int PT, int CT, bool XP = false>
 __global__ __launch_bounds__(64 * NW, 2) void mfma_kernel(const Args A) {
   extern __shared__ __attribute__((aligned(16))) char smem[];
   const int n = A.n_items[0];
   // Two passes over the workgroup's items, so that neither path's registers carry the other's.
+  int y0 = blockIdx.y;  // this workgroup's place in the rounds of items
+  if constexpr (XP) {  // as below, in rounds of all heads, so that an XCD's workgroups keep their heads
+    const int G = gridDim.x * gridDim.y, b = blockIdx.y * gridDim.x + blockIdx.x, per = G / A.H, na = A.X.counts[0];
+    if (b < per * A.H)
+      for (int r = 0; r * per < na; ++r) {
+        const int item = r * per + (r & 1 ? per - 1 - b / A.H : b / A.H);
+        if (item >= na) continue;
+        expanded_unit(A, A.X.att[item], b % A.H, smem);
+        __syncthreads();
+      }
+    // the other items begin with the workgroups that had no unit
+    y0 = (y0 + gridDim.y - min(na * A.H, G - 1) / gridDim.x) % gridDim.y;
+  }
   if constexpr (RT >= PAIRS) {
     // Tiles are dealt in rounds over the workgroups, every second one from its end: a prompt's later items have more keys,
     // and with one workgroup a CU each gets as many keys in all (4,096 tokens, as many workgroups as items: 341 us, here
     // 318).
-    for (int r = 0, b = blockIdx.y; r * (int)gridDim.y < n; ++r, b = gridDim.y - 1 - b) {
+    for (int r = 0, b = y0; r * (int)gridDim.y < n; ++r, b = gridDim.y - 1 - b) {
       const int item = r * gridDim.y + b;
       if (item >= n) continue;
       const int4 it = A.items[item];
-      if ((it.z & 0xff) <= A.dec_tokens) continue;
+      if ((it.z & 0xff) <= A.dec_tokens || expanded<XP>(A, it.x)) continue;
       pair_item<RT, PT>(A, it, smem);
       __syncthreads();
     }
   } else {
     for (int item = blockIdx.y; item < n; item += gridDim.y) {
       const int4 it = A.items[item];
-      if ((it.z & 0xff) <= A.dec_tokens) continue;
+      if ((it.z & 0xff) <= A.dec_tokens || expanded<XP>(A, it.x)) continue;
       tile_item<RT, PT, CT>(A, it, smem);
       __syncthreads();
     }
   }
-  for (int item = blockIdx.y; item < n; item += gridDim.y) {
+  for (int item = y0; item < n; item += gridDim.y) {
     const int4 it = A.items[item];
-    if ((it.z & 0xff) > A.dec_tokens) continue;
+    if ((it.z & 0xff) > A.dec_tokens || expanded<XP>(A, it.x)) continue;
     split_item<RT, PT>(A, it, smem);
     __syncthreads();
   }
@@ -818,31 +1272,35 @@ extern "C" int pa_latent_pad(int R) {
 extern "C" int pa_latent_attention(int fp32, void* out, float* part_o, float* part_ml, const void* q, const void* pages, const int* items, const int* n_items, int max_items,
                                    const int* q_start, const int* q_len, const int* ctx_len, const int* block_table,
                                    int max_blocks, int H, int Rp, int rp, int dec_tokens, int tile_tokens, int window,
-                                   float scale_log2, int simple, hipStream_t st) {
+                                   float scale_log2, int simple, const pa::la::Expand* expand, hipStream_t st) {
   if (max_items <= 0) return 0;
   const int D = Rp + rp, NB = (dec_tokens * H + 15) / 16;
   if (Rp % 32 || rp % 32 || H <= 0 || dec_tokens <= 0 || tile_tokens <= 0) return -1;
   pa::la::Args A{out, part_o, part_ml, q, pages, (const int4*)items, n_items, q_start, q_len, ctx_len,
-                 block_table, max_blocks, H, NB, Rp, D, dec_tokens, window, scale_log2};
+                 block_table, max_blocks, H, NB, Rp, D, dec_tokens, window, scale_log2, expand ? *expand : pa::la::Expand{}};
+  if (expand && (fp32 || simple || Rp != pa::la::X_RANK || rp != pa::la::X_ROT || H > 256)) return -1;
   const int RT = Rp / 32, PT = rp / 32;
   if (!fp32 && !simple && PT <= 2) {
-#define PA_LA(R, P)                                                                                           \
+#define PA_LAX(R, P, ...)                                                                                     \
   do {                                                                                                        \
     constexpr int CT = 1;                                                                                     \
-    constexpr int lds = pa::la::lds_bytes<R, P>();                                                            \
+    constexpr int lds = pa::la::lds_bytes<R, P __VA_ARGS__>();                                                \
     static bool attr = false;                                                                                 \
     if (!attr) {                                                                                              \
-      (void)hipFuncSetAttribute((const void*)pa::la::mfma_kernel<R, P, CT>,                                   \
+      (void)hipFuncSetAttribute((const void*)pa::la::mfma_kernel<R, P, CT __VA_ARGS__>,                       \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, lds);                             \
       attr = true;                                                                                            \
     }                                                                                                         \
     const int cw = 16 * pa::la::NW * CT, gt = (tile_tokens * H + cw - 1) / cw, gx = NB > gt ? NB : gt;                       \
     /* items are strided over the grid: at least one workgroup per CU */                                      \
     const int gy = R >= pa::la::PAIRS || max_items < 256 ? 256 : (max_items < 4096 ? max_items : 4096);       \
-    hipLaunchKernelGGL((pa::la::mfma_kernel<R, P, CT>), dim3(gx, gy), dim3(64 * pa::la::NW), lds, st, A);     \
-    hipLaunchKernelGGL((pa::la::merge_kernel<R>), dim3(16, std::min(gy, 256)), dim3(256), 0, st, A);           \
+    hipLaunchKernelGGL((pa::la::mfma_kernel<R, P, CT __VA_ARGS__>), dim3(gx, gy), dim3(64 * pa::la::NW), lds, st, A);     \
+    hipLaunchKernelGGL((pa::la::merge_kernel<R __VA_ARGS__>), dim3(16, std::min(gy, 256)), dim3(256), 0, st, A);           \
     return (int)hipGetLastError();                                                                            \
   } while (0)
+#define PA_LA(R, P) PA_LAX(R, P, )
+#define PA_COMMA ,
+    if (expand) PA_LAX(pa::la::X_RANK / 32, pa::la::X_ROT / 32, PA_COMMA true);
     switch (RT) {
 #define PA_X(N) case N: if (PT == 0) PA_LA(N, 0); else if (PT == 1) PA_LA(N, 1); else PA_LA(N, 2); break;
       PA_LA_RT(PA_X)
@@ -850,6 +1308,8 @@ extern "C" int pa_latent_attention(int fp32, void* out, float* part_o, float* pa
       default: break;
     }
 #undef PA_LA
+#undef PA_LAX
+#undef PA_COMMA
   }
   if (Rp > 2048 || D * 4 + 2048 > 64 * 1024) return -2;
   const dim3 grid(H, max_items < 4096 ? max_items : 4096);
@@ -859,3 +1319,29 @@ extern "C" int pa_latent_attention(int fp32, void* out, float* part_o, float* pa
   return (int)hipGetLastError();
 }
 
+
+// The plan of a step for requests with expanded keys: see expand_plan_kernel. X's work lists hold max_att and max_tiles
+// entries, its workspace `room` blocks and `slots` partial results.
+extern "C" int pa_latent_plan(const pa::la::Expand* X, const int* q_start, const int* q_len, const int* ctx_len, int S, int T, int H,
+                              int window, int room, int max_att, int max_tiles, int slots, hipStream_t st) {
+  hipLaunchKernelGGL(pa::la::expand_plan_kernel, dim3(1), dim3(1024), 0, st, *X, q_start, q_len, ctx_len, S, T, H, window, room,
+                     max_att, max_tiles, slots);
+  return (int)hipGetLastError();
+}
+
+// wk, wv: [H, 8, 16, 64, 8], the heads' rows of W_uk and of W_uv
+extern "C" int pa_latent_expand(const pa::la::Expand* X, const void* pages, const void* wk, const void* wv, const int* block_table, int max_blocks,
+                                int H, int D, int max_tiles, hipStream_t st) {
+  if (H <= 0 || D != pa::la::X_RANK + pa::la::X_ROT) return -1;
+  constexpr int lds = 4 * pa::la::X_RANK * 32;
+  static bool attr = false;
+  if (!attr) {
+    (void)hipFuncSetAttribute((const void*)pa::la::expand_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    attr = true;
+  }
+  const int per = H % 2 ? 1 : 2, groups = H / per, n = max_tiles * groups;  // two workgroups a CU
+  const int grid = groups <= 512 ? std::min(n, 512 / groups * groups) : n;
+  hipLaunchKernelGGL(pa::la::expand_kernel, dim3(grid), dim3(256), lds, st, *X, (const pa::bf16*)pages, (const pa::bf16*)wk,
+                     (const pa::bf16*)wv, block_table, max_blocks, H, D, per);
+  return (int)hipGetLastError();
+}

@@ -14,10 +14,12 @@ are the model's dtype (bf16, or fp32 throughout).
 One step of T tokens (decode rows and prompt portions alike):
 
   once      table_route       every expert layer's rows sorted by expert, from the token ids
+            (latent_plan      steps of prompts: the requests whose keys are expanded per head)
             residual_norm     x = E[id], norm -> h
   per run   linear            [query latent | kv latent | rotated key] = W_down h, one projection
             latent_cache      both latent norms, key rotation, paged cache row
             linear            q = W_uq c_q
+            (latent_expand    keys and values of those requests' heads, from their pages)
             head_gemm         q~ = [W_uk^T q | rotated part of q] per head
             latent_attention  windowed paged attention in the latent space
             head_gemm, linear W_uv per head, W_o
@@ -40,7 +42,7 @@ from pilottai_amd.models.cache import LatentKVCache, StepMeta
 from pilottai_amd.models.common import PackedLinear, checkpoint_reader, expert_tile_rows, layer_runs, parse_loop
 from pilottai_amd.models.hybrid import AttentionRoom, MixerBlock
 from pilottai_amd.models.latent import LatentAttention, LatentAttentionSpec
-from pilottai_amd.ops.latent import pad_to
+from pilottai_amd.ops.latent import ExpandPlan, expand_pays, pad_to
 from pilottai_amd.parallel.comm import TPGroup
 
 GLU_ALPHA = 1.702  # the gated unit g * sigmoid(alpha g) * (u + bias)
@@ -332,6 +334,9 @@ class BozupelModel:
         rows = meta.logit_rows[:num_logit_rows]
         routes = self._route(meta, T)
         room = AttentionRoom(part_o, part_ml, self.dec_tokens, self.tile_tokens, 0)
+        if expand_pays(T, num_logit_rows):
+            keys = {L["attn"].expand_key() for L in self.layers} - {None}
+            room = room._replace(expand={k: ExpandPlan(meta, T, *k) for k in keys})
         resid = torch.empty(T, d, dtype=torch.float32, device=dev)
         h = ops.residual_norm(resid, eps, emb=self.embed, ids=ids, w_next=self.layers[self.runs[0][0]]["norm1"], out=new_h())
         for j, (i, _) in enumerate(self.runs):

@@ -272,12 +272,14 @@ class SideStreams:
 
 
 class AttentionRoom(NamedTuple):
-    """What the engine's attention work items need: partial results and the tokens of an item."""
+    """What the engine's attention work items need: partial results and the tokens of an item. `expand`: by window, the
+    step's plans of requests whose latents are expanded (ops/latent.py ExpandPlan)."""
     part_o: torch.Tensor
     part_ml: torch.Tensor
     dec_tokens: int
     tile_tokens: int
     max_slots: int
+    expand: Dict[tuple, object] = {}
 
 
 class PagedAttention:

@@ -18,7 +18,7 @@ import torch
 from pilottai_amd import ops
 from pilottai_amd.models.cache import StepMeta
 from pilottai_amd.models.common import PackedLinear, pad_heads
-from pilottai_amd.ops.latent import latent_pad, pad_to
+from pilottai_amd.ops.latent import EXPAND_SIZES, Expanded, latent_pad, pad_to
 
 
 @dataclass(frozen=True)
@@ -118,11 +118,20 @@ class LatentAttention:
         uv = torch.zeros(H, self.vp, self.Rp, dtype=dtype, device=device)
         uv[:, :vd, :R] = t["uv"].to(device).view(H, vd, R)
         self.uv = ops.pack_groups(uv, dtype)
+        self.k_rows = None  # W_uk by its rows, for the keys of a prompt's heads, where the sizes have that form
+        sizes = dict(dim=n, vdim=vd, rot=r, rank=R)
+        if sizes == EXPAND_SIZES and m.rot_dims == r and source is None and not m.gate and dtype == torch.bfloat16 and \
+                torch.device(device).type == "cuda":
+            self.k_rows = ops.pack_groups(t["uk"].to(device).view(H, n, R), dtype)
         self.width, self.out_bias = H * self.vp, None
         self.w_out = pad_heads(t["o"].T.reshape(H, vd, -1), self.vp).reshape(self.width, -1).T
 
     def tensors(self):
-        return ([self.uq.w] if self.uq else []) + [self.uk, self.uv]
+        return ([self.uq.w] if self.uq else []) + [self.uk, self.uv] + ([self.k_rows] if self.k_rows is not None else [])
+
+    def expand_key(self) -> Optional[tuple]:
+        """What a step's plan of expanded requests depends on; None: this layer has no such form."""
+        return (self.spec.heads, self.spec.window) if self.k_rows is not None else None
 
     def cache_kind(self) -> tuple:
         return ("latent", self.D) if self.spec.kv_from is None else ("same", self.spec.kv_from)
@@ -136,13 +145,18 @@ class LatentAttention:
             ops.latent_cache(x[:, self.c_col:], m.q_rank, m.kv_rank, m.rot_dim, self.w_q, self.w_c, cq, pages, self.Rp,
                              meta.positions, meta.slots, self.cos_sin, self.eps)
         q = self.uq(cq) if self.uq else x
+        plan, ex, skip = room.expand.get(self.expand_key()), None, None
+        if plan is not None:
+            ex = Expanded(plan, pages, self.k_rows, self.uv, meta.block_table, q, self.cos_sin, out)
+            skip = ex.form
         qa = new(T, H, self.D)
         if self.D > self.Rp + self.rp:  # (another layer's rows have a rotated part, which these queries leave out)
             qa.zero_()
         ops.head_gemm(q, self.np + self.rp, self.uk, qa.view(T, -1), self.D,
-                      rot=(meta.positions, self.cos_sin, self.np, m.rot_dim, self.rp) if m.rot_dim else None)
+                      rot=(meta.positions, self.cos_sin, self.np, m.rot_dim, self.rp) if m.rot_dim else None, skip=skip)
         oc = new(T, H, self.Rp)
         ops.latent_attention(oc, room.part_o, room.part_ml, qa, pages, meta.items, meta.n_items, meta.q_start,
                              meta.q_len, meta.ctx_len, meta.block_table, m.scale, m.window, room.dec_tokens, room.tile_tokens,
-                             num_seqs=meta.num_seqs)
-        ops.head_gemm(oc.view(T, -1), self.Rp, self.uv, out, self.vp, gate=x[:, self.g_col:] if m.gate else None)
+                             num_seqs=meta.num_seqs, expand=ex)
+        ops.head_gemm(oc.view(T, -1), self.Rp, self.uv, out, self.vp, gate=x[:, self.g_col:] if m.gate else None,
+                      skip=skip)

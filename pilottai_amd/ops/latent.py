@@ -62,18 +62,67 @@ def latent_cache(x, nq: int, R: int, r: int, w_q, w_c, cq, pages, Rp: int, posit
 
 def latent_attention(out, part_o, part_ml, q, pages, items, n_items, q_start, q_len, ctx_len, block_table,
                      scale: float, window: int, dec_tokens: int, tile_tokens: int, num_seqs: Optional[int] = None,
-                     simple: bool = False):
+                     simple: bool = False, expand: Optional["Expanded"] = None):
     """Attention of absorbed queries q [T, H, D] over latent pages -> out [T, H, Rp]; `window` 0: none.
     dec_tokens / tile_tokens: the scheduler's items hold at most dec_tokens tokens (split over keys) or
-    tile_tokens (csrc/ops/latent_attention.hip). `simple`: the any-size kernel."""
+    tile_tokens (csrc/ops/latent_attention.hip). `simple`: the any-size kernel. `expand`: requests of its plan are left out
+    here, and their outputs in the heads' own dimensions go to its `out`."""
     if _on_gpu(q):
         require_latent().latent_attention(out, part_o, part_ml, q, pages, items, n_items, q_start, q_len,
                                           ctx_len, block_table, int(dec_tokens), int(tile_tokens), int(window),
-                                          float(scale), bool(simple))
+                                          float(scale), bool(simple), expand.plan if expand else [],
+                                          expand.tensors() if expand else [])
     else:
         ref.latent_attention(out, q, pages, q_start, q_len, ctx_len, block_table, scale, window,
                              len(q_len) if num_seqs is None else num_seqs)
     return out
+
+
+# Prompt portions with the keys expanded per head (csrc/ops/latent_expand.h): sizes that have the form
+EXPAND_SIZES = dict(dim=128, vdim=128, rot=64, rank=512)
+EXPAND_COLS, EXPAND_REQS = 128, 64
+
+
+def expand_pays(T: int, seqs: int) -> bool:
+    """Whether a step of T rows and at most `seqs` requests has the plan and the launch a layer that the form takes: with few
+    rows, or many decode rows beside short prompts, they cost more than the prompts gain. A step of 8 layers, us, without and
+    with: one prompt of 20 tokens 1,799, 1,820, of 33 with 200 cached, twice, 2,200, 2,123; 30 decode rows and 4 prompts of 60
+    2,573, 2,638, of 400 4,011, 3,824."""
+    return T >= max(48, 20 * seqs) or T >= max(256, 10 * seqs)
+
+
+class ExpandPlan:
+    """Which requests of a step of T rows have their keys expanded, decided on the device: [counts, base, form, attention
+    items, expansion tiles], and the room for it. `form` [T] is 1 for their rows."""
+
+    def __init__(self, meta, T: int, heads: int, window: int):
+        dev, S = meta.q_len.device, meta.q_len.numel()
+        # as many keys as rows, and the cached ones of a long context
+        self.blocks = (T + max(T, 4096)) // 16
+        self.slots = max(8, 768 // heads)
+        new = lambda *s: torch.empty(*s, dtype=torch.int32, device=dev)  # noqa: E731
+        self.form = new(T)
+        self.lists = [new(2), new(S), self.form, new(T // EXPAND_COLS + EXPAND_REQS + self.slots, 4),
+                      new(self.blocks // 4 + EXPAND_REQS, 4)]
+        require_latent().latent_plan(self.lists, meta.q_start, meta.q_len, meta.ctx_len, int(T), int(heads), int(window),
+                                     int(self.blocks), int(self.slots))
+
+
+class Expanded:
+    """Keys and values of the plan's requests, from their pages, with wk and wv = pack_groups([H, 128, 512]), the heads' rows of
+    W_uk and of W_uv; q [T, H (128 + 64)] and out [T, >= H 128] are what latent_attention reads and writes for them."""
+
+    def __init__(self, plan: ExpandPlan, pages, wk, wv, block_table, q, cos_sin, out):
+        H, dev = wk.shape[0], pages.device
+        new = lambda dt, *s: torch.empty(*s, dtype=dt, device=dev)  # noqa: E731
+        self.plan, self.form, self.q, self.cos_sin, self.out = plan.lists, plan.form, q, cos_sin, out
+        self.kx, self.kr = new(torch.bfloat16, plan.blocks, H, 32, 16, 8), new(torch.bfloat16, plan.blocks, 8, 16, 8)
+        self.part_o = new(torch.float32, plan.slots, H, EXPAND_COLS, 128)
+        self.part_ml = new(torch.float32, plan.slots, H, EXPAND_COLS, 2)
+        require_latent().latent_expand(self.plan, self.kx, self.kr, pages, wk, wv, block_table)
+
+    def tensors(self):
+        return [self.kx, self.kr, self.q, self.cos_sin, self.out, self.part_o, self.part_ml]
 
 
 # ---- grouped projections ----------------------------------------------------------------------
@@ -101,13 +150,15 @@ def interleave_gate_up(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     return torch.stack([gate.reshape(G, F // 16, 16, K), up.reshape(G, F // 16, 16, K)], 2).reshape(G, 2 * F, K)
 
 
-def head_gemm(x, x_step: int, w, out, out_step: int, rot: Optional[tuple] = None, gate: Optional[torch.Tensor] = None):
+def head_gemm(x, x_step: int, w, out, out_step: int, rot: Optional[tuple] = None, gate: Optional[torch.Tensor] = None,
+              skip: Optional[torch.Tensor] = None):
     """out[:, g * out_step : + N] = x[:, g * x_step : + K] @ w[g].T for every group g, times sigmoid(gate) (columns as
     out's) if given. rot = (positions, cos_sin, skip, r, rp): beside them, out[:, g * out_step + N : + rp] = x[:, g *
-    x_step + skip : + r] rotated by the row's position and padded with zeros."""
+    x_step + skip : + r] rotated by the row's position and padded with zeros. Rows whose entry of `skip` (int32 [T]) is not 0
+    stay as they are (on the GPU, bf16)."""
     if _on_gpu(x):
-        pos, cs, skip, r, rp = rot or (None, None, 0, 0, 0)
-        require_grouped().head_gemm(x, int(x_step), w, out, int(out_step), pos, cs, int(skip), int(r), int(rp), gate)
+        pos, cs, at, r, rp = rot or (None, None, 0, 0, 0)
+        require_grouped().head_gemm(x, int(x_step), w, out, int(out_step), pos, cs, int(at), int(r), int(rp), gate, skip)
     else:
         ref.head_gemm(x, x_step, unpack_groups(w), out, out_step, rot, gate)
     return out

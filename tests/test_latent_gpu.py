@@ -411,3 +411,66 @@ def test_latent_attention_window_edge(gpu, edge, reqs):
             last = int(m["q_start"][i]) + n - 1
             q[last] = (3.0 * pages[pg, :, off].reshape(1, -1).float()).to(q.dtype)
     run_attention(gpu, torch.bfloat16, 4, 128, 32, reqs, W, spike=spike)
+
+
+# (cached, new) of a step's requests at the edges of the expanded form: tiles of 128 tokens, stages of 64 keys, 12 new tokens
+# at least, keys split into parts (few tokens after many), none of them
+EXPANDED = {"one": [(0, 300)], "edges": [(0, 128), (0, 129), (8, 64), (0, 63), (63, 155), (63, 65), (500, 1)],
+            "parts": [(2100, 260), (700, 1), (0, 20)], "mixed": [(33, 1), (300, 300), (900, 20), (0, 700), (5, 1), (100, 64)],
+            "few": [(900, 12), (70, 11), (0, 13)], "none": [(900, 11), (300, 1)]}
+
+
+@pytest.mark.parametrize("window", [0, 45, 600])
+@pytest.mark.parametrize("step", list(EXPANDED))
+@pytest.mark.parametrize("H", [16, 5, 40])
+def test_latent_attention_expanded(gpu, H, step, window):
+    """Prompt portions whose keys are expanded per head, beside requests that keep the absorbed form: the step through both
+    of a layer's head projections. Keys, values and weights have 16 bits (2^-9 each, and the outputs'), as the absorbed
+    form's queries, rows and weights have."""
+    from types import SimpleNamespace
+
+    from pilottai_amd import ops
+    from pilottai_amd.ops.latent import Expanded, ExpandPlan
+
+    reqs = EXPANDED[step]
+    want = [i for i, (c, n) in enumerate(reqs) if n >= 12]
+    bf, R, n, r, V = torch.bfloat16, 512, 128, 64, 128
+    g = torch.Generator().manual_seed(H + window)
+    T, m, dec, tile = fed_meta(gpu, H, reqs, 384, window)
+    pages = torch.randn(600, (R + r) // 8, 16, 8, generator=g).to(bf)
+    uk, uv = ((torch.randn(H, k, R, generator=g) * R ** -0.5).to(bf) for k in (n, V))
+    q = torch.randn(T, H * (n + r), generator=g).to(bf)
+    cs, scale = ops.angle_table(4096, r, 1e4), (n + r) ** -0.5
+    d = lambda t: t.to(gpu)  # noqa: E731
+    mg, pos = {k: d(v) for k, v in m.items()}, torch.zeros(T, dtype=torch.int32)
+    for i, (c, k) in enumerate(reqs):
+        pos[int(m["q_start"][i]):][:k] = torch.arange(c, c + k)
+    out = torch.full((T, H * V), 9.0, dtype=bf, device=gpu)
+    plan = ExpandPlan(SimpleNamespace(**mg), T, H, window)
+    taken = [i for i in range(len(reqs)) if int(plan.lists[1][i]) > -(1 << 30)]
+    assert taken == want and int(plan.form.sum()) == sum(reqs[i][1] for i in taken)
+    qg, pg = d(q), d(pages)
+    ex = Expanded(plan, pg, ops.pack_groups(d(uk), bf), ops.pack_groups(d(uv), bf), mg["block_table"], qg, d(cs), out)
+    qa = torch.full((T, H, R + r), 7.0, dtype=bf, device=gpu)
+    ops.head_gemm(qg, n + r, ops.pack_groups(d(uk.transpose(1, 2).contiguous()), bf), qa.view(T, -1), R + r,
+                  rot=(d(pos), d(cs), n, r, r), skip=ex.form)
+    NB, mi = (dec * H + 15) // 16, m["items"].shape[0]
+    po, pm = torch.empty(mi * NB * 16 * R, device=gpu), torch.empty(mi * NB * 32, device=gpu)
+    oc = torch.zeros(T, H, R, dtype=bf, device=gpu)
+    ops.latent_attention(oc, po, pm, qa, pg, mg["items"], mg["n_items"], mg["q_start"], mg["q_len"], mg["ctx_len"],
+                         mg["block_table"], scale, window, dec, tile, expand=ex)
+    ops.head_gemm(oc.view(T, -1), R, ops.pack_groups(d(uv), bf), out, V, skip=ex.form)
+    o = out.float().cpu().view(T, H, V)
+    half = r // 2
+    turn = lambda x, at: torch.cat([x[..., :half] * cs[at, :half] - x[..., half:] * cs[at, half:],  # noqa: E731
+                                    x[..., half:] * cs[at, :half] + x[..., :half] * cs[at, half:]], -1)
+    for i, (c, k) in enumerate(reqs):
+        q0, ctx = int(m["q_start"][i]), c + k
+        rows = pages[m["block_table"][i, :(ctx + 15) // 16].long()].permute(0, 2, 1, 3).reshape(-1, R + r)[:ctx].float()
+        x = q[q0:q0 + k].float().view(k, H, n + r).transpose(0, 1)
+        keys = torch.matmul(rows[:, :R], uk.float().transpose(1, 2))  # [H, keys, n]
+        sc = torch.matmul(x[..., :n], keys.transpose(1, 2)) + torch.matmul(turn(x[..., n:], torch.arange(c, ctx)), rows[:, R:].T)
+        back = torch.arange(c, ctx)[:, None] - torch.arange(ctx)[None, :]
+        sc = (sc * scale).masked_fill(~((back >= 0) & ((back < window) if window else True)), -math.inf)
+        want = torch.matmul(torch.softmax(sc, -1), torch.matmul(rows[:, :R], uv.float().transpose(1, 2))).transpose(0, 1)
+        torch.testing.assert_close(o[q0:q0 + k], want, **tol(bf), msg=lambda s, i=i: f"request {i} {reqs[i]}: {s}")
