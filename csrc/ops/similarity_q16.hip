@@ -311,27 +311,32 @@ __global__ __launch_bounds__(512) void stage1_exact_kernel(
 // fragments of the 16x16x64 form (4 KiB per KiB of rows instead of 8) at the same MFMA cycles.
 // The A fragments come straight from the 16-row fragment-major planes: lane (r = l & 31,
 // h = l >> 5) of k-half kh of k-step s takes row tile 2G + r/16, lane position 16 (2 kh + h) +
-// r % 16 -- 16 B, in 256-B runs. The group streams in batches of 4 k-steps, double-buffered, the
-// next group's first batch issued before the epilogue. Everything that decides what stays in
+// r % 16 -- 16 B, in 256-B runs. The group streams in batches of 4 k-steps, double-buffered, both of
+// the next group's first batches in flight over the epilogue. Everything that decides what stays in
 // flight is static: the k-step count is a template constant (queries zero-padded to DSC*64
-// dims and 64 rows, loads past D clamped), the row loads are unconditional (clamped to the
-// slice's last tile), the load batches are pinned by sched_barrier, and the round barrier waits
-// for LDS only -- a branchy load block, a fenced __syncthreads or loads left to the scheduler
+// dims and whole tiles, loads past D clamped), the row loads are unconditional (clamped to the
+// slice's last tile), the load batches are pinned by sched_barrier, and waves go on by themselves, without a
+// barrier a round -- a branchy load block, a fenced __syncthreads, a load from scratch memory or loads left to the scheduler
 // each made the wait-count pass drain the row loads in flight (the first form: 3.2 TB/s).
-// Candidate stores are made visible by a full barrier only before a compaction.
-// A buffer holds LIM entries between rounds and 8 x 32 more that a round may admit. Compacting early (two lists' worth)
-// keeps the thresholds tight, and so the admissions few, now that a compaction costs a microsecond.
+// Bound by the row stream: 64 queries of 4M rows, 938 -> 731 us at 1,024 dimensions (4.4 -> 5.6 TB/s; 700 if no bound ever
+// reached its query's threshold), 64 of 131,000 rows 300 -> 87.
+// Candidate stores are made visible by a full barrier only before a compaction, which a wave asks for when it finds a
+// buffer at LIM or beyond. Until all have come, each of the others finishes at most the group it is in: LIM + 8 x 32 entries.
+// Compacting early (two lists' worth) keeps the thresholds tight, and so the admissions few, now that a compaction costs a
+// microsecond.
 constexpr int LIM = 2 * C;
-// Slices share what they know: after rounds 0, 7, 15, 31, .. each publishes the best L it has admitted per query, and a round
-// later reads the others'. The K-th best of those is the L of K different rows, so it bounds the answer as tauL does, from
-// the rows of all slices instead of one: of 4M rows, a slice then admits a row or two a query after the second round
-// instead of some 260, and the pass takes 0.94 instead of 1.47 ms (the row stream alone: 0.8).
+// Slices share what they know: after rounds 0, 7, 15, 31, .. each publishes the best L it has admitted per query. The K-th
+// best of those is the L of K different rows, so it bounds the answer as tauL does, from the rows of all slices instead of
+// one: of 4M rows, a slice then admits a row or two a query after the second round instead of some 260. In round 1 every
+// slice works it out for all queries; later one slice a query, for all to read a round after (for all in each: 18 us a time).
 __device__ __forceinline__ bool publishes(int round) { return round == 0 || (round >= 7 && ((round + 1) & round) == 0); }
 __global__ void clear_kernel(uint32_t* p, int n) {
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = 0;
 }
-// `pub` [Q][slices], cleared before the launch; null: slices of a round or two, which have no use for it.
-template <int DSC>
+// `pub` [Q][slices] and [Q], cleared before the launch; null: slices of one round, which have no use for it.
+// FULL: D is DSC * 64. NTQ: tiles of 32 queries, one of which takes half the products and LDS reads (8 queries of 4M rows, 1,024
+// dimensions: 746 us with two, 728).
+template <int DSC, bool FULL, int NTQ>
 __global__ __launch_bounds__(512) void stage1_bound_kernel(
     float* __restrict__ out_u, float* __restrict__ out_l, int* __restrict__ out_r, float* __restrict__ out_drop,
     float* __restrict__ cand_u, float* __restrict__ cand_l, int* __restrict__ cand_r,
@@ -339,14 +344,14 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
     const float* __restrict__ rmeta, int Q, int N, int D, int K, const int* __restrict__ row_prio,
     const uint64_t* __restrict__ row_tags, const float* __restrict__ row_exp, const int* __restrict__ q_minp,
     const uint64_t* __restrict__ q_tags, float now, uint32_t* pub) {
-  constexpr int TH = 512, NWV = TH / 64, KB = DSC >= 8 ? 4 : 2, NTQ = MAXQ / 32;
+  constexpr int TH = 512, NWV = TH / 64, KB = DSC >= 8 ? 4 : 2, ROWS = 32 * NTQ;
   constexpr int QLD = DSC * 64 + 16;  // padded LDS row (bytes)
   static_assert(DSC % (2 * KB) == 0, "k-steps in whole batch pairs");
   typedef int i32x16 __attribute__((ext_vector_type(16)));
   extern __shared__ __attribute__((aligned(16))) char smem[];
-  signed char* qh = reinterpret_cast<signed char*>(smem);  // [64][QLD]
-  signed char* ql = qh + (size_t)MAXQ * QLD;                // [64][QLD]
-  QState& st = *reinterpret_cast<QState*>(ql + (size_t)MAXQ * QLD);
+  signed char* qh = reinterpret_cast<signed char*>(smem);  // [ROWS][QLD]
+  signed char* ql = qh + (size_t)ROWS * QLD;                // [ROWS][QLD]
+  QState& st = *reinterpret_cast<QState*>(ql + (size_t)ROWS * QLD);
   // [2] some query's buffer must be compacted, by rounds in turn: a wave that is a round ahead must not be taken for this
   // one's (the others would miss its barrier)
   int* need = reinterpret_cast<int*>(&st + 1);
@@ -355,12 +360,14 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
   int* pr_lds = reinterpret_cast<int*>(rm_lds + NWV * 32);
   float* ex_lds = reinterpret_cast<float*>(pr_lds + NWV * 32);
   uint64_t* tg_lds = reinterpret_cast<uint64_t*>(ex_lds + NWV * 32);
+  uint32_t* first = reinterpret_cast<uint32_t*>(tg_lds + NWV * 32);  // [ROWS][65] the first round's lower bounds
 
   const int nwg = gridDim.x, wg = blockIdx.x;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane & 31, lh = lane >> 5;
-  const int DS = D / 64;
-  for (int v = threadIdx.x; v < MAXQ * 2 * (DSC * 4); v += TH) {
+  const int DS = FULL ? DSC : D / 64;
+  uint32_t* tau = pub + (size_t)Q * nwg;  // [Q] K-th best bounds over the slices
+  for (int v = threadIdx.x; v < ROWS * 2 * (DSC * 4); v += TH) {
     const int r = v / (2 * DSC * 4), rem = v % (2 * DSC * 4);
     const int plane = rem / (DSC * 4), c16 = (rem % (DSC * 4)) * 16;
     i32x4 x = i32x4{0, 0, 0, 0};
@@ -393,30 +400,72 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
     const int nrounds = (ngroups + NWV - 1) / NWV;
     const int last_tile = (r1 - 1) >> 4;
     static_assert(LIM + NWV * 32 <= CAND, "a buffer must absorb a round");
-    // this lane's two 16-B A pieces (k-halves) of k-step m + u, group grp_
+    // this lane's two 16-B A pieces (k-halves) of k-step m + u, group grp_: a base that the wave shares and 32 bits of the
+    // lane's own, so that no addresses are kept in registers
     auto load = [&](int grp_, int m, i32x4 (&dst)[KB][2]) {
-      const int tile = min((r0 >> 4) + 2 * min(grp_, ngroups - 1) + (lr >> 4), last_tile);
-      const signed char* base = hi + (size_t)tile * DS * 1024 + (size_t)(lr & 15) * 16;
+      const int tile = (r0 >> 4) + 2 * min(grp_, ngroups - 1);
+      const signed char* base = hi + (size_t)tile * DS * 1024;
+      const unsigned own = (tile < last_tile && lr > 15 ? DS * 1024 : 0) + (lr & 15) * 16 + lh * 256;
 #pragma unroll
       for (int u = 0; u < KB; ++u)
 #pragma unroll
         for (int kh = 0; kh < 2; ++kh)
-          dst[u][kh] = __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(
-              base + (size_t)min(m + u, DS - 1) * 1024 + (size_t)(2 * kh + lh) * 256));
+          dst[u][kh] = __builtin_nontemporal_load(reinterpret_cast<const i32x4*>(base + min(m + u, DS - 1) * 1024 + kh * 512 + own));
     };
-    // one round; X holds the group's first batch on entry and the next group's on exit
+    // (s_r, b_r) and the filter words of row gbase + lr of a group, issued ahead of its batches and of the last ones of the
+    // group before: the epilogue reads them back from this wave's LDS slot (16 B per 1-KiB row)
+    float2 rm_next;
+    int pr_next;
+    float ex_next;
+    uint64_t tg_next;
+    auto load_words = [&](int grp_) {
+      const int rowc = max(0, min(r0 + grp_ * 32 + lr, r1 - 1));
+      rm_next = *reinterpret_cast<const float2*>(rmeta + 2 * (size_t)rowc);
+      pr_next = row_prio[rowc];
+      ex_next = row_exp[rowc];
+      tg_next = row_tags[rowc];
+    };
+    auto lds_barrier = [] {  // the row loads stay in flight across it
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    };
+    auto flag = [&](int i) {
+      return __builtin_amdgcn_readfirstlane(__hip_atomic_load(need + i, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+    };
+    // Every wave that finds the flag set comes here, and the barrier holds it until all have.
+    auto compact_all = [&] {
+      __syncthreads();  // candidate stores complete and visible
+      if (threadIdx.x == 0) need[0] = 0;
+      for (int q = wid; q < Q; q += NWV)  // (those that would be due soon with them)
+        if (st.cnt[q] > C + C / 2) compact(my_u + q * CAND, my_l + q * CAND, my_r + q * CAND, st, q, K);
+      __syncthreads();
+    };
+    // the K-th best bound that the slices have published for a query (a few 1e-4 below it), 0: fewer than K have one
+    auto kth_published = [&](int q) {
+      constexpr int PER = MAX_WG / 64;
+      uint32_t key[PER];
+      int have = 0, own = lane;
+      asm volatile("" : "+v"(own));  // (no addresses from before the loop)
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int w = i * 64 + own;
+        key[i] = w < nwg ? __hip_atomic_load(pub + q * nwg + w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0;
+      }
+#pragma unroll
+      for (int i = 0; i < PER; ++i) have += __popcll(__ballot(key[i] != 0));
+      return have < K ? 0u : wave_select_floor<13>(key, K);
+    };
+    auto raise = [&](int q, uint32_t k) {
+      if (k && key_value(k) > st.tauL[q]) {
+        st.tauL[q] = key_value(k);
+        st.theta[q] = fmaxf(st.cap[q], key_value(k));
+      }
+    };
+    // one round; X and Y hold the group's first two batches on entry and the next group's on exit
     auto body = [&](int round, i32x4 (&X)[KB][2], i32x4 (&Y)[KB][2]) {
-      const int grp = round * NWV + wid;
+      const int grp = round * NWV + wid, next = grp + NWV;
       const int gbase = r0 + grp * 32;
-      // (s_r, b_r) of row gbase + lr, issued ahead of the group's later batches; the epilogue
-      // reads every row's pair back from this wave's LDS slot
-      const int rowc = max(0, min(gbase + lr, r1 - 1));
-      const float2 rmine = *reinterpret_cast<const float2*>(rmeta + 2 * (size_t)rowc);
-      // the row's filter words ride along (16 B per 1-KiB row): the admission path reads them
-      // from LDS instead of waiting on global loads behind the row stream
-      const int prmine = row_prio[rowc];
-      const float exmine = row_exp[rowc];
-      const uint64_t tgmine = row_tags[rowc];
       i32x16 acc_hh[NTQ], acc_lh[NTQ];
 #pragma unroll
       for (int t = 0; t < NTQ; ++t)
@@ -427,7 +476,7 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
         }
       auto compute = [&](const i32x4 (&ah)[KB][2], int m) {
 #pragma unroll
-        for (int u = 0; u < KB; ++u)
+        for (int u = 0; u < KB; ++u) {
 #pragma unroll
           for (int kh = 0; kh < 2; ++kh)
 #pragma unroll
@@ -438,142 +487,191 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
               acc_hh[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[u][kh], bh, acc_hh[t], 0, 0, 0);
               acc_lh[t] = __builtin_amdgcn_mfma_i32_32x32x32_i8(ah[u][kh], bl, acc_lh[t], 0, 0, 0);
             }
+        }
       };
       // sched_barrier pins each batch's loads where they are issued: left to the scheduler they
       // sink next to their first use and only ~1 load per wave stays in flight
-      // double-buffered batches: X holds the group's first batch on entry and the next group's
-      // on exit (a third buffer, two batches ahead, spilled registers at 64 queries)
+      // double-buffered batches, both of the next group in flight over the epilogue (a third buffer, two batches ahead,
+      // spilled registers at 64 queries)
 #pragma unroll
       for (int m = 0; m < DSC; m += 2 * KB) {
-        load(grp, m + KB, Y);
+        const bool more = m + 2 * KB < DSC;
         __builtin_amdgcn_sched_barrier(0);
-        if (m == 0 && lh == 0) {  // the row words to LDS: older than Y, waited with X
-          rm_lds[wid * 32 + lr] = rmine;
-          pr_lds[wid * 32 + lr] = prmine;
-          ex_lds[wid * 32 + lr] = exmine;
-          tg_lds[wid * 32 + lr] = tgmine;
-        }
         compute(X, m);
         __builtin_amdgcn_sched_barrier(0);
-        load(m + 2 * KB < DSC ? grp : grp + NWV, m + 2 * KB < DSC ? m + 2 * KB : 0, X);
+        if (m == 0 && lh == 0) {  // the words of this group, older than X
+          rm_lds[wid * 32 + lr] = rm_next;
+          pr_lds[wid * 32 + lr] = pr_next;
+          ex_lds[wid * 32 + lr] = ex_next;
+          tg_lds[wid * 32 + lr] = tg_next;
+        }
+        if (!more) load_words(next);
+        load(more ? grp : next, more ? m + 2 * KB : 0, X);
         __builtin_amdgcn_sched_barrier(0);
         compute(Y, m + KB);
+        __builtin_amdgcn_sched_barrier(0);
+        load(more ? grp : next, more ? m + 3 * KB : KB, Y);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      if (pub && round == 1) {
+        for (int q = wid; q < Q; q += NWV) raise(q, kth_published(q));
+        lds_barrier();  // no wave goes on without the first bounds
+      } else if (pub && round > 1) {
+        if (publishes(round - 1) && wid == 0 && wg < Q) {
+          const uint32_t k = kth_published(wg);
+          if (lane == 0) __hip_atomic_fetch_max(tau + wg, k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        }
+        if (round > 2 && publishes(round - 2) && wid == 0 && lane < Q)
+          raise(lane, __hip_atomic_load(tau + lane, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
+      }
+      if (round == 0) {
+        // The first groups show what their best rows reach before any is admitted: of every four rows the best lower bound
+        // that passes the query's filters, 64 of 256 rows, whose K-th best the query begins with. (With all 256 rows
+        // admitted for every query, 64 queries of 131,000 rows took 538 us a lookup, 450 so.)
+        const float2* rmw = rm_lds + wid * 32;
+#pragma unroll
+        for (int t = 0; t < NTQ; ++t) {
+          const int q = 32 * t + lr, minp = st.minp[q];
+          const uint64_t want = st.qtag[q];
+          const float sq = st.sq[q], cq = st.cq[q] * 1.0001f;
+#pragma unroll
+          for (int f = 0; f < 4; ++f) {
+            uint32_t best = 0;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const int ri = r + 8 * f + 4 * lh;
+              const float2 rm = rmw[ri];
+              const float ex = ex_lds[wid * 32 + ri];
+              const float sc = fmaf((float)acc_hh[t][4 * f + r], 65536.f, (float)acc_lh[t][4 * f + r] * 256.f) * (rm.x * sq);
+              const float e = fmaf(rm.y, cq, 1e-6f);
+              if (gbase + ri < r1 && (ex == 0.f || ex > now) && pr_lds[wid * 32 + ri] >= minp &&
+                  (tg_lds[wid * 32 + ri] & want) == want)
+                best = max(best, ord_key(sc - e));
+            }
+            first[q * 65 + (wid * 2 + lh) * 4 + f] = best;
+          }
+        }
+        lds_barrier();
+        for (int q = wid; q < Q; q += NWV) {
+          const uint32_t key[1] = {first[q * 65 + lane]};
+          if (__popcll(__ballot(key[0] != 0)) >= K) raise(q, wave_select_floor<13>(key, K));
+        }
+        lds_barrier();
       }
       if (grp < ngroups) {
         // lane holds queries 32 t + lr, rows gbase + (j & 3) + 8 (j >> 2) + 4 lh (j = 0..15).
-        // Fast path, branch-free: every (row, query) bound against its query's admission threshold
-        // theta (-> adm) and k-th lower bound tauL (tauL < U <= theta: refused for capacity ->
-        // one drop flag per query); only a lane holding an admissible bound takes the per-pair
-        // path (rare once the first compaction has set the thresholds). The branchy per-pair form,
-        // whose global loads drained the row stream at every refused-for-capacity row, cost
-        // ~10 ms of the 28.6-ms 100M-row pass (profiles/r6_q16_stage1.md)
+        // First only whether any lane's bound reaches its query's k-th lower bound tauL (theta is no lower): seven
+        // operations a pair, and once the bounds are tight most groups end there. (All of it for every group took 230 of
+        // the 940 us of 4M rows and 64 queries, as the waves' loads ran dry meanwhile.) Then the pairs (t, j) that some lane
+        // reaches, each behind a branch of the wave's: unrolled without, they do not fit the registers.
         const int nrow = r1 - gbase;  // rows ri < nrow are in the slice
-        float th[NTQ], tl[NTQ], sqv[NTQ], cqv[NTQ];
+        const float2* rmw = rm_lds + wid * 32;  // written by this wave (LDS order holds)
+        float tl[NTQ], sqv[NTQ], cqv[NTQ];
 #pragma unroll
         for (int t = 0; t < NTQ; ++t) {
           const int q = 32 * t + lr;
-          th[t] = q < Q ? st.theta[q] : INFINITY;
           tl[t] = q < Q ? st.tauL[q] : INFINITY;
           sqv[t] = st.sq[q];
           cqv[t] = st.cq[q] * 1.0001f;
         }
-        unsigned admbits = 0;  // bit 16 t + j: pair (query 32 t + lr, row j) is admissible
-        bool drp[NTQ];
-#pragma unroll
-        for (int t = 0; t < NTQ; ++t) drp[t] = false;
+        unsigned reach = 0;  // bit 16 t + j
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
-          const int ri = (j & 3) + 8 * (j >> 2) + 4 * lh;
-          const float2 rsv = rm_lds[wid * 32 + ri];  // written by this wave (LDS order holds)
-          const float rsx = rsv.x, rsy = rsv.y;
-          const bool rv = ri < nrow;
+          const float2 rm = rmw[(j & 3) + 8 * (j >> 2) + 4 * lh];
 #pragma unroll
           for (int t = 0; t < NTQ; ++t) {
-            const float sc = fmaf((float)acc_hh[t][j], 65536.f, (float)acc_lh[t][j] * 256.f) * (rsx * sqv[t]);
-            const float U = sc + fmaf(rsy, cqv[t], 1e-6f);
-            admbits |= (unsigned)((U > th[t]) & rv) << (16 * t + j);
-            drp[t] |= (U > tl[t]) & !(U > th[t]) & rv;  // refused for capacity, not by the k-th bound
+            const float U = fmaf(fmaf((float)acc_hh[t][j], 256.f, (float)acc_lh[t][j]), rm.x * (256.f * sqv[t]),
+                                 fmaf(rm.y, cqv[t], 2e-6f));  // (a margin over the bounds below)
+            if (__any(U > tl[t])) reach |= 1u << (16 * t + j);
           }
         }
-#pragma unroll
-        for (int t = 0; t < NTQ; ++t)
-          if (drp[t]) st.dropped[32 * t + lr] = 1;
-        if (admbits) {  // ~2 admissions per group: LDS reads and stores only on this path
-          const float2* rmw = rm_lds + wid * 32;
+        if (reach) {
+          // (what this path reads and writes is named here: addresses kept in registers from before the loop go to scratch
+          // memory, and each load from there waits for all row loads in flight)
+          int own = lr, half = 4 * lh + wid * 32, at = wg * (MAXQ * CAND);
+          asm volatile("" : "+v"(own), "+v"(half), "+s"(at));
 #pragma unroll
           for (int t = 0; t < NTQ; ++t) {
-            const int q = 32 * t + lr;
-            const float sq = sqv[t], cq = cqv[t];
+            const int q = 32 * t + own;
 #pragma unroll
             for (int j = 0; j < 16; ++j) {
-              if (!((admbits >> (16 * t + j)) & 1u)) continue;
-              const int ri = (j & 3) + 8 * (j >> 2) + 4 * lh;
-              const float2 rm = rmw[ri];  // == the shuffled pair of the fast path
-              const float sc = fmaf((float)acc_hh[t][j], 65536.f, (float)acc_lh[t][j] * 256.f) * (rm.x * sq);
-              const float e = fmaf(rm.y, cq, 1e-6f);  // margin: fp32 rounding of sc and e
-              if (pr_lds[wid * 32 + ri] < st.minp[q]) continue;
-              if ((tg_lds[wid * 32 + ri] & st.qtag[q]) != st.qtag[q]) continue;
-              const float ex = ex_lds[wid * 32 + ri];
-              if (ex != 0.f && !(ex > now)) continue;
+              if (!((reach >> (16 * t + j)) & 1u)) continue;
+              const int rw = (j & 3) + 8 * (j >> 2) + half, ri = rw - wid * 32;
+              const float2 rm = rm_lds[rw];
+              const float sc = fmaf((float)acc_hh[t][j], 65536.f, (float)acc_lh[t][j] * 256.f) * (rm.x * sqv[t]);
+              const float e = fmaf(rm.y, cqv[t], 1e-6f);  // margin: fp32 rounding of sc and e
+              if (ri >= nrow || !(sc + e > tl[t])) continue;
+              if (!(sc + e > st.theta[q])) {  // refused for capacity, not by the k-th bound
+                st.dropped[q] = 1;
+                continue;
+              }
+              const float ex = ex_lds[rw];
+              if (pr_lds[rw] < st.minp[q] || (tg_lds[rw] & st.qtag[q]) != st.qtag[q] ||
+                  (ex != 0.f && !(ex > now)))
+                continue;
               const int pos = atomicAdd(&st.cnt[q], 1);
               atomicMax(&st.top[q], ord_key(sc - e));
               if (pos < CAND) {
-                my_u[q * CAND + pos] = sc + e;
-                my_l[q * CAND + pos] = sc - e;
-                my_r[q * CAND + pos] = gbase + ri;
+                const unsigned to = at + q * CAND + pos;
+                cand_u[to] = sc + e;
+                cand_l[to] = sc - e;
+                cand_r[to] = gbase + ri;
               }
-              if (pos == LIM) need[round & 1] = 1;
+              if (pos >= LIM) __hip_atomic_store(need, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
             }
           }
         }
       }
-      // LDS-only barrier: the row loads stay in flight across it
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      __builtin_amdgcn_s_barrier();
-      asm volatile("" ::: "memory");
-      if (need[round & 1]) {  // workgroup-uniform; rare after the first rounds
-        __syncthreads();  // candidate stores complete and visible
-        if (threadIdx.x == 0) need[round & 1] = 0;
-        for (int q = wid; q < Q; q += NWV)  // (those that would be due soon with them)
-          if (st.cnt[q] > C + C / 2) compact(my_u + q * CAND, my_l + q * CAND, my_r + q * CAND, st, q, K);
-        __syncthreads();
-      }
-      if (pub && nwg >= K) {  // workgroup-uniform
-        if (publishes(round) && threadIdx.x < Q)
-          __hip_atomic_store(pub + threadIdx.x * nwg + wg, st.top[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (round && publishes(round - 1)) {
-          constexpr int QB = 4, PER = MAX_WG / 64;  // queries whose loads go out together
-          for (int q0 = wid * QB; q0 < Q; q0 += NWV * QB) {
-            uint32_t key[QB][PER];
-#pragma unroll
-            for (int b = 0; b < QB; ++b)
-#pragma unroll
-              for (int i = 0; i < PER; ++i) {
-                const int w = i * 64 + lane;
-                key[b][i] = w < nwg && q0 + b < Q ? __hip_atomic_load(pub + (q0 + b) * nwg + w, __ATOMIC_RELAXED,
-                                                                      __HIP_MEMORY_SCOPE_AGENT) : 0;
-              }
-#pragma unroll
-            for (int b = 0; b < QB; ++b) {
-              int have = 0;
-#pragma unroll
-              for (int i = 0; i < PER; ++i) have += __popcll(__ballot(key[b][i] != 0));
-              if (have < K) continue;
-              const float v = key_value(wave_select(key[b], K));
-              if (lane == 0 && v > st.tauL[q0 + b]) {
-                st.tauL[q0 + b] = v;
-                st.theta[q0 + b] = fmaxf(st.cap[q0 + b], v);
-              }
-            }
-          }
-        }
-      }
+      // (LDS only: the row loads stay in flight)
+      if (flag(0)) compact_all();
+      if (pub && publishes(round) && threadIdx.x < Q)
+        __hip_atomic_store(pub + threadIdx.x * nwg + wg, st.top[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     };
     i32x4 bA[KB][2], bB[KB][2];
+    load_words(wid);
     load(wid, 0, bA);
+    load(wid, KB, bB);
     for (int round = 0; round < nrounds; ++round) body(round, bA, bB);
+    // done: the others may still ask for a compaction
+    if (lane == 0) __hip_atomic_fetch_add(need + 1, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+    for (;;) {
+      const int done = flag(1);
+      if (flag(0)) compact_all();
+      else if (done == NWV) break;
+      else __builtin_amdgcn_s_sleep(4);
+    }
   }
   __syncthreads();
+  // The lists. Buffers of at most C entries, all of a wave's queries at once, so that their loads wait together.
+  constexpr int QW = ROWS / NWV;
+  int most = 0;
+#pragma unroll
+  for (int i = 0; i < QW; ++i) most = max(most, wid + NWV * i < Q ? st.cnt[wid + NWV * i] : 0);
+  if (most <= C) {
+    float u[QW], l[QW];
+    int row[QW];
+#pragma unroll
+    for (int i = 0; i < QW; ++i) {
+      const int q = min(wid + NWV * i, Q - 1), at = q * CAND + max(0, min(lane, st.cnt[q] - 1));
+      const bool ok = wid + NWV * i < Q && lane < st.cnt[q];
+      u[i] = ok ? my_u[at] : -INFINITY;
+      l[i] = ok ? my_l[at] : -INFINITY;
+      row[i] = ok ? my_r[at] : -1;
+    }
+#pragma unroll
+    for (int i = 0; i < QW; ++i) {
+      const int q = wid + NWV * i;
+      if (q >= Q) break;
+      const bool keep = row[i] >= 0 && !(u[i] < st.tauL[q]);  // (entries that the bound has overtaken go)
+      const unsigned long long kept = __ballot(keep), rest = ~kept;
+      const size_t o = ((size_t)q * nwg + wg) * C + (keep ? rank_in(kept) : (int)__popcll(kept) + rank_in(rest));
+      out_u[o] = keep ? u[i] : -INFINITY;
+      out_l[o] = keep ? l[i] : -INFINITY;
+      out_r[o] = keep ? row[i] : -1;
+      if (lane == 0) out_drop[(size_t)q * nwg + wg] = st.dropped[q] ? st.cap[q] : -INFINITY;
+    }
+    return;
+  }
   for (int q = wid; q < Q; q += NWV) {
     const size_t o = ((size_t)q * nwg + wg) * C;
     compact(my_u + q * CAND, my_l + q * CAND, my_r + q * CAND, st, q, K, out_u + o, out_l + o, out_r + o);
@@ -597,10 +695,10 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
   __shared__ Selection sel;
   __shared__ int crow[EXACT ? 1 : CL + MAXK];
   __shared__ uint32_t ckey[EXACT ? 1 : CL + MAXK];
-  __shared__ uint32_t cu[EXACT ? 1 : THREADS];
   __shared__ float best_s[MAXK];
   __shared__ int best_r[MAXK];
   __shared__ int ncand;
+  __shared__ uint32_t picked;
   const int q = blockIdx.x;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   const int total = nwg * C;
@@ -618,12 +716,6 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
     row[i] = e < total ? r[e] : -1;
     have += __popcll(__ballot(row[i] >= 0));
   }
-#pragma unroll
-  for (int i = 0; i < PER; ++i) {
-    const int e = i * THREADS + threadIdx.x;
-    key[i] = row[i] >= 0 ? ord_key(l[e]) : 0;
-    ukey[i] = !EXACT && row[i] >= 0 ? ord_key(u[e]) : 0;
-  }
   if (threadIdx.x == 0) ncand = 0;
   __syncthreads();
   int at = 0;
@@ -633,22 +725,34 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
   have = ncand;
   uint32_t tau = 1;
   if (EXACT || have > THREADS) {
+#pragma unroll
+    for (int i = 0; i < PER; ++i) {
+      const int e = min(i * THREADS + (int)threadIdx.x, total - 1);
+      key[i] = row[i] >= 0 ? ord_key(l[e]) : 0;
+      ukey[i] = !EXACT && row[i] >= 0 ? ord_key(u[e]) : 0;
+    }
     if (have >= K) tau = block_select<PER, NW>(key, K, red);
   } else {
-    // Slices that share their bounds list a row or two each: such entries move together, one a thread, which makes the
-    // selection's steps a ballot instead of 16.
+    // Slices that share their bounds list a row or two each: such entries move together, one a thread, which one
+    // wave selects from, and their bounds one load instead of 16 in turn (64 queries of 4M rows: 67 -> 53 us).
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const unsigned long long m = __ballot(row[i] >= 0);
       const int p = at + rank_in(m);
-      if (row[i] >= 0) { crow[p] = row[i]; ckey[p] = key[i]; cu[p] = ukey[i]; }
+      if (row[i] >= 0) { crow[p] = row[i]; ckey[p] = i * THREADS + threadIdx.x; }
       at += __popcll(m);
       row[i] = -1;
+      ukey[i] = 0;
     }
     __syncthreads();
-    uint32_t one[1] = {(int)threadIdx.x < have ? ckey[threadIdx.x] : 0};
-    if ((int)threadIdx.x < have) { row[0] = crow[threadIdx.x]; ukey[0] = cu[threadIdx.x]; }
-    if (have >= K) tau = block_select<1, NW>(one, K, red);
+    if ((int)threadIdx.x < have) {
+      const int e = ckey[threadIdx.x];
+      row[0] = crow[threadIdx.x];
+      ukey[0] = ord_key(u[e]);
+      ckey[threadIdx.x] = ord_key(l[e]);
+    }
+    __syncthreads();
+    if (have >= K) tau = lds_select(ckey, have, K, &picked);
   }
   // ---- B: a slice that refused a row for capacity at a level >= tau may have lost a top-k row
   if (EXACT) {  // the lists hold exact scores
@@ -740,7 +844,7 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
     if (n <= THREADS) {
       const uint32_t ck[1] = {(int)threadIdx.x < n ? ckey[threadIdx.x] : 0};
       const int cr[1] = {(int)threadIdx.x < n ? crow[threadIdx.x] : -1};
-      write_best(ck, cr, n > K ? block_select<1, NW>(ck, K, red) : 1, K, sel, bs, br);
+      write_best(ck, cr, n > K ? lds_select(ckey, n, K, &picked) : 1, K, sel, bs, br);
     } else {
       uint32_t ck[RR];
       int cr[RR];
@@ -852,11 +956,11 @@ __global__ __launch_bounds__(256) void prepare_kernel(const float* __restrict__ 
 }  // namespace q16
 }  // namespace pa
 
-// workspace: lists [3][Q][nwg][C] (U, L, row) + drop levels [Q][nwg] + published bounds [Q][nwg] + per-(slice, query)
+// workspace: lists [3][Q][nwg][C] (U, L, row) + drop levels [Q][nwg] + published bounds [Q][nwg] and [Q] + per-(slice, query)
 // candidate buffers [3][nwg][64][CAND]
 extern "C" long long pa_q16_topk_workspace_bytes(int Q, int N) {
   const long long w = pa::q16::num_wg(N);
-  return 3LL * Q * w * pa::q16::C * 4 + 2LL * Q * w * 4 + 3LL * w * pa::q16::MAXQ * pa::q16::CAND * 4;
+  return 3LL * Q * w * pa::q16::C * 4 + (2LL * w + 1) * Q * 4 + 3LL * w * pa::q16::MAXQ * pa::q16::CAND * 4;
 }
 
 // queries_q: [Q][2][D] int8 (qh, ql); qmeta [Q][2] (s_q, c_q); hi / lo: [N/16][D/64][64][16]
@@ -881,16 +985,17 @@ extern "C" int pa_q16_topk(float* out_scores, int* out_rows, int* unsafe, void* 
   int* lr = reinterpret_cast<int*>(ll + (size_t)Q * nwg * C);
   float* ldrop = reinterpret_cast<float*>(lr + (size_t)Q * nwg * C);
   uint32_t* pub = reinterpret_cast<uint32_t*>(ldrop + (size_t)Q * nwg);
-  float* cu = ldrop + 2 * (size_t)Q * nwg;
+  float* cu = ldrop + 2 * (size_t)Q * nwg + Q;
   float* cl = cu + (size_t)nwg * MAXQ * CAND;
   int* cr = reinterpret_cast<int*>(cl + (size_t)nwg * MAXQ * CAND);
   const int nqt = (Q + QT - 1) / QT;
   const size_t lds = (size_t)nqt * QT * (D + 16) * 2 + sizeof(QState) + 16;
   static bool attr_set = false;
   if (!attr_set) {
-    (void)hipFuncSetAttribute((const void*)stage1_bound_kernel<4>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    (void)hipFuncSetAttribute((const void*)stage1_bound_kernel<8>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    (void)hipFuncSetAttribute((const void*)stage1_bound_kernel<16>, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+#define PA_X(D) stage1_bound_kernel<D, true, 1>, stage1_bound_kernel<D, false, 1>, stage1_bound_kernel<D, true, 2>, stage1_bound_kernel<D, false, 2>
+    for (auto* k : {PA_X(4), PA_X(8), PA_X(16)})
+      (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+#undef PA_X
     (void)hipFuncSetAttribute((const void*)stage1_exact_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     attr_set = true;
   }
@@ -904,10 +1009,15 @@ extern "C" int pa_q16_topk(float* out_scores, int* out_rows, int* unsafe, void* 
                        ldrop, nwg, qv, qmeta, h, l, rmeta, D, K);
   } else {
     const int dsc = D <= 256 ? 4 : (D <= 512 ? 8 : 16);
-    const size_t ldsb = (size_t)MAXQ * (dsc * 64 + 16) * 2 + sizeof(QState) + 16 + 8 * 32 * 24;
-    if (N > 2 * MIN_ROWS_PER_WG * nwg) hipLaunchKernelGGL(clear_kernel, dim3(8), dim3(512), 0, st, pub, Q * nwg);
+    const int tiles = Q > 32 ? 2 : 1;
+    const size_t ldsb = (size_t)(32 * tiles) * (dsc * 64 + 16) * 2 + sizeof(QState) + 16 + 8 * 32 * 24 + 32 * tiles * 65 * 4;
+    if (N > MIN_ROWS_PER_WG * nwg) hipLaunchKernelGGL(clear_kernel, dim3(8), dim3(512), 0, st, pub, Q * (nwg + 1));
     else pub = nullptr;
-    auto* bound = dsc == 4 ? stage1_bound_kernel<4> : dsc == 8 ? stage1_bound_kernel<8> : stage1_bound_kernel<16>;
+    const bool full = D == dsc * 64;
+#define PA_X(D) (full ? (tiles == 1 ? stage1_bound_kernel<D, true, 1> : stage1_bound_kernel<D, true, 2>)    \
+                      : (tiles == 1 ? stage1_bound_kernel<D, false, 1> : stage1_bound_kernel<D, false, 2>))
+    auto* bound = dsc == 4 ? PA_X(4) : dsc == 8 ? PA_X(8) : PA_X(16);
+#undef PA_X
     hipLaunchKernelGGL(bound, dim3(nwg), dim3(512), ldsb, st, lu, ll, lr, ldrop, cu, cl, cr, qv, qmeta, h, rmeta, Q, N, D,
                        K, row_priority, row_tags, row_expiry, q_min_priority, q_tags, now, pub);
     hipLaunchKernelGGL(stage2_kernel<false>, dim3(Q), dim3(THREADS), 0, st, out_scores, out_rows, unsafe, lu, ll, lr,

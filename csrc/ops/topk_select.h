@@ -45,7 +45,21 @@ __device__ __forceinline__ uint32_t wave_select(const uint32_t (&key)[N], int wa
   return wave_umin(m);
 }
 
-// The same over a workgroup of NW waves; every thread calls it. `red` holds 2 * NW integers in LDS.
+// A lower bound of it: the largest value of 32 - LOW leading bits that at least `want` keys reach.
+template <int LOW, int N>
+__device__ __forceinline__ uint32_t wave_select_floor(const uint32_t (&key)[N], int want) {
+  uint32_t v = 0;
+  for (int b = 31; b >= LOW; --b) {
+    const uint32_t t = v | (1u << b);
+    int c = 0;
+#pragma unroll
+    for (int i = 0; i < N; ++i) c += __popcll(__ballot(key[i] >= t));
+    if (c >= want) v = t;
+  }
+  return v;
+}
+
+// wave_select over a workgroup of NW waves; every thread calls it. `red` holds 2 * NW integers in LDS.
 template <int N, int NW>
 __device__ __forceinline__ uint32_t block_select(const uint32_t (&key)[N], int want, int* red) {
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -78,6 +92,24 @@ __device__ __forceinline__ uint32_t block_select(const uint32_t (&key)[N], int w
 #pragma unroll
   for (int w = 0; w < NW; ++w) m = min(m, (uint32_t)red[w]);
   return m;
+}
+
+// The `want`-th largest of n <= 1,024 keys in LDS (at least `want` of them are not 0), by the first wave: its ballots need no
+// barriers, where block_select has one for every bit. Every thread of a workgroup calls it, the keys written before a
+// barrier; `res`: a word in LDS.
+__device__ __forceinline__ uint32_t lds_select(const uint32_t* keys, int n, int want, uint32_t* res) {
+  if (threadIdx.x < 64) {
+    uint32_t key[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) {
+      const int e = i * 64 + threadIdx.x;
+      key[i] = e < n ? keys[e] : 0;
+    }
+    const uint32_t v = n <= 256 ? wave_select(reinterpret_cast<const uint32_t(&)[4]>(key), want) : wave_select(key, want);
+    if (threadIdx.x == 0) *res = v;
+  }
+  __syncthreads();
+  return *res;
 }
 
 // The `K` best of (key, row) entries that gather() names, in order (key down, row up), to out_s / out_r, padded with

@@ -70,10 +70,35 @@ def test_q16_exact_scan_matches_reference(gpu, N, Q, K):
 
 @pytest.mark.parametrize("N,D,Q,K,filters", [
     (255, 64, 3, 64, False), (257, 192, 2, 7, True),  # one slice, two slices
-    (65_536 + 31, 256, 64, 33, True), (2 * 65_536, 256, 64, 64, False),  # the last size before slices share bounds
-    (2 * 65_536 + 1, 256, 64, 1, True), (600_011, 256, 5, 64, True)])  # and with them
+    (65_536 + 31, 256, 64, 33, True), (2 * 65_536, 256, 64, 64, False),  # slices of two rounds, which share bounds
+    (2 * 65_536 + 1, 256, 64, 1, True), (600_011, 256, 5, 64, True)])
 def test_q16_slices_and_shared_bounds(gpu, N, D, Q, K, filters):
     _check(gpu, N, D, Q, K, filters, seed=11)
+
+
+@pytest.mark.parametrize("N,D,Q,K", [  # one tile of queries and two, whole steps of dimensions and padded ones, slices of one round
+    (65_536, 512, 32, 64), (65_537, 448, 33, 1), (66_000, 1024, 1, 16), (131_073, 960, 64, 8), (400_000, 192, 32, 17)])
+def test_q16_tiles_of_queries(gpu, N, D, Q, K):
+    _check(gpu, N, D, Q, K, True, seed=3)
+
+
+@pytest.mark.parametrize("N,D,Q,K", [(3_000, 128, 64, 5), (70_000, 64, 40, 64), (140_000, 128, 3, 20)])
+def test_q16_rows_in_rising_order(gpu, N, D, Q, K):
+    """Every row is nearer to the queries than the one before: each round admits all of its rows, and the waves ask for
+    compactions all the time."""
+    g = torch.Generator(device=gpu).manual_seed(N)
+    q = torch.nn.functional.normalize(torch.randn(1, D, device=gpu, generator=g), dim=1)
+    x = torch.nn.functional.normalize(torch.randn(N, D, device=gpu, generator=g), dim=1) + torch.linspace(0, 2, N, device=gpu)[:, None] * q
+    pad = (-N) % 16
+    x = torch.cat([torch.nn.functional.normalize(x, dim=1), torch.zeros(pad, D, device=gpu)])
+    hi, lo, sc, bd = ops.q16_quantize(x)
+    hi, lo, rmeta = ops.q16_pack(hi).contiguous(), ops.q16_pack(lo).contiguous(), torch.stack([sc, bd], 1).contiguous()
+    qs = torch.nn.functional.normalize(q + 0.02 * torch.randn(Q, D, device=gpu, generator=g), dim=1)
+    filters = _filters(N, Q, gpu, True)
+    s, r = ops.q16_topk(qs, hi, lo, rmeta, N, K, *filters, 2.0)
+    qv, qm = ops.q16_queries(qs)
+    rs, rr = ref.q16_topk(qv.cpu(), qm.cpu(), hi.cpu(), lo.cpu(), rmeta.cpu(), N, K, *(f.cpu() for f in filters), 2.0)
+    assert torch.equal(r.cpu(), rr) and torch.equal(s.cpu(), rs)
 
 
 def test_q16_fewer_hits_than_k(gpu):
