@@ -4,6 +4,8 @@
 // current HIP stream, which keeps them hipGraph-capturable.
 #include "bind_common.h"
 
+#include <cstring>
+
 extern "C" {
 int pa_rmsnorm(void* out, const void* x, const void* w, int T, int D, float eps, hipStream_t st);
 int pa_fused_add_rmsnorm(void* out, void* resid, const void* x, const void* w, int T, int D,
@@ -67,7 +69,8 @@ int pa_cosine_topk(float* out_scores, int* out_rows, void* workspace, const void
                    const uint64_t* row_tags, const float* row_expiry, const int* q_min_priority,
                    const uint64_t* q_tags, float now, int n_valid, hipStream_t st);
 long long pa_q16_topk_workspace_bytes(int Q, int N);
-int pa_prepare_queries(const float* x, int Q, int D, int normalize, void* out, void* qv, float* qmeta, hipStream_t st);
+int pa_prepare_queries(const float* x, int Q, int D, int normalize, void* out, void* qv, float* qmeta, const int* minp,
+                       const uint64_t* tags, int* fminp, uint64_t* ftags, hipStream_t st);
 int pa_q16_topk(float* out_scores, int* out_rows, int* unsafe, void* workspace, const void* queries_q,
                 const float* qmeta, const void* hi, const void* lo, const float* rmeta, int Q, int N, int D, int K,
                 const int* row_priority, const uint64_t* row_tags, const float* row_expiry,
@@ -596,8 +599,50 @@ void prepare_queries(at::Tensor x, bool normalize, c10::optional<at::Tensor> out
     TORCH_CHECK(qmeta->is_contiguous() && qmeta->numel() == 2 * x.size(0), "qmeta [Q, 2]");
   }
   check_rc(pa_prepare_queries(x.data_ptr<float>(), (int)x.size(0), (int)x.size(1), normalize, out ? out->data_ptr() : nullptr,
-                              out ? nullptr : qv->data_ptr(), out ? nullptr : qmeta->data_ptr<float>(), cur_stream()),
+                              out ? nullptr : qv->data_ptr(), out ? nullptr : qmeta->data_ptr<float>(), nullptr, nullptr, nullptr,
+                              nullptr, cur_stream()),
            "prepare_queries");
+}
+
+// What a lookup by a caller who waits for it needs, on the current stream: queries (fp32 [Q, D], on the host or the GPU)
+// brought to unit length and rounded, filters (masks int64 [Q], minp int32 [Q], on the host) on the GPU, and room for the
+// results. -> [results int32 [Q (2 K + 1)] on the host, scores, rows, flags, minp, masks, queries (bf16, or int8 planes and
+// their scales)]. The pass reads the caller's values from pinned memory and writes scores, rows and flags, views of the
+// results as the GPU sees them, to it: a copy of either took as long as a small index. The first tensor keeps the pinned memory,
+// so it has to outlive the stream's work.
+std::vector<at::Tensor> lookup_begin(at::Tensor q, at::Tensor masks, at::Tensor minp, int64_t K, bool q16) {
+  const int device = c10::hip::current_device();
+  check_dtype(q, at::kFloat, "queries");
+  check_dtype(masks, at::kLong, "masks");
+  check_dtype(minp, at::kInt, "min_priority");
+  TORCH_CHECK(q.dim() == 2 && q.is_contiguous() && (q.is_cuda() ? q.get_device() == device : q.device().is_cpu()), "queries [Q, D]");
+  const int64_t Q = q.size(0), D = q.size(1), R = Q * (2 * K + 1);
+  TORCH_CHECK(Q >= 1 && K >= 1 && masks.device().is_cpu() && minp.device().is_cpu() && masks.is_contiguous() && minp.is_contiguous() &&
+                  masks.numel() == Q && minp.numel() == Q, "lookup filters");
+  const int64_t at_q = (16 * Q + 63) / 64 * 64, at_r = at_q + (q.is_cuda() ? 0 : 4 * Q * D + 63) / 64 * 64;
+  at::Tensor host = at::empty({at_r + 4 * R}, at::TensorOptions().dtype(at::kByte).pinned_memory(true));
+  char* h = (char*)host.data_ptr();
+  std::memcpy(h, masks.data_ptr(), 8 * Q);
+  std::memcpy(h + 8 * Q, minp.data_ptr(), 4 * Q);
+  if (!q.is_cuda()) std::memcpy(h + at_q, q.data_ptr(), 4 * Q * D);
+  const auto dev = [&](at::ScalarType t) { return at::TensorOptions().dtype(t).device(at::Device(at::kCUDA, device)); };
+  void* hd = nullptr;
+  TORCH_CHECK(hipHostGetDevicePointer(&hd, h, 0) == hipSuccess && hd == h, "lookup: the GPU does not see pinned memory at its address");
+  auto seen = [&](int64_t from, at::IntArrayRef sizes, at::ScalarType t) {
+    return at::from_blob(h + at_r + 4 * from, sizes, [host](void*) {}, dev(t), at::Device(at::kCUDA, device));
+  };
+  at::Tensor fminp = at::empty({Q}, dev(at::kInt)), ftags = at::empty({Q}, dev(at::kLong));
+  at::Tensor qa = q16 ? at::empty({Q, 2, D}, dev(at::kChar)) : at::empty({Q, D}, dev(at::kBFloat16)), qm;
+  if (q16) qm = at::empty({Q, 2}, dev(at::kFloat));
+  check_rc(pa_prepare_queries(q.is_cuda() ? q.data_ptr<float>() : (const float*)(h + at_q), (int)Q, (int)D, 1,
+                              q16 ? nullptr : qa.data_ptr(), q16 ? qa.data_ptr() : nullptr, q16 ? qm.data_ptr<float>() : nullptr,
+                              (const int*)(h + 8 * Q), (const uint64_t*)h, fminp.data_ptr<int>(), (uint64_t*)ftags.data_ptr<int64_t>(),
+                              cur_stream()),
+           "prepare_queries");
+  std::vector<at::Tensor> out{at::from_blob(h + at_r, {R}, [host](void*) {}, at::TensorOptions().dtype(at::kInt)),
+                              seen(0, {Q, K}, at::kFloat), seen(Q * K, {Q, K}, at::kInt), seen(2 * Q * K, {Q}, at::kInt), fminp, ftags, qa};
+  if (q16) out.push_back(qm);
+  return out;
 }
 
 int64_t q16_topk_workspace_bytes(int64_t Q, int64_t N) { return pa_q16_topk_workspace_bytes(Q, N); }
@@ -884,6 +929,7 @@ PYBIND11_MODULE(_C, m) {
   m.def("tp_topkp_phase", &tp_topkp_phase);
   m.def("cosine_topk_workspace_bytes", &cosine_topk_workspace_bytes);
   m.def("cosine_topk", &cosine_topk);
+  m.def("lookup_begin", &lookup_begin);
   m.def("prepare_queries", &prepare_queries, py::arg("x"), py::arg("normalize"), py::arg("out") = py::none(),
         py::arg("qv") = py::none(), py::arg("qmeta") = py::none());
   m.def("q16_topk_workspace_bytes", &q16_topk_workspace_bytes);

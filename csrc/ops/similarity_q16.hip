@@ -883,13 +883,30 @@ __device__ __forceinline__ float div_rn(float x, float y) {
 // One workgroup a query: normalised (if asked), then rounded to bf16, or to 16-bit fixed point as q16_quantize does:
 // s_q = max|x| / 32512, v = round(x / s_q) = 256 qh + ql, c_q = s_q ||v||_2 (a hair above). NaN goes where torch's
 // operations take it: a norm or a maximum of a query that holds one is one (s_q is then 1), and in v it is 0. One launch in
-// place of the 28 elementwise ones that took as long as the search of a small index.
+// place of the 28 elementwise ones that took as long as the search of a small index. x is read once, of up to PQ * 256
+// dimensions, as it may lie in the host's memory; so may the query's filters (minp, tags), which go to fminp and ftags.
+constexpr int PQ = 8;
 __global__ __launch_bounds__(256) void prepare_kernel(const float* __restrict__ x, int D, int normalize, bf16* __restrict__ out,
-                                                      signed char* __restrict__ qv, float* __restrict__ qmeta) {
+                                                      signed char* __restrict__ qv, float* __restrict__ qmeta,
+                                                      const int* __restrict__ minp, const uint64_t* __restrict__ tags,
+                                                      int* __restrict__ fminp, uint64_t* __restrict__ ftags) {
   __shared__ double red[4];
   __shared__ uint32_t redm[4];
   const int q = blockIdx.x, lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   x += (size_t)q * D;
+  if (fminp && threadIdx.x == 0) {
+    fminp[q] = minp[q];
+    ftags[q] = tags[q];
+  }
+  float xs[PQ];
+#pragma unroll
+  for (int k = 0; k < PQ; ++k) xs[k] = k * 256 + (int)threadIdx.x < D ? x[k * 256 + threadIdx.x] : 0.f;
+  auto each = [&](auto f) {  // f(dimension, value) of this thread's dimensions
+#pragma unroll
+    for (int k = 0; k < PQ; ++k)
+      if (k * 256 + (int)threadIdx.x < D) f(k * 256 + (int)threadIdx.x, xs[k]);
+    for (int i = PQ * 256 + threadIdx.x; i < D; i += 256) f(i, x[i]);
+  };
   auto sum = [&](double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
@@ -904,20 +921,19 @@ __global__ __launch_bounds__(256) void prepare_kernel(const float* __restrict__ 
   float by = 1.f;
   if (normalize) {
     double ss = 0.;
-    for (int i = threadIdx.x; i < D; i += 256) ss += (double)x[i] * (double)x[i];
+    each([&](int, float v) { ss += (double)v * (double)v; });
     ss = sum(ss);
     const long long over = __double_as_longlong(ss) - 0x7ff0000000000000ll;  // the norm is infinite (0) or NaN (above)
     by = fmaxf((float)sqrt(ss), 1e-12f);
     if (over >= 0 || size(by) == INF) {  // finite values become 0 or NaN, the others NaN
-      for (int i = threadIdx.x; i < D; i += 256) {
+      each([&](int i, float v) {
         if (out) {
-          reinterpret_cast<uint16_t*>(out)[(size_t)q * D + i] =
-              over > 0 || size(x[i]) >= INF ? 0x7fc0 : __float_as_uint(x[i]) >> 16 & 0x8000;
+          reinterpret_cast<uint16_t*>(out)[(size_t)q * D + i] = over > 0 || size(v) >= INF ? 0x7fc0 : __float_as_uint(v) >> 16 & 0x8000;
         } else {
           qv[(size_t)q * 2 * D + i] = 0;
           qv[(size_t)q * 2 * D + D + i] = 0;
         }
-      }
+      });
       if (!out && threadIdx.x == 0) {
         qmeta[2 * q] = 1.f;
         qmeta[2 * q + 1] = 0.f;
@@ -925,13 +941,13 @@ __global__ __launch_bounds__(256) void prepare_kernel(const float* __restrict__ 
       return;
     }
   }
-  auto at = [&](int i) { return normalize ? div_rn(x[i], by) : x[i]; };
+  auto at = [&](float v) { return normalize ? div_rn(v, by) : v; };
   if (out) {
-    for (int i = threadIdx.x; i < D; i += 256) out[(size_t)q * D + i] = (bf16)at(i);
+    each([&](int i, float v) { out[(size_t)q * D + i] = (bf16)at(v); });
     return;
   }
   uint32_t mb = 0;  // magnitudes in their bits' order, NaN above all
-  for (int i = threadIdx.x; i < D; i += 256) mb = max(mb, size(at(i)));
+  each([&](int, float v) { mb = max(mb, size(at(v))); });
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) mb = max(mb, (uint32_t)__shfl_xor((int)mb, o, 64));
   if (lane == 0) redm[wid] = mb;
@@ -939,13 +955,13 @@ __global__ __launch_bounds__(256) void prepare_kernel(const float* __restrict__ 
   mb = max(max(redm[0], redm[1]), max(redm[2], redm[3]));
   const float sc = mb > 0 && mb <= INF ? div_rn(__uint_as_float(mb), 32512.f) : 1.f;
   double vv = 0.;
-  for (int i = threadIdx.x; i < D; i += 256) {
-    const float f = rintf(div_rn(at(i), sc));
+  each([&](int i, float x) {
+    const float f = rintf(div_rn(at(x), sc));
     const int v = size(f) > INF ? 0 : (int)fminf(fmaxf(f, -32512.f), 32512.f), h = (v + 128) >> 8;
     qv[(size_t)q * 2 * D + i] = (signed char)h;
     qv[(size_t)q * 2 * D + D + i] = (signed char)(v - 256 * h);
     vv += (double)v * (double)v;  // whole numbers below 2^53: exact in any order
-  }
+  });
   vv = sum(vv);
   if (threadIdx.x == 0) {
     qmeta[2 * q] = sc;
@@ -1026,11 +1042,12 @@ extern "C" int pa_q16_topk(float* out_scores, int* out_rows, int* unsafe, void* 
   return (int)hipGetLastError();
 }
 
-// x fp32 [Q][D] -> bf16 [Q][D] (out), or, with out null, int8 [Q][2][D] (qv) and fp32 [Q][2] (qmeta).
-extern "C" int pa_prepare_queries(const float* x, int Q, int D, int normalize, void* out, void* qv, float* qmeta,
-                                  hipStream_t st) {
+// x fp32 [Q][D] -> bf16 [Q][D] (out), or, with out null, int8 [Q][2][D] (qv) and fp32 [Q][2] (qmeta). With fminp, the queries'
+// filters minp [Q] and tags [Q] are copied to fminp and ftags.
+extern "C" int pa_prepare_queries(const float* x, int Q, int D, int normalize, void* out, void* qv, float* qmeta, const int* minp,
+                                  const uint64_t* tags, int* fminp, uint64_t* ftags, hipStream_t st) {
   if (Q <= 0) return 0;
   hipLaunchKernelGGL(pa::q16::prepare_kernel, dim3(Q), dim3(256), 0, st, x, D, normalize, (pa::bf16*)out, (signed char*)qv,
-                     qmeta);
+                     qmeta, minp, tags, fminp, ftags);
   return (int)hipGetLastError();
 }

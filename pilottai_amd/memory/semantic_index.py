@@ -19,8 +19,10 @@ one all-gather (RCCL over xGMI).
 """
 from __future__ import annotations
 
+import contextlib
 import threading
 import time
+from itertools import islice
 from typing import Dict, Iterable, List, Optional, Sequence, Tuple
 
 import numpy as np
@@ -332,51 +334,47 @@ class SemanticIndex:
 
     def _search_host(self, q: torch.Tensor, k: int, min_priority, qmasks, now: Optional[float]):
         """search_tensors for a caller that waits for the answer, with filters as lists: (scores, rows) as arrays, [Q, k].
-        What the pass reads goes to the device in one pinned copy and comes back in one (queries and filters, scores, rows
-        and flags were four copies out and up to three back, each with its own wait)."""
+        The pass reads queries and filters from pinned memory and writes its results there (ops.lookup_begin)."""
         Q, D = q.shape
         caller = torch.cuda.current_stream(self.device) if q.is_cuda else None
+        words = []
+        for values, dtype in ((qmasks, np.int64), (min_priority, np.int32)):
+            if len(values) < Q:
+                raise ValueError(f"{len(values)} filters for {Q} queries")
+            to = np.empty(Q, dtype)
+            try:
+                to[:] = values[:Q]
+            except TypeError:  # (numbers on the GPU)
+                to[:] = torch.as_tensor(values[:Q]).cpu().numpy()
+            words.append(torch.from_numpy(to))
         with self._lock, self._stream_ctx():
-            here = torch.cuda.current_stream(self.device)
+            here = self._stream
             if caller is not None:
                 here.wait_stream(caller)
-            host = torch.empty(16 * Q + (0 if q.is_cuda else 4 * Q * D), dtype=torch.uint8, pin_memory=True)
-            h = host.numpy()
-            for values, to in ((qmasks, h[:8 * Q].view(np.int64)), (min_priority, h[8 * Q:12 * Q].view(np.int32))):
-                if len(values) < Q:
-                    raise ValueError(f"{len(values)} filters for {Q} queries")
-                try:
-                    to[:] = values[:Q]
-                except TypeError:  # (numbers on the GPU)
-                    to[:] = torch.as_tensor(values[:Q]).cpu().numpy()
-            if not q.is_cuda:
-                h[16 * Q:].view(np.float32).reshape(Q, D)[:] = q.detach().float().numpy()
-            dev = host.to(self.device, non_blocking=True)
-            qt, minp = dev[:8 * Q].view(torch.int64), dev[8 * Q:12 * Q].view(torch.int32)
-            qd = q.to(self.device, torch.float32).contiguous() if q.is_cuda else dev[16 * Q:].view(torch.float32).view(Q, D)
+            q = q.detach().to(self.device if q.is_cuda else "cpu", torch.float32).contiguous()
             ev = self._pass_event()
             t_now = self.now() if now is None else now - self.epoch
-            buf, s, r, unsafe = ops.topk_result(Q, k, self.device)
+            back, out, (minp, qt), qs = ops.lookup_begin(q, *words, k, self.storage == "q16")
             filters = (self.priority, self.tagbits, self.expiry, minp, qt, t_now)
-            if self.storage == "q16":
-                qv, qm = ops.q16_queries(qd, normalize=True)
-                args = (qv, qm, self.hi, self.lo, self.rmeta, self.count, k, *filters, (s, r, unsafe))
-                ops.q16_pass(*args, False, self._ws)
-            else:
-                ops.cosine_topk(ops.unit_queries(qd), self.packed, self.count, k, *filters, workspace=self._ws, out=(s, r))
-            if ev is not None:
-                ev[1].record()
-            back = torch.empty(buf.shape, dtype=torch.int32, pin_memory=True)
-            back.copy_(buf, non_blocking=True)
-        a = back.numpy()
+            try:
+                if self.storage == "q16":
+                    args = (*qs, self.hi, self.lo, self.rmeta, self.count, k, *filters, out)
+                    ops.q16_pass(*args, False, self._ws)
+                else:
+                    ops.cosine_topk(*qs, self.packed, self.count, k, *filters, workspace=self._ws, out=out[:2])
+                if ev is not None:
+                    ev[1].record()
+            except BaseException:
+                here.synchronize()  # (the pinned memory is not given back before the GPU is done with it)
+                raise
         here.synchronize()
+        a = back.numpy()
         if self.storage == "q16" and a[2 * Q * k:].any():  # a slice refused a row that might be in the top-k
             with self._lock, self._stream_ctx():
                 self.stats["q16_fallbacks"] += 1
                 ops.q16_pass(*args, True, self._ws)
                 if ev is not None:  # (both passes, as search_tensors has it)
                     ev[1].record()
-                back.copy_(buf, non_blocking=True)
             here.synchronize()
         if ev is not None:
             self.pass_events.append(ev)
@@ -400,17 +398,11 @@ class SemanticIndex:
         else:
             s, r = (t.numpy() for t in self.search_tensors(q, kk, list(min_priority), qmasks, now))
         out = []
-        for i in range(Q):
-            res = []
-            for row, sc in zip(r[i], s[i]):
-                if row < 0:
-                    break
-                if not exact[i] and not tag_sets[i] <= self._row_tags(int(row)):
-                    continue
-                res.append((int(row), float(sc)))
-                if len(res) >= k:
-                    break
-            out.append(res)
+        for i, (rows, scores) in enumerate(zip(r.tolist(), s.tolist())):
+            hits = zip(rows if rows[-1] >= 0 else rows[:rows.index(-1)], scores)  # (past the hits: -1)
+            if not exact[i]:
+                hits = (h for h in hits if tag_sets[i] <= self._row_tags(h[0]))
+            out.append(list(islice(hits, k)))
         return out
 
     def _stream_ctx(self):
@@ -418,18 +410,13 @@ class SemanticIndex:
         co-resident with a serving engine, a lookup pass overlaps the engine's step
         instead of queueing behind its graph, and waiting for the result syncs only
         this stream. Also pins the calling thread to the index's device."""
-        import contextlib
-
         if self.device.type != "cuda":
             return contextlib.nullcontext()
         if self._stream is None:
             # its own stream, at the default priority (work on streams of different priorities
             # has hung): a lookup pass shares the device with the engine's steps
             self._stream = torch.cuda.Stream(device=self.device)
-        st = contextlib.ExitStack()
-        st.enter_context(torch.cuda.device(self.device))
-        st.enter_context(torch.cuda.stream(self._stream))
-        return st
+        return torch.cuda.stream(self._stream)  # (and its device)
 
     def memory_bytes(self) -> int:
         rows = sum(p.numel() * p.element_size() for _, p in self._planes())

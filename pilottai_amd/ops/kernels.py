@@ -279,6 +279,15 @@ def topk_result(Q: int, K: int, device):
     return buf, buf[:Q * K].view(torch.float32).view(Q, K), buf[Q * K:2 * Q * K].view(Q, K), buf[2 * Q * K:]
 
 
+def lookup_begin(q: torch.Tensor, masks: torch.Tensor, min_priority: torch.Tensor, K: int, q16: bool):
+    """What a pass needs for a caller who waits for its results, on the current stream: q fp32 [Q, D] (on the host
+    or there), masks int64 and min_priority int32 [Q] on the host. -> (results int32 [Q (2 K + 1)] in pinned memory,
+    (scores, rows, flags) that the pass writes there, (min_priority, masks) and the queries as the pass reads them). The
+    results have to be kept until the stream's work is done."""
+    back, s, r, flags, minp, tags, *qs = require_native().lookup_begin(q, masks, min_priority, int(K), bool(q16))
+    return back, (s, r, flags), (minp, tags), qs
+
+
 def cosine_topk(queries, index, n_valid: int, K: int, row_priority, row_tags, row_expiry,
                 q_min_priority, q_tags, now: float, workspace: Optional[torch.Tensor] = None, out=None):
     """`out`: (scores, rows) to write to."""

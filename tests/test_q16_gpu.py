@@ -221,6 +221,29 @@ def test_search_takes_any_sequence_of_filters(gpu, storage):
         idx.search(q, 4, [0, 1, 1 << 40], none)
 
 
+@pytest.mark.parametrize("storage", ["bf16", "q16"])
+@pytest.mark.parametrize("Q", [1, 64, 65, 130])  # a pass, and several
+def test_search_takes_queries_from_anywhere(gpu, storage, Q):
+    """Queries as an array, as tensors of the host or the GPU, of other types and strides: the same results, in lists of plain
+    numbers that end with the hits."""
+    idx, v = _small_index(gpu, storage)
+    q = torch.from_numpy(v[:Q])
+    args = (3, [i % 3 for i in range(Q)], [()] * Q)
+    want = idx.search(v[:Q], *args)
+    assert [len(w) for w in want] == [3] * Q and all(type(r) is int and type(x) is float for w in want for r, x in w)
+    assert all(w[0][0] == i for i, w in enumerate(want))
+    for x in (q, q.double(), q.to(gpu), q.t().contiguous().t(), q.t().contiguous().to(gpu).t()):
+        assert idx.search(x, *args) == want
+    assert idx.search(q, 3, [2] * Q, [("unknown",)] * Q) == [[]] * Q
+
+
+@pytest.mark.parametrize("D", [1984, 2048, 2112])  # around what a workgroup keeps of a query
+def test_query_preparation_of_long_queries(gpu, D):
+    q = torch.randn(3, D)
+    assert torch.equal(ops.unit_queries(q.to(gpu)).cpu(), ops.unit_queries(q))
+    assert all(torch.equal(a.cpu(), b) for a, b in zip(ops.q16_queries(q.to(gpu), True), ops.q16_queries(q, True)))
+
+
 def test_search_times_its_second_pass_too(gpu, monkeypatch):
     """The events around a search that falls back to the exact scan lie around both passes."""
     idx, v = _small_index(gpu, n=40_000, same=True)
