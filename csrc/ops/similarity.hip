@@ -11,7 +11,7 @@
 // (priority index range, tag-set intersection, is_expired) evaluated in-kernel.
 //
 // Stage 1 (one pass over the index for up to 64 queries): each workgroup owns a
-// slice of rows; its 16 waves take 16-row groups and multiply them by EVERY query
+// slice of rows; its 16 (or 8) waves take 16-row groups and multiply them by EVERY query
 // tile with v_mfma_f32_16x16x32_bf16 — index rows stream from HBM straight into
 // the A operand once (the index is stored in 16-row tiles, fragment-major:
 // [N/16][D/32][64 lanes][8], so each wave load is 1 KiB contiguous instead of
@@ -30,16 +30,17 @@ constexpr int SIM_MAXK = 64;
 constexpr int SIM_QT = 16;        // queries per MFMA tile (N = 16)
 constexpr int SIM_MAXQ = 64;      // queries per pass (4 tiles resident in LDS)
 constexpr int SIM_MAXD = 1024;    // LDS query capacity per query (bf16)
-constexpr int SIM_THREADS = 1024; // 16 waves: 128 KB of row loads in flight per CU
-// one round of 16 waves x 16 rows a slice at least: 20,000 rows give 79 slices (10 with the 2,048 rows that the sorting
-// compactions needed: 126 us for 3 queries)
-constexpr int SIM_MIN_ROWS_PER_WG = 256;
+// One round of a workgroup's waves x 16 rows a slice at least: 16 waves, 128 KB of row loads in flight per CU, or for few
+// queries 8 while they leave the CUs a slice at most, as a CU's share of the rows is what a small index waits for (20,000 rows,
+// 3 queries: 79 slices 20 us, 157 15). With many queries their work on the first round is (40 of 5,000 rows: 29 and 33).
+constexpr int SIM_FEW = 128, SIM_MANY = 256, SIM_FEW_Q = 16;  // rows of a round, queries
 constexpr int SIM_LIM = 2 * SIM_MAXK;  // entries of a buffer between rounds; a round may admit 256 more
 constexpr int SIM_KB = 8;         // k-steps per row-load batch (two batches in flight)
 constexpr int SIM_MAX_WG = 256;    // one resident workgroup per CU: the threshold warm-up is paid once per CU
 
-__host__ __device__ inline int sim_num_wg(int N) {
-  int nwg = (N + SIM_MIN_ROWS_PER_WG - 1) / SIM_MIN_ROWS_PER_WG;
+inline int sim_rows(int Q, int N) { return Q <= SIM_FEW_Q && N <= SIM_FEW * SIM_MAX_WG ? SIM_FEW : SIM_MANY; }
+inline int sim_num_wg(int Q, int N) {
+  int nwg = (N + sim_rows(Q, N) - 1) / sim_rows(Q, N);
   if (nwg > SIM_MAX_WG) nwg = SIM_MAX_WG;
   if (nwg < 1) nwg = 1;
   return nwg;
@@ -87,6 +88,7 @@ __device__ __forceinline__ void compact_global(float* gs, int* gr, int* cnt, flo
   }
 }
 
+template <int SIM_THREADS>
 __global__ __launch_bounds__(SIM_THREADS) void cosine_stage1_kernel(
     float* __restrict__ ws_s, int* __restrict__ ws_r, float* __restrict__ cand_s, int* __restrict__ cand_r,
     const bf16* __restrict__ queries, const bf16* __restrict__ index, int Q, int N, int D, int K,
@@ -103,9 +105,14 @@ __global__ __launch_bounds__(SIM_THREADS) void cosine_stage1_kernel(
   uint64_t* qtag = reinterpret_cast<uint64_t*>(minp + SIM_MAXQ);              // [MAXQ]
   int* need = reinterpret_cast<int*>(qtag + SIM_MAXQ);  // [2] some buffer is full, by rounds in turn: a wave that is a
                                                         // round ahead must not be taken for this one's
+  // [waves][16] the filter words of a group's rows (tags, priority, expiry), and [NQT*16][65] the first round's scores
+  uint64_t* tg_lds = reinterpret_cast<uint64_t*>(need + 4);
+  int* pr_lds = reinterpret_cast<int*>(tg_lds + SIM_THREADS / 4);
+  float* ex_lds = reinterpret_cast<float*>(pr_lds + SIM_THREADS / 4);
+  uint32_t* first = reinterpret_cast<uint32_t*>(ex_lds + SIM_THREADS / 4);
 
   const int nwg = gridDim.x, wg = blockIdx.x;
-  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int g = lane >> 4, col = lane & 15;
   for (int v = threadIdx.x; v < NQT * SIM_QT * D / 8; v += SIM_THREADS) {
     const int r = (v * 8) / D, c = (v * 8) % D;
@@ -155,13 +162,19 @@ __global__ __launch_bounds__(SIM_THREADS) void cosine_stage1_kernel(
 
   for (int round = 0; round < nrounds; ++round) {
     const int grp = round * NW + wid;
+    const int gbase = r0 + grp * 16;
+    f32x4 acc[SIM_MAXQ / SIM_QT];
+#pragma unroll
+    for (int t = 0; t < SIM_MAXQ / SIM_QT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
     if (grp < ngroups) {
-      const int gbase = r0 + grp * 16;
       // packed tile gbase/16: k-step m is 64 lanes x 16 B contiguous (1 KiB per wave load)
       const bf16* ap = tile_ptr(grp);
-      f32x4 acc[SIM_MAXQ / SIM_QT];
-#pragma unroll
-      for (int t = 0; t < SIM_MAXQ / SIM_QT; ++t) acc[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+      // the rows' filter words ride along, older than the group's later batches: read where a row is admitted, each was
+      // a load to wait for behind the row stream
+      const int rowc = min(gbase + col, r1 - 1);
+      const int pr = row_prio[rowc];
+      const float ex = row_exp[rowc];
+      const uint64_t tg = row_tags[rowc];
       auto compute = [&](const bf16x8 (&av)[SIM_KB], int m) {
 #pragma unroll
         for (int u = 0; u < SIM_KB; ++u) {
@@ -177,31 +190,76 @@ __global__ __launch_bounds__(SIM_THREADS) void cosine_stage1_kernel(
       };
       for (int m = 0; m < ksteps; m += 2 * SIM_KB) {
         if (m + SIM_KB < ksteps) load_batch(ap, m + SIM_KB, bufB);
+        if (m == 0 && g == 0) {
+          tg_lds[wid * 16 + col] = tg;
+          pr_lds[wid * 16 + col] = pr;
+          ex_lds[wid * 16 + col] = ex;
+        }
         compute(bufA, m);
         if (m + 2 * SIM_KB < ksteps) load_batch(ap, m + 2 * SIM_KB, bufA);
         else if (grp + NW < ngroups) load_batch(tile_ptr(grp + NW), 0, bufA);  // next group's first batch
         if (m + SIM_KB < ksteps) compute(bufB, m + SIM_KB);
       }
-      // lane holds rows gbase + 4g + r for queries t*16 + col
+    }
+    // lane holds rows gbase + 4g + r for queries t*16 + col
+    auto passes = [&](int at, int q) {  // the row's words (its place in the LDS arrays) against a query's filters
+      const float ex = ex_lds[at];
+      return pr_lds[at] >= minp[q] && (tg_lds[at] & qtag[q]) == qtag[q] && (ex == 0.f || ex > now);
+    };
+    if (round == 0) {
+      // The first groups show their best before any row is admitted: of every four rows the best score that passes the
+      // query's filters, whose K-th best is where the query begins. (With all 256 rows admitted for every
+      // query, the first round was most of a small index's pass: 64 queries of 131,000 rows 292 us a lookup, 261 so.)
 #pragma unroll
       for (int t = 0; t < SIM_MAXQ / SIM_QT; ++t) {
+        if (t >= NQT) break;
         const int q = t * SIM_QT + col;
-        if (t >= NQT || q >= Q) continue;
+        uint32_t best = 0;
+        if (grp < ngroups) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = gbase + 4 * g + r;
-          const float sc = acc[t][r];
-          if (row >= r1 || !(sc > theta[q])) continue;
-          if (row_prio[row] < minp[q]) continue;
-          if ((row_tags[row] & qtag[q]) != qtag[q]) continue;
-          const float ex = row_exp[row];
-          if (ex != 0.f && !(ex > now)) continue;
-          const int pos = atomicAdd(&cnt[q], 1);
-          if (pos < SIM_CAND) {
-            my_s[q * SIM_CAND + pos] = sc;
-            my_r[q * SIM_CAND + pos] = row;
+          for (int r = 0; r < 4; ++r)
+            if (gbase + 4 * g + r < r1 && passes(wid * 16 + 4 * g + r, q) && is_finite(acc[t][r])) best = max(best, ord_key(acc[t][r]));
+        }
+        first[q * 65 + wid * 4 + g] = best;
+      }
+      __syncthreads();
+      for (int q = wid; q < Q; q += NW) {
+        const uint32_t key[1] = {lane < NW * 4 ? first[q * 65 + lane] : 0};
+        if (__popcll(__ballot(key[0] != 0)) >= K) {
+          const uint32_t k = wave_select_floor<13>(key, K);
+          // (rows that reach it are admitted: just below it, also where it is 0)
+          if (lane == 0) theta[q] = fminf(key_value(k - 1), key_value(k) - 1e-30f);
+        }
+      }
+      __syncthreads();
+    }
+    if (grp < ngroups) {
+      unsigned reach = 0;  // bit 4 t + r: some lane's score is above its query's threshold
+#pragma unroll
+      for (int t = 0; t < SIM_MAXQ / SIM_QT; ++t) {
+        if (t >= NQT) break;
+        const float th = t * SIM_QT + col < Q ? theta[t * SIM_QT + col] : INFINITY;
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          if (__any(acc[t][r] > th)) reach |= 1u << (4 * t + r);
+      }
+      if (reach) {
+#pragma unroll
+        for (int t = 0; t < SIM_MAXQ / SIM_QT; ++t) {
+          const int q = t * SIM_QT + col;
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            if (!((reach >> (4 * t + r)) & 1u)) continue;
+            const int row = gbase + 4 * g + r;
+            const float sc = acc[t][r];
+            if (row >= r1 || q >= Q || !(sc > theta[q]) || !passes(wid * 16 + 4 * g + r, q)) continue;
+            const int pos = atomicAdd(&cnt[q], 1);
+            if (pos < SIM_CAND) {
+              my_s[q * SIM_CAND + pos] = sc;
+              my_r[q * SIM_CAND + pos] = row;
+            }
+            if (pos == SIM_LIM) need[round & 1] = 1;
           }
-          if (pos == SIM_LIM) need[round & 1] = 1;
         }
       }
     }
@@ -255,7 +313,7 @@ __global__ __launch_bounds__(1024) void cosine_stage2_kernel(float* __restrict__
 // workspace = stage-1 top-k lists [Q][nwg][K] (score, row) + per-(slice, query)
 // candidate buffers [nwg][64][CAND] (score, row)
 extern "C" long long pa_cosine_topk_workspace_bytes(int Q, int N, int K) {
-  const long long w = pa::sim_num_wg(N);
+  const long long w = pa::sim_num_wg(1, N);  // (the most for any number of queries)
   return (long long)Q * w * K * 8 + w * pa::SIM_MAXQ * pa::SIM_CAND * 8;
 }
 
@@ -272,22 +330,23 @@ extern "C" int pa_cosine_topk(float* out_scores, int* out_rows, void* workspace,
     (void)hipMemsetAsync(out_rows, 0xff, (size_t)Q * K * sizeof(int), st);
     return (int)hipGetLastError();
   }
-  const int nwg = pa::sim_num_wg(N);
+  const int nwg = pa::sim_num_wg(Q, N);
   float* ws_s = reinterpret_cast<float*>(workspace);
   int* ws_r = reinterpret_cast<int*>(ws_s + (size_t)Q * nwg * K);
   float* cand_s = reinterpret_cast<float*>(ws_r + (size_t)Q * nwg * K);
   int* cand_r = reinterpret_cast<int*>(cand_s + (size_t)nwg * pa::SIM_MAXQ * pa::SIM_CAND);
-  const int nqt = (Q + pa::SIM_QT - 1) / pa::SIM_QT;
-  const size_t lds = (size_t)nqt * pa::SIM_QT * (D + 8) * 2 + pa::SIM_MAXQ * (4 + 4 + 4 + 8) + 16;
+  const int nqt = (Q + pa::SIM_QT - 1) / pa::SIM_QT, threads = pa::sim_rows(Q, N) * 4;
+  const size_t lds = (size_t)nqt * pa::SIM_QT * (D + 8) * 2 + pa::SIM_MAXQ * (4 + 4 + 4 + 8) + 16 +
+                     threads / 4 * 16 + (size_t)nqt * pa::SIM_QT * 65 * 4;
   static bool attr_set = false;
   if (!attr_set) {
-    (void)hipFuncSetAttribute((const void*)pa::cosine_stage1_kernel,
-                              hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+    for (auto* k : {pa::cosine_stage1_kernel<512>, pa::cosine_stage1_kernel<1024>})
+      (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
     attr_set = true;
   }
-  hipLaunchKernelGGL(pa::cosine_stage1_kernel, dim3(nwg), dim3(pa::SIM_THREADS), lds, st, ws_s, ws_r,
-                     cand_s, cand_r, (const pa::bf16*)queries, (const pa::bf16*)index, Q, N, D, K,
-                     row_priority, row_tags, row_expiry, q_min_priority, q_tags, now);
+  auto* scan = threads == 512 ? pa::cosine_stage1_kernel<512> : pa::cosine_stage1_kernel<1024>;
+  hipLaunchKernelGGL(scan, dim3(nwg), dim3(threads), lds, st, ws_s, ws_r, cand_s, cand_r, (const pa::bf16*)queries,
+                     (const pa::bf16*)index, Q, N, D, K, row_priority, row_tags, row_expiry, q_min_priority, q_tags, now);
   static_assert(pa::SIM_MAX_WG * pa::SIM_MAXK <= 16 * 1024, "stage 2 holds all lists");
   auto* merge = nwg * K <= 1024 ? pa::cosine_stage2_kernel<1>
                                 : nwg * K <= 4096 ? pa::cosine_stage2_kernel<4> : pa::cosine_stage2_kernel<16>;

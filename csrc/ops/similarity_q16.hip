@@ -545,7 +545,7 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
               const float sc = fmaf((float)acc_hh[t][4 * f + r], 65536.f, (float)acc_lh[t][4 * f + r] * 256.f) * (rm.x * sq);
               const float e = fmaf(rm.y, cq, 1e-6f);
               if (gbase + ri < r1 && (ex == 0.f || ex > now) && pr_lds[wid * 32 + ri] >= minp &&
-                  (tg_lds[wid * 32 + ri] & want) == want)
+                  (tg_lds[wid * 32 + ri] & want) == want && is_finite(sc - e))
                 best = max(best, ord_key(sc - e));
             }
             first[q * 65 + (wid * 2 + lh) * 4 + f] = best;

@@ -14,6 +14,9 @@ __device__ __forceinline__ float key_value(uint32_t k) {
   return __uint_as_float((k >> 31) ? k & 0x7fffffffu : ~k);
 }
 
+// (by its bits: the compiler is told that there is nothing else)
+__device__ __forceinline__ bool is_finite(float x) { return (__float_as_uint(x) & 0x7fffffffu) < 0x7f800000u; }
+
 __device__ __forceinline__ uint32_t wave_umin(uint32_t v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v = min(v, (uint32_t)__shfl_xor((int)v, o, 64));

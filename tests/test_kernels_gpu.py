@@ -574,6 +574,36 @@ def test_mid_qkv_rope(gpu, M, H, KV, K, fm, fn, splits):
     torch.testing.assert_close(vc.float().cpu(), rv, atol=3e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("storage", ["bf16", "q16"])
+@pytest.mark.parametrize("N,Q,K", [(100, 3, 64), (20_000, 16, 5), (20_000, 17, 33), (32_768, 16, 32), (32_769, 2, 9), (70_000, 5, 64)])
+def test_lookup_begins_with_its_best(gpu, storage, N, Q, K):
+    """The first round's threshold: rows of nothing but zeros (scores of 0), ties, rows that are not finite (they are never
+    hits, and do not count as the best of their four), few rows that pass, and more queries than a short slice takes."""
+    from pilottai_amd.memory.semantic_index import SemanticIndex
+
+    g = torch.Generator().manual_seed(N + Q)
+    v = torch.randn(N, 64, generator=g)
+    v[N // 3:] = 0.0
+    v[5:9] = v[4]
+    odd = torch.tensor([1, 40, 77])
+    idx = SemanticIndex(dim=64, capacity=N, device=gpu, growable=False, storage=storage)
+    prio, tags = torch.ones(N, dtype=torch.int32), torch.ones(N, dtype=torch.int64)
+    prio[odd] = 0
+    bad = v.clone()
+    bad[odd[0]], bad[odd[1], 3], bad[odd[2]] = float("nan"), float("nan"), float("inf")
+    norm = lambda x: x / x.norm(dim=1, keepdim=True).clamp(min=1e-12)  # noqa: E731
+    q = torch.cat([v[4:5], torch.zeros(1, 64), -v[:1], torch.randn(Q, 64, generator=g)])[:Q].numpy()
+    idx.add_device(norm(bad).to(gpu), prio.to(gpu), tags.to(gpu), normalized=True)
+    got, want = (idx.search(q, K, [p] * Q, [()] * Q) for p in (0, 1))  # (1: the odd rows are filtered out)
+    scores = lambda hits: [[x for _, x in h] for h in hits]  # noqa: E731  (of rows that tie any may be the hits)
+    assert scores(got) == scores(want) and all(len(h) == min(K, N - 3) for h in want)
+    if storage == "bf16":  # (in fixed point they are rows of zeros)
+        assert not any(r in odd.tolist() for h in got for r, _ in h)
+    idx.priority[50:] = -1
+    few = idx.search(q, K, [1] * Q, [()] * Q)
+    assert all({r for r, _ in h} <= set(range(50)) - set(odd.tolist()) and len(h) == min(K, 48) for h in few)
+
+
 def test_semantic_index_packed_storage(gpu):
     """SemanticIndex keeps rows in packed 16-row tiles: scattered and bulk writes
     (aligned and unaligned ranges, ring wrap) read back exactly, and the HIP
