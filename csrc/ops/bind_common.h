@@ -18,7 +18,7 @@ int pa_prefill_gemm(void* y, const void* x, const void* wp, const void* resid, f
                     int* counters, int n_counters, int M, int N, int K, int ldx, int ldy, int ldr, int epi,
                     const float* ss_in, float* ss_out, float* ss_zero, float eps, int full, int splits, int bn,
                     void* q_out, void* k_cache, void* v_cache, const int* positions, const int* slots,
-                    const float* cos_sin, int H, int KV, int kernel_variant, hipStream_t st);
+                    const float* cos_sin, int H, int KV, int kernel_variant, const int* live, hipStream_t st);
 }
 
 namespace {
@@ -106,12 +106,20 @@ bool rows_gemm(at::Tensor y, at::Tensor x, at::Tensor wp) {
   return rc == 0;
 }
 
+const int* opt_live(const c10::optional<at::Tensor>& t, int M) {
+  if (!t.has_value()) return nullptr;
+  check_gpu(*t, "live");
+  check_dtype(*t, at::kInt, "live");
+  TORCH_CHECK(t->numel() >= M, "live must have an entry for every row");
+  return t->data_ptr<int>();
+}
+
 // Large-M projections (csrc/ops/gemm_prefill.hip): 256x256 MFMA tiles on the packed
 // weights with the same epilogues as mid_gemm (0 plain, 1 SwiGLU, 2 residual, 3 rope-perm).
 bool prefill_gemm(at::Tensor y, at::Tensor x, at::Tensor wp, c10::optional<at::Tensor> resid, at::Tensor ws,
                   at::Tensor counters, int64_t epi, c10::optional<at::Tensor> ss_in, c10::optional<at::Tensor> ss_out,
                   c10::optional<at::Tensor> ss_zero, double eps, int64_t full, int64_t splits, int64_t bn,
-                  int64_t variant) {
+                  int64_t variant, c10::optional<at::Tensor> live) {
   check_gpu(wp, "wp"); check_gpu(ws, "ws"); check_gpu(counters, "counters");
   TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1, "x must be a 2-D GPU tensor, unit inner stride");
   TORCH_CHECK(y.is_cuda() && y.dim() == 2 && y.stride(1) == 1, "y must be a 2-D GPU tensor, unit inner stride");
@@ -146,7 +154,7 @@ bool prefill_gemm(at::Tensor y, at::Tensor x, at::Tensor wp, c10::optional<at::T
                                  (int)epi, opt_rows(ss_in, M, "ss_in"), const_cast<float*>(opt_rows(ss_out, M, "ss_out")),
                                  const_cast<float*>(opt_rows(ss_zero, M, "ss_zero")), (float)eps, (int)full,
                                  (int)splits, (int)bn, nullptr, nullptr, nullptr, nullptr, nullptr, nullptr, 0, 0,
-                                 (int)variant, cur_stream());
+                                 (int)variant, opt_live(live, M), cur_stream());
   TORCH_CHECK(rc >= 0, "prefill_gemm launch failed");
   return rc == 0;
 }

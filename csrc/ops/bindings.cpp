@@ -421,7 +421,7 @@ std::vector<int64_t> stream_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t e
 bool prefill_qkv_rope(at::Tensor x, at::Tensor wp, at::Tensor ss_in, double eps, at::Tensor q_out, at::Tensor k_cache,
                       at::Tensor v_cache, at::Tensor positions, at::Tensor slots, at::Tensor cos_sin, int64_t H,
                       int64_t KV, at::Tensor ws, at::Tensor counters, int64_t full, int64_t splits, int64_t bn,
-                      int64_t variant) {
+                      int64_t variant, c10::optional<at::Tensor> live) {
   check_gpu(wp, "wp"); check_gpu(q_out, "q_out"); check_gpu(k_cache, "k_cache"); check_gpu(v_cache, "v_cache");
   check_gpu(positions, "positions"); check_gpu(slots, "slots"); check_gpu(cos_sin, "cos_sin");
   check_gpu(ws, "ws"); check_gpu(counters, "counters");
@@ -450,7 +450,7 @@ bool prefill_qkv_rope(at::Tensor x, at::Tensor wp, at::Tensor ss_in, double eps,
                                  ss_in.data_ptr<float>(), nullptr, nullptr, (float)eps, (int)full, (int)splits,
                                  (int)bn, q_out.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(), positions.data_ptr<int>(),
                                  slots.data_ptr<int>(), cos_sin.data_ptr<float>(), (int)H, (int)KV, (int)variant,
-                                 cur_stream());
+                                 opt_live(live, M), cur_stream());
   TORCH_CHECK(rc >= 0, "prefill_qkv_rope launch failed");
   return rc == 0;
 }
@@ -897,11 +897,11 @@ PYBIND11_MODULE(_C, m) {
   m.def("prefill_gemm", &prefill_gemm, py::arg("y"), py::arg("x"), py::arg("wp"), py::arg("resid"), py::arg("ws"),
         py::arg("counters"), py::arg("epi") = 0, py::arg("ss_in") = py::none(), py::arg("ss_out") = py::none(),
         py::arg("ss_zero") = py::none(), py::arg("eps") = 1e-5, py::arg("full") = -1, py::arg("splits") = 0,
-        py::arg("bn") = 0, py::arg("variant") = -1);
+        py::arg("bn") = 0, py::arg("variant") = -1, py::arg("live") = py::none());
   m.def("prefill_qkv_rope", &prefill_qkv_rope, py::arg("x"), py::arg("wp"), py::arg("ss_in"), py::arg("eps"),
         py::arg("q_out"), py::arg("k_cache"), py::arg("v_cache"), py::arg("positions"), py::arg("slots"),
         py::arg("cos_sin"), py::arg("H"), py::arg("KV"), py::arg("ws"), py::arg("counters"), py::arg("full") = -1,
-        py::arg("splits") = 0, py::arg("bn") = 0, py::arg("variant") = -1);
+        py::arg("splits") = 0, py::arg("bn") = 0, py::arg("variant") = -1, py::arg("live") = py::none());
   m.def("prefill_set_variant", [](int v) { pa_prefill_set_variant(v); });
   m.def("prefill_gemm_plan", &prefill_gemm_plan, py::arg("M"), py::arg("N"), py::arg("K"), py::arg("bn") = 0,
         "default (full tiles, splits, workspace floats, tile width) of prefill_gemm");

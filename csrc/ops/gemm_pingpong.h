@@ -96,6 +96,8 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
   }
   const int mt = tile % A.MT, nt = tile / A.MT;
   const int row0 = mt * 256;
+  if constexpr (!GR)
+    if (no_token(A.live, row0)) return;
   const int nk = kt1 - kt0;  // >= 2 (launcher)
 
   if (A.ss_zero && bid == 0)

@@ -75,7 +75,12 @@ struct Args {
   int xdiv = 1;
   const float* row_w = nullptr;  // by xmap: weight of x's row (gated pair)
   float limit = 0.f, alpha = 0.f, cubic = 0.f, bias = 0.f;
+  // optional, by row: below 0 behind the last token of a step that is padded to the size its graph was captured for. Tiles
+  // of 256 rows that begin there are left out, all slices of a split one alike; the rows they would write keep what was there
+  const int* live = nullptr;
 };
+
+__device__ __forceinline__ bool no_token(const int* live, int row) { return live && live[row] < 0; }
 
 typedef __attribute__((address_space(3))) void lds_t;
 typedef __attribute__((address_space(1))) void gbl_t;
@@ -138,6 +143,7 @@ __global__ __launch_bounds__(512) void prefill_gemm_kernel(const Args A) {
   }
   const int mt = tile % A.MT, nt = tile / A.MT;
   const int row0 = mt * 256;
+  if (no_token(A.live, row0)) return;
   const int nk = kt1 - kt0;
 
   if (A.ss_zero && blockIdx.x == 0)
@@ -389,6 +395,7 @@ __global__ __launch_bounds__(512) void prefill_gemm_n128_kernel(const Args A) {
   }
   const int mt = tile % A.MT, nt = tile / A.MT;
   const int row0 = mt * 256;
+  if (no_token(A.live, row0)) return;
   const int nk = kt1 - kt0;
 
   if (A.ss_zero && blockIdx.x == 0)
@@ -556,6 +563,12 @@ namespace pf {
 constexpr int kPfDefaultVariant = 3;
 static int g_pf_variant = kPfDefaultVariant;
 
+// Tiles without a token are looked for above this many rows. The engine's graphs are 64 rows or less apart up to here, and
+// a whole tile of padding is rare; above they are 1,024 apart. One prompt, us a step (8 layers of each model) before and
+// after: llama 2,101 tokens (3 of 12 row tiles hold none) 9118, 7874; 2,500 9293, 8441; 3,300 11618, 10590; 3,700 (1 of 16)
+// 11919, 11588; mudepel 2,101 4980, 4641; 3,300 6456, 6021. A step without padding is as before (bozupel, 4,096 6395, 6386).
+constexpr int LIVE_MIN_ROWS = 2048;
+
 // Default decomposition: whole tiles while they fill complete rounds of 256 CUs; a
 // remainder of at most half a round is split over K so that the last round is (nearly)
 // full. Measured on MI355X (profiles/r3_prefill_gemm_variants.jsonl): a split slice costs
@@ -614,7 +627,7 @@ extern "C" int pa_prefill_gemm(void* y, const void* x, const void* wp, const voi
                                int ldy, int ldr, int epi, const float* ss_in, float* ss_out, float* ss_zero,
                                float eps, int full, int splits, int bn, void* q_out, void* k_cache, void* v_cache,
                                const int* positions, const int* slots, const float* cos_sin, int H, int KV,
-                               int kernel_variant, hipStream_t st) {
+                               int kernel_variant, const int* live, hipStream_t st) {
   using namespace pa::pf;
   if (M <= 0) return 0;
   if (bn <= 0) bn = pick_bn(M, N);
@@ -650,6 +663,7 @@ extern "C" int pa_prefill_gemm(void* y, const void* x, const void* wp, const voi
          M, N, K, ldx, ldy, ldr, MT, NT, full, S, per, eps, ss_in, ss_out, ss_zero,
          (pa::bf16*)q_out, (pa::bf16*)k_cache, (pa::bf16*)v_cache, positions, slots, cos_sin, H, KV,
          pa::g_handoff_acquire};
+  a.live = M > LIVE_MIN_ROWS ? live : nullptr;
   const int grid = full + (tiles - full) * S;
   // Mixed tail (variant 3, the default, and 8; 9 = without it): full rounds of 256 x 256
   // tiles over the first c1 column tiles,
@@ -742,6 +756,7 @@ __global__ __launch_bounds__(512) void pingpong_grouped_kernel(Args A, const int
   const int b = blockIdx.x, w = (b & 7) * per + (b >> 3);
   if ((b >> 3) >= per || w >= W) return;
   const int4 tl = tiles[w / A.NT];
+  if (no_token(A.live, tl.y)) return;
   A.wp += (size_t)tl.x * wstride;
   A.M = tl.z;
   if (x_div) {
@@ -762,7 +777,7 @@ __global__ __launch_bounds__(512) void pingpong_grouped_kernel(Args A, const int
 extern "C" int pa_expert_tiles(void* y, const void* x, const void* wp, long long wstride, int N, int K, int ldx, int ldy,
                                const int* tiles, int max_tiles, const int* n_tiles, const int* order, int x_div,
                                int out_order, int epi, float limit, float alpha, float cubic, float bias,
-                               const float* row_w, hipStream_t st) {
+                               const float* row_w, const int* live, hipStream_t st) {
   using namespace pa::pf;
   if (K % 64 || K < 128 || N % 128 || ldx % 8 || ldy % 8 || (epi != EP_PLAIN && epi != EP_GLU && epi != EP_RELU2)) return -1;
   if (max_tiles <= 0) return 0;
@@ -776,6 +791,7 @@ extern "C" int pa_expert_tiles(void* y, const void* x, const void* wp, long long
   a.ldy = ldy;
   if (row_w && !x_div) return -1;
   a.row_w = row_w;
+  a.live = live;
   a.limit = limit;
   a.alpha = alpha;
   a.cubic = cubic;

@@ -22,13 +22,14 @@ class PackedLinear:
         self.N, self.K = full.shape
         self.w = ops.pack_decode_weight(full) if dtype == torch.bfloat16 else full
 
-    def __call__(self, x: torch.Tensor) -> torch.Tensor:
+    def __call__(self, x: torch.Tensor, live: Optional[torch.Tensor] = None) -> torch.Tensor:
+        """`live`: see ops.prefill_gemm."""
         if self.w.dim() == 2:
             return F.linear(x, self.w)
         if x.shape[0] <= 64:
             return ops.decode_gemm(x, self.w)
         y = ops.rows_gemm(x, self.w) if ops.rows_gemm_pays(x.shape[0], self.w.shape[0] * 16, x.shape[1]) else None
-        return ops.prefill_gemm(x, self.w) if y is None else y
+        return ops.prefill_gemm(x, self.w, live=live) if y is None else y
 
 
 def pad_heads(w: torch.Tensor, padded: int) -> torch.Tensor:

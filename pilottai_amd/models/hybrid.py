@@ -483,16 +483,16 @@ class MixerBlock:
             out[:, self.cols:].zero_()
 
         def mix():
-            x = self.proj(h)
+            x = self.proj(h, meta.slots)
             each = [lambda m=m, a=a, b=b, c=c: m(x[:, a:], out[:, b:b + m.width], meta, c, room)
                     for m, a, b, c in zip(self.mixers, self.at_in, self.at_out, caches)]
             run(*each, at=1)
 
         def feed():
-            self.mlp.activate(h, out[:, self.at_out[-1]:self.at_out[-1] + self.mlp.fp])
+            self.mlp.activate(h, out[:, self.at_out[-1]:self.at_out[-1] + self.mlp.fp], meta.slots)
         run = side.run if side is not None else lambda *fs, at=0: [f() for f in fs]
         run(mix, *([feed] if self.mlp is not None else []))
-        return self.o(out), 1, None, self.bias
+        return self.o(out, meta.slots), 1, None, self.bias
 
 
 def _pack_gate_up(gate, up, fp: int, dk: int, dtype, device):
@@ -518,7 +518,7 @@ class GatedMLP:
     def tensors(self):
         return [self.w13] + ([self.down.w] if self.down else [])
 
-    def activate(self, h, act):
+    def activate(self, h, act, live=None):
         T = h.shape[0]
         if T not in self._tiles:  # (before graph capture: the capture's warm-up runs come first)
             n = self.w13.numel()
@@ -528,12 +528,12 @@ class GatedMLP:
             self._tiles[T] = (tiles.to(self.device), torch.tensor([len(tiles)], dtype=torch.int32, device=self.device),
                               torch.arange(T, dtype=torch.int32, device=self.device), tm)
         tiles, n, order, tm = self._tiles[T]
-        ops.expert_gemm(h, self.w13, act, tiles, n, order, T, x_div=0, out_order=False, tm=tm, glu=self.spec.act)
+        ops.expert_gemm(h, self.w13, act, tiles, n, order, T, x_div=0, out_order=False, tm=tm, glu=self.spec.act, live=live)
 
     def __call__(self, h, meta: StepMeta):
         act = torch.empty(h.shape[0], self.fp, dtype=self.dtype, device=self.device)
-        self.activate(h, act)
-        return self.down(act), 1, None, None
+        self.activate(h, act, meta.slots)
+        return self.down(act, meta.slots), 1, None, None
 
 
 class PolyMLP:
@@ -548,8 +548,8 @@ class PolyMLP:
         return [self.up.w, self.down.w]
 
     def __call__(self, h, meta: StepMeta):
-        z = self.up(h)[:, :self.down.K]
-        return self.down(ops.poly_norm(z, self.spec.ff, self.act, self.eps)), 1, None, None
+        z = self.up(h, meta.slots)[:, :self.down.K]
+        return self.down(ops.poly_norm(z, self.spec.ff, self.act, self.eps), meta.slots), 1, None, None
 
 
 class ScoredExperts:

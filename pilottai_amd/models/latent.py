@@ -144,7 +144,7 @@ class LatentAttention:
         if m.kv_from is None:
             ops.latent_cache(x[:, self.c_col:], m.q_rank, m.kv_rank, m.rot_dim, self.w_q, self.w_c, cq, pages, self.Rp,
                              meta.positions, meta.slots, self.cos_sin, self.eps)
-        q = self.uq(cq) if self.uq else x
+        q = self.uq(cq, meta.slots) if self.uq else x
         plan, ex, skip = room.expand.get(self.expand_key()), None, None
         if plan is not None:
             ex = Expanded(plan, pages, self.k_rows, self.uv, meta.block_table, q, self.cos_sin, out)

@@ -632,9 +632,11 @@ class LlamaModel:
                     return path, cfg
         return "mid", self._mid_cfg(kind, T)
 
-    def _gemm(self, kind: str, T: int, x, wp, epi: str, **kw):
+    def _gemm(self, kind: str, T: int, x, wp, epi: str, live=None, **kw):
         path, cfg = self._proj_path(kind, T, wp.shape[0] * 16, wp.shape[1] * 32)
         fn = {"pf": ops.prefill_gemm, "stream": ops.stream_gemm}.get(path, ops.mid_gemm)
+        if path == "pf":
+            cfg["live"] = live
         return fn(x, wp, epi, **cfg, **kw)
 
     def _qkv_rope(self, T: int, x, wp, eps, q, k_cache, v_cache, meta, ss_in):
@@ -644,6 +646,8 @@ class LlamaModel:
                                        H, KVh)
         path, cfg = self._proj_path("qkv", T, wp.shape[0] * 16, wp.shape[1] * 32)
         fn = {"pf": ops.prefill_qkv_rope, "stream": ops.stream_qkv_rope}.get(path, ops.mid_qkv_rope)
+        if path == "pf":
+            cfg["live"] = meta.slots
         return fn(x, wp, eps, q, k_cache, v_cache, meta.positions, meta.slots, self.cos_sin, H, KVh,
                   ss_in=ss_in, **cfg)
 
@@ -687,12 +691,12 @@ class LlamaModel:
                 # ss_b was zeroed by the previous down all-reduce (or above), ss_a is zeroed here
                 self.tp.all_reduce_add(self._gemm("o", T, a2, L["wo_p"], "plain"), h, ss=ss_b, ss_zero=ss_a)
             else:  # ss_b was zeroed by the previous down launch (or above)
-                self._gemm("o", T, a2, L["wo_p"], "resid", resid=h, out=h, ss_out=ss_b, ss_zero=ss_a)
-            a = self._gemm("gate_up", T, h, L["w13_p"], "silu", norm=True, eps=eps, ss_in=ss_b)
+                self._gemm("o", T, a2, L["wo_p"], "resid", live=meta.slots, resid=h, out=h, ss_out=ss_b, ss_zero=ss_a)
+            a = self._gemm("gate_up", T, h, L["w13_p"], "silu", live=meta.slots, norm=True, eps=eps, ss_in=ss_b)
             if tp:
                 self.tp.all_reduce_add(self._gemm("down", T, a, L["w2_p"], "plain"), h, ss=ss_a, ss_zero=ss_b)
             else:
-                self._gemm("down", T, a, L["w2_p"], "resid", resid=h, out=h, ss_out=ss_a, ss_zero=ss_b)
+                self._gemm("down", T, a, L["w2_p"], "resid", live=meta.slots, resid=h, out=h, ss_out=ss_a, ss_zero=ss_b)
         if embed is not None:
             self._pool_embed(ops.rmsnorm(h, self.norm, eps), T, embed)
         rows = meta.logit_rows[:num_logit_rows]

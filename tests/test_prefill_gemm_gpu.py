@@ -182,3 +182,47 @@ def test_prefill_gemm_strided_views(gpu, epi):
     odd = torch.zeros(M, N + 4, dtype=torch.bfloat16, device=gpu)[:, 4:]  # 8-byte aligned only
     with pytest.raises(RuntimeError, match="16-byte"):
         ops.prefill_gemm(x, wp, epi, resid=resid, out=odd)
+
+
+@pytest.mark.parametrize("epi", ["plain", "resid", "silu"])
+@pytest.mark.parametrize("M,live,N,K,bn", [(2049, 1, 512, 128, 0), (2304, 2047, 512, 192, 0), (2304, 2048, 1536, 512, 192),
+                                           (2500, 2049, 512, 1024, 128), (3072, 2101, 7168, 256, 0), (4096, 0, 512, 128, 256)])
+def test_prefill_tiles_without_a_token(gpu, M, live, N, K, bn, epi):
+    """Whole tiles of 256 rows behind the last token stay as they were, on every tile width, in split tiles and in a mixed
+    tail; all other rows are those of a launch that knows of no padding."""
+    g = torch.Generator().manual_seed(M + N)
+    x = torch.randn(M, K, generator=g).to(gpu, torch.bfloat16)
+    w = (torch.randn(N, K, generator=g) * K ** -0.5).to(gpu, torch.bfloat16)
+    slots = torch.arange(M, dtype=torch.int32)
+    slots[live:] = -1
+    NO = N // 2 if epi == "silu" else N
+    kw = dict(bn=bn, resid=torch.randn(M, N, generator=g).to(gpu, torch.bfloat16) if epi == "resid" else None)
+    wp = ops.pack_decode_weight(w)
+    want = ops.prefill_gemm(x, wp, epi, **kw)
+    got = torch.full((M, NO), 7.0, device=gpu, dtype=torch.bfloat16)
+    ops.prefill_gemm(x, wp, epi, out=got, live=slots.to(gpu), **kw)
+    edge = (live + 255) // 256 * 256
+    assert torch.equal(got[:edge], want[:edge])
+    assert (got[edge:] == 7.0).all()
+    ops.prefill_gemm(x, wp, epi, out=got, **kw)  # (tickets of tiles left out are as they were)
+    assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("T,live", [(700, 300), (512, 256), (257, 256), (300, 0)])
+def test_dense_unit_tiles_without_a_token(gpu, T, live):
+    """The same of the gated unit's tiles of 256 rows (one group)."""
+    g = torch.Generator().manual_seed(T)
+    x = torch.randn(T, 256, generator=g).to(gpu, torch.bfloat16)
+    w = (torch.randn(1, 512, 256, generator=g) / 16).to(gpu, torch.bfloat16)
+    wp = ops.pack_groups(w, torch.bfloat16)
+    tiles = torch.tensor([[0, i, min(256, T - i), 0] for i in range(0, T, 256)], dtype=torch.int32, device=gpu)
+    n = torch.tensor([len(tiles)], dtype=torch.int32, device=gpu)
+    order = torch.arange(T, dtype=torch.int32, device=gpu)
+    slots = torch.where(order < live, order, -1)
+
+    def run(**kw):
+        out = torch.full((T, 256), 7.0, device=gpu, dtype=torch.bfloat16)
+        return ops.expert_gemm(x, wp, out, tiles, n, order, T, x_div=0, out_order=False, tm=256, glu=(3e38, 1.0, 0.0), **kw)
+    want, got, edge = run(), run(live=slots.to(torch.int32)), (live + 255) // 256 * 256
+    assert torch.equal(got[:edge], want[:edge])
+    assert (got[edge:] == 7.0).all()
