@@ -495,6 +495,11 @@ class MixerBlock:
         return self.o(out, meta.slots), 1, None, self.bias
 
 
+def _live(meta: Optional[StepMeta]):
+    """What tells padding rows (see ops.prefill_gemm); None outside an engine's step."""
+    return None if meta is None else meta.slots
+
+
 def _pack_gate_up(gate, up, fp: int, dk: int, dtype, device):
     g = torch.zeros(2, 1, fp, dk, dtype=dtype, device=device)
     f, d = gate.shape
@@ -532,8 +537,9 @@ class GatedMLP:
 
     def __call__(self, h, meta: StepMeta):
         act = torch.empty(h.shape[0], self.fp, dtype=self.dtype, device=self.device)
-        self.activate(h, act, meta.slots)
-        return self.down(act, meta.slots), 1, None, None
+        live = _live(meta)
+        self.activate(h, act, live)
+        return self.down(act, live), 1, None, None
 
 
 class PolyMLP:
@@ -548,8 +554,9 @@ class PolyMLP:
         return [self.up.w, self.down.w]
 
     def __call__(self, h, meta: StepMeta):
-        z = self.up(h, meta.slots)[:, :self.down.K]
-        return self.down(ops.poly_norm(z, self.spec.ff, self.act, self.eps), meta.slots), 1, None, None
+        live = _live(meta)
+        z = self.up(h, live)[:, :self.down.K]
+        return self.down(ops.poly_norm(z, self.spec.ff, self.act, self.eps), live), 1, None, None
 
 
 class ScoredExperts:
