@@ -7,8 +7,8 @@
 extern "C" {
 int pa_residual_norm(int fp32, float* resid, const void* y, int K, int ldy, float y_scale, const float* w_post,
                      const void* emb, const int* ids, int vocab, int emb_add, const float* mix, float* hist,
-                     long long hist_step, int n_hist, const float* w_next, void* out, int ldo, const int* rows, int n, int D,
-                     int post_groups, int next_groups, float eps, hipStream_t st);
+                     long long hist_step, int n_hist, const float* w_next, void* out, int ldo, const int* rows, const int* live,
+                     int n, int D, int post_groups, int next_groups, float eps, hipStream_t st);
 int pa_latent_cache(int fp32, const void* x, int ldx, int NQ, int R, int r, int rd, const float* w_q, const float* w_c,
                     void* cq, int ldq, void* pages, int Rp, int D, const int* positions, const int* slots,
                     const float* cos_sin, float eps, int T, hipStream_t st);
@@ -27,7 +27,8 @@ int pa_latent_expand(const pa::la::Expand* X, const void* pages, const void* wk,
 namespace {
 
 void residual_norm(at::Tensor resid, Opt y, int64_t K, double y_scale, Opt w_post, Opt emb, Opt ids, bool emb_add,
-                   Opt w_next, Opt out, Opt rows, double eps, int64_t post_groups, int64_t next_groups, Opt mix, Opt hist) {
+                   Opt w_next, Opt out, Opt rows, double eps, int64_t post_groups, int64_t next_groups, Opt mix, Opt hist,
+                   Opt live) {
   check_gpu(resid, "resid");
   check_dtype(resid, at::kFloat, "resid");
   TORCH_CHECK(resid.dim() == 2, "resid must be [T, D]");
@@ -67,7 +68,8 @@ void residual_norm(at::Tensor resid, Opt y, int64_t K, double y_scale, Opt w_pos
                             emb.has_value() ? ints(*ids, T, "ids") : nullptr, emb.has_value() ? emb->size(0) : 0,
                             emb_add ? 1 : 0, opt_f32(mix, 2, "mix"), n_hist ? hist->data_ptr<float>() : nullptr, hist_step,
                             n_hist, opt_f32(w_next, D, "w_next"), out.has_value() ? out->data_ptr() : nullptr,
-                            ldo, rows.has_value() ? ints(*rows, n, "rows") : nullptr, (int)n, (int)D, (int)post_groups,
+                            ldo, rows.has_value() ? ints(*rows, n, "rows") : nullptr,
+                            live.has_value() ? ints(*live, T, "live") : nullptr, (int)n, (int)D, (int)post_groups,
                             (int)next_groups, (float)eps, cur_stream()),
            "residual_norm");
 }

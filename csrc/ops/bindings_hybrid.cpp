@@ -8,7 +8,7 @@
 extern "C" {
 int pa_hyper_norm(int fp32, float* x, int S, const void* y, int K, int ldy, const float* y_w, const void* y2, int ldy2,
                   const float* bias, const float* mix, const float* post, const float* pre, const void* emb, const int* ids, int vocab,
-                  const float* w_next, void* out, int ldo, const int* rows, int n, int D, float eps, hipStream_t st);
+                  const float* w_next, void* out, int ldo, const int* rows, const int* live, int n, int D, float eps, hipStream_t st);
 int pa_softcap(int fp32, void* x, int ld, int rows, int cols, float cap, hipStream_t st);
 int pa_paged_kv(int fp32, const void* x, const float* bias, void* q, void* kp, void* vp, void* pk, void* pv,
                 const int* positions, const int* slots, const int* q_start, const int* q_len, const int* ctx_len,
@@ -45,7 +45,7 @@ int64_t seqs_of(const at::Tensor& block_table) {
 }
 
 void hyper_norm(at::Tensor x, Opt y, int64_t K, Opt y_w, Opt y2, Opt bias, Opt mix, Opt post, Opt pre, Opt emb, Opt ids,
-                Opt w_next, Opt out, Opt rows, double eps) {
+                Opt w_next, Opt out, Opt rows, double eps, Opt live) {
   check_gpu(x, "x");
   check_dtype(x, at::kFloat, "x");
   TORCH_CHECK(x.dim() == 3, "x must be [T, streams, D]");
@@ -81,7 +81,8 @@ void hyper_norm(at::Tensor x, Opt y, int64_t K, Opt y_w, Opt y2, Opt bias, Opt m
                          opt_f32(post, S, "post"), opt_f32(pre, S, "pre"), emb.has_value() ? emb->data_ptr() : nullptr,
                          emb.has_value() ? ints(*ids, T, "ids") : nullptr, emb.has_value() ? emb->size(0) : 0,
                          opt_f32(w_next, D, "w_next"), out.has_value() ? out->data_ptr() : nullptr, ldo,
-                         rows.has_value() ? ints(*rows, n, "rows") : nullptr, (int)n, (int)D, (float)eps, cur_stream()),
+                         rows.has_value() ? ints(*rows, n, "rows") : nullptr, live.has_value() ? ints(*live, T, "live") : nullptr, (int)n,
+                         (int)D, (float)eps, cur_stream()),
            "hyper_norm");
 }
 

@@ -33,6 +33,7 @@ struct Args {
   const float* w_next;
   void* out;
   const int* rows;
+  const int* live;      // by row: below 0 from the first row without a token on (with rows: not looked at)
   long long hist_step;  // elements from one X to the next
   int K, ldy, vocab, emb_add, n_hist, ldo, D, post_groups, next_groups;
   float y_scale, eps;
@@ -77,6 +78,7 @@ struct GroupNorm {
 template <typename T, int VEC, bool WHOLE>
 __global__ __launch_bounds__(256) void residual_norm_kernel(const Args A) {
   extern __shared__ __attribute__((aligned(16))) float row[];  // [D], slots, groups' factors
+  if (A.live && A.live[blockIdx.x] < 0) return;
   const int D = A.D, t = A.rows ? A.rows[blockIdx.x] : blockIdx.x;
   float* rr = A.resid + (size_t)t * D;
   float* slots = row + (D + 3) / 4 * 4;
@@ -184,6 +186,7 @@ __global__ __launch_bounds__(256) void residual_norm_wave_kernel(const Args A, i
   __shared__ float slots[W > 1 ? R : 1][W > 1 ? W * NV : 1];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, w = wid % W, r = wid / W;
   const int b = blockIdx.x * R + r, D = A.D;
+  if (A.live && A.live[blockIdx.x * R] < 0) return;  // (whole workgroups)
   if (W == 1 && b >= n) return;  // (whole waves; with W > 1 all take the barriers)
   const int t = A.rows ? A.rows[min(b, n - 1)] : min(b, n - 1);
   auto at = [&](int s) { return ((s * W + w) * 64 + lane) * 8; };
@@ -344,13 +347,15 @@ __global__ __launch_bounds__(256) void residual_norm_wave_kernel(const Args A, i
 extern "C" int pa_residual_norm(int fp32, float* resid, const void* y, int K, int ldy, float y_scale,
                                 const float* w_post, const void* emb, const int* ids, int vocab, int emb_add,
                                 const float* mix, float* hist, long long hist_step, int n_hist, const float* w_next,
-                                void* out, int ldo, const int* rows, int n, int D, int post_groups, int next_groups,
-                                float eps, hipStream_t st) {
+                                void* out, int ldo, const int* rows, const int* live, int n, int D, int post_groups,
+                                int next_groups, float eps, hipStream_t st) {
   using namespace pa::rn;
   if (n <= 0) return 0;
   if (D <= 0 || D * 4 > 96 * 1024) return -1;  // the row in LDS
   if (post_groups < 1 || next_groups < 1 || D % post_groups || D % next_groups || (mix && (!emb || !hist || n_hist < 1))) return -1;
-  const Args A{resid, y, w_post, emb, ids, mix, hist, w_next, out, rows, hist_step, K, ldy, vocab, emb_add, n_hist, ldo, D,
+  // Rows without a token stay as they are above 2,048 rows, where the steps that graphs are captured for are 1,024 apart
+  if (rows || n <= 2048) live = nullptr;
+  const Args A{resid, y, w_post, emb, ids, mix, hist, w_next, out, rows, live, hist_step, K, ldy, vocab, emb_add, n_hist, ldo, D,
                post_groups, next_groups, y_scale, eps};
   // whole 8s, and groups that are lanes of a wave (a power of two) or whole wave steps
   auto lanes = [&](int g) { const int len = D / g, l = len / 8; return g == 1 || len % 512 == 0 || (len % 8 == 0 && l <= 64 && (l & (l - 1)) == 0); };

@@ -338,13 +338,14 @@ class BozupelModel:
             keys = {L["attn"].expand_key() for L in self.layers} - {None}
             room = room._replace(expand={k: ExpandPlan(meta, T, *k) for k in keys})
         resid = torch.empty(T, d, dtype=torch.float32, device=dev)
-        h = ops.residual_norm(resid, eps, emb=self.embed, ids=ids, w_next=self.layers[self.runs[0][0]]["norm1"], out=new_h())
+        h = ops.residual_norm(resid, eps, emb=self.embed, ids=ids, w_next=self.layers[self.runs[0][0]]["norm1"], out=new_h(),
+                              live=meta.slots)
         for j, (i, _) in enumerate(self.runs):
             L = self.layers[i]
             y, *_ = L["block"](h, meta, [(kv.pages[j],)], room)
             post, k = L["norm1b"], 1
             if L["mlp"] is not None:
-                h = ops.residual_norm(resid, eps, y=y, w_post=post, w_next=L["norm2"], out=new_h())
+                h = ops.residual_norm(resid, eps, y=y, w_post=post, w_next=L["norm2"], out=new_h(), live=meta.slots)
                 y = L["mlp"](h, T, routes[L["route"]])
                 post, k = L["norm2b"], L["mlp"].spec.top
             step = dict(y=y, partials=k, y_scale=1.0 / k, w_post=post)
@@ -356,7 +357,7 @@ class BozupelModel:
                 nxt, again = self.runs[j + 1]
                 if again:
                     step.update(emb=self.embed, ids=ids, emb_add=True)
-                h = ops.residual_norm(resid, eps, w_next=self.layers[nxt]["norm1"], out=new_h(), **step)
+                h = ops.residual_norm(resid, eps, w_next=self.layers[nxt]["norm1"], out=new_h(), live=meta.slots, **step)
         if embed is not None:
             hn = ops.residual_norm(resid, eps, w_next=self.norm, out=new_h(), **step)
             pool_rows, pool = embed

@@ -227,10 +227,10 @@ class MudepelModel(HybridModel):
         step, room = dict(emb=self.embed, ids=meta.input_ids[:T]), self.room(part_o, part_ml)
         for j, i in enumerate(self.runs):
             L = self.layers[i]
-            h = ops.hyper_norm(x, eps, pre=L["hc1"]["in"], w_next=L["norm1"], out=new_h(), **step)
+            h = ops.hyper_norm(x, eps, pre=L["hc1"]["in"], w_next=L["norm1"], out=new_h(), live=meta.slots, **step)
             step = self._into_streams(L["mixer"](h, meta, kv.layers[j], room), L["hc1"])
             if L["mlp"] is not None:
-                h = ops.hyper_norm(x, eps, pre=L["hc2"]["in"], w_next=L["norm2"], out=new_h(), **step)
+                h = ops.hyper_norm(x, eps, pre=L["hc2"]["in"], w_next=L["norm2"], out=new_h(), live=meta.slots, **step)
                 step = self._into_streams(L["mlp"](h, meta), L["hc2"])
             if residuals is not None:
                 after = x.clone()

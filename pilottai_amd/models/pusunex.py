@@ -274,15 +274,15 @@ class PusunexModel(HybridModel):
         token = dict(emb=self.embed, ids=ids)
         step = dict(token)
         for i, L in enumerate(self.layers):
-            h = ops.residual_norm(resid, eps, w_next=L["norm1"], next_groups=G, out=new_h(), **step)
+            h = ops.residual_norm(resid, eps, w_next=L["norm1"], next_groups=G, out=new_h(), live=meta.slots, **step)
             y, *_ = L["mixer"](h, meta, kv.layers[i], room)
             step = dict(y=y, w_post=L["norm1b"], post_groups=G)
             if L["mlp"] is not None:
-                h = ops.residual_norm(resid, eps, w_next=L["norm2"], next_groups=G, out=new_h(), **step)
+                h = ops.residual_norm(resid, eps, w_next=L["norm2"], next_groups=G, out=new_h(), live=meta.slots, **step)
                 y, k, _, _ = L["mlp"](h, meta)
                 step = dict(y=y, partials=k, w_post=L["norm2b"], post_groups=G)
             if L["side"]:
-                x = ops.residual_norm(resid, eps, out=new_h(), **step)
+                x = ops.residual_norm(resid, eps, out=new_h(), live=meta.slots, **step)
                 step = dict(y=L["side"](x, self.side, ids), w_post=L["side"].norm)
             step.update(mix=L["dwa"], hist=hist, **token)
             if residuals is not None:

@@ -245,7 +245,7 @@ class SalipelModel(HybridModel):
         room = self.room(part_o, part_ml)
         step = dict(emb=self.embed, ids=meta.input_ids[:T])
         for i, L in enumerate(self.layers):
-            h = ops.hyper_norm(x, eps, pre=self.one, w_next=L["norm"], out=new_h(), **step)
+            h = ops.hyper_norm(x, eps, pre=self.one, w_next=L["norm"], out=new_h(), live=meta.slots, **step)
             side = self.side if T <= self.SIDE_MAX_T else None
             mixer, mlp = lambda: L["mixer"](h, meta, kv.layers[i], room, side), lambda: L["mlp"](h, meta)  # noqa: E731, B023
             both = [mixer] + ([mlp] if L["mlp"] is not None else [])

@@ -42,13 +42,15 @@ def hyper_norm(x: torch.Tensor, eps: float, *, y: Optional[torch.Tensor] = None,
                bias: Optional[torch.Tensor] = None, mix: Optional[torch.Tensor] = None, post: Optional[torch.Tensor] = None,
                pre: Optional[torch.Tensor] = None, emb: Optional[torch.Tensor] = None,
                ids: Optional[torch.Tensor] = None, w_next: Optional[torch.Tensor] = None,
-               out: Optional[torch.Tensor] = None, rows: Optional[torch.Tensor] = None):
+               out: Optional[torch.Tensor] = None, rows: Optional[torch.Tensor] = None,
+               live: Optional[torch.Tensor] = None):
     """x (fp32 [T, streams, D], in place): x_t = sum_s mix[s, t] x_s + post[t] (sum_k w_k y_k + y2 + bias), or
     x_t = emb[ids]; out = norm(sum_s pre[s] x_s) * w_next. Returns out. `rows`: out row i is row rows[i]'s,
-    and x keeps its value."""
+    and x keeps its value. `live` (ints by row, without `rows`): rows from the first one below 0 on are padding and may be
+    left as they were."""
     if _on_gpu(x):
         require_hybrid().hyper_norm(x, y, int(partials), y_weights, y2, bias, mix, post, pre, emb, ids, w_next, out, rows,
-                                    float(eps))
+                                    float(eps), live)
         return out
     return ref.hyper_norm(x, eps, y, partials, y_weights, y2, bias, mix, post, pre, emb, ids, w_next, out, rows)
 

@@ -35,15 +35,17 @@ def residual_norm(resid: torch.Tensor, eps: float, *, y: Optional[torch.Tensor] 
                   y_scale: float = 1.0, w_post: Optional[torch.Tensor] = None, emb: Optional[torch.Tensor] = None,
                   ids: Optional[torch.Tensor] = None, emb_add: bool = False, w_next: Optional[torch.Tensor] = None,
                   out: Optional[torch.Tensor] = None, rows: Optional[torch.Tensor] = None, post_groups: int = 1,
-                  next_groups: int = 1, mix: Optional[torch.Tensor] = None, hist: Optional[torch.Tensor] = None):
+                  next_groups: int = 1, mix: Optional[torch.Tensor] = None, hist: Optional[torch.Tensor] = None,
+                  live: Optional[torch.Tensor] = None):
     """resid (fp32 [T, D], in place) += norm(y_scale * sum of a token's `partials` rows of y) * w_post
     (w_post None: without the norm), then += emb[ids] (emb_add) or = emb[ids]; out = norm(resid) * w_next (w_next
     None: resid as it is). The norms are of `post_groups` and `next_groups` equal parts of a row. Depth average, with
     mix [n + 1]: resid joins hist (fp32 [n, T, D]) as its last entry, and becomes mix[0] emb[ids] + sum_j mix[j]
-    hist[j - 1]. Returns out. `rows`: out row i is row rows[i]'s, and resid and hist keep their values."""
+    hist[j - 1]. Returns out. `rows`: out row i is row rows[i]'s, and resid and hist keep their values. `live`
+    (ints by row, without `rows`): rows from the first one below 0 on are padding and may be left as they were."""
     if _on_gpu(resid):
         require_latent().residual_norm(resid, y, int(partials), float(y_scale), w_post, emb, ids, bool(emb_add),
-                                       w_next, out, rows, float(eps), int(post_groups), int(next_groups), mix, hist)
+                                       w_next, out, rows, float(eps), int(post_groups), int(next_groups), mix, hist, live)
         return out
     return ref.residual_norm(resid, eps, y, partials, y_scale, w_post, emb, ids, emb_add, w_next, out, rows, post_groups,
                              next_groups, mix, hist)

@@ -67,6 +67,26 @@ def test_hyper_norm_of_few_wide_rows(gpu, S, D):
     test_hyper_norm(gpu, BF16, S, D, 2, False)
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,live,S,D", [(2049, 1, 4, 256), (2500, 2047, 2, 100), (2304, 0, 1, 1280)])
+def test_hyper_norm_leaves_rows_without_a_token(gpu, T, live, S, D):
+    from pilottai_amd import ops
+
+    g = gen(T)
+    x, y, w = (torch.randn(*s, generator=g).to(gpu) for s in ((T, S, D), (T, D), (D,)))
+    mix, post, pre = (torch.randn(*s, generator=g).to(gpu) for s in ((S, S), (S,), (S,)))
+    slots = torch.arange(T, dtype=torch.int32, device=gpu)
+    slots[live:] = -1
+
+    def run(**kw):
+        xs, out = x.clone(), torch.full((T, D), 7.0, dtype=BF16, device=gpu)
+        ops.hyper_norm(xs, 1e-5, y=y.to(BF16), mix=mix, post=post, pre=pre, w_next=w, out=out, **kw)
+        return xs, out
+    (xa, a), (xb, b) = run(), run(live=slots)
+    assert torch.equal(xa[:live], xb[:live]) and torch.equal(a[:live], b[:live])
+    assert torch.equal(xb[live:], x[live:]) and (b[live:] == 7.0).all()
+
+
 @kinds
 def test_softcap(device, dt):
     from pilottai_amd import ops

@@ -48,6 +48,25 @@ def test_residual_norm(gpu, dt, D, K, add):
     torch.testing.assert_close(out.float().cpu()[:, :D], norm(want, wn, eps), **tol(dt))
 
 
+@pytest.mark.parametrize("T,live,D", [(2049, 1, 512), (2500, 2046, 1024), (2304, 3, 2048), (2050, 2049, 4096), (2100, 77, 100)])
+def test_residual_norm_leaves_rows_without_a_token(gpu, T, live, D):
+    """One, two and four waves a row and widths that are no whole 8s; a workgroup with a token does all of its rows."""
+    from pilottai_amd import ops
+
+    g = torch.Generator().manual_seed(T)
+    r, y, w = (torch.randn(*s, generator=g).to(gpu) for s in ((T, D), (T, D), (D,)))
+    slots = torch.arange(T, dtype=torch.int32, device=gpu)
+    slots[live:] = -1
+
+    def run(**kw):
+        rg, out = r.clone(), torch.full((T, D), 7.0, dtype=torch.bfloat16, device=gpu)
+        ops.residual_norm(rg, 1e-5, y=y.to(torch.bfloat16), w_post=w, w_next=w, out=out, **kw)
+        return rg, out
+    (ra, a), (rb, b), edge = run(), run(live=slots), (live + 3) // 4 * 4
+    assert torch.equal(ra[:live], rb[:live]) and torch.equal(a[:live], b[:live])
+    assert torch.equal(rb[edge:], r[edge:]) and (b[edge:] == 7.0).all()
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("T", [1, 40, 130])
 @pytest.mark.parametrize("G,N,K", [(3, 48, 32), (5, 208, 96), (2, 512, 128)])
