@@ -155,7 +155,9 @@ __global__ __launch_bounds__(512) void stage1_exact_kernel(
   signed char* qh = reinterpret_cast<signed char*>(smem);           // [NQT*16][QLD]
   signed char* ql = qh + (size_t)NQT * QT * QLD;                    // [NQT*16][QLD]
   QState& st = *reinterpret_cast<QState*>(ql + (size_t)NQT * QT * QLD);
-  int* need = reinterpret_cast<int*>(&st + 1);  // as in the bound scan
+  // [2] some query's buffer must be compacted, by rounds in turn: a wave that is a round ahead must not be taken for this
+  // one's (the others would miss its barrier)
+  int* need = reinterpret_cast<int*>(&st + 1);
 
   const int nwg = gridDim.x, wg = blockIdx.x;
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -352,9 +354,7 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
   signed char* qh = reinterpret_cast<signed char*>(smem);  // [ROWS][QLD]
   signed char* ql = qh + (size_t)ROWS * QLD;                // [ROWS][QLD]
   QState& st = *reinterpret_cast<QState*>(ql + (size_t)ROWS * QLD);
-  // [2] some query's buffer must be compacted, by rounds in turn: a wave that is a round ahead must not be taken for this
-  // one's (the others would miss its barrier)
-  int* need = reinterpret_cast<int*>(&st + 1);
+  int* need = reinterpret_cast<int*>(&st + 1);  // [0] some query's buffer must be compacted, [1] waves that are done
   // [NWV][32] per group row: (s_r, b_r), then the filter words (priority, expiry, tags)
   float2* rm_lds = reinterpret_cast<float2*>(need + 4);
   int* pr_lds = reinterpret_cast<int*>(rm_lds + NWV * 32);
@@ -623,6 +623,9 @@ __global__ __launch_bounds__(512) void stage1_bound_kernel(
         }
       }
       // (LDS only: the row loads stay in flight)
+      // Round 1 begins with a barrier of its own: a wave that waits there must not meet others in a compaction's. So no wave
+      // leaves round 0 before all have admitted its rows, and all find the same flag. Later rounds have no other barrier.
+      if (round == 0) lds_barrier();
       if (flag(0)) compact_all();
       if (pub && publishes(round) && threadIdx.x < Q)
         __hip_atomic_store(pub + threadIdx.x * nwg + wg, st.top[threadIdx.x], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);

@@ -77,7 +77,8 @@ def test_q16_slices_and_shared_bounds(gpu, N, D, Q, K, filters):
 
 
 @pytest.mark.parametrize("N,D,Q,K", [  # one tile of queries and two, whole steps of dimensions and padded ones, slices of one round
-    (65_536, 512, 32, 64), (65_537, 448, 33, 1), (66_000, 1024, 1, 16), (131_073, 960, 64, 8), (400_000, 192, 32, 17)])
+    (65_536, 512, 32, 64), (65_537, 448, 33, 1), (66_000, 1024, 1, 16), (131_073, 960, 64, 8), (400_000, 192, 32, 17),
+    (300_000, 128, 33, 64)])  # (whose first round fills buffers)
 def test_q16_tiles_of_queries(gpu, N, D, Q, K):
     _check(gpu, N, D, Q, K, True, seed=3)
 
