@@ -35,12 +35,13 @@ struct Args {
   float eps;
 };
 
-template <typename T, int VEC, int S, int NW>
+// LIVE: with `live` (bf16 rows of whole 4s, the others do all rows)
+template <typename T, int VEC, int S, int NW, bool LIVE = false>
 __global__ __launch_bounds__(64 * NW) void hyper_norm_kernel(const Args A) {
   constexpr int NT = 64 * NW;
   extern __shared__ __attribute__((aligned(16))) float row[];
   __shared__ float red[NW];
-  if (A.live && A.live[blockIdx.x] < 0) return;
+  if (LIVE && A.live[blockIdx.x] < 0) return;
   const int t = A.rows ? A.rows[blockIdx.x] : blockIdx.x, D = A.D;
   float* xr = A.x + (size_t)t * S * D;
   float mix[S][S], post[S], pre[S];
@@ -158,21 +159,23 @@ extern "C" int pa_hyper_norm(int fp32, float* x, int S, const void* y, int K, in
   // 6.8 -> 5.7 us)
   const bool few = n <= 256 && D > 1024;
   const bool vec = D % 4 == 0 && (!y || ldy % 4 == 0) && (!y2 || ldy2 % 4 == 0) && (!out || ldo % 4 == 0);
-#define PA_HN(T, V, N, W)                                                                                       \
+#define PA_HN(T, V, N, W, ...)                                                                                  \
   do {                                                                                                          \
     static bool attr = false;                                                                                   \
     if (!attr) {                                                                                                \
-      (void)hipFuncSetAttribute((const void*)hyper_norm_kernel<T, V, N, W>,                                     \
+      (void)hipFuncSetAttribute((const void*)hyper_norm_kernel<T, V, N, W __VA_OPT__(,) __VA_ARGS__>,           \
                                 hipFuncAttributeMaxDynamicSharedMemorySize, 96 * 1024);                         \
       attr = true;                                                                                              \
     }                                                                                                           \
-    hipLaunchKernelGGL((hyper_norm_kernel<T, V, N, W>), dim3(n), dim3(64 * W), (size_t)D * 4, st, A);           \
+    hipLaunchKernelGGL((hyper_norm_kernel<T, V, N, W __VA_OPT__(,) __VA_ARGS__>), dim3(n), dim3(64 * W),        \
+                       (size_t)D * 4, st, A);                                                                   \
   } while (0)
 #define PA_HN_S(N)                                                             \
   case N:                                                                      \
     if (fp32) { if (vec) PA_HN(float, 4, N, 4); else PA_HN(float, 1, N, 4); }  \
     else if (!vec) PA_HN(pa::bf16, 1, N, 4);                                   \
     else if (few) PA_HN(pa::bf16, 4, N, 8);                                    \
+    else if (live) PA_HN(pa::bf16, 4, N, 4, true);                             \
     else PA_HN(pa::bf16, 4, N, 4);                                             \
     break
   switch (S) {

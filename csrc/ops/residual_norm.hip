@@ -179,14 +179,15 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(const Args A) {
 }
 
 // The same for rows of whole 8s whose groups are whole wave steps of 512 elements or a power of two of lanes: W waves a row
-// (4 / W rows a workgroup), NV vectors a thread in registers, all of a row's loads ahead of the first sum.
-template <typename T, int W, int NV>
+// (4 / W rows a workgroup), NV vectors a thread in registers, all of a row's loads ahead of the first sum. LIVE: with `live`
+// (a kernel of its own, so that the launches of small steps, 5 us each, wait for no load more).
+template <typename T, int W, int NV, bool LIVE>
 __global__ __launch_bounds__(256) void residual_norm_wave_kernel(const Args A, int n) {
   constexpr int R = 4 / W;
   __shared__ float slots[W > 1 ? R : 1][W > 1 ? W * NV : 1];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6, w = wid % W, r = wid / W;
   const int b = blockIdx.x * R + r, D = A.D;
-  if (A.live && A.live[blockIdx.x * R] < 0) return;  // (whole workgroups)
+  if (LIVE && A.live[blockIdx.x * R] < 0) return;  // (whole workgroups)
   if (W == 1 && b >= n) return;  // (whole waves; with W > 1 all take the barriers)
   const int t = A.rows ? A.rows[min(b, n - 1)] : min(b, n - 1);
   auto at = [&](int s) { return ((s * W + w) * 64 + lane) * 8; };
@@ -363,7 +364,8 @@ extern "C" int pa_residual_norm(int fp32, float* resid, const void* y, int K, in
   if (D % 8 == 0 && ldy % 8 == 0 && ldo % 8 == 0 && lanes(post_groups) && lanes(next_groups) && steps <= 16) {
     // many rows: as few waves a row as hold it in 4 vectors a thread; few: 4 waves
     const int w = n >= 1024 ? (steps <= 4 ? 1 : steps <= 8 ? 2 : 4) : 4, nv = (steps + w - 1) / w;
-#define PA_RW(T, W, N) hipLaunchKernelGGL((residual_norm_wave_kernel<T, W, N>), dim3((n + 4 / W - 1) / (4 / W)), dim3(256), 0, st, A, n)
+#define PA_RW_L(T, W, N, L) hipLaunchKernelGGL((residual_norm_wave_kernel<T, W, N, L>), dim3((n + 4 / W - 1) / (4 / W)), dim3(256), 0, st, A, n)
+#define PA_RW(T, W, N) do { if (live) PA_RW_L(T, W, N, true); else PA_RW_L(T, W, N, false); } while (0)
 #define PA_RW_N(T, W)                       \
   do {                                      \
     if (nv == 1) PA_RW(T, W, 1);            \
@@ -375,6 +377,7 @@ extern "C" int pa_residual_norm(int fp32, float* resid, const void* y, int K, in
 #undef PA_RW_T
 #undef PA_RW_N
 #undef PA_RW
+#undef PA_RW_L
     return (int)hipGetLastError();
   }
   const int most = post_groups > next_groups ? post_groups : next_groups;
