@@ -1035,15 +1035,18 @@ __device__ __forceinline__ void expanded_unit(const Args& A, const int4 it, int 
 }
 
 // Which requests of a step are expanded, where their keys go, and the launches' work lists (one workgroup): those of at least
-// X_MIN new tokens, however many are cached. A step of 8 layers, us, absorbed and expanded: 1 prompt of 20 new tokens after
-// 500 2,098, 1,898; of 28 after 3,000 2,172, 2,177, of 70 2,313, 2,295; 4 of 20 after 500 2,336, 2,249; of 500 after 300 4,355, 4,221; 8
-// of 400 5,832, 5,628; one of 2,500 6,037, 5,228. Fewer tokens fill too little of a unit's 128 columns. Requests beyond X_REQS
-// or the workspace's `room` blocks keep the absorbed form. Tiles whose keys are more than a workgroup's average are split.
-constexpr int X_MIN = 12;
+// X_MIN new tokens, however many are cached, and all of them or none. None where they are more than X_REQS or their keys more
+// than the workspace's `room` blocks: a launch ends with its longest item, and the absorbed items of one prompt that is left
+// take as long as those of all (2 prompts of 256 after 2,500, 8 layers: 3,216 us absorbed, one of them expanded 3,520). None where
+// more than X_FEW units have less than half of their columns filled: 10 of 50 after 150 beside 200 decode rows 3,292 us refused,
+// 3,407 expanded; 60 of 12 after 60 3,033, 3,370; 7 of 72 after 150 beside 30 2,912, 2,800. Tiles whose keys are more than a
+// workgroup's average are split.
+constexpr int X_MIN = 12, X_FEW = 96;
 __global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const int* __restrict__ q_start,
                                                            const int* __restrict__ q_len, const int* __restrict__ ctx_len, int S,
                                                            int T, int H, int window, int room, int max_att, int max_tiles, int slots) {
-  __shared__ int ws[16], req[X_REQS], qs[X_REQS], ql[X_REQS], cl[X_REQS], to[X_REQS], tiles[X_REQS], n_req, n_tiles;
+  static_assert(X_REQS == 64, "a lane a request");
+  __shared__ int ws[16], req[X_REQS], qs[X_REQS], ql[X_REQS], cl[X_REQS], to[X_REQS], tiles[X_REQS];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   for (int t = threadIdx.x; t < T; t += 1024) X.form[t] = 0;
   int found = 0;
@@ -1067,46 +1070,55 @@ __global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const
     }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    const int n = min(found, X_REQS);
-    int used = 0, nt = 0, total = 0;
-    for (int i = 0; i < n; ++i) {
-      const int p0 = cl[i] - ql[i];
-      int lo, hi;
-      unit_stages(p0, ql[i], window, lo, hi);
-      const int blocks = ((cl[i] + 15) >> 4) - 4 * lo, t = (blocks + 3) >> 2;
-      to[i] = X_NONE;
-      if (used + blocks > room || nt + t > max_tiles) continue;
-      to[i] = used - 4 * lo;
-      tiles[i] = nt;
-      used += blocks;
-      nt += t;
-      for (int q = 0; q < ql[i]; q += X_COLS) {
-        unit_stages(p0 + q, min(X_COLS, ql[i] - q), window, lo, hi);
-        total += hi - lo;
-      }
+  // every wave works out all of this, a request a lane
+  int n = found <= X_REQS ? found : 0, lo = 0, hi, blocks = 0, nt = 0, total = 0, units = 0, tokens = 0;
+  if (lane < n) {
+    const int p0 = cl[lane] - ql[lane];
+    unit_stages(p0, ql[lane], window, lo, hi);
+    blocks = ((cl[lane] + 15) >> 4) - 4 * lo;
+    nt = (blocks + 3) >> 2;
+    for (int q = 0; q < ql[lane]; q += X_COLS) {
+      int a, b;
+      unit_stages(p0 + q, min(X_COLS, ql[lane] - q), window, a, b);
+      total += b - a;
+      units += H;
     }
+    tokens = ql[lane];
+  }
+  int used = blocks, all = nt;  // with the lanes before
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(used, o, 64), v = __shfl_up(all, o, 64);
+    if (lane >= o) {
+      used += u;
+      all += v;
+    }
+    total += __shfl_xor(total, o, 64);
+    units += __shfl_xor(units, o, 64);
+    tokens += __shfl_xor(tokens, o, 64);
+  }
+  const int listed = __shfl(all, 63, 64);
+  if (__shfl(used, 63, 64) > room || listed > max_tiles || (units > X_FEW && 2 * H * tokens < X_COLS * units)) n = 0;
+  if (threadIdx.x < n) {
+    to[lane] = used - blocks - 4 * lo;
+    tiles[lane] = all - nt;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) {
     const int fair = max(8, (total * H + 255) / 256);
     int na = 0, slot = 0;
-    for (int i = 0; i < n; ++i) {
-      if (to[i] == X_NONE) continue;
+    for (int i = 0; i < n; ++i)
       for (int q = 0; q < ql[i]; q += X_COLS) {
-        int lo, hi;
         unit_stages(cl[i] - ql[i] + q, min(X_COLS, ql[i] - q), window, lo, hi);
         int parts = min(8, (hi - lo + fair - 1) / fair);
         if (slot + parts > slots) parts = 1;
         for (int p = 0; p < parts && na < max_att; ++p) X.att[na++] = int4{req[i], q / X_COLS, p | parts << 16, slot};
         if (parts > 1) slot += parts;
       }
-    }
     X.counts[0] = na;
-    X.counts[1] = nt;
-    n_req = n;
+    X.counts[1] = n ? listed : 0;
   }
-  __syncthreads();
-  for (int i = 0; i < n_req; ++i) {
-    if (to[i] == X_NONE) continue;
-    int lo, hi;
+  for (int i = 0; i < n; ++i) {
     unit_stages(cl[i] - ql[i], ql[i], window, lo, hi);
     const int nb = (cl[i] + 15) >> 4;
     if (threadIdx.x == 0) X.base[req[i]] = to[i];

@@ -1,8 +1,8 @@
 // Prompt portions of a latent attention in the expanded form: keys and values of every head, k_h = W_uk,h c and v_h =
 // W_uv,h c, in a workspace, and an attention of heads of 128 + 64 (keys) and 128 (values) dimensions over them. A (query,
 // key) pair and head then takes 2 (128 + 64 + 128) products instead of the absorbed form's 2 (512 + 64 + 512), and a key 2 *
-// 512 * 256 once. Which requests run so is decided on the device, step by step (expand_plan_kernel), since a captured step
-// serves any mix of requests; the others keep the absorbed form, in the same launches.
+// 512 * 256 once. Whether a step's prompts run so is decided on the device, step by step (expand_plan_kernel), since a captured
+// step serves any mix of requests; the other requests keep the absorbed form, in the same launches.
 //
 // Workspace: kx [blocks of 16 keys][H][(128 + 128) / 8][16][8], a head's key then its value, both in the page layout;
 // kr [blocks][64 / 8][16][8], the rotated key part that the heads share.

@@ -493,3 +493,53 @@ def test_latent_attention_expanded(gpu, H, step, window):
         sc = (sc * scale).masked_fill(~((back >= 0) & ((back < window) if window else True)), -math.inf)
         want = torch.matmul(torch.softmax(sc, -1), torch.matmul(rows[:, :R], uv.float().transpose(1, 2))).transpose(0, 1)
         torch.testing.assert_close(o[q0:q0 + k], want, **tol(bf), msg=lambda s, i=i: f"request {i} {reqs[i]}: {s}")
+
+
+def plan_of(gpu, reqs, H, window):
+    """(the plan of a step of [(cached, new)], its rows)."""
+    from types import SimpleNamespace
+
+    from pilottai_amd.ops.latent import ExpandPlan
+
+    new = torch.tensor([n for _, n in reqs] + [0] * 3, dtype=torch.int32)  # (slots without a request)
+    meta = SimpleNamespace(q_len=new.to(gpu), q_start=(new.cumsum(0) - new).to(torch.int32).to(gpu),
+                           ctx_len=torch.tensor([c + n for c, n in reqs] + [0] * 3, dtype=torch.int32, device=gpu))
+    T = int(new.sum())
+    return ExpandPlan(meta, T, H, window), T
+
+
+@pytest.mark.parametrize("H,window,reqs,taken", [
+    (16, 0, [(0, 64)] * 64, True), (16, 0, [(0, 64)] * 65, False), (16, 0, [(5, 1)] * 70 + [(0, 64)] * 64, True),  # X_REQS
+    (16, 0, [(4096, 512)], True), (16, 0, [(4097, 512)], False),  # 288 blocks of keys are the room of 512 rows
+    (16, 0, [(2500, 256)] * 2, False), (16, 600, [(2500, 256)] * 2, True), (40, 0, [(0, 300), (4000, 300)], True),
+    (16, 0, [(0, 64)] * 7, True), (16, 0, [(0, 64)] * 6 + [(0, 63)], False),  # half of 112 units' columns
+    (16, 0, [(0, 40)] * 6, True), (5, 0, [(100, 12)] * 19, True), (5, 0, [(100, 12)] * 20, False),  # 96 units
+    (16, 0, [(900, 11), (3, 1)], False), (200, 45, [(0, 2000), (100, 700), (7, 1)], True), (1, 0, [(3000, 1000)], True)])
+def test_expand_plan_takes_all_prompts_or_none(gpu, H, window, reqs, taken):
+    """At the limits of requests, of keys and of units' fill; the work lists of what is taken name every block of its keys and
+    every tile of its tokens once, inside the workspace."""
+    plan, T = plan_of(gpu, reqs, H, window)
+    counts, base, form, att, tiles = (t.cpu() for t in plan.lists)
+    want = [i for i, (_, n) in enumerate(reqs) if n >= 12] if taken else []
+    assert [i for i, b in enumerate(base.tolist()) if b > -(1 << 30)] == want
+    assert form.tolist() == [int(i in want) for i, (_, n) in enumerate(reqs) for _ in range(n)]
+    na, nt = counts.tolist()
+    if not want:
+        assert (na, nt) == (0, 0)
+        return
+    at, listed, first = 0, [], {}
+    for i in want:
+        c, n = reqs[i]
+        first[i] = max(0, c - window + 1) // 64 * 4 if window else 0
+        blocks = (c + n + 15) // 16 - first[i]
+        assert int(base[i]) == at - first[i]
+        listed += [[i, first[i] + j, min(4, blocks - j), at + j] for j in range(0, blocks, 4)]
+        at += blocks
+    assert at <= plan.blocks and nt == len(listed) <= len(tiles) and tiles[:nt].tolist() == listed
+    parts = {}
+    for i, tile, p, slot in att[:na].tolist():
+        parts.setdefault((i, tile, p >> 16, slot if p >> 16 > 1 else -1), []).append(p & 0xffff)
+    assert [k[:2] for k in parts] == [(i, t) for i in want for t in range((reqs[i][1] + 127) // 128)]
+    assert all(v == list(range(k[2])) for k, v in parts.items())
+    used = [slot + p for i, t, n, slot in parts for p in range(n) if n > 1]
+    assert used == list(range(len(used))) and len(used) <= plan.slots
