@@ -334,7 +334,7 @@ class BozupelModel:
         rows = meta.logit_rows[:num_logit_rows]
         routes = self._route(meta, T)
         room = AttentionRoom(part_o, part_ml, self.dec_tokens, self.tile_tokens, 0)
-        if expand_pays(T, num_logit_rows):
+        if expand_pays(T, meta.q_len.numel()):
             keys = {L["attn"].expand_key() for L in self.layers} - {None}
             room = room._replace(expand={k: ExpandPlan(meta, T, *k) for k in keys})
         resid = torch.empty(T, d, dtype=torch.float32, device=dev)

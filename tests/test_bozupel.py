@@ -46,6 +46,9 @@ DESIGNS = {
                               width=64, loop={"start": 1, "stop": 2, "times": 2}, logit_scale=1.0),
     "once": design([(mixer(5, 10, 6, 12, 16, 20, 1), moe(3, 1, 20, 5.0)), (mixer(2, 20, 10, 24, 30, 40, 64), moe(9, 2, 24, 0.3))],
                    width=50, vocab=64, loop={"start": 0, "stop": 2, "times": 1}, logit_scale=3.0),
+    # sizes whose prompts may have their keys expanded per head (in bf16), with and without a window
+    "expanded": design([(mixer(3, 128, 64, 128, 64, 512, 0, scale=0.07), moe(5, 2, 40, 0.8)),
+                        (mixer(4, 128, 64, 128, 32, 512, 150, scale=0.07), None)]),
     "no_loop": design([(mixer(4, 32, 32, 24, 48, 72, 17), moe(6, 2, 48, 1.0))], width=128, vocab=257),
 }
 
@@ -343,6 +346,73 @@ def test_bucket_graphs_replay_exactly(gpu, folder):
         torch.randn(1 << 20, device=gpu).sum().item()
         assert [o.token_ids for o in got] == [o.token_ids for o in want]
     assert eng.stats["graph_replays"] > 0
+
+
+def test_form_of_a_step_does_not_depend_on_its_logits(folder, monkeypatch):
+    from pilottai_amd.models import bozupel
+
+    asked = []
+    monkeypatch.setattr(bozupel, "expand_pays", lambda *a: bool(asked.append(a)))
+    eng = engine(folder, "once", "cpu", "float32")
+    for rid, want in enumerate(([], [59], list(range(60)))):
+        eng.feed_step([(rid, tokens("once", 60), want)])
+        eng.release_fed(rid)
+    assert asked == [(asked[0][0], 4)] * 3 and asked[0][0] >= 60
+
+
+def expanding(folder, gpu, **kw):
+    return engine(folder, "expanded", gpu, "bfloat16", **dict(dict(max_num_batched_tokens=512, max_model_len=640, num_kv_blocks=120), **kw))
+
+
+@pytest.mark.gpu
+def test_prompts_with_expanded_keys(gpu, folder, monkeypatch):
+    """Portions that take the form, after none and after others; the same bits whatever is asked for. A step that the plan
+    refuses has the bits of one without a plan."""
+    from pilottai_amd.models import bozupel, latent
+
+    taken = []
+    real = latent.Expanded
+    monkeypatch.setattr(latent, "Expanded", lambda plan, *a: (taken.append(plan), real(plan, *a))[1])
+    eng, ids = expanding(folder, gpu), tokens("expanded", 590)
+    close(feed(eng, 1, ids, [270, 30, 290]), expect(folder, "expanded", ids), "bfloat16")
+    assert len(taken) == 2 * 2 and all(int(p.form.sum()) in (270, 290) for p in taken)  # (30 rows: without the plan)
+    eng.release_fed(1)
+
+    def residuals(entries):
+        out = []
+        eng.feed_step(entries, residuals=out)
+        for rid, _, _ in entries:
+            eng.release_fed(rid)
+        return [r[:sum(len(t) for _, t, _ in entries)].clone() for r in out]
+    form = [residuals([(rid, ids[:300], want)]) for rid, want in ((2, [299]), (3, list(range(300))), (4, []))]
+    assert all(torch.equal(a, b) for f in form[1:] for a, b in zip(f, form[0]))
+    monkeypatch.setattr(eng, "buckets", [512])
+    few = [(10 + i, ids[i * 20:i * 20 + 11], []) for i in range(4)]
+    refused = residuals(few)
+    assert not taken[-1].form.any()
+    monkeypatch.setattr(bozupel, "expand_pays", lambda *a: False)
+    assert all(torch.equal(a, b) for a, b in zip(refused, residuals(few)))
+    monkeypatch.undo()
+    monkeypatch.setattr(bozupel, "expand_pays", lambda *a: False)
+    absorbed = residuals([(5, ids[:300], [299])])
+    assert not any(torch.equal(a, b) for a, b in zip(absorbed, form[0]))
+    assert all((a - b).norm() < 0.02 * b.norm() for a, b in zip(absorbed, form[0]))
+
+
+@pytest.mark.gpu
+def test_expanded_keys_in_served_steps(gpu, folder):
+    """Prompts beside decoding requests through captured steps, again and again: the eager steps' tokens."""
+    ids = [tokens("expanded", n, 30 + n) for n in (400, 300, 20, 270, 333)]
+    kw = dict(temperature=0.0, max_tokens=6, ignore_eos=True)
+    want = expanding(folder, gpu, token_buckets=[4, 64, 512]).generate(ids, **kw)
+    eng = expanding(folder, gpu, use_graphs=True, token_buckets=[4, 64, 512])
+    for _ in range(3):
+        got = eng.generate(ids, **kw)
+        torch.randn(1 << 20, device=gpu).sum().item()
+        assert [o.token_ids for o in got] == [o.token_ids for o in want]
+    assert eng.stats["graph_replays"] > 0
+    for p, o in zip(ids, want):
+        greedy_is_right(folder, "expanded", p, o.token_ids, "bfloat16")
 
 
 @pytest.mark.parametrize("device", DEVICES)
