@@ -58,7 +58,7 @@ __device__ __forceinline__ bool skipped(const Args& A, int start, int n) {
   return __all(lane >= n || A.skip[start + min(lane, n - 1)] != 0);
 }
 
-// The rotated columns of `n` rows from `start` of group grp (one workgroup).
+// The rotated columns of `n` rows from `start` of group grp (one workgroup), of those that are not left out.
 template <typename T>
 __device__ __forceinline__ void rotate_rows(const Args& A, int grp, int start, int n) {
   const int half = A.rd >> 1, N = A.N16 * 16;
@@ -68,6 +68,7 @@ __device__ __forceinline__ void rotate_rows(const Args& A, int grp, int start, i
     const int hp = half >> 3;
     for (int e = threadIdx.x; e < n * hp; e += 256) {
       const int t = start + e / hp, j = (e % hp) * 8;
+      if (A.skip && A.skip[t]) continue;
       const bf16* src = (const bf16*)A.x + (size_t)t * A.ldx + (size_t)grp * A.xg + A.rskip + j;
       bf16* dst = (bf16*)A.out + (size_t)t * A.ldo + (size_t)grp * A.og + N + j;
       const float* cs = A.cos_sin + (size_t)A.positions[t] * A.rd + j;
@@ -84,8 +85,11 @@ __device__ __forceinline__ void rotate_rows(const Args& A, int grp, int start, i
       *reinterpret_cast<bf16x8*>(dst) = a;
       *reinterpret_cast<bf16x8*>(dst + half) = b;
     }
-    for (int e = threadIdx.x; e < n * (A.rp - A.r); e += 256)
-      ((T*)A.out)[(size_t)(start + e / (A.rp - A.r)) * A.ldo + (size_t)grp * A.og + N + A.r + e % (A.rp - A.r)] = (T)0.f;
+    for (int e = threadIdx.x; e < n * (A.rp - A.r); e += 256) {
+      const int t = start + e / (A.rp - A.r);
+      if (A.skip && A.skip[t]) continue;
+      ((T*)A.out)[(size_t)t * A.ldo + (size_t)grp * A.og + N + A.r + e % (A.rp - A.r)] = (T)0.f;
+    }
     return;
   }
   const int per = max(1, 256 / A.rp), i0 = threadIdx.x / A.rp;  // rows at a time
@@ -93,6 +97,7 @@ __device__ __forceinline__ void rotate_rows(const Args& A, int grp, int start, i
 #pragma unroll 4
     for (int i = i0; i < n; i += per) {
       const int t = start + i;
+      if (A.skip && A.skip[t]) continue;
       const T* src = (const T*)A.x + (size_t)t * A.ldx + (size_t)grp * A.xg + A.rskip;
       float v = 0.f;
       if (j < A.r) {

@@ -543,3 +543,25 @@ def test_expand_plan_takes_all_prompts_or_none(gpu, H, window, reqs, taken):
     assert all(v == list(range(k[2])) for k, v in parts.items())
     used = [slot + p for i, t, n, slot in parts for p in range(n) if n > 1]
     assert used == list(range(len(used))) and len(used) <= plan.slots
+
+
+@pytest.mark.parametrize("T,G", [(9, 3), (70, 5), (300, 9), (2100, 16)])  # tiles of 16 and of 64 rows, rows through LDS
+@pytest.mark.parametrize("N,K,r,rp", [(512, 128, 64, 64), (512, 128, 48, 64), (48, 32, 12, 32)])  # whole vectors, padding, pairs
+def test_head_gemm_leaves_rows_out(gpu, T, G, N, K, r, rp):
+    """Rows with an entry in `skip` stay as they are, their rotated columns too, in tiles with other rows and without; the
+    others have the bits of a launch that leaves none out."""
+    from pilottai_amd import ops
+
+    bf, g = torch.bfloat16, torch.Generator().manual_seed(T + N)
+    step = K + (r + 7) // 8 * 8
+    x = torch.randn(T, G * step, generator=g).to(gpu, bf)
+    w = ops.pack_groups(torch.randn(G, N, K, generator=g).to(gpu, bf) * K ** -0.5, bf)
+    pos, cs = torch.randint(0, 64, (T,), generator=g, dtype=torch.int32).to(gpu), ops.angle_table(64, r, 100.0).to(gpu)
+    skip = (torch.rand(T, generator=g) < 0.5).to(torch.int32)
+    skip[64:128], skip[0], skip[T - 1] = 1, 1, 0
+
+    def run(**kw):
+        out = torch.full((T, G * (N + rp)), 7.0, dtype=bf, device=gpu)
+        return ops.head_gemm(x, step, w, out, N + rp, rot=(pos, cs, K, r, rp), **kw)
+    want, got, gone = run(), run(skip=skip.to(gpu)), skip.bool().to(gpu)
+    assert (got[gone] == 7.0).all() and torch.equal(got[~gone], want[~gone])
