@@ -18,7 +18,7 @@ import torch
 from pilottai_amd import ops
 from pilottai_amd.models.cache import StepMeta
 from pilottai_amd.models.common import PackedLinear, pad_heads
-from pilottai_amd.ops.latent import EXPAND_SIZES, Expanded, latent_pad, pad_to
+from pilottai_amd.ops.latent import EXPAND_HEADS, EXPAND_SIZES, Expanded, latent_pad, pad_to
 
 
 @dataclass(frozen=True)
@@ -120,7 +120,7 @@ class LatentAttention:
         self.uv = ops.pack_groups(uv, dtype)
         self.k_rows = None  # W_uk by its rows, for the keys of a prompt's heads, where the sizes have that form
         sizes = dict(dim=n, vdim=vd, rot=r, rank=R)
-        if sizes == EXPAND_SIZES and m.rot_dims == r and source is None and not m.gate and dtype == torch.bfloat16 and \
+        if sizes == EXPAND_SIZES and H <= EXPAND_HEADS and m.rot_dims == r and source is None and not m.gate and dtype == torch.bfloat16 and \
                 torch.device(device).type == "cuda":
             self.k_rows = ops.pack_groups(t["uk"].to(device).view(H, n, R), dtype)
         self.width, self.out_bias = H * self.vp, None

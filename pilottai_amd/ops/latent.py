@@ -80,8 +80,9 @@ def latent_attention(out, part_o, part_ml, q, pages, items, n_items, q_start, q_
     return out
 
 
-# Prompt portions with the keys expanded per head (csrc/ops/latent_expand.h): sizes that have the form
-EXPAND_SIZES = dict(dim=128, vdim=128, rot=64, rank=512)
+# Prompt portions with the keys expanded per head (csrc/ops/latent_expand.h): sizes that have the form, and the most heads (an
+# item's heads are units of as many workgroups, 256 of which the launch is sure to have)
+EXPAND_SIZES, EXPAND_HEADS = dict(dim=128, vdim=128, rot=64, rank=512), 256
 EXPAND_COLS, EXPAND_REQS = 128, 64
 
 

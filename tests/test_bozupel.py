@@ -400,6 +400,26 @@ def test_prompts_with_expanded_keys(gpu, folder, monkeypatch):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("heads", [256, 257])  # (more than the form has: absorbed, as without it)
+def test_steps_of_many_heads(gpu, heads, monkeypatch):
+    from pilottai_amd.engine.engine import EngineConfig, LLMEngine
+    from pilottai_amd.models import bozupel
+
+    spec = bozupel.LatentAttentionSpec(heads=heads, dim=128, rot_dim=64, vdim=128, q_rank=64, kv_rank=512, scale=0.07,
+                                       rot_base=1e4, rot_dims=64, window=300)
+    cfg = bozupel.BozupelConfig(name="many heads", vocab_size=512, hidden_size=64, layers=[bozupel.BozupelLayer(spec, None)])
+    eng = LLMEngine(EngineConfig(model=cfg, max_num_seqs=4, max_num_batched_tokens=512, max_model_len=512, num_kv_blocks=60,
+                                 exact_kv_blocks=True, prefix_caching=False, use_graphs=False), device=gpu)
+    form, absorbed = [], []
+    for rid, out in enumerate((form, absorbed)):
+        eng.feed_step([(rid, list(range(400)), [])], residuals=out)
+        eng.release_fed(rid)
+        monkeypatch.setattr(bozupel, "expand_pays", lambda *a: False)
+    a, b = form[0][:400], absorbed[0][:400]
+    assert torch.equal(a, b) == (heads > 256) and (a - b).norm() < 0.02 * b.norm()
+
+
+@pytest.mark.gpu
 def test_expanded_keys_in_served_steps(gpu, folder):
     """Prompts beside decoding requests through captured steps, again and again: the eager steps' tokens."""
     ids = [tokens("expanded", n, 30 + n) for n in (400, 300, 20, 270, 333)]
