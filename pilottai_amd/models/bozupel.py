@@ -215,7 +215,7 @@ class BozupelModel:
             if key not in rot:
                 rot[key] = m.angles(self.max_len).to(self.device)
             attn = LatentAttention(m, {k: get(f"{pre}mix.{k}", s) for k, s in m.shapes(d).items()}, eps, dtype,
-                                   self.device, rot[key])
+                                   self.device, rot[key], expand=True)
             layer = {"norm1": f32(pre + "norm1"), "norm1b": f32(pre + "norm1b"), "mlp": None,
                      "attn": attn, "block": MixerBlock([attn], dtype, self.device)}
             if p is not None:

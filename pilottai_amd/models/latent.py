@@ -79,10 +79,10 @@ class LatentAttentionSpec:
 
 class LatentAttention:
     """Projection rows [query latent or queries | latent | rotated key part | gate]. `source`: the mixer of the layer
-    that kv_from names."""
+    that kv_from names. `expand`: the model's steps have plans of expanded requests (AttentionRoom.expand)."""
 
     def __init__(self, spec: LatentAttentionSpec, t: Dict[str, torch.Tensor], eps: float, dtype, device, cos_sin=None,
-                 source: Optional["LatentAttention"] = None):
+                 source: Optional["LatentAttention"] = None, expand: bool = False):
         m = self.spec = spec
         self.eps, self.dtype, self.device, self.cos_sin = eps, dtype, device, cos_sin
         H, n, r, vd, R = m.heads, m.dim, m.rot_dim, m.vdim, m.kv_rank
@@ -120,8 +120,8 @@ class LatentAttention:
         self.uv = ops.pack_groups(uv, dtype)
         self.k_rows = None  # W_uk by its rows, for the keys of a prompt's heads, where the sizes have that form
         sizes = dict(dim=n, vdim=vd, rot=r, rank=R)
-        if sizes == EXPAND_SIZES and H <= EXPAND_HEADS and m.rot_dims == r and source is None and not m.gate and dtype == torch.bfloat16 and \
-                torch.device(device).type == "cuda":
+        if expand and sizes == EXPAND_SIZES and H <= EXPAND_HEADS and m.rot_dims == r and source is None and not m.gate and \
+                dtype == torch.bfloat16 and torch.device(device).type == "cuda":
             self.k_rows = ops.pack_groups(t["uk"].to(device).view(H, n, R), dtype)
         self.width, self.out_bias = H * self.vp, None
         self.w_out = pad_heads(t["o"].T.reshape(H, vd, -1), self.vp).reshape(self.width, -1).T

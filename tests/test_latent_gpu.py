@@ -565,3 +565,21 @@ def test_head_gemm_leaves_rows_out(gpu, T, G, N, K, r, rp):
         return ops.head_gemm(x, step, w, out, N + rp, rot=(pos, cs, K, r, rp), **kw)
     want, got, gone = run(), run(skip=skip.to(gpu)), skip.bool().to(gpu)
     assert (got[gone] == 7.0).all() and torch.equal(got[~gone], want[~gone])
+
+
+@pytest.mark.parametrize("family,offered", [("bozupel", True), ("pusunex", False)])
+def test_weights_of_expanded_keys_where_plans_are_made(gpu, family, offered):
+    """Layers of the sizes that have the form hold the keys' weights only in a model whose steps have plans."""
+    from pilottai_amd.models import bozupel, pusunex
+    from pilottai_amd.models.latent import LatentAttentionSpec
+    from pilottai_amd.models.registry import model_class
+
+    spec = LatentAttentionSpec(heads=2, dim=128, rot_dim=64, vdim=128, q_rank=64, kv_rank=512, scale=0.07, rot_base=1e4, rot_dims=64)
+    if family == "bozupel":
+        cfg = bozupel.BozupelConfig("x", 512, 64, [bozupel.BozupelLayer(spec, None)])
+    else:
+        cfg = pusunex.PusunexConfig("x", 512, 64, [pusunex.PusunexLayer(spec, None)], norm_groups=4, side_dim=16)
+    model = model_class(cfg)(cfg, gpu, max_len=64)
+    L = model.layers[0]
+    layer = L["attn"] if family == "bozupel" else L["mixer"].mixers[0]
+    assert (layer.expand_key() == (2, 0)) == offered and len(layer.tensors()) == 3 + offered
