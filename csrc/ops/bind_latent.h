@@ -116,8 +116,10 @@ pa::la::Expand expand_plan(const Tensors& p, int64_t S, int64_t T) {
   return X;
 }
 
-// The workspace: kx [blocks, H, 32, 16, 8] and kr [blocks, 8, 16, 8]
-void expand_room(pa::la::Expand& X, const at::Tensor& kx, const at::Tensor& kr, int64_t H) {
+// The workspace: kx [blocks, H, 32, 16, 8] and kr [blocks, 8, 16, 8], of at least the `room` blocks that the plan may give
+// away; block_table: of all requests that the plan may name
+void expand_room(pa::la::Expand& X, const Tensors& plan, const at::Tensor& kx, const at::Tensor& kr, const at::Tensor& block_table,
+                 int64_t H, int64_t room) {
   for (auto* t : {&kx, &kr}) {
     check_gpu(*t, "workspace");
     check_dtype(*t, at::kBFloat16, "workspace");
@@ -125,6 +127,8 @@ void expand_room(pa::la::Expand& X, const at::Tensor& kx, const at::Tensor& kr, 
   TORCH_CHECK(kx.dim() == 5 && kx.size(1) == H && kx.size(2) * 8 == 2 * pa::la::X_DIM && kx.size(3) == 16 && kx.size(4) == 8 &&
                   kr.dim() == 4 && kr.size(0) == kx.size(0) && kr.size(1) * 8 == pa::la::X_ROT && kr.size(2) == 16 && kr.size(3) == 8,
               "workspace must be [blocks, H, 32, 16, 8] and [blocks, 8, 16, 8]");
+  TORCH_CHECK(kx.size(0) >= room && room >= 1, "workspace of ", kx.size(0), " blocks for a plan of ", room);
+  TORCH_CHECK(block_table.dim() == 2 && block_table.size(0) == plan[1].numel(), "a plan is for the requests of its block table");
   X.kx = kx.data_ptr();
   X.kr = kr.data_ptr();
 }
@@ -142,10 +146,11 @@ void latent_plan(const Tensors& plan, at::Tensor q_start, at::Tensor q_len, at::
            "latent_plan");
 }
 
-// keys and values of the planned requests from their pages: wk, wv [H, 8, 16, 64, 8], the heads' rows of W_uk and of W_uv
-void latent_expand(const Tensors& plan, at::Tensor kx, at::Tensor kr, at::Tensor pages, at::Tensor wk, at::Tensor wv,
+// keys and values of the planned requests from their pages: wk, wv [H, 8, 16, 64, 8], the heads' rows of W_uk and of W_uv;
+// room: as the plan was made with
+void latent_expand(const Tensors& plan, int64_t room, at::Tensor kx, at::Tensor kr, at::Tensor pages, at::Tensor wk, at::Tensor wv,
                    at::Tensor block_table) {
-  pa::la::Expand X = expand_plan(plan, block_table.size(0), 0);
+  pa::la::Expand X = expand_plan(plan, 0, 0);
   const int64_t H = wk.size(0);
   for (auto* t : {&pages, &wk, &wv}) {
     check_gpu(*t, "latent_expand arg");
@@ -156,8 +161,7 @@ void latent_expand(const Tensors& plan, at::Tensor kx, at::Tensor kr, at::Tensor
                     w->size(3) == 64 && w->size(4) == 8, "weights must be packed [H, 8, 16, 64, 8]");
   TORCH_CHECK(pages.dim() == 4 && pages.size(1) * 8 == pa::la::X_RANK + pa::la::X_ROT && pages.size(2) == 16 && pages.size(3) == 8,
               "pages must be [blocks, 72, 16, 8]");
-  TORCH_CHECK(block_table.dim() == 2, "block_table [seqs, blocks]");
-  expand_room(X, kx, kr, H);
+  expand_room(X, plan, kx, kr, block_table, H, room);
   check_rc(pa_latent_expand(&X, pages.data_ptr(), wk.data_ptr(), wv.data_ptr(), ints(block_table, 0, "block_table"), block_table.size(1),
                             H, pages.size(1) * 8, plan[4].size(0), cur_stream()),
            "latent_expand");
@@ -166,7 +170,8 @@ void latent_expand(const Tensors& plan, at::Tensor kx, at::Tensor kr, at::Tensor
 void latent_attention(at::Tensor out, at::Tensor part_o, at::Tensor part_ml, at::Tensor q,
                       at::Tensor pages, at::Tensor items, at::Tensor n_items, at::Tensor q_start, at::Tensor q_len,
                       at::Tensor ctx_len, at::Tensor block_table, int64_t dec_tokens, int64_t tile_tokens,
-                      int64_t window, double scale, bool simple, const Tensors& plan, const Tensors& expand) {
+                      int64_t window, double scale, bool simple, const Tensors& plan, const Tensors& expand, int64_t room,
+                      int64_t slots) {
   const int f = is_f32(q, "q");
   for (auto* t : {&out, &q, &pages}) {
     check_gpu(*t, "latent_attention arg");
@@ -181,13 +186,14 @@ void latent_attention(at::Tensor out, at::Tensor part_o, at::Tensor part_ml, at:
   const int64_t NB = (dec_tokens * H + 15) / 16;
   TORCH_CHECK(Rp > 0 && rp >= 0 && dec_tokens >= 1 && tile_tokens >= 1, "latent_attention sizes");
   TORCH_CHECK(part_o.numel() >= mi * NB * 16 * Rp && part_ml.numel() >= mi * NB * 32, "partition workspace too small");
-  // expanded requests: expand = [kx, kr, q not yet absorbed or rotated, cos_sin, their outputs, partial outputs and (max, sum)]
+  // expanded requests: expand = [kx, kr, q not yet absorbed or rotated, cos_sin, their outputs, partial outputs and (max, sum)];
+  // room and slots: as the plan was made with
   pa::la::Expand X{};
   if (!expand.empty()) {
-    const int64_t T = q.size(0), slot = H * pa::la::X_COLS, slots = expand.size() == 7 ? expand[6].numel() / (2 * slot) : 0;
+    const int64_t T = q.size(0), slot = H * pa::la::X_COLS;
     TORCH_CHECK(!f && expand.size() == 7 && Rp == pa::la::X_RANK && rp == pa::la::X_ROT, "latent_attention: expanded sizes");
     X = expand_plan(plan, S, T);
-    expand_room(X, expand[0], expand[1], H);
+    expand_room(X, plan, expand[0], expand[1], block_table, H, room);
     const at::Tensor &xq = expand[2], &xo = expand[4];
     check_rows(xq, at::kBFloat16, "q");
     check_rows(xo, at::kBFloat16, "expanded out");
@@ -201,7 +207,7 @@ void latent_attention(at::Tensor out, at::Tensor part_o, at::Tensor part_ml, at:
     X.out = xo.data_ptr();
     X.ldo = xo.stride(0);
     X.part_o = (float*)opt_f32(expand[5], slots * slot * pa::la::X_DIM, "partial outputs");
-    X.part_ml = (float*)opt_f32(expand[6], 0, "partial sums");
+    X.part_ml = (float*)opt_f32(expand[6], slots * slot * 2, "partial sums");
   }
   check_rc(pa_latent_attention(f, out.data_ptr(), (float*)opt_f32(part_o, 0, "part_o"),
                                (float*)opt_f32(part_ml, 0, "part_ml"), q.data_ptr(),

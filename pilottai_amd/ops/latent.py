@@ -69,11 +69,13 @@ def latent_attention(out, part_o, part_ml, q, pages, items, n_items, q_start, q_
     dec_tokens / tile_tokens: the scheduler's items hold at most dec_tokens tokens (split over keys) or
     tile_tokens (csrc/ops/latent_attention.hip). `simple`: the any-size kernel. `expand`: requests of its plan are left out
     here, and their outputs in the heads' own dimensions go to its `out`."""
+    if expand and expand.window != window:
+        raise ValueError(f"a plan for a window of {expand.window} with one of {window}")
     if _on_gpu(q):
         require_latent().latent_attention(out, part_o, part_ml, q, pages, items, n_items, q_start, q_len,
                                           ctx_len, block_table, int(dec_tokens), int(tile_tokens), int(window),
                                           float(scale), bool(simple), expand.plan if expand else [],
-                                          expand.tensors() if expand else [])
+                                          expand.tensors() if expand else [], *(expand.sizes if expand else (0, 0)))
     else:
         ref.latent_attention(out, q, pages, q_start, q_len, ctx_len, block_table, scale, window,
                              len(q_len) if num_seqs is None else num_seqs)
@@ -101,7 +103,7 @@ class ExpandPlan:
     items, expansion tiles], and the room for it. `form` [T] is 1 for their rows."""
 
     def __init__(self, meta, T: int, heads: int, window: int):
-        dev, S = meta.q_len.device, meta.q_len.numel()
+        dev, S, self.window = meta.q_len.device, meta.q_len.numel(), window
         # as many keys as rows, and the cached ones of a long context
         self.blocks = (T + max(T, 4096)) // 16
         self.slots = max(8, 768 // heads)
@@ -121,10 +123,11 @@ class Expanded:
         H, dev = wk.shape[0], pages.device
         new = lambda dt, *s: torch.empty(*s, dtype=dt, device=dev)  # noqa: E731
         self.plan, self.form, self.q, self.cos_sin, self.out = plan.lists, plan.form, q, cos_sin, out
+        self.sizes, self.window = (plan.blocks, plan.slots), plan.window
         self.kx, self.kr = new(torch.bfloat16, plan.blocks, H, 32, 16, 8), new(torch.bfloat16, plan.blocks, 8, 16, 8)
         self.part_o = new(torch.float32, plan.slots, H, EXPAND_COLS, 128)
         self.part_ml = new(torch.float32, plan.slots, H, EXPAND_COLS, 2)
-        require_latent().latent_expand(self.plan, self.kx, self.kr, pages, wk, wv, block_table)
+        require_latent().latent_expand(self.plan, plan.blocks, self.kx, self.kr, pages, wk, wv, block_table)
 
     def tensors(self):
         return [self.kx, self.kr, self.q, self.cos_sin, self.out, self.part_o, self.part_ml]

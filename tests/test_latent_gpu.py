@@ -583,3 +583,39 @@ def test_weights_of_expanded_keys_where_plans_are_made(gpu, family, offered):
     L = model.layers[0]
     layer = L["attn"] if family == "bozupel" else L["mixer"].mixers[0]
     assert (layer.expand_key() == (2, 0)) == offered and len(layer.tensors()) == 3 + offered
+
+
+def test_expanded_workspace_is_the_plans(gpu):
+    """A workspace, partial results, a block table or a window other than the plan's are refused before any launch."""
+    from pilottai_amd import ops
+    from pilottai_amd.ops.latent import Expanded
+
+    bf, H, d = torch.bfloat16, 2, dict(device=gpu)
+    plan, T = plan_of(gpu, [(0, 300)], H, 0)
+    S = plan.lists[1].numel()
+    pages, table = torch.zeros(20, 72, 16, 8, dtype=bf, **d), torch.zeros(S, 19, dtype=torch.int32, **d)
+    w, q, out = torch.zeros(H, 8, 16, 64, 8, dtype=bf, **d), torch.zeros(T, H * 192, dtype=bf, **d), torch.zeros(T, H * 128, dtype=bf, **d)
+    cs = torch.zeros(400, 64, **d)
+
+    def attend(ex, table=table, window=0):
+        qa, oc = torch.zeros(T, H, 576, dtype=bf, **d), torch.zeros(T, H, 512, dtype=bf, **d)
+        z, i = torch.zeros(1 << 20, **d), torch.zeros(4, 4, dtype=torch.int32, **d)
+        n, one = torch.zeros(S, dtype=torch.int32, **d), torch.zeros(1, dtype=torch.int32, **d)
+        ops.latent_attention(oc, z, z, qa, pages, i, one, n, n, n, table, 1.0, window, 8, 64, expand=ex)
+    ex = Expanded(plan, pages, w, w, table, q, cs, out)
+    with pytest.raises(RuntimeError, match="block table"):
+        Expanded(plan, pages, w, w, table[:1], q, cs, out)
+    with pytest.raises(RuntimeError, match="block table"):
+        attend(ex, table[:1].contiguous())
+    with pytest.raises(ValueError, match="window"):
+        attend(ex, window=5)
+    for name, match in (("kx", "workspace"), ("part_o", "too short"), ("part_ml", "too short")):
+        whole = getattr(ex, name)
+        setattr(ex, name, whole[:-1])
+        if name == "kx":
+            ex.kr = ex.kr[:-1]
+        with pytest.raises(RuntimeError, match=match):
+            attend(ex)
+        setattr(ex, name, whole)
+        if name == "kx":
+            ex.kr = torch.zeros(len(whole), 8, 16, 8, dtype=bf, **d)
