@@ -347,16 +347,17 @@ class SemanticIndex:
             except TypeError:  # (numbers on the GPU)
                 to[:] = torch.as_tensor(values[:Q]).cpu().numpy()
             words.append(torch.from_numpy(to))
-        with self._lock, self._stream_ctx():
-            here = self._stream
-            if caller is not None:
-                here.wait_stream(caller)
-            q = q.detach().to(self.device if q.is_cuda else "cpu", torch.float32).contiguous()
-            ev = self._pass_event()
-            t_now = self.now() if now is None else now - self.epoch
-            back, out, (minp, qt), qs = ops.lookup_begin(q, *words, k, self.storage == "q16")
-            filters = (self.priority, self.tagbits, self.expiry, minp, qt, t_now)
-            try:
+        here = None
+        try:
+            with self._lock, self._stream_ctx():
+                here = self._stream
+                if caller is not None:
+                    here.wait_stream(caller)
+                q = q.detach().to(self.device if q.is_cuda else "cpu", torch.float32).contiguous()
+                ev = self._pass_event()
+                t_now = self.now() if now is None else now - self.epoch
+                back, out, (minp, qt), qs = ops.lookup_begin(q, *words, k, self.storage == "q16")
+                filters = (self.priority, self.tagbits, self.expiry, minp, qt, t_now)
                 if self.storage == "q16":
                     args = (*qs, self.hi, self.lo, self.rmeta, self.count, k, *filters, out)
                     ops.q16_pass(*args, False, self._ws)
@@ -364,18 +365,19 @@ class SemanticIndex:
                     ops.cosine_topk(*qs, self.packed, self.count, k, *filters, workspace=self._ws, out=out[:2])
                 if ev is not None:
                     ev[1].record()
-            except BaseException:
-                here.synchronize()  # (the pinned memory is not given back before the GPU is done with it)
-                raise
-        here.synchronize()
-        a = back.numpy()
-        if self.storage == "q16" and a[2 * Q * k:].any():  # a slice refused a row that might be in the top-k
-            with self._lock, self._stream_ctx():
-                self.stats["q16_fallbacks"] += 1
-                ops.q16_pass(*args, True, self._ws)
-                if ev is not None:  # (both passes, as search_tensors has it)
-                    ev[1].record()
             here.synchronize()
+            a = back.numpy()
+            if self.storage == "q16" and a[2 * Q * k:].any():  # a slice refused a row that might be in the top-k
+                with self._lock, self._stream_ctx():
+                    self.stats["q16_fallbacks"] += 1
+                    ops.q16_pass(*args, True, self._ws)
+                    if ev is not None:  # (both passes, as search_tensors has it)
+                        ev[1].record()
+                here.synchronize()
+        except BaseException:
+            if here is not None:  # (the pinned memory is not given back before the GPU is done with it)
+                here.synchronize()
+            raise
         if ev is not None:
             self.pass_events.append(ev)
         return a[:Q * k].view(np.float32).reshape(Q, k), a[Q * k:2 * Q * k].reshape(Q, k)

@@ -259,3 +259,24 @@ def test_search_times_its_second_pass_too(gpu, monkeypatch):
     assert idx.stats["q16_fallbacks"] == 1 and len(ends) == 2 and len(idx.pass_events) == 1
     (start, end), = idx.pass_events
     assert 0 < start.elapsed_time(ends[0]) < start.elapsed_time(ends[1]) <= start.elapsed_time(end)
+
+
+@pytest.mark.parametrize("exact", [False, True])
+def test_search_that_fails_waits_for_its_passes(gpu, monkeypatch, exact):
+    """A pass that raises behind its launches, the first or the one that stands behind it: the pinned memory that the kernels
+    write to stays until they are done."""
+    idx, v = _small_index(gpu, n=40_000, same=True)
+    idx.search(v, 5, [0], [()])
+    run = ops.q16_pass
+
+    def fails(*args):
+        run(*args)
+        if args[-2] == exact:
+            torch.cuda._sleep(50_000_000)
+            raise KeyError("pass")
+    monkeypatch.setattr(ops, "q16_pass", fails)
+    with pytest.raises(KeyError):
+        idx.search(v, 5, [0], [()])
+    assert idx._stream.query()
+    monkeypatch.setattr(ops, "q16_pass", run)
+    assert [r for r, _ in idx.search(v, 5, [0], [()])[0]]
