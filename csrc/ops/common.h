@@ -25,6 +25,12 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 __device__ __forceinline__ float bf2f(bf16 x) { return (float)x; }
 __device__ __forceinline__ bf16 f2bf(float x) { return (bf16)x; }
 
+// Rows without a token are looked for in launches of more rows than this. The engine's default steps are captured 64 rows or
+// less apart up to here, where a whole tile of 256 rows of padding does not occur, 1,024 apart up to 4,096 rows and 2,048
+// apart beyond. So only engines whose budget is above 2,048 tokens (the default) have launches that look; steps of other sizes of a
+// caller's own that are further apart below compute their padding.
+constexpr int LIVE_MIN_ROWS = 2048;
+
 __device__ __forceinline__ float wave_sum(float v) {
 #pragma unroll
   for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);

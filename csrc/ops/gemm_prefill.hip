@@ -563,11 +563,9 @@ namespace pf {
 constexpr int kPfDefaultVariant = 3;
 static int g_pf_variant = kPfDefaultVariant;
 
-// Tiles without a token are looked for above this many rows. The engine's graphs are 64 rows or less apart up to here, and
-// a whole tile of padding is rare; above they are 1,024 apart. One prompt, us a step (8 layers of each model) before and
+// Tiles without a token are left out above LIVE_MIN_ROWS rows. One prompt, us a step (8 layers of each model) before and
 // after: llama 2,101 tokens (3 of 12 row tiles hold none) 9118, 7874; 2,500 9293, 8441; 3,300 11618, 10590; 3,700 (1 of 16)
 // 11919, 11588; mudepel 2,101 4980, 4641; 3,300 6456, 6021. A step without padding is as before (bozupel, 4,096 6395, 6386).
-constexpr int LIVE_MIN_ROWS = 2048;
 
 // Default decomposition: whole tiles while they fill complete rounds of 256 CUs; a
 // remainder of at most half a round is split over K so that the last round is (nearly)
@@ -663,7 +661,7 @@ extern "C" int pa_prefill_gemm(void* y, const void* x, const void* wp, const voi
          M, N, K, ldx, ldy, ldr, MT, NT, full, S, per, eps, ss_in, ss_out, ss_zero,
          (pa::bf16*)q_out, (pa::bf16*)k_cache, (pa::bf16*)v_cache, positions, slots, cos_sin, H, KV,
          pa::g_handoff_acquire};
-  a.live = M > LIVE_MIN_ROWS ? live : nullptr;
+  a.live = M > pa::LIVE_MIN_ROWS ? live : nullptr;
   const int grid = full + (tiles - full) * S;
   // Mixed tail (variant 3, the default, and 8; 9 = without it): full rounds of 256 x 256
   // tiles over the first c1 column tiles,

@@ -151,9 +151,9 @@ extern "C" int pa_hyper_norm(int fp32, float* x, int S, const void* y, int K, in
   using namespace pa::hn;
   if (n <= 0) return 0;
   if (D <= 0 || D * 4 > 96 * 1024 || S < 1 || S > MAX_S) return -1;
-  // Rows without a token stay as they are above 2,048 rows, where the steps that graphs are captured for are 1,024 apart (a step
-  // of mudepel's 8 layers, 4 streams of 2,048 columns: 3,658 tokens in 4,096 rows 2 % of its 5,840 us, 2,101 in 3,072 3 % of 4,640)
-  if (rows || n <= 2048) live = nullptr;
+  // Rows without a token stay as they are in launches that look for them (a step of mudepel's 8 layers, 4 streams of 2,048
+  // columns: 3,658 tokens in 4,096 rows 2 % of its 5,840 us, 2,101 in 3,072 3 % of 4,640)
+  if (rows || n <= pa::LIVE_MIN_ROWS) live = nullptr;
   const Args A{x, y, y_w, y2, bias, mix, post, pre, emb, ids, w_next, out, rows, live, K, ldy, ldy2, vocab, ldo, D, eps};
   // fewer rows than CUs: twice the waves to a row, all of it in one pass up to 2,048 columns (64 rows, 4 streams of 2,048:
   // 6.8 -> 5.7 us)

@@ -354,8 +354,8 @@ extern "C" int pa_residual_norm(int fp32, float* resid, const void* y, int K, in
   if (n <= 0) return 0;
   if (D <= 0 || D * 4 > 96 * 1024) return -1;  // the row in LDS
   if (post_groups < 1 || next_groups < 1 || D % post_groups || D % next_groups || (mix && (!emb || !hist || n_hist < 1))) return -1;
-  // Rows without a token stay as they are above 2,048 rows, where the steps that graphs are captured for are 1,024 apart
-  if (rows || n <= 2048) live = nullptr;
+  // Rows without a token stay as they are in launches that look for them
+  if (rows || n <= pa::LIVE_MIN_ROWS) live = nullptr;
   const Args A{resid, y, w_post, emb, ids, mix, hist, w_next, out, rows, live, hist_step, K, ldy, vocab, emb_add, n_hist, ldo, D,
                post_groups, next_groups, y_scale, eps};
   // whole 8s, and groups that are lanes of a wave (a power of two) or whole wave steps
