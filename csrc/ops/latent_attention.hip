@@ -1038,22 +1038,24 @@ __device__ __forceinline__ void expanded_unit(const Args& A, const int4 it, int 
 // X_MIN new tokens, however many are cached, and all of them or none. None where they are more than X_REQS or their keys more
 // than the workspace's `room` blocks: a launch ends with its longest item, and the absorbed items of one prompt that is left
 // take as long as those of all (2 prompts of 256 after 2,500, 8 layers: 3,216 us absorbed, one of them expanded 3,520). None where
-// more than X_FEW units have less than half of their columns filled: 10 of 50 after 150 beside 200 decode rows 3,292 us refused,
-// 3,407 expanded; 60 of 12 after 60 3,033, 3,370; 7 of 72 after 150 beside 30 2,912, 2,800. Tiles whose keys are more than a
-// workgroup's average are split.
-constexpr int X_MIN = 12, X_FEW = 96;
+// they fill less than half of the columns of more than two tiles: 10 of 50 after 150 beside 200 decode rows 3,292 us refused,
+// 3,407 expanded; 60 of 12 after 60 3,033, 3,370; 7 of 72 after 150 beside 30 2,912, 2,800. And none where they are less than twice
+// the tokens of the other requests, whose items wait for the units: 2 of 140 after 600 beside 230 rows of 1,500 keys 3,409, 3,464; 4
+// of 132 after 700 beside 200 of 1,000 3,615, 3,605. Tiles whose keys are more than a workgroup's average are split.
+constexpr int X_MIN = 12;
 __global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const int* __restrict__ q_start,
                                                            const int* __restrict__ q_len, const int* __restrict__ ctx_len, int S,
                                                            int T, int H, int window, int room, int max_att, int max_tiles, int slots) {
   static_assert(X_REQS == 64, "a lane a request");
-  __shared__ int ws[16], req[X_REQS], qs[X_REQS], ql[X_REQS], cl[X_REQS], to[X_REQS], tiles[X_REQS];
+  __shared__ int ws[16], others[16], req[X_REQS], qs[X_REQS], ql[X_REQS], cl[X_REQS], to[X_REQS], tiles[X_REQS];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
   for (int t = threadIdx.x; t < T; t += 1024) X.form[t] = 0;
-  int found = 0;
+  int found = 0, rest = 0;
   for (int s0 = 0; s0 < S; s0 += 1024) {
     const int s = s0 + threadIdx.x, n = s < S ? q_len[s] : 0;
     const bool yes = n >= X_MIN && s < S && q_start[s] + n <= T;
     if (s < S) X.base[s] = X_NONE;
+    if (!yes) rest += n;
     const unsigned long long b = __ballot(yes);
     if (lane == 0) ws[wid] = __popcll(b);
     __syncthreads();
@@ -1070,8 +1072,14 @@ __global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const
     }
     __syncthreads();
   }
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) rest += __shfl_xor(rest, o, 64);
+  if (lane == 0) others[wid] = rest;
+  __syncthreads();
+  rest = 0;
+  for (int w = 0; w < 16; ++w) rest += others[w];
   // every wave works out all of this, a request a lane
-  int n = found <= X_REQS ? found : 0, lo = 0, hi, blocks = 0, nt = 0, total = 0, units = 0, tokens = 0;
+  int n = found <= X_REQS ? found : 0, lo = 0, hi, blocks = 0, nt = 0, total = 0, cols = 0, tokens = 0;
   if (lane < n) {
     const int p0 = cl[lane] - ql[lane];
     unit_stages(p0, ql[lane], window, lo, hi);
@@ -1081,7 +1089,7 @@ __global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const
       int a, b;
       unit_stages(p0 + q, min(X_COLS, ql[lane] - q), window, a, b);
       total += b - a;
-      units += H;
+      cols += X_COLS;
     }
     tokens = ql[lane];
   }
@@ -1094,11 +1102,11 @@ __global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const
       all += v;
     }
     total += __shfl_xor(total, o, 64);
-    units += __shfl_xor(units, o, 64);
+    cols += __shfl_xor(cols, o, 64);
     tokens += __shfl_xor(tokens, o, 64);
   }
   const int listed = __shfl(all, 63, 64);
-  if (__shfl(used, 63, 64) > room || listed > max_tiles || (units > X_FEW && 2 * H * tokens < X_COLS * units)) n = 0;
+  if (__shfl(used, 63, 64) > room || listed > max_tiles || (cols > 2 * X_COLS && 2 * tokens < cols) || tokens < 2 * rest) n = 0;
   if (threadIdx.x < n) {
     to[lane] = used - blocks - 4 * lo;
     tiles[lane] = all - nt;

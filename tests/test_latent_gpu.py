@@ -513,7 +513,9 @@ def plan_of(gpu, reqs, H, window):
     (16, 0, [(4096, 512)], True), (16, 0, [(4097, 512)], False),  # 288 blocks of keys are the room of 512 rows
     (16, 0, [(2500, 256)] * 2, False), (16, 600, [(2500, 256)] * 2, True), (40, 0, [(0, 300), (4000, 300)], True),
     (16, 0, [(0, 64)] * 7, True), (16, 0, [(0, 64)] * 6 + [(0, 63)], False),  # half of 112 units' columns
-    (16, 0, [(0, 40)] * 6, True), (5, 0, [(100, 12)] * 19, True), (5, 0, [(100, 12)] * 20, False),  # 96 units
+    (16, 0, [(0, 12)] * 2, True), (16, 0, [(0, 12)] * 3, False),  # two tiles, whatever they hold
+    (16, 0, [(9, 1)] * 2 + [(9, 11)] * 3 + [(3, 70)], True), (16, 0, [(9, 1)] * 3 + [(9, 11)] * 3 + [(3, 70)], False),  # 35 other tokens
+    (16, 0, [(70, 1)] * 1100 + [(0, 2200)], True), (16, 0, [(70, 1)] * 1101 + [(0, 2200)], False),
     (16, 0, [(900, 11), (3, 1)], False), (200, 45, [(0, 2000), (100, 700), (7, 1)], True), (1, 0, [(3000, 1000)], True)])
 def test_expand_plan_takes_all_prompts_or_none(gpu, H, window, reqs, taken):
     """At the limits of requests, of keys and of units' fill; the work lists of what is taken name every block of its keys and
