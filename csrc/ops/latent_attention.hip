@@ -799,7 +799,8 @@ __device__ __forceinline__ void pair_item(const Args& A, const int4 it, char* sm
 // buffers), one barrier each; the two waves' outputs meet in LDS. 4,096 tokens, 16 heads: 125 us back to back with the merge
 // launch (MFMAs 38, without the softmax 102, without the loads 104: LDS reads, 1,280 cycles a stage as the MFMAs, and the
 // softmax's 1,600 of a SIMD's VALU overlap in part); pair_item takes 318 and two head projections of 32 each, here the
-// expansion's 25. 499 tokens after 3,584: 49 and 25 us, 110 and 22 in the absorbed form.
+// expansion's 25. 499 tokens after 3,584: 49 and 25 us, 110 and 22 in the absorbed form. (In a step's launches: 132 and 6 for the
+// merge, 28; 38 and 12, 27.)
 constexpr int X_BLOCK = (2 * X_DIM + X_ROT) * 32, X_STAGE = 4 * X_BLOCK;  // bytes of 16 keys, of a stage
 
 // stages [lo, hi) of 64 keys that the tokens of a tile see

@@ -91,9 +91,10 @@ EXPAND_COLS, EXPAND_REQS = 128, 64
 def expand_pays(T: int, slots: int) -> bool:
     """Whether a step of T rows has the plan and the launch a layer that the form takes, in an engine of `slots` requests.
     By what a captured step knows, so that its outputs depend on its tokens alone; the plan refuses on the device what does
-    not pay (expand_plan_kernel), and then costs 1 to 2 %. From twice as many rows as slots on, at most half of them decode. A step of 8 layers of 16 heads, us, without the plan and with it: 256 slots, one prompt of 512 tokens 2,924, 2,636,
-    of 2,000 4,726, 4,124, 4 of 400 beside 30 decode rows 3,977, 3,806, one of 500 after 700 beside 200 3,602, 3,389;
-    below, 4 of 60 beside 30 2,521, 2,559, 64 decode rows alone 2,256, 2,285; 16 slots, one of 260 2,574, 2,484."""
+    not pay (expand_plan_kernel), and then costs 1 to 2 %. From twice as many rows as slots on, at most half of them decode.
+    A step of 8 layers of 16 heads, us, without the plan and with it: 256 slots, one prompt of 512 tokens 2,935, 2,655, of
+    2,000 4,941, 4,282, 4 of 400 beside 30 decode rows 3,973, 3,796, one of 500 after 700 beside 200 3,623, 3,411; below, 4 of 60
+    beside 30 2,521, 2,559, 64 decode rows alone 2,256, 2,285; 16 slots, one of 260 2,574, 2,484."""
     return T >= max(256, 2 * slots)
 
 
