@@ -436,7 +436,7 @@ def test_latent_attention_window_edge(gpu, edge, reqs):
 # at least, keys split into parts (few tokens after many), none of them
 EXPANDED = {"one": [(0, 300)], "edges": [(0, 128), (0, 129), (8, 64), (0, 63), (63, 155), (63, 65), (500, 1)],
             "parts": [(2100, 260), (700, 1), (0, 20)], "mixed": [(33, 1), (300, 300), (900, 20), (0, 700), (5, 1), (100, 64)],
-            "few": [(900, 12), (70, 11), (0, 13)], "none": [(900, 11), (300, 1)]}
+            "few": [(900, 12), (70, 11), (0, 13)], "none": [(900, 11), (300, 1)], "many": [(37 * i % 200, 65 + 9 * i) for i in range(12)] + [(250, 1), (8, 9)]}
 
 
 @pytest.mark.parametrize("window", [0, 45, 600])
