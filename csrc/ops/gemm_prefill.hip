@@ -743,17 +743,28 @@ extern "C" int pa_prefill_gemm(void* y, const void* x, const void* wp, const voi
 // gated unit. K % 64 == 0, K >= 128, N % 128 == 0; y rows 16-byte aligned.
 namespace pa {
 namespace pf {
+constexpr int RUN = 4;  // a power of two
 template <int EPI, int F>
 __global__ __launch_bounds__(512) void pingpong_grouped_kernel(Args A, const int4* __restrict__ tiles,
                                                                const int* __restrict__ n_tiles,
                                                                const int* __restrict__ order, long long wstride,
-                                                               int x_div, int out_order) {
+                                                               int x_div, int out_order, int one_group) {
   __shared__ __attribute__((aligned(1024))) char smem[(F == 8 ? 2 * 4 : 3 * 3) * PP_PART];
-  // column tiles of one row tile next to each other on one XCD: they share its rows of x
-  const int W = A.NT * n_tiles[0], per = (W + 7) >> 3;
+  // Column tiles of one row tile lie next to each other on one XCD: they share its rows of x. A single group's tiles go in
+  // blocks of RUN row tiles, column tile by column tile, so that an XCD takes in a block's rows and its own share of the
+  // weights once (beside the MFMAs, that is the bound). 2 x 8192 x 2048 outputs, us, one row tile after the other -> RUN 4:
+  // 1,000 rows 55.6 -> 54.2, 2,000 113 -> 106, 3,840 212 -> 201, 4,096 221 -> 208 (1.32 PFLOP/s); RUN 2 the last in 226, 8 as
+  // 4. Many groups have one or two tiles each and lose by it (4,096 tokens, 6 of 64 experts of 2 x 1408 x 2048: 294 -> 305).
+  const int n = n_tiles[0], W = A.NT * n, per = (W + 7) >> 3;
   const int b = blockIdx.x, w = (b & 7) * per + (b >> 3);
   if ((b >> 3) >= per || w >= W) return;
-  const int4 tl = tiles[w / A.NT];
+  int k = w / A.NT, nt = w - k * A.NT;
+  if (one_group) {
+    const int c0 = k & ~(RUN - 1), m = min(RUN, n - c0), j = w - c0 * A.NT;
+    nt = j / m;
+    k = c0 + j - nt * m;
+  }
+  const int4 tl = tiles[k];
   if (no_token(A.live, tl.y)) return;
   A.wp += (size_t)tl.x * wstride;
   A.M = tl.z;
@@ -767,12 +778,12 @@ __global__ __launch_bounds__(512) void pingpong_grouped_kernel(Args A, const int
   else A.y += (size_t)tl.y * A.ldy;
   A.MT = 1;
   // MT = 1: pingpong_tile's tile index is the column tile
-  pingpong_tile<EPI, false, false, F, true>(A, w % A.NT, A.NT, smem);
+  pingpong_tile<EPI, false, false, F, true>(A, nt, A.NT, smem);
 }
 }  // namespace pf
 }  // namespace pa
 
-extern "C" int pa_expert_tiles(void* y, const void* x, const void* wp, long long wstride, int N, int K, int ldx, int ldy,
+extern "C" int pa_expert_tiles(void* y, const void* x, const void* wp, long long wstride, int groups, int N, int K, int ldx, int ldy,
                                const int* tiles, int max_tiles, const int* n_tiles, const int* order, int x_div,
                                int out_order, int epi, float limit, float alpha, float cubic, float bias,
                                const float* row_w, const int* live, hipStream_t st) {
@@ -799,7 +810,7 @@ extern "C" int pa_expert_tiles(void* y, const void* x, const void* wp, long long
   const int grid = (a.NT * max_tiles + 7) / 8 * 8;
 #define PA_EX(E, F)                                                                                              \
   hipLaunchKernelGGL((pingpong_grouped_kernel<E, F>), dim3(grid), dim3(512), 0, st, a, (const int4*)tiles, n_tiles, \
-                     order, wstride, x_div, out_order)
+                     order, wstride, x_div, out_order, (int)(groups == 1))
   if (epi == EP_GLU) { if (wide) PA_EX(EP_GLU, 8); else PA_EX(EP_GLU, 4); }
   else if (epi == EP_RELU2) { if (wide) PA_EX(EP_RELU2, 8); else PA_EX(EP_RELU2, 4); }
   else { if (wide) PA_EX(EP_PLAIN, 8); else PA_EX(EP_PLAIN, 4); }

@@ -16,7 +16,7 @@
 // Sorted rows may have weights: the product is that of weight * x.
 #include "packed_epi.h"
 
-extern "C" int pa_expert_tiles(void* y, const void* x, const void* wp, long long wstride, int N, int K, int ldx, int ldy,
+extern "C" int pa_expert_tiles(void* y, const void* x, const void* wp, long long wstride, int groups, int N, int K, int ldx, int ldy,
                                const int* tiles, int max_tiles, const int* n_tiles, const int* order, int x_div,
                                int out_order, int epi, float limit, float alpha, float cubic, float bias, const float* row_w,
                                const int* live, hipStream_t st);
@@ -771,7 +771,7 @@ extern "C" int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out
     return (int)hipGetLastError();
   }
   if (tiles && tm == 256)
-    return pa_expert_tiles(out, x, w, wstride, N16 * 16, K32 * 32, ldx, ldo, tiles, max_tiles, n_tiles, order, x_div,
+    return pa_expert_tiles(out, x, w, wstride, groups, N16 * 16, K32 * 32, ldx, ldo, tiles, max_tiles, n_tiles, order, x_div,
                            out_order, epi == 1 ? pa::pk::EP_GLU : epi == 2 ? pa::pk::EP_RELU2 : pa::pk::EP_PLAIN, limit, alpha, cubic, bias, row_w, live, st);
   if (epi == 4) {  // tiles as large as leave most of the chip busy
 #define PA_SK(MT, NT)                                                                                                       \

@@ -221,6 +221,12 @@ def test_sorted_rows_of_whole_tiles(gpu, counts, N, K):
     sorted_rows(gpu, 256, counts, N, K)
 
 
+@pytest.mark.parametrize("rows", [1, 257, 1024, 1025, 1600, 2049])  # below, at and past a block of four row tiles, a second block's 1 to 4
+@pytest.mark.parametrize("N,K", [(1280, 128), (384, 192)])  # 5 columns of 256 and 3 of 128: XCDs start amid a block
+def test_row_tiles_of_one_group(gpu, rows, N, K):
+    sorted_rows(gpu, 256, [rows], N, K)
+
+
 @pytest.mark.parametrize("dt", DTYPES)
 @pytest.mark.parametrize("NQ,R,r,rd,H", [(72, 104, 48, 48, 3), (50, 70, 24, 12, 5), (256, 512, 64, 64, 2)])
 def test_latent_cache_and_query_rotation(gpu, dt, NQ, R, r, rd, H):
