@@ -28,8 +28,8 @@
 //     profiles/r3_pingpong_ph2_ab.jsonl.)
 //   * s_setprio(1) around every MFMA cluster (guide §5.5 T5).
 //
-// Work items are those of the prefill launcher: whole tiles (XCD-aware bijective remap, row
-// tiles of one W panel on one XCD) and, for the remainder, K-slices whose fp32 partials
+// Work items are those of the prefill launcher: whole tiles (XCD-aware bijective remap, blocks of
+// row tiles column by column: gemm_prefill.hip block_rows) and, for the remainder, K-slices whose fp32 partials
 // are handed to the tile's last arriver through common.h handoff_last.
 #pragma once
 #include "common.h"
@@ -94,7 +94,16 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
     kt0 = slice * A.per;
     kt1 = min(KT, kt0 + A.per);
   }
-  const int mt = tile % A.MT, nt = tile / A.MT;
+  int mt = tile % A.MT, nt = tile / A.MT;
+  if constexpr (!GR) {
+    // blocks of A.run row tiles: of the column tiles that run whole, and of those that are split (unless a column is both)
+    const int whole = A.full / A.MT, c0 = nt < whole ? 0 : whole, cols = nt < whole ? whole : A.NT - whole;
+    if (nt < whole || A.full == whole * A.MT) {
+      const int at = tile - c0 * A.MT, first = at / (A.run * cols) * A.run, m = min(A.run, A.MT - first), j = at - first * cols;
+      nt = c0 + j / m;
+      mt = first + j % m;
+    }
+  }
   const int row0 = mt * 256;
   if constexpr (!GR)
     if (no_token(A.live, row0)) return;

@@ -39,6 +39,7 @@
 #include "packed_epi.h"
 
 #include <algorithm>
+#include <cmath>
 #include <type_traits>
 
 namespace pa {
@@ -78,6 +79,7 @@ struct Args {
   // optional, by row: below 0 behind the last token of a step that is padded to the size its graph was captured for. Tiles
   // of 256 rows that begin there are left out, all slices of a split one alike; the rows they would write keep what was there
   const int* live = nullptr;
+  int run = 1;  // row tiles of a block (ping-pong kernels)
 };
 
 __device__ __forceinline__ bool no_token(const int* live, int row) { return live && live[row] < 0; }
@@ -589,6 +591,18 @@ static void plan_default(int M, int N, int K, int bn, int& full, int& S) {
   }
 }
 
+// The ping-pong kernels go through their tiles in blocks of so many row tiles, column tile by column tile. An XCD's P = 32 tiles
+// in flight (or its eighth of fewer) are then R row tiles of C = P / R column tiles each, and it takes in 256 R rows of x
+// and bn C of the weights, fewest at R = sqrt(P bn / 256): 4 row tiles of 128 columns, 5.7 of 256. Blocks are as even as they
+// come near that. us, all row tiles one block -> so: 4,096 x 2048 x 8192 (rows, outputs, inputs; 256 x 128 tiles) 120 -> 113,
+// x 2048 x 4096 62.1 -> 59.4, x 10368 x 2048 177 -> 168, 2,000 x 2048 x 8192 70.7 -> 67.6, 1,930 x 4096 x 14336 (two slices of k,
+// P = 16) 193 -> 189. One block where that is nearer: 1,300 x 28672 x 4096 265 in one of 6, 275 in 4 and 2.
+static int block_rows(int MT, int tiles, int bn) {
+  const double R = std::sqrt(std::max(1, std::min(32, tiles / 8)) * bn / 256.);
+  const int blocks = std::max(1, (int)(MT / R + 0.5));
+  return (MT + blocks - 1) / blocks;
+}
+
 // Tile width when the caller leaves it open: 256 x 128 tiles for the narrow projections
 // (N <= 6,144: qkv / o / down of Llama-3-8B, 0.6-0.85x the 256-wide kernel's time at
 // M <= 1,024), 256 x 256 for wide ones (gate_up: 1.08x faster).
@@ -662,6 +676,7 @@ extern "C" int pa_prefill_gemm(void* y, const void* x, const void* wp, const voi
          (pa::bf16*)q_out, (pa::bf16*)k_cache, (pa::bf16*)v_cache, positions, slots, cos_sin, H, KV,
          pa::g_handoff_acquire};
   a.live = M > pa::LIVE_MIN_ROWS ? live : nullptr;
+  a.run = block_rows(MT, tiles, bn);
   const int grid = full + (tiles - full) * S;
   // Mixed tail (variant 3, the default, and 8; 9 = without it): full rounds of 256 x 256
   // tiles over the first c1 column tiles,
@@ -676,6 +691,7 @@ extern "C" int pa_prefill_gemm(void* y, const void* x, const void* wp, const voi
       const int nbig = c1 * MT;
       Args big = a;
       big.full = nbig;
+      big.run = block_rows(MT, nbig, 256);
       big.S = 1;
       big.per = KT;
       Args sm = a;
@@ -685,6 +701,7 @@ extern "C" int pa_prefill_gemm(void* y, const void* x, const void* wp, const voi
       sm.resid = a.resid ? a.resid + co : nullptr;
       sm.N = N - co;
       sm.NT = sm.N / 128;
+      sm.run = block_rows(MT, nsmall, 128);
       sm.full = nsmall;
       sm.S = 1;
       sm.per = KT;

@@ -26,7 +26,9 @@ def _bf(*shape, dev, scale=1.0):
     # more than one round of 256-wide tiles with a short tail (the default variant runs the
     # tail columns on 256 x 128 tiles in the same launch)
     (1024, 20480, 512, "rope_perm", True, -1, 0), (768, 24576, 256, "resid", False, -1, 0),
-    (1000, 28672, 256, "plain", False, -1, 0)])
+    (1000, 28672, 256, "plain", False, -1, 0),
+    # blocks of row tiles, the last one smaller: whole columns, a split from amid a column on, whole and split columns
+    (2100, 1280, 256, "plain", True, -1, 1), (2100, 1280, 512, "resid", False, 13, 2), (4000, 768, 512, "silu", False, 32, 2)])
 @pytest.mark.parametrize("bn,variant", [(256, 3), (256, 9), (256, 1), (128, 3), (128, 1)])
 def test_prefill_gemm(gpu, M, N, K, epi, norm, full, splits, bn, variant):
     """Every epilogue and the folded row norm; run twice so the self-resetting tickets of
