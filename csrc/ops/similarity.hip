@@ -11,7 +11,7 @@
 // (priority index range, tag-set intersection, is_expired) evaluated in-kernel.
 //
 // Stage 1 (one pass over the index for up to 64 queries): each workgroup owns a
-// slice of rows; its 16 (or 8) waves take 16-row groups and multiply them by EVERY query
+// slice of rows; its 16 waves take 16-row groups and multiply them by EVERY query
 // tile with v_mfma_f32_16x16x32_bf16 — index rows stream from HBM straight into
 // the A operand once (the index is stored in 16-row tiles, fragment-major:
 // [N/16][D/32][64 lanes][8], so each wave load is 1 KiB contiguous instead of
@@ -23,6 +23,8 @@
 // slice writes its top-k. Stage 2 (one WG per query) merges the slices' lists.
 #include "topk_select.h"
 
+#include <algorithm>
+
 namespace pa {
 
 constexpr int SIM_CAND = 512;     // candidate buffer per (slice, query), power of two
@@ -30,20 +32,20 @@ constexpr int SIM_MAXK = 64;
 constexpr int SIM_QT = 16;        // queries per MFMA tile (N = 16)
 constexpr int SIM_MAXQ = 64;      // queries per pass (4 tiles resident in LDS)
 constexpr int SIM_MAXD = 1024;    // LDS query capacity per query (bf16)
-// One round of a workgroup's waves x 16 rows a slice at least: 16 waves, 128 KB of row loads in flight per CU, or for few
-// queries 8 while they leave the CUs a slice at most, as a CU's share of the rows is what a small index waits for (20,000 rows,
-// 3 queries: 79 slices 20 us, 157 15). With many queries their work on the first round is (40 of 5,000 rows: 29 and 33).
-constexpr int SIM_FEW = 128, SIM_MANY = 256, SIM_FEW_Q = 16;  // rows of a round, queries
+// A round of 16 waves x 16 rows a slice at least, 128 KB of row loads in flight per CU. Few queries of an index of which no CU
+// has more than 8 waves' rows take cosine_short_kernel; with many queries their work on the first round is what they wait for
+// (40 of 5,000 rows: slices of 128 rows 29 us, of 256 33).
+constexpr int SIM_ROUND = 256, SIM_SHORT = 32768, SIM_FEW_Q = 16;  // rows of a round; rows and queries of a short index
+constexpr int SIM_THREADS = 4 * SIM_ROUND;
 constexpr int SIM_LIM = 2 * SIM_MAXK;  // entries of a buffer between rounds; a round may admit 256 more
 constexpr int SIM_KB = 8;         // k-steps per row-load batch (two batches in flight)
 constexpr int SIM_MAX_WG = 256;    // one resident workgroup per CU: the threshold warm-up is paid once per CU
 
-inline int sim_rows(int Q, int N) { return Q <= SIM_FEW_Q && N <= SIM_FEW * SIM_MAX_WG ? SIM_FEW : SIM_MANY; }
+inline bool sim_short(int Q, int N) { return Q <= SIM_FEW_Q && N <= SIM_SHORT; }
+inline int sim_short_waves(int N) { return N <= 4 * 16 * SIM_MAX_WG ? 4 : (N + 16 * SIM_MAX_WG - 1) / (16 * SIM_MAX_WG); }  // at most 8
 inline int sim_num_wg(int Q, int N) {
-  int nwg = (N + sim_rows(Q, N) - 1) / sim_rows(Q, N);
-  if (nwg > SIM_MAX_WG) nwg = SIM_MAX_WG;
-  if (nwg < 1) nwg = 1;
-  return nwg;
+  const int rows = sim_short(Q, N) ? 16 * sim_short_waves(N) : SIM_ROUND;
+  return std::max(1, std::min(SIM_MAX_WG, (N + rows - 1) / rows));
 }
 
 // Cut query buffer `gs/gr` to its best K and raise the threshold: one wave, no barrier, about a microsecond (a bitonic sort
@@ -88,7 +90,6 @@ __device__ __forceinline__ void compact_global(float* gs, int* gr, int* cnt, flo
   }
 }
 
-template <int SIM_THREADS>
 __global__ __launch_bounds__(SIM_THREADS) void cosine_stage1_kernel(
     float* __restrict__ ws_s, int* __restrict__ ws_r, float* __restrict__ cand_s, int* __restrict__ cand_r,
     const bf16* __restrict__ queries, const bf16* __restrict__ index, int Q, int N, int D, int K,
@@ -280,6 +281,90 @@ __global__ __launch_bounds__(SIM_THREADS) void cosine_stage1_kernel(
   }
 }
 
+// Few queries of a short index: a workgroup's slice is one 16-row tile a wave. All of a tile is on its way before the queries
+// are in LDS, and a slice's scores are chosen from in LDS, a wave a query, with no threshold and no buffers in memory (each
+// a trip that the whole launch waited for). Bound by latency: 3 queries of 20,011 rows x 1,024 15.2 -> 9.0 us (slices of 128 rows
+// through cosine_stage1_kernel before), of which the rows' 41 MB are 6; 16 of 32,768 25 -> 16.5, 1 of 1,000 x 256 8.9 -> 4.5.
+template <int KS>
+__global__ __launch_bounds__(512) void cosine_short_kernel(
+    float* __restrict__ ws_s, int* __restrict__ ws_r, const bf16* __restrict__ queries, const bf16* __restrict__ index, int Q, int N,
+    int D, int K, const int* __restrict__ row_prio, const uint64_t* __restrict__ row_tags, const float* __restrict__ row_exp,
+    const int* __restrict__ q_minp, const uint64_t* __restrict__ q_tags, float now) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];
+  const int QLD = D + 8, NW = blockDim.x >> 6, rows = 16 * NW, ksteps = D / 32;
+  bf16* qt = reinterpret_cast<bf16*>(smem);                                // [16][QLD], the first Q of them
+  uint32_t* keys = reinterpret_cast<uint32_t*>(smem + SIM_QT * QLD * 2);   // [16][rows]
+  const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int g = lane >> 4, col = lane & 15, r0 = blockIdx.x * rows + wid * 16;  // (the first row of a tile is below N or not at all)
+  const bf16* ap = index + (size_t)(min(r0, (N - 1) & ~15) >> 4) * ksteps * 512 + lane * 8;
+  bf16x8 a[KS];
+#pragma unroll
+  for (int m = 0; m < KS; ++m)
+    a[m] = m < ksteps ? __builtin_nontemporal_load(reinterpret_cast<const bf16x8*>(ap + 512 * m)) : bf16x8{};
+  // the words of this lane's four rows and of its query
+  int pr[4];
+  float ex[4];
+  uint64_t tg[4];
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const int row = min(r0 + 4 * g + r, N - 1);
+    pr[r] = row_prio[row];
+    ex[r] = row_exp[row];
+    tg[r] = row_tags[row];
+  }
+  const int q = min(col, Q - 1), minp = q_minp[q];
+  const uint64_t qtag = q_tags[q];
+  for (int v = threadIdx.x; v < Q * D / 8; v += blockDim.x) {
+    const int r = (v * 8) / D, c = (v * 8) % D;
+    *reinterpret_cast<bf16x8*>(qt + (size_t)r * QLD + c) = *reinterpret_cast<const bf16x8*>(queries + (size_t)r * D + c);
+  }
+  __syncthreads();
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  const bf16* qr = qt + (size_t)q * QLD + 8 * g;
+#pragma unroll
+  for (int m = 0; m < KS; ++m)
+    if (m < ksteps) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[m], *reinterpret_cast<const bf16x8*>(qr + 32 * m), acc, 0, 0, 0);
+  // lane holds rows r0 + 4 g + r for query col
+  constexpr uint32_t LOWEST = 0x007fffffu, HIGHEST = 0xff800000u;  // -inf, inf
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const bool passes = r0 + 4 * g + r < N && pr[r] >= minp && (tg[r] & qtag) == qtag && (ex[r] == 0.f || ex[r] > now);
+    const uint32_t key = ord_key(acc[r]);  // (neither -inf nor what is no number: by their places in the order)
+    keys[col * rows + wid * 16 + 4 * g + r] = passes && key > LOWEST && key <= HIGHEST ? key : 0;
+  }
+  __syncthreads();
+  for (int i = wid; i < Q; i += NW) {
+    uint32_t key[2];
+    int have = 0, at = 0;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      key[j] = 64 * j + lane < rows ? keys[i * rows + 64 * j + lane] : 0;
+      have += __popcll(__ballot(key[j] != 0));
+    }
+    uint32_t cut = 1;  // entries above it stay, and of those at it as many as there is room for
+    int room = K;
+    if (have >= K) {
+      cut = wave_select(key, K);
+#pragma unroll
+      for (int j = 0; j < 2; ++j) room -= __popcll(__ballot(key[j] > cut));
+    }
+    const size_t o = ((size_t)i * gridDim.x + blockIdx.x) * K;
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      const unsigned long long ties = __ballot(key[j] == cut);
+      const bool keep = key[j] > cut || (key[j] == cut && rank_in(ties) < room);
+      room -= __popcll(ties);
+      const unsigned long long kept = __ballot(keep);
+      if (keep) {
+        ws_s[o + at + rank_in(kept)] = key_value(key[j]);
+        ws_r[o + at + rank_in(kept)] = blockIdx.x * rows + 64 * j + lane;
+      }
+      at += __popcll(kept);
+    }
+    if (lane >= at && lane < K) { ws_s[o + lane] = -INFINITY; ws_r[o + lane] = -1; }
+  }
+}
+
 // Stage 2: one workgroup per query picks the best K of the slices' lists, PER entries a thread.
 template <int PER>
 __global__ __launch_bounds__(1024) void cosine_stage2_kernel(float* __restrict__ out_s, int* __restrict__ out_r,
@@ -335,18 +420,24 @@ extern "C" int pa_cosine_topk(float* out_scores, int* out_rows, void* workspace,
   int* ws_r = reinterpret_cast<int*>(ws_s + (size_t)Q * nwg * K);
   float* cand_s = reinterpret_cast<float*>(ws_r + (size_t)Q * nwg * K);
   int* cand_r = reinterpret_cast<int*>(cand_s + (size_t)nwg * pa::SIM_MAXQ * pa::SIM_CAND);
-  const int nqt = (Q + pa::SIM_QT - 1) / pa::SIM_QT, threads = pa::sim_rows(Q, N) * 4;
+  const int nqt = (Q + pa::SIM_QT - 1) / pa::SIM_QT, threads = pa::SIM_ROUND * 4;
   const size_t lds = (size_t)nqt * pa::SIM_QT * (D + 8) * 2 + pa::SIM_MAXQ * (4 + 4 + 4 + 8) + 16 +
                      threads / 4 * 16 + (size_t)nqt * pa::SIM_QT * 65 * 4;
-  static bool attr_set = false;
-  if (!attr_set) {
-    for (auto* k : {pa::cosine_stage1_kernel<512>, pa::cosine_stage1_kernel<1024>})
-      (void)hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
-    attr_set = true;
+  if (pa::sim_short(Q, N)) {
+    const int waves = pa::sim_short_waves(N);
+    auto* scan = D <= 256 ? pa::cosine_short_kernel<8> : D <= 512 ? pa::cosine_short_kernel<16> : pa::cosine_short_kernel<32>;
+    hipLaunchKernelGGL(scan, dim3(nwg), dim3(64 * waves), pa::SIM_QT * ((D + 8) * 2 + 16 * waves * 4), st, ws_s, ws_r,
+                       (const pa::bf16*)queries, (const pa::bf16*)index, Q, N, D, K, row_priority, row_tags, row_expiry, q_min_priority,
+                       q_tags, now);
+  } else {
+    static bool attr_set = false;
+    if (!attr_set) {
+      (void)hipFuncSetAttribute((const void*)pa::cosine_stage1_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+      attr_set = true;
+    }
+    hipLaunchKernelGGL(pa::cosine_stage1_kernel, dim3(nwg), dim3(threads), lds, st, ws_s, ws_r, cand_s, cand_r, (const pa::bf16*)queries,
+                       (const pa::bf16*)index, Q, N, D, K, row_priority, row_tags, row_expiry, q_min_priority, q_tags, now);
   }
-  auto* scan = threads == 512 ? pa::cosine_stage1_kernel<512> : pa::cosine_stage1_kernel<1024>;
-  hipLaunchKernelGGL(scan, dim3(nwg), dim3(threads), lds, st, ws_s, ws_r, cand_s, cand_r, (const pa::bf16*)queries,
-                     (const pa::bf16*)index, Q, N, D, K, row_priority, row_tags, row_expiry, q_min_priority, q_tags, now);
   static_assert(pa::SIM_MAX_WG * pa::SIM_MAXK <= 16 * 1024, "stage 2 holds all lists");
   auto* merge = nwg * K <= 1024 ? pa::cosine_stage2_kernel<1>
                                 : nwg * K <= 4096 ? pa::cosine_stage2_kernel<4> : pa::cosine_stage2_kernel<16>;

@@ -271,7 +271,9 @@ def test_sample_distribution(gpu):
     assert (emp - exp).abs().max().item() < 0.03
 
 
-@pytest.mark.parametrize("N,D,Q,K", [(20000, 1024, 5, 8), (150000, 256, 70, 64), (3000, 768, 17, 10)])
+@pytest.mark.parametrize("N,D,Q,K", [(20000, 1024, 5, 8), (150000, 256, 70, 64), (3000, 768, 17, 10),
+                                     # short indexes: slices of 4, 5 and 8 tiles, a last tile of one row, every width of the kernel
+                                     (1250, 96, 2, 64), (16384, 992, 16, 3), (16385, 288, 7, 33), (32768, 512, 15, 64), (32753, 64, 2, 1)])
 def test_cosine_topk(gpu, N, D, Q, K):
     torch.manual_seed(6)
     idx = torch.nn.functional.normalize(torch.randn(N, D), dim=1).to(torch.bfloat16)
@@ -575,7 +577,7 @@ def test_mid_qkv_rope(gpu, M, H, KV, K, fm, fn, splits):
 
 
 @pytest.mark.parametrize("storage", ["bf16", "q16"])
-@pytest.mark.parametrize("N,Q,K", [(100, 3, 64), (20_000, 16, 5), (20_000, 17, 33), (32_768, 16, 32), (32_769, 2, 9), (70_000, 5, 64)])
+@pytest.mark.parametrize("N,Q,K", [(100, 3, 64), (81, 2, 40), (20_000, 16, 5), (20_000, 17, 33), (32_768, 16, 32), (32_769, 2, 9), (70_000, 5, 64)])
 def test_lookup_begins_with_its_best(gpu, storage, N, Q, K):
     """The first round's threshold: rows of nothing but zeros (scores of 0), ties, rows that are not finite (they are never
     hits, and do not count as the best of their four), few rows that pass, and more queries than a short slice takes."""
