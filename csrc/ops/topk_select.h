@@ -123,6 +123,18 @@ struct Selection {
   uint32_t key[SEL];
   int row[SEL], n;
 };
+// The entries of s in order, behind a barrier
+__device__ __forceinline__ void write_ranked(const Selection& s, int K, float* out_s, int* out_r) {
+  const int n = min(s.n, SEL), t = threadIdx.x;
+  if (t < n) {
+    const uint32_t k = s.key[t];
+    const int r = s.row[t];
+    int rank = 0;
+    for (int j = 0; j < n; ++j) rank += s.key[j] > k || (s.key[j] == k && s.row[j] < r);
+    if (rank < K) { out_s[rank] = key_value(k); out_r[rank] = r; }
+  }
+  if (t < K && t >= n) { out_s[t] = -INFINITY; out_r[t] = -1; }
+}
 template <int N>
 __device__ __forceinline__ void write_best(const uint32_t (&key)[N], const int (&row)[N], uint32_t kth, int K, Selection& s,
                                            float* out_s, int* out_r) {
@@ -141,15 +153,7 @@ __device__ __forceinline__ void write_best(const uint32_t (&key)[N], const int (
 #pragma unroll
   for (int i = 0; i < N; ++i) take(key[i] == kth, key[i], row[i]);
   __syncthreads();
-  const int n = min(s.n, SEL), t = threadIdx.x;
-  if (t < n) {
-    const uint32_t k = s.key[t];
-    const int r = s.row[t];
-    int rank = 0;
-    for (int j = 0; j < n; ++j) rank += s.key[j] > k || (s.key[j] == k && s.row[j] < r);
-    if (rank < K) { out_s[rank] = key_value(k); out_r[rank] = r; }
-  }
-  if (t < K && t >= n) { out_s[t] = -INFINITY; out_r[t] = -1; }
+  write_ranked(s, K, out_s, out_r);
 }
 
 }  // namespace pa

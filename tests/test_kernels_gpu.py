@@ -295,6 +295,27 @@ def test_cosine_topk(gpu, N, D, Q, K):
     assert (r.cpu() == rr).float().mean().item() > 0.95
 
 
+@pytest.mark.parametrize("N,K", [(9000, 64), (20000, 33), (60000, 64), (60000, 5)])  # lists of up to 16,384 entries, of each width
+def test_best_rows_lie_together(gpu, N, K):
+    """The second stage of a lookup where the first's lists say little: all of the best in one slice, and all rows alike."""
+    g = torch.Generator().manual_seed(N + K)
+    idx = torch.nn.functional.normalize(torch.randn(N, 64, generator=g), dim=1)
+    q = torch.nn.functional.normalize(torch.randn(2, 64, generator=g), dim=1).to(torch.bfloat16)
+    idx[32:132] = torch.nn.functional.normalize(q[:1].float() + 0.02 * torch.randn(100, 64, generator=g), dim=1)
+    idx = idx.to(torch.bfloat16)
+    ints = lambda n, dt=torch.int32: torch.zeros(n, dtype=dt, device=gpu)  # noqa: E731
+    for rows in (idx, idx[32:33].expand(N, -1)):
+        packed = ops.pack_decode_weight(torch.cat([rows, rows[:-N % 16]]).to(gpu))
+        s, r = ops.cosine_topk(q.to(gpu), packed, N, K, ints(N), ints(N, torch.int64), torch.zeros(N, device=gpu), ints(2),
+                               ints(2, torch.int64), 0.0)
+        exact = q.double() @ rows.double().T
+        # (sums of 64 products in fp32)
+        torch.testing.assert_close(s.double().cpu(), exact.topk(K, 1).values, atol=64 * 2.0 ** -24, rtol=0)
+        r = r.long().cpu()
+        assert all(len(set(x.tolist())) == K for x in r)
+        torch.testing.assert_close(exact.gather(1, r), s.double().cpu(), atol=64 * 2.0 ** -24, rtol=0)
+
+
 @pytest.mark.parametrize("M,N,K", [(1, 4096, 4096), (13, 6144, 4096), (64, 28672, 4096), (64, 4096, 14336),
                                    (100, 4096, 4096), (128, 1024, 512), (37, 128256, 4096)])
 def test_skinny_gemm(gpu, M, N, K):
