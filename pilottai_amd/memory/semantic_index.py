@@ -324,17 +324,18 @@ class SemanticIndex:
                 self.pass_events.append(ev)
         return s, r
 
-    def _pass_event(self):
+    def _pass_event(self, stream=None):
         """(start, end) events around a pass, the first recorded, where passes are timed."""
         if self.pass_events is None or self.device.type != "cuda":
             return None
         ev = (torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True))
-        ev[0].record()
+        ev[0].record(stream)
         return ev
 
     def _search_host(self, q: torch.Tensor, k: int, min_priority, qmasks, now: Optional[float]):
         """search_tensors for a caller that waits for the answer, with filters as lists: (scores, rows) as arrays, [Q, k].
-        The pass reads queries and filters from pinned memory and writes its results there (ops.lookup_begin)."""
+        The pass reads queries and filters from pinned memory and writes its results there (ops.lookup_begin); over a bf16
+        index with queries of the host it is one native call (ops.lookup)."""
         Q, D = q.shape
         caller = torch.cuda.current_stream(self.device) if q.is_cuda else None
         words = []
@@ -349,22 +350,26 @@ class SemanticIndex:
             words.append(torch.from_numpy(to))
         here = None
         try:
-            with self._lock, self._stream_ctx():
-                here = self._stream
-                if caller is not None:
-                    here.wait_stream(caller)
-                q = q.detach().to(self.device if q.is_cuda else "cpu", torch.float32).contiguous()
-                ev = self._pass_event()
+            with self._lock:
+                here = self._own_stream()
                 t_now = self.now() if now is None else now - self.epoch
-                back, out, (minp, qt), qs = ops.lookup_begin(q, *words, k, self.storage == "q16")
-                filters = (self.priority, self.tagbits, self.expiry, minp, qt, t_now)
-                if self.storage == "q16":
-                    args = (*qs, self.hi, self.lo, self.rmeta, self.count, k, *filters, out)
-                    ops.q16_pass(*args, False, self._ws)
+                if self.storage == "bf16" and caller is None:
+                    q, ev = q.detach().to(torch.float32).contiguous(), self._pass_event(here)
+                    back = ops.lookup(q, *words, k, self.packed, self.count, self.priority, self.tagbits, self.expiry, t_now, here)
                 else:
-                    ops.cosine_topk(*qs, self.packed, self.count, k, *filters, workspace=self._ws, out=out[:2])
+                    with self._stream_ctx():
+                        if caller is not None:
+                            here.wait_stream(caller)
+                        q, ev = q.detach().to(self.device if caller is not None else "cpu", torch.float32).contiguous(), self._pass_event()
+                        back, out, (minp, qt), qs = ops.lookup_begin(q, *words, k, self.storage == "q16")
+                        filters = (self.priority, self.tagbits, self.expiry, minp, qt, t_now)
+                        if self.storage == "q16":
+                            args = (*qs, self.hi, self.lo, self.rmeta, self.count, k, *filters, out)
+                            ops.q16_pass(*args, False, self._ws)
+                        else:
+                            ops.cosine_topk(*qs, self.packed, self.count, k, *filters, workspace=self._ws, out=out[:2])
                 if ev is not None:
-                    ev[1].record()
+                    ev[1].record(here)
             here.synchronize()
             a = back.numpy()
             if self.storage == "q16" and a[2 * Q * k:].any():  # a slice refused a row that might be in the top-k
@@ -414,11 +419,14 @@ class SemanticIndex:
         this stream. Also pins the calling thread to the index's device."""
         if self.device.type != "cuda":
             return contextlib.nullcontext()
+        return torch.cuda.stream(self._own_stream())  # (and its device)
+
+    def _own_stream(self):
         if self._stream is None:
             # its own stream, at the default priority (work on streams of different priorities
             # has hung): a lookup pass shares the device with the engine's steps
             self._stream = torch.cuda.Stream(device=self.device)
-        return torch.cuda.stream(self._stream)  # (and its device)
+        return self._stream
 
     def memory_bytes(self) -> int:
         rows = sum(p.numel() * p.element_size() for _, p in self._planes())

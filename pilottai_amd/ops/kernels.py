@@ -288,6 +288,13 @@ def lookup_begin(q: torch.Tensor, masks: torch.Tensor, min_priority: torch.Tenso
     return back, (s, r, flags), (minp, tags), qs
 
 
+def lookup(q: torch.Tensor, masks: torch.Tensor, min_priority: torch.Tensor, K: int, index, n_valid: int, row_priority,
+           row_tags, row_expiry, now: float, stream: torch.cuda.Stream) -> torch.Tensor:
+    """lookup_begin and the passes over a bf16 index (cosine_topk) in one call, on `stream`. -> lookup_begin's results."""
+    return require_native().lookup(q, masks, min_priority, K, index, n_valid, row_priority, row_tags, row_expiry, now,
+                                   (stream.stream_id, stream.device_index, stream.device_type))
+
+
 def cosine_topk(queries, index, n_valid: int, K: int, row_priority, row_tags, row_expiry,
                 q_min_priority, q_tags, now: float, workspace: Optional[torch.Tensor] = None, out=None):
     """`out`: (scores, rows) to write to."""

@@ -280,3 +280,29 @@ def test_search_that_fails_waits_for_its_passes(gpu, monkeypatch, exact):
     assert idx._stream.query()
     monkeypatch.setattr(ops, "q16_pass", run)
     assert [r for r, _ in idx.search(v, 5, [0], [()])[0]]
+
+
+def test_search_in_one_call(gpu):
+    """A bf16 index and queries of the host: events lie around the pass, a call that raises has waited for its launches, and
+    threads on streams of their own get what one gets."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    idx, v = _small_index(gpu, "bf16")
+    args = (3, [0] * 70, [()] * 70)
+    want = idx.search(v[:70], *args)
+    idx.pass_events = []
+    assert idx.search(v[:70], *args) == want
+    (start, end), = idx.pass_events
+    assert start.elapsed_time(end) > 0
+    idx.pass_events = None
+    with pytest.raises(RuntimeError):  # (behind the queries' preparation)
+        idx.search(v[:70, :32], *args)
+    assert idx._stream.query()
+    before = torch.cuda.current_stream(gpu)
+
+    def one(i):
+        with torch.cuda.stream(torch.cuda.Stream(gpu)):
+            return idx.search(v[i:i + 1], 3, [0], [()])[0]
+    with ThreadPoolExecutor(4) as pool:
+        assert list(pool.map(one, range(70))) == want
+    assert torch.cuda.current_stream(gpu) == before
