@@ -9,7 +9,7 @@ int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out, long long
                     const int* order, int x_div, int out_order, int tm, int epi, float limit, float alpha, float cubic, float bias,
                     const int* positions, const float* cos_sin, int rskip, int r, int rp, int rd, const float* row_w,
                     const void* gate, int ldg, const void* table, const int* ids, int ldt, int tcol, int vocab, const int* skip,
-                    const int* live, hipStream_t st);
+                    const int* live, int always, hipStream_t st);
 }
 
 namespace {
@@ -91,7 +91,7 @@ void head_gemm(at::Tensor x, int64_t xg, at::Tensor w, at::Tensor out, int64_t o
                            x.size(0), N / 16, K / 32, nullptr, 0, nullptr, nullptr, 0, 0, 0, gate.has_value() ? 3 : 0, 0.f, 0.f,
                            0.f, 0.f, pos, cs, rskip, r, rp, rd, nullptr, gate.has_value() ? gate->data_ptr() : nullptr,
                            gate.has_value() ? gate->stride(0) : 0, nullptr, nullptr, 0, 0, 0,
-                           skip.has_value() ? ints(*skip, x.size(0), "skip") : nullptr, nullptr, cur_stream()),
+                           skip.has_value() ? ints(*skip, x.size(0), "skip") : nullptr, nullptr, 0, cur_stream()),
            "head_gemm");
 }
 
@@ -111,16 +111,16 @@ void table_gemm(at::Tensor x, at::Tensor w, at::Tensor out, at::Tensor table, at
   check_rc(pa_grouped_gemm(f, x.data_ptr(), w.data_ptr(), out.data_ptr(), N * K, 1, x.stride(0), 0, out.stride(0), 0,
                            x.size(0), N / 16, K / 32, nullptr, 0, nullptr, nullptr, 0, 0, 0, 4, (float)limit, (float)alpha,
                            (float)cubic, (float)bias, nullptr, nullptr, 0, 0, 0, 0, nullptr, nullptr, 0, table.data_ptr(),
-                           ints(ids, x.size(0), "ids"), table.stride(0), (int)tcol, table.size(0), nullptr, nullptr, cur_stream()),
+                           ints(ids, x.size(0), "ids"), table.stride(0), (int)tcol, table.size(0), nullptr, nullptr, 0, cur_stream()),
            "table_gemm");
 }
 
 // rows sorted by group: x row = order[p] / x_div (x_div 0: p), out row = out_order ? order[p] : p; epi 1: the gated
 // unit, 2: the square of relu; row_w: weights of x's rows by order[p] (epi 1);
-// live: tiles of 256 rows whose first position has an entry below 0 are left out
+// live: tiles of 256 rows whose first position has an entry below 0 are left out; always: the last groups, so many, hold every row
 void expert_gemm(at::Tensor x, at::Tensor w, at::Tensor out, at::Tensor tiles, at::Tensor n_tiles, at::Tensor order,
                  int64_t rows, int64_t x_div, bool out_order, int64_t tm, int64_t epi, double limit, double alpha,
-                 double bias, double cubic, Opt row_w, Opt live) {
+                 double bias, double cubic, Opt row_w, Opt live, int64_t always) {
   const int f = is_f32(x, "x");
   check_rows(x, x.scalar_type(), "x");
   check_rows(out, x.scalar_type(), "out");
@@ -135,12 +135,13 @@ void expert_gemm(at::Tensor x, at::Tensor w, at::Tensor out, at::Tensor tiles, a
                                ((uintptr_t)out.data_ptr() & 15) == 0),
               "expert_gemm: tiles of 256 rows need K % 64 == 0, K >= 128, N % 128 == 0");
   TORCH_CHECK(tiles.dim() == 2 && tiles.size(1) == 4, "tiles must be [n, 4]");
+  TORCH_CHECK(always == 0 || (always > 0 && always < G), "expert_gemm: always is a number of groups, fewer than there are");
   check_rc(pa_grouped_gemm(f, x.data_ptr(), w.data_ptr(), out.data_ptr(), N * K, G, x.stride(0), 0, out.stride(0), 0, 0,
                            N / 16, K / 32, ints(tiles, 4, "tiles"), tiles.size(0), ints(n_tiles, 1, "n_tiles"),
                            ints(order, rows, "order"), x_div, out_order ? 1 : 0, tm, (int)epi, (float)limit,
                            (float)alpha, (float)cubic, (float)bias, nullptr, nullptr, 0, 0, 0, 0, opt_f32(row_w, rows, "row_w"),
                            nullptr, 0, nullptr, nullptr, 0, 0, 0, nullptr,
-                           live.has_value() ? ints(*live, rows, "live") : nullptr, cur_stream()),
+                           live.has_value() ? ints(*live, rows, "live") : nullptr, (int)always, cur_stream()),
            "expert_gemm");
 }
 

@@ -761,25 +761,56 @@ extern "C" int pa_prefill_gemm(void* y, const void* x, const void* wp, const voi
 namespace pa {
 namespace pf {
 constexpr int RUN = 4;  // a power of two
-template <int EPI, int F>
+enum { IN_ORDER = 0, ONE_GROUP = 1, HEAVY_FIRST = 2 };  // how a launch goes through its tiles (an instance each: others lose 0.3 % by the choice)
+template <int EPI, int F, int WALK>
 __global__ __launch_bounds__(512) void pingpong_grouped_kernel(Args A, const int4* __restrict__ tiles,
                                                                const int* __restrict__ n_tiles,
                                                                const int* __restrict__ order, long long wstride,
-                                                               int x_div, int out_order, int one_group) {
+                                                               int x_div, int out_order, int heavy) {
   __shared__ __attribute__((aligned(1024))) char smem[(F == 8 ? 2 * 4 : 3 * 3) * PP_PART];
   // Column tiles of one row tile lie next to each other on one XCD: they share its rows of x. A single group's tiles go in
   // blocks of RUN row tiles, column tile by column tile, so that an XCD takes in a block's rows and its own share of the
   // weights once (beside the MFMAs, that is the bound). 2 x 8192 x 2048 outputs, us, one row tile after the other -> RUN 4:
   // 1,000 rows 55.6 -> 54.2, 2,000 113 -> 106, 3,840 212 -> 201, 4,096 221 -> 208 (1.32 PFLOP/s); RUN 2 the last in 226, 8 as
   // 4. Many groups have one or two tiles each and lose by it (4,096 tokens, 6 of 64 experts of 2 x 1408 x 2048: 294 -> 305).
-  const int n = n_tiles[0], W = A.NT * n, per = (W + 7) >> 3;
-  const int b = blockIdx.x, w = (b & 7) * per + (b >> 3);
-  if ((b >> 3) >= per || w >= W) return;
-  int k = w / A.NT, nt = w - k * A.NT;
-  if (one_group) {
-    const int c0 = k & ~(RUN - 1), m = min(RUN, n - c0), j = w - c0 * A.NT;
+  // Groups from number `heavy` on hold every row. Their tiles, the last of the list and full ones whose products take longer
+  // than the others' weights, were all on one XCD, behind the others; they go first, the same number on each XCD (6 of 64 such experts and
+  // one for all, gate and up, us: 260 tokens 137 -> 131, 700 151 -> 140, 1,000 157 -> 146, 1,500 194 -> 191, 2,000 205 -> 205, 4,000
+  // 333 -> 316. The second product, of fewer columns, gains nothing up to 1,500 tokens and loses 2 % at 2,000 to 3,000.)
+  const int n = n_tiles[0], xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+  // item i of this XCD's share of `count` tiles from `first` on; false: it has fewer
+  int k = 0, nt = 0;
+  auto in_order = [&](int i, int count) {
+    const int items = count * A.NT, per = (items + 7) >> 3, w = xcd * per + i;
+    k = w / A.NT;
+    nt = w - k * A.NT;
+    return i < per && w < items;
+  };
+  auto in_blocks = [&](int i, int first, int count) {
+    const int items = count * A.NT, per = (items + 7) >> 3, w = xcd * per + i;
+    const int c0 = w / A.NT & ~(RUN - 1), m = min(RUN, count - c0), j = w - c0 * A.NT;
+    if (i >= per || w >= items) return false;
     nt = j / m;
-    k = c0 + j - nt * m;
+    k = first + c0 + j - nt * m;
+    return true;
+  };
+  if constexpr (WALK == ONE_GROUP) {
+    if (!in_blocks(at, 0, n)) return;
+  } else if constexpr (WALK == IN_ORDER) {
+    if (!in_order(at, n)) return;
+  } else {
+    const int lane = threadIdx.x & 63;
+    int last = 0;  // tiles of the groups from `heavy` on
+    for (bool more = true; more;) {
+      const int t = n - 1 - last - lane;
+      const unsigned long long in = __ballot(t >= 0 && tiles[max(t, 0)].x >= heavy);
+      const int len = ~in ? __builtin_ctzll(~in) : 64;
+      last += len;
+      more = len == 64;
+    }
+    // (their eighths are rounded up: the last XCDs may have fewer, of which the others' share takes no notice)
+    const int per = (last * A.NT + 7) >> 3;
+    if (at < per ? !in_blocks(at, n - last, last) : !in_order(at - per, n - last)) return;
   }
   const int4 tl = tiles[k];
   if (no_token(A.live, tl.y)) return;
@@ -803,10 +834,11 @@ __global__ __launch_bounds__(512) void pingpong_grouped_kernel(Args A, const int
 extern "C" int pa_expert_tiles(void* y, const void* x, const void* wp, long long wstride, int groups, int N, int K, int ldx, int ldy,
                                const int* tiles, int max_tiles, const int* n_tiles, const int* order, int x_div,
                                int out_order, int epi, float limit, float alpha, float cubic, float bias,
-                               const float* row_w, const int* live, hipStream_t st) {
+                               const float* row_w, const int* live, int always, hipStream_t st) {
   using namespace pa::pf;
   if (K % 64 || K < 128 || N % 128 || ldx % 8 || ldy % 8 || (epi != EP_PLAIN && epi != EP_GLU && epi != EP_RELU2)) return -1;
   if (max_tiles <= 0) return 0;
+  if (always < 0 || (groups > 1 && always >= groups)) return -1;
   Args a{};
   a.y = (pa::bf16*)y;
   a.x = (const pa::bf16*)x;
@@ -824,13 +856,20 @@ extern "C" int pa_expert_tiles(void* y, const void* x, const void* wp, long long
   a.bias = bias;
   const bool wide = N % 256 == 0;
   a.NT = N / (wide ? 256 : 128);
-  const int grid = (a.NT * max_tiles + 7) / 8 * 8;
-#define PA_EX(E, F)                                                                                              \
-  hipLaunchKernelGGL((pingpong_grouped_kernel<E, F>), dim3(grid), dim3(512), 0, st, a, (const int4*)tiles, n_tiles, \
-                     order, wstride, x_div, out_order, (int)(groups == 1))
+  const int grid = (a.NT * max_tiles + 7) / 8 * 8 + (always ? 8 : 0);  // (two shares may both be rounded up)
+#define PA_EXW(E, F, W)                                                                                             \
+  hipLaunchKernelGGL((pingpong_grouped_kernel<E, F, W>), dim3(grid), dim3(512), 0, st, a, (const int4*)tiles, n_tiles, \
+                     order, wstride, x_div, out_order, groups - always)
+#define PA_EX(E, F)                                   \
+  do {                                                \
+    if (groups == 1) PA_EXW(E, F, ONE_GROUP);         \
+    else if (always) PA_EXW(E, F, HEAVY_FIRST);       \
+    else PA_EXW(E, F, IN_ORDER);                      \
+  } while (0)
   if (epi == EP_GLU) { if (wide) PA_EX(EP_GLU, 8); else PA_EX(EP_GLU, 4); }
   else if (epi == EP_RELU2) { if (wide) PA_EX(EP_RELU2, 8); else PA_EX(EP_RELU2, 4); }
   else { if (wide) PA_EX(EP_PLAIN, 8); else PA_EX(EP_PLAIN, 4); }
+#undef PA_EXW
 #undef PA_EX
   return (int)hipGetLastError();
 }

@@ -19,7 +19,7 @@
 extern "C" int pa_expert_tiles(void* y, const void* x, const void* wp, long long wstride, int groups, int N, int K, int ldx, int ldy,
                                const int* tiles, int max_tiles, const int* n_tiles, const int* order, int x_div,
                                int out_order, int epi, float limit, float alpha, float cubic, float bias, const float* row_w,
-                               const int* live, hipStream_t st);
+                               const int* live, int always, hipStream_t st);
 
 namespace pa {
 namespace gg {
@@ -743,14 +743,15 @@ extern "C" int pa_table_route(const int* tables, const int* desc, int layers, co
   return (int)hipGetLastError();
 }
 
-// tm: rows per sorted tile (16, 32, 64, 128 or 256; dense: the kernel's choice by row count)
+// tm: rows per sorted tile (16, 32, 64, 128 or 256; dense: the kernel's choice by row count). always: so many of the last
+// groups hold every row (pa_expert_tiles; the others do not look at it)
 extern "C" int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out, long long wstride, int groups,
                                int ldx, int xg, int ldo, int og, int rows, int N16, int K32, const int* tiles,
                                int max_tiles, const int* n_tiles, const int* order, int x_div, int out_order, int tm,
                                int epi, float limit, float alpha, float cubic, float bias, const int* positions,
                                const float* cos_sin, int rskip, int r, int rp, int rd, const float* row_w, const void* gate,
                                int ldg, const void* table, const int* ids, int ldt, int tcol, int vocab, const int* skip,
-                               const int* live, hipStream_t st) {
+                               const int* live, int always, hipStream_t st) {
   if (skip && (fp32 || tiles || epi == 4)) return -1;
   if (N16 <= 0 || K32 <= 0 || (epi == 1 && N16 % 2)) return -1;
   if (row_w && (!tiles || epi != 1 || !x_div)) return -1;
@@ -772,7 +773,7 @@ extern "C" int pa_grouped_gemm(int fp32, const void* x, const void* w, void* out
   }
   if (tiles && tm == 256)
     return pa_expert_tiles(out, x, w, wstride, groups, N16 * 16, K32 * 32, ldx, ldo, tiles, max_tiles, n_tiles, order, x_div,
-                           out_order, epi == 1 ? pa::pk::EP_GLU : epi == 2 ? pa::pk::EP_RELU2 : pa::pk::EP_PLAIN, limit, alpha, cubic, bias, row_w, live, st);
+                           out_order, epi == 1 ? pa::pk::EP_GLU : epi == 2 ? pa::pk::EP_RELU2 : pa::pk::EP_PLAIN, limit, alpha, cubic, bias, row_w, live, always, st);
   if (epi == 4) {  // tiles as large as leave most of the chip busy
 #define PA_SK(MT, NT)                                                                                                       \
   do {                                                                                                                      \

@@ -608,7 +608,7 @@ class ScoredExperts:
                         s.groups, s.keep, s.always, tm, softmax=s.softmax, correction=self.correction, share=s.share, scale=s.scale)
         act = torch.empty(rows, self.fp, dtype=self.dtype, device=dev)
         ops.expert_gemm(h, self.w13, act, tiles, n_tiles, order, rows, x_div=K, out_order=False, tm=tm, glu=s.act,
-                        relu2=s.act is None, row_w=weights if s.weigh_input else None)
+                        relu2=s.act is None, row_w=weights if s.weigh_input else None, always=s.always)
         y = torch.empty(rows, self.dn, dtype=self.dtype, device=dev)
         ops.expert_gemm(act, self.w2, y, tiles, n_tiles, order, rows, x_div=0, out_order=True, tm=tm)
         return y, K, None if s.weigh_input else weights, None

@@ -158,7 +158,7 @@ def test_table_experts(gpu, dt, tm, T, E, top, ff, D):
             torch.testing.assert_close(y[t, k], (a * torch.sigmoid(1.702 * a) * (u + 1)) @ w2[e].float().T, **tol(dt))
 
 
-def sorted_rows(gpu, tm, counts, N, K):
+def sorted_rows(gpu, tm, counts, N, K, always=0):
     """The grouped projections of sorted rows of one tile size: plain, the square of relu and gated with weights of rows,
     gathered and scattered. Sums of K products in fp32 err by K 2^-24 of their magnitudes at most, a bf16 result rounds by
     2^-8; silu(g) u moves by at most 1.1 |u| dg + |g| du."""
@@ -189,7 +189,7 @@ def sorted_rows(gpu, tm, counts, N, K):
     for relu2 in (False, True):
         want = z.clamp(min=0) ** 2 if relu2 else z
         err = 2.0 ** -8 * want.abs() + slack * ((2 * z.abs() + slack) if relu2 else 1)
-        ops.expert_gemm(x, pw, out[:, :N], *args, x_div=top, out_order=True, tm=tm, relu2=relu2)
+        ops.expert_gemm(x, pw, out[:, :N], *args, x_div=top, out_order=True, tm=tm, relu2=relu2, always=always)
         assert bool(((out[order.long(), :N].float() - want).abs() <= err).all()) and bool((out[:, N:] == 9.0).all())
     if N % 32:
         return
@@ -200,7 +200,7 @@ def sorted_rows(gpu, tm, counts, N, K):
     want = torch.nn.functional.silu(a) * u
     err = 2.0 ** -8 * want.abs() + 1.1 * u.abs() * sl[:, :, 0] + a.abs() * sl[:, :, 1] + 2.0 ** -20 * want.abs() + 1e-30
     out = torch.empty(rows, N // 2, dtype=torch.bfloat16, device=gpu)
-    ops.expert_gemm(x, pw, out, *args, x_div=top, out_order=False, tm=tm, glu=(3e38, 1.0, 0.0), row_w=rw)
+    ops.expert_gemm(x, pw, out, *args, x_div=top, out_order=False, tm=tm, glu=(3e38, 1.0, 0.0), row_w=rw, always=always)
     assert bool(((out.float() - want.reshape(rows, -1)).abs() <= err.reshape(rows, -1)).all())
 
 
@@ -219,6 +219,23 @@ def test_sorted_rows(gpu, tm, counts, N, K):
 def test_sorted_rows_of_whole_tiles(gpu, counts, N, K):
     """Tiles of 256 rows that hold every number of their 64-row parts."""
     sorted_rows(gpu, 256, counts, N, K)
+
+
+@pytest.mark.parametrize("counts,always", [([3, 0, 70, 12] * 4 + [290], 1), ([40] * 3 + [1300], 1), ([9] * 5 + [600, 600], 2), ([0, 0, 513], 1),
+                                           ([20, 30, 0], 1), ([1] * 7 + [16400], 1)])  # of no rows; of more than 64 tiles
+@pytest.mark.parametrize("N,K", [(1280, 128), (384, 192)])
+def test_tiles_of_groups_of_every_row(gpu, counts, always, N, K):
+    sorted_rows(gpu, 256, counts, N, K, always)
+
+
+def test_groups_of_every_row_are_some(gpu):
+    from pilottai_amd import ops
+
+    x, w = torch.zeros(4, 128, device=gpu).bfloat16(), ops.pack_groups(torch.zeros(2, 128, 128, device=gpu), torch.bfloat16)
+    ints = lambda *n: torch.zeros(*n, dtype=torch.int32, device=gpu)  # noqa: E731
+    for always in (-1, 2):
+        with pytest.raises(RuntimeError):
+            ops.expert_gemm(x, w, x.clone(), ints(1, 4), ints(1), ints(4), 4, x_div=0, out_order=False, tm=256, always=always)
 
 
 @pytest.mark.parametrize("rows", [1, 257, 1024, 1025, 1600, 2049])  # below, at and past a block of four row tiles, a second block's 1 to 4
