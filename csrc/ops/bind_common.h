@@ -13,6 +13,7 @@ extern "C" {
 int pa_decode_gemm(void* y, const void* x, const void* wp, const void* resid, int M, int N, int K,
                    int ldx, int ldy, int ldr, int epi, int norm, float eps, int nt, int waves, int splits,
                    float* ws, long long ws_floats, int* counters, int n_counters, hipStream_t st);
+int pa_rows_sums(float* y, const void* x, const void* wp, int M, int N, int K, int S, int ldx, hipStream_t st);
 int pa_rows_gemm(void* y, const void* x, const void* wp, int M, int N, int K, int ldx, int ldy, hipStream_t st);
 int pa_prefill_gemm(void* y, const void* x, const void* wp, const void* resid, float* ws, long long ws_floats,
                     int* counters, int n_counters, int M, int N, int K, int ldx, int ldy, int ldr, int epi,
@@ -88,6 +89,19 @@ bool decode_gemm(at::Tensor y, at::Tensor x, at::Tensor wp, c10::optional<at::Te
                                 cp, cn, cur_stream());
   TORCH_CHECK(rc >= 0, "decode_gemm launch failed");
   return rc == 0;
+}
+
+// y [M * S, N] fp32: row m's sums over each of S slices of k, at m * S + slice (gemm_decode.hip pa_rows_sums)
+[[maybe_unused]] void rows_sums(at::Tensor y, at::Tensor x, at::Tensor wp, int64_t S) {
+  check_gpu(wp, "wp");
+  check_gpu(y, "y");
+  TORCH_CHECK(x.is_cuda() && x.dim() == 2 && x.stride(1) == 1, "x must be a 2-D GPU tensor, unit inner stride");
+  check_dtype(x, at::kBFloat16, "x"); check_dtype(wp, at::kBFloat16, "wp"); check_dtype(y, at::kFloat, "y");
+  TORCH_CHECK(wp.dim() == 4 && wp.size(2) == 64 && wp.size(3) == 8, "wp must be packed [N/16, K/32, 64, 8]");
+  const int M = x.size(0), K = x.size(1), N = wp.size(0) * 16;
+  TORCH_CHECK(wp.size(1) * 32 == K && y.dim() == 2 && y.size(0) == M * S && y.size(1) == N, "rows_sums sizes");
+  TORCH_CHECK(pa_rows_sums(y.data_ptr<float>(), x.data_ptr(), wp.data_ptr(), M, N, K, (int)S, x.stride(0), cur_stream()) == 0,
+              "rows_sums: ", S, " slices of ", K, " inputs, 16-byte aligned rows");
 }
 
 // y = x W^T on packed weights, as decode_gemm's plain form, for more rows (gemm_decode.hip dispatch_rows). Returns false if

@@ -6,7 +6,7 @@
 #include "bind_mixed.h"
 
 extern "C" {
-int pa_hyper_norm(int fp32, float* x, int S, const void* y, int K, int ldy, const float* y_w, const void* y2, int ldy2,
+int pa_hyper_norm(int fp32, float* x, int S, const void* y, const float* sums, int K, int ldy, const float* y_w, const void* y2, int ldy2,
                   const float* bias, const float* mix, const float* post, const float* pre, const void* emb, const int* ids, int vocab,
                   const float* w_next, void* out, int ldo, const int* rows, const int* live, int n, int D, float eps, hipStream_t st);
 int pa_softcap(int fp32, void* x, int ld, int rows, int cols, float cap, hipStream_t st);
@@ -45,7 +45,7 @@ int64_t seqs_of(const at::Tensor& block_table) {
 }
 
 void hyper_norm(at::Tensor x, Opt y, int64_t K, Opt y_w, Opt y2, Opt bias, Opt mix, Opt post, Opt pre, Opt emb, Opt ids,
-                Opt w_next, Opt out, Opt rows, double eps, Opt live) {
+                Opt w_next, Opt out, Opt rows, double eps, Opt live, Opt sums) {
   check_gpu(x, "x");
   check_dtype(x, at::kFloat, "x");
   TORCH_CHECK(x.dim() == 3, "x must be [T, streams, D]");
@@ -59,6 +59,13 @@ void hyper_norm(at::Tensor x, Opt y, int64_t K, Opt y_w, Opt y2, Opt bias, Opt m
     TORCH_CHECK(K >= 1 && y->size(0) == T * K && y->size(1) >= D && mix.has_value() && post.has_value(),
                 "y must be [T * K, >= D], with mix and post");
     ldy = y->stride(0);
+  }
+  if (sums.has_value()) {
+    check_gpu(*sums, "sums");
+    check_dtype(*sums, at::kFloat, "sums");
+    TORCH_CHECK(!y.has_value() && !y_w.has_value() && K >= 1 && sums->dim() == 2 && sums->size(0) == T * K && sums->size(1) >= D &&
+                    mix.has_value() && post.has_value(), "sums must be [T * K, >= D], in place of y, with mix and post");
+    ldy = sums->stride(0);
   }
   if (y2.has_value()) {
     check_rows(*y2, dt, "y2");
@@ -76,8 +83,8 @@ void hyper_norm(at::Tensor x, Opt y, int64_t K, Opt y_w, Opt y2, Opt bias, Opt m
     TORCH_CHECK(out->size(0) >= n && out->size(1) >= D && out->stride(0) == out->size(1), "out must be [>= n, >= D]");
     ldo = out->stride(0);
   }
-  check_rc(pa_hyper_norm(dt == at::kFloat, x.data_ptr<float>(), S, y.has_value() ? y->data_ptr() : nullptr, (int)K, ldy,
-                         opt_f32(y_w, T * K, "y_w"), y2.has_value() ? y2->data_ptr() : nullptr, ldy2, opt_f32(bias, D, "bias"), opt_f32(mix, S * S, "mix"),
+  check_rc(pa_hyper_norm(dt == at::kFloat, x.data_ptr<float>(), S, y.has_value() ? y->data_ptr() : nullptr,
+                         sums.has_value() ? sums->data_ptr<float>() : nullptr, (int)K, ldy, opt_f32(y_w, T * K, "y_w"), y2.has_value() ? y2->data_ptr() : nullptr, ldy2, opt_f32(bias, D, "bias"), opt_f32(mix, S * S, "mix"),
                          opt_f32(post, S, "post"), opt_f32(pre, S, "pre"), emb.has_value() ? emb->data_ptr() : nullptr,
                          emb.has_value() ? ints(*ids, T, "ids") : nullptr, emb.has_value() ? emb->size(0) : 0,
                          opt_f32(w_next, D, "w_next"), out.has_value() ? out->data_ptr() : nullptr, ldo,
@@ -288,5 +295,6 @@ PYBIND11_MODULE(_hybrid, m) {
   m.def("empty_uncached", &empty_uncached);
   m.def("decode_gemm", &decode_gemm);
   m.def("rows_gemm", &rows_gemm);
+  m.def("rows_sums", &rows_sums);
   m.def("prefill_gemm", &prefill_gemm);
 }

@@ -366,7 +366,8 @@ static int pick_nw(int nt, int waves, const DgArgs& a, hipStream_t st) {
 // column group reads whole: hence the largest tile that still gives every CU one (dispatch_rows).
 // us at 64 rows, before -> after (x from L2, cold weights): N x K 2048 x 8192 37 -> 20, 2048 x 4096 20 -> 11.4, 2048 x 2048
 // 11.7 -> 7.3, 10368 x 2048 17.8 -> 15.8, 128256 x 2048 144 -> 105.
-template <int MT, int NT, int WK, int D>
+// SUMS: a workgroup takes one of A.S slices of k and leaves its fp32 sums, row m's of slice s at y [M, A.S, N] (pa_rows_sums).
+template <int MT, int NT, int WK, int D, bool SUMS = false>
 __global__ __launch_bounds__(512) void decode_rows_kernel(const DgArgs A) {
   constexpr int WN = 8 / WK;                // waves side by side, NT tiles each
   constexpr int TM = MT * 16, TN = NT * WN * 16, NTH = 512;
@@ -378,10 +379,18 @@ __global__ __launch_bounds__(512) void decode_rows_kernel(const DgArgs A) {
   const int g = lane >> 4, c = lane & 15, wk = wid % WK, wn = wid / WK;
   const int xrow = threadIdx.x / LR, xu = threadIdx.x % LR;
   const int nwg = gridDim.x, bid = blockIdx.x, q = nwg / 8, rr = nwg % 8, xcd = bid % 8;
-  const int work = (xcd < rr ? xcd * (q + 1) : rr * (q + 1) + (xcd - rr) * q) + bid / 8;
+  int work = (xcd < rr ? xcd * (q + 1) : rr * (q + 1) + (xcd - rr) * q) + bid / 8;
   const int RG = (A.M + TM - 1) / TM;
+  const int K = A.K, KS = K / 32;
+  int slice = 0, first = 0, nst = (K + KC - 1) / KC;  // stages [first, nst)
+  if constexpr (SUMS) {  // (a slice's workgroups next to each other: they share its columns of x)
+    const int G = nwg / A.S, per = (nst + A.S - 1) / A.S;
+    slice = work / G;
+    work -= slice * G;
+    first = slice * per;
+    nst = min(nst, first + per);
+  }
   const int row0 = (work % RG) * TM, tile0 = (work / RG) * NT * WN, tiles = A.N / 16;
-  const int K = A.K, KS = K / 32, nst = (K + KC - 1) / KC;
   const bf16x8* wt[NT];
 #pragma unroll
   for (int j = 0; j < NT; ++j)
@@ -411,8 +420,9 @@ __global__ __launch_bounds__(512) void decode_rows_kernel(const DgArgs A) {
     __builtin_amdgcn_sched_barrier(0);
   };
 #pragma unroll
-  for (int d = 0; d < D; ++d) load(d, d);
-  for (int st0 = 0; st0 < nst; st0 += D) {
+  for (int d = 0; d < D; ++d)
+    if (!SUMS || first + d < nst) load(first + d, d);  // (the next stage may be another slice's)
+  for (int st0 = first; st0 < nst; st0 += D) {
 #pragma unroll
     for (int d = 0; d < D; ++d) {
       const int st = st0 + d;
@@ -437,7 +447,7 @@ __global__ __launch_bounds__(512) void decode_rows_kernel(const DgArgs A) {
                 acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[i], wb[d][u][j], acc[i][j], 0, 0, 0);
           }
         }
-        load(st + D, d);
+        if (!SUMS || st + D < nst) load(st + D, d);
       }
     }
   }
@@ -457,27 +467,31 @@ __global__ __launch_bounds__(512) void decode_rows_kernel(const DgArgs A) {
     for (int wv = 0; wv < WK; ++wv) t += *reinterpret_cast<const f32x4*>(red + wv * TM * TN + e);
     const int m = row0 + e / TN, n = tile0 * 16 + e % TN;
     if (m < A.M && n < A.N) {
-      bf16x4 o;
+      if constexpr (SUMS) {
+        *reinterpret_cast<f32x4*>(reinterpret_cast<float*>(A.y) + ((size_t)m * A.S + slice) * A.N + n) = t;
+      } else {
+        bf16x4 o;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) o[r] = (bf16)t[r];
-      *reinterpret_cast<bf16x4*>(A.y + (size_t)m * A.ldy + n) = o;
+        for (int r = 0; r < 4; ++r) o[r] = (bf16)t[r];
+        *reinterpret_cast<bf16x4*>(A.y + (size_t)m * A.ldy + n) = o;
+      }
     }
   }
 }
 
-template <int MT, int NT, int WK>
+template <int MT, int NT, int WK, bool SUMS = false>
 static int launch_rows(const DgArgs& a, hipStream_t st) {
   constexpr int D = 2;  // (4 stages deep: no faster)
   constexpr int TM = MT * 16, TN = NT * (8 / WK) * 16;
   constexpr size_t lds = std::max((size_t)2 * TM * (128 * WK + 16), (size_t)WK * TM * TN * sizeof(float));
   static_assert(lds <= 160 * 1024, "LDS of a CU");
-  auto kern = decode_rows_kernel<MT, NT, WK, D>;
+  auto kern = decode_rows_kernel<MT, NT, WK, D, SUMS>;
   static bool attr = false;
   if (!attr) {
     hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
     attr = true;
   }
-  hipLaunchKernelGGL(kern, dim3((a.N + TN - 1) / TN * ((a.M + TM - 1) / TM)), dim3(512), lds, st, a);
+  hipLaunchKernelGGL(kern, dim3((a.N + TN - 1) / TN * ((a.M + TM - 1) / TM) * (SUMS ? a.S : 1)), dim3(512), lds, st, a);
   return (int)hipGetLastError() == 0 ? 0 : -2;
 }
 
@@ -622,4 +636,15 @@ extern "C" int pa_rows_gemm(void* y, const void* x, const void* wp, int M, int N
   using namespace pa;
   DgArgs a{(bf16*)y, (const bf16*)x, (const bf16*)wp, nullptr, M, N, K, ldx, ldy, 0, 0.f, RopeArgs{}, 1, nullptr, nullptr};
   return dispatch_rows(a, st);
+}
+
+// y [M, S, N] fp32: the sums of x W^T over each of S slices of k, for a reader that adds them up; 1 if the sizes are not taken.
+extern "C" int pa_rows_sums(float* y, const void* x, const void* wp, int M, int N, int K, int S, int ldx, hipStream_t st) {
+  using namespace pa;
+  if (M <= 0) return 0;
+  const int stages = (K + 511) / 512;
+  if (S < 1 || S > stages || (stages + S - 1) / S * (S - 1) >= stages || K % 32 || N % 16 || ldx % 8 || (((uintptr_t)x | (uintptr_t)wp | (uintptr_t)y) & 15))
+    return 1;
+  DgArgs a{reinterpret_cast<bf16*>(y), (const bf16*)x, (const bf16*)wp, nullptr, M, N, K, ldx, 0, 0, 0.f, RopeArgs{}, S, nullptr, nullptr};
+  return M <= 32 ? launch_rows<2, 4, 8, true>(a, st) : launch_rows<4, 4, 8, true>(a, st);
 }

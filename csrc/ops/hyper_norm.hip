@@ -21,6 +21,7 @@ constexpr int MAX_S = 8;
 struct Args {
   float* x;             // [T, S, D]
   const void* y;        // [T, K, ldy]
+  const float* sums;    // [T, K, ldy] in place of y, or null
   const float* y_w;     // [T, K] or null
   const void* y2;       // [T, ldy2] or null
   const float* bias;    // [D] or null
@@ -48,11 +49,13 @@ __global__ __launch_bounds__(64 * NW) void hyper_norm_kernel(const Args A) {
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     pre[s] = A.pre ? A.pre[s] : 0.f;
-    post[s] = A.y ? A.post[s] : 0.f;
+    post[s] = A.y || A.sums ? A.post[s] : 0.f;
 #pragma unroll
-    for (int r = 0; r < S; ++r) mix[s][r] = A.y ? A.mix[s * S + r] : 0.f;
+    for (int r = 0; r < S; ++r) mix[s][r] = A.y || A.sums ? A.mix[s * S + r] : 0.f;
   }
+  const bool add = A.y || A.sums;
   const T* yr = (const T*)A.y + (size_t)t * A.K * A.ldy;
+  const float* sr = A.sums + (size_t)t * A.K * A.ldy;
   const float* yw = A.y_w ? A.y_w + (size_t)t * A.K : nullptr;
   const T* er = A.emb ? (const T*)A.emb + (size_t)min(max(A.ids[t], 0), A.vocab - 1) * D : nullptr;
   float ss = 0.f;
@@ -72,7 +75,7 @@ __global__ __launch_bounds__(64 * NW) void hyper_norm_kernel(const Args A) {
       for (int s = 0; s < S; ++s)
         __builtin_memcpy(x[s], __builtin_assume_aligned(xr + (size_t)s * D + i, 4 * VEC), 4 * VEC);
     }
-    if (A.y) {
+    if (add) {
       float y[VEC];
 #pragma unroll
       for (int j = 0; j < VEC; ++j) y[j] = A.bias ? A.bias[i + j] : 0.f;
@@ -81,8 +84,17 @@ __global__ __launch_bounds__(64 * NW) void hyper_norm_kernel(const Args A) {
 #pragma unroll
         for (int j = 0; j < VEC; ++j) y[j] += (float)a[j];
       }
+      if (A.sums) {
+#pragma unroll 8
+        for (int k = 0; k < A.K; ++k) {
+          float f[VEC];
+          __builtin_memcpy(f, __builtin_assume_aligned(sr + (size_t)k * A.ldy + i, 4 * VEC), 4 * VEC);
+#pragma unroll
+          for (int j = 0; j < VEC; ++j) y[j] += f[j];
+        }
+      }
 #pragma unroll 4
-      for (int k = 0; k < A.K; ++k) {
+      for (int k = 0; A.y && k < A.K; ++k) {
         __builtin_memcpy(a, __builtin_assume_aligned(yr + (size_t)k * A.ldy + i, sizeof(T) * VEC), sizeof(T) * VEC);
         const float w = yw ? yw[k] : 1.f;
 #pragma unroll
@@ -101,7 +113,7 @@ __global__ __launch_bounds__(64 * NW) void hyper_norm_kernel(const Args A) {
         for (int r = 0; r < S; ++r) x[r][j] = z[r];
       }
     }
-    if ((A.y || er) && !A.rows) {
+    if ((add || er) && !A.rows) {
 #pragma unroll
       for (int s = 0; s < S; ++s)
         __builtin_memcpy(__builtin_assume_aligned(xr + (size_t)s * D + i, 4 * VEC), x[s], 4 * VEC);
@@ -144,7 +156,7 @@ __global__ __launch_bounds__(256) void softcap_kernel(T* __restrict__ x, int ld,
 }  // namespace hn
 }  // namespace pa
 
-extern "C" int pa_hyper_norm(int fp32, float* x, int S, const void* y, int K, int ldy, const float* y_w,
+extern "C" int pa_hyper_norm(int fp32, float* x, int S, const void* y, const float* sums, int K, int ldy, const float* y_w,
                              const void* y2, int ldy2, const float* bias, const float* mix, const float* post, const float* pre, const void* emb,
                              const int* ids, int vocab, const float* w_next, void* out, int ldo, const int* rows, const int* live,
                              int n, int D, float eps, hipStream_t st) {
@@ -154,11 +166,11 @@ extern "C" int pa_hyper_norm(int fp32, float* x, int S, const void* y, int K, in
   // Rows without a token stay as they are in launches that look for them (a step of mudepel's 8 layers, 4 streams of 2,048
   // columns: 3,658 tokens in 4,096 rows 2 % of its 5,840 us, 2,101 in 3,072 3 % of 4,640)
   if (rows || n <= pa::LIVE_MIN_ROWS) live = nullptr;
-  const Args A{x, y, y_w, y2, bias, mix, post, pre, emb, ids, w_next, out, rows, live, K, ldy, ldy2, vocab, ldo, D, eps};
+  const Args A{x, y, sums, y_w, y2, bias, mix, post, pre, emb, ids, w_next, out, rows, live, K, ldy, ldy2, vocab, ldo, D, eps};
   // fewer rows than CUs: twice the waves to a row, all of it in one pass up to 2,048 columns (64 rows, 4 streams of 2,048:
   // 6.8 -> 5.7 us)
   const bool few = n <= 256 && D > 1024;
-  const bool vec = D % 4 == 0 && (!y || ldy % 4 == 0) && (!y2 || ldy2 % 4 == 0) && (!out || ldo % 4 == 0);
+  const bool vec = D % 4 == 0 && ((!y && !sums) || ldy % 4 == 0) && (!y2 || ldy2 % 4 == 0) && (!out || ldo % 4 == 0);
 #define PA_HN(T, V, N, W, ...)                                                                                  \
   do {                                                                                                          \
     static bool attr = false;                                                                                   \

@@ -31,6 +31,11 @@ class PackedLinear:
         y = ops.rows_gemm(x, self.w) if ops.rows_gemm_pays(x.shape[0], self.w.shape[0] * 16, x.shape[1]) else None
         return ops.prefill_gemm(x, self.w, live=live) if y is None else y
 
+    def parts(self, x: torch.Tensor, live: Optional[torch.Tensor] = None):
+        """(y, n) for a reader that adds up n rows of y a row: unrounded parts (fp32) where they are the faster form, else y itself."""
+        n = ops.rows_sums_slices(x.shape[0], self.N, self.K) if self.w.dim() == 4 and x.is_cuda else 1
+        return (self(x, live), 1) if n == 1 else (ops.rows_sums(x, self.w, n), n)
+
 
 def pad_heads(w: torch.Tensor, padded: int) -> torch.Tensor:
     """[heads, size, k] -> [heads, padded, k], zeros behind every head."""

@@ -443,9 +443,10 @@ class LinearAttention:
 
 class MixerBlock:
     """Mixers side by side on one projection and one output matrix. `mlp`: a GatedMLP that reads the same input and
-    whose second matrix is part of the output matrix."""
+    whose second matrix is part of the output matrix. `parts`: the output may come in unrounded parts (PackedLinear.parts)."""
 
-    def __init__(self, mixers: Sequence, dtype, device, mlp: Optional["GatedMLP"] = None):
+    def __init__(self, mixers: Sequence, dtype, device, mlp: Optional["GatedMLP"] = None, parts: bool = False):
+        self.parts = parts
         self.mixers, self.mlp, self.dtype, self.device = list(mixers), mlp, dtype, device
         self.at_in: List[int] = []
         self.at_out: List[int] = []
@@ -492,7 +493,8 @@ class MixerBlock:
             self.mlp.activate(h, out[:, self.at_out[-1]:self.at_out[-1] + self.mlp.fp], meta.slots)
         run = side.run if side is not None else lambda *fs, at=0: [f() for f in fs]
         run(mix, *([feed] if self.mlp is not None else []))
-        return self.o(out, meta.slots), 1, None, self.bias
+        y, n = self.o.parts(out, meta.slots) if self.parts else (self.o(out, meta.slots), 1)
+        return y, n, None, self.bias
 
 
 def _live(meta: Optional[StepMeta]):
@@ -508,11 +510,12 @@ def _pack_gate_up(gate, up, fp: int, dk: int, dtype, device):
 
 
 class GatedMLP:
-    """down(act(gate h) * up h): the gate and up rows interleaved in one grouped projection of one group."""
+    """down(act(gate h) * up h): the gate and up rows interleaved in one grouped projection of one group. `parts` as MixerBlock's."""
 
     SMALL, LARGE = 1 << 24, 1 << 26  # elements of weights: few workgroups; not found in the caches by the next tile again
 
-    def __init__(self, spec: DenseSpec, t: Dict[str, torch.Tensor], width: int, dtype, device, alone: bool = True):
+    def __init__(self, spec: DenseSpec, t: Dict[str, torch.Tensor], width: int, dtype, device, alone: bool = True, parts: bool = False):
+        self.parts = parts
         self.spec, self.dtype, self.device = spec, dtype, device
         self.dk, self.fp = pad_to(width, 64), pad_to(spec.ff, 64)
         self.w_out = t["down"]
@@ -539,7 +542,8 @@ class GatedMLP:
         act = torch.empty(h.shape[0], self.fp, dtype=self.dtype, device=self.device)
         live = _live(meta)
         self.activate(h, act, live)
-        return self.down(act, live), 1, None, None
+        y, n = self.down.parts(act, live) if self.parts else (self.down(act, live), 1)
+        return y, n, None, None
 
 
 class PolyMLP:

@@ -188,8 +188,9 @@ class MudepelModel(HybridModel):
                 mixer = StateSpace(L.mixer, sub("mix."), cfg.eps, dtype, dev)
             mlp = None
             if L.mlp is not None:
-                mlp = (GatedMLP if isinstance(L.mlp, DenseSpec) else ScoredExperts)(L.mlp, sub("mlp."), d, dtype, dev)
-            layer = {"mixer": MixerBlock([mixer], dtype, dev), "mlp": mlp}
+                mlp = GatedMLP(L.mlp, sub("mlp."), d, dtype, dev, parts=True) if isinstance(L.mlp, DenseSpec) else \
+                    ScoredExperts(L.mlp, sub("mlp."), d, dtype, dev)
+            layer = {"mixer": MixerBlock([mixer], dtype, dev, parts=True), "mlp": mlp}
             for q in (1, 2) if mlp else (1,):
                 layer[f"norm{q}"] = f32(1 + t[f"norm{q}"].float())
                 layer[f"hc{q}"] = {k: f32(v) for k, v in sub(f"hc{q}.").items()}
@@ -246,7 +247,6 @@ class MudepelModel(HybridModel):
             ops.softcap(logits, cfg.vocab_size, cfg.softcap)
         return logits[:, :cfg.vocab_size]
 
-    @staticmethod
-    def _into_streams(result, hc) -> dict:
+    def _into_streams(self, result, hc) -> dict:
         y, partials, weights, bias = result
-        return dict(y=y, partials=partials, y_weights=weights, bias=bias, mix=hc["mix"], post=hc["out"])
+        return dict([("y" if y.dtype == self.dtype else "sums", y)], partials=partials, y_weights=weights, bias=bias, mix=hc["mix"], post=hc["out"])

@@ -12,7 +12,7 @@ from typing import Optional, Tuple
 import torch
 
 from . import reference as ref
-from .kernels import MIXED, _on_gpu, require_family, require_hybrid
+from .kernels import MIXED, _on_gpu, require_family, require_hybrid, unpack_decode_weight
 from .latent import SCAN_CHUNK, SCAN_MIN, unpack_groups
 
 # (key width, value width) in 32s with MFMA kernels (window_attention.hip PA_WA_DIMS)
@@ -43,16 +43,31 @@ def hyper_norm(x: torch.Tensor, eps: float, *, y: Optional[torch.Tensor] = None,
                pre: Optional[torch.Tensor] = None, emb: Optional[torch.Tensor] = None,
                ids: Optional[torch.Tensor] = None, w_next: Optional[torch.Tensor] = None,
                out: Optional[torch.Tensor] = None, rows: Optional[torch.Tensor] = None,
-               live: Optional[torch.Tensor] = None):
+               live: Optional[torch.Tensor] = None, sums: Optional[torch.Tensor] = None):
     """x (fp32 [T, streams, D], in place): x_t = sum_s mix[s, t] x_s + post[t] (sum_k w_k y_k + y2 + bias), or
     x_t = emb[ids]; out = norm(sum_s pre[s] x_s) * w_next. Returns out. `rows`: out row i is row rows[i]'s,
     and x keeps its value. `live` (ints by row, without `rows`): rows from the first one below 0 on are padding and may be
-    left as they were."""
+    left as they were. `sums` (fp32 [T * partials, D]): unrounded partial sums in place of y (rows_sums)."""
     if _on_gpu(x):
         require_hybrid().hyper_norm(x, y, int(partials), y_weights, y2, bias, mix, post, pre, emb, ids, w_next, out, rows,
-                                    float(eps), live)
+                                    float(eps), live, sums)
         return out
-    return ref.hyper_norm(x, eps, y, partials, y_weights, y2, bias, mix, post, pre, emb, ids, w_next, out, rows)
+    return ref.hyper_norm(x, eps, sums if y is None else y, partials, y_weights, y2, bias, mix, post, pre, emb, ids, w_next, out, rows)
+
+
+def rows_sums(x: torch.Tensor, wp: torch.Tensor, slices: int) -> torch.Tensor:
+    """x W^T in parts that add up to it, fp32 [rows * slices, N]: row m's sums over each of `slices` slices of k (whole
+    stages of 512) at m * slices + slice; W packed by pack_decode_weight (csrc/ops/gemm_decode.hip pa_rows_sums)."""
+    M, K = x.shape
+    y = torch.empty(M * slices, wp.shape[0] * 16, dtype=torch.float32, device=x.device)
+    if _on_gpu(x):
+        require_hybrid().rows_sums(y, x, wp, int(slices))
+        return y
+    per = -(-(-(-K // 512)) // slices) * 512
+    w = unpack_decode_weight(wp).float()
+    for s in range(slices):
+        y.view(M, slices, -1)[:, s] = x[:, s * per:(s + 1) * per].float() @ w[:, s * per:(s + 1) * per].T
+    return y
 
 
 def softcap(x: torch.Tensor, cols: int, cap: float) -> torch.Tensor:

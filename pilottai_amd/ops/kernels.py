@@ -532,6 +532,18 @@ def rows_gemm(x: torch.Tensor, wp: torch.Tensor, out: Optional[torch.Tensor] = N
     return y if _packed_module().rows_gemm(y, x, wp) else None
 
 
+def rows_sums_slices(M: int, N: int, K: int) -> int:
+    """Slices of k in which rows_sums is the faster form for a reader that adds up (hyper_norm), 1 where it is not. As many as
+    leave 64 columns and up to 64 rows a workgroup a CU: what a workgroup takes in of x shrinks with its slice, where unsliced
+    tiles of few columns read all of x. us with the norm behind it, unsliced, sliced: 64 rows of 2048 x 8192 24.9, 18.2 (8), x 4096 16.5, 14.2,
+    x 2048 12.6, 12.9; 16 rows 18.4, 14.6, 13.1, 11.2; 128 rows 28.4, 22.0 (4), 18.6, 17.3; 256 rows 35.0, 28.8 (2), 22.3, 20.6; 768
+    x 3072, 64 rows 13.3, 11.9 (6); 3072 x 3072, 40 rows 16.2, 16.5 (3)."""
+    tiles, stages = -(-M // (32 if M <= 32 else 64)) * -(-N // 64), -(-K // 512)
+    n = min(stages, max(1, 256 // tiles))
+    n = -(-stages // -(-stages // n))  # (none empty)
+    return n if n >= 6 or (n >= 2 and K >= 4096) else 1
+
+
 # per-head tile order of the rope-fused QKV weights: tiles (i, i + 4) adjacent
 _ROPE_TILE_ORDER = (0, 4, 1, 5, 2, 6, 3, 7)
 

@@ -87,6 +87,80 @@ def test_hyper_norm_leaves_rows_without_a_token(gpu, T, live, S, D):
     assert torch.equal(xb[live:], x[live:]) and (b[live:] == 7.0).all()
 
 
+@pytest.mark.gpu
+# rows and columns of part of a tile, both row tiles and two of them; slices of a stage and of several, a last one of few steps
+@pytest.mark.parametrize("M,N,K,S", [(1, 64, 512, 1), (17, 144, 1088, 3), (32, 2048, 4096, 8), (33, 80, 1600, 2), (64, 192, 4160, 3), (65, 128, 6144, 6), (200, 2048, 4096, 2)])
+def test_rows_sums(gpu, M, N, K, S):
+    """Every slice's sums, unrounded: K products of bf16 in fp32 err by K 2^-24 of their magnitudes at most."""
+    from pilottai_amd import ops
+
+    g = torch.Generator(device=gpu).manual_seed(M + N + K)
+    x = torch.randn(M, K + 8, device=gpu, generator=g).bfloat16()[:, :K]
+    w = torch.randn(N, K, device=gpu, generator=g).bfloat16()
+    got = ops.rows_sums(x, ops.pack_decode_weight(w), S).view(M, S, N)
+    per = -(-(-(-K // 512)) // S) * 512
+    for s in range(S):
+        a, b = x[:, s * per:(s + 1) * per].double(), w[:, s * per:(s + 1) * per].double()
+        assert bool(((got[:, s] - a @ b.T).abs() <= K * 2.0 ** -24 * (a.abs() @ b.abs().T)).all())
+
+
+@pytest.mark.gpu
+def test_rows_sums_refuses_empty_slices(gpu):
+    from pilottai_amd import ops
+
+    x, w = torch.zeros(4, 2560, device=gpu).bfloat16(), ops.pack_decode_weight(torch.zeros(64, 2560, device=gpu).bfloat16())
+    for S in (0, 4, 6):  # (5 stages: 4 slices would be of 2, 2, 1 and 0)
+        with pytest.raises(RuntimeError):
+            ops.rows_sums(x, w, S)
+
+
+def test_slices_of_sums():
+    from pilottai_amd import ops
+
+    for M in (1, 16, 32, 33, 64, 65, 130, 256, 257, 2000):
+        for N in (128, 768, 2048, 4096, 10368):
+            for K in (64, 2048, 3072, 4160, 8192, 14336):
+                n, stages = ops.rows_sums_slices(M, N, K), -(-K // 512)
+                assert 1 <= n <= stages and -(-stages // n) * (n - 1) < stages
+                assert n == 1 or n * -(-M // (32 if M <= 32 else 64)) * -(-N // 64) <= 256
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,S,D,n", [(9, 4, 2048, 8), (300, 1, 100, 2), (20, 3, 50, 6)])  # whole 4s or not; both widths of a workgroup
+def test_hyper_norm_of_sums(gpu, T, S, D, n):
+    """Unrounded parts in place of y: as their sum, and refused beside y."""
+    from pilottai_amd import ops
+
+    g = gen(T)
+    x, w, parts = (torch.randn(*s, generator=g).to(gpu) for s in ((T, S, D), (D,), (T * n, D + 14)))
+    kw = dict(mix=torch.randn(S, S, generator=g).to(gpu), post=torch.randn(S, generator=g).to(gpu), pre=torch.rand(S, generator=g).to(gpu) + 0.1,
+              bias=torch.randn(D, generator=g).to(gpu), w_next=w, partials=n)
+    xs, out, want = x.clone(), torch.empty(T, D, dtype=BF16, device=gpu), torch.empty(T, D, device=gpu)
+    ops.hyper_norm(xs, 1e-5, sums=parts, out=out, **kw)
+    xw = x.double().cpu()
+    yw = parts.double().cpu().view(T, n, -1)[:, :, :D].sum(1) + kw["bias"].double().cpu()
+    xw = torch.einsum("st,nsd->ntd", kw["mix"].double().cpu(), xw) + kw["post"].double().cpu()[None, :, None] * yw[:, None]
+    torch.testing.assert_close(xs.double().cpu(), xw, rtol=1e-5, atol=1e-4)
+    ops.hyper_norm(x.clone(), 1e-5, y=parts, out=want, **kw)  # (all in fp32)
+    torch.testing.assert_close(out.float(), want, rtol=2.0 ** -8, atol=1e-5)
+    with pytest.raises(RuntimeError):
+        ops.hyper_norm(x.clone(), 1e-5, sums=parts, y=parts.to(BF16), out=out, **kw)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 20, 100])
+def test_linear_in_parts(gpu, M):
+    from pilottai_amd.models.common import PackedLinear
+
+    g = torch.Generator(device=gpu).manual_seed(M)
+    lin = PackedLinear(torch.randn(2000, 4100, device=gpu, generator=g) / 64, BF16, gpu)
+    x = torch.randn(M, lin.K, device=gpu, generator=g).to(BF16)
+    y, n = lin.parts(x)
+    assert n > 1 and y.dtype == torch.float32 and y.shape == (M * n, lin.N)
+    # (the other form is rounded, by 2^-9 of a value at most)
+    torch.testing.assert_close(y.view(M, n, -1).sum(1), lin(x).float(), rtol=2.0 ** -8, atol=1e-4)
+
+
 @kinds
 def test_softcap(device, dt):
     from pilottai_amd import ops
