@@ -498,8 +498,10 @@ static int launch_rows(const DgArgs& a, hipStream_t st) {
 // The smallest tile that leaves at most one workgroup a CU (a second round of workgroups, or half the CUs idle, both
 // measured slower for every shape of 16 to 512 rows and 1,408 to 10,368 outputs): 64 rows x 2048 outputs 32x16 (20 us at K
 // = 8192; 32x32 23), 3072 32x32 (8.2 us at K = 2048; 32x16 10.1), 10368 64x64; 512 rows x 2048 64x64 (13.3 us, the
-// 256-row prefill tiles 19.8), 3072 64x128 (18.3 / 22.0). Where not even 64x128 does (1): up to 64 rows tiles of 64 columns
-// with the waves' loads side by side, which stream the weights at 5 TB/s (64 rows x 128256 x 2048: 105 us); above, the
+// 256-row prefill tiles 19.8), 3072 64x128 (18.3 / 22.0). Where not even 64x128 does (1), up to 64 rows: what every workgroup
+// takes in of x counts against small tiles, a last round that few CUs take part in against large ones. 128 columns (64 rows of 33024
+// x 2048 35.0 us, 64 columns 36.2; 65536 48.8, 52.2; 152064 113, 123; 128256 92, 102), or 256, two a CU, where they fill 7 of 8
+// places at least (128256 x 2048 88.9 us, 5.9 TB/s; x 4096 173, 128 columns 190; 152064 x 2048 123, 98304 71.8). Above, the
 // prefill kernels (512 rows x 10368: 30 us against 52).
 static int dispatch_rows(const DgArgs& a, hipStream_t st) {
   if (a.M <= 0) return 0;
@@ -511,7 +513,8 @@ static int dispatch_rows(const DgArgs& a, hipStream_t st) {
   if (fits(64, 64)) return launch_rows<4, 4, 8>(a, st);
   if (fits(64, 128)) return launch_rows<4, 4, 4>(a, st);
   if (a.M <= 32) return launch_rows<2, 2, 4>(a, st);
-  if (a.M <= 64) return launch_rows<4, 2, 4>(a, st);
+  const int wide = (a.N + 255) / 256;
+  if (a.M <= 64) return wide >= 448 && wide <= 512 ? launch_rows<4, 2, 1>(a, st) : launch_rows<4, 2, 2>(a, st);
   return 1;
 }
 
