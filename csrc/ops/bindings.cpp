@@ -9,7 +9,9 @@
 #include <cstring>
 
 extern "C" {
-int pa_rmsnorm(void* out, const void* x, const void* w, int T, int D, float eps, hipStream_t st);
+int pa_rmsnorm(void* out, const void* x, const void* w, const int* rows, int nx, int T, int D, float eps, hipStream_t st);
+int pa_embed_rows(void* out, const void* emb, const int* ids, float* ss, float* ss_zero, int T, int V, int D, long long lde,
+                  hipStream_t st);
 int pa_fused_add_rmsnorm(void* out, void* resid, const void* x, const void* w, int T, int D,
                          float eps, hipStream_t st);
 int pa_rope_cache(void* q_out, void* k_cache, void* v_cache, const void* qkv, const int* positions,
@@ -94,15 +96,41 @@ int pa_car_all_reduce(void* const* bases, int W, int rank0, int nranks_local, co
 
 namespace {
 
-void rmsnorm(at::Tensor out, at::Tensor x, at::Tensor w, double eps) {
+// out = rmsnorm of x, or of x's rows rows[i] (int32; x 2-D then)
+void rmsnorm(at::Tensor out, at::Tensor x, at::Tensor w, double eps, c10::optional<at::Tensor> rows) {
   check_gpu(out, "out"); check_gpu(x, "x"); check_gpu(w, "w");
   check_dtype(x, at::kBFloat16, "x"); check_dtype(out, at::kBFloat16, "out");
   check_dtype(w, at::kBFloat16, "w");
   const int D = x.size(-1);
-  const int T = x.numel() / D;
-  TORCH_CHECK(w.numel() == D && out.numel() == x.numel(), "rmsnorm shape mismatch");
-  check_rc(pa_rmsnorm(out.data_ptr(), x.data_ptr(), w.data_ptr(), T, D, (float)eps, cur_stream()),
+  int T = x.numel() / D;
+  const int nx = T;
+  if (rows) {
+    check_gpu(*rows, "rows"); check_dtype(*rows, at::kInt, "rows");
+    T = rows->numel();
+    TORCH_CHECK(x.dim() == 2 && (T == 0 || nx > 0), "rows need a 2-D x that has any");
+  }
+  TORCH_CHECK(w.numel() == D && out.numel() == (int64_t)T * D, "rmsnorm shape mismatch");
+  check_rc(pa_rmsnorm(out.data_ptr(), x.data_ptr(), w.data_ptr(), rows ? rows->data_ptr<int>() : nullptr, nx, T, D, (float)eps,
+                      cur_stream()),
            "rmsnorm");
+}
+
+// out row t = emb's row ids[t]; ss[t] its sum of squares, ss_zero[t] = 0 (both optional)
+void embed_rows(at::Tensor out, at::Tensor emb, at::Tensor ids, c10::optional<at::Tensor> ss, c10::optional<at::Tensor> ss_zero) {
+  check_gpu(out, "out"); check_gpu(ids, "ids");
+  TORCH_CHECK(emb.is_cuda() && emb.dim() == 2 && emb.stride(1) == 1, "emb must be a 2-D GPU tensor, unit inner stride");
+  check_dtype(emb, at::kBFloat16, "emb"); check_dtype(out, at::kBFloat16, "out"); check_dtype(ids, at::kInt, "ids");
+  const int T = ids.numel(), D = emb.size(1);
+  TORCH_CHECK(out.numel() == (int64_t)T * D, "embed_rows shape mismatch");
+  TORCH_CHECK(((uintptr_t)emb.data_ptr() | (uintptr_t)out.data_ptr()) % 16 == 0, "emb and out must be aligned to 16 bytes");
+  for (auto* s : {&ss, &ss_zero})
+    if (*s) {
+      check_gpu(**s, "ss"); check_dtype(**s, at::kFloat, "ss");
+      TORCH_CHECK((*s)->numel() >= T, "ss shorter than ids");
+    }
+  check_rc(pa_embed_rows(out.data_ptr(), emb.data_ptr(), ids.data_ptr<int>(), ss ? ss->data_ptr<float>() : nullptr,
+                         ss_zero ? ss_zero->data_ptr<float>() : nullptr, T, emb.size(0), D, emb.stride(0), cur_stream()),
+           "embed_rows");
 }
 
 void fused_add_rmsnorm(at::Tensor out, at::Tensor resid, at::Tensor x, at::Tensor w, double eps) {
@@ -893,7 +921,9 @@ PYBIND11_MODULE(_C, m) {
   m.def("empty_uncached", &empty_uncached, py::arg("numel"), py::arg("dtype"), py::arg("device"),
         "zero-filled device tensor in uncached memory (hipDeviceMallocUncached)");
   m.doc() = "pilottai_amd CDNA4 (gfx950) HIP kernels";
-  m.def("rmsnorm", &rmsnorm);
+  m.def("rmsnorm", &rmsnorm, py::arg("out"), py::arg("x"), py::arg("w"), py::arg("eps"), py::arg("rows") = py::none());
+  m.def("embed_rows", &embed_rows, py::arg("out"), py::arg("emb"), py::arg("ids"), py::arg("ss") = py::none(),
+        py::arg("ss_zero") = py::none());
   m.def("fused_add_rmsnorm", &fused_add_rmsnorm);
   m.def("rope_cache", &rope_cache);
   m.def("silu_mul", &silu_mul);

@@ -461,6 +461,18 @@ class LlamaModel:
         self.tp.all_reduce(h)
         return h
 
+    def _first_rows(self, ids: torch.Tensor, ss=None, ss_zero=None) -> torch.Tensor:
+        """The residual stream's first rows, with their statistics in ss and ss_zero cleared for
+        the first residual epilogue: one launch; under TP rows of other ranks' shards arrive by
+        an all-reduce, behind which the statistics are taken."""
+        if self.tp.size == 1:
+            return ops.embed_rows(self.embed, ids, ss, ss_zero)
+        h = self._embed(ids.long() if self.device.type == "cpu" else ids).contiguous()
+        if ss is not None:
+            ops.row_sumsq(h, out=ss)
+            ss_zero.zero_()
+        return h
+
     def forward(self, meta: StepMeta, kv: KVCache, num_tokens: int, num_logit_rows: int,
                 part_o: torch.Tensor, part_ml: torch.Tensor, embed=None) -> torch.Tensor:
         """Returns local-vocab logits [num_logit_rows, V/tp] (bf16).
@@ -517,10 +529,7 @@ class LlamaModel:
         H, KVh, hd = self.h_local, self.kv_local, cfg.head_dim
         eps = cfg.rms_eps
         tp = self.tp.size > 1
-        ids = meta.input_ids[:T].long() if self.device.type == "cpu" else meta.input_ids[:T]
-        h = self._embed(ids)
-        if not h.is_contiguous():
-            h = h.contiguous()
+        h = self._first_rows(meta.input_ids[:T])
         for li, L in enumerate(self.layers):
             q = torch.empty(T, H, hd, dtype=self.dtype, device=self.device)
             ops.decode_qkv_rope(h, L["wqkv_p"], eps, q, kv.k[li], kv.v[li], meta.positions, meta.slots,
@@ -543,8 +552,7 @@ class LlamaModel:
         if embed is not None:
             self._pool_embed(ops.rmsnorm(h, self.norm, eps), T, embed)
         rows = meta.logit_rows[:num_logit_rows]
-        rows = rows.long() if self.device.type == "cpu" else rows
-        xs = ops.rmsnorm(h.index_select(0, rows), self.norm, eps)
+        xs = ops.rmsnorm(h, self.norm, eps, rows=rows)
         return ops.decode_gemm(xs, self.lm_head_p, "plain")
 
     @staticmethod
@@ -671,13 +679,8 @@ class LlamaModel:
         H, KVh, hd = self.h_local, self.kv_local, cfg.head_dim
         eps = cfg.rms_eps
         tp = self.tp.size > 1
-        ids = meta.input_ids[:T].long() if self.device.type == "cpu" else meta.input_ids[:T]
-        h = self._embed(ids)
-        if not h.is_contiguous():
-            h = h.contiguous()
         ss_a, ss_b = self._ss[0, :T], self._ss[1, :T]
-        ops.row_sumsq(h, out=ss_a)
-        ss_b.zero_()
+        h = self._first_rows(meta.input_ids[:T], ss_a, ss_b)
         for li, L in enumerate(self.layers):
             q = torch.empty(T, H, hd, dtype=self.dtype, device=self.device)
             self._qkv_rope(T, h, L["wqkv_p"], eps, q, kv.k[li], kv.v[li], meta, ss_a)
@@ -700,8 +703,7 @@ class LlamaModel:
         if embed is not None:
             self._pool_embed(ops.rmsnorm(h, self.norm, eps), T, embed)
         rows = meta.logit_rows[:num_logit_rows]
-        rows = rows.long() if self.device.type == "cpu" else rows
-        xs = ops.rmsnorm(h.index_select(0, rows), self.norm, eps)
+        xs = ops.rmsnorm(h, self.norm, eps, rows=rows)
         return self._lm_head(xs, num_logit_rows)
 
     def _lm_head(self, xs, n: int):

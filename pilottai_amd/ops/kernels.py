@@ -126,16 +126,37 @@ def empty_handoff(numel: int, dtype=torch.float32, device=None) -> torch.Tensor:
     return torch.zeros(int(numel), dtype=dtype, device=device)
 
 
-def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, out: Optional[torch.Tensor] = None):
+def rmsnorm(x: torch.Tensor, w: torch.Tensor, eps: float, out: Optional[torch.Tensor] = None,
+            rows: Optional[torch.Tensor] = None):
+    """The norm of x's rows, or of its rows `rows` in their order."""
     if _on_gpu(x):
-        out = torch.empty_like(x) if out is None else out
-        require_native().rmsnorm(out, x, w, float(eps))
+        if rows is not None:
+            rows = rows.int()
+        if out is None:
+            out = torch.empty_like(x) if rows is None else x.new_empty(rows.numel(), x.shape[-1])
+        require_native().rmsnorm(out, x, w, float(eps), rows)
         return out
-    r = ref.rmsnorm(x, w, eps)
+    r = ref.rmsnorm(x if rows is None else x.index_select(0, rows.long()), w, eps)
     if out is not None:
         out.copy_(r)
         return out
     return r
+
+
+def embed_rows(emb: torch.Tensor, ids: torch.Tensor, ss: Optional[torch.Tensor] = None,
+               ss_zero: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """emb's rows `ids`; ss[t] <- row t's sum of squares, ss_zero[t] <- 0 (fp32, both optional)."""
+    if _on_gpu(emb):
+        ids = ids.int()
+        out = emb.new_empty(ids.numel(), emb.shape[1])
+        require_native().embed_rows(out, emb, ids, ss, ss_zero)
+        return out
+    h = torch.nn.functional.embedding(ids.long(), emb)
+    if ss is not None:
+        row_sumsq(h, out=ss)
+    if ss_zero is not None:
+        ss_zero[:h.shape[0]].zero_()
+    return h
 
 
 def fused_add_rmsnorm(resid: torch.Tensor, x: torch.Tensor, w: torch.Tensor, eps: float,

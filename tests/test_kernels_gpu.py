@@ -25,6 +25,23 @@ def test_rmsnorm(gpu, D):
     torch.testing.assert_close(y.cpu().float(), r.float(), atol=2e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("T,D", [(1, 4096), (5, 520), (64, 64), (67, 8192), (130, 4104)])
+def test_first_and_last_rows(gpu, T, D):
+    """Gathers inside the step's first launch and its last norm: the bits of the launches that they stand for."""
+    gen = torch.Generator().manual_seed(T)
+    emb = torch.randn(301, D + 8, generator=gen).to(torch.bfloat16).to(gpu)[:, :D]  # (rows that lie apart)
+    ids = torch.randint(0, 301, (T,), generator=gen, dtype=torch.int32)
+    ids[0], ids[-1] = 0, 300
+    ss, zero = torch.full((2, T + 1), 7.0, device=gpu)
+    h = ops.embed_rows(emb, ids.to(gpu), ss[:T], zero[:T])
+    assert torch.equal(h.cpu(), emb.cpu()[ids.long()])
+    assert torch.equal(ss[:T], ops.row_sumsq(h)) and not zero[:T].any() and ss[T] == zero[T] == 7
+    assert torch.equal(ops.embed_rows(emb, ids.to(gpu)), h)
+    w = torch.randn(D, generator=gen).to(torch.bfloat16).to(gpu)
+    rows = torch.randint(0, T, (T + 3,), generator=gen, dtype=torch.int32).to(gpu)
+    assert torch.equal(ops.rmsnorm(h, w, 1e-5, rows=rows), ops.rmsnorm(h.index_select(0, rows), w, 1e-5))
+
+
 @pytest.mark.parametrize("D", [4096, 8192, 520])
 def test_fused_add_rmsnorm(gpu, D):
     torch.manual_seed(1)
