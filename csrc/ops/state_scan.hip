@@ -44,13 +44,18 @@ struct Args {
   const int *q_start, *q_len, *ctx_len, *state_slot;
   const int4* items;
   const int* n_items;
-  int ldp, ldy, H, G, V, N, Cc, taps, RING, scan_min, long_too, vsplit;
+  int ldp, ldy, H, G, V, N, Cc, taps, RING, scan_min, long_too;
+  int vsplit;     // workgroups of step_kernel a head: 1, 2, 4 or 8
+  int per_group;  // heads
   float* work;   // [items, H, V, N]: every chunk's state
   float* total;  // [items, H]: a chunk's summed log2 decay
   int* form;     // null, or 1 where the step's long portions go through the three launches, else 0 (pick_form)
   float chain, fixed;
 };
 
+// (a base that is the same for a wave and an offset of 32 bits: one register a load in flight instead of two)
+template <typename T>
+__device__ __forceinline__ T& at_byte(const void* p, uint32_t off) { return *(T*)((char*)p + off); }
 template <typename T>
 __device__ __forceinline__ float ld(const void* p, size_t i) { return (float)((const T*)p)[i]; }
 __device__ __forceinline__ float silu(float x) { return x / (1.f + __expf(-x)); }
@@ -156,65 +161,114 @@ constexpr int REGS = 8;  // state vectors of a thread that stay in registers ove
 template <typename T, int TAPS, int TN>
 __global__ __launch_bounds__(256, 4) void step_kernel(const Args A) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
-  const int h = blockIdx.x / A.vsplit, vpart = blockIdx.x % A.vsplit, s = blockIdx.y;
-  const int n = A.q_len[s];
-  if (n <= 0 || A.state_slot[s] < 0) return;
+  const int vlog = __builtin_ctz(A.vsplit), h = blockIdx.x >> vlog, vpart = blockIdx.x & (A.vsplit - 1), s = blockIdx.y;
+  const int n = A.q_len[s], slot = A.state_slot[s], q0 = A.q_start[s], p0 = A.ctx_len[s] - n;
+  if (n <= 0 || slot < 0) return;
   const bool conv = n <= A.scan_min;  // short: the convolution is done here
   if (!conv && !A.long_too) return;
-  const int V = A.V, N = TN ? 4 * TN : A.N, g = h / (A.H / A.G), inner = A.H * V;
+  const int V = A.V, N = TN ? 4 * TN : A.N, g = (uint32_t)h / (uint32_t)A.per_group, inner = A.H * V;
   float *sB = sm, *sC = sm + N, *sx = sm + 2 * N, *sdt = sm + 2 * N + V;  // one token
-  const int q0 = A.q_start[s], p0 = A.ctx_len[s] - n;
-  float* S = A.state + ((size_t)A.state_slot[s] * A.H + h) * V * N;
-  T* ring = (T*)A.ring + (size_t)A.state_slot[s] * A.RING * A.Cc;
+  float* S = A.state + ((size_t)slot * A.H + h) * V * N;
+  T* ring = (T*)A.ring + (size_t)slot * A.RING * A.Cc;
   const float* W = (const float*)A.conv_w;
   // lanes along N, 4 values each (a power of two of them, whole groups inside a wave), the rest along V
   int tn = TN ? TN : 1;
   if constexpr (TN == 0)
     while (tn < 64 && (N >> 2) % (2 * tn) == 0) tn *= 2;
   const int ln = threadIdx.x % tn, lv = threadIdx.x / tn, nv = 256 / tn;
-  const int v0 = vpart * (V / A.vsplit), v1 = v0 + V / A.vsplit;
+  const int v0 = vpart * (V >> vlog), v1 = v0 + (V >> vlog);
   const float a = A.a[h], dd = A.d[h], bias = A.dt_bias[h];
   // The state in registers over the portion: a lane's vectors are of rows v0 + lv + k nv. Read and written once a step, past
-  // the caches' usual place, which is left to the weights and keys (64 rows, 64 heads of 64 x 128: 69 -> 65 us, and 10 us
-  // more of the step's other kernels a layer; 8 rows: no slower).
+  // the caches' usual place, which is left to the weights and keys. Bound by these bytes: 64 rows, 64 heads of 64 x 128 take
+  // 48 us, 5.5 TB/s, where nothing but the update of the same bytes takes 43 (4 workgroups a CU or 5: the same).
   f32x4 st[TN ? REGS : 1];
-  float* mine = S + (size_t)(v0 + lv) * N + 4 * ln;
-  if constexpr (TN > 0) {
+  // The first token's inputs of a short portion are asked for ahead of the state: its wait then leaves the state's loads in
+  // flight, and a thread's second channel waits with the first (64 -> 51 us). That token is apart from the others' loop,
+  // whose addresses would take its registers.
+  constexpr int EC = TN ? (8 * TN + REGS * 256 / TN + 255) / 256 : 1;  // channels of a thread
+  const int n_ch = 2 * N + v1 - v0;
+  auto channel = [&](int e) {
+    return e < N ? inner + g * N + e : e < 2 * N ? inner + A.G * N + g * N + e - N : h * V + v0 + e - 2 * N;
+  };
+  float x0[EC][TAPS], w0[EC][TAPS], b0[EC], dt0 = 0.f;
+  const bool ahead = TN > 0 && conv;
+  if (ahead) {
+    const T* row = (const T*)A.proj + (size_t)q0 * A.ldp + inner;
+    const int at = (uint32_t)p0 % (uint32_t)A.RING;
 #pragma unroll
-    for (int k = 0; k < REGS; ++k) {
-      st[k] = f32x4{0.f, 0.f, 0.f, 0.f};
-      if (p0 > 0 && v0 + lv + k * nv < v1) st[k] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(mine + (size_t)k * nv * N));
+    for (int j = 0; j < EC; ++j) {
+      const int c = channel(min((int)threadIdx.x + j * 256, n_ch - 1));
+#pragma unroll
+      for (int k = 0; k < TAPS; ++k) {
+        const int i = k - (TAPS - 1);  // positions before the first hold no input: row 0 is read for them and not used
+        const int r = p0 + i < 0 ? 0 : at + i + (at + i < 0 ? A.RING : 0);
+        x0[j][k] = (float)at_byte<T>(k == TAPS - 1 ? row : ring + (size_t)r * A.Cc, c * sizeof(T));
+        w0[j][k] = at_byte<float>(W + (size_t)k * A.Cc, c * 4);
+      }
+      b0[j] = at_byte<float>(A.conv_b, c * 4);
+    }
+    dt0 = (float)row[A.Cc + h];
+  }
+  if constexpr (TN > 0) {
+    // (rows beyond the part's last: its last again)
+#pragma unroll
+    for (int k = 0; k < REGS; ++k) st[k] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (p0 > 0) {
+#pragma unroll
+      for (int k = 0; k < REGS; ++k)
+        if (k * nv < v1 - v0)
+          st[k] = __builtin_nontemporal_load(&at_byte<f32x4>(S, 4u * (min(v0 + lv + k * nv, v1 - 1) * N + 4 * ln)));
     }
   }
-  for (int t = 0; t < n; ++t) {
+  auto token = [&](int t, auto first) {
     const T* row = (const T*)A.proj + (size_t)(q0 + t) * A.ldp;
     __syncthreads();
-    for (int e = threadIdx.x; e < 2 * N + v1 - v0; e += 256) {
-      const int c = e < N ? inner + g * N + e : e < 2 * N ? inner + A.G * N + g * N + e - N : h * V + v0 + e - 2 * N;
-      float v;
-      if (conv) {
-        v = A.conv_b[c];
-        float x[TAPS];
-#pragma unroll
-        for (int k = 0; k < TAPS; ++k) {
-          const int i = t - (TAPS - 1) + k;
-          x[k] = 0.f;
-          if (i >= 0) x[k] = (float)((const T*)A.proj)[(size_t)(q0 + i) * A.ldp + inner + c];
-          else if (p0 + i >= 0) x[k] = (float)ring[(size_t)((p0 + i) % A.RING) * A.Cc + c];
-        }
-#pragma unroll
-        for (int k = 0; k < TAPS; ++k) v = fmaf(W[(size_t)k * A.Cc + c], x[k], v);
-        v = (float)(T)silu(v);
-        // the owner of a channel keeps its input (rows that no token of this portion reads)
-        if (e >= 2 * N || (h % (A.H / A.G) == 0 && vpart == 0)) ring[(size_t)((p0 + t) % A.RING) * A.Cc + c] = row[inner + c];
-      } else {
-        v = (float)((const T*)A.u)[(size_t)(q0 + t) * A.Cc + c];
-      }
+    auto put = [&](int e, float v) {
       if (e < 2 * N) sm[e] = v;
       else sx[v0 + e - 2 * N] = v;
+    };
+    // the owner of a channel keeps its input (rows that no token of this portion reads)
+    auto keep = [&](int e, int c) {
+      if (e >= 2 * N || (h == g * A.per_group && vpart == 0)) ring[(size_t)((uint32_t)(p0 + t) % (uint32_t)A.RING) * A.Cc + c] = row[inner + c];
+    };
+    if constexpr (first) {
+#pragma unroll
+      for (int j = 0; j < EC; ++j) {
+        const int e = threadIdx.x + j * 256;
+        float v = b0[j];
+#pragma unroll
+        for (int k = 0; k < TAPS; ++k) v = fmaf(w0[j][k], p0 + k < TAPS - 1 ? 0.f : x0[j][k], v);
+        if (e < n_ch) {
+          put(e, (float)(T)silu(v));
+          keep(e, channel(e));
+        }
+      }
+    } else {
+      for (int e = threadIdx.x; e < n_ch; e += 256) {
+        const int c = channel(e);
+        float v;
+        if (conv) {
+          v = A.conv_b[c];
+          float x[TAPS];
+#pragma unroll
+          for (int k = 0; k < TAPS; ++k) {
+            const int i = t - (TAPS - 1) + k;
+            x[k] = 0.f;
+            if (i >= 0) x[k] = (float)((const T*)A.proj)[(size_t)(q0 + i) * A.ldp + inner + c];
+            else if (p0 + i >= 0) x[k] = (float)ring[(size_t)((p0 + i) % A.RING) * A.Cc + c];
+          }
+#pragma unroll
+          for (int k = 0; k < TAPS; ++k) v = fmaf(W[(size_t)k * A.Cc + c], x[k], v);
+          v = (float)(T)silu(v);
+          keep(e, c);
+        } else {
+          v = (float)((const T*)A.u)[(size_t)(q0 + t) * A.Cc + c];
+        }
+        put(e, v);
+      }
     }
     if (threadIdx.x == 255) {  // (a thread of the last wave, which has the fewest channels)
-      const float dt = softplus((float)row[inner + A.Cc + h] + bias);
+      const float dt = softplus((first ? dt0 : (float)row[inner + A.Cc + h]) + bias);
       sdt[0] = dt;
       sdt[1] = expf(-a * dt);
     }
@@ -231,21 +285,28 @@ __global__ __launch_bounds__(256, 4) void step_kernel(const Args A) {
       }
       return acc;
     };
-    auto finish = [&](float acc, int v, float x) {
-#pragma unroll
-      for (int o = 32; o > 0; o >>= 1)
-        if (tn > o) acc += __shfl_xor(acc, o, 64);
-      if (ln == 0) ((T*)A.y)[(size_t)(q0 + t) * A.ldy + h * V + v] = (T)(acc + dd * x);
-    };
     if constexpr (TN > 0) {
+      // Rows beyond the part's last are steps of no use, so that nothing branches. The sums over a row's lanes halve the rows
+      // that a lane holds in their first three rounds: the same sums in the same order, with 9 shuffles for 40 where 32 lanes
+      // share a row (51 -> 48 us).
+      float acc[REGS];
 #pragma unroll
-      for (int k = 0; k < REGS; ++k) {
-        const int v = v0 + lv + k * nv;
-        if (v < v1) {
-          const float x = sx[v];
-          finish(step(st[k], 4 * ln, dt * x), v, x);
+      for (int k = 0; k < REGS; ++k) acc[k] = step(st[k], 4 * ln, dt * sx[min(v0 + lv + k * nv, v1 - 1)]);
+      int k = 0;
+#pragma unroll
+      for (int left = REGS / 2, o = TN / 2; left > 0; left /= 2, o /= 2) {
+        const bool upper = ln & o;
+#pragma unroll
+        for (int i = 0; i < left; ++i) {
+          const float other = __shfl_xor(upper ? acc[i] : acc[i + left], o, 64);
+          acc[i] = (upper ? acc[i + left] : acc[i]) + other;
         }
+        k += upper ? left : 0;
       }
+#pragma unroll
+      for (int o = TN / 16; o > 0; o /= 2) acc[0] += __shfl_xor(acc[0], o, 64);
+      const int v = v0 + lv + k * nv;
+      if (ln % (TN / 8) == 0 && v < v1) ((T*)A.y)[(size_t)(q0 + t) * A.ldy + h * V + v] = (T)(acc[0] + dd * sx[v]);
     } else {
       const bool fresh = p0 + t == 0;
       for (int v = v0 + lv; v < v1; v += nv) {
@@ -257,14 +318,20 @@ __global__ __launch_bounds__(256, 4) void step_kernel(const Args A) {
           acc += step(w, i, dt * x);
           *p = w;
         }
-        finish(acc, v, x);
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1)
+          if (tn > o) acc += __shfl_xor(acc, o, 64);
+        if (ln == 0) ((T*)A.y)[(size_t)(q0 + t) * A.ldy + h * V + v] = (T)(acc + dd * x);
       }
     }
-  }
+  };
+  int t = 0;
+  if (ahead) token(t++, std::true_type{});
+  for (; t < n; ++t) token(t, std::false_type{});
   if constexpr (TN > 0) {
 #pragma unroll
     for (int k = 0; k < REGS; ++k)
-      if (v0 + lv + k * nv < v1) __builtin_nontemporal_store(st[k], reinterpret_cast<f32x4*>(mine + (size_t)k * nv * N));
+      if (v0 + lv + k * nv < v1) __builtin_nontemporal_store(st[k], &at_byte<f32x4>(S, 4u * ((v0 + lv + k * nv) * N + 4 * ln)));
   }
   if (!conv && vpart == 0) {
     const int per = (A.Cc + A.H - 1) / A.H;
@@ -843,7 +910,7 @@ extern "C" int pa_state_scan(int fp32, const void* proj, int ldp, void* u, void*
   if (seqs <= 0) return 0;
   if (V % 16 || N % 32 || H % G || scan_min > MAX_SHORT || ring_rows < taps - 1 + scan_min || (taps != 4 && taps != 8)) return -1;  // (shorter ones are padded)
   Args A{proj, u, y, state, ring, conv_w, conv_b, dt_bias, a, d, q_start, q_len, ctx_len, state_slot,
-         (const int4*)items, n_items, ldp, ldy, H, G, V, N, H * V + 2 * G * N, taps, ring_rows, scan_min, fp32, 1,
+         (const int4*)items, n_items, ldp, ldy, H, G, V, N, H * V + 2 * G * N, taps, ring_rows, scan_min, fp32, 1, H / G,
          work, total, nullptr, chain, fixed};
   if (A.Cc % 8 || ldp % 8) return -1;
   // the three launches: (bf16) states that scan_kernel is not built for, or a choice

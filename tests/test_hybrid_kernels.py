@@ -546,6 +546,36 @@ def test_state_scan_form_in_a_graph(gpu):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("V,N,taps", [(64, 128, 4), (48, 128, 8), (32, 256, 4), (128, 64, 4), (256, 32, 8), (16, 256, 4)])
+def test_state_scan_many_sequences(gpu, V, N, taps):
+    """A head in one workgroup, whole and with rows left over, where few sequences spread it over eight: the same bits. Portions
+    of one token and of several, from the first positions (fewer inputs than taps) and later ones."""
+    from pilottai_amd import ops
+
+    H, G, S, g = 8, 2, 66, gen(V + N)
+    C = H * V + 2 * G * N
+    cols, rows = (H * V + C + H + 7) // 8 * 8, taps - 1 + ops.SCAN_MIN
+    f = lambda *sh, by=1.0: (torch.randn(*sh, generator=g) * by).to(gpu)  # noqa: E731
+    iv = lambda v: torch.tensor(list(v), dtype=torch.int32, device=gpu)  # noqa: E731
+    lens, past = [1 + (i % 3) * (i % 2) for i in range(S)], [(0, 1, 2, 3, 6, 40, 1001)[i % 7] for i in range(S)]
+    starts = np.cumsum([0] + lens)
+    proj = f(int(starts[-1]), cols).to(BF16)
+    w, cb, bias, a, d = f(taps, C, by=0.5), f(C, by=0.2), f(H) - 2, torch.linspace(0.02, 3.0, H).to(gpu), f(H)
+    state0, ring0 = f(S, H, V, N), f(S, rows, C).to(BF16)
+
+    def run(groups):
+        state, ring = state0.clone(), ring0.clone()
+        y = torch.zeros(len(proj), (H * V + 63) // 64 * 64, dtype=BF16, device=gpu)
+        for i in groups:
+            ops.state_scan(proj, y, state, ring, w, cb, bias, a, d, iv(starts[i]), iv(lens[j] for j in i),
+                           iv(past[j] + lens[j] for j in i), iv(i), iv([-1] * len(i)),
+                           torch.zeros(1, 4, dtype=torch.int32, device=gpu), iv([0]), G)
+        return y, state, ring
+    for one, few in zip(run([list(range(S))]), run([list(range(i, i + 3)) for i in range(0, S, 3)])):
+        assert torch.equal(one, few)
+
+
+@pytest.mark.gpu
 def test_state_scan_keeps_the_state_in_fp32(gpu):
     """The state a chunked portion leaves equals the one that single tokens leave to fp32's order, not bf16's."""
     from pilottai_amd import ops
