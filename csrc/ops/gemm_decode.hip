@@ -365,7 +365,7 @@ static int pick_nw(int nt, int waves, const DgArgs& a, hipStream_t st) {
 // drains the other, and the stage barrier waits for LDS alone. What bounds it then is the L2s' rate on x, which every
 // column group reads whole: hence the largest tile that still gives every CU one (dispatch_rows).
 // us at 64 rows, before -> after (x from L2, cold weights): N x K 2048 x 8192 37 -> 20, 2048 x 4096 20 -> 11.4, 2048 x 2048
-// 11.7 -> 7.3, 10368 x 2048 17.8 -> 15.8, 128256 x 2048 144 -> 105.
+// 11.7 -> 7.3, 10368 x 2048 17.8 -> 15.8, 128256 x 2048 144 -> 89.
 // SUMS: a workgroup takes one of A.S slices of k and leaves its fp32 sums, row m's of slice s at y [M, A.S, N] (pa_rows_sums).
 template <int MT, int NT, int WK, int D, bool SUMS = false>
 __global__ __launch_bounds__(512) void decode_rows_kernel(const DgArgs A) {

@@ -21,7 +21,6 @@ constexpr int MAX_S = 8;
 struct Args {
   float* x;             // [T, S, D]
   const void* y;        // [T, K, ldy]
-  const float* sums;    // [T, K, ldy] in place of y, or null
   const float* y_w;     // [T, K] or null
   const void* y2;       // [T, ldy2] or null
   const float* bias;    // [D] or null
@@ -34,10 +33,12 @@ struct Args {
   const int* live;      // by row: below 0 from the first row without a token on (with rows: not looked at)
   int K, ldy, ldy2, vocab, ldo, D;
   float eps;
+  const float* sums;    // [T, K, ldy] in place of y, or null
 };
 
-// LIVE: with `live` (bf16 rows of whole 4s, the others do all rows)
-template <typename T, int VEC, int S, int NW, bool LIVE = false>
+// LIVE: with `live` (bf16 rows of whole 4s, the others do all rows). SUMS: y may be sums; launches without are apart (304 rows, 4
+// streams of 2,048: 8.8 us with the test, 8.6 without; and 9.1 where `sums` lay among the other arguments, not behind them).
+template <typename T, int VEC, int S, int NW, bool LIVE = false, bool SUMS = true>
 __global__ __launch_bounds__(64 * NW) void hyper_norm_kernel(const Args A) {
   constexpr int NT = 64 * NW;
   extern __shared__ __attribute__((aligned(16))) float row[];
@@ -45,15 +46,15 @@ __global__ __launch_bounds__(64 * NW) void hyper_norm_kernel(const Args A) {
   if (LIVE && A.live[blockIdx.x] < 0) return;
   const int t = A.rows ? A.rows[blockIdx.x] : blockIdx.x, D = A.D;
   float* xr = A.x + (size_t)t * S * D;
+  const bool add = A.y || (SUMS && A.sums);
   float mix[S][S], post[S], pre[S];
 #pragma unroll
   for (int s = 0; s < S; ++s) {
     pre[s] = A.pre ? A.pre[s] : 0.f;
-    post[s] = A.y || A.sums ? A.post[s] : 0.f;
+    post[s] = add ? A.post[s] : 0.f;
 #pragma unroll
-    for (int r = 0; r < S; ++r) mix[s][r] = A.y || A.sums ? A.mix[s * S + r] : 0.f;
+    for (int r = 0; r < S; ++r) mix[s][r] = add ? A.mix[s * S + r] : 0.f;
   }
-  const bool add = A.y || A.sums;
   const T* yr = (const T*)A.y + (size_t)t * A.K * A.ldy;
   const float* sr = A.sums + (size_t)t * A.K * A.ldy;
   const float* yw = A.y_w ? A.y_w + (size_t)t * A.K : nullptr;
@@ -84,7 +85,7 @@ __global__ __launch_bounds__(64 * NW) void hyper_norm_kernel(const Args A) {
 #pragma unroll
         for (int j = 0; j < VEC; ++j) y[j] += (float)a[j];
       }
-      if (A.sums) {
+      if (SUMS && A.sums) {
 #pragma unroll 8
         for (int k = 0; k < A.K; ++k) {
           float f[VEC];
@@ -94,7 +95,7 @@ __global__ __launch_bounds__(64 * NW) void hyper_norm_kernel(const Args A) {
         }
       }
 #pragma unroll 4
-      for (int k = 0; A.y && k < A.K; ++k) {
+      for (int k = 0; (!SUMS || A.y) && k < A.K; ++k) {
         __builtin_memcpy(a, __builtin_assume_aligned(yr + (size_t)k * A.ldy + i, sizeof(T) * VEC), sizeof(T) * VEC);
         const float w = yw ? yw[k] : 1.f;
 #pragma unroll
@@ -166,7 +167,7 @@ extern "C" int pa_hyper_norm(int fp32, float* x, int S, const void* y, const flo
   // Rows without a token stay as they are in launches that look for them (a step of mudepel's 8 layers, 4 streams of 2,048
   // columns: 3,658 tokens in 4,096 rows 2 % of its 5,840 us, 2,101 in 3,072 3 % of 4,640)
   if (rows || n <= pa::LIVE_MIN_ROWS) live = nullptr;
-  const Args A{x, y, sums, y_w, y2, bias, mix, post, pre, emb, ids, w_next, out, rows, live, K, ldy, ldy2, vocab, ldo, D, eps};
+  const Args A{x, y, y_w, y2, bias, mix, post, pre, emb, ids, w_next, out, rows, live, K, ldy, ldy2, vocab, ldo, D, eps, sums};
   // fewer rows than CUs: twice the waves to a row, all of it in one pass up to 2,048 columns (64 rows, 4 streams of 2,048:
   // 6.8 -> 5.7 us)
   const bool few = n <= 256 && D > 1024;
@@ -186,9 +187,12 @@ extern "C" int pa_hyper_norm(int fp32, float* x, int S, const void* y, const flo
   case N:                                                                      \
     if (fp32) { if (vec) PA_HN(float, 4, N, 4); else PA_HN(float, 1, N, 4); }  \
     else if (!vec) PA_HN(pa::bf16, 1, N, 4);                                   \
-    else if (few) PA_HN(pa::bf16, 4, N, 8);                                    \
-    else if (live) PA_HN(pa::bf16, 4, N, 4, true);                             \
-    else PA_HN(pa::bf16, 4, N, 4);                                             \
+    else if (few && sums) PA_HN(pa::bf16, 4, N, 8);                            \
+    else if (few) PA_HN(pa::bf16, 4, N, 8, false, false);                      \
+    else if (live && sums) PA_HN(pa::bf16, 4, N, 4, true);                     \
+    else if (live) PA_HN(pa::bf16, 4, N, 4, true, false);                      \
+    else if (sums) PA_HN(pa::bf16, 4, N, 4);                                   \
+    else PA_HN(pa::bf16, 4, N, 4, false, false);                               \
     break
   switch (S) {
     PA_HN_S(1); PA_HN_S(2); PA_HN_S(3); PA_HN_S(4); PA_HN_S(5); PA_HN_S(6); PA_HN_S(7); PA_HN_S(8);

@@ -45,12 +45,12 @@ struct Args {
   const int4* items;
   const int* n_items;
   int ldp, ldy, H, G, V, N, Cc, taps, RING, scan_min, long_too;
-  int vsplit;     // workgroups of step_kernel a head: 1, 2, 4 or 8
-  int per_group;  // heads
+  int vsplit;    // workgroups of step_kernel a head: 1, 2, 4 or 8
   float* work;   // [items, H, V, N]: every chunk's state
   float* total;  // [items, H]: a chunk's summed log2 decay
   int* form;     // null, or 1 where the step's long portions go through the three launches, else 0 (pick_form)
   float chain, fixed;
+  int per_group;  // heads
 };
 
 // (a base that is the same for a wave and an offset of 32 bits: one register a load in flight instead of two)
@@ -162,8 +162,10 @@ template <typename T, int TAPS, int TN>
 __global__ __launch_bounds__(256, 4) void step_kernel(const Args A) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int vlog = __builtin_ctz(A.vsplit), h = blockIdx.x >> vlog, vpart = blockIdx.x & (A.vsplit - 1), s = blockIdx.y;
-  const int n = A.q_len[s], slot = A.state_slot[s], q0 = A.q_start[s], p0 = A.ctx_len[s] - n;
-  if (n <= 0 || slot < 0) return;
+  const int n = A.q_len[s];
+  if (n <= 0) return;
+  const int slot = A.state_slot[s], q0 = A.q_start[s], p0 = A.ctx_len[s] - n;
+  if (slot < 0) return;
   const bool conv = n <= A.scan_min;  // short: the convolution is done here
   if (!conv && !A.long_too) return;
   const int V = A.V, N = TN ? 4 * TN : A.N, g = (uint32_t)h / (uint32_t)A.per_group, inner = A.H * V;
@@ -180,7 +182,8 @@ __global__ __launch_bounds__(256, 4) void step_kernel(const Args A) {
   const float a = A.a[h], dd = A.d[h], bias = A.dt_bias[h];
   // The state in registers over the portion: a lane's vectors are of rows v0 + lv + k nv. Read and written once a step, past
   // the caches' usual place, which is left to the weights and keys. Bound by these bytes: 64 rows, 64 heads of 64 x 128 take
-  // 48 us, 5.5 TB/s, where nothing but the update of the same bytes takes 43 (4 workgroups a CU or 5: the same).
+  // 48 us, 5.5 TB/s, where nothing but the update of the same bytes takes 43 (4 workgroups a CU or 5: the
+  // same, but those of rows without a sequence, which are gone at once, start faster: 16,384 of them 6.7 us, 5.1 with 5).
   f32x4 st[TN ? REGS : 1];
   // The first token's inputs of a short portion are asked for ahead of the state: its wait then leaves the state's loads in
   // flight, and a thread's second channel waits with the first (64 -> 51 us). That token is apart from the others' loop,
@@ -244,7 +247,9 @@ __global__ __launch_bounds__(256, 4) void step_kernel(const Args A) {
         }
       }
     } else {
-      for (int e = threadIdx.x; e < n_ch; e += 256) {
+      int first_e = threadIdx.x;
+      asm volatile("" : "+v"(first_e));  // (addresses are made anew for every token: kept, they are a workgroup a CU fewer)
+      for (int e = first_e; e < n_ch; e += 256) {
         const int c = channel(e);
         float v;
         if (conv) {
@@ -290,8 +295,10 @@ __global__ __launch_bounds__(256, 4) void step_kernel(const Args A) {
       // that a lane holds in their first three rounds: the same sums in the same order, with 9 shuffles for 40 where 32 lanes
       // share a row (51 -> 48 us).
       float acc[REGS];
+      int top = v0 + lv;
+      if constexpr (!first) asm volatile("" : "+v"(top));
 #pragma unroll
-      for (int k = 0; k < REGS; ++k) acc[k] = step(st[k], 4 * ln, dt * sx[min(v0 + lv + k * nv, v1 - 1)]);
+      for (int k = 0; k < REGS; ++k) acc[k] = step(st[k], 4 * ln, dt * sx[min(top + k * nv, v1 - 1)]);
       int k = 0;
 #pragma unroll
       for (int left = REGS / 2, o = TN / 2; left > 0; left /= 2, o /= 2) {
@@ -305,7 +312,7 @@ __global__ __launch_bounds__(256, 4) void step_kernel(const Args A) {
       }
 #pragma unroll
       for (int o = TN / 16; o > 0; o /= 2) acc[0] += __shfl_xor(acc[0], o, 64);
-      const int v = v0 + lv + k * nv;
+      const int v = top + k * nv;
       if (ln % (TN / 8) == 0 && v < v1) ((T*)A.y)[(size_t)(q0 + t) * A.ldy + h * V + v] = (T)(acc[0] + dd * sx[v]);
     } else {
       const bool fresh = p0 + t == 0;
@@ -910,8 +917,8 @@ extern "C" int pa_state_scan(int fp32, const void* proj, int ldp, void* u, void*
   if (seqs <= 0) return 0;
   if (V % 16 || N % 32 || H % G || scan_min > MAX_SHORT || ring_rows < taps - 1 + scan_min || (taps != 4 && taps != 8)) return -1;  // (shorter ones are padded)
   Args A{proj, u, y, state, ring, conv_w, conv_b, dt_bias, a, d, q_start, q_len, ctx_len, state_slot,
-         (const int4*)items, n_items, ldp, ldy, H, G, V, N, H * V + 2 * G * N, taps, ring_rows, scan_min, fp32, 1, H / G,
-         work, total, nullptr, chain, fixed};
+         (const int4*)items, n_items, ldp, ldy, H, G, V, N, H * V + 2 * G * N, taps, ring_rows, scan_min, fp32, 1,
+         work, total, nullptr, chain, fixed, H / G};
   if (A.Cc % 8 || ldp % 8) return -1;
   // the three launches: (bf16) states that scan_kernel is not built for, or a choice
   const int lds_s = 2 * LC * 4 + (N + 2 * V) * LD * 2;
