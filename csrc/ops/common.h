@@ -98,6 +98,39 @@ __device__ __forceinline__ bool handoff_last(int* counter, int n, int* lflag, in
   return *lflag != 0;
 }
 
+// acc <- a split tile's sum, for the last arriver (handoff_last): its S slices added in their order, so that the sum has the same
+// bits whichever slice arrives last. One of the first two begins with its own registers (their sum is the same either way), another
+// reads its own slab too, at its place. `slab` floats a slice, a lane's quads [I][J] from quad `at` on, 64 apart.
+template <int I, int J>
+__device__ __forceinline__ void sum_slices(f32x4 (&acc)[I][J], const float* base, int slab, int S, int slice, int at) {
+#pragma clang fp reassociate(off)
+  constexpr int G = 8 / J < I ? 8 / J : I;  // 8 loads in flight at least (the accumulators hold the rest)
+  static_assert(I % G == 0, "whole groups");
+  if (slice > 1)
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int j = 0; j < J; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int p = 0; p < S; ++p) {
+    if (p == slice && slice < 2) continue;
+    const __amdgpu_buffer_rsrc_t rp =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float*>(base) + (size_t)p * slab, 0, slab * 4, 0x00020000);
+#pragma unroll
+    for (int i = 0; i < I; i += G) {
+      f32x4 v[G][J];
+#pragma unroll
+      for (int h = 0; h < G; ++h)
+#pragma unroll
+        for (int j = 0; j < J; ++j)
+          v[h][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, (at + ((i + h) * J + j) * 64) * 16, 0, 16));
+#pragma unroll
+      for (int h = 0; h < G; ++h)
+#pragma unroll
+        for (int j = 0; j < J; ++j) acc[i + h][j] += v[h][j];
+    }
+  }
+}
+
 // host-side hand-off modes passed to the kernels with an in-launch hand-off: the GEMM
 // split-K slabs (decode / wide / mid / prefill) and the attention partition merge
 extern int g_handoff_acquire;

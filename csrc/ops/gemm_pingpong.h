@@ -437,7 +437,7 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
   if (G == 0) raw_barrier();  // balance the stagger
   if constexpr (STAMP) st2 = __builtin_amdgcn_s_memtime();
 
-  // ---- split tiles: publish, the last arriver sums the other slices into its registers
+  // ---- split tiles: publish, the last arriver sums the slices
   if (slice >= 0) {
     float* base = A.ws + (size_t)(tile - A.full) * A.S * SLABF;
     {
@@ -452,25 +452,7 @@ __device__ __forceinline__ void pingpong_tile(const Args& A, const int bid, cons
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (!handoff_last(A.counters + (tile - A.full), A.S, reinterpret_cast<int*>(smem), A.acq)) return;
-    for (int p = 0; p < A.S; ++p) {
-      if (p == slice) continue;
-      const __amdgpu_buffer_rsrc_t rp =
-          __builtin_amdgcn_make_buffer_rsrc(base + (size_t)p * SLABF, 0, SLABF * 4, 0x00020000);
-#pragma unroll
-      for (int i = 0; i < F; i += 2) {
-        f32x4 tt[2][4];
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int j = 0; j < 4; ++j)
-            tt[h][j] = __builtin_bit_cast(
-                f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, (((wid * F + i + h) * 4 + j) * 64 + lane) * 16, 0, 16));
-#pragma unroll
-        for (int h = 0; h < 2; ++h)
-#pragma unroll
-          for (int j = 0; j < 4; ++j) acc[i + h][j] += tt[h][j];
-      }
-    }
+    sum_slices(acc, base, SLABF, A.S, slice, wid * F * 256 + lane);
   }
 
   // ---- register epilogue: acc[i][j] holds token row0 + 64 wc + 16 j + c (a group's: row0 + 64 j + 16 wc + c), columns

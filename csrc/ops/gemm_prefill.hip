@@ -33,8 +33,8 @@
 //   * wave quantisation: tiles [0, full) run whole, the remaining tiles are split over S
 //     K-slices (one more round of shorter items instead of a half-empty round). The slices
 //     publish fp32 partials write-through in the accumulators' own fragment order and the
-//     last arriver adds them to its registers after the agent-scope acquire of
-//     common.h handoff_last.
+//     last arriver adds them up, in their order (common.h sum_slices), after the agent-scope
+//     acquire of common.h handoff_last.
 #include "common.h"
 #include "packed_epi.h"
 
@@ -292,7 +292,7 @@ __global__ __launch_bounds__(512) void prefill_gemm_kernel(const Args A) {
     }
   }
 
-  // ---- split tiles: publish, last arriver sums the other slices into its registers
+  // ---- split tiles: publish, the last arriver sums the slices
   if (slice >= 0) {
     float* base = A.ws + (size_t)(tile - A.full) * A.S * SLAB;
     {
@@ -306,24 +306,7 @@ __global__ __launch_bounds__(512) void prefill_gemm_kernel(const Args A) {
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (!handoff_last(A.counters + (tile - A.full), A.S, reinterpret_cast<int*>(smem), A.acq)) return;
-    for (int p = 0; p < A.S; ++p) {
-      if (p == slice) continue;
-      const __amdgpu_buffer_rsrc_t rp = __builtin_amdgcn_make_buffer_rsrc(base + (size_t)p * SLAB, 0, SLAB * 4, 0x00020000);
-#pragma unroll
-      for (int i = 0; i < 8; i += 8 / CPW) {  // 8 loads in flight per lane (the accumulators hold the rest)
-        f32x4 t[8 / CPW][CPW];
-#pragma unroll
-        for (int h = 0; h < 8 / CPW; ++h)
-#pragma unroll
-          for (int j = 0; j < CPW; ++j)
-            t[h][j] = __builtin_bit_cast(f32x4, __builtin_amdgcn_raw_buffer_load_b128(
-                                                    rp, (((wid * 8 + i + h) * CPW + j) * 64 + lane) * 16, 0, 16));
-#pragma unroll
-        for (int h = 0; h < 8 / CPW; ++h)
-#pragma unroll
-          for (int j = 0; j < CPW; ++j) acc[i + h][j] += t[h][j];
-      }
-    }
+    sum_slices(acc, base, SLAB, A.S, slice, wid * 8 * CPW * 64 + lane);
   }
 
   // ---- register epilogue: lane (g, c) of tile (i, j) holds token row 16 i + c (of its
@@ -501,22 +484,7 @@ __global__ __launch_bounds__(512) void prefill_gemm_n128_kernel(const Args A) {
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     if (!handoff_last(A.counters + (tile - A.full), A.S, reinterpret_cast<int*>(smem), A.acq)) return;
-    for (int p = 0; p < A.S; ++p) {
-      if (p == slice) continue;
-      const __amdgpu_buffer_rsrc_t rp =
-          __builtin_amdgcn_make_buffer_rsrc(base + (size_t)p * SLAB128, 0, SLAB128 * 4, 0x00020000);
-      f32x4 t[4][4];
-#pragma unroll
-      for (int i2 = 0; i2 < 4; ++i2)
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          t[i2][j] = __builtin_bit_cast(
-              f32x4, __builtin_amdgcn_raw_buffer_load_b128(rp, (((wid * 4 + i2) * 4 + j) * 64 + lane) * 16, 0, 16));
-#pragma unroll
-      for (int i2 = 0; i2 < 4; ++i2)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i2][j] += t[i2][j];
-    }
+    sum_slices(acc, base, SLAB128, A.S, slice, wid * 1024 + lane);
   }
 
   const float inv_k = 1.f / (float)A.K;

@@ -228,3 +228,22 @@ def test_dense_unit_tiles_without_a_token(gpu, T, live):
     want, got, edge = run(), run(live=slots.to(torch.int32)), (live + 255) // 256 * 256
     assert torch.equal(got[:edge], want[:edge])
     assert (got[edge:] == 7.0).all()
+
+
+@pytest.mark.parametrize("bn,variant", [(256, 3), (256, 1), (192, 3), (128, 3), (128, 1)])
+@pytest.mark.parametrize("S", [3, 4])
+def test_split_tiles_add_up_in_the_order_of_the_slices(gpu, bn, variant, S):
+    """A split tile's sum does not depend on which slice arrives last. Slices of 2^30, 1, (1,) -2^30 are 0 in fp32 added in their
+    order and 1 or 2 from the last one on; values of no such kind give the same bits on every run."""
+    M, N, K = 700, 1536, S * 256
+    x = torch.zeros(M, K, device=gpu, dtype=torch.bfloat16)
+    for s in range(S):
+        x[:, s * 256] = 2.0 ** 30 if s == 0 else -2.0 ** 30 if s == S - 1 else 1.0
+    ones = ops.pack_decode_weight(torch.ones(N, K, device=gpu, dtype=torch.bfloat16))
+    torch.manual_seed(S)
+    y, w = _bf(M, K, dev=gpu), ops.pack_decode_weight(_bf(N, K, dev=gpu))
+    kw = dict(full=0, splits=S, bn=bn, variant=variant)
+    first = ops.prefill_gemm(y, w, **kw)
+    for _ in range(20):
+        assert not ops.prefill_gemm(x, ones, **kw).any()
+        assert torch.equal(ops.prefill_gemm(y, w, **kw), first)
