@@ -685,7 +685,7 @@ at::Tensor lookup(at::Tensor q, at::Tensor masks, at::Tensor minp, int64_t K, at
   const std::vector<at::Tensor> b = lookup_begin(q, masks, minp, K, false);
   try {
     const int64_t Q = q.size(0);
-    at::Tensor ws = at::empty({std::max<int64_t>(16, pa_cosine_topk_workspace_bytes(std::min<int64_t>(Q, 64), std::max<int64_t>(n_valid, 1), K))},
+    at::Tensor ws = at::empty({std::max<int64_t>(16, pa_cosine_topk_workspace_bytes(Q, std::max<int64_t>(n_valid, 1), K))},
                               b[4].options().dtype(at::kByte));
     for (int64_t i = 0; i < Q; i += 64) {
       const int64_t n = std::min<int64_t>(64, Q - i);

@@ -417,11 +417,14 @@ __global__ __launch_bounds__(1024) void cosine_stage2_kernel(float* __restrict__
 
 }  // namespace pa
 
-// workspace = stage-1 top-k lists [Q][nwg][K] (score, row) + per-(slice, query)
-// candidate buffers [nwg][64][CAND] (score, row)
+// workspace = stage-1 top-k lists [Q][nwg][K] (score, row) and, but for a short index, per-(slice, query) candidate buffers
+// [nwg][64][CAND] (score, row). Q > 64: what the largest of its passes of 64 needs (a last one of few queries has more slices of
+// a short index).
 extern "C" long long pa_cosine_topk_workspace_bytes(int Q, int N, int K) {
-  const long long w = pa::sim_num_wg(1, N);  // (the most for any number of queries)
-  return (long long)Q * w * K * 8 + w * pa::SIM_MAXQ * pa::SIM_CAND * 8;
+  if (Q > pa::SIM_MAXQ)
+    return std::max(pa_cosine_topk_workspace_bytes(pa::SIM_MAXQ, N, K), pa_cosine_topk_workspace_bytes((Q - 1) % pa::SIM_MAXQ + 1, N, K));
+  const long long w = pa::sim_num_wg(Q, N);
+  return Q * w * K * 8 + (pa::sim_short(Q, N) ? 0 : w * pa::SIM_MAXQ * pa::SIM_CAND * 8);
 }
 
 extern "C" int pa_cosine_topk(float* out_scores, int* out_rows, void* workspace,

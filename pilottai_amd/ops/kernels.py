@@ -323,8 +323,7 @@ def cosine_topk(queries, index, n_valid: int, K: int, row_priority, row_tags, ro
         C = require_native()
         Q = queries.shape[0]
         out_s, out_r = out if out is not None else topk_result(Q, K, index.device)[1:3]
-        qc = min(Q, COSINE_MAX_Q)
-        need = C.cosine_topk_workspace_bytes(qc, max(1, int(n_valid)), K)
+        need = C.cosine_topk_workspace_bytes(Q, max(1, int(n_valid)), K)
         if workspace is None or workspace.numel() * workspace.element_size() < need:
             workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=index.device)
         # one pass over the index per <= 64 queries (csrc/ops/similarity.hip)

@@ -312,6 +312,36 @@ def test_cosine_topk(gpu, N, D, Q, K):
     assert (r.cpu() == rr).float().mean().item() > 0.95
 
 
+@pytest.mark.parametrize("Q,N", [(1, 1000), (16, 32_768), (17, 32_768), (3, 32_769), (16, 20_000), (17, 20_000), (64, 300)])
+def test_cosine_topk_workspace(gpu, Q, N):
+    """A pass takes what it is said to need, is refused with less and leaves what lies behind alone; a short index needs its
+    slices' lists and nothing else."""
+    C, K, D = ops.kernels.require_native(), 7, 64
+    need = C.cosine_topk_workspace_bytes(Q, N, K)
+    if Q <= 16 and N <= 32_768:
+        assert need <= Q * 256 * K * 8  # (a score and a row)
+    g = torch.Generator(device=gpu).manual_seed(Q)
+    rows = torch.nn.functional.normalize(torch.randn((N + 15) // 16 * 16, D, device=gpu, generator=g), dim=1).to(torch.bfloat16)
+    q = torch.nn.functional.normalize(torch.randn(Q, D, device=gpu, generator=g), dim=1).to(torch.bfloat16)
+    ints = lambda n, dt=torch.int32: torch.zeros(n, dtype=dt, device=gpu)  # noqa: E731
+    room = torch.full((need + 4096,), 77, dtype=torch.uint8, device=gpu)
+    s, r = torch.empty(Q, K, device=gpu), torch.empty(Q, K, dtype=torch.int32, device=gpu)
+    args = (q, ops.pack_decode_weight(rows), N, K, ints(N), ints(N, torch.int64), torch.zeros(N, device=gpu), ints(Q), ints(Q, torch.int64), 0.0)
+    C.cosine_topk(s, r, room[:need], *args)
+    exact = (q.double() @ rows[:N].double().T).topk(K, 1).values
+    torch.testing.assert_close(s.double(), exact, atol=64 * 2.0 ** -24, rtol=0)  # (sums of 64 products in fp32)
+    assert bool((room[need:] == 77).all())
+    with pytest.raises(RuntimeError, match="workspace too small"):
+        C.cosine_topk(s, r, room[:need - 1], *args)
+
+
+@pytest.mark.parametrize("Q", [65, 70, 80, 81, 128, 134])  # a last pass of 1 to 64 queries, on both sides of a short index's 16
+@pytest.mark.parametrize("N", [1000, 20_000, 32_768, 32_769, 1_000_000])
+def test_cosine_topk_workspace_of_passes(Q, N):
+    C = ops.kernels.require_native()
+    assert C.cosine_topk_workspace_bytes(Q, N, 9) == max(C.cosine_topk_workspace_bytes(n, N, 9) for n in (64, Q % 64 or 64))
+
+
 @pytest.mark.parametrize("N,K", [(9000, 64), (20000, 33), (60000, 64), (60000, 5)])  # lists of up to 16,384 entries, of each width
 def test_best_rows_lie_together(gpu, N, K):
     """The second stage of a lookup where the first's lists say little: all of the best in one slice, and all rows alike."""
