@@ -365,7 +365,7 @@ static int pick_nw(int nt, int waves, const DgArgs& a, hipStream_t st) {
 // drains the other, and the stage barrier waits for LDS alone. What bounds it then is the L2s' rate on x, which every
 // column group reads whole: hence the largest tile that still gives every CU one (dispatch_rows).
 // us at 64 rows, before -> after (x from L2, cold weights): N x K 2048 x 8192 37 -> 20, 2048 x 4096 20 -> 11.4, 2048 x 2048
-// 11.7 -> 7.3, 10368 x 2048 17.8 -> 15.8, 128256 x 2048 144 -> 89.
+// 11.7 -> 7.3, 10368 x 2048 17.8 -> 15.8, 128256 x 2048 144 -> 90.
 // SUMS: a workgroup takes one of A.S slices of k and leaves its fp32 sums, row m's of slice s at y [M, A.S, N] (pa_rows_sums).
 template <int MT, int NT, int WK, int D, bool SUMS = false>
 __global__ __launch_bounds__(512) void decode_rows_kernel(const DgArgs A) {
@@ -500,9 +500,11 @@ static int launch_rows(const DgArgs& a, hipStream_t st) {
 // = 8192; 32x32 23), 3072 32x32 (8.2 us at K = 2048; 32x16 10.1), 10368 64x64; 512 rows x 2048 64x64 (13.3 us, the
 // 256-row prefill tiles 19.8), 3072 64x128 (18.3 / 22.0). Where not even 64x128 does (1), up to 64 rows: what every workgroup
 // takes in of x counts against small tiles, a last round that few CUs take part in against large ones. 128 columns (64 rows of 33024
-// x 2048 35.0 us, 64 columns 36.2; 65536 48.8, 52.2; 152064 113, 123; 128256 92, 102), or 256, two a CU, where they fill 7 of 8
-// places at least (128256 x 2048 88.9 us, 5.9 TB/s; x 4096 173, 128 columns 190; 152064 x 2048 123, 98304 71.8). Above, the
-// prefill kernels (512 rows x 10368: 30 us against 52).
+// x 2048 35.0 us, 64 columns 36.2; 65536 48.8, 52.2; 152064 113, 123; 128256 93, 101), or 256, two a CU, where less than a quarter
+// of the last round's 512 places is idle (64 rows, 128 columns -> 256: 106496 x 2048 83.6 -> 76.6 us, 128256 93.0 -> 90.0, 5.8 TB/s,
+// 237568 175 -> 168, 256000 183 -> 180, 368640 268 -> 260; x 4096 167 -> 144, 188 -> 173, 366 -> 342, 385 -> 364, 566 -> 538). With a
+// quarter idle they are as fast, and above slower: one round, 98304 x 2048 72.7 -> 71.6, at 40 rows 68.1 -> 69.7; two, 229376 164.7 ->
+// 165.1; three, 344064 247.0 -> 247.8; 151936 112 -> 124. Above, the prefill kernels (512 rows x 10368: 30 us against 52).
 static int dispatch_rows(const DgArgs& a, hipStream_t st) {
   if (a.M <= 0) return 0;
   if (a.K % 32 || a.N % 16 || a.ldx % 8 || a.ldy % 4 || ((uintptr_t)a.x & 15) || ((uintptr_t)a.wp & 15) || ((uintptr_t)a.y & 7)) return 1;
@@ -513,8 +515,8 @@ static int dispatch_rows(const DgArgs& a, hipStream_t st) {
   if (fits(64, 64)) return launch_rows<4, 4, 8>(a, st);
   if (fits(64, 128)) return launch_rows<4, 4, 4>(a, st);
   if (a.M <= 32) return launch_rows<2, 2, 4>(a, st);
-  const int wide = (a.N + 255) / 256;
-  if (a.M <= 64) return wide >= 448 && wide <= 512 ? launch_rows<4, 2, 1>(a, st) : launch_rows<4, 2, 2>(a, st);
+  const int wide = (a.N + 255) / 256, idle = (512 - wide % 512) % 512;
+  if (a.M <= 64) return idle < 128 ? launch_rows<4, 2, 1>(a, st) : launch_rows<4, 2, 2>(a, st);
   return 1;
 }
 

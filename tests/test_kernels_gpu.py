@@ -444,6 +444,7 @@ def test_decode_gemm(gpu, M, N, K, epi, norm):
 @pytest.mark.parametrize("M,N,K", [
     (17, 16, 32), (32, 4096, 96), (33, 2048, 544), (64, 2048, 8192), (64, 128256, 64), (31, 40_960, 160),  # up to 64 rows
     (33, 33_040, 96), (40, 114_416, 160), (64, 114_448, 32), (48, 131_072, 96), (64, 131_088, 64),  # 128 and 256 columns a tile
+    (64, 98_304, 32), (40, 98_320, 96), (33, 229_376, 32), (64, 229_392, 32), (50, 262_144, 64), (64, 262_160, 32),  # the lines
     (65, 2064, 512), (96, 10368, 2048), (129, 4112, 1056), (512, 2048, 768), (1000, 1040, 64)])             # and more
 def test_rows_gemm(gpu, M, N, K):
     """Every tile of dispatch_rows, at its edges: rows and columns past the tiles, k past the last stage. A bf16 result
