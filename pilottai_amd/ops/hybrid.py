@@ -52,7 +52,11 @@ def hyper_norm(x: torch.Tensor, eps: float, *, y: Optional[torch.Tensor] = None,
         require_hybrid().hyper_norm(x, y, int(partials), y_weights, y2, bias, mix, post, pre, emb, ids, w_next, out, rows,
                                     float(eps), live, sums)
         return out
-    return ref.hyper_norm(x, eps, sums if y is None else y, partials, y_weights, y2, bias, mix, post, pre, emb, ids, w_next, out, rows)
+    if sums is not None:
+        if y is not None or y_weights is not None or sums.dtype != torch.float32:
+            raise RuntimeError("sums must be fp32, in place of y and without weights")
+        y = sums
+    return ref.hyper_norm(x, eps, y, partials, y_weights, y2, bias, mix, post, pre, emb, ids, w_next, out, rows)
 
 
 def rows_sums(x: torch.Tensor, wp: torch.Tensor, slices: int) -> torch.Tensor:
@@ -63,7 +67,10 @@ def rows_sums(x: torch.Tensor, wp: torch.Tensor, slices: int) -> torch.Tensor:
     if _on_gpu(x):
         require_hybrid().rows_sums(y, x, wp, int(slices))
         return y
-    per = -(-(-(-K // 512)) // slices) * 512
+    stages = -(-K // 512)
+    if not 1 <= slices <= stages or -(-stages // slices) * (slices - 1) >= stages:
+        raise RuntimeError(f"rows_sums: {slices} slices of {K} inputs")
+    per = -(-stages // slices) * 512
     w = unpack_decode_weight(wp).float()
     for s in range(slices):
         y.view(M, slices, -1)[:, s] = x[:, s * per:(s + 1) * per].float() @ w[:, s * per:(s + 1) * per].T
