@@ -549,8 +549,8 @@ def test_state_scan_form_in_a_graph(gpu):
 @pytest.mark.gpu
 @pytest.mark.parametrize("V,N,taps", [(64, 128, 4), (48, 128, 8), (32, 256, 4), (128, 64, 4), (256, 32, 8), (16, 256, 4)])
 def test_state_scan_many_sequences(gpu, V, N, taps):
-    """A head in one workgroup, whole and with rows left over, where few sequences spread it over eight: the same bits. Portions
-    of one token and of several, from the first positions (fewer inputs than taps) and later ones."""
+    """A head in one workgroup, whole and with rows left over, against the reference, and the same bits where few sequences spread
+    it over eight. Portions of one token and of several, from the first positions (fewer inputs than taps) and later ones."""
     from pilottai_amd import ops
 
     H, G, S, g = 8, 2, 66, gen(V + N)
@@ -564,16 +564,26 @@ def test_state_scan_many_sequences(gpu, V, N, taps):
     w, cb, bias, a, d = f(taps, C, by=0.5), f(C, by=0.2), f(H) - 2, torch.linspace(0.02, 3.0, H).to(gpu), f(H)
     state0, ring0 = f(S, H, V, N), f(S, rows, C).to(BF16)
 
-    def run(groups):
-        state, ring = state0.clone(), ring0.clone()
-        y = torch.zeros(len(proj), (H * V + 63) // 64 * 64, dtype=BF16, device=gpu)
+    def run(groups, dev=gpu):
+        state, ring = state0.to(dev, copy=True), ring0.to(dev, copy=True)
+        y = torch.zeros(len(proj), (H * V + 63) // 64 * 64, dtype=BF16, device=dev)
+        on = lambda *ts: (t.to(dev) for t in ts)  # noqa: E731
         for i in groups:
-            ops.state_scan(proj, y, state, ring, w, cb, bias, a, d, iv(starts[i]), iv(lens[j] for j in i),
+            ops.state_scan(*on(proj), y, state, ring, *on(w, cb, bias, a, d, iv(starts[i]), iv(lens[j] for j in i),
                            iv(past[j] + lens[j] for j in i), iv(i), iv([-1] * len(i)),
-                           torch.zeros(1, 4, dtype=torch.int32, device=gpu), iv([0]), G)
+                           torch.zeros(1, 4, dtype=torch.int32, device=gpu), iv([0])), G)
         return y, state, ring
-    for one, few in zip(run([list(range(S))]), run([list(range(i, i + 3)) for i in range(0, S, 3)])):
-        assert torch.equal(one, few)
+    one = run([list(range(S))])
+    for all_, few in zip(one, run([list(range(i, i + 3)) for i in range(0, S, 3)])):
+        assert torch.equal(all_, few)
+    y, state, ring = run([list(range(S))], "cpu")
+    assert torch.equal(one[2].cpu(), ring)
+    torch.testing.assert_close(one[0].float().cpu(), y.float(), **tol(BF16, float(y.abs().float().mean())))
+    # The state, in fp32: 2^-18 of what it is made of at nearly all places. A convolved value within fp32's error of the middle of two
+    # bf16 values may round to the other one, here and there (1 in 10^4): by 2^-8 of it, or twice that where two meet, in each of three tokens.
+    err, made = (one[1].cpu() - state).abs(), state.abs() + state0.cpu().abs()
+    assert float((err > 2.0 ** -18 * made + 2.0 ** -20).float().mean()) < 1e-3
+    assert float(err.max()) < 3 * 2 * 2.0 ** -8 * float(made.max())
 
 
 @pytest.mark.gpu
