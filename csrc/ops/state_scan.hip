@@ -159,7 +159,7 @@ constexpr int REGS = 8;  // state vectors of a thread that stay in registers ove
 
 // TN: N / 4 as a constant (8 .. 64) where the state fits the registers of the workgroup; 0: any sizes.
 template <typename T, int TAPS, int TN>
-__global__ __launch_bounds__(256, 4) void step_kernel(const Args A) {
+__global__ __launch_bounds__(256, 5) void step_kernel(const Args A) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int vlog = __builtin_ctz(A.vsplit), h = blockIdx.x >> vlog, vpart = blockIdx.x & (A.vsplit - 1), s = blockIdx.y;
   const int n = A.q_len[s];
@@ -183,7 +183,9 @@ __global__ __launch_bounds__(256, 4) void step_kernel(const Args A) {
   // The state in registers over the portion: a lane's vectors are of rows v0 + lv + k nv. Read and written once a step, past
   // the caches' usual place, which is left to the weights and keys. Bound by these bytes: 64 rows, 64 heads of 64 x 128 take
   // 48 us, 5.5 TB/s, where nothing but the update of the same bytes takes 43 (4 workgroups a CU or 5: the
-  // same, but those of rows without a sequence, which are gone at once, start faster: 16,384 of them 6.7 us, 5.1 with 5).
+  // same, but those of rows without a sequence, which are gone at once, start faster: 16,384 of them 6.7 us, 5.1 with 5. Five are
+  // what the launch bound asks for, 96 registers; the kernel has 82 to 93. Without the two asm statements below it would have
+  // 90 to 99, and under the bound spill up to two of them).
   f32x4 st[TN ? REGS : 1];
   // The first token's inputs of a short portion are asked for ahead of the state: its wait then leaves the state's loads in
   // flight, and a thread's second channel waits with the first (64 -> 51 us). That token is apart from the others' loop,
