@@ -33,8 +33,9 @@ constexpr int SIM_QT = 16;        // queries per MFMA tile (N = 16)
 constexpr int SIM_MAXQ = 64;      // queries per pass (4 tiles resident in LDS)
 constexpr int SIM_MAXD = 1024;    // LDS query capacity per query (bf16)
 // A round of 16 waves x 16 rows a slice at least, 128 KB of row loads in flight per CU. Few queries of an index of which no CU
-// has more than 8 waves' rows take cosine_short_kernel; with many queries their work on the first round is what they wait for
-// (40 of 5,000 rows: slices of 128 rows 29 us, of 256 33).
+// has more than 8 waves' rows take cosine_short_kernel; with many queries their work on the first round is what they wait for,
+// and the merge has more lists to read (both stages, slices of 256 rows and of 128, x 1,024: 40 queries of 5,000 rows 34.8 us and
+// 41.0, 64 48.8 and 53.5, 64 of 32,768 52.5 and 60.9; 17 of 5,000, 29.1 and 27.9, are the other way round).
 constexpr int SIM_ROUND = 256, SIM_SHORT = 32768, SIM_FEW_Q = 16;  // rows of a round; rows and queries of a short index
 constexpr int SIM_THREADS = 4 * SIM_ROUND;
 constexpr int SIM_LIM = 2 * SIM_MAXK;  // entries of a buffer between rounds; a round may admit 256 more
