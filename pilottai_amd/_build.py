@@ -39,7 +39,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 # Per-file code-generation flags. gemm_mid.hip: MFMA accumulators in the VGPR form; with
 # the AGPR form hipcc shuffles them through v_accvgpr moves in the software-pipelined loop.
 # gemm_prefill.hip: its short loops (720 to 1,070 bytes a k-tile of few rows) run at the rate their place in the cache lines
-# gives, and that moved with every change elsewhere in the file: a step of 499 tokens of Bozupel 3,009 to 3,031 us by it, aligned 3,015.
+# gives, and that moved with every change elsewhere in the file: a step of 499 tokens of Bozupel 3,009 to 3,031 us by it, aligned
+# 3,015. This is for times that stay, not for speed: the best places were as fast.
 # No file may use packed fp32 arithmetic (v_pk_*_f32): some forms have given wrong results.
 HIP_FLAGS = ["-ffast-math", "-fno-gpu-rdc", "-Wno-unused-result", "-Xclang", "-target-feature", "-Xclang",
              "-packed-fp32-ops"]
