@@ -53,8 +53,8 @@ def hyper_norm(x: torch.Tensor, eps: float, *, y: Optional[torch.Tensor] = None,
                                     float(eps), live, sums)
         return out
     if sums is not None:
-        if y is not None or y_weights is not None or sums.dtype != torch.float32:
-            raise RuntimeError("sums must be fp32, in place of y and without weights")
+        if y is not None or y_weights is not None or y2 is not None or sums.dtype != torch.float32:
+            raise RuntimeError("sums must be fp32, in place of y, without weights and y2")
         y = sums
     return ref.hyper_norm(x, eps, y, partials, y_weights, y2, bias, mix, post, pre, emb, ids, w_next, out, rows)
 

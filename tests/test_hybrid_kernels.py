@@ -129,7 +129,7 @@ def test_slices_of_sums():
 @devices
 @pytest.mark.parametrize("T,S,D,n", [(9, 4, 2048, 8), (300, 1, 100, 2), (20, 3, 50, 6)])  # whole 4s or not; both widths of a workgroup
 def test_hyper_norm_of_sums(device, T, S, D, n):
-    """Unrounded parts in place of y: as their sum, and refused beside y."""
+    """Unrounded parts in place of y: as their sum, and refused beside y, its weights or a second output."""
     from pilottai_amd import ops
 
     g = gen(T)
@@ -144,8 +144,9 @@ def test_hyper_norm_of_sums(device, T, S, D, n):
     torch.testing.assert_close(xs.double().cpu(), xw, rtol=1e-5, atol=1e-4)
     ops.hyper_norm(x.clone(), 1e-5, y=parts, out=want, **kw)  # (all in fp32)
     torch.testing.assert_close(out.float(), want, rtol=2.0 ** -8, atol=1e-5)
-    with pytest.raises(RuntimeError):
-        ops.hyper_norm(x.clone(), 1e-5, sums=parts, y=parts.to(BF16), out=out, **kw)
+    for beside in (dict(y=parts.to(BF16)), dict(y_weights=torch.ones(T, n, device=device)), dict(y2=torch.ones(T, D, dtype=BF16, device=device))):
+        with pytest.raises(RuntimeError):
+            ops.hyper_norm(x.clone(), 1e-5, sums=parts, out=out, **beside, **kw)
 
 
 @pytest.mark.gpu
