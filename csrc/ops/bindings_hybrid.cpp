@@ -9,6 +9,10 @@ extern "C" {
 int pa_hyper_norm(int fp32, float* x, int S, const void* y, const float* sums, int K, int ldy, const float* y_w, const void* y2, int ldy2,
                   const float* bias, const float* mix, const float* post, const float* pre, const void* emb, const int* ids, int vocab,
                   const float* w_next, void* out, int ldo, const int* rows, const int* live, int n, int D, float eps, hipStream_t st);
+int pa_stream_norm(const void* const* term, const int* ld, int nf, int n_terms, const int* ids, int vocab,
+                   const float* coef, const float* pre, int S, float* x, const void* y, const float* sums, int K, int ldy,
+                   const float* y_w, float* y_kept, const float* w_next, void* out, int ldo, const int* rows, const int* live, int n,
+                   int D, float eps, hipStream_t st);
 int pa_softcap(int fp32, void* x, int ld, int rows, int cols, float cap, hipStream_t st);
 int pa_paged_kv(int fp32, const void* x, const float* bias, void* q, void* kp, void* vp, void* pk, void* pv,
                 const int* positions, const int* slots, const int* q_start, const int* q_len, const int* ctx_len,
@@ -91,6 +95,74 @@ void hyper_norm(at::Tensor x, Opt y, int64_t K, Opt y_w, Opt y2, Opt bias, Opt m
                          rows.has_value() ? ints(*rows, n, "rows") : nullptr, live.has_value() ? ints(*live, T, "live") : nullptr, (int)n,
                          (int)D, (float)eps, cur_stream()),
            "hyper_norm");
+}
+
+// csrc/ops/stream_norm.hip. f: fp32 rows [T, >= D], or [D] for all rows; b: bf16 rows [T, >= D], the first
+// [vocab, >= D] by ids where they are given
+void stream_norm(std::vector<at::Tensor> f, std::vector<at::Tensor> b, Opt ids, at::Tensor coef, at::Tensor pre, Opt x, Opt y, Opt sums,
+                 int64_t K, Opt y_w, Opt y_kept, at::Tensor w_next, at::Tensor out, Opt rows, Opt live, double eps) {
+  check_rows(out, at::kBFloat16, "out");
+  check_gpu(w_next, "w_next");
+  check_gpu(pre, "pre");
+  const int64_t D = w_next.numel(), S = pre.numel(), n = f.size() + b.size();
+  TORCH_CHECK(!(y.has_value() && sums.has_value()), "y or sums");
+  TORCH_CHECK(D % 4 == 0 && n <= 63, "stream_norm takes rows of whole 4s and up to 63 terms");
+  int64_t T = ids.has_value() ? ids->numel() : -1;
+  const auto whole = [](const at::Tensor& t) {
+    return t.stride(0) % 4 == 0 && (uintptr_t)t.data_ptr() % (4 * t.element_size()) == 0;
+  };
+  const auto rows_of = [&](const at::Tensor& t, int64_t per, const char* name) {
+    TORCH_CHECK(t.size(1) >= D && t.size(0) % per == 0 && whole(t), name, " must be [rows, >= D], aligned rows in whole 4s");
+    TORCH_CHECK(T < 0 || t.size(0) / per == T, name, " has other rows than what came before it");
+    T = t.size(0) / per;
+  };
+  std::vector<const void*> tp;
+  std::vector<int> ld;
+  for (auto& t : f) {
+    if (t.dim() == 1) {
+      TORCH_CHECK((uintptr_t)t.data_ptr() % 16 == 0, "a row for all rows must be 16-byte aligned");
+      opt_f32(Opt(t), D, "fp32 term");
+    } else {
+      check_rows(t, at::kFloat, "fp32 term");
+      rows_of(t, 1, "fp32 term");
+    }
+    tp.push_back(t.data_ptr());
+    ld.push_back(t.dim() == 1 ? 0 : t.stride(0));
+  }
+  for (size_t i = 0; i < b.size(); ++i) {
+    check_rows(b[i], at::kBFloat16, "bf16 term");
+    if (i == 0 && ids.has_value()) {
+      TORCH_CHECK(b[0].size(1) >= D && b[0].size(0) > 0 && whole(b[0]), "embedding must be [vocab, >= D], aligned rows in whole 4s");
+    } else {
+      rows_of(b[i], 1, "bf16 term");
+    }
+    tp.push_back(b[i].data_ptr());
+    ld.push_back(b[i].stride(0));
+  }
+  int ldy = 0;
+  TORCH_CHECK(K >= 1 && (!b.empty() || !ids.has_value()), "partials, and a term for ids");
+  for (const Opt* o : {&y, &sums})
+    if (o->has_value()) {
+      check_rows(**o, o == &y ? at::kBFloat16 : at::kFloat, "y");
+      rows_of(**o, K, "y");
+      ldy = (*o)->stride(0);
+    }
+  const bool fresh = y.has_value() || sums.has_value();
+  TORCH_CHECK(T >= 0 && (y.has_value() || !y_w.has_value()) && (fresh || !y_kept.has_value()), "weights and y_kept go with y");
+  const int64_t rows_out = rows.has_value() ? rows->numel() : T;
+  TORCH_CHECK(out.size(0) >= rows_out && out.size(1) >= D && out.stride(0) == out.size(1) && whole(out), "out must be [>= n, >= D], whole 4s");
+  TORCH_CHECK(!rows.has_value() || (!x.has_value() && !y_kept.has_value()), "nothing is kept with rows");
+  const auto fp32 = [&](const Opt& t, int64_t count, const char* name) {
+    TORCH_CHECK(!t.has_value() || (uintptr_t)t->data_ptr() % 16 == 0, name, " must be 16-byte aligned");
+    return const_cast<float*>(opt_f32(t, count, name));
+  };
+  check_rc(pa_stream_norm(tp.data(), ld.data(), (int)f.size(), (int)n, ids.has_value() ? ints(*ids, T, "ids") : nullptr,
+                          ids.has_value() ? b[0].size(0) : 0, opt_f32(Opt(coef), (n + fresh) * S, "coef"), opt_f32(Opt(pre), S, "pre"), S,
+                          fp32(x, T * S * D, "x"), y.has_value() ? y->data_ptr() : nullptr, sums.has_value() ? sums->data_ptr<float>() : nullptr,
+                          (int)K, ldy, opt_f32(y_w, T * K, "y_w"), fp32(y_kept, T * D, "y_kept"), opt_f32(Opt(w_next), D, "w_next"),
+                          out.data_ptr(), out.stride(0), rows.has_value() ? ints(*rows, rows_out, "rows") : nullptr,
+                          live.has_value() ? ints(*live, T, "live") : nullptr, (int)rows_out, (int)D, (float)eps, cur_stream()),
+           "stream_norm");
 }
 
 void softcap(at::Tensor x, int64_t cols, double cap) {
@@ -276,6 +348,7 @@ void matrix_memory(at::Tensor x, at::Tensor y, at::Tensor div, at::Tensor state,
 PYBIND11_MODULE(_hybrid, m) {
   m.doc() = "pilottai_amd CDNA4 (gfx950) kernels: paged attention, recurrent layers, score-routed experts";
   m.def("hyper_norm", &hyper_norm);
+  m.def("stream_norm", &stream_norm);
   m.def("softcap", &softcap);
   m.def("paged_kv", &paged_kv);
   m.def("window_pad", [](int k, int v) {

@@ -49,7 +49,7 @@ SHARED_HIP = ["gemm_decode.hip", "gemm_prefill.hip"]
 MODULES = {
     "latent": (["grouped_gemm.hip", "latent_attention.hip", "latent_cache.hip", "residual_norm.hip"], "bindings_latent.cpp"),
     "hybrid": (["gated_norm.hip", "grouped_gemm.hip", "head_difference.hip", "hyper_norm.hip", "matrix_memory.hip", "paged_kv.hip",
-                "score_route.hip", "state_scan.hip", "window_attention.hip"], "bindings_hybrid.cpp"),
+                "score_route.hip", "state_scan.hip", "stream_norm.hip", "window_attention.hip"], "bindings_hybrid.cpp"),
     "latent_linear": (["gated_norm.hip", "grouped_gemm.hip", "latent_attention.hip", "latent_cache.hip", "linear_attention.hip",
                        "poly_norm.hip", "residual_norm.hip", "score_route.hip"], "bindings_latent_linear.cpp"),
 }

@@ -26,6 +26,8 @@ One step of T tokens (decode rows and prompt portions alike), sublayers in model
   experts     score_route       choices, weights, rows sorted by expert, the shared expert among them
               expert_gemm x 2   one partial output per (token, expert)
   between     hyper_norm        weighted partials + bias into the streams, next norm -> h
+
+Steps of many rows keep no streams: `once` and `between` are stream_norm, sums over the outputs so far (models/streams.py).
 """
 from __future__ import annotations
 
@@ -39,6 +41,7 @@ from pilottai_amd.models.cache import HybridCache, StepMeta
 from pilottai_amd.models.common import PackedLinear, layer_runs, parse_loop
 from pilottai_amd.models.hybrid import (AttentionSpec, DenseSpec, GatedMLP, HybridModel, MixerBlock, PagedAttention, ScoredExperts,
                                         ScoredExpertsSpec, StateSpace, StateSpaceSpec)
+from pilottai_amd.models.streams import Hyper, Residual, StreamPlan
 from pilottai_amd.ops.latent import pad_to
 from pilottai_amd.parallel.comm import TPGroup
 
@@ -167,6 +170,9 @@ PRESETS: Dict[str, MudepelConfig] = {
 
 class MudepelModel(HybridModel):
     NAME = "Mudepel"
+    # Steps of so many rows by sums. One prompt, 8 layers of 4 streams of 2,048, us with streams and by sums: 240 tokens 1,226 and 1,262 (up to
+    # 256 rows hyper_norm has 8 waves to a row), 257 1,451, 1,439, 400 1,546, 1,522, 1,000 2,223, 2,158, 3,658 5,923, 5,707
+    SUMS_MIN_T = 257
 
     def __init__(self, cfg: MudepelConfig, device, dtype=torch.bfloat16, tp: Optional[TPGroup] = None, seed: int = 0,
                  weights_path: Optional[str] = None, max_len: int = 8192, **_):
@@ -195,6 +201,12 @@ class MudepelModel(HybridModel):
                 layer[f"norm{q}"] = f32(1 + t[f"norm{q}"].float())
                 layer[f"hc{q}"] = {k: f32(v) for k, v in sub(f"hc{q}.").items()}
             self.layers.append(layer)
+        self.sums = None
+        if dtype == torch.bfloat16 and 2 <= cfg.streams <= StreamPlan.MAX_STREAMS and d % 4 == 0:
+            subs = [Hyper(L[f"hc{q}"]["mix"], L[f"hc{q}"]["out"], L["mixer"].bias if q == 1 else None,
+                          2 if q == 2 and isinstance(L["mlp"], ScoredExperts) else 1)
+                    for L in (self.layers[i] for i in self.runs) for q in (1, 2) if q == 1 or L["mlp"]]
+            self.sums = StreamPlan(subs, dev)
         self.finish()
 
     def _draw(self, part: str, rand: torch.Tensor, g: torch.Generator):
@@ -224,29 +236,21 @@ class MudepelModel(HybridModel):
         eps, d = cfg.eps, cfg.hidden_size
         ldh = pad_to(d, 64)
         new_h = lambda n=T: torch.empty(n, ldh, dtype=self.dtype, device=dev)  # noqa: E731
-        x = torch.empty(T, cfg.streams, d, dtype=torch.float32, device=dev)
-        step, room = dict(emb=self.embed, ids=meta.input_ids[:T]), self.room(part_o, part_ml)
+        room = self.room(part_o, part_ml)
+        x = Residual(self.sums if T >= self.SUMS_MIN_T and residuals is None else None, cfg.streams, self.embed, meta.input_ids[:T])
         for j, i in enumerate(self.runs):
             L = self.layers[i]
-            h = ops.hyper_norm(x, eps, pre=L["hc1"]["in"], w_next=L["norm1"], out=new_h(), live=meta.slots, **step)
-            step = self._into_streams(L["mixer"](h, meta, kv.layers[j], room), L["hc1"])
+            h = x.norm(eps, pre=L["hc1"]["in"], w_next=L["norm1"], out=new_h(), live=meta.slots)
+            x.add(L["mixer"](h, meta, kv.layers[j], room), L["hc1"]["mix"], L["hc1"]["out"])
             if L["mlp"] is not None:
-                h = ops.hyper_norm(x, eps, pre=L["hc2"]["in"], w_next=L["norm2"], out=new_h(), live=meta.slots, **step)
-                step = self._into_streams(L["mlp"](h, meta), L["hc2"])
+                h = x.norm(eps, pre=L["hc2"]["in"], w_next=L["norm2"], out=new_h(), live=meta.slots)
+                x.add(L["mlp"](h, meta), L["hc2"]["mix"], L["hc2"]["out"])
             if residuals is not None:
-                after = x.clone()
-                ops.hyper_norm(after, eps, **step)
-                residuals.append(after.sum(1))
+                residuals.append(x.sum(eps))
         final = dict(pre=self.ones, w_next=self.norm)
         if embed is not None:
-            self.into_pool(ops.hyper_norm(x, eps, out=new_h(), **final, **step), embed)
-            step = {}
-        hs = ops.hyper_norm(x, eps, out=new_h(num_logit_rows), rows=meta.logit_rows[:num_logit_rows], **final, **step)
-        logits = self.head(hs)
+            self.into_pool(x.norm(eps, out=new_h(), **final), embed)
+        logits = self.head(x.norm(eps, out=new_h(num_logit_rows), rows=meta.logit_rows[:num_logit_rows], **final))
         if cfg.softcap:
             ops.softcap(logits, cfg.vocab_size, cfg.softcap)
         return logits[:, :cfg.vocab_size]
-
-    def _into_streams(self, result, hc) -> dict:
-        y, partials, weights, bias = result
-        return dict([("y" if y.dtype == self.dtype else "sums", y)], partials=partials, y_weights=weights, bias=bias, mix=hc["mix"], post=hc["out"])

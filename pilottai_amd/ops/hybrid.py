@@ -1,13 +1,13 @@
 """Dispatch of the hybrid models' kernels (module _hybrid): attention over paged keys and values with its
 masks, biases and gates, state-space and matrix-memory layers, score-routed experts and fp32 residuals.
 
-Device tensors run the HIP kernels of csrc/ops/{hyper_norm, paged_kv, window_attention, head_difference,
+Device tensors run the HIP kernels of csrc/ops/{hyper_norm, stream_norm, paged_kv, window_attention, head_difference,
 state_scan, matrix_memory, gated_norm, score_route}.hip and raise when the module is missing; CPU tensors run the fp32 references of
 ops/reference.py. Every function takes its constants as arguments and works in bf16 or fp32.
 """
 from __future__ import annotations
 
-from typing import Optional, Tuple
+from typing import Optional, Sequence, Tuple
 
 import torch
 
@@ -57,6 +57,36 @@ def hyper_norm(x: torch.Tensor, eps: float, *, y: Optional[torch.Tensor] = None,
             raise RuntimeError("sums must be fp32, in place of y, without weights and y2")
         y = sums
     return ref.hyper_norm(x, eps, y, partials, y_weights, y2, bias, mix, post, pre, emb, ids, w_next, out, rows)
+
+
+def stream_norm(f: Sequence[torch.Tensor], b: Sequence[torch.Tensor], coef: torch.Tensor, eps: float, *, pre: torch.Tensor,
+                w_next: torch.Tensor, out: torch.Tensor, ids: Optional[torch.Tensor] = None, y: Optional[torch.Tensor] = None,
+                sums: Optional[torch.Tensor] = None, partials: int = 1, y_weights: Optional[torch.Tensor] = None,
+                y_kept: Optional[torch.Tensor] = None, x: Optional[torch.Tensor] = None, rows: Optional[torch.Tensor] = None,
+                live: Optional[torch.Tensor] = None) -> torch.Tensor:
+    """hyper_norm of streams that are sums x_s = sum_t coef[t, s] term_t (csrc/ops/stream_norm.hip). Terms, in
+    this order: f, fp32 [T, >= D] or [D] for all rows; b, bf16 [T, >= D], b[0] by ids if they are given; the sum of y's or sums'
+    partials. out = norm(sum_s pre[s] x_s) * w_next; x [T, S, D] and y_kept [T, D] (fp32, optional) <- the streams and y's sum.
+    `rows`, `live`: as hyper_norm's; nothing is kept with rows."""
+    if _on_gpu(out):
+        require_hybrid().stream_norm(list(f), list(b), ids, coef, pre, x, y, sums, int(partials), y_weights, y_kept, w_next, out, rows,
+                                     live, float(eps))
+        return out
+    D, S = w_next.numel(), pre.numel()
+    vs = [(t[None] if t.dim() == 1 else t)[:, :D] for t in f]
+    vs += [(t[ids.long().clamp(0, len(t) - 1)] if i == 0 and ids is not None else t)[:, :D].float() for i, t in enumerate(b)]
+    if y is not None or sums is not None:
+        v = (sums if y is None else y)[:, :D].float().view(-1, partials, D)
+        vs.append(v.sum(1) if y_weights is None else (v * y_weights.view(-1, partials)[:, :, None]).sum(1))
+        if y_kept is not None:
+            y_kept.copy_(vs[-1])
+    s = sum(c[:, None] * v[:, None] for c, v in zip(coef.view(-1, S), vs))
+    if x is not None:
+        x.copy_(s)
+    u = (pre[:, None] * (s if rows is None else s[rows.long()])).sum(1)
+    out[:len(u), :D] = (u * torch.rsqrt(u.pow(2).mean(-1, keepdim=True) + eps) * w_next).to(out.dtype)
+    out[:len(u), D:] = 0
+    return out
 
 
 def rows_sums(x: torch.Tensor, wp: torch.Tensor, slices: int) -> torch.Tensor:

@@ -1,0 +1,100 @@
+"""Sums over a step's outputs in place of its residual streams (models/streams.py) against the streams themselves in float64."""
+import pytest
+import torch
+
+from pilottai_amd.models.streams import Hyper, Residual, StreamPlan
+from test_mudepel import close, engine, expect, feed, folder, tokens  # noqa: F401
+
+DEVICES = ["cpu", pytest.param("cuda:0", marks=pytest.mark.gpu)]
+
+
+@pytest.mark.parametrize("device", DEVICES)
+# sums to the end, and up to where streams take over; widths of part of a pass, one, and two; more biases than a sum's terms
+@pytest.mark.parametrize("S,subs,D,T,biases", [(4, 16, 1024, 5, 3), (2, 13, 16, 3, 2), (3, 13, 2056, 4, 3), (4, 27, 44, 300, 3), (8, 40, 64, 1, 1),
+                                               (2, 3, 8, 2, 1)])
+def test_sums_are_the_streams(device, S, subs, D, T, biases):
+    g = torch.Generator().manual_seed(S * subs + D)
+    rand = lambda *s: torch.randn(*s, generator=g).to(device)  # noqa: E731
+    parts = [(1, 3, 1, 7, 2)[j % 5] for j in range(subs)]
+    layers = [Hyper(rand(S, S) / S ** 0.5, rand(S), rand(D) if j % biases == 0 else None, 1 + (parts[j] > 1)) for j in range(subs)]
+    w, embed, ld = rand(D), rand(31, D).bfloat16(), D + 64
+    ids = torch.randint(-2, 33, (T,), generator=g, dtype=torch.int32).to(device)
+    X = embed[ids.long().clamp(0, 30)].double()[:, None].expand(-1, S, -1)
+    size = X.abs()  # what the sums' magnitudes come to: fp32 sums of n terms err by n 2^-24 of it
+    plan = StreamPlan(layers, device)
+    units = sum(h.units for h in layers)
+    assert plan.whole == (units <= 5 * S and subs + sum(h.bias is not None for h in layers) < 63) and 0 < plan.end <= subs
+    step = Residual(plan, S, embed, ids)
+
+    def check(**kw):
+        pre, rows = rand(S), kw.get("rows")
+        got = step.norm(1e-5, pre=pre, w_next=w, out=torch.full((T if rows is None else len(rows), ld), 7.0, device=device).bfloat16(), **kw)
+        u, m = (torch.einsum("s,tsd->td", p, x)[slice(None) if rows is None else rows.long()] for p, x in ((pre.double(), X), (pre.double().abs(), size)))
+        r = torch.rsqrt(u.pow(2).mean(-1, keepdim=True) + 1e-5)
+        want, bound = u * r * w.double(), 8 * (S + subs) * 2.0 ** -24 * (m + m.pow(2).mean(-1, keepdim=True).sqrt()) * r * w.double().abs()
+        assert bool(((got[:, :D].double() - want).abs() <= bound + 2.0 ** -8 * want.abs()).all()) and not got[:, D:].any()
+    for h, K in zip(layers, parts):
+        check()
+        y, yw = rand(T * K, D + 8).bfloat16(), torch.rand(T, K, generator=g).to(device) if K > 2 else None
+        if K == 2:
+            y = y.float()  # unrounded parts
+        step.add((y, K, yw, h.bias), h.mix, h.post)
+        v = y[:, :D].double().view(T, K, D) * (1.0 if yw is None else yw.double()[:, :, None])
+        each, v = v.abs().sum(1), v.sum(1)
+        if h.bias is not None:
+            v, each = v + h.bias.double(), each + h.bias.double().abs()
+        X = torch.einsum("st,nsd->ntd", h.mix.double(), X) + h.post.double()[None, :, None] * v[:, None]
+        size = torch.einsum("st,nsd->ntd", h.mix.double().abs(), size) + h.post.double().abs()[None, :, None] * each[:, None]
+    rows = torch.tensor([T - 1, 0, T - 1], dtype=torch.int32, device=device)
+    check(rows=rows)
+    check()
+    check(rows=rows)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("D,T", [(2048, 300), (72, 257)])
+def test_same_bits_without_mixing(gpu, D, T):
+    """Where streams are not mixed, sums come to the bits of hyper_norm."""
+    g = torch.Generator(device=gpu).manual_seed(D)
+    rand = lambda *s: torch.randn(*s, device=gpu, generator=g)  # noqa: E731
+    mix, post, embed, w = torch.eye(4, device=gpu), torch.ones(4, device=gpu), rand(31, D).bfloat16(), rand(D)
+    ids = torch.arange(T, dtype=torch.int32, device=gpu) % 31
+    subs = [Hyper(mix, post, None, 1)] * 16
+    a, b = Residual(StreamPlan(subs, gpu), 4, embed, ids), Residual(None, 4, embed, ids)
+    for _ in range(16):
+        y = rand(T, D + 8).bfloat16()
+        got, want = (r.norm(1e-5, pre=post / 4, w_next=w, out=torch.empty(T, D, dtype=torch.bfloat16, device=gpu)) for r in (a, b))
+        assert torch.equal(got, want)
+        for r in (a, b):
+            r.add((y, 1, None, None), mix, post)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,live", [(2049, 1), (2500, 2047)])
+def test_rows_without_a_token_stay(gpu, T, live):
+    """Padding rows of large steps are left as they were, in the input and in what is kept."""
+    from pilottai_amd import ops
+
+    g = torch.Generator(device=gpu).manual_seed(T)
+    terms = [torch.randn(T, 256, device=gpu, generator=g), torch.randn(T, 256, device=gpu, generator=g).bfloat16()]
+    slots = torch.arange(T, dtype=torch.int32, device=gpu)
+    slots[live:] = -1
+    coef, pre, w = (torch.randn(*s, device=gpu, generator=g) for s in ((2, 3), (3,), (256,)))
+
+    def run(**kw):
+        out, x = torch.full((T, 256), 7.0, device=gpu).bfloat16(), torch.full((T, 3, 256), 7.0, device=gpu)
+        return ops.stream_norm(terms[:1], terms[1:], coef, 1e-5, pre=pre, w_next=w, out=out, x=x, **kw), x
+    (a, xa), (c, xc) = run(), run(live=slots)
+    assert torch.equal(a[:live], c[:live]) and torch.equal(xa[:live], xc[:live]) and (c[live:] == 7.0).all() and (xc[live:] == 7.0).all()
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("name", ["varied", "state_only", "wide"])
+def test_model_of_sums(folder, monkeypatch, name, device):
+    """Portions of any length by sums: routed experts' partials, biases, a looped stack."""
+    from pilottai_amd.models.mudepel import MudepelModel
+
+    monkeypatch.setattr(MudepelModel, "SUMS_MIN_T", 1)
+    eng, ids = engine(folder, name, device, "bfloat16"), tokens(name, 150)
+    assert eng.model.sums is not None
+    close(feed(eng, 1, ids, [70, 1, 79]), expect(folder, name, ids), "bfloat16")
