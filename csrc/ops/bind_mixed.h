@@ -41,9 +41,11 @@ void score_route(at::Tensor h, at::Tensor w, at::Tensor slots, at::Tensor weight
   const int64_t T = h.size(0), P = T * (top + always);
   TORCH_CHECK(G == 1 && N >= E && K <= h.size(1) && h.stride(0) % 8 == 0 && tm >= 1, "score_route sizes");
   TORCH_CHECK(tiles.dim() == 2 && tiles.size(1) == 4, "tiles must be [n, 4]");
+  out_ints(counts, E + always, "counts");  // (a place of the caller's, where one workgroup counts for all)
+  const at::Tensor each = T > 16 ? at::empty({(T + 15) / 16, E + always}, counts.options()) : counts;
   check_rc(pa_score_route(f, h.data_ptr(), h.stride(0), w.data_ptr(), K, ints(slots, T, "slots"),
                           (float*)opt_f32(weights, P, "weights"), out_ints(choice, P, "choice"), out_ints(rank, P, "rank"),
-                          out_ints(counts, E + always, "counts"), out_ints(order, P, "order"), out_ints(tiles, 4, "tiles"),
+                          each.data_ptr<int>(), out_ints(order, P, "order"), out_ints(tiles, 4, "tiles"),
                           out_ints(n_tiles, 1, "n_tiles"), T, E, top, groups, keep, always, tm, tiles.size(0), softmax ? 1 : 0,
                           opt_f32(correction, E, "correction"), share ? 1 : 0, (float)scale, cur_stream()),
            "score_route");

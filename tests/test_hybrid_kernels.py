@@ -709,3 +709,10 @@ def test_gated_mlp_module(device, dt, T, d, ff):
     y = mod(h.to(device), None)[0].double().cpu()[:, :d]
     want = oracle.gated(h[:, :d].double(), {k: v.double() for k, v in t.items()}, "", oracle.gelu_tanh)
     torch.testing.assert_close(y, want, **tol(dt, 2.0))
+
+
+@pytest.mark.gpu
+# rows of one and several workgroups' counts, a last part; more experts than threads; more workgroups than the 64 that place them
+@pytest.mark.parametrize("T,E,top,always", [(65, 64, 6, 1), (1100, 64, 6, 1), (300, 700, 4, 2), (4300, 20, 3, 0)])
+def test_rows_of_many_workgroups_are_placed(gpu, T, E, top, always):
+    test_score_route(gpu, BF16, T, E, top, 1, 1, always)
