@@ -735,7 +735,7 @@ __global__ __launch_bounds__(512) void pingpong_grouped_kernel(Args A, const int
                                                                const int* __restrict__ n_tiles,
                                                                const int* __restrict__ order, long long wstride,
                                                                int x_div, int out_order, int heavy) {
-  __shared__ __attribute__((aligned(1024))) char smem[(F == 8 ? 2 * 4 : 3 * 3) * PP_PART];
+  __shared__ __attribute__((aligned(1024))) char smem[3 * 3 * PP_PART];
   // Column tiles of one row tile lie next to each other on one XCD: they share its rows of x. A single group's tiles go in
   // blocks of RUN row tiles, column tile by column tile, so that an XCD takes in a block's rows and its own share of the
   // weights once (beside the MFMAs, that is the bound). 2 x 8192 x 2048 outputs, us, one row tile after the other -> RUN 4:
@@ -744,8 +744,9 @@ __global__ __launch_bounds__(512) void pingpong_grouped_kernel(Args A, const int
   // Groups from number `heavy` on hold every row. Their tiles, the last of the list and full ones whose products take longer
   // than the others' weights, were all on one XCD, behind the others; they go first, the same number on each XCD (6 of 64 such experts and
   // one for all, gate and up, us: 260 tokens 137 -> 131, 700 151 -> 140, 1,000 157 -> 146, 1,500 194 -> 191, 2,000 205 -> 205, 4,000
-  // 333 -> 316. The second product, of fewer columns, gains nothing up to 1,500 tokens and loses 2 % at 2,000 to 3,000.)
-  const int n = n_tiles[0], xcd = blockIdx.x & 7, at = blockIdx.x >> 3;
+  // 333 -> 316. Of the second product they are the last XCD's tail: with the halves below, 1,000 tokens both products 277 in their order, 271 so.)
+  const int n = n_tiles[0], xcd = blockIdx.x & 7;
+  int at = blockIdx.x >> 3, half = -1;
   // item i of this XCD's share of `count` tiles from `first` on; false: it has fewer
   int k = 0, nt = 0;
   auto in_order = [&](int i, int count) {
@@ -762,9 +763,20 @@ __global__ __launch_bounds__(512) void pingpong_grouped_kernel(Args A, const int
     k = first + c0 + j - nt * m;
     return true;
   };
+  // Of a share of `count` items, those behind its last whole round of an XCD's 32 CUs go as two of 128 columns each, where the CUs
+  // hold them all and there are workgroups for them. 64 experts of 2 x 1408 x 2048 and back, 6 a token and one for all, us: 400 tokens (a share
+  // of 66 in the second product) 250 -> 243, 500 255 -> 245, 1,000 277 -> 271, 2,000 350 -> 333, 3,000 (other remainders) 473, 473.
+  auto narrow_tail = [&](int count) {
+    const int full = count & ~31, tail = at - full;
+    if (F == 8 && tail >= 0 && 2 * (count - full) <= 32 && 2 * count - full <= (int)gridDim.x >> 3) {
+      half = tail & 1;
+      at = full + (tail >> 1);
+    }
+  };
   if constexpr (WALK == ONE_GROUP) {
     if (!in_blocks(at, 0, n)) return;
   } else if constexpr (WALK == IN_ORDER) {
+    narrow_tail((n * A.NT + 7) >> 3);
     if (!in_order(at, n)) return;
   } else {
     const int lane = threadIdx.x & 63;
@@ -778,6 +790,7 @@ __global__ __launch_bounds__(512) void pingpong_grouped_kernel(Args A, const int
     }
     // (their eighths are rounded up: the last XCDs may have fewer, of which the others' share takes no notice)
     const int per = (last * A.NT + 7) >> 3;
+    narrow_tail(per + (((n - last) * A.NT + 7) >> 3));
     if (at < per ? !in_blocks(at, n - last, last) : !in_order(at - per, n - last)) return;
   }
   const int4 tl = tiles[k];
@@ -794,6 +807,11 @@ __global__ __launch_bounds__(512) void pingpong_grouped_kernel(Args A, const int
   else A.y += (size_t)tl.y * A.ldy;
   A.MT = 1;
   // MT = 1: pingpong_tile's tile index is the column tile
+  if constexpr (F == 8 && WALK != ONE_GROUP)
+    if (__builtin_expect(half >= 0, 0)) {
+      pingpong_tile<EPI, false, false, 4, true>(A, 2 * nt + half, 2 * A.NT, smem);
+      return;
+    }
   pingpong_tile<EPI, false, false, F, true>(A, nt, A.NT, smem);
 }
 }  // namespace pf

@@ -614,7 +614,7 @@ class ScoredExperts:
         ops.expert_gemm(h, self.w13, act, tiles, n_tiles, order, rows, x_div=K, out_order=False, tm=tm, glu=s.act,
                         relu2=s.act is None, row_w=weights if s.weigh_input else None, always=s.always)
         y = torch.empty(rows, self.dn, dtype=self.dtype, device=dev)
-        ops.expert_gemm(act, self.w2, y, tiles, n_tiles, order, rows, x_div=0, out_order=True, tm=tm)
+        ops.expert_gemm(act, self.w2, y, tiles, n_tiles, order, rows, x_div=0, out_order=True, tm=tm, always=s.always)
         return y, K, None if s.weigh_input else weights, None
 
 

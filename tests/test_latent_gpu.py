@@ -228,6 +228,13 @@ def test_tiles_of_groups_of_every_row(gpu, counts, always, N, K):
     sorted_rows(gpu, 256, counts, N, K, always)
 
 
+@pytest.mark.parametrize("counts,always", [([3] * 70 + [0] * 40, 0), ([4] * 6 + [0] * 10, 0), ([70, 0] * 26 + [0] * 20 + [300], 1), ([9] * 64 + [0] * 40, 0)])
+@pytest.mark.parametrize("N,K", [(1280, 128), (512, 320)])
+def test_remainders_of_whole_rounds(gpu, counts, always, N, K):
+    """Tiles behind an XCD's last 32, none and up to 16 of them, in halves."""
+    sorted_rows(gpu, 256, counts, N, K, always)
+
+
 def test_groups_of_every_row_are_some(gpu):
     from pilottai_amd import ops
 
