@@ -17,7 +17,7 @@ int pa_latent_attention(int fp32, void* out, float* part_o, float* part_ml, cons
                         const int* items, const int* n_items, int max_items, const int* q_start,
                         const int* q_len, const int* ctx_len, const int* block_table, int max_blocks, int H, int Rp,
                         int rp, int dec_tokens, int tile_tokens, int window, float scale_log2, int simple,
-                        const pa::la::Expand* expand, hipStream_t st);
+                        const pa::la::Expand* expand, const void* uv, void* y, int ldy, int vp, int T, hipStream_t st);
 int pa_latent_plan(const pa::la::Expand* X, const int* q_start, const int* q_len, const int* ctx_len, int S, int T, int H, int window,
                    int room, int max_att, int max_tiles, int slots, hipStream_t st);
 int pa_latent_expand(const pa::la::Expand* X, const void* pages, const void* wk, const void* wv, const int* block_table, int max_blocks, int H, int D,
@@ -171,7 +171,7 @@ void latent_attention(at::Tensor out, at::Tensor part_o, at::Tensor part_ml, at:
                       at::Tensor pages, at::Tensor items, at::Tensor n_items, at::Tensor q_start, at::Tensor q_len,
                       at::Tensor ctx_len, at::Tensor block_table, int64_t dec_tokens, int64_t tile_tokens,
                       int64_t window, double scale, bool simple, const Tensors& plan, const Tensors& expand, int64_t room,
-                      int64_t slots) {
+                      int64_t slots, Opt uv, Opt y) {
   const int f = is_f32(q, "q");
   for (auto* t : {&out, &q, &pages}) {
     check_gpu(*t, "latent_attention arg");
@@ -186,6 +186,18 @@ void latent_attention(at::Tensor out, at::Tensor part_o, at::Tensor part_ml, at:
   const int64_t NB = (dec_tokens * H + 15) / 16;
   TORCH_CHECK(Rp > 0 && rp >= 0 && dec_tokens >= 1 && tile_tokens >= 1, "latent_attention sizes");
   TORCH_CHECK(part_o.numel() >= mi * NB * 16 * Rp && part_ml.numel() >= mi * NB * 32, "partition workspace too small");
+  // uv: the heads' products with W_uv, to y [T, >= H vp] in place of out (which then holds anything)
+  int ldy = 0, vp = 0;
+  if (uv.has_value()) {
+    check_gpu(*uv, "uv");
+    check_dtype(*uv, at::kBFloat16, "uv");
+    TORCH_CHECK(!f && y.has_value() && uv->dim() == 5 && uv->size(0) == H && uv->size(2) * 32 == Rp && uv->size(3) == 64 && uv->size(4) == 8,
+                "uv must be packed [H, vp/16, Rp/32, 64, 8], with y");
+    check_rows(*y, at::kBFloat16, "y");
+    vp = uv->size(1) * 16;
+    ldy = y->stride(0);
+    TORCH_CHECK(y->size(0) == q.size(0) && y->size(1) >= H * vp && ldy % 4 == 0 && ((uintptr_t)y->data_ptr() & 7) == 0, "y must be [T, >= H vp], 8-byte aligned");
+  }
   // expanded requests: expand = [kx, kr, q not yet absorbed or rotated, cos_sin, their outputs, partial outputs and (max, sum)];
   // room and slots: as the plan was made with
   pa::la::Expand X{};
@@ -215,7 +227,8 @@ void latent_attention(at::Tensor out, at::Tensor part_o, at::Tensor part_ml, at:
                                ints(q_start, S, "q_start"), ints(q_len, S, "q_len"), ints(ctx_len, S, "ctx_len"),
                                ints(block_table, 0, "block_table"), block_table.size(1), H, Rp, rp, dec_tokens,
                                tile_tokens, window, (float)(scale * 1.4426950408889634), simple ? 1 : 0,
-                               expand.empty() ? nullptr : &X, cur_stream()),
+                               expand.empty() ? nullptr : &X, uv.has_value() ? uv->data_ptr() : nullptr,
+                               uv.has_value() ? y->data_ptr() : nullptr, ldy, vp, q.size(0), cur_stream()),
            "latent_attention");
 }
 

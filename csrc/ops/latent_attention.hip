@@ -28,6 +28,8 @@
 //                     tiles that arrive by direct global -> LDS loads. A step with few such items
 //                     has them cut into partitions of their keys too (8 slots each).
 //
+// Steps of few tokens have the heads' products with W_uv behind the merge in the same launch (merge_heads_kernel).
+//
 // Prompt portions of the widest latents have a second form (latent_expand.h), whose units the same launches run.
 #include "common.h"
 #include "latent_expand.h"
@@ -1275,6 +1277,136 @@ __global__ __launch_bounds__(64 * NW, 2) void mfma_kernel(const Args A) {
   }
 }
 
+// merge_kernel and the next product in one launch, y[row, head h] = W_uv[h] (merged latent): a workgroup of 16 waves per (head, `per`
+// columns, up to 16: tokens of the items in their order). The waves share the columns' partitions, while the head's W_uv is on its
+// way: a wave has 16 of its (at most 128) rows and half of their inputs. A chain of dependent reads bounds it (items, (max, sum) pairs, partitions),
+// where two launches had each their own: 4 rows after 2,000 tokens, 16 heads of 512 and 128, a step's 8 layers 1,064 -> 1,040 us, 32 rows
+// 2,037 -> 2,005. (A workgroup for 16 items, whatever tokens they hold, took 3 to 5 % longer for steps of short prompts.)
+constexpr int MH_WAVES = 16;
+template <int RT>
+__global__ __launch_bounds__(64 * MH_WAVES) void merge_heads_kernel(const Args A, const bf16* __restrict__ uv, bf16* __restrict__ y, int ldy,
+                                                                    int vp, int max_items, int per) {
+  constexpr int RP = 32 * RT, LD = RP + 8, HALF = (RT + 1) / 2;
+  __shared__ __attribute__((aligned(16))) bf16 xs[16][LD];
+  __shared__ __attribute__((aligned(16))) float ps[MH_WAVES][RP < 256 ? 256 : RP];
+  __shared__ int4 cols[16];  // {the first partition's column, the item's z, sequence, token}
+  __shared__ int sums[MH_WAVES];
+  const int h = blockIdx.x, lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tiles = vp / 16;
+  const int g = lane >> 4, c16 = lane & 15, d = min(lane * 8, RP - 8), tile = wid & 7, k0 = wid >> 3 ? HALF : 0;
+  const float2* ml = reinterpret_cast<const float2*>(A.part_ml);
+  bf16x8 w[HALF];
+#pragma unroll
+  for (int k = 0; k < HALF; ++k)
+    w[k] = *reinterpret_cast<const bf16x8*>(uv + (((size_t)h * tiles + min(tile, tiles - 1)) * RT + min(k0 + k, RT - 1)) * 512 + lane * 8);
+  const int lo = blockIdx.y * per;
+  int total = 0;
+  for (int b = 0; b < max_items && total < lo + per; b += 64 * MH_WAVES) {
+    const int4 it = A.items[min(b + (int)threadIdx.x, max_items - 1)];  // (on its way with the list's length)
+    const bool in = b + (int)threadIdx.x < A.n_items[0] && ((it.z >> 8) & 0xfff) == 0;
+    const int nq = in ? it.z & 0xff : 0;
+    int at = nq;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(at, o, 64);
+      if (lane >= o) at += v;
+    }
+    if (lane == 63) sums[wid] = at;
+    __syncthreads();
+    int before = total - nq;
+#pragma unroll
+    for (int q = 0; q < MH_WAVES; ++q) {
+      if (q < wid) before += sums[q];
+      total += sums[q];
+    }
+    at += before;  // this item's first column
+    for (int t = max(0, lo - at); t < nq && at + t < lo + per; ++t)
+      cols[at + t - lo] = int4{it.w * A.NB * 16 + t * A.H + h, it.z, it.x, it.y + t};
+    __syncthreads();
+  }
+  const int m = min(per, total - lo);
+  if (m <= 0) return;
+  const int mine = min(c16, m - 1), row = A.q_start[cols[mine].z] + cols[mine].w;
+  const int shift = m > 8 ? 0 : m > 4 ? 1 : m > 2 ? 2 : m > 1 ? 3 : 4, waves = 1 << shift;  // of a column
+  const int c = wid >> shift, part = wid & (waves - 1);
+  float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  if (c < m) {
+    const int4 e = cols[c];
+    const int nparts = e.y >> 20, step = (e.y & 0xff) <= A.dec_tokens ? 1 : 8;
+    if (nparts <= 1) {
+      if (part == 0) {
+        const bf16x8 o = *reinterpret_cast<const bf16x8*>((const bf16*)A.out + ((size_t)(A.q_start[e.z] + e.w) * A.H + h) * RP + d);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) a[j] = (float)o[j];
+      }
+    } else {
+      auto slot = [&](int p) { return (size_t)e.x + (size_t)p * step * A.NB * 16; };
+      float gm = NEG_BIG, L = 0.f;
+      for (int p0 = 0; p0 < nparts; p0 += 64) gm = fmaxf(gm, p0 + lane < nparts ? ml[slot(p0 + lane)].x : NEG_BIG);
+      gm = wave_max(gm);
+      for (int p0 = 0; p0 < nparts; p0 += 64) {
+        float wt = 0.f;
+        if (p0 + lane < nparts) {
+          const float2 v = ml[slot(p0 + lane)];
+          wt = exp2f(v.x - gm);
+          L += wt * v.y;
+        }
+        const int np = min(64, nparts - p0);
+#pragma unroll 8
+        for (int p = part; p < np; p += waves) {
+          const float wp = __shfl(wt, p, 64);
+          const f32x4* s = reinterpret_cast<const f32x4*>(A.part_o + slot(p0 + p) * RP + d);
+          const f32x4 x = s[0], z = s[1];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            a[j] += wp * x[j];
+            a[4 + j] += wp * z[j];
+          }
+        }
+      }
+      const float inv = 1.f / wave_sum(L);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) a[j] *= inv;
+    }
+    if (lane * 8 < RP) {
+      if (shift == 0) {
+        bf16x8 v;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = (bf16)a[j];
+        *reinterpret_cast<bf16x8*>(&xs[c][d]) = v;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) ps[wid][d + j] = a[j];
+      }
+    }
+  }
+  __syncthreads();
+  if (shift) {
+    for (int i = threadIdx.x; i < m * RP; i += 64 * MH_WAVES) {
+      const int q = i / RP, k = i - q * RP;
+      float v = 0.f;
+      for (int r = 0; r < waves; ++r) v += ps[q * waves + r][k];
+      xs[q][k] = (bf16)v;
+    }
+    __syncthreads();
+  }
+  // (columns behind the last one hold anything: their products are not stored)
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int k = 0; k < HALF; ++k)
+    if (k0 + k < RT)
+      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[k], *reinterpret_cast<const bf16x8*>(&xs[c16][32 * (k0 + k) + 8 * g]), acc, 0, 0, 0);
+  f32x4* other = reinterpret_cast<f32x4*>(ps[tile]) + lane;
+  if (k0) *other = acc;
+  __syncthreads();
+  if (!k0 && c16 < m && tile < tiles) {
+    acc += *other;
+    bf16x4 o;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) o[r] = (bf16)acc[r];
+    *reinterpret_cast<bf16x4*>(y + (size_t)row * ldy + (size_t)h * vp + tile * 16 + 4 * g) = o;
+  }
+}
+
 }  // namespace la
 }  // namespace pa
 
@@ -1293,7 +1425,9 @@ extern "C" int pa_latent_pad(int R) {
 extern "C" int pa_latent_attention(int fp32, void* out, float* part_o, float* part_ml, const void* q, const void* pages, const int* items, const int* n_items, int max_items,
                                    const int* q_start, const int* q_len, const int* ctx_len, const int* block_table,
                                    int max_blocks, int H, int Rp, int rp, int dec_tokens, int tile_tokens, int window,
-                                   float scale_log2, int simple, const pa::la::Expand* expand, hipStream_t st) {
+                                   float scale_log2, int simple, const pa::la::Expand* expand, const void* uv, void* y, int ldy, int vp,
+                                   int T, hipStream_t st) {
+  // uv [H, vp / 16, RT, 64, 8] (optional): y [T, H vp] is written in place of out, see merge_heads_kernel
   if (max_items <= 0) return 0;
   const int D = Rp + rp, NB = (dec_tokens * H + 15) / 16;
   if (Rp % 32 || rp % 32 || H <= 0 || dec_tokens <= 0 || tile_tokens <= 0) return -1;
@@ -1301,6 +1435,10 @@ extern "C" int pa_latent_attention(int fp32, void* out, float* part_o, float* pa
                  block_table, max_blocks, H, NB, Rp, D, dec_tokens, window, scale_log2, expand ? *expand : pa::la::Expand{}};
   if (expand && (fp32 || simple || Rp != pa::la::X_RANK || rp != pa::la::X_ROT || H > 256)) return -1;
   const int RT = Rp / 32, PT = rp / 32;
+  int per = 1;  // columns of a workgroup of merge_heads_kernel: as leave about one a CU
+  while (per < 16 && (long long)T * H > 256ll * per) per *= 2;
+  if (uv && (fp32 || simple || expand || PT > 2 || Rp > 512 || pa_latent_pad(Rp) != Rp || vp < 16 || vp > 128 || vp % 16 || ldy % 4 ||
+             T <= 0)) return -1;
   if (!fp32 && !simple && PT <= 2) {
 #define PA_LAX(R, P, ...)                                                                                     \
   do {                                                                                                        \
@@ -1316,7 +1454,9 @@ extern "C" int pa_latent_attention(int fp32, void* out, float* part_o, float* pa
     /* items are strided over the grid: at least one workgroup per CU */                                      \
     const int gy = R >= pa::la::PAIRS || max_items < 256 ? 256 : (max_items < 4096 ? max_items : 4096);       \
     hipLaunchKernelGGL((pa::la::mfma_kernel<R, P, CT __VA_ARGS__>), dim3(gx, gy), dim3(64 * pa::la::NW), lds, st, A);     \
-    hipLaunchKernelGGL((pa::la::merge_kernel<R __VA_ARGS__>), dim3(16, std::min(gy, 256)), dim3(256), 0, st, A);           \
+    if (uv) hipLaunchKernelGGL((pa::la::merge_heads_kernel<R>), dim3(H, (T + per - 1) / per), dim3(64 * pa::la::MH_WAVES), 0, st, A, \
+                               (const pa::bf16*)uv, (pa::bf16*)y, ldy, vp, max_items, per);                    \
+    else hipLaunchKernelGGL((pa::la::merge_kernel<R __VA_ARGS__>), dim3(16, std::min(gy, 256)), dim3(256), 0, st, A);      \
     return (int)hipGetLastError();                                                                            \
   } while (0)
 #define PA_LA(R, P) PA_LAX(R, P, )

@@ -155,8 +155,11 @@ class LatentAttention:
         ops.head_gemm(q, self.np + self.rp, self.uk, qa.view(T, -1), self.D,
                       rot=(meta.positions, self.cos_sin, self.np, m.rot_dim, self.rp) if m.rot_dim else None, skip=skip)
         oc = new(T, H, self.Rp)
+        merged = plan is None and not m.gate and ops.merge_heads(T, self.Rp, self.rp, self.vp, self.dtype)
         ops.latent_attention(oc, room.part_o, room.part_ml, qa, pages, meta.items, meta.n_items, meta.q_start,
                              meta.q_len, meta.ctx_len, meta.block_table, m.scale, m.window, room.dec_tokens, room.tile_tokens,
-                             num_seqs=meta.num_seqs, expand=ex)
+                             num_seqs=meta.num_seqs, expand=ex, heads=(self.uv, out) if merged else None)
+        if merged:
+            return
         ops.head_gemm(oc.view(T, -1), self.Rp, self.uv, out, self.vp, gate=x[:, self.g_col:] if m.gate else None,
                       skip=skip)

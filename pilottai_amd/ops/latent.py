@@ -64,22 +64,37 @@ def latent_cache(x, nq: int, R: int, r: int, w_q, w_c, cq, pages, Rp: int, posit
 
 def latent_attention(out, part_o, part_ml, q, pages, items, n_items, q_start, q_len, ctx_len, block_table,
                      scale: float, window: int, dec_tokens: int, tile_tokens: int, num_seqs: Optional[int] = None,
-                     simple: bool = False, expand: Optional["Expanded"] = None):
+                     simple: bool = False, expand: Optional["Expanded"] = None, heads: Optional[tuple] = None):
     """Attention of absorbed queries q [T, H, D] over latent pages -> out [T, H, Rp]; `window` 0: none.
     dec_tokens / tile_tokens: the scheduler's items hold at most dec_tokens tokens (split over keys) or
     tile_tokens (csrc/ops/latent_attention.hip). `simple`: the any-size kernel. `expand`: requests of its plan are left out
-    here, and their outputs in the heads' own dimensions go to its `out`."""
+    here, and their outputs in the heads' own dimensions go to its `out`. `heads` = (W_uv packed by pack_groups, y): y = every head's
+    product with W_uv, as head_gemm(out, Rp, W_uv, y, vp) behind this; `out` then holds anything (merge_heads: which sizes)."""
     if expand and expand.window != window:
         raise ValueError(f"a plan for a window of {expand.window} with one of {window}")
     if _on_gpu(q):
         require_latent().latent_attention(out, part_o, part_ml, q, pages, items, n_items, q_start, q_len,
                                           ctx_len, block_table, int(dec_tokens), int(tile_tokens), int(window),
                                           float(scale), bool(simple), expand.plan if expand else [],
-                                          expand.tensors() if expand else [], *(expand.sizes if expand else (0, 0)))
+                                          expand.tensors() if expand else [], *(expand.sizes if expand else (0, 0)),
+                                          *(heads or (None, None)))
     else:
         ref.latent_attention(out, q, pages, q_start, q_len, ctx_len, block_table, scale, window,
                              len(q_len) if num_seqs is None else num_seqs)
+        if heads:
+            head_gemm(out.view(out.shape[0], -1), out.shape[2], heads[0], heads[1], heads[0].shape[1] * 16 if heads[0].dim() == 5 else heads[0].shape[1])
     return out
+
+
+# Tokens of a step up to which the heads' products go with the merge. A step of bozupel-base, us apart and so: 128 decoding rows 2,290, 2,272, 256
+# 2,572, 2,552, one prompt of 60 tokens 2,020, 2,018, of 120 2,199, 2,200, four of 60 2,445, 2,452
+MERGE_HEADS_T = 192
+
+
+def merge_heads(T: int, rank: int, rot: int, vdim: int, dtype) -> bool:
+    """Whether latent_attention's `heads` is the faster form for T tokens, and has these (padded) sizes."""
+    return T <= MERGE_HEADS_T and dtype == torch.bfloat16 and rank <= 512 and \
+        latent_pad(rank) == rank and rot <= 64 and vdim <= 128 and vdim % 16 == 0
 
 
 # Prompt portions with the keys expanded per head (csrc/ops/latent_expand.h): sizes that have the form, and the most heads (an

@@ -386,6 +386,38 @@ def test_latent_attention_split_tiles(gpu, H, R, r, window):
     run_attention(gpu, torch.bfloat16, H, R, r, [(1500, tile + 1), (900, 2 * tile + 16 // min(H, 16))], window, tiles=64, part=256)
 
 
+MERGED = {"one": [(2000, 1)], "two": [(1500, 1), (700, 1)], "rows": [(60 * i, 1) for i in range(15)], "portions": [(1500, 9), (3, 1), (700, 20), (0, 3)]}
+
+
+@pytest.mark.parametrize("step", list(MERGED))  # 1, 2 and more columns of 16 items, of one and several partitions; tokens of an item
+@pytest.mark.parametrize("H,R,r,vp", [(16, 512, 64, 128), (20, 256, 32, 80), (3, 96, 24, 16), (40, 192, 64, 64)])
+def test_merged_heads(gpu, H, R, r, vp, step):
+    """The heads' products behind the merge: of rows whose bf16 roundings may fall differently, sums of Rp products in fp32."""
+    from pilottai_amd import ops
+    from pilottai_amd.ops.latent import latent_pad, pad_to
+
+    g = torch.Generator(device=gpu).manual_seed(H + vp)
+    rnd = lambda *s: torch.randn(*s, device=gpu, generator=g).bfloat16()  # noqa: E731
+    Rp, rp = latent_pad(R), pad_to(r, 32)
+    T, m, dec, tile = fed_meta(gpu, H, MERGED[step], 64, 0, tiles=64, part=256)
+    NB, mi, D = (dec * H + 15) // 16, m["items"].shape[0], Rp + rp
+    q, pages, uv = rnd(T, H, D), rnd(600, D // 8, 16, 8), rnd(H, vp, Rp) / Rp ** 0.5
+    m = {k: v.to(gpu) for k, v in m.items()}
+    f32 = lambda n: torch.empty(n, dtype=torch.float32, device=gpu)  # noqa: E731
+
+    def run(**kw):
+        out = torch.full((T, H, Rp), 9.0, dtype=torch.bfloat16, device=gpu)
+        ops.latent_attention(out, f32(mi * NB * 16 * Rp), f32(mi * NB * 32), q, pages, m["items"], m["n_items"], m["q_start"], m["q_len"],
+                             m["ctx_len"], m["block_table"], D ** -0.5, 0, dec, tile, **kw)
+        return out
+    y = torch.full((T, H * vp + 8), 7.0, dtype=torch.bfloat16, device=gpu)
+    run(heads=(ops.pack_groups(uv, torch.bfloat16), y[:, :H * vp]))
+    o, w = run().float(), uv.float()
+    want, size = torch.einsum("thk,hvk->thv", o, w), torch.einsum("thk,hvk->thv", o.abs(), w.abs())
+    err = (y[:, :H * vp].float().view(T, H, vp) - want).abs()
+    assert bool((err <= 2.0 ** -8 * want.abs() + (2.0 ** -8 + Rp * 2.0 ** -24) * size).all()) and bool((y[:, H * vp:] == 7.0).all())
+
+
 @pytest.mark.parametrize("R,r", [(256, 32), (512, 64)])
 def test_latent_attention_item_rounds(gpu, R, r):
     """More items than workgroups, a round that is not full, decode rows among them."""
