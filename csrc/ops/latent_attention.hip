@@ -1044,21 +1044,22 @@ __device__ __forceinline__ void expanded_unit(const Args& A, const int4 it, int 
 // they fill less than half of the columns of more than two tiles: 10 of 50 after 150 beside 200 decode rows 3,292 us refused,
 // 3,407 expanded; 60 of 12 after 60 3,033, 3,370; 7 of 72 after 150 beside 30 2,912, 2,800. And none where they are less than twice
 // the tokens of the other requests, whose items wait for the units: 2 of 140 after 600 beside 230 rows of 1,500 keys 3,409, 3,464; 4
-// of 132 after 700 beside 200 of 1,000 3,615, 3,605. Tiles whose keys are more than a workgroup's average are split.
+// of 132 after 700 beside 200 of 1,000 3,615, 3,605. Tiles whose keys are more than a workgroup's average are split. Rows behind the last request's are nobody's
+// and left out like the expanded: 13 of 512 had the head products walk their whole inputs, W_uv's 11.9 us and W_uk's 7.4, 4.7 and 5.2 without (3,007 -> 2,885 a step of 8 layers).
 constexpr int X_MIN = 12;
 __global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const int* __restrict__ q_start,
                                                            const int* __restrict__ q_len, const int* __restrict__ ctx_len, int S,
                                                            int T, int H, int window, int room, int max_att, int max_tiles, int slots) {
   static_assert(X_REQS == 64, "a lane a request");
-  __shared__ int ws[16], others[16], req[X_REQS], qs[X_REQS], ql[X_REQS], cl[X_REQS], to[X_REQS], tiles[X_REQS];
+  __shared__ int ws[16], others[16], tops[16], req[X_REQS], qs[X_REQS], ql[X_REQS], cl[X_REQS], to[X_REQS], tiles[X_REQS];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  for (int t = threadIdx.x; t < T; t += 1024) X.form[t] = 0;
-  int found = 0, rest = 0;
+  int found = 0, rest = 0, top = 0;
   for (int s0 = 0; s0 < S; s0 += 1024) {
     const int s = s0 + threadIdx.x, n = s < S ? q_len[s] : 0;
     const bool yes = n >= X_MIN && s < S && q_start[s] + n <= T;
     if (s < S) X.base[s] = X_NONE;
     if (!yes) rest += n;
+    if (n > 0) top = max(top, q_start[s] + n);
     const unsigned long long b = __ballot(yes);
     if (lane == 0) ws[wid] = __popcll(b);
     __syncthreads();
@@ -1076,11 +1077,21 @@ __global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const
     __syncthreads();
   }
 #pragma unroll
-  for (int o = 1; o < 64; o <<= 1) rest += __shfl_xor(rest, o, 64);
-  if (lane == 0) others[wid] = rest;
+  for (int o = 1; o < 64; o <<= 1) {
+    rest += __shfl_xor(rest, o, 64);
+    top = max(top, __shfl_xor(top, o, 64));
+  }
+  if (lane == 0) {
+    others[wid] = rest;
+    tops[wid] = top;
+  }
   __syncthreads();
   rest = 0;
-  for (int w = 0; w < 16; ++w) rest += others[w];
+  for (int w = 0; w < 16; ++w) {
+    rest += others[w];
+    top = max(top, tops[w]);
+  }
+  for (int t = threadIdx.x; t < T; t += 1024) X.form[t] = t >= top;
   // every wave works out all of this, a request a lane
   int n = found <= X_REQS ? found : 0, lo = 0, hi, blocks = 0, nt = 0, total = 0, cols = 0, tokens = 0;
   if (lane < n) {

@@ -557,8 +557,8 @@ def test_latent_attention_expanded(gpu, H, step, window):
         torch.testing.assert_close(o[q0:q0 + k], want, **tol(bf), msg=lambda s, i=i: f"request {i} {reqs[i]}: {s}")
 
 
-def plan_of(gpu, reqs, H, window):
-    """(the plan of a step of [(cached, new)], its rows)."""
+def plan_of(gpu, reqs, H, window, rest=0):
+    """(the plan of a step of [(cached, new)] and `rest` rows of no request, its rows)."""
     from types import SimpleNamespace
 
     from pilottai_amd.ops.latent import ExpandPlan
@@ -566,7 +566,7 @@ def plan_of(gpu, reqs, H, window):
     new = torch.tensor([n for _, n in reqs] + [0] * 3, dtype=torch.int32)  # (slots without a request)
     meta = SimpleNamespace(q_len=new.to(gpu), q_start=(new.cumsum(0) - new).to(torch.int32).to(gpu),
                            ctx_len=torch.tensor([c + n for c, n in reqs] + [0] * 3, dtype=torch.int32, device=gpu))
-    T = int(new.sum())
+    T = int(new.sum()) + rest
     return ExpandPlan(meta, T, H, window), T
 
 
@@ -607,6 +607,15 @@ def test_expand_plan_takes_all_prompts_or_none(gpu, H, window, reqs, taken):
     assert all(v == list(range(k[2])) for k, v in parts.items())
     used = [slot + p for i, t, n, slot in parts for p in range(n) if n > 1]
     assert used == list(range(len(used))) and len(used) <= plan.slots
+
+
+@pytest.mark.parametrize("reqs", [[(0, 40)], [(9, 1), (3, 1020)], [(900, 11), (3, 1)]])  # taken, beside a decoding row, refused
+@pytest.mark.parametrize("rest", [1, 13, 1100])
+def test_rows_behind_the_last_request_are_left_out(gpu, reqs, rest):
+    """A captured step's rows that no request has: the head products leave them out, whatever the plan takes."""
+    plan, T = plan_of(gpu, reqs, 16, 0, rest)
+    held = [int(n >= 12) for _, n in reqs for _ in range(n)]
+    assert plan.form.tolist() == held + [1] * rest and T == len(held) + rest
 
 
 @pytest.mark.parametrize("T,G", [(9, 3), (70, 5), (300, 9), (2100, 16)])  # tiles of 16 and of 64 rows, rows through LDS
