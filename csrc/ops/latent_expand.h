@@ -14,6 +14,7 @@ namespace la {
 
 constexpr int X_DIM = 128, X_ROT = 64, X_RANK = 512;  // sizes that have this form
 constexpr int X_COLS = 128;                           // tokens of an attention unit
+constexpr int X_PARTS = 8;                            // parts of a unit's keys, at most
 constexpr int X_REQS = 64;                            // requests of a step that may take it
 constexpr int X_NONE = -(1 << 30);
 
@@ -21,7 +22,7 @@ constexpr int X_NONE = -(1 << 30);
 struct Expand {
   int* counts;  // attention items, expansion tiles
   int* base;    // [S] workspace block of the request's key block 0 (blocks before its window have none), or X_NONE
-  int* form;    // [T] 1: the row belongs to an expanded request, or to none
+  int* form;    // [T] 1: the row belongs to an expanded request, or to none, or to none
   int4* att;    // {request, tile of X_COLS tokens, part | parts << 16, partial slot}
   int4* tiles;  // {request, first key block, blocks, workspace block}
   void *kx, *kr;
