@@ -1171,84 +1171,98 @@ __global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const
   }
 }
 
-// Keys and values of the heads: 64 keys' latents in LDS, as the pages hold them, times W_uk,h and W_uv,h, the 256 outputs of a
-// head a round; a wave 64 of them. The outputs' lanes hold 4 dims of a key: 512 bytes of the workspace a store. A
-// head pair's weights (512 KB) stay on one XCD. Bound by the weights' way from L2, a step of 64 x 64 outputs 4 KB a wave: 4,096
-// keys of 16 heads 25 us (17 GFLOP, 34 MB written), with the next step's weights alone in flight and keys held over heads 90.
-__global__ __launch_bounds__(256, 2) void expand_kernel(const Expand X, const bf16* __restrict__ pages, const bf16* __restrict__ wk,
-                                                        const bf16* __restrict__ wv, const int* __restrict__ block_table, int max_blocks, int H, int D, int per) {
-  extern __shared__ __attribute__((aligned(16))) char smem[];  // [4][X_RANK / 32][1 KB]
-  constexpr int KS = X_RANK / 32, NT = 4, RING = 4;
+// Keys and values of the heads: the latents of a block of 16 keys, as the pages hold them, times W_uk,h and W_uv,h. A workgroup keeps the
+// weights of one head (256 KB) in registers, 32 of the 256 outputs a wave, and takes its share of the blocks through LDS, X_AHEAD ahead by
+// direct loads; the outputs' lanes hold 4 dims of a key: 512 bytes of the workspace a store. 4,096 keys of 16 heads 23 us (17 GFLOP, 34 MB
+// written): the products take 14 behind 5 of weights on their way, the stores 4 more (stores of 1 KB as long; four waves of 64 outputs, which
+// read half as much LDS, 25; XCDs of 4 or 16 heads 23 and 26). With two heads' weights streamed from L2 past a workgroup's 64 keys, two
+// workgroups a CU, arrival, products and stores came one after the other. us so -> now: 100 keys 11.0 -> 5.3, 512 11.6 -> 6.9,
+// 1,000 12.5 -> 9.1, 2,000 15.6 -> 14.3, 3,000 23.0 -> 18.9, 4,096 27.6 -> 23.1; 5 heads 4,096 13.7 -> 12.2, 40 heads 512 13.6 -> 11.2, 4,096 60.5 -> 46.0.
+constexpr int X_AHEAD = 6, X_RING = 8;  // blocks
+__global__ __launch_bounds__(512, 2) void expand_kernel(const Expand X, const bf16* __restrict__ pages, const bf16* __restrict__ wk,
+                                                        const bf16* __restrict__ wv, const int* __restrict__ block_table, int max_blocks, int H, int D,
+                                                        int shares) {
+  extern __shared__ __attribute__((aligned(16))) char smem[];  // [X_RING][X_RANK / 32][1 KB]
+  constexpr int KS = X_RANK / 32, NT = 2, P = X_AHEAD, EARLY = 6;
+  static_assert(P < X_RING, "a block arrives where nobody reads");
   const int lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), g = lane >> 4, c = lane & 15;
-  const int groups = H / per, n = X.counts[1] * groups;
-  for (int u = blockIdx.x; u < n; u += gridDim.x) {
-    const int4 tl = X.tiles[u / groups];
-    const int h0 = u % groups * per;
-    const int* bt = block_table + (size_t)tl.x * max_blocks + tl.y;
-    __syncthreads();  // (the last unit's reads)
-    int ids[4];
+  const int h = blockIdx.x % H, n = 4 * X.counts[1], per = (n + shares - 1) / shares, i0 = blockIdx.x / H * per, i1 = min(n, i0 + per);
+  if (i0 >= i1) return;
+  // a block a lane, 64 from c0 on: its page and its place in the workspace (of a tile's missing blocks: those of its last one)
+  int id, to;
+  auto places = [&](int c0) {
+    const int e = min(c0 + lane, i1 - 1);
+    const int4 tl = X.tiles[e >> 2];
+    const int b = min(e & 3, tl.z - 1);
+    to = tl.w + b;
+    id = block_table[(size_t)tl.x * max_blocks + tl.y + b];
+  };
+  places(i0);
+  asm volatile("" ::"v"(id) : "memory");  // (before the weights are under way, which a later wait would be for too)
+  const int t16 = wid * NT;  // the wave's first tile of the head's 8 of keys and 8 of values
+  const bf16* wp = (t16 < 8 ? wk : wv) + ((size_t)h * 8 + (t16 & 7)) * (KS * 512) + lane * 8;
+  bf16x8 a[KS][NT];
 #pragma unroll
-    for (int b = 0; b < 4; ++b) ids[b] = bt[min(b, tl.z - 1)];
+  for (int s = 0; s < KS; ++s)
 #pragma unroll
-    for (int b = 0; b < 4; ++b)
+    for (int i = 0; i < NT; ++i) a[s][i] = *reinterpret_cast<const bf16x8*>(wp + (size_t)(i * KS + s) * 512);
+  for (int c0 = i0; c0 < i1; c0 += 64) {
+    const int m = min(64, i1 - c0);
+    if (c0 > i0) places(c0);
+    auto issue = [&](int i) {  // (past the end: the last block again, so that the waits stay counted)
+      const bf16* src = pages + (size_t)__builtin_amdgcn_readlane(id, min(i, m - 1)) * (D * 16) + wid * 512 + lane * 8;
+      char* dst = smem + (i % X_RING) * (KS * 1024) + wid * 1024;
 #pragma unroll
-      for (int i = 0; i < KS / 4; ++i) {
-        const int m = i * 4 + wid;
-        __builtin_amdgcn_global_load_lds((glb_void*)(pages + (size_t)ids[b] * (D * 16) + m * 512 + lane * 8),
-                                         (lds_void*)(smem + (b * KS + m) * 1024), 16, 0, 0);
+      for (int j = 0; j < KS / 8; ++j)
+        __builtin_amdgcn_global_load_lds((glb_void*)(src + j * 4096), (lds_void*)(dst + j * 8192), 16, 0, 0);
+    };
+    for (int i = 0; i < P; ++i) issue(i);
+    for (int i = 0; i < m; ++i) {
+      // this wave's two loads of block i have arrived: behind them the loads of P - 1 blocks are under way and, once they
+      // are P blocks old, two stores of each of the last P too
+      asm volatile("" ::: "memory");
+      __builtin_amdgcn_sched_barrier(0);
+      if (i < P) __builtin_amdgcn_s_waitcnt(0x0F70 | (2 * P - 2));
+      else __builtin_amdgcn_s_waitcnt(0x0F70 | ((4 * P - 2) & 15) | (4 * P - 2) >> 4 << 14);
+      __builtin_amdgcn_s_barrier();  // block i is whole, and nobody reads block i - 1 any more
+      asm volatile("" ::: "memory");
+      issue(i + P);
+      __builtin_amdgcn_sched_barrier(0);
+      const char* from = smem + (i % X_RING) * (KS * 1024) + lane * 16;
+      f32x4 acc[NT];
+#pragma unroll
+      for (int j = 0; j < NT; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      bf16x8 k[EARLY];  // (left to itself the compiler waits for each pair)
+#pragma unroll
+      for (int s = 0; s < EARLY; ++s) k[s] = *reinterpret_cast<const bf16x8*>(from + s * 1024);
+#pragma unroll
+      for (int s = 0; s < KS; ++s) {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int j = 0; j < NT; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[s][j], k[s % EARLY], acc[j], 0, 0, 0);
+        if (s + EARLY < KS) k[s % EARLY] = *reinterpret_cast<const bf16x8*>(from + (s + EARLY) * 1024);
       }
-    if (h0 == 0 && wid < tl.z) {  // the rotated part, a block a wave
-      const bf16x8* src = reinterpret_cast<const bf16x8*>(pages + (size_t)bt[wid] * (D * 16) + X_RANK * 16) + lane;
-      bf16x8* dst = reinterpret_cast<bf16x8*>((bf16*)X.kr + (size_t)(tl.w + wid) * (X_ROT * 16)) + lane;
+      bf16* dst = (bf16*)X.kx + ((size_t)__builtin_amdgcn_readlane(to, i) * H + h) * (X_DIM * 32) + (2 * t16 + (g >> 1)) * 128 + c * 8 + (g & 1) * 4;
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int j = 0; j < NT; ++j) {
+        bf16x4 v;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = (bf16)acc[j][r];
+        *reinterpret_cast<bf16x4*>(dst + j * 256) = v;
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    // the rotated parts, a block a wave, shared out over the heads
+    for (int i = wid; i < m; i += 8) {
+      if ((c0 + i) % H != h) continue;
+      const bf16x8* src = reinterpret_cast<const bf16x8*>(pages + (size_t)__builtin_amdgcn_readlane(id, i) * (D * 16) + X_RANK * 16) + lane;
+      bf16x8* dst = reinterpret_cast<bf16x8*>((bf16*)X.kr + (size_t)__builtin_amdgcn_readlane(to, i) * (X_ROT * 16)) + lane;
       dst[0] = src[0];
       dst[64] = src[64];
     }
-    // the weights of all `per` heads are one stream, loaded RING steps ahead
-    const bf16* wp = (wid < 2 ? wk : wv) + ((size_t)h0 * 8 + (wid & 1) * NT) * (KS * 512) + lane * 8;
-    bf16x8 a[RING][NT];
-    auto load = [&](int q, bf16x8 (&a)[NT]) {  // (past the end: the last step's again)
-      q = min(q, per * KS - 1);
-      const bf16* from = wp + ((size_t)(q / KS) * 8 * KS + q % KS) * 512;
-#pragma unroll
-      for (int i = 0; i < NT; ++i) a[i] = *reinterpret_cast<const bf16x8*>(from + i * (KS * 512));
-    };
-#pragma unroll
-    for (int d = 0; d < RING; ++d) load(d, a[d]);
-    __syncthreads();  // (waits for the loads to LDS)
-    for (int j = 0; j < per; ++j) {
-      f32x4 acc[4][NT];
-#pragma unroll
-      for (int b = 0; b < 4; ++b)
-#pragma unroll
-        for (int i = 0; i < NT; ++i) acc[b][i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 1
-      for (int s = 0; s < KS; s += RING)
-#pragma unroll
-        for (int d = 0; d < RING; ++d) {
-          bf16x8 k[4];
-#pragma unroll
-          for (int b = 0; b < 4; ++b) k[b] = *reinterpret_cast<const bf16x8*>(smem + (b * KS + s + d) * 1024 + lane * 16);
-#pragma unroll
-          for (int b = 0; b < 4; ++b)
-#pragma unroll
-            for (int i = 0; i < NT; ++i) acc[b][i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[d][i], k[b], acc[b][i], 0, 0, 0);
-          __builtin_amdgcn_sched_barrier(0);
-          load(j * KS + s + d + RING, a[d]);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        if (b >= tl.z) break;
-        bf16* dst = (bf16*)X.kx + ((size_t)(tl.w + b) * H + h0 + j) * (X_DIM * 32) + (2 * NT * wid + (g >> 1)) * 128 + c * 8 + (g & 1) * 4;
-#pragma unroll
-        for (int i = 0; i < NT; ++i) {
-          bf16x4 v;
-#pragma unroll
-          for (int r = 0; r < 4; ++r) v[r] = (bf16)acc[b][i][r];
-          *reinterpret_cast<bf16x4*>(dst + i * 256) = v;
-        }
-      }
-    }
+    __builtin_amdgcn_s_waitcnt(0x0070);  // every load to LDS has arrived, before others come or the workgroup ends
+    __syncthreads();
   }
 }
 
@@ -1526,15 +1540,14 @@ extern "C" int pa_latent_plan(const pa::la::Expand* X, const int* q_start, const
 extern "C" int pa_latent_expand(const pa::la::Expand* X, const void* pages, const void* wk, const void* wv, const int* block_table, int max_blocks,
                                 int H, int D, int max_tiles, hipStream_t st) {
   if (H <= 0 || D != pa::la::X_RANK + pa::la::X_ROT) return -1;
-  constexpr int lds = 4 * pa::la::X_RANK * 32;
+  constexpr int lds = pa::la::X_RING * pa::la::X_RANK * 32;
   static bool attr = false;
   if (!attr) {
     (void)hipFuncSetAttribute((const void*)pa::la::expand_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, lds);
     attr = true;
   }
-  const int per = H % 2 ? 1 : 2, groups = H / per, n = max_tiles * groups;  // two workgroups a CU
-  const int grid = groups <= 512 ? std::min(n, 512 / groups * groups) : n;
-  hipLaunchKernelGGL(pa::la::expand_kernel, dim3(grid), dim3(256), lds, st, *X, (const pa::bf16*)pages, (const pa::bf16*)wk,
-                     (const pa::bf16*)wv, block_table, max_blocks, H, D, per);
+  const int shares = std::min(4 * max_tiles, std::max(1, 256 / H));  // one workgroup a CU
+  hipLaunchKernelGGL(pa::la::expand_kernel, dim3(H * shares), dim3(512), lds, st, *X, (const pa::bf16*)pages, (const pa::bf16*)wk,
+                     (const pa::bf16*)wv, block_table, max_blocks, H, D, shares);
   return (int)hipGetLastError();
 }

@@ -609,6 +609,36 @@ def test_expand_plan_takes_all_prompts_or_none(gpu, H, window, reqs, taken):
     assert used == list(range(len(used))) and len(used) <= plan.slots
 
 
+@pytest.mark.parametrize("H,reqs", [(130, [(0, 2100), (3, 20)]), (16, [(0, 17)]), (1, [(40, 4050)]), (5, [(0, 64), (70, 140)])])
+def test_expanded_keys_and_values(gpu, H, reqs):
+    """Every block of the plan's requests, whether a workgroup has none, one or more than 64 of them: products of 512 terms added
+    up in fp32 and rounded to bf16, the rotated part as it is."""
+    from pilottai_amd import ops
+    from pilottai_amd.ops.latent import Expanded
+
+    plan, T = plan_of(gpu, reqs, H, 0)
+    g, bf, R = torch.Generator().manual_seed(H), torch.bfloat16, 512
+    blocks = [(c + n + 15) // 16 for c, n in reqs]
+    pages = torch.randn(sum(blocks) + 3, 72, 16, 8, generator=g).to(bf)
+    table, ids = torch.zeros(len(reqs) + 3, max(blocks), dtype=torch.int32), torch.randperm(sum(blocks) + 3, generator=g).int()
+    for i, n in enumerate(blocks):
+        table[i, :n] = ids[sum(blocks[:i]):][:n]
+    w = [(torch.randn(H, 128, R, generator=g) * R ** -0.5).to(bf) for _ in range(2)]
+    ex = Expanded(plan, pages.to(gpu), *(ops.pack_groups(x.to(gpu), bf) for x in w), table.to(gpu),
+                  torch.zeros(T, H * 192, dtype=bf, device=gpu), ops.angle_table(4608, 64, 1e4).to(gpu),
+                  torch.zeros(T, H * 128, dtype=bf, device=gpu))
+    base, kx, kr = plan.lists[1].tolist(), ex.kx.cpu(), ex.kr.cpu()
+    both = torch.cat(w, 1).float()
+    for i, n in enumerate(blocks):
+        for b in range(n):
+            page = pages[int(table[i, b])]
+            assert torch.equal(kr[base[i] + b], page[R // 8:])
+            x = page[:R // 8].permute(1, 0, 2).reshape(16, R).float()
+            want, slack = both @ x.T, R * 2.0 ** -24 * (both.abs() @ x.abs().T)  # [H, 256, 16]
+            got = kx[base[i] + b].float().permute(0, 1, 3, 2).reshape(H, 256, 16)
+            assert bool(((got - want).abs() <= 2.0 ** -8 * want.abs() + 2 * slack).all()), (i, b)
+
+
 @pytest.mark.parametrize("reqs", [[(0, 40)], [(9, 1), (3, 1020)], [(900, 11), (3, 1)]])  # taken, beside a decoding row, refused
 @pytest.mark.parametrize("rest", [1, 13, 1100])
 def test_rows_behind_the_last_request_are_left_out(gpu, reqs, rest):
