@@ -64,7 +64,7 @@ int pa_stream_gemm(void* y, const void* x, const void* wp, const void* resid, fl
                    void* k_cache, void* v_cache, const int* positions, const int* slots, const float* cos_sin, int H,
                    int KV, int rel, unsigned long long* stamps, hipStream_t st);
 void pa_prefill_gemm_plan(int M, int N, int K, int bn, int* full, int* S);
-int pa_prefill_pick_bn(int M, int N);
+int pa_prefill_pick_bn(int M, int N, int K);
 void pa_prefill_set_variant(int v);
 long long pa_prefill_gemm_ws_floats(int M, int N, int bn, int full, int S);
 long long pa_cosine_topk_workspace_bytes(int Q, int N, int K);
@@ -487,7 +487,7 @@ bool prefill_qkv_rope(at::Tensor x, at::Tensor wp, at::Tensor ss_in, double eps,
 
 std::vector<int64_t> prefill_gemm_plan(int64_t M, int64_t N, int64_t K, int64_t bn) {
   int full, S;
-  if (bn <= 0) bn = pa_prefill_pick_bn((int)M, (int)N);
+  if (bn <= 0) bn = pa_prefill_pick_bn((int)M, (int)N, (int)K);
   pa_prefill_gemm_plan((int)M, (int)N, (int)K, (int)bn, &full, &S);
   return {full, S, pa_prefill_gemm_ws_floats((int)M, (int)N, (int)bn, full, S), bn};
 }

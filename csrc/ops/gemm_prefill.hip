@@ -571,12 +571,38 @@ static int block_rows(int MT, int tiles, int bn) {
   return (MT + blocks - 1) / blocks;
 }
 
-// Tile width when the caller leaves it open: 256 x 128 tiles for the narrow projections
-// (N <= 6,144: qkv / o / down of Llama-3-8B, 0.6-0.85x the 256-wide kernel's time at
-// M <= 1,024), 256 x 256 for wide ones (gate_up: 1.08x faster).
-static int pick_bn(int M, int N) {
-  (void)M;
-  return (N % 256 || N <= 6144) ? 128 : 256;
+// Tile width when the caller leaves it open: what a launch takes, in rounds of one 256 x 128 tile a CU. Tiles of 192 and of 256
+// columns take 1.32 and 1.63 of its time (K 2048: 32.5, 43, 53 us a full round), so a wider one is ahead where it saves a round
+// and behind where one round holds narrower ones; a round that is not full takes 0.6 of its time and 0.4 by its tiles.
+// The line by N (128 columns up to 6,144) stays where the estimate is less than 5 % better, and where either launch has tiles in slices of
+// k: whole tiles add up in the same order whatever their width, so that a step keeps its bits, where a recurrent layer's step sizes
+// make another order's last bits 0.7 to 1.1 of a logit's root mean square. us, by N -> so, rows, outputs, inputs: 4,096 x 3072 x
+// 768 28.7 -> 23.0, x 4096 x 2048 64 -> 53, 2,048 x 4608 x 1024 32.3 -> 23.6, 1,024 x 10752 x 2048 46.3 -> 40.6.
+static double rounds_cost(int tiles) {
+  const int rem = tiles % 256;
+  return tiles / 256 + (rem ? 0.6 + 0.4 / 256 * rem : 0.);
+}
+constexpr double SLICED = 1e30;
+static double width_cost(int M, int N, int K, int bn) {
+  const int MT = (M + 255) / 256, NT = N / bn, tiles = MT * NT, wide = tiles / 256 * 256 / MT, rest = 2 * MT * (NT - wide);
+  if (bn == 256 && tiles % 256 && wide && rest <= 256) return 1.63 / 256 * wide * MT + rounds_cost(rest);  // (pingpong_mixed_kernel)
+  int full, S;
+  plan_default(M, N, K, bn, full, S);
+  return S > 1 ? SLICED : (bn == 128 ? 1. : bn == 192 ? 1.32 : 1.63) * rounds_cost(tiles);
+}
+static int pick_bn(int M, int N, int K, int variant, bool default_plan) {
+  const int bn = (N % 256 || N <= 6144) ? 128 : 256;
+  // (the other families and a caller's slices keep the line by N: they have no tiles of 192 columns)
+  if (N % 128 || K < 128 || variant < 3 || !default_plan) return bn;
+  const double old = width_cost(M, N, K, bn);
+  int best = bn;
+  double least = 0.95 * old;
+  for (int w : {128, 192, 256})
+    if (w != bn && N % w == 0 && old < SLICED && width_cost(M, N, K, w) < least) {
+      best = w;
+      least = width_cost(M, N, K, w);
+    }
+  return best;
 }
 
 }  // namespace pf
@@ -584,15 +610,13 @@ static int pick_bn(int M, int N) {
 
 extern "C" void pa_prefill_set_variant(int v) { pa::pf::g_pf_variant = v < 0 ? pa::pf::kPfDefaultVariant : v; }
 
-extern "C" int pa_prefill_pick_bn(int M, int N) { return pa::pf::pick_bn(M, N); }
+extern "C" int pa_prefill_pick_bn(int M, int N, int K) { return pa::pf::pick_bn(M, N, K, pa::pf::g_pf_variant, true); }
 
 extern "C" void pa_prefill_gemm_plan(int M, int N, int K, int bn, int* full, int* S) {
-  if (bn <= 0) bn = pa::pf::pick_bn(M, N);
   pa::pf::plan_default(M, N, K, bn, *full, *S);
 }
 
 extern "C" long long pa_prefill_gemm_ws_floats(int M, int N, int bn, int full, int S) {
-  if (bn <= 0) bn = pa::pf::pick_bn(M, N);
   const long long tiles = (long long)((M + 255) / 256) * (N / bn);
   return S > 1 ? (tiles - full) * S * (long long)(256 * bn) : 0;
 }
@@ -610,7 +634,7 @@ extern "C" int pa_prefill_gemm(void* y, const void* x, const void* wp, const voi
                                int kernel_variant, const int* live, hipStream_t st) {
   using namespace pa::pf;
   if (M <= 0) return 0;
-  if (bn <= 0) bn = pick_bn(M, N);
+  if (bn <= 0) bn = pick_bn(M, N, K, kernel_variant >= 0 ? kernel_variant : g_pf_variant, full < 0 && splits <= 0);
   if (bn != 128 && bn != 192 && bn != 256) return 1;
   if (K % 64 != 0 || N % bn != 0 || epi < 0 || epi > 4 || ldx % 8 != 0) return 1;
   const int norm = ss_in != nullptr;

@@ -86,6 +86,24 @@ def test_prefill_gemm_192_refuses_other_widths(gpu):
         ops.prefill_gemm(x, wp, "plain", bn=192)
 
 
+@pytest.mark.parametrize("M,N,K,bn", [
+    (2817, 3072, 128, 192), (2816, 3072, 768, 192), (2560, 3072, 768, 128), (2561, 4096, 192, 256), (4096, 4096, 512, 256), (2304, 4096, 1024, 128),
+    (2048, 4096, 256, 128), (500, 10752, 256, 128), (1000, 10752, 1024, 192), (500, 10752, 1024, 256), (1500, 10752, 256, 256),
+    (2900, 1920, 128, 128), (2900, 3072, 64, 128)])
+def test_prefill_gemm_default_width(gpu, M, N, K, bn):
+    """The width that a call leaves open follows the rounds of its tiles, on both sides of the lines, and changes no bits; launches with slices of k
+    and the kernels of fewer than two k-tiles keep the line by N."""
+    from pilottai_amd.ops import kernels
+
+    assert kernels.require_native().prefill_gemm_plan(M, N, K)[3] == bn
+    _check_prefill_gemm(gpu, M, N, K, "plain", False, -1, 0, 0)
+    x, wp = _bf(M, K, dev=gpu), ops.pack_decode_weight(_bf(N, K, dev=gpu, scale=0.05))
+    line = 128 if N % 256 or N <= 6144 else 256
+    assert torch.equal(ops.prefill_gemm(x, wp), ops.prefill_gemm(x, wp, bn=line))
+    if K >= 128:
+        _check_prefill_gemm(gpu, M, N, K, "plain", False, 0, 2, 0)
+
+
 @pytest.mark.parametrize("bn,variant", [(256, -1), (192, -1), (128, -1), (256, 1)])
 def test_prefill_gemm_asymmetric_identity(gpu, bn, variant):
     """x = I (rows), W asymmetric: the output must be exactly W^T's rows (catches a
