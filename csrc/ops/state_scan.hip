@@ -51,6 +51,7 @@ struct Args {
   int* form;     // null, or 1 where the step's long portions go through the three launches, else 0 (pick_form)
   float chain, fixed;
   int per_group;  // heads
+  int conv_x, conv_y, conv_rows;  // the convolution's workgroups; the rows of step_kernel's that they are, 0: none
 };
 
 // (a base that is the same for a wave and an offset of 32 bits: one register a load in flight instead of two)
@@ -81,14 +82,15 @@ __device__ __forceinline__ void pick_form(const Args& A) {
   if (lane == 0) A.form[0] = A.chain * most > A.fixed + n_items;
 }
 
+// workgroup (x, y) of conv_x, conv_y
 template <typename T, int TAPS>
-__global__ __launch_bounds__(256) void conv_kernel(const Args A) {
-  if (A.form && blockIdx.x == gridDim.x - 1) {  // (a column of workgroups past the channels)
-    if (blockIdx.y == 0 && threadIdx.x < 64) pick_form(A);
+__device__ __forceinline__ void convolve(const Args& A, int x, int y) {
+  if (A.form && x == A.conv_x - 1) {  // (a column of workgroups past the channels)
+    if (y == 0 && threadIdx.x < 64) pick_form(A);
     return;
   }
-  const int c8 = (blockIdx.x * 64 + (threadIdx.x & 63)) * 8, sub = threadIdx.x >> 6;
-  if (c8 >= A.Cc) return;
+  const int c8 = (x * 64 + (threadIdx.x & 63)) * 8, sub = threadIdx.x >> 6, n_items = A.n_items[0];
+  if (c8 >= A.Cc || y >= n_items) return;
   const int inner = A.H * A.V;
   const float* W = (const float*)A.conv_w;
   float w[TAPS][8], b[8];
@@ -98,8 +100,7 @@ __global__ __launch_bounds__(256) void conv_kernel(const Args A) {
     for (int j = 0; j < 8; ++j) w[k][j] = W[(size_t)k * A.Cc + c8 + j];
 #pragma unroll
   for (int j = 0; j < 8; ++j) b[j] = A.conv_b[c8 + j];
-  const int n_items = A.n_items[0];
-  for (int item = blockIdx.y; item < n_items; item += gridDim.y) {
+  for (int item = y; item < n_items; item += A.conv_y) {
     const int4 it = A.items[item];
     const int s = it.x, t0 = it.y + sub * 16, t1 = min(it.y + it.z, t0 + 16);
     if (t0 >= t1) continue;
@@ -142,6 +143,9 @@ __global__ __launch_bounds__(256) void conv_kernel(const Args A) {
   }
 }
 
+template <typename T, int TAPS>
+__global__ __launch_bounds__(256) void conv_kernel(const Args A) { convolve<T, TAPS>(A, blockIdx.x, blockIdx.y); }
+
 // Channels [c0, c1) of the last `rows` positions of a long portion go to the ring: nobody reads it any
 // more in this step (the convolution was a launch of its own).
 template <typename T>
@@ -157,11 +161,20 @@ __device__ __forceinline__ void store_ring(const Args& A, int s, int c0, int c1)
 // ---- token by token: a workgroup per (sequence, head, part of V) -------------------------------------
 constexpr int REGS = 8;  // state vectors of a thread that stay in registers over the portion
 
-// TN: N / 4 as a constant (8 .. 64) where the state fits the registers of the workgroup; 0: any sizes.
-template <typename T, int TAPS, int TN>
+// TN: N / 4 as a constant (8 .. 64) where the state fits the registers of the workgroup; 0: any sizes. CONV: the first conv_rows
+// rows of workgroups are the long portions' convolution, which no short portion waits for: a launch of its own took 4.6 us of every layer of a
+// decoding step, which has none. 4 such layers, 64 decoding rows 1,089 -> 1,079 us a step; 3,658 tokens of prompts, convolution and
+// steps 30 -> 27 us a layer, though under this bound the convolution spills 9 registers. (4 taps; with 8 it wants twice the bound's.)
+template <typename T, int TAPS, int TN, bool CONV>
 __global__ __launch_bounds__(256, 5) void step_kernel(const Args A) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
-  const int vlog = __builtin_ctz(A.vsplit), h = blockIdx.x >> vlog, vpart = blockIdx.x & (A.vsplit - 1), s = blockIdx.y;
+  if constexpr (CONV)
+    if ((int)blockIdx.y < A.conv_rows) {
+      const int w = blockIdx.y * gridDim.x + blockIdx.x, y = w / A.conv_x;
+      if (y < A.conv_y) convolve<T, TAPS>(A, w - y * A.conv_x, y);
+      return;
+    }
+  const int vlog = __builtin_ctz(A.vsplit), h = blockIdx.x >> vlog, vpart = blockIdx.x & (A.vsplit - 1), s = blockIdx.y - (CONV ? A.conv_rows : 0);
   const int n = A.q_len[s];
   if (n <= 0) return;
   const int slot = A.state_slot[s], q0 = A.q_start[s], p0 = A.ctx_len[s] - n;
@@ -920,7 +933,7 @@ extern "C" int pa_state_scan(int fp32, const void* proj, int ldp, void* u, void*
   if (V % 16 || N % 32 || H % G || scan_min > MAX_SHORT || ring_rows < taps - 1 + scan_min || (taps != 4 && taps != 8)) return -1;  // (shorter ones are padded)
   Args A{proj, u, y, state, ring, conv_w, conv_b, dt_bias, a, d, q_start, q_len, ctx_len, state_slot,
          (const int4*)items, n_items, ldp, ldy, H, G, V, N, H * V + 2 * G * N, taps, ring_rows, scan_min, fp32, 1,
-         work, total, nullptr, chain, fixed, H / G};
+         work, total, nullptr, chain, fixed, H / G, 0, 0, 0};
   if (A.Cc % 8 || ldp % 8) return -1;
   // the three launches: (bf16) states that scan_kernel is not built for, or a choice
   const int lds_s = 2 * LC * 4 + (N + 2 * V) * LD * 2;
@@ -932,8 +945,16 @@ extern "C" int pa_state_scan(int fp32, const void* proj, int ldp, void* u, void*
     A.long_too = 1;
   }
   if (three && !wide) A.form = (int*)(total + (size_t)max_items * H);
+  // few sequences: a head's V over more workgroups
+  while (A.vsplit < 8 && H * seqs * A.vsplit < 512 && V % (A.vsplit * 2) == 0) A.vsplit *= 2;
+  const bool apart = taps != 4 || A.long_too;  // (its readers are in step_kernel, or too many registers)
   if (max_items > 0) {
-    const dim3 grid((A.Cc / 8 + 63) / 64 + (A.form ? 1 : 0), std::min(max_items, 4096));
+    A.conv_x = (A.Cc / 8 + 63) / 64 + (A.form ? 1 : 0);
+    A.conv_y = std::min(max_items, 4096);
+    if (!apart) A.conv_rows = (A.conv_x * A.conv_y + H * A.vsplit - 1) / (H * A.vsplit);
+  }
+  if (max_items > 0 && apart) {
+    const dim3 grid(A.conv_x, A.conv_y);
 #define PA_CONV(T)                                                                                        \
   do {                                                                                                    \
     if (taps == 4) hipLaunchKernelGGL((conv_kernel<T, 4>), grid, dim3(256), 0, st, A);                    \
@@ -942,16 +963,14 @@ extern "C" int pa_state_scan(int fp32, const void* proj, int ldp, void* u, void*
     if (fp32) PA_CONV(float); else PA_CONV(pa::bf16);
 #undef PA_CONV
   }
-  // few sequences: a head's V over more workgroups
-  while (A.vsplit < 8 && H * seqs * A.vsplit < 512 && V % (A.vsplit * 2) == 0) A.vsplit *= 2;
   const int step_lds = (2 * N + V + 2) * 4;
   if (step_lds > 64 * 1024) return -2;
-  const dim3 sgrid(H * A.vsplit, seqs);
+  const dim3 sgrid(H * A.vsplit, A.conv_rows + seqs);
   const int tn = V / A.vsplit <= REGS * 1024 / N ? N / 4 : 0;
 #define PA_STEP_N(T, K)                                                                                   \
   do {                                                                                                    \
-    if (taps == 4) hipLaunchKernelGGL((step_kernel<T, 4, K>), sgrid, dim3(256), step_lds, st, A);         \
-    else hipLaunchKernelGGL((step_kernel<T, 8, K>), sgrid, dim3(256), step_lds, st, A);                   \
+    if (taps == 4) hipLaunchKernelGGL((step_kernel<T, 4, K, sizeof(T) == 2>), sgrid, dim3(256), step_lds, st, A); \
+    else hipLaunchKernelGGL((step_kernel<T, 8, K, false>), sgrid, dim3(256), step_lds, st, A);            \
   } while (0)
 #define PA_STEP(T)                                                                                        \
   do {                                                                                                    \

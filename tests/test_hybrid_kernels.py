@@ -449,6 +449,13 @@ def test_state_scan(device, dt, H, V, N, G, taps):
     assert (state[:2] == 1e4).all() and (ring[:2] == 1e3).all()  # nobody's slots
 
 
+@kinds
+@pytest.mark.parametrize("H,V,N,G,taps", [(1, 16, 32, 1, 4), (5, 256, 32, 5, 3)])
+def test_state_scan_convolution_beside_the_steps(device, dt, H, V, N, G, taps):
+    """Rows of workgroups that hold one of the convolution's, and many."""
+    test_state_scan(device, dt, H, V, N, G, taps)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("V,N,lens", [
     (48, 128, [9 + 7 * (i % 9) for i in range(41)]),           # more portions than the grid has rows for
