@@ -7,7 +7,9 @@
 
 extern "C" {
 int pa_table_route(const int* tables, const int* desc, int layers, const int* ids, const int* slots, int T, int tm,
-                   int* order, int* tiles, int* n_tiles, hipStream_t st);
+                   int* order, int* tiles, int* n_tiles, int* counts, int slices, hipStream_t st);
+int pa_table_route_slices(int T, int most);
+int pa_table_route_counts();
 }
 
 
@@ -20,14 +22,19 @@ void table_route(at::Tensor tables, at::Tensor desc, at::Tensor desc_host, at::T
                   desc_host.size(1) == 8 && desc_host.is_contiguous(), "desc_host must be int32 [layers, 8] on the CPU");
   const int64_t L = desc_host.size(0);
   const int* d = desc_host.data_ptr<int>();
-  for (int64_t l = 0; l < L; ++l, d += 8)
+  int most = 1;
+  for (int64_t l = 0; l < L; ++l, d += 8) {
     TORCH_CHECK(d[3] >= 1 && d[3] <= 2048 && d[2] >= 1 && d[0] >= 0 && (int64_t)d[0] + (int64_t)d[1] * d[2] <= tables.numel() &&
                     d[4] >= 0 && d[4] + T * d[2] <= order.numel() && d[5] >= 0 &&
                     ((int64_t)d[5] + d[6]) * 4 <= tiles.numel() && tm >= 1,
                 "table_route: layer ", l, " does not fit its buffers");
+    most = std::max(most, d[2]);
+  }
+  const int slices = pa_table_route_slices((int)T, most);
+  const at::Tensor counts = at::empty({slices * L * pa_table_route_counts()}, order.options());
   check_rc(pa_table_route(ints(tables, 1, "tables"), ints(desc, L * 8, "desc"), L, ints(ids, T, "ids"),
                           ints(slots, T, "slots"), T, tm, (int*)ints(order, 0, "order"), (int*)ints(tiles, 0, "tiles"),
-                          (int*)ints(n_tiles, L, "n_tiles"), cur_stream()),
+                          (int*)ints(n_tiles, L, "n_tiles"), slices ? counts.data_ptr<int>() : nullptr, slices, cur_stream()),
            "table_route");
 }
 

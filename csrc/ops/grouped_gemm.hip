@@ -666,35 +666,71 @@ __global__ __launch_bounds__(256) void gemm_f32_kernel(const Args A) {
   }
 }
 
-// Routing by token id, for every expert layer of the model in one launch (workgroup = layer):
+// Routing by token id, for every expert layer of the model (blockIdx.x: the layer):
 // layer l's table [vocab, top] (int32, at tables + desc[0]) names the token's experts. Rows with
 // slot < 0 (padding) are left out. Writes, at the layer's offsets,
 //   order[p] = token * top + k, positions sorted by expert;  tiles: at most tm rows of one expert each.
+// Bound by a workgroup's instructions and by the wait for an id and then its table row, 1,024 positions at a time. So steps of more
+// than one and a half slices of ROUTE_SLICE positions count in one launch, a workgroup a slice, and place in another. 8 layers of 64 experts,
+// 6 a token, back to back, us in one launch and in two: 4,096 tokens 35.0, 10.9, 2,048 19.5, 10.5, 1,300 13.5, 10.4, 1,000 (in one) 11.6; in
+// a step, whose tables are not in the caches, 4,096 64, 18.
 constexpr int ROUTE_DESC = 8;  // {table offset, vocab, top, experts, order offset, tile offset, max tiles, 0}
-constexpr int ROUTE_EMAX = 2048;
+constexpr int ROUTE_EMAX = 2048, ROUTE_SLICE = 4096;
+enum { ROUTE_ALL = 0, ROUTE_COUNT = 1, ROUTE_PLACE = 2 };
 
+template <int PART>
 __global__ __launch_bounds__(1024) void table_route_kernel(const int* __restrict__ tables, const int* __restrict__ desc,
                                                            const int* __restrict__ ids, const int* __restrict__ slots,
                                                            int T, int tm, int* __restrict__ order,
-                                                           int4* __restrict__ tiles, int* __restrict__ n_tiles) {
+                                                           int4* __restrict__ tiles, int* __restrict__ n_tiles,
+                                                           int* __restrict__ counts) {  // [layers, slices, ROUTE_EMAX]
   __shared__ int cnt[ROUTE_EMAX], base[ROUTE_EMAX], tbase[ROUTE_EMAX], ws[2][16];
   const int* d = desc + blockIdx.x * ROUTE_DESC;
   const int V = d[1], top = d[2], E = d[3];
   const int* tab = tables + d[0];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
-  for (int e = threadIdx.x; e < E; e += 1024) cnt[e] = 0;
-  __syncthreads();
+  const int p0 = PART == ROUTE_ALL ? 0 : blockIdx.y * ROUTE_SLICE, p1 = PART == ROUTE_ALL ? T * top : min(T * top, p0 + ROUTE_SLICE);
+  constexpr int U = PART == ROUTE_ALL ? 1 : ROUTE_SLICE / 1024;
+  int* mine = counts + ((size_t)blockIdx.x * gridDim.y + blockIdx.y) * ROUTE_EMAX;
   auto expert = [&](int p) {
     const int t = p / top;
     if (slots[t] < 0) return -1;
     const int e = tab[(size_t)min(max(ids[t], 0), V - 1) * top + (p - t * top)];
     return min(max(e, 0), E - 1);
   };
-  for (int p = threadIdx.x; p < T * top; p += 1024) {
-    const int e = expert(p);
-    if (e >= 0) atomicAdd(&cnt[e], 1);
+  if constexpr (PART != ROUTE_PLACE) {
+    for (int e = threadIdx.x; e < E; e += 1024) cnt[e] = 0;
+    __syncthreads();
+#pragma unroll U
+    for (int p = p0 + threadIdx.x; p < p1; p += 1024) {
+      const int e = expert(p);
+      if (e >= 0) atomicAdd(&cnt[e], 1);
+    }
+    __syncthreads();
   }
-  __syncthreads();
+  if constexpr (PART == ROUTE_COUNT) {
+    for (int e = threadIdx.x; e < E; e += 1024) mine[e] = cnt[e];
+    return;
+  }
+  constexpr int EPT = ROUTE_EMAX / 1024;
+  int before[EPT];  // an expert's rows in the slices ahead of this one
+  if constexpr (PART == ROUTE_PLACE) {
+#pragma unroll
+    for (int k = 0; k < EPT; ++k) {
+      const int e = threadIdx.x + k * 1024;
+      if (e >= E) break;
+      int all = 0, ahead = 0;
+      const int* from = counts + (size_t)blockIdx.x * gridDim.y * ROUTE_EMAX + e;
+#pragma unroll 8
+      for (int y = 0; y < (int)gridDim.y; ++y) {
+        const int n = from[(size_t)y * ROUTE_EMAX];
+        ahead += y < (int)blockIdx.y ? n : 0;
+        all += n;
+      }
+      cnt[e] = all;
+      before[k] = ahead;
+    }
+  }
   // exclusive scans of the row and tile counts, 1,024 experts at a time
   int carry_r = 0, carry_t = 0;
   for (int e0 = 0; e0 < E; e0 += 1024) {
@@ -719,14 +755,21 @@ __global__ __launch_bounds__(1024) void table_route_kernel(const int* __restrict
     carry_t += tq;
     __syncthreads();
   }
-  int4* tl = tiles + d[5];
-  for (int e = threadIdx.x; e < E; e += 1024)
-    for (int i = 0, k = tbase[e]; i < cnt[e]; i += tm, ++k)
-      if (k < d[6]) tl[k] = int4{e, base[e] + i, min(tm, cnt[e] - i), 0};
-  if (threadIdx.x == 0) n_tiles[blockIdx.x] = min(carry_t, d[6]);
+  if (PART == ROUTE_ALL || blockIdx.y == 0) {
+    int4* tl = tiles + d[5];
+    for (int e = threadIdx.x; e < E; e += 1024)
+      for (int i = 0, k = tbase[e]; i < cnt[e]; i += tm, ++k)
+        if (k < d[6]) tl[k] = int4{e, base[e] + i, min(tm, cnt[e] - i), 0};
+    if (threadIdx.x == 0) n_tiles[blockIdx.x] = min(carry_t, d[6]);
+  }
+  if constexpr (PART == ROUTE_PLACE)
+#pragma unroll
+    for (int k = 0; k < EPT; ++k)
+      if ((int)threadIdx.x + k * 1024 < E) base[threadIdx.x + k * 1024] += before[k];  // (by the thread that read it for the tiles)
   __syncthreads();
   int* ord = order + d[4];
-  for (int p = threadIdx.x; p < T * top; p += 1024) {
+#pragma unroll U
+  for (int p = p0 + threadIdx.x; p < p1; p += 1024) {
     const int e = expert(p);
     if (e >= 0) ord[atomicAdd(&base[e], 1)] = p;
   }
@@ -735,11 +778,26 @@ __global__ __launch_bounds__(1024) void table_route_kernel(const int* __restrict
 }  // namespace gg
 }  // namespace pa
 
+// The slices of pa_table_route's counts, each ROUTE_EMAX ints a layer; 0: it needs none. `most`: the largest top of the layers.
+extern "C" int pa_table_route_slices(int T, int most) {
+  const long long rows = (long long)T * most, n = (rows + pa::gg::ROUTE_SLICE - 1) / pa::gg::ROUTE_SLICE;
+  return 2 * rows > 3 * pa::gg::ROUTE_SLICE && n <= 65535 ? (int)n : 0;
+}
+extern "C" int pa_table_route_counts() { return pa::gg::ROUTE_EMAX; }
+
 extern "C" int pa_table_route(const int* tables, const int* desc, int layers, const int* ids, const int* slots, int T,
-                              int tm, int* order, int* tiles, int* n_tiles, hipStream_t st) {
+                              int tm, int* order, int* tiles, int* n_tiles, int* counts, int slices, hipStream_t st) {
   if (layers <= 0 || T <= 0) return 0;
-  hipLaunchKernelGGL(pa::gg::table_route_kernel, dim3(layers), dim3(1024), 0, st, tables, desc, ids, slots, T, tm,
-                     order, (int4*)tiles, n_tiles);
+#define PA_ROUTE(PART, Y)                                                                                                                 \
+  hipLaunchKernelGGL((pa::gg::table_route_kernel<pa::gg::PART>), dim3(layers, Y), dim3(1024), 0, st, tables, desc, ids, slots, T, tm, order, \
+                     (int4*)tiles, n_tiles, counts)
+  if (slices > 0) {
+    PA_ROUTE(ROUTE_COUNT, slices);
+    PA_ROUTE(ROUTE_PLACE, slices);
+  } else {
+    PA_ROUTE(ROUTE_ALL, 1);
+  }
+#undef PA_ROUTE
   return (int)hipGetLastError();
 }
 

@@ -114,6 +114,36 @@ def test_head_gemm_of_many_rows(gpu, T, G, N, K, gated):
             assert not o[:, N + r:N + 32].any()
 
 
+@pytest.mark.parametrize("T,layers", [(4096, [(64, 2), (2048, 3)]), (4097, [(64, 2), (5, 1)]), (1367, [(1025, 6), (7, 7)]), (9000, [(3, 2)])])
+def test_table_route_slices(gpu, T, layers):
+    """Up to two slices of positions and more, a layer with fewer slices than its neighbour, slices of padding alone: rows by
+    expert and tiles of them, whatever the order of an expert's rows."""
+    from pilottai_amd import ops
+
+    g, V, tm = torch.Generator().manual_seed(T), 97, 64
+    tabs = [torch.stack([torch.randperm(max(E, top), generator=g)[:top] % E for _ in range(V)]).int() for E, top in layers]
+    ids, slots = torch.randint(0, V, (T,), generator=g, dtype=torch.int32), torch.arange(T, dtype=torch.int32)
+    slots[T // 2: T // 2 + T // 5] = -1
+    rows, o, t, tab = [], 0, 0, 0
+    for E, top in layers:
+        cap = T * top // tm + E
+        rows.append([tab, V, top, E, o, t, cap, 0])
+        tab, o, t = tab + V * top, o + T * top, t + cap
+    desc = torch.tensor(rows, dtype=torch.int32)
+    order, tiles, n = (torch.full(x, -7, dtype=torch.int32, device=gpu) for x in ((o,), (t, 4), (len(layers),)))
+    for _ in range(2):
+        ops.table_route(torch.cat([x.reshape(-1) for x in tabs]).to(gpu), desc.to(gpu), desc, ids.to(gpu), slots.to(gpu), T, tm, order, tiles, n)
+    for k, (E, top) in enumerate(layers):
+        expert = torch.where(slots[:, None] >= 0, tabs[k][ids.long()], -1).reshape(-1)
+        got, at, listed = order[rows[k][4]:].cpu(), 0, []
+        for e in range(E):
+            want = torch.nonzero(expert == e).view(-1)
+            assert torch.equal(got[at:at + len(want)].sort().values.long(), want)
+            listed += [[e, at + b, min(tm, len(want) - b), 0] for b in range(0, len(want), tm)]
+            at += len(want)
+        assert int(n[k]) == len(listed) and tiles[rows[k][5]:][:len(listed)].tolist() == listed
+
+
 @pytest.mark.parametrize("dt,tm", [(torch.bfloat16, 16), (torch.bfloat16, 64), (torch.bfloat16, 256), (torch.float32, 16)])
 @pytest.mark.parametrize("T,E,top,ff,D", [(1, 5, 2, 40, 96), (900, 4, 2, 72, 200), (600, 2, 2, 128, 256), (77, 7, 3, 96, 160), (300, 12, 1, 64, 64), (130, 70, 5, 32, 128)])
 def test_table_experts(gpu, dt, tm, T, E, top, ff, D):
