@@ -391,18 +391,8 @@ def q16_pass(qv, qm, hi, lo, rmeta, n_valid: int, K: int, row_priority, row_tags
              now: float, out, exact: bool, workspace: Optional[torch.Tensor] = None) -> None:
     """One pass of quantised queries over a GPU's index into `out` (scores, rows, flags): flags[q] != 0 asks for the batch
     again with exact = True."""
-    C = require_native()
-    Q = qv.shape[0]
-    out_s, out_r, unsafe = out
-    qc = min(Q, COSINE_MAX_Q)
-    need = C.q16_topk_workspace_bytes(qc, max(1, int(n_valid)))
-    if workspace is None or workspace.numel() * workspace.element_size() < need:
-        workspace = torch.empty(max(need, 16), dtype=torch.uint8, device=hi.device)
-    for q0 in range(0, Q, COSINE_MAX_Q):
-        q1 = min(Q, q0 + COSINE_MAX_Q)
-        C.q16_topk(out_s[q0:q1], out_r[q0:q1], unsafe[q0:q1], workspace, qv[q0:q1], qm[q0:q1], hi, lo, rmeta,
-                   int(n_valid), int(K), row_priority, row_tags, row_expiry,
-                   q_min_priority[q0:q1].contiguous(), q_tags[q0:q1].contiguous(), float(now), int(exact))
+    require_native().q16_pass(qv, qm, hi, lo, rmeta, int(n_valid), int(K), row_priority, row_tags, row_expiry, q_min_priority, q_tags,
+                              float(now), *out, bool(exact), workspace)
 
 
 def q16_topk(queries, hi, lo, rmeta, n_valid: int, K: int, row_priority, row_tags, row_expiry,
