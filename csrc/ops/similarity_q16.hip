@@ -694,6 +694,8 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
   constexpr int PER = MAX_WG * C / THREADS;  // entries a thread
   constexpr int CL = 8 * THREADS;            // re-ranked entries at a time
   constexpr int RR = CL / THREADS + 1;
+  constexpr int MOVED = 4;
+  static_assert(MOVED <= PER && MOVED * THREADS <= CL, "entries that move have room");
   __shared__ int red[2 * NW];
   __shared__ Selection sel;
   __shared__ int crow[EXACT ? 1 : CL + MAXK];
@@ -712,13 +714,30 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
   int* orow = out_rows + (size_t)q * K;
   // ---- A: tau = the K-th best lower bound over every slice's list (no bound with fewer than K entries)
   uint32_t key[PER], ukey[PER];
-  int row[PER], have = 0;
+  int row[PER], have = 0, per = (total + THREADS - 1) / THREADS;  // a thread's first `per` may hold an entry
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
     const int e = i * THREADS + threadIdx.x;
+    row[i] = -1;
+    if (i >= per) continue;
     row[i] = e < total ? r[e] : -1;
     have += __popcll(__ballot(row[i] >= 0));
   }
+  // what C and B read is on its way with the lists
+  const float sq = qmeta[2 * q];
+  const int DS = D / 64;
+  // a lane holds 16 dimensions of a row: k-step lane / 4, lane group lane % 4 of it (D <= 1024)
+  const bool on = !EXACT && lane < DS * 4;
+  i32x4 qa = i32x4{0, 0, 0, 0}, qb = qa;
+  if (on) {
+    const signed char* qp = qv + (size_t)q * 2 * D + 16 * lane;
+    qa = *reinterpret_cast<const i32x4*>(qp);
+    qb = *reinterpret_cast<const i32x4*>(qp + D);
+  }
+  const uint32_t none = ord_key(-INFINITY);
+  uint32_t drop = none;
+  if (!EXACT)
+    for (int i = threadIdx.x; i < nwg; i += THREADS) drop = max(drop, ord_key(ldrop[(size_t)q * nwg + i]));
   if (threadIdx.x == 0) ncand = 0;
   __syncthreads();
   int at = 0;
@@ -727,7 +746,7 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
   __syncthreads();
   have = ncand;
   uint32_t tau = 1;
-  if (EXACT || have > THREADS) {
+  if (EXACT || have > MOVED * THREADS) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
       const int e = min(i * THREADS + (int)threadIdx.x, total - 1);
@@ -736,10 +755,15 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
     }
     if (have >= K) tau = block_select<PER, NW>(key, K, red);
   } else {
-    // Slices that share their bounds list a row or two each: such entries move together, one a thread, which one
-    // wave selects from, and their bounds one load instead of 16 in turn (64 queries of 4M rows: 67 -> 53 us).
+    // Slices that share their bounds list a row or two each, and few slices a dozen: such entries move together, up to
+    // MOVED a thread, which one wave selects from where there is one, and their bounds one load instead of 16 in turn (64 queries of 4M
+    // rows: 67 -> 53 us; 3 of 20,011, 1,204 entries in 79 lists, where those of more than 1,024 stayed, 23 -> 18).
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
+      if (i >= per) {
+        ukey[i] = 0;
+        continue;
+      }
       const unsigned long long m = __ballot(row[i] >= 0);
       const int p = at + rank_in(m);
       if (row[i] >= 0) { crow[p] = row[i]; ckey[p] = i * THREADS + threadIdx.x; }
@@ -748,14 +772,26 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
       ukey[i] = 0;
     }
     __syncthreads();
-    if ((int)threadIdx.x < have) {
-      const int e = ckey[threadIdx.x];
-      row[0] = crow[threadIdx.x];
-      ukey[0] = ord_key(u[e]);
-      ckey[threadIdx.x] = ord_key(l[e]);
+    per = (have + THREADS - 1) / THREADS;
+    uint32_t low[MOVED];
+#pragma unroll
+    for (int i = 0; i < MOVED; ++i) {
+      const int at = i * THREADS + threadIdx.x;
+      low[i] = 0;
+      if (at < have) {
+        const int e = ckey[at];
+        row[i] = crow[at];
+        ukey[i] = ord_key(u[e]);
+        low[i] = ord_key(l[e]);
+      }
     }
-    __syncthreads();
-    if (have >= K) tau = lds_select(ckey, have, K, &picked);
+    if (per > 1) {
+      if (have >= K) tau = block_select<MOVED, NW>(low, K, red);
+    } else {
+      if ((int)threadIdx.x < have) ckey[threadIdx.x] = low[0];  // (each reads its own before)
+      __syncthreads();
+      if (have >= K) tau = lds_select(ckey, have, K, &picked);
+    }
   }
   // ---- B: a slice that refused a row for capacity at a level >= tau may have lost a top-k row
   if (EXACT) {  // the lists hold exact scores
@@ -763,14 +799,13 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
     write_best(key, row, tau, K, sel, os, orow);
     return;
   }
-  uint32_t none = ord_key(-INFINITY), drop = none;
-  for (int i = threadIdx.x; i < nwg; i += THREADS) drop = max(drop, ord_key(ldrop[(size_t)q * nwg + i]));
   const bool lost = __syncthreads_or(drop > none && drop >= tau);
   if (threadIdx.x == 0) unsafe[q] = lost;
   // ---- C: re-rank every listed row whose upper bound reaches tau, exactly
   int cand = 0;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
+    if (i >= per) continue;
     if (ukey[i] < tau) row[i] = -1;
     cand += __popcll(__ballot(row[i] >= 0));
   }
@@ -780,23 +815,13 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
   cand = 0;
 #pragma unroll
   for (int w = 0; w < NW; ++w) cand += red[w];
-  const float sq = qmeta[2 * q];
-  const int DS = D / 64;
-  // a lane holds 16 dimensions of a row: k-step lane / 4, lane group lane % 4 of it (D <= 1024)
-  const bool on = lane < DS * 4;
-  i32x4 qa = i32x4{0, 0, 0, 0}, qb = qa;
-  if (on) {
-    const signed char* qp = qv + (size_t)q * 2 * D + 16 * lane;
-    qa = *reinterpret_cast<const i32x4*>(qp);
-    qb = *reinterpret_cast<const i32x4*>(qp + D);
-  }
   int kept = 0;  // best entries so far, ahead of the next ones in crow / ckey
   const int step = cand <= CL ? PER : CL / THREADS;
 #pragma unroll 1
   for (int part = 0; part < PER; part += step) {
 #pragma unroll
     for (int i = 0; i < PER; ++i) {
-      if (i < part || i >= part + step) continue;
+      if (i < part || i >= part + step || i >= per) continue;
       const unsigned long long m = __ballot(row[i] >= 0);
       int at = 0;
       if (lane == 0 && m) at = atomicAdd(&ncand, (int)__popcll(m));
@@ -809,9 +834,11 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
     for (int j0 = kept + wid * RB; j0 < n; j0 += NW * RB) {
       i32x4 a[RB], b[RB];
       int rw[RB];
+      float sr[RB];
 #pragma unroll
       for (int k = 0; k < RB; ++k) {
         rw[k] = crow[min(j0 + k, n - 1)];
+        sr[k] = rmeta[2 * (size_t)rw[k]];
         if (on) {
           const size_t off = (((size_t)(rw[k] >> 4) * DS + (lane >> 2)) * 64 + 16 * (lane & 3) + (rw[k] & 15)) * 16;
           a[k] = *reinterpret_cast<const i32x4*>(hi + off);
@@ -837,14 +864,16 @@ __global__ __launch_bounds__(THREADS) void stage2_kernel(
           lh += __shfl_xor(lh, o, 64);
           lls += __shfl_xor(lls, o, 64);
         }
-        if (lane == 0 && j0 + k < n) ckey[j0 + k] = ord_key(exact_score(hh, hl, lh, lls, rmeta[2 * (size_t)rw[k]], sq));
+        if (lane == 0 && j0 + k < n) ckey[j0 + k] = ord_key(exact_score(hh, hl, lh, lls, sr[k], sq));
       }
     }
     __syncthreads();
     const bool last = part + step >= PER;
     float* bs = last ? os : best_s;
     int* br = last ? orow : best_r;
-    if (n <= THREADS) {
+    if (n <= 64) {
+      write_best_few(ckey, crow, n, K, bs, br);
+    } else if (n <= THREADS) {
       const uint32_t ck[1] = {(int)threadIdx.x < n ? ckey[threadIdx.x] : 0};
       const int cr[1] = {(int)threadIdx.x < n ? crow[threadIdx.x] : -1};
       write_best(ck, cr, n > K ? lds_select(ckey, n, K, &picked) : 1, K, sel, bs, br);

@@ -28,11 +28,10 @@ __device__ __forceinline__ int rank_in(unsigned long long ballot) {
   return __builtin_amdgcn_mbcnt_hi((uint32_t)(ballot >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)ballot, 0));
 }
 
-// The `want`-th largest of a wave's keys (N a lane; at least `want` of them are not 0).
+// The `want`-th largest of a wave's keys (N a lane; at least `want` of them are not 0, and those are v in the bits above `top`).
 template <int N>
-__device__ __forceinline__ uint32_t wave_select(const uint32_t (&key)[N], int want) {
-  uint32_t v = 0;
-  for (int b = 31; b >= 0; --b) {
+__device__ __forceinline__ uint32_t wave_select(const uint32_t (&key)[N], int want, uint32_t v = 0, int top = 31) {
+  for (int b = top; b >= 0; --b) {
     const uint32_t t = v | (1u << b);
     int c = 0;
 #pragma unroll
@@ -97,18 +96,47 @@ __device__ __forceinline__ uint32_t block_select(const uint32_t (&key)[N], int w
   return m;
 }
 
+// wave_select behind the bits that all keys share: scores of a query have about ten.
+template <int N>
+__device__ __forceinline__ uint32_t wave_select_rest(const uint32_t (&key)[N], int want) {
+  uint32_t lo = 0xffffffffu, hi = 0;
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    lo = key[i] ? min(lo, key[i]) : lo;
+    hi = max(hi, key[i]);
+  }
+  lo = wave_umin(lo);
+  hi = ~wave_umin(~hi);
+  if (lo >= hi) return hi;
+  const int top = 31 - __builtin_clz(lo ^ hi);
+  return wave_select(key, want, hi & ~((2u << top) - 1), top);  // (2u << 31: 0)
+}
+
 // The `want`-th largest of n <= 1,024 keys in LDS (at least `want` of them are not 0), by the first wave: its ballots need no
 // barriers, where block_select has one for every bit. Every thread of a workgroup calls it, the keys written before a
 // barrier; `res`: a word in LDS.
 __device__ __forceinline__ uint32_t lds_select(const uint32_t* keys, int n, int want, uint32_t* res) {
-  if (threadIdx.x < 64) {
+  if (n <= 64) {  // by its rank: where a bit has its ballot, count and branch to wait for, 2.0 us for 62 keys, so 1.5
+    if (threadIdx.x < 64) {
+      const uint32_t k = (int)threadIdx.x < n ? keys[threadIdx.x] : 0;
+      int above = 0, upto = 0;
+      for (int j0 = 0; j0 < n; j0 += 16)
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const uint32_t kj = __builtin_amdgcn_readlane((int)k, j0 + j);
+          above += kj > k;
+          upto += kj >= k;
+        }
+      if (above < want && upto >= want) *res = k;  // (lanes of equal keys write the same)
+    }
+  } else if (threadIdx.x < 64) {
     uint32_t key[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) {
       const int e = i * 64 + threadIdx.x;
       key[i] = e < n ? keys[e] : 0;
     }
-    const uint32_t v = n <= 256 ? wave_select(reinterpret_cast<const uint32_t(&)[4]>(key), want) : wave_select(key, want);
+    const uint32_t v = n <= 256 ? wave_select_rest(reinterpret_cast<const uint32_t(&)[4]>(key), want) : wave_select_rest(key, want);
     if (threadIdx.x == 0) *res = v;
   }
   __syncthreads();
@@ -133,6 +161,23 @@ __device__ __forceinline__ void write_ranked(const Selection& s, int K, float* o
     for (int j = 0; j < n; ++j) rank += s.key[j] > k || (s.key[j] == k && s.row[j] < r);
     if (rank < K) { out_s[rank] = key_value(k); out_r[rank] = r; }
   }
+  if (t < K && t >= n) { out_s[t] = -INFINITY; out_r[t] = -1; }
+}
+// The K <= 64 best of n <= 64 entries in LDS, by the first wave
+__device__ __forceinline__ void write_best_few(const uint32_t* keys, const int* rows, int n, int K, float* out_s, int* out_r) {
+  const int t = threadIdx.x;
+  if (t >= 64) return;
+  const uint32_t k = t < n ? keys[t] : 0;
+  const int r = t < n ? rows[t] : -1;
+  int rank = 0;
+  for (int j0 = 0; j0 < n; j0 += 16)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) {  // (behind the last: keys of 0)
+      const uint32_t kj = __builtin_amdgcn_readlane((int)k, j0 + j);
+      const int rj = __builtin_amdgcn_readlane(r, j0 + j);
+      rank += (int)(kj > k) | ((int)(kj == k) & (int)(rj < r));
+    }
+  if (t < n && rank < K) { out_s[rank] = key_value(k); out_r[rank] = r; }
   if (t < K && t >= n) { out_s[t] = -INFINITY; out_r[t] = -1; }
 }
 template <int N>

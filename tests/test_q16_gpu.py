@@ -63,6 +63,13 @@ def test_q16_two_stage_matches_exact_reference(gpu, N, D, Q, K, filters):
     assert st.get("q16_fallbacks", 0) == 0  # random unit vectors: the drop check never fires
 
 
+@pytest.mark.parametrize("K", [1, 5, 32, 64])
+@pytest.mark.parametrize("N", [40, 64, 65, 250, 1000, 2000, 4100, 16_000, 16_500, 20_011])  # lists of 64 in slices of 256 rows
+def test_q16_lists_of_any_length(gpu, N, K):
+    """Around the lines between the selections of the second stage: up to 64, 256, 1,024 and 4,096 listed entries, and 64 re-ranked."""
+    _check(gpu, N, 256, 3, K, N % 2 == 1, seed=K)
+
+
 @pytest.mark.parametrize("N,Q,K", [(20_000, 16, 5), (200_000, 64, 10)])
 def test_q16_exact_scan_matches_reference(gpu, N, Q, K):
     _check(gpu, N, 1024, Q, K, True, exact=True, seed=5)
