@@ -81,7 +81,8 @@ __device__ __forceinline__ void write_tiles(const Args& A, const int* cnt, const
   if (threadIdx.x == 0) A.n_tiles[0] = min(n, A.max_tiles);
 }
 
-template <typename T>
+// MANY: one of several workgroups
+template <typename T, bool MANY>
 __global__ __launch_bounds__(NT) void score_kernel(const Args A) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int Ep = (A.E + 15) / 16 * 16, EA = A.E + A.always;
@@ -105,22 +106,32 @@ __global__ __launch_bounds__(NT) void score_kernel(const Args A) {
       const bf16* wt[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) wt[i] = (const bf16*)A.w + (size_t)min(e0 + i, tiles - 1) * K32 * 512 + lane * 8;
-      // (8 steps' loads are under way before the first product: one after the other they were what a workgroup waited for. 1,000 tokens,
-      // 64 experts of 2,048 inputs: 20.2 -> 17.5 us, 7 of them these loads, 320 KB a CU)
-      for (int k0 = wid; k0 < K32; k0 += 8 * AHEAD) {
-        bf16x8 b[AHEAD], w[AHEAD][4];
+      if constexpr (MANY) {
+        // (8 steps' loads are under way before the first product: one after the other they were what a workgroup waited for. 1,000 tokens,
+        // 64 experts of 2,048 inputs: 20.2 -> 17.5 us, 7 of them these loads, 320 KB a CU. A workgroup alone, 3 tokens, takes 11.5 so, 11.0 one behind the other)
+        for (int k0 = wid; k0 < K32; k0 += 8 * AHEAD) {
+          bf16x8 b[AHEAD], w[AHEAD][4];
 #pragma unroll
-        for (int q = 0; q < AHEAD; ++q) {
-          const int k = min(k0 + 8 * q, K32 - 1);
-          b[q] = *reinterpret_cast<const bf16x8*>(hr + 32 * k);
+          for (int q = 0; q < AHEAD; ++q) {
+            const int k = min(k0 + 8 * q, K32 - 1);
+            b[q] = *reinterpret_cast<const bf16x8*>(hr + 32 * k);
 #pragma unroll
-          for (int i = 0; i < 4; ++i) w[q][i] = *reinterpret_cast<const bf16x8*>(wt[i] + (size_t)k * 512);
+            for (int i = 0; i < 4; ++i) w[q][i] = *reinterpret_cast<const bf16x8*>(wt[i] + (size_t)k * 512);
+          }
+#pragma unroll
+          for (int q = 0; q < AHEAD; ++q)
+            if (k0 + 8 * q < K32)
+#pragma unroll
+              for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[q][i], b[q], acc[i], 0, 0, 0);
         }
+      } else {
+#pragma unroll 8
+        for (int k = wid; k < K32; k += 8) {
+          const bf16x8 b = *reinterpret_cast<const bf16x8*>(hr + 32 * k);
 #pragma unroll
-        for (int q = 0; q < AHEAD; ++q)
-          if (k0 + 8 * q < K32)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[q][i], b[q], acc[i], 0, 0, 0);
+          for (int i = 0; i < 4; ++i)
+            acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*reinterpret_cast<const bf16x8*>(wt[i] + (size_t)k * 512), b, acc[i], 0, 0, 0);
+        }
       }
       __syncthreads();
 #pragma unroll
@@ -324,14 +335,15 @@ extern "C" int pa_score_route(int fp32, const void* h, int ldh, const void* w, i
   const int Ep = (E + 15) / 16 * 16, lds = (TOK * (Ep + groups + top) + 3 * (E + always) + std::max(8 * 16 * 68, TOK * Ep) + 64) * 4;
   static bool attr = false;
   if (!attr) {
-    (void)hipFuncSetAttribute((const void*)score_kernel<float>, hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);
-    (void)hipFuncSetAttribute((const void*)score_kernel<pa::bf16>, hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);
+    for (const void* f : {(const void*)score_kernel<float, false>, (const void*)score_kernel<pa::bf16, false>, (const void*)score_kernel<pa::bf16, true>})
+      (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);
     attr = true;
   }
   if (lds > 159 * 1024) return -2;
   const int wgs = (T + TOK - 1) / TOK;
-  if (fp32) hipLaunchKernelGGL(score_kernel<float>, dim3(wgs), dim3(NT), lds, st, A);
-  else hipLaunchKernelGGL(score_kernel<pa::bf16>, dim3(wgs), dim3(NT), lds, st, A);
+  if (fp32) hipLaunchKernelGGL((score_kernel<float, false>), dim3(wgs), dim3(NT), lds, st, A);
+  else if (wgs == 1) hipLaunchKernelGGL((score_kernel<pa::bf16, false>), dim3(wgs), dim3(NT), lds, st, A);
+  else hipLaunchKernelGGL((score_kernel<pa::bf16, true>), dim3(wgs), dim3(NT), lds, st, A);
   if (wgs > 1) {
     const int per = std::max(4, std::min((wgs + 63) / 64, PLACE_INTS / (E + always) - 3));
     hipLaunchKernelGGL(place_kernel, dim3((wgs + per - 1) / per), dim3(NT), (3 + per) * (E + always) * 4, st, A, wgs, per);
