@@ -178,6 +178,81 @@ __global__ __launch_bounds__(256) void paged_kv_kernel(const Args A) {
   }
 }
 
+// The same for many rows, without pooling: a workgroup takes MANY neighbouring tokens, a thread 8 dimensions of all of them with the
+// loads of four under way at once, and a page's 16-byte pieces of neighbouring keys leave one after the other. A token a
+// workgroup waited for its slot, its row and its angles in turn: 3,658 rows of 16 heads on 4 of 128 (45 MB) 24.3 us, so 18.3 (groups of four 18.8).
+constexpr int MANY = 8, MANY_ROWS = 1536;  // us, a token a workgroup and groups: 512 rows 4.8, 7.5, 1,024 7.3, 8.0, 2,048 11.7, 8.8, 4,096 20.4, 16.3
+template <typename T>
+__global__ __launch_bounds__(512) void many_kv_kernel(const Args A) {
+  constexpr int N = 4;
+  const int group = token_of(blockIdx.x, (A.T + MANY - 1) / MANY);
+  if (group < 0) return;
+  const int t0 = group * MANY, half = A.rd >> 1;
+  int slot[MANY], pos[MANY];
+#pragma unroll
+  for (int i = 0; i < MANY; ++i) {
+    slot[i] = A.slots[min(t0 + i, A.T - 1)];
+    pos[i] = max(0, A.positions[min(t0 + i, A.T - 1)]);
+  }
+  bool any = false;
+#pragma unroll
+  for (int i = 0; i < MANY; ++i) {
+    if (t0 + i >= A.T) slot[i] = -1;
+    if (slot[i] < 0) pos[i] = 0;
+    any = any || slot[i] >= 0;
+  }
+  if (!any) return;
+  const int ck = A.DK >> 3, cv = A.DV >> 3, nq = A.H * ck, nk = A.G * ck, nv = A.GV * cv;
+  for (int u = threadIdx.x; u < nq + nk + nv; u += blockDim.x) {
+    const bool query = u < nq, value = u >= nq + nk;
+    const int w = query ? u : value ? u - nq - nk : u - nq, per = value ? cv : ck, D = value ? A.DV : A.DK;
+    const int h = quot(w, value ? A.icv : A.ick), o = w - h * per, d = o * 8;
+    const int off = (query ? 0 : value ? A.vcol : A.H * A.DK) + h * D;
+    const bool turn = !value && d < A.rd;
+    const int pd = d < half ? d + half : d - half, ci = d < half ? d : pd;
+    float b[8], pb[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) b[j] = pb[j] = 0.f;
+    if (A.bias) {
+      load8(A.bias + off + d, b);
+      if (turn) load8(A.bias + off + pd, pb);
+    }
+    const float sign = d < half ? -1.f : 1.f;
+#pragma unroll
+    for (int i0 = 0; i0 < MANY; i0 += N) {
+      T a[N][8], p[N][8];
+      float c[N][8], s[N][8];
+#pragma unroll
+      for (int i = 0; i < N; ++i)
+        __builtin_memcpy(a[i], __builtin_assume_aligned((const T*)A.x + (size_t)min(t0 + i0 + i, A.T - 1) * A.ldx + off + d, sizeof(T) * 8), sizeof(T) * 8);
+      if (turn)
+#pragma unroll
+        for (int i = 0; i < N; ++i) {
+          __builtin_memcpy(p[i], __builtin_assume_aligned((const T*)A.x + (size_t)min(t0 + i0 + i, A.T - 1) * A.ldx + off + pd, sizeof(T) * 8), sizeof(T) * 8);
+          load8(A.cos_sin + (size_t)pos[i0 + i] * A.rd + ci, c[i]);
+          load8(A.cos_sin + (size_t)pos[i0 + i] * A.rd + half + ci, s[i]);
+        }
+#pragma unroll
+      for (int i = 0; i < N; ++i) {
+        if (slot[i0 + i] < 0) continue;
+        float v[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) v[j] = A.bias ? (float)a[i][j] + b[j] : (float)a[i][j];
+        if (turn)
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const float q = A.bias ? (float)p[i][j] + pb[j] : (float)p[i][j];
+            v[j] = v[j] * c[i][j] + sign * q * s[i][j];
+          }
+        const size_t page = (size_t)(slot[i0 + i] >> 4);
+        T* to = query ? (T*)A.q + ((size_t)(t0 + i0 + i) * A.H + h) * A.DK + d
+                      : (T*)(value ? A.vp : A.kp) + ((page * (value ? A.GV : A.G) + h) * per + o) * 128 + (slot[i0 + i] & 15) * 8;
+        put(to, v);
+      }
+    }
+  }
+}
+
 // lanes of a head of D dimensions, as a power of two
 __host__ __device__ __forceinline__ int head_bits(int D) {
   int b = 0;
@@ -308,10 +383,14 @@ extern "C" int pa_paged_kv(int fp32, const void* x, const float* bias, void* q, 
     return (int)hipGetLastError();
   }
   const bool later = pool > 0 && T > 64, now = pool > 0 && !later;
+  const bool many = T >= pa::kv::MANY_ROWS && rd / 2 % 8 == 0;  // (whole pieces of a head turn together)
+  const int units = (H * DK + G * DK + GV * DV) / 8, rounds = (units + 511) / 512;
+  const dim3 mgrid(((T + pa::kv::MANY - 1) / pa::kv::MANY + 7) / 8 * 8), mwg(((units + rounds - 1) / rounds + 63) / 64 * 64);
   const int rows = pool < 8 ? pool : 8;  // of a workgroup of the second launch
 #define PA_KV(TYPE)                                                                                              \
   do {                                                                                                           \
     if (now) hipLaunchKernelGGL((pa::kv::paged_kv_kernel<TYPE, true>), grid, dim3(256), 0, st, A);               \
+    else if (many) hipLaunchKernelGGL((pa::kv::many_kv_kernel<TYPE>), mgrid, mwg, 0, st, A);                    \
     else hipLaunchKernelGGL((pa::kv::paged_kv_kernel<TYPE, false>), grid, dim3(256), 0, st, A);                  \
     if (later) hipLaunchKernelGGL(pa::kv::pool_kernel<TYPE>, dim3((T + rows - 1) / rows), dim3(256), 0, st, A, rows); \
   } while (0)
