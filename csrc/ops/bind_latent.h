@@ -19,7 +19,7 @@ int pa_latent_attention(int fp32, void* out, float* part_o, float* part_ml, cons
                         int rp, int dec_tokens, int tile_tokens, int window, float scale_log2, int simple,
                         const pa::la::Expand* expand, const void* uv, void* y, int ldy, int vp, int T, hipStream_t st);
 int pa_latent_plan(const pa::la::Expand* X, const int* q_start, const int* q_len, const int* ctx_len, int S, int T, int H, int window,
-                   int room, int max_att, int max_tiles, int slots, hipStream_t st);
+                   int room, int max_att, int max_tiles, int slots, int* skip, hipStream_t st);
 int pa_latent_expand(const pa::la::Expand* X, const void* pages, const void* wk, const void* wv, const int* block_table, int max_blocks, int H, int D,
                      int max_tiles, hipStream_t st);
 }
@@ -136,13 +136,13 @@ void expand_room(pa::la::Expand& X, const Tensors& plan, const at::Tensor& kx, c
 // Decides which requests of the step have their keys expanded and writes the plan; `slots` partial results and `room` blocks
 // are what the launches with this plan have.
 void latent_plan(const Tensors& plan, at::Tensor q_start, at::Tensor q_len, at::Tensor ctx_len, int64_t T, int64_t H, int64_t window,
-                 int64_t room, int64_t slots) {
+                 int64_t room, int64_t slots, at::Tensor skip) {
   const int64_t S = q_len.numel();
   const pa::la::Expand X = expand_plan(plan, S, T);
   TORCH_CHECK(T >= 1 && H >= 1 && room >= 1 && slots >= 0 &&
                   plan[3].size(0) >= T / pa::la::X_COLS + pa::la::X_REQS + slots, "latent_plan sizes");
   check_rc(pa_latent_plan(&X, ints(q_start, S, "q_start"), ints(q_len, S, "q_len"), ints(ctx_len, S, "ctx_len"), S, T, H, window, room,
-                          plan[3].size(0), plan[4].size(0), slots, cur_stream()),
+                          plan[3].size(0), plan[4].size(0), slots, (int*)ints(skip, T, "skip"), cur_stream()),
            "latent_plan");
 }
 

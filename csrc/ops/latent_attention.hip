@@ -1065,12 +1065,14 @@ __device__ __forceinline__ void expanded_unit(const Args& A, const int4 it, int 
 // they fill less than half of the columns of more than two tiles: 10 of 50 after 150 beside 200 decode rows 3,292 us refused,
 // 3,407 expanded; 60 of 12 after 60 3,033, 3,370; 7 of 72 after 150 beside 30 2,912, 2,800. And none where they are less than twice
 // the tokens of the other requests, whose items wait for the units: 2 of 140 after 600 beside 230 rows of 1,500 keys 3,409, 3,464; 4
-// of 132 after 700 beside 200 of 1,000 3,615, 3,605. Tiles whose keys are more than a workgroup's average are split. Rows behind the last request's are nobody's
-// and left out like the expanded: 13 of 512 had the head products walk their whole inputs, W_uv's 11.9 us and W_uk's 7.4, 4.7 and 5.2 without (3,007 -> 2,885 a step of 8 layers).
+// of 132 after 700 beside 200 of 1,000 3,615, 3,605. Tiles whose keys are more than a workgroup's average are split. Rows
+// behind the last request's are nobody's, and the head products leave them out like the expanded (`skip`): 13 of 512 had them walk
+// their whole inputs, W_uv's 11.9 us and W_uk's 7.4, 4.7 and 5.2 without (3,007 -> 2,885 a step of 8 layers).
 constexpr int X_MIN = 12;
 __global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const int* __restrict__ q_start,
                                                            const int* __restrict__ q_len, const int* __restrict__ ctx_len, int S,
-                                                           int T, int H, int window, int room, int max_att, int max_tiles, int slots) {
+                                                           int T, int H, int window, int room, int max_att, int max_tiles, int slots,
+                                                           int* __restrict__ skip) {
   static_assert(X_REQS == 64, "a lane a request");
   __shared__ int ws[16], others[16], tops[16], req[X_REQS], qs[X_REQS], ql[X_REQS], cl[X_REQS], to[X_REQS], tiles[X_REQS];
   const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
@@ -1112,7 +1114,10 @@ __global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const
     rest += others[w];
     top = max(top, tops[w]);
   }
-  for (int t = threadIdx.x; t < T; t += 1024) X.form[t] = t >= top;
+  for (int t = threadIdx.x; t < T; t += 1024) {
+    X.form[t] = 0;
+    skip[t] = t >= top;
+  }
   // every wave works out all of this, a request a lane
   int n = found <= X_REQS ? found : 0, lo = 0, hi, blocks = 0, nt = 0, total = 0, cols = 0, tokens = 0;
   if (lane < n) {
@@ -1167,7 +1172,7 @@ __global__ __launch_bounds__(1024) void expand_plan_kernel(const Expand X, const
     if (threadIdx.x == 0) X.base[req[i]] = to[i];
     for (int j = threadIdx.x; 4 * (lo + j) < nb; j += 1024)
       X.tiles[tiles[i] + j] = int4{req[i], 4 * (lo + j), min(4, nb - 4 * (lo + j)), to[i] + 4 * (lo + j)};
-    for (int t = threadIdx.x; t < ql[i]; t += 1024) X.form[qs[i] + t] = 1;
+    for (int t = threadIdx.x; t < ql[i]; t += 1024) X.form[qs[i] + t] = skip[qs[i] + t] = 1;
   }
 }
 
@@ -1528,11 +1533,11 @@ extern "C" int pa_latent_attention(int fp32, void* out, float* part_o, float* pa
 
 
 // The plan of a step for requests with expanded keys: see expand_plan_kernel. X's work lists hold max_att and max_tiles
-// entries, its workspace `room` blocks and `slots` partial results.
+// entries, its workspace `room` blocks and `slots` partial results. skip [T]: 1 for the rows of expanded requests and of none.
 extern "C" int pa_latent_plan(const pa::la::Expand* X, const int* q_start, const int* q_len, const int* ctx_len, int S, int T, int H,
-                              int window, int room, int max_att, int max_tiles, int slots, hipStream_t st) {
+                              int window, int room, int max_att, int max_tiles, int slots, int* skip, hipStream_t st) {
   hipLaunchKernelGGL(pa::la::expand_plan_kernel, dim3(1), dim3(1024), 0, st, *X, q_start, q_len, ctx_len, S, T, H, window, room,
-                     max_att, max_tiles, slots);
+                     max_att, max_tiles, slots, skip);
   return (int)hipGetLastError();
 }
 

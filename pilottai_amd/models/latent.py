@@ -148,7 +148,7 @@ class LatentAttention:
         plan, ex, skip = room.expand.get(self.expand_key()), None, None
         if plan is not None:
             ex = Expanded(plan, pages, self.k_rows, self.uv, meta.block_table, q, self.cos_sin, out)
-            skip = ex.form
+            skip = ex.skip
         qa = new(T, H, self.D)
         if self.D > self.Rp + self.rp:  # (another layer's rows have a rotated part, which these queries leave out)
             qa.zero_()

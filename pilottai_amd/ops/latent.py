@@ -115,7 +115,7 @@ def expand_pays(T: int, slots: int) -> bool:
 
 class ExpandPlan:
     """Which requests of a step of T rows have their keys expanded, decided on the device: [counts, base, form, attention
-    items, expansion tiles], and the room for it. `form` [T] is 1 for their rows."""
+    items, expansion tiles], and the room for it. `form` [T] is 1 for their rows, `skip` [T] for those and the rows of no request."""
 
     def __init__(self, meta, T: int, heads: int, window: int):
         dev, S, self.window = meta.q_len.device, meta.q_len.numel(), window
@@ -123,11 +123,11 @@ class ExpandPlan:
         self.blocks = (T + max(T, 4096)) // 16
         self.slots = max(8, 768 // heads)
         new = lambda *s: torch.empty(*s, dtype=torch.int32, device=dev)  # noqa: E731
-        self.form = new(T)
+        self.form, self.skip = new(T), new(T)
         self.lists = [new(2), new(S), self.form, new(T // EXPAND_COLS + EXPAND_REQS + self.slots, 4),
                       new(self.blocks // 4 + EXPAND_REQS, 4)]
         require_latent().latent_plan(self.lists, meta.q_start, meta.q_len, meta.ctx_len, int(T), int(heads), int(window),
-                                     int(self.blocks), int(self.slots))
+                                     int(self.blocks), int(self.slots), self.skip)
 
 
 class Expanded:
@@ -137,7 +137,7 @@ class Expanded:
     def __init__(self, plan: ExpandPlan, pages, wk, wv, block_table, q, cos_sin, out):
         H, dev = wk.shape[0], pages.device
         new = lambda dt, *s: torch.empty(*s, dtype=dt, device=dev)  # noqa: E731
-        self.plan, self.form, self.q, self.cos_sin, self.out = plan.lists, plan.form, q, cos_sin, out
+        self.plan, self.form, self.skip, self.q, self.cos_sin, self.out = plan.lists, plan.form, plan.skip, q, cos_sin, out
         self.sizes, self.window = (plan.blocks, plan.slots), plan.window
         self.kx, self.kr = new(torch.bfloat16, plan.blocks, H, 32, 16, 8), new(torch.bfloat16, plan.blocks, 8, 16, 8)
         self.part_o = new(torch.float32, plan.slots, H, EXPAND_COLS, 128)

@@ -675,7 +675,8 @@ def test_rows_behind_the_last_request_are_left_out(gpu, reqs, rest):
     """A captured step's rows that no request has: the head products leave them out, whatever the plan takes."""
     plan, T = plan_of(gpu, reqs, 16, 0, rest)
     held = [int(n >= 12) for _, n in reqs for _ in range(n)]
-    assert plan.form.tolist() == held + [1] * rest and T == len(held) + rest
+    form = held if reqs[-1][1] >= 12 else [0] * len(held)
+    assert plan.form.tolist() == form + [0] * rest and plan.skip.tolist() == form + [1] * rest and T == len(held) + rest
 
 
 @pytest.mark.parametrize("T,G", [(9, 3), (70, 5), (300, 9), (2100, 16)])  # tiles of 16 and of 64 rows, rows through LDS
