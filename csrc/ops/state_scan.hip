@@ -14,7 +14,7 @@
 // Short portions (at most `scan_min` tokens, decode rows among them): step_kernel, convolution included,
 // token after token; the ring has room for their inputs beside the taps they read.
 // Longer ones (bf16), in chunks of 64 tokens (l = running sum of -a dt over the chunk, L = its end; held in log2):
-//   conv_kernel   u for all their rows
+//   convolution   u for all their rows, in step_kernel's launch (bf16, 4 taps) or ahead of it (conv_kernel)
 //   scan_kernel   y_i = exp(l_i) C_i . S + sum_{j <= i} exp(l_i - l_j) dt_j (C_i . B_j) x_j + D x_i,
 //                 S <- exp(L) S + sum_j exp(L - l_j) dt_j B_j x_j^T, chunk after chunk
 //   or the same in three launches, each over all chunks: chunk_state_kernel, state_pass_kernel, chunk_out_kernel
@@ -147,7 +147,7 @@ template <typename T, int TAPS>
 __global__ __launch_bounds__(256) void conv_kernel(const Args A) { convolve<T, TAPS>(A, blockIdx.x, blockIdx.y); }
 
 // Channels [c0, c1) of the last `rows` positions of a long portion go to the ring: nobody reads it any
-// more in this step (the convolution was a launch of its own).
+// more in this step (the convolution was in an earlier launch).
 template <typename T>
 __device__ __forceinline__ void store_ring(const Args& A, int s, int c0, int c1) {
   const int q0 = A.q_start[s], n = A.q_len[s], p0 = A.ctx_len[s] - n, inner = A.H * A.V, rows = min(A.taps - 1, n);
