@@ -43,10 +43,10 @@ class StreamPlan:
         self.subs = [(f64(h.mix), f64(h.post)[None], h.bias is not None) for h in subs[:self.end]]
         self._coef: Dict[tuple, torch.Tensor] = {}
 
-    def coef(self, summed: tuple) -> torch.Tensor:
+    def coef(self, summed: tuple, kept: bool) -> torch.Tensor:
         """[terms, streams] behind len(summed) outputs, in the kernel's order: biases and what is summed from partials (fp32), then the
-        embedding row and the other outputs (bf16); the last one's sum stands behind them until it is kept."""
-        if summed not in self._coef:  # (before graph capture: the capture's warm-up runs come first)
+        embedding row and the other outputs (bf16). The last one's sum is one of the first if it is `kept`, else it stands behind all."""
+        if (summed, kept) not in self._coef:  # (before graph capture: the capture's warm-up runs come first)
             narrow = torch.ones(1, self.subs[0][0].shape[0], dtype=torch.float64)
             wide = last = narrow[:0]
             for partials, (mix, post, bias) in zip(summed, self.subs):
@@ -57,8 +57,9 @@ class StreamPlan:
                     last = post
                 else:
                     narrow = torch.cat([narrow, post])
-            self._coef[summed] = torch.cat([wide, narrow, last]).float().to(self.device).contiguous()
-        return self._coef[summed]
+            order = [wide, last, narrow] if kept else [wide, narrow, last]
+            self._coef[summed, kept] = torch.cat(order).float().to(self.device).contiguous()
+        return self._coef[summed, kept]
 
 
 class Residual:
@@ -101,9 +102,9 @@ class Residual:
         D, kept, x = self.embed.shape[1], None, None
         if rows is None and self.at == self.plan.end and not self.plan.whole:
             x = self._rows(self.streams, D)
-        elif rows is None and self.step:
+        elif rows is None and self.step and self.at < self.plan.end:  # (behind the last output nobody adds to it)
             kept = self._rows(D)
-        out = ops.stream_norm(self.f, self.b, self.plan.coef(self.summed), eps, ids=self.ids, rows=rows, x=x, y_kept=kept, **kw, **self.step)
+        out = ops.stream_norm(self.f, self.b, self.plan.coef(self.summed, not self.step), eps, ids=self.ids, rows=rows, x=x, y_kept=kept, **kw, **self.step)
         if x is not None:
             self.x, self.f, self.b, self.step = x, [], [], {}
         elif kept is not None:

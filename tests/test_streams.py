@@ -3,19 +3,22 @@ import pytest
 import torch
 
 from pilottai_amd.models.streams import Hyper, Residual, StreamPlan
-from test_mudepel import close, engine, expect, feed, folder, tokens  # noqa: F401
+from test_mudepel import DESIGNS, close, engine, expect, feed, folder, oracle, tokens  # noqa: F401
 
 DEVICES = ["cpu", pytest.param("cuda:0", marks=pytest.mark.gpu)]
 
 
 @pytest.mark.parametrize("device", DEVICES)
 # sums to the end, and up to where streams take over; widths of part of a pass, one, and two; more biases than a sum's terms
-@pytest.mark.parametrize("S,subs,D,T,biases", [(4, 16, 1024, 5, 3), (2, 13, 16, 3, 2), (3, 13, 2056, 4, 3), (4, 27, 44, 300, 3), (8, 40, 64, 1, 1),
-                                               (2, 3, 8, 2, 1)])
-def test_sums_are_the_streams(device, S, subs, D, T, biases):
+# (the last sublayer's parts: as the others', or weighted bf16 ones, or fp32 ones, with a bias of its own and without)
+@pytest.mark.parametrize("S,subs,D,T,biases,end", [(4, 16, 1024, 5, 3, 0), (2, 13, 16, 3, 2, 0), (3, 13, 2056, 4, 3, 0), (4, 27, 44, 300, 3, 0),
+                                                   (8, 40, 64, 1, 1, 0), (2, 3, 8, 2, 1, 0), (4, 12, 1032, 5, 11, 7), (4, 12, 64, 7, 3, 3),
+                                                   (3, 9, 2056, 3, 4, 2), (5, 10, 16, 300, 4, 2), (2, 1, 8, 3, 1, 7)])
+def test_sums_are_the_streams(device, S, subs, D, T, biases, end):
     g = torch.Generator().manual_seed(S * subs + D)
     rand = lambda *s: torch.randn(*s, generator=g).to(device)  # noqa: E731
     parts = [(1, 3, 1, 7, 2)[j % 5] for j in range(subs)]
+    parts[-1] = end or parts[-1]
     layers = [Hyper(rand(S, S) / S ** 0.5, rand(S), rand(D) if j % biases == 0 else None, 1 + (parts[j] > 1)) for j in range(subs)]
     w, embed, ld = rand(D), rand(31, D).bfloat16(), D + 64
     ids = torch.randint(-2, 33, (T,), generator=g, dtype=torch.int32).to(device)
@@ -24,17 +27,23 @@ def test_sums_are_the_streams(device, S, subs, D, T, biases):
     plan = StreamPlan(layers, device)
     units = sum(h.units for h in layers)
     assert plan.whole == (units <= 5 * S and subs + sum(h.bias is not None for h in layers) < 63) and 0 < plan.end <= subs
+    assert plan.whole or not end
     step = Residual(plan, S, embed, ids)
 
-    def check(**kw):
-        pre, rows = rand(S), kw.get("rows")
+    def check(pre=None, **kw):
+        pre, rows = rand(S) if pre is None else pre, kw.get("rows")
         got = step.norm(1e-5, pre=pre, w_next=w, out=torch.full((T if rows is None else len(rows), ld), 7.0, device=device).bfloat16(), **kw)
         u, m = (torch.einsum("s,tsd->td", p, x)[slice(None) if rows is None else rows.long()] for p, x in ((pre.double(), X), (pre.double().abs(), size)))
         r = torch.rsqrt(u.pow(2).mean(-1, keepdim=True) + 1e-5)
         want, bound = u * r * w.double(), 8 * (S + subs) * 2.0 ** -24 * (m + m.pow(2).mean(-1, keepdim=True).sqrt()) * r * w.double().abs()
         assert bool(((got[:, :D].double() - want).abs() <= bound + 2.0 ** -8 * want.abs()).all()) and not got[:, D:].any()
+        return got
+    rows = torch.tensor([T - 1, 0, T - 1], dtype=torch.int32, device=device)
     for h, K in zip(layers, parts):
+        check(rows=rows)  # asked for again, also behind what was kept
         check()
+        check()
+        check(rows=rows)
         y, yw = rand(T * K, D + 8).bfloat16(), torch.rand(T, K, generator=g).to(device) if K > 2 else None
         if K == 2:
             y = y.float()  # unrounded parts
@@ -45,10 +54,10 @@ def test_sums_are_the_streams(device, S, subs, D, T, biases):
             v, each = v + h.bias.double(), each + h.bias.double().abs()
         X = torch.einsum("st,nsd->ntd", h.mix.double(), X) + h.post.double()[None, :, None] * v[:, None]
         size = torch.einsum("st,nsd->ntd", h.mix.double().abs(), size) + h.post.double().abs()[None, :, None] * each[:, None]
-    rows = torch.tensor([T - 1, 0, T - 1], dtype=torch.int32, device=device)
-    check(rows=rows)
-    check()
-    check(rows=rows)
+    pre = rand(S)
+    first, every, again = check(pre, rows=rows), check(pre), check(pre, rows=rows)
+    if plan.whole:  # all rows, for a pool, leave the logits' rows their bits
+        assert torch.equal(again, first) and torch.equal(every[rows.long()], first)
 
 
 @pytest.mark.gpu
@@ -98,3 +107,29 @@ def test_model_of_sums(folder, monkeypatch, name, device):
     eng, ids = engine(folder, name, device, "bfloat16"), tokens(name, 150)
     assert eng.model.sums is not None
     close(feed(eng, 1, ids, [70, 1, 79]), expect(folder, name, ids), "bfloat16")
+
+
+@pytest.mark.parametrize("device", DEVICES)
+@pytest.mark.parametrize("rows", [1, 257])  # by sums from the first row on, and behind the line
+def test_a_pool_beside_logits(folder, monkeypatch, rows, device):
+    """A step that also pools embeddings: logits have the bits of the step without, and the pool has the streams' sum."""
+    from pilottai_amd.models.mudepel import MudepelModel
+
+    monkeypatch.setattr(MudepelModel, "SUMS_MIN_T", rows)
+    T = max(rows, 40) + 3
+    got, ids = [], tokens("wide", T)
+    for pooled in (False, True):
+        eng = engine(folder, "wide", device, "bfloat16", max_num_batched_tokens=320, max_model_len=320)
+        assert eng.model.sums is not None and eng.model.sums.whole and T >= rows
+        forward, embed = eng.model.forward, (torch.zeros(T + 512, dtype=torch.int32, device=device), torch.zeros(2, 96, device=device))
+        embed[0][T:] = 1  # (padding)
+        if pooled:
+            monkeypatch.setattr(eng.model, "forward", lambda *a, **kw: forward(*a, **{**kw, "embed": embed}))
+        got.append(feed(eng, 1, ids, [T]))
+    assert torch.equal(*got)
+    close(got[0], expect(folder, "wide", ids), "bfloat16")
+    tw, lay = oracle.read_checkpoint(folder("wide")), []
+    oracle.forward(DESIGNS["wide"], tw, ids, layers=lay)
+    want = oracle.norm(lay[-1], tw["final.norm"].double(), 1e-4).mean(0)
+    off = (embed[1][0].double().cpu() / T - want).pow(2).mean().sqrt() / want.std()
+    assert off < 0.08, float(off)  # (of `close`: bf16, median)
