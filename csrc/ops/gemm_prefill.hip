@@ -590,10 +590,11 @@ static double width_cost(int M, int N, int K, int bn) {
   plan_default(M, N, K, bn, full, S);
   return S > 1 ? SLICED : (bn == 128 ? 1. : bn == 192 ? 1.32 : 1.63) * rounds_cost(tiles);
 }
+static int bn_by_n(int N) { return (N % 256 || N <= 6144) ? 128 : 256; }
 static int pick_bn(int M, int N, int K, int variant, bool default_plan) {
-  const int bn = (N % 256 || N <= 6144) ? 128 : 256;
+  const int bn = bn_by_n(N);
   // (the other families and a caller's slices keep the line by N: they have no tiles of 192 columns)
-  if (N % 128 || K < 128 || variant < 3 || !default_plan) return bn;
+  if (M <= 0 || N % 128 || K < 128 || variant < 3 || !default_plan) return bn;
   const double old = width_cost(M, N, K, bn);
   int best = bn;
   double least = 0.95 * old;
@@ -613,10 +614,12 @@ extern "C" void pa_prefill_set_variant(int v) { pa::pf::g_pf_variant = v < 0 ? p
 extern "C" int pa_prefill_pick_bn(int M, int N, int K) { return pa::pf::pick_bn(M, N, K, pa::pf::g_pf_variant, true); }
 
 extern "C" void pa_prefill_gemm_plan(int M, int N, int K, int bn, int* full, int* S) {
+  if (bn <= 0) bn = pa_prefill_pick_bn(M, N, K);
   pa::pf::plan_default(M, N, K, bn, *full, *S);
 }
 
 extern "C" long long pa_prefill_gemm_ws_floats(int M, int N, int bn, int full, int S) {
+  if (bn <= 0) bn = pa::pf::bn_by_n(N);  // (launches with slices have that width)
   const long long tiles = (long long)((M + 255) / 256) * (N / bn);
   return S > 1 ? (tiles - full) * S * (long long)(256 * bn) : 0;
 }
