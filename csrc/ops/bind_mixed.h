@@ -30,7 +30,7 @@ void gated_norm(at::Tensor y, at::Tensor z, at::Tensor w, at::Tensor slots, int6
 }
 
 void score_route(at::Tensor h, at::Tensor w, at::Tensor slots, at::Tensor weights, at::Tensor choice, at::Tensor rank,
-                 at::Tensor counts, at::Tensor order, at::Tensor tiles, at::Tensor n_tiles, int64_t E, int64_t top,
+                 Opt counts, at::Tensor order, at::Tensor tiles, at::Tensor n_tiles, int64_t E, int64_t top,
                  int64_t groups, int64_t keep, int64_t always, int64_t tm, bool softmax, Opt correction, bool share,
                  double scale) {
   const int f = is_f32(h, "h");
@@ -41,8 +41,11 @@ void score_route(at::Tensor h, at::Tensor w, at::Tensor slots, at::Tensor weight
   const int64_t T = h.size(0), P = T * (top + always);
   TORCH_CHECK(G == 1 && N >= E && K <= h.size(1) && h.stride(0) % 8 == 0 && tm >= 1, "score_route sizes");
   TORCH_CHECK(tiles.dim() == 2 && tiles.size(1) == 4, "tiles must be [n, 4]");
-  out_ints(counts, E + always, "counts");  // (a place of the caller's, where one workgroup counts for all)
-  const at::Tensor each = T > 16 ? at::empty({(T + 15) / 16, E + always}, counts.options()) : counts;
+  // counts: room for E + always of every workgroup; allocated where the caller gives none or has less
+  const int64_t room = T > 16 ? (T + 15) / 16 * (E + always) : 0;
+  if (counts.has_value()) out_ints(*counts, E + always, "counts");
+  const bool fits = counts.has_value() && counts->numel() >= room;
+  const at::Tensor each = fits ? *counts : at::empty({room}, slots.options().dtype(at::kInt));
   check_rc(pa_score_route(f, h.data_ptr(), h.stride(0), w.data_ptr(), K, ints(slots, T, "slots"),
                           (float*)opt_f32(weights, P, "weights"), out_ints(choice, P, "choice"), out_ints(rank, P, "rank"),
                           each.data_ptr<int>(), out_ints(order, P, "order"), out_ints(tiles, 4, "tiles"),

@@ -607,8 +607,7 @@ class ScoredExperts:
         ints = lambda *n: torch.empty(*n, dtype=torch.int32, device=dev)  # noqa: E731
         weights = torch.empty(T, K, dtype=torch.float32, device=dev)
         choice, rank, order, tiles, n_tiles = ints(rows), ints(rows), ints(rows), ints(rows // tm + min(E, rows), 4), ints(1)
-        counts = ints(E)
-        ops.score_route(h, self.router, meta.slots, weights, choice, rank, counts, order, tiles, n_tiles, s.experts, s.top,
+        ops.score_route(h, self.router, meta.slots, weights, choice, rank, None, order, tiles, n_tiles, s.experts, s.top,
                         s.groups, s.keep, s.always, tm, softmax=s.softmax, correction=self.correction, share=s.share, scale=s.scale)
         act = torch.empty(rows, self.fp, dtype=self.dtype, device=dev)
         ops.expert_gemm(h, self.w13, act, tiles, n_tiles, order, rows, x_div=K, out_order=False, tm=tm, glu=s.act,

@@ -748,3 +748,25 @@ def test_gated_mlp_module(device, dt, T, d, ff):
 @pytest.mark.parametrize("T,E,top,always", [(65, 64, 6, 1), (1100, 64, 6, 1), (300, 700, 4, 2), (4300, 20, 3, 0)])
 def test_rows_of_many_workgroups_are_placed(gpu, T, E, top, always):
     test_score_route(gpu, BF16, T, E, top, 1, 1, always)
+
+
+@kinds
+@pytest.mark.parametrize("T", [16, 17, 200])
+def test_score_route_with_any_room_for_counts(device, dt, T):
+    """No room of the caller's, too little for all workgroups and enough: the same rows of every expert."""
+    from pilottai_amd import ops
+
+    g, E, top, always = gen(T), 9, 2, 1
+    h, w = torch.randn(T, 64, generator=g).to(dt).to(device), ops.pack_groups(torch.randn(1, 16, 64, generator=g).to(dt), dt).to(device)
+    slots, KA, EA = torch.arange(T, dtype=torch.int32, device=device), top + always, E + always
+    ints, got = lambda *n: torch.full(n, -7, dtype=torch.int32, device=device), []  # noqa: E731
+    for room in (None, EA, (T + 15) // 16 * EA):
+        weights, choice, order, tiles, n = torch.zeros(T, KA, device=device), ints(T * KA), ints(T * KA), ints(T * KA // 16 + EA, 4), ints(1)
+        ops.score_route(h, w, slots, weights, choice, ints(T * KA), room and ints(room), order, tiles, n, E, top, 1, 1, always, 16)
+        used = tiles[:int(n)].tolist()
+        rows = [sorted(r for f, at, k, _ in used if f == e for r in order[at:at + k].tolist()) for e in range(EA)]
+        got.append((weights.tolist(), choice.tolist(), used, rows))
+    assert got[0] == got[1] == got[2] and sum(map(len, got[0][3])) == T * KA
+    if h.is_cuda:
+        with pytest.raises(RuntimeError, match="counts"):
+            ops.score_route(h, w, slots, weights, choice, ints(T * KA), ints(EA - 1), order, tiles, n, E, top, 1, 1, always, 16)
