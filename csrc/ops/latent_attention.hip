@@ -287,7 +287,7 @@ __device__ __forceinline__ void split_item(const Args& A, const int4 it, char* s
 
 // The partitions of the expanded units. Each part of a tile merges its share of the tile's tokens (groups of four, in turn), a wave
 // four tokens of a head, two at a time with 4 dims a lane: all parts' loads of a wave are under way at once. Four tiles in four parts (499 tokens
-// after 3,584), 17 MB: with a wave a token of the first parts, the others idle, 11.6 us, so 8.0 (a launch that finds none takes 4.7).
+// after 3,584), 17 MB: with a wave a token of the first parts, the others idle, 11.6 us, so 8.2 (a launch that finds none takes 4.7).
 __device__ __forceinline__ void merge_expanded(const Args& A) {
   constexpr int TOK = 4, UNITS = X_COLS / TOK;
   const int lane = threadIdx.x & 63, n = A.X.counts[0] * A.H * UNITS, half = lane >> 5, d = 4 * (lane & 31);
@@ -319,9 +319,11 @@ __device__ __forceinline__ void merge_expanded(const Args& A) {
       for (int p = 0; p < X_PARTS; ++p) m = fmaxf(m, ml[j][p].x);
 #pragma unroll
       for (int p = 0; p < X_PARTS; ++p) {
-        const float f = p < parts ? exp2f(ml[j][p].x - m) : 0.f;
-        L += f * ml[j][p].y;
-        v += f * o[j][p];
+        // (written out: left to the compiler, the unrolled sums of products are rounded in other places than one after the other)
+        const float f = exp2f(ml[j][p].x - m);
+        L = p < parts ? fmaf(f, ml[j][p].y, L) : L;
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = p < parts ? fmaf(f, o[j][p][r], v[r]) : v[r];
       }
       if (2 * j + half >= left) continue;
       const float inv = 1.f / L;
