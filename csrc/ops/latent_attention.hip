@@ -35,6 +35,7 @@
 #include "latent_expand.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace pa {
 namespace la {
@@ -1331,22 +1332,65 @@ __global__ __launch_bounds__(64 * NW, 2) void mfma_kernel(const Args A) {
 }
 
 // merge_kernel and the next product in one launch, y[row, head h] = W_uv[h] (merged latent): a workgroup of 16 waves per (head, `per`
-// columns, up to 16: tokens of the items in their order). The waves share the columns' partitions, while the head's W_uv is on its
+// columns, up to 16: tokens of the items in their order). The waves share the columns' dimensions, while the head's W_uv is on its
 // way: a wave has 16 of its (at most 128) rows and half of their inputs. A chain of dependent reads bounds it (items, (max, sum) pairs, partitions),
-// where two launches had each their own: 4 rows after 2,000 tokens, 16 heads of 512 and 128, a step's 8 layers 1,064 -> 1,040 us, 32 rows
-// 2,037 -> 2,005. (A workgroup for 16 items, whatever tokens they hold, took 3 to 5 % longer for steps of short prompts.)
+// where two launches had each their own: 8 rows after 2,048 tokens, 16 heads of 512 and 128, a step's 8 layers 1,430 -> 1,399 us, 64 rows
+// 2,241 -> 2,213, the launch 7.3 and 8.6. Partitions and inputs are added up in the order of the two launches: a request's bits do not
+// depend on the step's form. (With partitions shared out over the waves, whose sums meet in LDS, the launch took 7.4 and 8.9; a workgroup for
+// 16 items, whatever tokens they hold, 3 to 5 % more of a step of short prompts.)
 constexpr int MH_WAVES = 16;
+
+// Columns [d, d + VW) of the partitions of one token and head, added up in their order; all loads of a round are under way at once.
+template <int VW>
+__device__ __forceinline__ void merge_dims(const Args& A, int4 e, int RP, int d, float (&a)[8]) {
+  typedef float vec __attribute__((ext_vector_type(VW > 4 ? 4 : VW)));
+  constexpr int PIECES = VW > 4 ? 2 : 1, ROUND = VW == 1 ? 16 : VW == 2 ? 8 : 4;  // (few columns are of long splits)
+  const int lane = threadIdx.x & 63, nparts = e.y >> 20, step = (e.y & 0xff) <= A.dec_tokens ? 1 : 8;
+  const float2* ml = reinterpret_cast<const float2*>(A.part_ml);
+  auto slot = [&](int p) { return (size_t)e.x + (size_t)p * step * A.NB * 16; };
+  float gm = NEG_BIG, L = 0.f;
+  for (int p0 = 0; p0 < nparts; p0 += 64) gm = fmaxf(gm, p0 + lane < nparts ? ml[slot(p0 + lane)].x : NEG_BIG);
+  gm = wave_max(gm);
+  for (int p0 = 0; p0 < nparts; p0 += 64) {
+    float wt = 0.f;
+    if (p0 + lane < nparts) {
+      const float2 v = ml[slot(p0 + lane)];
+      wt = exp2f(v.x - gm);
+      L += wt * v.y;
+    }
+    const int np = min(64, nparts - p0);
+#pragma unroll 1
+    for (int q = 0; q < np; q += ROUND) {
+      vec x[ROUND][PIECES];
+#pragma unroll
+      for (int p = 0; p < ROUND; ++p) {  // (behind the last: its values again)
+        const vec* s = reinterpret_cast<const vec*>(A.part_o + slot(p0 + min(q + p, np - 1)) * RP + d);
+#pragma unroll
+        for (int i = 0; i < PIECES; ++i) x[p][i] = s[i];
+      }
+#pragma unroll
+      for (int p = 0; p < ROUND; ++p) {
+        const float wp = __shfl(wt, (q + p) & 63, 64);
+#pragma unroll
+        for (int j = 0; j < VW; ++j) a[j] = q + p < np ? fmaf(wp, x[p][j / 4][j % 4], a[j]) : a[j];
+      }
+    }
+  }
+  const float inv = 1.f / wave_sum(L);
+#pragma unroll
+  for (int j = 0; j < VW; ++j) a[j] *= inv;
+}
+
 template <int RT>
 __global__ __launch_bounds__(64 * MH_WAVES) void merge_heads_kernel(const Args A, const bf16* __restrict__ uv, bf16* __restrict__ y, int ldy,
                                                                     int vp, int max_items, int per) {
   constexpr int RP = 32 * RT, LD = RP + 8, HALF = (RT + 1) / 2;
   __shared__ __attribute__((aligned(16))) bf16 xs[16][LD];
-  __shared__ __attribute__((aligned(16))) float ps[MH_WAVES][RP < 256 ? 256 : RP];
+  __shared__ __attribute__((aligned(16))) float ps[8][256];
   __shared__ int4 cols[16];  // {the first partition's column, the item's z, sequence, token}
   __shared__ int sums[MH_WAVES];
   const int h = blockIdx.x, lane = threadIdx.x & 63, wid = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), tiles = vp / 16;
-  const int g = lane >> 4, c16 = lane & 15, d = min(lane * 8, RP - 8), tile = wid & 7, k0 = wid >> 3 ? HALF : 0;
-  const float2* ml = reinterpret_cast<const float2*>(A.part_ml);
+  const int g = lane >> 4, c16 = lane & 15, tile = wid & 7, k0 = wid >> 3 ? HALF : 0;
   bf16x8 w[HALF];
 #pragma unroll
   for (int k = 0; k < HALF; ++k)
@@ -1379,80 +1423,49 @@ __global__ __launch_bounds__(64 * MH_WAVES) void merge_heads_kernel(const Args A
   const int m = min(per, total - lo);
   if (m <= 0) return;
   const int mine = min(c16, m - 1), row = A.q_start[cols[mine].z] + cols[mine].w;
-  const int shift = m > 8 ? 0 : m > 4 ? 1 : m > 2 ? 2 : m > 1 ? 3 : 4, waves = 1 << shift;  // of a column
-  const int c = wid >> shift, part = wid & (waves - 1);
-  float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+  // a column's waves have 512 of its dimensions between them: 8 a lane where a wave has a column to itself, 1 where there are 8
+  const int shift = m > 8 ? 0 : m > 4 ? 1 : m > 2 ? 2 : 3, c = wid >> shift;
   if (c < m) {
     const int4 e = cols[c];
-    const int nparts = e.y >> 20, step = (e.y & 0xff) <= A.dec_tokens ? 1 : 8;
-    if (nparts <= 1) {
-      if (part == 0) {
-        const bf16x8 o = *reinterpret_cast<const bf16x8*>((const bf16*)A.out + ((size_t)(A.q_start[e.z] + e.w) * A.H + h) * RP + d);
-#pragma unroll
-        for (int j = 0; j < 8; ++j) a[j] = (float)o[j];
-      }
-    } else {
-      auto slot = [&](int p) { return (size_t)e.x + (size_t)p * step * A.NB * 16; };
-      float gm = NEG_BIG, L = 0.f;
-      for (int p0 = 0; p0 < nparts; p0 += 64) gm = fmaxf(gm, p0 + lane < nparts ? ml[slot(p0 + lane)].x : NEG_BIG);
-      gm = wave_max(gm);
-      for (int p0 = 0; p0 < nparts; p0 += 64) {
-        float wt = 0.f;
-        if (p0 + lane < nparts) {
-          const float2 v = ml[slot(p0 + lane)];
-          wt = exp2f(v.x - gm);
-          L += wt * v.y;
-        }
-        const int np = min(64, nparts - p0);
-#pragma unroll 8
-        for (int p = part; p < np; p += waves) {
-          const float wp = __shfl(wt, p, 64);
-          const f32x4* s = reinterpret_cast<const f32x4*>(A.part_o + slot(p0 + p) * RP + d);
-          const f32x4 x = s[0], z = s[1];
-#pragma unroll
-          for (int j = 0; j < 4; ++j) {
-            a[j] += wp * x[j];
-            a[4 + j] += wp * z[j];
-          }
-        }
-      }
-      const float inv = 1.f / wave_sum(L);
-#pragma unroll
-      for (int j = 0; j < 8; ++j) a[j] *= inv;
-    }
-    if (lane * 8 < RP) {
-      if (shift == 0) {
-        bf16x8 v;
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[j] = (bf16)a[j];
-        *reinterpret_cast<bf16x8*>(&xs[c][d]) = v;
+    const int vw = 8 >> shift, d = ((wid & ((1 << shift) - 1)) * 64 + lane) * vw, at = min(d, RP - vw);
+    float a[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    auto merged = [&](auto width) {
+      constexpr int VW = decltype(width)::value;
+      typedef bf16 vec __attribute__((ext_vector_type(VW)));
+      vec v;
+      if (e.y >> 20 <= 1) {
+        v = *reinterpret_cast<const vec*>((const bf16*)A.out + ((size_t)(A.q_start[e.z] + e.w) * A.H + h) * RP + at);
       } else {
+        merge_dims<VW>(A, e, RP, at, a);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) ps[wid][d + j] = a[j];
+        for (int j = 0; j < VW; ++j) v[j] = (bf16)a[j];
       }
-    }
+      if (d < RP) *reinterpret_cast<vec*>(&xs[c][d]) = v;
+    };
+    if (shift == 0) merged(std::integral_constant<int, 8>{});
+    else if (shift == 1) merged(std::integral_constant<int, 4>{});
+    else if (shift == 2) merged(std::integral_constant<int, 2>{});
+    else merged(std::integral_constant<int, 1>{});
   }
   __syncthreads();
-  if (shift) {
-    for (int i = threadIdx.x; i < m * RP; i += 64 * MH_WAVES) {
-      const int q = i / RP, k = i - q * RP;
-      float v = 0.f;
-      for (int r = 0; r < waves; ++r) v += ps[q * waves + r][k];
-      xs[q][k] = (bf16)v;
-    }
-    __syncthreads();
-  }
   // (columns behind the last one hold anything: their products are not stored)
-  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int k = 0; k < HALF; ++k)
-    if (k0 + k < RT)
-      acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[k], *reinterpret_cast<const bf16x8*>(&xs[c16][32 * (k0 + k) + 8 * g]), acc, 0, 0, 0);
   f32x4* other = reinterpret_cast<f32x4*>(ps[tile]) + lane;
-  if (k0) *other = acc;
+  f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+  auto products = [&]() {
+#pragma unroll
+    for (int k = 0; k < HALF; ++k)
+      if (k0 + k < RT)
+        acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[k], *reinterpret_cast<const bf16x8*>(&xs[c16][32 * (k0 + k) + 8 * g]), acc, 0, 0, 0);
+  };
+  if (wid < 8) {
+    products();
+    *other = acc;
+  }
   __syncthreads();
-  if (!k0 && c16 < m && tile < tiles) {
-    acc += *other;
+  if (wid >= 8) {
+    acc = *other;
+    products();
+    if (c16 >= m || tile >= tiles) return;
     bf16x4 o;
 #pragma unroll
     for (int r = 0; r < 4; ++r) o[r] = (bf16)acc[r];

@@ -86,8 +86,9 @@ def latent_attention(out, part_o, part_ml, q, pages, items, n_items, q_start, q_
     return out
 
 
-# Tokens of a step up to which the heads' products go with the merge. A step of bozupel-base, us apart and so: 128 decoding rows 2,290, 2,272, 256
-# 2,572, 2,552, one prompt of 60 tokens 2,020, 2,018, of 120 2,199, 2,200, four of 60 2,445, 2,452
+# Tokens of a step up to which the heads' products go with the merge. A step of bozupel-base, us apart and so: a decoding row 756, 730, 16 1,805,
+# 1,768, 128 after 1,000 tokens 2,455, 2,432, 180 2,720, 2,690, 256 after 2,048 2,572, 2,552; one prompt of 60 tokens 2,055, 2,044, of 120 2,205, 2,195,
+# four of 40 2,345, 2,331
 MERGE_HEADS_T = 192
 
 

@@ -416,21 +416,24 @@ def test_latent_attention_split_tiles(gpu, H, R, r, window):
     run_attention(gpu, torch.bfloat16, H, R, r, [(1500, tile + 1), (900, 2 * tile + 16 // min(H, 16))], window, tiles=64, part=256)
 
 
-MERGED = {"one": [(2000, 1)], "two": [(1500, 1), (700, 1)], "rows": [(60 * i, 1) for i in range(15)], "portions": [(1500, 9), (3, 1), (700, 20), (0, 3)]}
+MERGED = {"one": [(2000, 1)], "two": [(1500, 1), (700, 1)], "rows": [(60 * i, 1) for i in range(15)], "portions": [(1500, 9), (3, 1), (700, 20), (0, 3)],
+          "long": [(4000, 1)], "long rows": [(100 + 400 * i, 1) for i in range(6)]}
 
 
-@pytest.mark.parametrize("step", list(MERGED))  # 1, 2 and more columns of 16 items, of one and several partitions; tokens of an item
+@pytest.mark.parametrize("step", list(MERGED))  # 1, 2 and more columns of 16 items, of one to more than 64 partitions; tokens of an item
 @pytest.mark.parametrize("H,R,r,vp", [(16, 512, 64, 128), (20, 256, 32, 80), (3, 96, 24, 16), (40, 192, 64, 64)])
 def test_merged_heads(gpu, H, R, r, vp, step):
-    """The heads' products behind the merge: of rows whose bf16 roundings may fall differently, sums of Rp products in fp32."""
+    """The heads' products behind the merge, sums of Rp products in fp32: the bits of the merge and the products on their own."""
     from pilottai_amd import ops
     from pilottai_amd.ops.latent import latent_pad, pad_to
 
     g = torch.Generator(device=gpu).manual_seed(H + vp)
     rnd = lambda *s: torch.randn(*s, device=gpu, generator=g).bfloat16()  # noqa: E731
     Rp, rp = latent_pad(R), pad_to(r, 32)
-    T, m, dec, tile = fed_meta(gpu, H, MERGED[step], 64, 0, tiles=64, part=256)
+    target, part = (192, 16) if step.startswith("long") else (64, 256)
+    T, m, dec, tile = fed_meta(gpu, H, MERGED[step], target, 0, tiles=64, part=part)
     NB, mi, D = (dec * H + 15) // 16, m["items"].shape[0], Rp + rp
+    assert step != "long" or H > 16 or int(m["items"][0, 2]) >> 20 > 64
     q, pages, uv = rnd(T, H, D), rnd(600, D // 8, 16, 8), rnd(H, vp, Rp) / Rp ** 0.5
     m = {k: v.to(gpu) for k, v in m.items()}
     f32 = lambda n: torch.empty(n, dtype=torch.float32, device=gpu)  # noqa: E731
@@ -441,8 +444,12 @@ def test_merged_heads(gpu, H, R, r, vp, step):
                              m["ctx_len"], m["block_table"], D ** -0.5, 0, dec, tile, **kw)
         return out
     y = torch.full((T, H * vp + 8), 7.0, dtype=torch.bfloat16, device=gpu)
-    run(heads=(ops.pack_groups(uv, torch.bfloat16), y[:, :H * vp]))
-    o, w = run().float(), uv.float()
+    wp, two = ops.pack_groups(uv, torch.bfloat16), torch.zeros(T, H * vp, dtype=torch.bfloat16, device=gpu)
+    run(heads=(wp, y[:, :H * vp]))
+    oc = run()
+    ops.head_gemm(oc.view(T, -1), Rp, wp, two, vp)
+    assert torch.equal(y[:, :H * vp], two)
+    o, w = oc.float(), uv.float()
     want, size = torch.einsum("thk,hvk->thv", o, w), torch.einsum("thk,hvk->thv", o.abs(), w.abs())
     err = (y[:, :H * vp].float().view(T, H, vp) - want).abs()
     assert bool((err <= 2.0 ** -8 * want.abs() + (2.0 ** -8 + Rp * 2.0 ** -24) * size).all()) and bool((y[:, H * vp:] == 7.0).all())
