@@ -22,7 +22,7 @@ constexpr int X_NONE = -(1 << 30);
 struct Expand {
   int* counts;  // attention items, expansion tiles
   int* base;    // [S] workspace block of the request's key block 0 (blocks before its window have none), or X_NONE
-  int* form;    // [T] 1: the row belongs to an expanded request, or to none
+  int* form;    // [T] 1: the row belongs to an expanded request (the head products go by the plan's `skip`, 1 for rows of no request too)
   int4* att;    // {request, tile of X_COLS tokens, part | parts << 16, partial slot}
   int4* tiles;  // {request, first key block, blocks, workspace block}
   void *kx, *kr;

@@ -555,6 +555,7 @@ def test_latent_attention_expanded(gpu, H, step, window):
     bf, R, n, r, V = torch.bfloat16, 512, 128, 64, 128
     g = torch.Generator().manual_seed(H + window)
     T, m, dec, tile = fed_meta(gpu, H, reqs, 384, window)
+    T += 5  # rows of no request
     pages = torch.randn(600, (R + r) // 8, 16, 8, generator=g).to(bf)
     uk, uv = ((torch.randn(H, k, R, generator=g) * R ** -0.5).to(bf) for k in (n, V))
     q = torch.randn(T, H * (n + r), generator=g).to(bf)
@@ -571,13 +572,14 @@ def test_latent_attention_expanded(gpu, H, step, window):
     ex = Expanded(plan, pg, ops.pack_groups(d(uk), bf), ops.pack_groups(d(uv), bf), mg["block_table"], qg, d(cs), out)
     qa = torch.full((T, H, R + r), 7.0, dtype=bf, device=gpu)
     ops.head_gemm(qg, n + r, ops.pack_groups(d(uk.transpose(1, 2).contiguous()), bf), qa.view(T, -1), R + r,
-                  rot=(d(pos), d(cs), n, r, r), skip=ex.form)
+                  rot=(d(pos), d(cs), n, r, r), skip=ex.skip)
     NB, mi = (dec * H + 15) // 16, m["items"].shape[0]
     po, pm = torch.empty(mi * NB * 16 * R, device=gpu), torch.empty(mi * NB * 32, device=gpu)
     oc = torch.zeros(T, H, R, dtype=bf, device=gpu)
     ops.latent_attention(oc, po, pm, qa, pg, mg["items"], mg["n_items"], mg["q_start"], mg["q_len"], mg["ctx_len"],
                          mg["block_table"], scale, window, dec, tile, expand=ex)
-    ops.head_gemm(oc.view(T, -1), R, ops.pack_groups(d(uv), bf), out, V, skip=ex.form)
+    ops.head_gemm(oc.view(T, -1), R, ops.pack_groups(d(uv), bf), out, V, skip=ex.skip)
+    assert (out[-5:] == 9.0).all() and (qa[-5:] == 7.0).all()
     o = out.float().cpu().view(T, H, V)
     half = r // 2
     turn = lambda x, at: torch.cat([x[..., :half] * cs[at, :half] - x[..., half:] * cs[at, half:],  # noqa: E731
