@@ -578,30 +578,32 @@ static int block_rows(int MT, int tiles, int bn) {
 // k: whole tiles add up in the same order whatever their width, so that a step keeps its bits, where a recurrent layer's step sizes
 // make another order's last bits 0.7 to 1.1 of a logit's root mean square. us, by N -> so, rows, outputs, inputs: 4,096 x 3072 x
 // 768 28.7 -> 23.0, x 4096 x 2048 64 -> 53, 2,048 x 4608 x 1024 32.3 -> 23.6, 1,024 x 10752 x 2048 46.3 -> 40.6.
+// `tail`: whether the launch may have a mixed tail. The epilogue with rotation and cache has none: priced with one, 3,500 x 6144 x 1024 had 256
+// columns in slices of k and 75 us, where 128 take 65 and 192, as priced now, 59.
 static double rounds_cost(int tiles) {
   const int rem = tiles % 256;
   return tiles / 256 + (rem ? 0.6 + 0.4 / 256 * rem : 0.);
 }
 constexpr double SLICED = 1e30;
-static double width_cost(int M, int N, int K, int bn) {
+static double width_cost(int M, int N, int K, int bn, bool tail) {
   const int MT = (M + 255) / 256, NT = N / bn, tiles = MT * NT, wide = tiles / 256 * 256 / MT, rest = 2 * MT * (NT - wide);
-  if (bn == 256 && tiles % 256 && wide && rest <= 256) return 1.63 / 256 * wide * MT + rounds_cost(rest);  // (pingpong_mixed_kernel)
+  if (tail && bn == 256 && tiles % 256 && wide && rest <= 256) return 1.63 / 256 * wide * MT + rounds_cost(rest);  // (pingpong_mixed_kernel)
   int full, S;
   plan_default(M, N, K, bn, full, S);
   return S > 1 ? SLICED : (bn == 128 ? 1. : bn == 192 ? 1.32 : 1.63) * rounds_cost(tiles);
 }
 static int bn_by_n(int N) { return (N % 256 || N <= 6144) ? 128 : 256; }
-static int pick_bn(int M, int N, int K, int variant, bool default_plan) {
+static int pick_bn(int M, int N, int K, int variant, bool default_plan, bool tail = true) {
   const int bn = bn_by_n(N);
   // (the other families and a caller's slices keep the line by N: they have no tiles of 192 columns)
   if (M <= 0 || N % 128 || K < 128 || variant < 3 || !default_plan) return bn;
-  const double old = width_cost(M, N, K, bn);
+  const double old = width_cost(M, N, K, bn, tail);
   int best = bn;
   double least = 0.95 * old;
   for (int w : {128, 192, 256})
-    if (w != bn && N % w == 0 && old < SLICED && width_cost(M, N, K, w) < least) {
+    if (w != bn && N % w == 0 && old < SLICED && width_cost(M, N, K, w, tail) < least) {
       best = w;
-      least = width_cost(M, N, K, w);
+      least = width_cost(M, N, K, w, tail);
     }
   return best;
 }
@@ -637,7 +639,7 @@ extern "C" int pa_prefill_gemm(void* y, const void* x, const void* wp, const voi
                                int kernel_variant, const int* live, hipStream_t st) {
   using namespace pa::pf;
   if (M <= 0) return 0;
-  if (bn <= 0) bn = pick_bn(M, N, K, kernel_variant >= 0 ? kernel_variant : g_pf_variant, full < 0 && splits <= 0);
+  if (bn <= 0) bn = pick_bn(M, N, K, kernel_variant >= 0 ? kernel_variant : g_pf_variant, full < 0 && splits <= 0, epi != EP_ROPEKV);
   if (bn != 128 && bn != 192 && bn != 256) return 1;
   if (K % 64 != 0 || N % bn != 0 || epi < 0 || epi > 4 || ldx % 8 != 0) return 1;
   const int norm = ss_in != nullptr;

@@ -179,6 +179,21 @@ def test_prefill_qkv_rope(gpu, M, H, KV, K, full, splits, bn):
     torch.testing.assert_close(vc.float().cpu(), rv, atol=4e-2, rtol=2e-2)
 
 
+@pytest.mark.parametrize("M,H,KV,K", [(3500, 32, 8, 1024), (4096, 32, 8, 1024), (2900, 16, 4, 128), (1100, 64, 8, 1024)])
+def test_prefill_qkv_rope_default_width(gpu, M, H, KV, K):
+    """The width that a call leaves open: this epilogue has no mixed tail, so that a wider tile would bring slices of k. The bits are the
+    line's by N."""
+    N = (H + 2 * KV) * 128
+    x, wp = _bf(M, K, dev=gpu), ops.pack_decode_qkv_rope(_bf(N, K, dev=gpu, scale=0.05))
+    cos_sin, rows = ref.rope_cos_sin(4096).to(gpu), torch.arange(M, dtype=torch.int32, device=gpu)
+    got = []
+    for bn in (0, 128 if N % 256 or N <= 6144 else 256):
+        q, kc, vc = (torch.zeros(*s, dtype=torch.bfloat16, device=gpu) for s in ((M, H, 128), (M // 16 + 1, KV, 16, 16, 8), (M // 16 + 1, KV, 128, 16)))
+        ops.prefill_qkv_rope(x, wp, 1e-5, q, kc, vc, rows, rows, cos_sin, H, KV, bn=bn)
+        got.append((q, kc, vc))
+    assert all(torch.equal(a, b) for a, b in zip(*got))
+
+
 @pytest.mark.parametrize("epi", ["plain", "resid"])
 def test_prefill_gemm_strided_views(gpu, epi):
     """The plain / residual epilogues store (and read the residual) 16 B per lane: a padded
