@@ -597,6 +597,7 @@ static int pick_bn(int M, int N, int K, int variant, bool default_plan, bool tai
   const int bn = bn_by_n(N);
   // (the other families and a caller's slices keep the line by N: they have no tiles of 192 columns)
   if (M <= 0 || N % 128 || K < 128 || variant < 3 || !default_plan) return bn;
+  tail = tail && (variant == 3 || variant == 8);
   const double old = width_cost(M, N, K, bn, tail);
   int best = bn;
   double least = 0.95 * old;

@@ -104,6 +104,12 @@ def test_prefill_gemm_default_width(gpu, M, N, K, bn):
         _check_prefill_gemm(gpu, M, N, K, "plain", False, 0, 2, 0)
 
 
+@pytest.mark.parametrize("variant", [3, 4, 8, 9])  # with a mixed tail and without
+def test_prefill_gemm_default_width_of_a_family(gpu, variant):
+    x, wp = _bf(3500, 1024, dev=gpu), ops.pack_decode_weight(_bf(6144, 1024, dev=gpu, scale=0.05))
+    assert torch.equal(ops.prefill_gemm(x, wp, variant=variant), ops.prefill_gemm(x, wp, bn=128, variant=variant))
+
+
 @pytest.mark.parametrize("bn,variant", [(256, -1), (192, -1), (128, -1), (256, 1)])
 def test_prefill_gemm_asymmetric_identity(gpu, bn, variant):
     """x = I (rows), W asymmetric: the output must be exactly W^T's rows (catches a
