@@ -41,8 +41,8 @@ void score_route(at::Tensor h, at::Tensor w, at::Tensor slots, at::Tensor weight
   const int64_t T = h.size(0), P = T * (top + always);
   TORCH_CHECK(G == 1 && N >= E && K <= h.size(1) && h.stride(0) % 8 == 0 && tm >= 1, "score_route sizes");
   TORCH_CHECK(tiles.dim() == 2 && tiles.size(1) == 4, "tiles must be [n, 4]");
-  // counts: room for E + always of every workgroup; allocated where the caller gives none or has less
-  const int64_t room = T > 16 ? (T + 15) / 16 * (E + always) : 0;
+  // counts: room for E + always of every workgroup and of a quarter as many groups; allocated where the caller gives none or has less
+  const int64_t wgs = (T + 15) / 16, room = T > 16 ? (wgs + (wgs + 3) / 4) * (E + always) : 0;
   if (counts.has_value()) out_ints(*counts, E + always, "counts");
   const bool fits = counts.has_value() && counts->numel() >= room;
   const at::Tensor each = fits ? *counts : at::empty({room}, slots.options().dtype(at::kInt));

@@ -20,7 +20,7 @@
 namespace pa {
 namespace sr {
 
-constexpr int TOK = 16, NT = 512, MAX_E = 1024, AHEAD = 8, PLACE_INTS = 12 * 1024;
+constexpr int TOK = 16, NT = 512, MAX_E = 1024, PLACE_INTS = 12 * 1024, GROUP_INTS = 32 * 1024;
 
 struct Args {
   const void* h;      // [T, ldh]
@@ -28,7 +28,7 @@ struct Args {
   const int* slots;
   float* weights;     // [T, top + always]
   int *choice, *rank; // [T, top + always]
-  int* counts;        // [workgroups][E + always] (unused with one workgroup)
+  int* counts;        // [workgroups][E + always] (unused with one workgroup); behind them [groups][E + always] (group_kernel)
   int* order;         // position -> token * (top + always) + k
   int4* tiles;        // {expert, first position, rows, 0}
   int* n_tiles;
@@ -81,8 +81,8 @@ __device__ __forceinline__ void write_tiles(const Args& A, const int* cnt, const
   if (threadIdx.x == 0) A.n_tiles[0] = min(n, A.max_tiles);
 }
 
-// MANY: one of several workgroups
-template <typename T, bool MANY>
+// AHEAD: steps whose loads are under way before their products; 0: as the compiler has them
+template <typename T, int AHEAD>
 __global__ __launch_bounds__(NT) void score_kernel(const Args A) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   const int Ep = (A.E + 15) / 16 * 16, EA = A.E + A.always;
@@ -106,9 +106,7 @@ __global__ __launch_bounds__(NT) void score_kernel(const Args A) {
       const bf16* wt[4];
 #pragma unroll
       for (int i = 0; i < 4; ++i) wt[i] = (const bf16*)A.w + (size_t)min(e0 + i, tiles - 1) * K32 * 512 + lane * 8;
-      if constexpr (MANY) {
-        // (8 steps' loads are under way before the first product: one after the other they were what a workgroup waited for. 1,000 tokens,
-        // 64 experts of 2,048 inputs: 20.2 -> 17.5 us, 7 of them these loads, 320 KB a CU. A workgroup alone, 3 tokens, takes 11.5 so, 11.0 one behind the other)
+      if constexpr (AHEAD > 0) {
         for (int k0 = wid; k0 < K32; k0 += 8 * AHEAD) {
           bf16x8 b[AHEAD], w[AHEAD][4];
 #pragma unroll
@@ -264,9 +262,31 @@ __global__ __launch_bounds__(NT) void score_kernel(const Args A) {
   for (int e = threadIdx.x; e < EA; e += NT) A.counts[(size_t)blockIdx.x * EA + e] = cnt[e];
 }
 
+// Many counts: those of `per` workgroups become what those before them in their group have, and their sums go to sums [groups][EA].
+__global__ __launch_bounds__(NT) void group_kernel(int* __restrict__ counts, int* __restrict__ sums, const int EA, const int wgs, const int per) {
+  const int w0 = blockIdx.x * per, n = min(per, wgs - w0);
+  for (int e = threadIdx.x; e < EA; e += NT) {
+    int low = 0;
+    for (int q0 = 0; q0 < n; q0 += 16) {
+      int v[16];
+#pragma unroll
+      for (int q = 0; q < 16; ++q) v[q] = counts[(size_t)(w0 + min(q0 + q, n - 1)) * EA + e];
+#pragma unroll
+      for (int q = 0; q < 16; ++q)
+        if (q0 + q < n) {
+          counts[(size_t)(w0 + q0 + q) * EA + e] = low;
+          low += v[q];
+        }
+    }
+    sums[(size_t)blockIdx.x * EA + e] = low;
+  }
+}
+
 // One workgroup for the rows of `per` of score_kernel's: what all have for every expert, and what those before its own have. (Global
-// counters took a launch that clears them and score_kernel's turns at them: 1,000 tokens, all of routing 30.7 -> 24.1 us.)
-__global__ __launch_bounds__(NT) void place_kernel(const Args A, const int wgs, const int per) {
+// counters took a launch that clears them and score_kernel's turns at them.) Every workgroup reads all counts: from GROUP_INTS on those of
+// groups, behind group_kernel, whose launch takes 1 to 1.5 us. All of routing, us, without and with: 64 experts, 5,000 rows (20 K counts) 31.3,
+// 32.0, 8,192 37.6, 36.5, 16,384 66.8, 66.0; 160 and 4,096 52.4, 52.0, 16,384 140.8, 129.5; 512 and 300 (10 K) 236.7, 237.6, 1,000 238.8, 236.5.
+__global__ __launch_bounds__(NT) void place_kernel(const Args A, const int wgs, const int per, const int* __restrict__ sums) {
   extern __shared__ __attribute__((aligned(16))) float sm[];
   __shared__ int ws[2][NT / 64], part[2][NT];
   const int EA = A.E + A.always, KA = A.top + A.always;
@@ -274,7 +294,10 @@ __global__ __launch_bounds__(NT) void place_kernel(const Args A, const int wgs, 
   const int w0 = blockIdx.x * per, n = min(per, wgs - w0);
   const int p0 = w0 * TOK * KA, p1 = min((w0 + n) * TOK, A.T) * KA, mine = min(p0 + (int)threadIdx.x, p1 - 1);
   const int choice = A.choice[mine], rank = A.rank[mine];  // (on their way while the counts are added up)
-  const int cols = min(EA, NT), segs = NT / cols, sg = threadIdx.x / cols;
+  const int* from = sums ? sums : A.counts;
+  const int rows = sums ? gridDim.x : wgs, r0 = sums ? blockIdx.x : w0;
+  // (segments of fewer than 16 rows have nothing to win, and are added one after the other: 8 experts and 17 rows, 4.6 -> 2.6 us)
+  const int cols = min(EA, NT), segs = min(NT / cols, (rows + 15) / 16), sg = threadIdx.x / cols;
   for (int e0 = 0; e0 < EA; e0 += cols) {
     const int e = e0 + threadIdx.x % cols;
     int all = 0, low = 0, own[4] = {0, 0, 0, 0};
@@ -282,15 +305,15 @@ __global__ __launch_bounds__(NT) void place_kernel(const Args A, const int wgs, 
       if (sg == 0)
 #pragma unroll
         for (int q = 0; q < 4; ++q) own[q] = A.counts[(size_t)min(w0 + q, wgs - 1) * EA + e];
-      for (int w = sg; w < wgs; w += 16 * segs) {  // (the loads of a round are independent)
+      for (int w = sg; w < rows; w += 16 * segs) {  // (the loads of a round are independent)
         int v[16];
 #pragma unroll
-        for (int q = 0; q < 16; ++q) v[q] = A.counts[(size_t)min(w + q * segs, wgs - 1) * EA + e];
+        for (int q = 0; q < 16; ++q) v[q] = from[(size_t)min(w + q * segs, rows - 1) * EA + e];
 #pragma unroll
         for (int q = 0; q < 16; ++q) {
           const int r = w + q * segs;
-          all += r < wgs ? v[q] : 0;
-          low += r < min(w0, wgs) ? v[q] : 0;
+          all += r < rows ? v[q] : 0;
+          low += r < min(r0, rows) ? v[q] : 0;
         }
       }
     }
@@ -304,8 +327,9 @@ __global__ __launch_bounds__(NT) void place_kernel(const Args A, const int wgs, 
       }
       cnt[e] = all;
       for (int q = 0; q < n; ++q) {
-        before[q * EA + e] = low;
-        low += q < 4 ? own[q & 3] : A.counts[(size_t)(w0 + q) * EA + e];
+        const int o = q < 4 ? own[q & 3] : A.counts[(size_t)(w0 + q) * EA + e];
+        before[q * EA + e] = sums ? low + o : low;
+        if (!sums) low += o;
       }
     }
     __syncthreads();
@@ -322,6 +346,7 @@ __global__ __launch_bounds__(NT) void place_kernel(const Args A, const int wgs, 
 }  // namespace sr
 }  // namespace pa
 
+// counts: room for E + always of every 16 rows and of a quarter as many groups (of at least 4 workgroups); unused up to 16 rows.
 extern "C" int pa_score_route(int fp32, const void* h, int ldh, const void* w, int K, const int* slots, float* weights,
                               int* choice, int* rank, int* counts, int* order, int* tiles, int* n_tiles, int T, int E,
                               int top, int groups, int keep, int always, int tm, int max_tiles, int softmax,
@@ -335,18 +360,27 @@ extern "C" int pa_score_route(int fp32, const void* h, int ldh, const void* w, i
   const int Ep = (E + 15) / 16 * 16, lds = (TOK * (Ep + groups + top) + 3 * (E + always) + std::max(8 * 16 * 68, TOK * Ep) + 64) * 4;
   static bool attr = false;
   if (!attr) {
-    for (const void* f : {(const void*)score_kernel<float, false>, (const void*)score_kernel<pa::bf16, false>, (const void*)score_kernel<pa::bf16, true>})
+    for (const void* f : {(const void*)score_kernel<float, 0>, (const void*)score_kernel<pa::bf16, 0>, (const void*)score_kernel<pa::bf16, 4>,
+                          (const void*)score_kernel<pa::bf16, 8>})
       (void)hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, 159 * 1024);
     attr = true;
   }
   if (lds > 159 * 1024) return -2;
   const int wgs = (T + TOK - 1) / TOK;
-  if (fp32) hipLaunchKernelGGL((score_kernel<float, false>), dim3(wgs), dim3(NT), lds, st, A);
-  else if (wgs == 1) hipLaunchKernelGGL((score_kernel<pa::bf16, false>), dim3(wgs), dim3(NT), lds, st, A);
-  else hipLaunchKernelGGL((score_kernel<pa::bf16, true>), dim3(wgs), dim3(NT), lds, st, A);
+  // Steps under way at once. 8 where a wave's steps are whole rounds of them and a CU has one workgroup (it would hold two of fewer
+  // registers), else 4, and as the compiler has them where weights come from the caches (few workgroups). All of routing, us, 0, 4 and 8:
+  // 512 experts of 4,096 inputs 300 rows 242, 237, 231, 4,096 rows 260, 251, 245, 16,384 681, 658, 956; 160 of 2,048 17 rows 37.6, 39.0, 38.6,
+  // 4,096 53.8, 52.4, 51.4; 160 of 5,120 (20 steps a wave) 17 rows 53.2, 55.0, 60.4, 4,096 78.6, 74.8, 77.7; 8 of 1,024 17 rows 10.3, 10.4, 12.5.
+  const int ahead = fp32 || wgs == 1 ? 0 : wgs <= 256 && K % 2048 == 0 ? 8 : wgs > 96 ? 4 : 0;
+  if (fp32) hipLaunchKernelGGL((score_kernel<float, 0>), dim3(wgs), dim3(NT), lds, st, A);
+  else if (ahead == 8) hipLaunchKernelGGL((score_kernel<pa::bf16, 8>), dim3(wgs), dim3(NT), lds, st, A);
+  else if (ahead == 4) hipLaunchKernelGGL((score_kernel<pa::bf16, 4>), dim3(wgs), dim3(NT), lds, st, A);
+  else hipLaunchKernelGGL((score_kernel<pa::bf16, 0>), dim3(wgs), dim3(NT), lds, st, A);
   if (wgs > 1) {
-    const int per = std::max(4, std::min((wgs + 63) / 64, PLACE_INTS / (E + always) - 3));
-    hipLaunchKernelGGL(place_kernel, dim3((wgs + per - 1) / per), dim3(NT), (3 + per) * (E + always) * 4, st, A, wgs, per);
+    const int EA = E + always, per = std::max(4, std::min((wgs + 63) / 64, PLACE_INTS / EA - 3)), parts = (wgs + per - 1) / per;
+    int* sums = (long long)wgs * EA >= GROUP_INTS ? counts + (size_t)wgs * EA : nullptr;
+    if (sums) hipLaunchKernelGGL(group_kernel, dim3(parts), dim3(NT), 0, st, counts, sums, EA, wgs, per);
+    hipLaunchKernelGGL(place_kernel, dim3(parts), dim3(NT), (3 + per) * EA * 4, st, A, wgs, per, sums);
   }
   return (int)hipGetLastError();
 }

@@ -249,7 +249,7 @@ def score_route(h, w, slots, weights, choice, rank, counts, order, tiles, n_tile
     best of `groups` groups (scored by their two best members), with weights scale * s (`share`: s / (sum of the
     chosen s + 1e-20)); `always` more experts follow with weight 1. Writes weights [T, top + always] and the rows
     sorted by expert (csrc/ops/score_route.hip). counts: scratch of at least E + always ints, any values; more than 16
-    rows take E + always a workgroup of 16, allocated where it is None or has less."""
+    rows take as many for each 16 of them and a quarter more, allocated where it is None or has less."""
     if _on_gpu(h):
         require_family(*MIXED).score_route(h, w, slots, weights, choice, rank, counts, order, tiles, n_tiles, int(E), int(top),
                                      int(groups), int(keep), int(always), int(tm), bool(softmax), correction, bool(share),

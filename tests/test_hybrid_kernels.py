@@ -666,13 +666,13 @@ def test_gated_norm(device, dt, H, V, Vp, parts):
 @kinds
 @pytest.mark.parametrize("T", [1, 16, 17, 300])
 @pytest.mark.parametrize("E,top,groups,keep,always", [(8, 2, 1, 1, 0), (6, 2, 3, 2, 1), (64, 6, 8, 4, 1), (12, 12, 2, 2, 3), (5, 1, 5, 1, 0), (160, 5, 4, 1, 2), (1, 1, 1, 1, 1), (70, 3, 35, 2, 0)])
-def test_score_route(device, dt, T, E, top, groups, keep, always):
+def test_score_route(device, dt, T, E, top, groups, keep, always, K=128):
     from pilottai_amd import ops
 
-    g, D, tm, KA = gen(T + E), 72, 16 if T < 300 else 64, top + always
-    h, w = torch.randn(T, 128, generator=g).to(dt), torch.zeros(1, (E + 15) // 16 * 16, 128).to(dt)
+    g, D, tm, KA = gen(T + E), K - 56, 16 if T < 300 else 64, top + always
+    h, w = torch.randn(T, K, generator=g).to(dt), torch.zeros(1, (E + 15) // 16 * 16, K).to(dt)
     h[:, D:] = 0
-    w[0, :E, :D] = (torch.randn(E, D, generator=g) * 0.3).to(dt)
+    w[0, :E, :D] = (torch.randn(E, D, generator=g) * 0.3 * (72 / D) ** 0.5).to(dt)
     slots = torch.arange(T, dtype=torch.int32)
     slots[T // 3:T // 3 + T // 8] = -1
     ints = lambda *n: torch.full(n, -7, dtype=torch.int32, device=device)  # noqa: E731
@@ -744,10 +744,13 @@ def test_gated_mlp_module(device, dt, T, d, ff):
 
 
 @pytest.mark.gpu
-# rows of one and several workgroups' counts, a last part; more experts than threads; more workgroups than the 64 that place them
-@pytest.mark.parametrize("T,E,top,always", [(65, 64, 6, 1), (1100, 64, 6, 1), (300, 700, 4, 2), (4300, 20, 3, 0)])
-def test_rows_of_many_workgroups_are_placed(gpu, T, E, top, always):
-    test_score_route(gpu, BF16, T, E, top, 1, 1, always)
+# rows of one and several workgroups' counts, a last part; more experts than threads; more workgroups than the 64 that place them; counts of
+# groups, a last one of fewer; 0, 4 and 8 steps ahead, steps that are no whole rounds
+@pytest.mark.parametrize("T,E,top,always,K", [(65, 64, 6, 1, 128), (1100, 64, 6, 1, 128), (300, 700, 4, 2, 128), (4300, 20, 3, 0, 128),
+                                              (2100, 300, 4, 0, 64), (4400, 1000, 2, 1, 128), (17, 70, 3, 0, 2048), (1600, 40, 2, 1, 1056),
+                                              (4113, 8, 2, 0, 2048), (500, 5, 1, 0, 4096)])
+def test_rows_of_many_workgroups_are_placed(gpu, T, E, top, always, K):
+    test_score_route(gpu, BF16, T, E, top, 1, 1, always, K)
 
 
 @kinds
@@ -760,7 +763,7 @@ def test_score_route_with_any_room_for_counts(device, dt, T):
     h, w = torch.randn(T, 64, generator=g).to(dt).to(device), ops.pack_groups(torch.randn(1, 16, 64, generator=g).to(dt), dt).to(device)
     slots, KA, EA = torch.arange(T, dtype=torch.int32, device=device), top + always, E + always
     ints, got = lambda *n: torch.full(n, -7, dtype=torch.int32, device=device), []  # noqa: E731
-    for room in (None, EA, (T + 15) // 16 * EA):
+    for room in (None, EA, ((T + 15) // 16 * 5 + 3) // 4 * EA):
         weights, choice, order, tiles, n = torch.zeros(T, KA, device=device), ints(T * KA), ints(T * KA), ints(T * KA // 16 + EA, 4), ints(1)
         ops.score_route(h, w, slots, weights, choice, ints(T * KA), room and ints(room), order, tiles, n, E, top, 1, 1, always, 16)
         used = tiles[:int(n)].tolist()
