@@ -181,7 +181,10 @@ __global__ __launch_bounds__(256) void paged_kv_kernel(const Args A) {
 // The same for many rows, without pooling: a workgroup takes MANY neighbouring tokens, a thread 8 dimensions of all of them with the
 // loads of four under way at once, and a page's 16-byte pieces of neighbouring keys leave one after the other. A token a
 // workgroup waited for its slot, its row and its angles in turn: 3,658 rows of 16 heads on 4 of 128 (45 MB) 24.3 us, so 18.3 (groups of four 18.8).
-constexpr int MANY = 8, MANY_ROWS = 1536;  // us, a token a workgroup and groups: 512 rows 4.8, 7.5, 1,024 7.3, 8.0, 2,048 11.7, 8.8, 4,096 20.4, 16.3
+// From so many rows and pieces of 8 dimensions on. us, a token a workgroup and groups, bf16, 384 pieces a row: 512 rows 4.8, 7.5, 1,024 7.3, 8.0, 2,048
+// 11.7, 8.9, 4,096 20.9, 16.5; 256: 1,536 rows 6.9, 7.0, 2,048 8.4, 7.5; 192: 1,536 6.2, 6.6, 2,048 7.4, 6.8; 96: 3,000 6.1, 7.3, 4,096 7.6, 7.6; 32: 4,096 5.4,
+// 6.0, 8,192 8.0, 7.0. Rows of fp32 leave fewer of them in flight: 768 pieces, 3,000 rows 30.3, 33.4, 8,192 134, 99; 384: 8,192 39.0, 40.9.
+constexpr int MANY = 8, MANY_ROWS = 1536, MANY_PIECES = 1536 * 256, MANY_ALL = 8192, MANY_PIECES_F32 = 4 << 20;
 template <typename T>
 __global__ __launch_bounds__(512) void many_kv_kernel(const Args A) {
   constexpr int N = 4;
@@ -383,8 +386,11 @@ extern "C" int pa_paged_kv(int fp32, const void* x, const float* bias, void* q, 
     return (int)hipGetLastError();
   }
   const bool later = pool > 0 && T > 64, now = pool > 0 && !later;
-  const bool many = T >= pa::kv::MANY_ROWS && rd / 2 % 8 == 0;  // (whole pieces of a head turn together)
-  const int units = (H * DK + G * DK + GV * DV) / 8, rounds = (units + 511) / 512;
+  const int units = (H * DK + G * DK + GV * DV) / 8;
+  const long long pieces = (long long)T * units;
+  const bool many = rd / 2 % 8 == 0 &&  // (whole pieces of a head turn together)
+      (fp32 ? pieces >= pa::kv::MANY_PIECES_F32 : T >= pa::kv::MANY_ALL || (T >= pa::kv::MANY_ROWS && pieces >= pa::kv::MANY_PIECES));
+  const int rounds = (units + 511) / 512;
   const dim3 mgrid(((T + pa::kv::MANY - 1) / pa::kv::MANY + 7) / 8 * 8), mwg(((units + rounds - 1) / rounds + 63) / 64 * 64);
   const int rows = pool < 8 ? pool : 8;  // of a workgroup of the second launch
 #define PA_KV(TYPE)                                                                                              \

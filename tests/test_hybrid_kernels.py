@@ -289,7 +289,7 @@ def test_paged_kv(device, dt, H, G, dk, dv, rd, P, bias, step):
 @pytest.mark.gpu
 @pytest.mark.parametrize("dt", [BF16, F32])
 @pytest.mark.parametrize("H,G,dk,dv,rd,bias", [(16, 4, 128, 128, 128, False), (3, 3, 64, 32, 32, True), (5, 1, 32, 96, 0, True), (40, 8, 128, 64, 64, False), (2, 2, 96, 32, 20, False)])
-@pytest.mark.parametrize("T", [1536, 1543, 2100])
+@pytest.mark.parametrize("T", [1536, 1543, 2100, 8199])  # from the first line on; small rows and fp32 ones from the last
 def test_paged_kv_of_many_rows(gpu, T, H, G, dk, dv, rd, bias, dt):
     """Tokens in groups write what they write one by one, and rows of no sequence among them nothing."""
     from pilottai_amd import ops
@@ -297,13 +297,14 @@ def test_paged_kv_of_many_rows(gpu, T, H, G, dk, dv, rd, bias, dt):
     g, d = gen(T + rd), lambda t: t.to(gpu)  # noqa: E731
     cols = (H + G) * dk + G * dv
     x, b = d(torch.randn(T, cols + 8, generator=g).to(dt)), d(torch.randn(cols, generator=g)) if bias else None
-    slots = torch.randperm(140 * 16, generator=g)[:T].int()
+    nb = max(140, T // 16 + 4)
+    slots = torch.randperm(nb * 16, generator=g)[:T].int()
     slots[::7], slots[-9:] = -1, -1
     pos, cs = torch.randint(0, 900, (T,), generator=g).int(), d(ops.angle_table(1000, rd, 200.0))
     one = torch.zeros(1, dtype=torch.int32, device=gpu)
     got = []
     for rows in (T, 64):
-        q, kp, vp, p0 = (torch.full(s, 4.0, dtype=dt, device=gpu) for s in ((T, H, dk), (140, G, dk // 8, 16, 8), (140, G, dv // 8, 16, 8), (0, 1, G, dk)))
+        q, kp, vp, p0 = (torch.full(s, 4.0, dtype=dt, device=gpu) for s in ((T, H, dk), (nb, G, dk // 8, 16, 8), (nb, G, dv // 8, 16, 8), (0, 1, G, dk)))
         for t in range(0, T, rows):
             e = min(T, t + rows)
             ops.paged_kv(x[t:e], b, q[t:e], kp, vp, p0, p0, d(pos[t:e]), d(slots[t:e]), one, one, one, one.view(1, 1), cs, 0, num_seqs=1)
