@@ -170,9 +170,11 @@ PRESETS: Dict[str, MudepelConfig] = {
 
 class MudepelModel(HybridModel):
     NAME = "Mudepel"
-    # Steps of so many rows by sums. One prompt, 8 layers of 4 streams of 2,048, us with streams and by sums: 240 tokens 1,226 and 1,262 (up to
-    # 256 rows hyper_norm has 8 waves to a row), 257 1,451, 1,439, 400 1,546, 1,522, 1,000 2,223, 2,158, 3,658 5,923, 5,707
-    SUMS_MIN_T = 257
+    # Steps of so many rows, of so wide ones and of so many elements by sums. One prompt, 8 layers of 4 streams, us with streams and by sums: width
+    # 2,048, 240 tokens 1,226 and 1,262 (up to 256 rows hyper_norm has 8 waves to a row), 257 1,451, 1,439, 400 1,546, 1,522, 1,000 2,223, 2,158,
+    # 3,658 5,923, 5,707; 1,536 310 1,704, 1,718, 350 1,835, 1,832, 1,000 2,486, 2,448; 1,280 350 1,646, 1,660, 400 1,776, 1,772,
+    # 3,900 4,935, 4,860; 1,024 257 1,377, 1,423, 1,000 2,003, 2,015, 3,900 4,193, 4,202; 256 257 927, 981, 3,900 2,540, 2,718
+    SUMS_MIN_T, SUMS_MIN_D, SUMS_MIN = 257, 1280, 257 * 2048
 
     def __init__(self, cfg: MudepelConfig, device, dtype=torch.bfloat16, tp: Optional[TPGroup] = None, seed: int = 0,
                  weights_path: Optional[str] = None, max_len: int = 8192, **_):
@@ -227,6 +229,12 @@ class MudepelModel(HybridModel):
             return rand.normal_(0.0, rand.shape[1] ** -0.5, generator=g)
         return rand.normal_(0.0, cfg.init_std, generator=g)
 
+    def plan_for(self, T: int, residuals: Optional[list]):
+        """The plan of a step of T rows by sums, or None: streams."""
+        d = self.cfg.hidden_size
+        wide = T >= self.SUMS_MIN_T and d >= self.SUMS_MIN_D and T * d >= self.SUMS_MIN
+        return self.sums if wide and residuals is None else None
+
     # -- forward -----------------------------------------------------------------
     def forward(self, meta: StepMeta, kv: HybridCache, num_tokens: int, num_logit_rows: int, part_o: torch.Tensor,
                 part_ml: torch.Tensor, embed=None, residuals: Optional[list] = None) -> torch.Tensor:
@@ -237,7 +245,7 @@ class MudepelModel(HybridModel):
         ldh = pad_to(d, 64)
         new_h = lambda n=T: torch.empty(n, ldh, dtype=self.dtype, device=dev)  # noqa: E731
         room = self.room(part_o, part_ml)
-        x = Residual(self.sums if T >= self.SUMS_MIN_T and residuals is None else None, cfg.streams, self.embed, meta.input_ids[:T])
+        x = Residual(self.plan_for(T, residuals), cfg.streams, self.embed, meta.input_ids[:T])
         for j, i in enumerate(self.runs):
             L = self.layers[i]
             h = x.norm(eps, pre=L["hc1"]["in"], w_next=L["norm1"], out=new_h(), live=meta.slots)

@@ -97,13 +97,19 @@ def test_rows_without_a_token_stay(gpu, T, live):
     assert torch.equal(a[:live], c[:live]) and torch.equal(xa[:live], xc[:live]) and (c[live:] == 7.0).all() and (xc[live:] == 7.0).all()
 
 
+def by_sums(monkeypatch, model, rows):
+    """Steps of so many rows take the form, whatever their width."""
+    for name, least in (("SUMS_MIN_T", rows), ("SUMS_MIN_D", 1), ("SUMS_MIN", 1)):
+        monkeypatch.setattr(model, name, least)
+
+
 @pytest.mark.parametrize("device", DEVICES)
 @pytest.mark.parametrize("name", ["varied", "state_only", "wide"])
 def test_model_of_sums(folder, monkeypatch, name, device):
     """Portions of any length by sums: routed experts' partials, biases, a looped stack."""
     from pilottai_amd.models.mudepel import MudepelModel
 
-    monkeypatch.setattr(MudepelModel, "SUMS_MIN_T", 1)
+    by_sums(monkeypatch, MudepelModel, 1)
     eng, ids = engine(folder, name, device, "bfloat16"), tokens(name, 150)
     assert eng.model.sums is not None
     close(feed(eng, 1, ids, [70, 1, 79]), expect(folder, name, ids), "bfloat16")
@@ -115,7 +121,7 @@ def test_a_pool_beside_logits(folder, monkeypatch, rows, device):
     """A step that also pools embeddings: logits have the bits of the step without, and the pool has the streams' sum."""
     from pilottai_amd.models.mudepel import MudepelModel
 
-    monkeypatch.setattr(MudepelModel, "SUMS_MIN_T", rows)
+    by_sums(monkeypatch, MudepelModel, rows)
     T = max(rows, 40) + 3
     got, ids = [], tokens("wide", T)
     for pooled in (False, True):
@@ -133,3 +139,17 @@ def test_a_pool_beside_logits(folder, monkeypatch, rows, device):
     want = oracle.norm(lay[-1], tw["final.norm"].double(), 1e-4).mean(0)
     off = (embed[1][0].double().cpu() / T - want).pow(2).mean().sqrt() / want.std()
     assert off < 0.08, float(off)  # (of `close`: bf16, median)
+
+
+@pytest.mark.parametrize("name,T,taken", [("varied", 300, False), ("mudepel-base", 256, False), ("mudepel-base", 257, True), ("mudepel-wide", 257, True)])
+def test_steps_that_are_wide_enough(folder, monkeypatch, name, T, taken):
+    """Few rows and narrow ones keep their streams."""
+    from pilottai_amd.models import mudepel
+
+    if name == "varied":
+        model = engine(folder, name, "cpu", "bfloat16").model
+    else:  # (what forward reads before it knows)
+        model = mudepel.MudepelModel.__new__(mudepel.MudepelModel)
+        model.cfg = mudepel.PRESETS[name]
+        model.sums = object()
+    assert (model.plan_for(T, None) is not None) == taken and model.plan_for(T, []) is None
